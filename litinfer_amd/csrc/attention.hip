@@ -1039,6 +1039,18 @@ __device__ __forceinline__ float max3f(float a, float b, float c) {
     return r;
 }
 
+// The largest of a lane's 16 scores.  The first maximum is an ordinary one: vector instructions must not read a
+// matrix instruction's result for some cycles after its issue, the compiler keeps that distance only for
+// instructions it made itself, not for inline assembly, and every later maximum waits for the first.  (With the
+// assembly first the maxima were taken of whatever the registers still held: the reference that the exponentials
+// are taken against, and with it the last bits of the output, changed from run to run.)
+__device__ __forceinline__ float largest_of(const f32x16_t& sv) {
+    float mx = fmaxf(sv[0], sv[1]);
+#pragma unroll
+    for (int r = 2; r < 16; r += 2) mx = max3f(mx, sv[r], sv[r + 1]);
+    return mx;
+}
+
 template <int DH>
 __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_mfma_kernel(
     const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __restrict__ out,
@@ -1229,11 +1241,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_mfma_k
                     sv[r] = (key <= pq && key >= lq) ? sv[r] : -INFINITY;
                 }
             }
-            float mx = max3f(sv[0], sv[1], sv[2]);
-#pragma unroll
-            for (int r = 3; r < 15; r += 2) mx = max3f(mx, sv[r], sv[r + 1]);
-            mx = max3f(mx, sv[15], sv[15]);
-            mx = both_halves_max(mx) * scale2;                          // (scale2 > 0)
+            const float mx = both_halves_max(largest_of(sv)) * scale2;                          // (scale2 > 0)
             if (__any(mx > m + 8.0f)) {
                 const float mn = fmaxf(m, mx);
                 const float alpha = (mn == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - mn);   // (m = -inf: nothing summed yet)
@@ -1521,11 +1529,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
                     sv[r] = (key <= pq && key >= lq) ? sv[r] : -INFINITY;
                 }
             }
-            float mx = max3f(sv[0], sv[1], sv[2]);
-#pragma unroll
-            for (int r = 3; r < 15; r += 2) mx = max3f(mx, sv[r], sv[r + 1]);
-            mx = max3f(mx, sv[15], sv[15]);
-            mx = both_halves_max(mx) * scale2;                          // (scale2 > 0)
+            const float mx = both_halves_max(largest_of(sv)) * scale2;                          // (scale2 > 0)
             if (__any(mx > m + 8.0f)) {
                 const float mn = fmaxf(m, mx);
                 const float alpha = (mn == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - mn);   // (m = -inf: nothing summed yet)
@@ -1793,11 +1797,7 @@ __global__ __launch_bounds__(2 * PRE_WAVES * 64) void paged_attention_prefill_sp
                     sv[r] = (key <= pq && key >= lq) ? sv[r] : -INFINITY;
                 }
             }
-            float mx = max3f(sv[0], sv[1], sv[2]);
-#pragma unroll
-            for (int r = 3; r < 15; r += 2) mx = max3f(mx, sv[r], sv[r + 1]);
-            mx = max3f(mx, sv[15], sv[15]);
-            mx = both_halves_max(mx) * scale2;                          // (scale2 > 0)
+            const float mx = both_halves_max(largest_of(sv)) * scale2;                          // (scale2 > 0)
             if (__any(mx > m + 8.0f)) {
                 const float mn = fmaxf(m, mx);
                 const float alpha = (mn == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - mn);   // (m = -inf: nothing summed yet)
