@@ -170,15 +170,21 @@ __global__ __launch_bounds__(256) void gemm_f32_big_kernel(const float* __restri
 // reads consecutive words, and the transposing writes of the 16-byte global loads (lane = row / k-quarter)
 // meet no bank twice.  Two stages: the next step's global loads are in registers while this step is
 // multiplied.  K a multiple of 4; rows and columns past the end repeat the last and are not stored.
+// gridDim.z > 1: K is cut into that many parts of `part_steps` steps (the last one shorter), and part z's sums go to
+// the z-th [M, N] matrix behind `out`, without bias (splitk_reduce_kernel adds them up in order; see f32_split_parts).
 #define F32M_BM 128
 #define F32M_BN 128
 #define F32M_BK 16
 #define F32M_LD (F32M_BM + 4)
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ out,
-                                                             int M, int N, int K, float accumulate) {
+                                                             int M, int N, int row_len, float accumulate, int part_steps) {
     __shared__ float As[2][F32M_BK * F32M_LD];
     __shared__ float Bs[2][F32M_BK * F32M_LD];
+    // this block's k-values: [k_first, k_first + K) of rows of row_len
+    const int k_first = blockIdx.z * part_steps * F32M_BK;
+    const int K = gridDim.z == 1 || blockIdx.z + 1 == gridDim.z ? row_len - k_first : part_steps * F32M_BK;
+    out += (size_t)blockIdx.z * M * N;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m0 = blockIdx.y * F32M_BM, n0 = blockIdx.x * F32M_BN;
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
@@ -189,8 +195,8 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int ra = m0 + lrow + 64 * h, rb = n0 + lrow + 64 * h;
-        xa[h] = x + (size_t)(ra < M ? ra : M - 1) * K + 4 * lkq;
-        wb[h] = w + (size_t)(rb < N ? rb : N - 1) * K + 4 * lkq;
+        xa[h] = x + (size_t)(ra < M ? ra : M - 1) * row_len + k_first + 4 * lkq;
+        wb[h] = w + (size_t)(rb < N ? rb : N - 1) * row_len + k_first + 4 * lkq;
     }
     floatx4 ga[2], gb[2];
     // WHOLE: the step's 16 k-values lie inside K; nothing is then chosen or replaced (a value chosen between what
@@ -1966,8 +1972,50 @@ static int split_parts_many_rows(int M, int N, int K) {
     return nsplit < 2 ? 1 : nsplit;
 }
 
+static void launch_f32_mfma(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
+                            float accumulate, int parts, hipStream_t stream) {
+    const int steps = (K + F32M_BK - 1) / F32M_BK;
+    const dim3 tiles((N + F32M_BN - 1) / F32M_BN, (M + F32M_BM - 1) / F32M_BM, parts);
+    gemm_f32_mfma_kernel<<<tiles, 256, 0, stream>>>(x, w, bias, out, M, N, K, accumulate, (steps + parts - 1) / parts);
+}
+
+// Into how many parts K is cut for the float32 tiles of 128 x 128 (more than 64 rows): a narrow matrix has fewer tiles
+// than the chip has compute units (810 rows against 1,536 columns: 84), and a tile's time is the length of K whatever the
+// others do.  The least estimated time, in microseconds: a step of 16 k-values takes a unit 1.2 us (0.43 TFLOP/s a unit;
+// blocks that share a unit overlap by some 5 %), a block 6 for its start and end, and the parts' sums are written and
+// read again at 5 TB/s by a kernel of its own (4 us).  Measured, one part against the parts taken here: 65 to 128 rows
+// x 1,536 x 8,960 685 -> 60 us (16 parts), 300 rows 683 -> 130 (6), 810 rows 682 -> 227 (6), x 1,536 x 1,536 138 -> 56,
+// 810 x 2,048 x 1,536 135 -> 75 (2), 1,024 x 3,584 x 18,944 1,464 -> 1,107 (8), 2,048 x 3,584 x 3,584 495 -> 452 (4);
+// from some thousand tiles on (810 x 17,920: 980) parts cost what they give, and K stays whole.  The rule is within
+// 6 % of the best number of parts measured at 65 to 4,096 rows against seven matrices (13 % at 128 rows x 1,536 x 1,536
+// and 810 x 4,608 x 3,584).  At most 256 MB of parts.
+#define F32_MAX_PARTS 16
+#define F32_PARTS_MAX_BYTES (256l << 20)
+#define F32_PART_MIN_STEPS 6
+static int f32_split_parts(int M, int N, int K) {
+    if (M <= F32_ROWS_MAX || K % 4) return 1;
+    const long tiles = (long)((M + F32M_BM - 1) / F32M_BM) * ((N + F32M_BN - 1) / F32M_BN);
+    const int steps = (K + F32M_BK - 1) / F32M_BK, cu = compute_units();
+    int pick = 1;
+    double best = 0.0;
+    for (int p = 1; p <= F32_MAX_PARTS && p * F32_PART_MIN_STEPS <= steps; ++p) {
+        const int per = (steps + p - 1) / p;
+        if ((long)per * (p - 1) >= steps) continue;                      // (a part would be empty)
+        if (p > 1 && (long)p * M * N * (long)sizeof(float) > F32_PARTS_MAX_BYTES) break;
+        const long rounds = (tiles * p + cu - 1) / cu;
+        double us = rounds * (per * 1.2 * (rounds > 1 ? 0.95 : 1.0)) + 6.0;
+        if (p > 1) us += 4.0 + (p + 2) * 4.0 * M * N / 5.0e6;
+        if (p == 1 || us < best) { best = us; pick = p; }
+    }
+    return pick;
+}
+
 // Bytes of workspace with which li_linear cuts this product along K (0: it would not).
 extern "C" long li_linear_work_bytes(int M, int N, int K, int in_dtype) {
+    if (in_dtype == LI_F32) {
+        const int parts = N > 0 && K > 0 ? f32_split_parts(M, N, K) : 1;
+        return parts < 2 ? 0 : (long)parts * M * N * (long)sizeof(float);
+    }
     if (in_dtype != LI_BF16 || N <= 0 || K <= 0 || K % 64 || li_few_rows_preferred(M, N, K)) return 0;
     int nsplit = 1;
     if (M <= 64) {
@@ -2059,9 +2107,16 @@ extern "C" int li_linear(const void* x, const void* w, const float* bias, void* 
         if (M <= F32_ROWS_MAX && K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0)
             return launch_f32_rows((const float*)x, (const float*)w, bias, (float*)out, M, N, K, accumulate, stream);
         if (K % 4 == 0 && (((uintptr_t)x | (uintptr_t)w) & 15) == 0) {       // the matrix cores' float32 form
-            dim3 tiles((N + F32M_BN - 1) / F32M_BN, (M + F32M_BM - 1) / F32M_BM);
-            if (tiles.y > 65535) return LI_ERR_SIZE;
-            gemm_f32_mfma_kernel<<<tiles, 256, 0, stream>>>((const float*)x, (const float*)w, bias, (float*)out, M, N, K, accumulate);
+            if ((M + F32M_BM - 1) / F32M_BM > 65535) return LI_ERR_SIZE;
+            const int parts = f32_split_parts(M, N, K);
+            const size_t mn = (size_t)M * N;
+            if (parts > 1 && work && (size_t)work_bytes >= (size_t)parts * mn * sizeof(float)) {
+                launch_f32_mfma((const float*)x, (const float*)w, nullptr, (float*)work, M, N, K, 0.f, parts, stream);
+                const unsigned blocks = (unsigned)((mn + 255) / 256);
+                splitk_reduce_kernel<float><<<blocks, 256, 0, stream>>>((const float*)work, parts, mn, N, bias, (float*)out, accumulate);
+            } else {
+                launch_f32_mfma((const float*)x, (const float*)w, bias, (float*)out, M, N, K, accumulate, 1, stream);
+            }
             return li_launch_status();
         }
         if (M >= 2 * F32B_BM && N >= F32B_BN) {              // enough of both for the large tile to fill the chip

@@ -958,7 +958,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: 
     x [M, K] and w [N, K] of one dtype (float32 or bfloat16); out [M, N] of that
     dtype or float32; accumulation of the product is float32.  `ws` lends the
     memory for partial sums where the kernel cuts K into parts (17 rows and more
-    against a matrix of few columns); without it
+    against a matrix of few columns, in float32 65 rows and more); without it
     such a product takes a slower kernel."""
     _gpu(x, w, bias, out)
     _chk(x.dim() == 2 and w.dim() == 2 and out.dim() == 2, "linear: needs matrices")
@@ -976,8 +976,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: 
          "linear: bias must be float32 [N]")
     if m:
         work, work_bytes = 0, 0
-        if ws is not None and x.dtype is torch.bfloat16 and not few_rows_preferred(m, n, k):
-            # few rows over a long k and few columns: the library cuts k into parts if it is lent room for their sums
+        if ws is not None and (not few_rows_preferred(m, n, k) if x.dtype is torch.bfloat16 else m > SKINNY_MAX_ROWS):
+            # too few tiles to fill the chip: the library cuts k into parts if it is lent room for their sums
             need = _work_bytes(m, n, k, _DT[x.dtype])
             if need:
                 if m <= SKINNY_MAX_ROWS:            # one size for all row counts of a decode batch: the buffer does not move

@@ -187,6 +187,33 @@ def test_linear_with_k_in_parts(ops, m, n, k, out_dtype, bias, acc):
     assert torch.equal(again, outs[0])                   # the parts are added in a fixed order
 
 
+@pytest.mark.parametrize("m,n,k,bias,factor", [
+    (65, 100, 204, False, 1.0),              # one row more than the few-row kernel takes; parts of 7 and 6 steps, the last step of 12 k-values
+    (129, 1536, 8960, True, 1.0),            # the most parts
+    (300, 1537, 1540, True, 0.5),            # a column and a piece of a step over
+    (810, 1536, 1536, False, 1.0),
+    (257, 260, 4096, True, 0.0),             # not accumulating
+    (2048, 300, 92, True, 1.0),              # too short a K for parts
+])
+def test_float32_linear_with_k_in_parts(ops, m, n, k, bias, factor):
+    from litinfer_amd.kernels.ops import _work_bytes
+    g = torch.Generator().manual_seed(62)
+    x = torch.randn(m, k, generator=g)
+    w = torch.randn(n, k, generator=g) / math.sqrt(k)
+    b = torch.randn(n, generator=g) if bias else None
+    base = torch.randn(m, n, generator=g)
+    assert (_work_bytes(m, n, k, 0) > 0) == (k > 100)          # the case is what it says
+    y = x.double().numpy() @ w.double().numpy().T + (0 if b is None else b.double().numpy())
+    y = base.double().numpy() + factor * y if factor else y
+    outs = []
+    for ws in (_Lender(), None, _Lender()):
+        out = base.to(DEV) if factor else torch.full((m, n), float("nan"), device=DEV)
+        ops.linear(x.to(DEV), w.to(DEV), None if b is None else b.to(DEV), out, bool(factor), ws=ws, factor=factor or 1.0)
+        assert rel(out, y) < 4 * math.sqrt(k) * 2.0 ** -24     # (as for the product in one piece)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[2])                       # the parts are added in a fixed order
+
+
 @pytest.mark.parametrize("m,n,k,bias,taken", [
     (64, 3584, 18944, False, True),      # a decoding batch of 64 at the 7B sizes
     (40, 200, 1024, True, True),
