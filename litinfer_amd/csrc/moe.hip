@@ -5,11 +5,15 @@
 // sized by what a step can have at most.
 #include "common.h"
 
+#include <type_traits>
+
 #define MOE_TILE 32            // rows of one expert that a tile holds
 #define MOE_BIG_TILE 64        // ... where experts get hundreds of rows each (a prompt's portion): the tiles of the LDS kernel,
 #define MOE_HUGE_TILE 128      // and twice that where they get still more
 #define MOE_NARROW_BYTES (16l << 20)   // a decoding step's tiles against matrices below this size take 64 columns a block: more blocks, filled more evenly (1.5B sizes 38 -> 32 us; 7B sizes 138 against 155 us)
-#define MOE_FEW_ROWS 32        // rows of a step up to which every row is a matrix-vector product of its own
+#define MOE_FEW_ROWS 32        // rows of a step up to which every row may be a matrix-vector product of its own,
+#define MOE_VECTOR_ROWS 4      // ... and up to which it is one also where the kernel that streams the matrices could take them
+#define MOE_STREAM_ROWS_A_TILE 12  // rows a tile, on average, up to which that kernel is taken (see moe_linear_launch)
 
 // ------------------------------------------------------------------------------------------------ router
 // One block a token.  logits[e] = b[e] + sum_k W[e, k] x[k] in float32 (a wave an expert, in turns); the `top`
@@ -357,6 +361,7 @@ __global__ __launch_bounds__(256) void moe_linear_kernel(const TA* __restrict__ 
 // 16-byte pieces of rows as they lie in memory and a lane ends with four consecutive outputs of its row.
 typedef __bf16 moe_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float moe_f32x16 __attribute__((ext_vector_type(16)));
+typedef float moe_f32x4 __attribute__((ext_vector_type(4)));
 union moe_frag8 { uint4 raw; uint32_t w[4]; moe_bf16x8 v; };
 
 template <bool EXT, typename TA, typename TO>
@@ -608,6 +613,115 @@ __global__ __launch_bounds__(256) void moe_linear_rows_kernel(const bf16_t* __re
     }
 }
 
+// A decoding step of a batch: few rows an expert, and every tile streams its expert's matrix, so the product is bound by
+// how many bytes of the matrices are on their way.  A block takes a tile and 16 NT outputs; its four waves take K in
+// chunks of 128 in turn, each with the loads of its NEXT chunk (16 bytes a lane, 64 neighbouring bytes of a matrix row an
+// instruction; whole chunks without conditions) in flight while it multiplies one, and add up through LDS in wave order.
+// v_mfma_f32_16x16x32_bf16 has the matrix as the row operand and 16 of the tile's rows as the column operand, so a lane
+// ends with four neighbouring outputs of one row; a tile of more than 16 rows is gone through twice (the block's share
+// of the matrix is in the L2 by then).  The rows are read 256 neighbouring bytes of a row at a time and turned into the
+// operand's order through a piece of LDS of the wave's own, as in the few-row product of a dense layer.
+#define MS_CHUNK 128
+template <bool EXT, typename TO, int NT>
+__global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __restrict__ a, long a_stride, const int* __restrict__ row_token,
+                                                                const bf16_t* __restrict__ w, const int* __restrict__ plan,
+                                                                TO* __restrict__ out, long out_stride, int n_out, int K, MoeEpilogue ep) {
+    constexpr int WAVES = 4;
+    const int tile = blockIdx.y;              // (columns first: see the kernel of few rows)
+    if (tile >= plan[0]) return;
+    const int e = plan[4 + 4 * tile], r0 = plan[5 + 4 * tile], nr = plan[6 + 4 * tile];
+    __shared__ moe_f32x4 red[WAVES][NT][64];
+    __shared__ __attribute__((aligned(16))) uint16_t xs_all[WAVES][16 * MS_CHUNK];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, r16 = lane & 15;
+    const int j0 = blockIdx.x * 16 * NT;
+    uint16_t* xs = xs_all[wave];
+    // (piece p of row r lies at place p ^ r: the rows that a fragment read touches fall into all banks)
+    auto xslot = [](int row, int piece) { return row * MS_CHUNK + ((piece ^ row) << 3); };
+    const bf16_t* wrow[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int j = j0 + 16 * nt + r16;
+        wrow[nt] = w + ((size_t)e * n_out + (j < n_out ? j : n_out - 1)) * K + 8 * g;
+    }
+    const int nfull = K / MS_CHUNK, nchunks = (K + MS_CHUNK - 1) / MS_CHUNK;
+    const moe_frag8 zero = {};
+    for (int rc = 0; rc < nr; rc += 16) {
+        const bf16_t* xrow[4];                // this lane's rows of x: g + 4 i, the last one repeated past the tile's end
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = r0 + (rc + g + 4 * i < nr ? rc + g + 4 * i : nr - 1);
+            xrow[i] = a + (size_t)(row_token ? row_token[r] : r) * a_stride + 8 * r16;
+        }
+        moe_f32x4 acc[NT];
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[nt] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
+        moe_frag8 wbuf[2][NT][4], xbuf[2][4];
+        auto load_chunk = [&](int c, moe_frag8 (*wd)[4], moe_frag8* xd, auto tail_tag) {
+            constexpr bool TAIL = decltype(tail_tag)::value;
+            const int kb = c * MS_CHUNK;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if constexpr (TAIL) { xd[i] = zero; if (kb + 8 * r16 < K) xd[i].raw = *reinterpret_cast<const uint4*>(xrow[i] + kb); }
+                else xd[i].raw = *reinterpret_cast<const uint4*>(xrow[i] + kb);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int nt = 0; nt < NT; ++nt) {
+                    if constexpr (TAIL) { wd[nt][j] = zero; if (kb + 8 * g + 32 * j < K) wd[nt][j].raw = *reinterpret_cast<const uint4*>(wrow[nt] + kb + 32 * j); }
+                    else wd[nt][j].raw = *reinterpret_cast<const uint4*>(wrow[nt] + kb + 32 * j);
+                }
+        };
+        auto multiply = [&](moe_frag8 (*wa)[4], moe_frag8* xd) {
+            __builtin_amdgcn_wave_barrier();  // (a wave's LDS instructions are carried out in order; keep the compiler's too)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&xs[xslot(g + 4 * i, r16)]) = xd[i].raw;
+            __builtin_amdgcn_wave_barrier();
+            moe_frag8 xa[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) xa[j].raw = *reinterpret_cast<const uint4*>(&xs[xslot(r16, g + 4 * j)]);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[nt][j].v, xa[j].v, acc[nt], 0, 0, 0);
+            __builtin_amdgcn_wave_barrier();
+        };
+        // Nothing about the loads inside the loop is conditional: it runs while both of a turn's loads exist, and the one or
+        // two chunks that are left are taken behind it (where a path with loads and one without meet, the compiler waits for all).
+        int c = wave;
+        if (c < nfull) {
+            load_chunk(c, wbuf[0], xbuf[0], std::false_type{});
+            for (; c + 2 * WAVES < nfull; c += 2 * WAVES) {
+                load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
+                multiply(wbuf[0], xbuf[0]);
+                load_chunk(c + 2 * WAVES, wbuf[0], xbuf[0], std::false_type{});
+                multiply(wbuf[1], xbuf[1]);
+            }
+            const bool more = c + WAVES < nfull;
+            if (more) load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
+            multiply(wbuf[0], xbuf[0]);
+            if (more) multiply(wbuf[1], xbuf[1]);
+        }
+        if (nfull < nchunks && wave == nfull % WAVES) {      // the chunk that K ends in
+            load_chunk(nfull, wbuf[0], xbuf[0], std::true_type{});
+            multiply(wbuf[0], xbuf[0]);
+        }
+        if (rc) __syncthreads();              // the sums of the 16 rows before have been read
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) red[wave][nt][lane] = acc[nt];
+        __syncthreads();
+        if (wave < NT) {                      // wave nt writes the 16 outputs of column tile nt
+            moe_f32x4 s = red[0][wave][lane];
+#pragma unroll
+            for (int v = 1; v < WAVES; ++v) s += red[v][wave][lane];
+            const int row = rc + r16, col = j0 + 16 * wave + 4 * g;
+            if (row < nr && col < n_out)
+                moe_store4<EXT>(out + (size_t)(r0 + row) * out_stride, col, s[0], s[1], s[2], s[3], ep, moe_row_factor<EXT>(ep, r0 + row));
+        }
+    }
+}
+
 // Many rows an expert (tiles of up to 64 rows): a block takes a tile and 128 outputs, K in steps of 32 through LDS, so
 // that a matrix row that came from memory serves 64 rows and a token's row 128 outputs; its four waves are two by two,
 // each with 32 rows x 64 outputs (two accumulators).  The block is small on purpose: five or more of them share a compute
@@ -754,9 +868,28 @@ static int moe_linear_launch(const void* a, int a_dtype, long a_stride, const in
         return li_launch_status();
     }
     if (tile_rows != MOE_TILE) return LI_ERR_SIZE;
-    // a handful of rows in all: a matrix-vector product a row (each tile streams its expert's matrix anyway)
-    if (rows <= MOE_FEW_ROWS && a_dtype == LI_BF16 && w_dtype == LI_BF16 && K % 8 == 0 && a_stride % 8 == 0 &&
-        ((uintptr_t)a | (uintptr_t)w) % 16 == 0 && (out_dtype == LI_BF16 || out_dtype == LI_F32)) {
+    // A decoding step: each tile streams its expert's matrix.  16 experts, us a product before (matrix-vector products up to
+    // 32 rows, tiles of 32 rows with K in quarters above) and with the kernel that streams, 1.5B sizes (2,240 x 1,536):
+    // 2 rows 6.6 / 6.7, 4 rows 8.5 / 8.7, 8 rows 15.0 / 13.2, 32 rows 23.2 / 19.5, 64 rows 37.8 / 23.3 (110 MB: 4.7 TB/s),
+    // 128 rows 39.0 / 24.7, 256 rows 40.3 / 37; gate and up together (4,480) at 32 rows 42.4 / 33.6; 7B sizes (4,736 x
+    // 3,584) at 2 rows 14.1 / 14.9, 32 rows 81 / 75, 64 rows 146 / 93.5, 256 rows 155 / 136.  Above 16 rows a tile it goes
+    // through the matrix twice, so tiles of more than 12 rows on average stay with the wider ones.  Two column tiles a
+    // block (half the reads of x) from four rows a tile on: 128 rows 25.4 / 24.7, 8 rows 13.2 / 14.3.
+    const bool pieces = a_dtype == LI_BF16 && w_dtype == LI_BF16 && K % 8 == 0 && a_stride % 8 == 0 &&
+                        ((uintptr_t)a | (uintptr_t)w) % 16 == 0 && (out_dtype == LI_BF16 || out_dtype == LI_F32);
+    const int gate2 = ep.act == 2 || ep.act == 3 ? 2 : 1;        // (a store takes four sums: two outputs where they are pairs)
+    if (pieces && rows > MOE_VECTOR_ROWS && rows <= MOE_STREAM_ROWS_A_TILE * (long)max_tiles && n_out % 4 == 0 &&
+        out_stride % (4 / gate2) == 0 && (uintptr_t)out % (4 / gate2 * (out_dtype == LI_BF16 ? 2 : 4)) == 0 && max_tiles <= 65535) {
+        const bool two = rows >= 4l * max_tiles;
+        const dim3 grid((n_out + (two ? 31 : 15)) / (two ? 32 : 16), max_tiles);
+#define MS(TO, NT) moe_linear_stream_kernel<EXT, TO, NT><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (TO*)out, out_stride, n_out, K, ep)
+        if (out_dtype == LI_BF16) { if (two) MS(bf16_t, 2); else MS(bf16_t, 1); }
+        else { if (two) MS(float, 2); else MS(float, 1); }
+#undef MS
+        return li_launch_status();
+    }
+    // a handful of rows in all: a matrix-vector product a row
+    if (rows <= MOE_FEW_ROWS && pieces) {
         const dim3 grid((n_out + 4 * MR_OUT - 1) / (4 * MR_OUT), max_tiles);
         if (out_dtype == LI_BF16)
             moe_linear_rows_kernel<EXT, bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (bf16_t*)out, out_stride, n_out, K, ep);

@@ -1094,3 +1094,48 @@ def test_decode_attention_refuses_block_tables_beyond_the_keys_its_page_quotient
     q = torch.zeros(1, nh * dh, dtype=torch.bfloat16, device=DEV)
     with pytest.raises(ValueError, match="beyond the decode kernel"):
         ops.paged_attention(q, torch.empty_like(q), kc, kc.clone(), meta, nh, nkv, dh, page, 0, 0.1)
+
+
+@pytest.mark.parametrize("counts,n_out,k,act,weigh,gather,out_dtype", [
+    ([1, 16, 0, 17, 32, 3], 36, 1000, 0, False, True, torch.float32),      # one row, whole and broken halves of a tile; a last chunk of 104 k-values, a last column tile of 4
+    ([5, 2], 4, 8, 0, False, False, torch.bfloat16),                       # less than a chunk
+    ([3, 0, 2], 64, 1280, 2, False, True, torch.bfloat16),                 # pairs of gate and up
+    ([2, 9, 40], 100, 520, 3, False, True, torch.float32),                 # the clamped pairs; an expert of two tiles
+    ([7, 6, 1], 20, 136, 4, True, True, torch.bfloat16),                   # weights on the input, gelu
+    ([30, 1, 28], 132, 1160, 1, False, False, torch.bfloat16),
+    ([9, 11, 10], 34, 264, 0, False, True, torch.float32),                 # 34 outputs: not a multiple of 4, another kernel
+])
+def test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, weigh, gather, out_dtype):
+    """Rows of every expert against its matrix; a float32 result within the random walk of K products' sums, a bfloat16
+    one within its rounding (2^-9 of a value, taken twice)."""
+    g = torch.Generator().manual_seed(63)
+    rows, E = sum(counts), len(counts)
+    tokens = rows if not gather else rows + 3
+    a = torch.randn(tokens, k + 8, generator=g).to(torch.bfloat16)[:, :k]             # rows with a stride of their own
+    w = (torch.randn(E, n_out, k, generator=g) / math.sqrt(k) * 2).to(torch.bfloat16)
+    src = torch.randperm(tokens, generator=g)[:rows] if gather else torch.arange(rows)
+    row_wt = torch.rand(rows, generator=g) + 0.5 if weigh else None
+    tiles, r, ref = [], 0, []
+    for e, n in enumerate(counts):
+        tiles += [(e, r + o, min(32, n - o), 0) for o in range(0, n, 32)]
+        y = a[src[r:r + n]].double() @ w[e].double().t()
+        ref.append(y * row_wt[r:r + n, None].double() if weigh else y)
+        r += n
+    y = torch.cat(ref)
+    if act == 1:
+        y = y.clamp(min=0) ** 2
+    elif act == 2:
+        y = torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2]
+    elif act == 3:
+        gate, up = y[:, 0::2].clamp(max=1.5), y[:, 1::2].clamp(-1.5, 1.5)
+        y = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+    elif act == 4:
+        y = torch.nn.functional.gelu(y)
+    plan = torch.tensor([len(tiles), rows, 0, 0] + [v for t in tiles for v in t], dtype=torch.int32)
+    plan = torch.cat([plan, torch.full((8,), -1, dtype=torch.int32)])                  # two tiles that the plan does not have
+    out = torch.full((rows, y.shape[1]), float("nan"), dtype=out_dtype, device=DEV)
+    wide = torch.zeros(tokens, k + 8, dtype=torch.bfloat16, device=DEV)
+    wide[:, :k] = a.to(DEV)
+    ops.moe_linear(wide[:, :k], src.to(torch.int32).to(DEV) if gather else None, w.to(DEV), plan.to(DEV), len(tiles) + 2, out, rows,
+                   act=act, limit=1.5 if act == 3 else 0.0, row_wt=None if row_wt is None else row_wt.to(DEV))
+    assert rel(out, y.numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
