@@ -171,17 +171,18 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_kernel(
     const float Dh = (MODE == 0 && active && Dw) ? Dw[head] : 0.f;
     for (int b0 = 0; b0 < ntok; b0 += SSM_TB) {
         __syncthreads();
-        for (int i = threadIdx.x; i < SSM_TB * NP; i += 64 * SSM_WAVES) {
+        const int nt = (ntok - b0 < SSM_TB) ? ntok - b0 : SSM_TB;          // (one in a decoding step: what is staged for the others would be waited for)
+        for (int i = threadIdx.x; i < nt * NP; i += 64 * SSM_WAVES) {
             const int tt = i / NP, n = i % NP;
-            const bool ok = b0 + tt < ntok && n < N;
+            const bool ok = n < N;
             const float* row = xbc + (size_t)(t0 + b0 + tt) * xbc_stride + inner + (size_t)g * N + n;
             sB[i] = ok ? silu_if<SILU>(row[0]) : 0.f;
             sC[i] = ok ? silu_if<SILU>(row[(size_t)G * N]) : 0.f;
         }
         if (active) {
-            for (int i = lane; i < SSM_TB * PW; i += 64) {
+            for (int i = lane; i < nt * PW; i += 64) {
                 const int tt = i / PW, pp = pbase + i % PW;
-                const bool ok = b0 + tt < ntok && pp < vdim;
+                const bool ok = pp < vdim;
                 sX[(w * SSM_TB + tt) * PW + i % PW] = ok ? silu_if<SILU>(xbc[(size_t)(t0 + b0 + tt) * xbc_stride + (size_t)head * vdim + pp]) : 0.f;
             }
             if (lane < SSM_TB) {
@@ -194,7 +195,6 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_kernel(
         }
         __syncthreads();
         if (!active) continue;
-        const int nt = (ntok - b0 < SSM_TB) ? ntok - b0 : SSM_TB;
         for (int tt = 0; tt < nt; ++tt) {
             const float a = sA[w * SSM_TB + tt], dtv = sDt[w * SSM_TB + tt];
             const float xv = sX[(w * SSM_TB + tt) * PW + pl];
@@ -299,17 +299,18 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
     const float Dh = (MODE == 0 && active && Dw) ? Dw[head] : 0.f;
     for (int b0 = 0; b0 < ntok; b0 += SSM_TB) {
         __syncthreads();
-        for (int i = threadIdx.x; i < SSM_TB * NP; i += 64 * SSM_WAVES) {
+        const int nt = (ntok - b0 < SSM_TB) ? ntok - b0 : SSM_TB;          // (one in a decoding step: what is staged for the others would be waited for)
+        for (int i = threadIdx.x; i < nt * NP; i += 64 * SSM_WAVES) {
             const int tt = i / NP, n = i % NP;
-            const bool ok = b0 + tt < ntok && n < N;
+            const bool ok = n < N;
             const float* row = xbc + (size_t)(t0 + b0 + tt) * xbc_stride + inner + (size_t)g * N + n;
             sB[i] = ok ? silu_if<SILU>(row[0]) : 0.f;
             sC[i] = ok ? silu_if<SILU>(row[(size_t)G * N]) : 0.f;
         }
         if (active) {
-            for (int i = lane; i < SSM_TB * PW; i += 64) {
+            for (int i = lane; i < nt * PW; i += 64) {
                 const int tt = i / PW, pp = pbase + i % PW;
-                const bool ok = b0 + tt < ntok && pp < vdim;
+                const bool ok = pp < vdim;
                 sX[(w * SSM_TB + tt) * PW + i % PW] = ok ? silu_if<SILU>(xbc[(size_t)(t0 + b0 + tt) * xbc_stride + (size_t)head * vdim + pp]) : 0.f;
             }
             if (lane < SSM_TB) {
@@ -322,7 +323,6 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
         }
         __syncthreads();
         if (!active) continue;
-        const int nt = (ntok - b0 < SSM_TB) ? ntok - b0 : SSM_TB;
         for (int tt = 0; tt < nt; ++tt) {
             const float a = sA[w * SSM_TB + tt], dtv = sDt[w * SSM_TB + tt];
             const float4 xv = *reinterpret_cast<const float4*>(sX + (w * SSM_TB + tt) * PW + 4 * pq);
@@ -746,6 +746,23 @@ static int ssm_quad_layout(int N, int vdim, int* slices, int* per_lane) {
     return 1;
 }
 
+// A decoding step (one chunk a request) reads the state once and writes it once, so it is bound by how many of its loads
+// are on their way: the columns of a head go to more lanes, and so to more waves and blocks, until there are four blocks
+// a compute unit or a lane holds 8 or 4 values of its columns (a wave 8 loads of 1 KB).  Us a step, before (columns spread
+// only until a block's four waves work, and the staging of 16 tokens gone through for one) and now: state-space, 48 heads
+// of 64 columns, 128 values, 1 / 8 / 32 requests 14.3 / 15.6 / 30.3 -> 6.9 / 9.5 / 23.7 (100 MB: 4.2 TB/s), retention,
+// 12 heads of 128 8.8 / 9.3 / 14.0 -> 6.0 / 6.7 / 12.0, delta rule, 12 heads of 128 16.1 / 16.5 / 17.9 -> 7.5 / 7.9 / 12.5,
+// 28 heads at 64 requests 67.6 -> 54.5.  (256 blocks as the limit: 28.3, 13.7 and 14.4 us at 32 requests.)
+static void ssm_quad_spread(int segs, int heads, int vdim, int G, int* slices, int* per_lane) {
+    const int hpg = heads / G;
+    while (*slices < 16 && *per_lane > 4) {
+        const int pw = 256 / *slices, units = hpg * ((vdim + pw - 1) / pw);
+        if ((long)segs * G * ((units + SSM_WAVES - 1) / SSM_WAVES) >= 1024) return;
+        *slices *= 2;
+        *per_lane /= 2;
+    }
+}
+
 // How a state of N values a column is spread: slices (lanes a column) and values a lane; 0 if no kernel has it.
 extern "C" int li_ssm_scan_layout(int N, int vdim, int* slices, int* per_lane) {
     if (N <= 0 || N > 256 || vdim <= 0) return 0;
@@ -804,6 +821,7 @@ extern "C" int li_ssm_scan(const float* xbc, long xbc_stride, const float* dt_ra
     if (aligned && ssm_quad_layout(N, vdim, &qs, &qr)) {
         // heads that share no B and C have a block of four waves each: columns are spread over more lanes until all four work
         while (!chunked && G == heads && qs < 16 && qr > 4 && vdim <= 2 * (256 / qs)) { qs *= 2; qr /= 2; }
+        if (!chunked) ssm_quad_spread(segs, heads, vdim, G, &qs, &qr);
 #define SSM_QUAD(NR_, NS_)                                                                                                \
     if (qr == NR_ && qs == NS_)                                                                                           \
         return ssm_launch<NR_, NS_, true>(silu_in, xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log, Dw, state, slots, q_start, q_len, \
@@ -917,17 +935,18 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
     }
     for (int b0 = 0; b0 < ntok; b0 += DR_TB) {
         __syncthreads();
-        for (int i = threadIdx.x; i < DR_TB * NP; i += 64 * SSM_WAVES) {
+        const int nt = (ntok - b0 < DR_TB) ? ntok - b0 : DR_TB;
+        for (int i = threadIdx.x; i < nt * NP; i += 64 * SSM_WAVES) {
             const int tt = i / NP, n = i % NP;
-            const bool ok = b0 + tt < ntok && n < N;
+            const bool ok = n < N;
             const float* row = xkq + (size_t)(t0 + b0 + tt) * x_stride + inner + (size_t)g * N + n;
             sK[i] = ok ? row[0] : 0.f;
             sQ[i] = ok ? row[(size_t)G * N] : 0.f;
         }
         if (active) {
-            for (int i = lane; i < DR_TB * PW; i += 64) {
+            for (int i = lane; i < nt * PW; i += 64) {
                 const int tt = i / PW, pp = pbase + i % PW;
-                const bool ok = !is_p && b0 + tt < ntok && pp < vdim;
+                const bool ok = !is_p && pp < vdim;
                 sX[(w * DR_TB + tt) * PW + i % PW] = ok ? xkq[(size_t)(t0 + b0 + tt) * x_stride + (size_t)head * vdim + pp] : 0.f;
             }
             if (lane < DR_TB) {
@@ -938,7 +957,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
             }
         }
         __syncthreads();
-        {   // unit vectors: token tt = thread / 16, sixteen neighbouring lanes share its N values
+        if ((int)(threadIdx.x >> 4) < nt) {   // unit vectors: token tt = thread / 16, sixteen neighbouring lanes share its N values
             const int tt = threadIdx.x >> 4, part = threadIdx.x & 15;
             float sk = 0.f, sq = 0.f;
             for (int n = part; n < NP; n += 16) {
@@ -959,7 +978,6 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
         }
         __syncthreads();
         if (!active) continue;
-        const int nt = (ntok - b0 < DR_TB) ? ntok - b0 : DR_TB;
         for (int tt = 0; tt < nt; ++tt) {
             const float gd = sG[w * DR_TB + tt], beta = sBeta[w * DR_TB + tt];
             float xv[CW];
@@ -1216,6 +1234,7 @@ extern "C" int li_delta_scan(const float* xkq, long x_stride, const float* ba, l
     const bool aligned = ((uintptr_t)state | (uintptr_t)y | (uintptr_t)carry) % 16 == 0 && y_stride % 4 == 0;
     int qs = 0, qr = 0;
     if (aligned && ssm_quad_layout(N, vdim, &qs, &qr)) {
+        if (!chunked) ssm_quad_spread(segs, heads, vdim, G, &qs, &qr);
 #define DR_QUAD(NR_, NS_) if (qr == NR_ && qs == NS_) return delta_launch<NR_, NS_, 4>(DR_ARGS);
         DR_QUAD(4, 2) DR_QUAD(8, 2) DR_QUAD(16, 2) DR_QUAD(32, 2)
         DR_QUAD(4, 4) DR_QUAD(8, 4) DR_QUAD(16, 4) DR_QUAD(32, 4)

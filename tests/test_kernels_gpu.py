@@ -1139,3 +1139,60 @@ def test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, weigh, g
     ops.moe_linear(wide[:, :k], src.to(torch.int32).to(DEV) if gather else None, w.to(DEV), plan.to(DEV), len(tiles) + 2, out, rows,
                    act=act, limit=1.5 if act == 3 else 0.0, row_wt=None if row_wt is None else row_wt.to(DEV))
     assert rel(out, y.numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
+
+
+def _one_token_batch(n):
+    import types
+    at = np.arange(n, dtype=np.int32)
+    dev = lambda a: torch.from_numpy(a).to(DEV)
+    return types.SimpleNamespace(num_tokens=n, num_segments=n, max_q_len=1, host_state_slots=at[::-1].copy(), state_slots=dev(at[::-1].copy()),
+                                 q_start=dev(at), q_len=dev(np.ones(n, dtype=np.int32)))
+
+
+@pytest.mark.parametrize("n,heads,vdim,n_state,groups", [
+    (1, 48, 64, 128, 8),          # few requests: a head's columns over the most lanes
+    (3, 6, 20, 100, 2),           # columns and values that fill neither a wave nor the lanes' shares
+    (2, 4, 256, 256, 4),
+    (5, 2, 4, 12, 1),             # one piece of columns
+    (40, 48, 64, 128, 8),         # enough requests: fewer lanes a column
+])
+@pytest.mark.parametrize("kind", ["ssm", "fixed", "delta"])
+def test_recurrences_of_a_decoding_step(ops, kind, n, heads, vdim, n_state, groups):
+    """One token a request from its state, in slots in reverse order; against the equations in float64, within the random
+    walk of a column's 2 n_state products."""
+    g = torch.Generator().manual_seed(64)
+    R = lambda *s: torch.randn(*s, generator=g)
+    inner, rep = heads * vdim, heads // groups
+    ctx = _one_token_batch(n)
+    state = R(n + 1, heads, n_state, vdim) * 0.3
+    rows = R(n, inner + 2 * groups * n_state)
+    aux, bias, a_log, d = R(n, 2 * heads), R(heads) - 2.0, torch.rand(heads, generator=g), R(heads)
+    fixed = torch.linspace(0.9, 0.99, heads)
+    old = state.double()[torch.arange(n - 1, -1, -1)]
+    w = rows.double()
+    v = w[:, :inner].view(n, heads, vdim)
+    b = w[:, inner:inner + groups * n_state].view(n, groups, n_state).repeat_interleave(rep, 1)
+    c = w[:, inner + groups * n_state:].view(n, groups, n_state).repeat_interleave(rep, 1)
+    dev_state, y = state.to(DEV), torch.full((n, inner), float("nan"), device=DEV)
+    sp = torch.nn.functional.softplus
+    if kind == "delta":
+        unit = lambda z: z / (z.square().sum(-1, keepdim=True) + 1e-6).sqrt()
+        k, q = unit(b), unit(c) * n_state ** -0.5
+        beta, decay = torch.sigmoid(aux.double()[:, :heads]), torch.exp(-a_log.double().exp() * sp(aux.double()[:, heads:] + bias.double()))
+        new = old * decay[:, :, None, None]
+        u = beta[:, :, None] * (v - (new * k[..., None]).sum(2))
+        new = new + k[..., None] * u[:, :, None]
+        want = (new * q[..., None]).sum(2)
+        ops.delta_scan(rows.to(DEV), aux.to(DEV), bias.to(DEV), a_log.to(DEV), dev_state, ctx, y, heads, vdim, n_state, groups, n_state ** -0.5)
+    else:
+        dt = torch.full((n, heads), 0.3, dtype=torch.float64) if kind == "fixed" else sp(aux.double()[:, :heads] + bias.double())
+        decay = fixed.double().expand(n, heads) if kind == "fixed" else torch.exp(-a_log.double().exp() * dt)
+        new = old * decay[:, :, None, None] + (dt[:, :, None] * b)[..., None] * v[:, :, None]
+        want = (new * c[..., None]).sum(2) + d.double()[None, :, None] * v
+        gpu = lambda z: None if kind == "fixed" else z.contiguous().to(DEV)
+        ops.ssm_scan(rows.to(DEV), gpu(aux[:, :heads]), gpu(bias), gpu(a_log), d.to(DEV), dev_state, ctx, y, heads, vdim, n_state, groups, None,
+                     fixed_decay=fixed.to(DEV) if kind == "fixed" else None, fixed_step=0.3)
+    tol_ = 8 * math.sqrt(2 * n_state) * 2.0 ** -24
+    assert rel(y, want.reshape(n, -1).numpy()) < tol_
+    assert rel(dev_state[torch.arange(n - 1, -1, -1)], new.numpy()) < tol_
+    assert torch.equal(dev_state[n].cpu(), state[n])                       # a slot that is not in the batch
