@@ -474,37 +474,77 @@ static int ssm_launch(int silu_in, A... args) { return silu_in ? ssm_launch_as<N
 // Which k-value a step of the matrix cores takes is free as long as both operands agree: the scores K Q^T take the four
 // k-values 8 t + 4 (l / 32) .. + 3 of a 16-byte piece in four steps, and their result, keys as rows, is the row operand of
 // the product with V as it is (register r holds the key whose number the column operand then reads).
+// VAR: a decay a_t = exp(l_t), l_t = -exp(A_log) dt_t, and a step f_t = dt_t of every token's own (the state-space
+// recurrence, whose heads share keys and queries in groups and whose output has a term D_h x_t).  With c_t = l_0 + .. + l_t
+// the powers become exp(c_i - c_j): the sums are taken in float64, because the difference of two sums of sixty-four terms
+// would lose in float32 what the neighbouring tokens, whose factors are near one, need; the factors themselves and all
+// products are float32, as in the recurrence token by token.  48 heads of 64 columns, 128 state values in 8 groups: 2,048
+// tokens 430 us token by token in chunks side by side -> 155 us, 8 portions of 100 tokens 391 -> 97, 65 tokens 176 -> 33;
+// 112 heads, 2,048 tokens 833 -> 318.
 #define RET_Q 64               // tokens of a chunk (SSM chunks of the same length are what the host numbers)
 typedef float ret_f32x16 __attribute__((ext_vector_type(16)));
+
+struct RetDecay {              // where a chunk's decays and steps come from
+    const float* fixed_a;      // [heads]: the same for every token, with `step` ...
+    float step;
+    const float* dt_raw;       // ... or (VAR) the raw steps [T, heads] with their bias, and the heads' rates
+    long dt_stride;
+    const float* dt_bias;
+    const float* A_log;
+};
+
+// c_t and dt_t of a chunk's tokens, by the block's first wave (a token a lane; past the last token c stays as it is)
+__device__ __forceinline__ void ret_chunk_decays(const RetDecay& dc, int t0, int ntok, int head, double* cum, float* dt) {
+    if (threadIdx.x >= RET_Q) return;
+    const int j = threadIdx.x;
+    const float d = j < ntok ? softplus_f32(dc.dt_raw[(size_t)(t0 + j) * dc.dt_stride + head] + dc.dt_bias[head]) : 0.f;
+    double c = (double)(-expf(dc.A_log[head]) * d);
+#pragma unroll
+    for (int o = 1; o < RET_Q; o <<= 1) {
+        const double before = __shfl_up(c, o, LI_WAVE);
+        if (j >= o) c += before;
+    }
+    cum[j] = c;
+    dt[j] = d;
+}
 
 __device__ __forceinline__ float4 silu_if4(float4 v, int on) { return on ? float4{silu_f32(v.x), silu_f32(v.y), silu_f32(v.z), silu_f32(v.w)} : v; }
 
 // WT: fragments of 32 rows (state values) and of 32 columns a wave; the four waves are two by two, a block takes 64 WT of both.
-template <int WT>
+// VAR: chunk_decay[chunk, head] receives what the chunk multiplies the state by.
+template <int WT, bool VAR>
 __global__ __launch_bounds__(256) void retention_states_kernel(
     const float* __restrict__ xbc, long xbc_stride, const int* __restrict__ q_start, const int* __restrict__ q_len,
-    const int* __restrict__ chunk_seg, const int* __restrict__ chunk_idx, float* __restrict__ carry, int heads, int vdim, int N,
-    const float* __restrict__ fixed_a, float step, int silu_in) {
+    const int* __restrict__ chunk_seg, const int* __restrict__ chunk_idx, float* __restrict__ carry, int heads, int groups, int vdim, int N,
+    RetDecay dc, float* __restrict__ chunk_decay, int silu_in) {
     constexpr int B = 64 * WT;
     extern __shared__ __align__(16) float lds[];
     float* sK = lds;                                   // [RET_Q][B]
     float* sV = lds + RET_Q * B;                       // [RET_Q][B], times a^(n-1-j) f
+    __shared__ double cum[VAR ? RET_Q : 1];
+    __shared__ float dts[VAR ? RET_Q : 1];
     const int bx = blockIdx.x, seg = chunk_seg[bx];
     if (seg < 0) return;
     const int first = chunk_idx[bx] * RET_Q, L = q_len[seg];
     const int ntok = L - first < RET_Q ? L - first : RET_Q, t0 = q_start[seg] + first, head = blockIdx.y;
     const int vb = (vdim + B - 1) / B, n0 = (blockIdx.z / vb) * B, p0 = (blockIdx.z % vb) * B;
-    const float a = fixed_a[head];
-    const int inner = heads * vdim;
+    const int inner = heads * vdim, group = head / (heads / groups);
+    if constexpr (VAR) {
+        ret_chunk_decays(dc, t0, ntok, head, cum, dts);
+        __syncthreads();
+        if (blockIdx.z == 0 && threadIdx.x == 0) chunk_decay[(size_t)bx * heads + head] = expf((float)cum[RET_Q - 1]);
+    }
     const int rows = (ntok + 1) & ~1;                  // (whole pairs of tokens: the row behind an odd last one is zero)
     for (int i = threadIdx.x; i < rows * (B / 4); i += 256) {
         const int j = i / (B / 4), c = 4 * (i % (B / 4));
         const float* row = xbc + (size_t)(t0 + j) * xbc_stride;
         float4 k = float4{0.f, 0.f, 0.f, 0.f}, v = k;
-        if (j < ntok && n0 + c < N) k = silu_if4(*reinterpret_cast<const float4*>(row + inner + (size_t)head * N + n0 + c), silu_in);
+        if (j < ntok && n0 + c < N) k = silu_if4(*reinterpret_cast<const float4*>(row + inner + (size_t)group * N + n0 + c), silu_in);
         if (j < ntok && p0 + c < vdim) {
             v = silu_if4(*reinterpret_cast<const float4*>(row + (size_t)head * vdim + p0 + c), silu_in);
-            const float f = powf(a, (float)(ntok - 1 - j)) * step;
+            float f;
+            if constexpr (VAR) f = expf((float)(cum[RET_Q - 1] - cum[j])) * dts[j];
+            else f = powf(dc.fixed_a[head], (float)(ntok - 1 - j)) * dc.step;
             v = float4{v.x * f, v.y * f, v.z * f, v.w * f};
         }
         *reinterpret_cast<float4*>(sK + j * B + c) = k;
@@ -546,76 +586,89 @@ __global__ __launch_bounds__(256) void retention_states_kernel(
 // carry[chunk]: in: what the chunk alone adds; out: the state with which it begins.  The next eight chunks' values are on
 // their way while a chunk is worked on.  NV4: a head's state in 16-byte pieces.
 #define RET_AHEAD 8
+template <bool VAR>
 __global__ __launch_bounds__(64) void retention_carry_kernel(float4* __restrict__ carry, float4* __restrict__ state,
                                                              const int* __restrict__ slots, const int* __restrict__ q_len,
                                                              const int* __restrict__ chunk_first, int heads, int NV4,
-                                                             const float* __restrict__ fixed_a) {
+                                                             const float* __restrict__ fixed_a, const float* __restrict__ chunk_decay) {
     const int seg = blockIdx.x, head = blockIdx.y, e = blockIdx.z * 64 + threadIdx.x;
     if (e >= NV4) return;
     const int L = q_len[seg], nch = (L + RET_Q - 1) / RET_Q;
-    const float a = fixed_a[head], whole = powf(a, (float)RET_Q), tail = powf(a, (float)(L - (nch - 1) * RET_Q));
+    const float a = VAR ? 1.f : fixed_a[head], whole = VAR ? 1.f : powf(a, (float)RET_Q), tail = VAR ? 1.f : powf(a, (float)(L - (nch - 1) * RET_Q));
+    const float* factors = VAR ? chunk_decay + (size_t)chunk_first[seg] * heads + head : nullptr;
     float4* at = carry + ((size_t)chunk_first[seg] * heads + head) * NV4 + e;
     const size_t next = (size_t)heads * NV4;
     float4* st = state + ((size_t)slots[seg] * heads + head) * NV4 + e;
     float4 run = *st, own[RET_AHEAD];
+    float fown[RET_AHEAD];
 #pragma unroll
-    for (int u = 0; u < RET_AHEAD; ++u) own[u] = at[(size_t)(u < nch ? u : nch - 1) * next];
+    for (int u = 0; u < RET_AHEAD; ++u) {
+        own[u] = at[(size_t)(u < nch ? u : nch - 1) * next];
+        if constexpr (VAR) fown[u] = factors[(size_t)(u < nch ? u : nch - 1) * heads];
+    }
     for (int c0 = 0; c0 < nch; c0 += RET_AHEAD) {
         float4 ahead[RET_AHEAD];
+        float fahead[RET_AHEAD];
 #pragma unroll
         for (int u = 0; u < RET_AHEAD; ++u) {
             const int c = c0 + RET_AHEAD + u;
             ahead[u] = at[(size_t)(c < nch ? c : nch - 1) * next];      // (past the end: the last chunk's again, not used)
+            if constexpr (VAR) fahead[u] = factors[(size_t)(c < nch ? c : nch - 1) * heads];
         }
 #pragma unroll
         for (int u = 0; u < RET_AHEAD; ++u) {
             const int c = c0 + u;
             if (c < nch) {
-                const float f = c + 1 < nch ? whole : tail;
+                const float f = VAR ? fown[u] : c + 1 < nch ? whole : tail;
                 at[(size_t)c * next] = run;
                 run = float4{fmaf(f, run.x, own[u].x), fmaf(f, run.y, own[u].y), fmaf(f, run.z, own[u].z), fmaf(f, run.w, own[u].w)};
             }
         }
 #pragma unroll
-        for (int u = 0; u < RET_AHEAD; ++u) own[u] = ahead[u];
+        for (int u = 0; u < RET_AHEAD; ++u) {
+            own[u] = ahead[u];
+            if constexpr (VAR) fown[u] = fahead[u];
+        }
     }
     *st = run;
 }
 
 // NQ: 8-value pieces of a query (N <= 8 NQ); PT: fragments of 32 columns a wave.  The four waves are two query tiles of 32 by two
 // column ranges; a query lies in registers (16-byte pieces 2 t + l / 32 of row l % 32), keys and values in LDS.
-template <int NQ, int PT>
-__global__ __launch_bounds__(256) void retention_outputs_kernel(
+template <int NQ, int PT, bool VAR>
+__global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void retention_outputs_kernel(
     const float* __restrict__ xbc, long xbc_stride, const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ chunk_seg, const int* __restrict__ chunk_idx, const float* __restrict__ carry, float* __restrict__ y,
-    long y_stride, int heads, int vdim, int N, const float* __restrict__ fixed_a, float step, int silu_in) {
+    long y_stride, int heads, int groups, int vdim, int N, RetDecay dc, const float* __restrict__ Dw, int silu_in) {
     constexpr int NP = 8 * NQ, KS = NP + 4, VB = 64 * PT;
     extern __shared__ __align__(16) float lds[];
     float* sK = lds;                                   // [RET_Q][KS]: four floats of padding spread the 16-byte reads over the banks
     float* sV = sK + RET_Q * KS;                       // [RET_Q][VB]
-    float* pw = sV + RET_Q * VB;                       // [RET_Q + 1]: the powers of the decay
+    float* pw = sV + RET_Q * VB;                       // [RET_Q + 1]: the powers of the decay (VAR: the tokens' steps)
+    __shared__ double cum[VAR ? RET_Q : 1];
     const int bx = blockIdx.x, seg = chunk_seg[bx];
     if (seg < 0) return;
     const int first = chunk_idx[bx] * RET_Q, L = q_len[seg];
     const int ntok = L - first < RET_Q ? L - first : RET_Q, t0 = q_start[seg] + first, head = blockIdx.y, p0 = blockIdx.z * VB;
-    const int inner = heads * vdim;
+    const int inner = heads * vdim, group = head / (heads / groups);
     const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, ql = lane & 31, h = lane >> 5;
     const int it = w >> 1, pc = p0 + (w & 1) * 32 * PT, i = it * 32 + ql;
     // the wave's queries, asked for before keys and values are staged
     float4 q[NQ];
     {
-        const float* row = xbc + (size_t)(t0 + (i < ntok ? i : ntok - 1)) * xbc_stride + inner + (size_t)(heads + head) * N;
+        const float* row = xbc + (size_t)(t0 + (i < ntok ? i : ntok - 1)) * xbc_stride + inner + (size_t)(groups + group) * N;
 #pragma unroll
         for (int t = 0; t < NQ; ++t) {
             const int n = 8 * t + 4 * h;
             q[t] = n < N ? *reinterpret_cast<const float4*>(row + n) : float4{0.f, 0.f, 0.f, 0.f};
         }
     }
-    if (threadIdx.x <= RET_Q) pw[threadIdx.x] = powf(fixed_a[head], (float)threadIdx.x);
+    if constexpr (VAR) ret_chunk_decays(dc, t0, ntok, head, cum, pw);
+    else if (threadIdx.x <= RET_Q) pw[threadIdx.x] = powf(dc.fixed_a[head], (float)threadIdx.x);
     for (int x = threadIdx.x; x < RET_Q * (NP / 4); x += 256) {
         const int j = x / (NP / 4), c = 4 * (x % (NP / 4));
         float4 k = float4{0.f, 0.f, 0.f, 0.f};
-        if (j < ntok && c < N) k = silu_if4(*reinterpret_cast<const float4*>(xbc + (size_t)(t0 + j) * xbc_stride + inner + (size_t)head * N + c), silu_in);
+        if (j < ntok && c < N) k = silu_if4(*reinterpret_cast<const float4*>(xbc + (size_t)(t0 + j) * xbc_stride + inner + (size_t)group * N + c), silu_in);
         *reinterpret_cast<float4*>(sK + j * KS + c) = k;
     }
     for (int x = threadIdx.x; x < RET_Q * (VB / 4); x += 256) {
@@ -628,42 +681,66 @@ __global__ __launch_bounds__(256) void retention_outputs_kernel(
     for (int t = 0; t < NQ; ++t) q[t] = silu_if4(q[t], silu_in);        // (silu(0) = 0)
     __syncthreads();
     if (it * 32 >= ntok || pc >= vdim) return;
-    ret_f32x16 out[PT];
+    [[maybe_unused]] const double ci = VAR ? cum[i] : 0.0;
+    // VAR: a sum of sixty-four steps of the matrix cores is taken as four (of the products with V: two) side by side, which
+    // halves what it loses to rounding: with one, y was 2.4e-7 off the float64 result where the recurrence token by token is
+    // 8.2e-8 off, with these 8.1e-8
+    constexpr int CH = VAR ? 4 : 1, CV = VAR ? 2 : 1;
+    ret_f32x16 out[PT][CV];
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) out[pt][r] = 0.f;
-    for (int jt = 0; jt <= it; ++jt) {
-        ret_f32x16 sc;                                 // keys as rows, the wave's queries as columns
+        for (int v = 0; v < CV; ++v)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) sc[r] = 0.f;
+            for (int r = 0; r < 16; ++r) out[pt][v][r] = 0.f;
+    for (int jt = 0; jt <= it; ++jt) {
+        ret_f32x16 part[CH];                           // keys as rows, the wave's queries as columns
+#pragma unroll
+        for (int e = 0; e < CH; ++e)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) part[e][r] = 0.f;
         const float* krow = sK + (jt * 32 + ql) * KS + 4 * h;
 #pragma unroll
         for (int t = 0; t < NQ; ++t) {
             const float4 k = *reinterpret_cast<const float4*>(krow + 8 * t);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k.x, q[t].x, sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k.y, q[t].y, sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k.z, q[t].z, sc, 0, 0, 0);
-            sc = __builtin_amdgcn_mfma_f32_32x32x2f32(k.w, q[t].w, sc, 0, 0, 0);
+            part[0 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.x, q[t].x, part[0 % CH], 0, 0, 0);
+            part[1 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.y, q[t].y, part[1 % CH], 0, 0, 0);
+            part[2 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.z, q[t].z, part[2 % CH], 0, 0, 0);
+            part[3 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.w, q[t].w, part[3 % CH], 0, 0, 0);
+        }
+        ret_f32x16 sc = part[0];
+        if constexpr (VAR) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sc[r] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const int d = i - (jt * 32 + 8 * (r >> 2) + 4 * h + (r & 3));
-            sc[r] = d >= 0 ? sc[r] * (pw[d >= 0 ? d : 0] * step) : 0.f;
+            const int j = jt * 32 + 8 * (r >> 2) + 4 * h + (r & 3), d = i - j;
+            if constexpr (VAR) sc[r] = d >= 0 ? sc[r] * (expf((float)(ci - cum[j])) * pw[j]) : 0.f;
+            else sc[r] = d >= 0 ? sc[r] * (pw[d >= 0 ? d : 0] * dc.step) : 0.f;
         }
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const float* vrow = sV + (jt * 32 + 8 * (r >> 2) + 4 * h + (r & 3)) * VB + (pc - p0) + ql;
 #pragma unroll
-            for (int pt = 0; pt < PT; ++pt) out[pt] = __builtin_amdgcn_mfma_f32_32x32x2f32(sc[r], vrow[32 * pt], out[pt], 0, 0, 0);
+            for (int pt = 0; pt < PT; ++pt) out[pt][r % CV] = __builtin_amdgcn_mfma_f32_32x32x2f32(sc[r], vrow[32 * pt], out[pt][r % CV], 0, 0, 0);
         }
     }
     // what the state at the chunk's beginning adds
     const float* S = carry + ((size_t)bx * heads + head) * N * vdim;
-    const float f = pw[i + 1];
+    [[maybe_unused]] const float f = VAR ? 1.f : pw[i + 1];              // (VAR: the factors go on the sums)
     int col[PT];
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt) col[pt] = pc + 32 * pt + ql < vdim ? pc + 32 * pt + ql : vdim - 1;     // (a column past the last is not written)
+    ret_f32x16 more[VAR ? PT : 1][VAR ? CH : 1];
+    if constexpr (VAR) {
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt)
+#pragma unroll
+            for (int e = 0; e < CH; ++e)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) more[pt][e][r] = 0.f;
+    }
 #pragma unroll
     for (int t = 0; t < NQ; ++t) {
         const float qs[4] = {q[t].x * f, q[t].y * f, q[t].z * f, q[t].w * f};
@@ -678,52 +755,64 @@ __global__ __launch_bounds__(256) void retention_outputs_kernel(
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
-            for (int pt = 0; pt < PT; ++pt) out[pt] = __builtin_amdgcn_mfma_f32_32x32x2f32(qs[e], sv[e][pt], out[pt], 0, 0, 0);
+            for (int pt = 0; pt < PT; ++pt) {
+                if constexpr (VAR) more[pt][e] = __builtin_amdgcn_mfma_f32_32x32x2f32(qs[e], sv[e][pt], more[pt][e], 0, 0, 0);
+                else out[pt][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(qs[e], sv[e][pt], out[pt][0], 0, 0, 0);
+            }
     }
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = it * 32 + 8 * (r >> 2) + 4 * h + (r & 3), p = pc + 32 * pt + ql;
-            if (row < ntok && p < vdim) y[(size_t)(t0 + row) * y_stride + (size_t)head * vdim + p] = out[pt][r];
+            if (row < ntok && p < vdim) {
+                float v = out[pt][0][r];
+                if constexpr (VAR) {
+                    v = fmaf(expf((float)cum[row]), (more[pt][0][r] + more[pt][1][r]) + (more[pt][2][r] + more[pt][3][r]), out[pt][0][r] + out[pt][1][r]);
+                    if (Dw) v = fmaf(Dw[head], sV[row * VB + p - p0], v);
+                }
+                y[(size_t)(t0 + row) * y_stride + (size_t)head * vdim + p] = v;
+            }
         }
 }
 
-template <int NQ, int PT>
+template <int NQ, int PT, bool VAR>
 static int retention_outputs_launch(const dim3& grid, const float* xbc, long xbc_stride, const int* q_start, const int* q_len,
                                     const int* chunk_seg, const int* chunk_idx, const float* carry, float* y, long y_stride,
-                                    int heads, int vdim, int N, const float* fixed_a, float step, int silu_in, hipStream_t stream) {
+                                    int heads, int groups, int vdim, int N, const RetDecay& dc, const float* Dw, int silu_in, hipStream_t stream) {
     constexpr int bytes = (RET_Q * (8 * NQ + 4) + RET_Q * 64 * PT + RET_Q + 4) * 4;
     static bool configured = false;
     if (!configured) {
-        if (hipFuncSetAttribute((const void*)retention_outputs_kernel<NQ, PT>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
+        if (hipFuncSetAttribute((const void*)retention_outputs_kernel<NQ, PT, VAR>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess)
             return LI_ERR_LAUNCH;
         configured = true;
     }
-    retention_outputs_kernel<NQ, PT><<<grid, 256, bytes, stream>>>(xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride,
-                                                                   heads, vdim, N, fixed_a, step, silu_in);
+    retention_outputs_kernel<NQ, PT, VAR><<<grid, 256, bytes, stream>>>(xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride,
+                                                                        heads, groups, vdim, N, dc, Dw, silu_in);
     return li_launch_status();
 }
 
-// The chunked form of a retention (every head with keys of its own); operands in 16-byte pieces, N and vdim multiples of four.
+// The chunked form of a retention (VAR: of the state-space recurrence); operands in 16-byte pieces, N and vdim multiples of four.
+template <bool VAR>
 static int retention_launch(const float* xbc, long xbc_stride, float* state, const int* slots, const int* q_start, const int* q_len,
-                            int* chunk_tab, float* carry, float* y, long y_stride, int heads, int vdim, int N, int segs, int max_chunks,
-                            const float* fixed_a, float step, int silu_in, hipStream_t stream) {
+                            int* chunk_tab, float* carry, float* chunk_decay, float* y, long y_stride, int heads, int groups, int vdim, int N,
+                            int segs, int max_chunks, const RetDecay& dc, const float* Dw, int silu_in, hipStream_t stream) {
     int* chunk_seg = chunk_tab;
     int* chunk_idx = chunk_tab + max_chunks;
     int* chunk_first = chunk_tab + 2 * max_chunks;
     ssm_chunk_index_kernel<<<1, 256, 0, stream>>>(q_len, segs, RET_Q, max_chunks, chunk_seg, chunk_idx, chunk_first);
-    const int wt = (N > 64 || vdim > 64) ? 2 : 1, b = 64 * wt;
+    // (where a head has at most 64 columns, wide blocks would leave two of their four waves without any)
+    const int wt = (VAR ? vdim > 64 : N > 64 || vdim > 64) ? 2 : 1, b = 64 * wt;
     const dim3 gs(max_chunks, heads, ((N + b - 1) / b) * ((vdim + b - 1) / b));
-    if (wt == 2) retention_states_kernel<2><<<gs, 256, 2 * RET_Q * 128 * 4, stream>>>(xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, heads, vdim, N, fixed_a, step, silu_in);
-    else retention_states_kernel<1><<<gs, 256, 2 * RET_Q * 64 * 4, stream>>>(xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, heads, vdim, N, fixed_a, step, silu_in);
+#define RET_STATES(WT_) retention_states_kernel<WT_, VAR><<<gs, 256, 2 * RET_Q * 64 * WT_ * 4, stream>>>(xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry,                                                                                                          heads, groups, vdim, N, dc, chunk_decay, silu_in)
+    if (wt == 2) RET_STATES(2); else RET_STATES(1);
+#undef RET_STATES
     const int NV4 = N * vdim / 4;
-    retention_carry_kernel<<<dim3(segs, heads, (NV4 + 63) / 64), 64, 0, stream>>>((float4*)carry, (float4*)state, slots, q_len, chunk_first, heads, NV4, fixed_a);
-    const int pt = vdim > 64 ? 2 : 1;
+    retention_carry_kernel<VAR><<<dim3(segs, heads, (NV4 + 63) / 64), 64, 0, stream>>>((float4*)carry, (float4*)state, slots, q_len, chunk_first, heads, NV4,
+                                                                                       dc.fixed_a, chunk_decay);
+    const int pt = !VAR && vdim > 64 ? 2 : 1;          // (VAR: the sums side by side leave no registers for a second fragment of columns)
     const dim3 go(max_chunks, heads, (vdim + 64 * pt - 1) / (64 * pt));
-#define RET_GO(NQ_)                                                                                                                  \
-    return pt == 2 ? retention_outputs_launch<NQ_, 2>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, heads, vdim, N, fixed_a, step, silu_in, stream) \
-                   : retention_outputs_launch<NQ_, 1>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, heads, vdim, N, fixed_a, step, silu_in, stream)
+#define RET_GO(NQ_)                                                                                                                      return pt == 2 ? retention_outputs_launch<NQ_, VAR ? 1 : 2, VAR>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, heads, groups, vdim, N, dc, Dw, silu_in, stream)                    : retention_outputs_launch<NQ_, 1, VAR>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, heads, groups, vdim, N, dc, Dw, silu_in, stream)
     if (N <= 32) RET_GO(4);
     if (N <= 64) RET_GO(8);
     if (N <= 128) RET_GO(16);
@@ -814,9 +903,15 @@ extern "C" int li_ssm_scan(const float* xbc, long xbc_stride, const float* dt_ra
         decay = carry + (size_t)max_chunks * heads * N * vdim;
     }
     const bool aligned = ((uintptr_t)state | (uintptr_t)y | (uintptr_t)carry) % 16 == 0 && y_stride % 4 == 0;
-    if (chunked && fixed_a && G == heads && !Dw && aligned && Q == RET_Q && N % 4 == 0 && vdim % 4 == 0 && xbc_stride % 4 == 0 && ((uintptr_t)xbc % 16) == 0)
-        return retention_launch(xbc, xbc_stride, state, slots, q_start, q_len, chunk_tab, carry, y, y_stride, heads, vdim, N, segs,
-                                max_chunks, fixed_a, fixed_dt, silu_in, stream);
+    if (chunked && aligned && Q == RET_Q && N % 4 == 0 && vdim % 4 == 0 && xbc_stride % 4 == 0 && ((uintptr_t)xbc % 16) == 0) {
+        const RetDecay dc{fixed_a, fixed_dt, dt_raw, dt_stride, dt_bias, A_log};
+        if (!fixed_a)
+            return retention_launch<true>(xbc, xbc_stride, state, slots, q_start, q_len, chunk_tab, carry, decay, y, y_stride, heads, G, vdim, N,
+                                          segs, max_chunks, dc, Dw, silu_in, stream);
+        if (G == heads && !Dw)
+            return retention_launch<false>(xbc, xbc_stride, state, slots, q_start, q_len, chunk_tab, carry, nullptr, y, y_stride, heads, G, vdim, N,
+                                           segs, max_chunks, dc, nullptr, silu_in, stream);
+    }
     int qs = 0, qr = 0;
     if (aligned && ssm_quad_layout(N, vdim, &qs, &qr)) {
         // heads that share no B and C have a block of four waves each: columns are spread over more lanes until all four work

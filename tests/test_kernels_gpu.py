@@ -1196,3 +1196,40 @@ def test_recurrences_of_a_decoding_step(ops, kind, n, heads, vdim, n_state, grou
     assert rel(y, want.reshape(n, -1).numpy()) < tol_
     assert rel(dev_state[torch.arange(n - 1, -1, -1)], new.numpy()) < tol_
     assert torch.equal(dev_state[n].cpu(), state[n])                       # a slot that is not in the batch
+
+
+@pytest.mark.parametrize("lens,heads,vdim,n_state,groups,skip_d", [
+    ([65], 6, 64, 128, 2, False),                # a chunk and one token
+    ([64, 1, 130, 7], 4, 20, 100, 4, False),     # one whole chunk, one token, a short last chunk, less than a chunk; values that fill no fragment
+    ([200, 190], 3, 68, 24, 1, True),            # columns over a second block; no term of x
+    ([96], 2, 8, 256, 2, False),
+    ([70], 4, 6, 30, 2, False),                  # not in 16-byte pieces: token by token in chunks
+])
+def test_state_space_recurrence_of_long_portions(ops, lens, heads, vdim, n_state, groups, skip_d):
+    """Against the equations in float64, within the random walk of a column's 2 n_state + 128 products."""
+    import types
+    g = torch.Generator().manual_seed(65)
+    R = lambda *s: torch.randn(*s, generator=g)
+    n, T, inner, rep = len(lens), sum(lens), heads * vdim, heads // groups
+    starts = np.concatenate([[0], np.cumsum(lens)[:-1]]).astype(np.int32)
+    dev = lambda a: torch.from_numpy(np.asarray(a, dtype=np.int32)).to(DEV)
+    slots = list(range(n))[::-1]
+    ctx = types.SimpleNamespace(num_tokens=T, num_segments=n, max_q_len=max(lens), host_state_slots=np.array(slots, dtype=np.int32),
+                                state_slots=dev(slots), q_start=dev(starts), q_len=dev(lens))
+    state, rows, dt = R(n, heads, n_state, vdim) * 0.3, R(T, inner + 2 * groups * n_state), R(T, heads)
+    bias, a_log, d = R(heads) - 3.0, 2.0 * torch.rand(heads, generator=g), None if skip_d else R(heads)
+    dev_state, y = state.to(DEV), torch.full((T, inner), float("nan"), device=DEV)
+    ops.ssm_scan(rows.to(DEV), dt.to(DEV), bias.to(DEV), a_log.to(DEV), None if skip_d else d.to(DEV), dev_state, ctx, y, heads, vdim,
+                 n_state, groups, _Lender())
+    step = torch.nn.functional.softplus(dt.double() + bias.double())
+    decay = torch.exp(-a_log.double().exp() * step)
+    tol_ = 8 * math.sqrt(2 * n_state + 128) * 2.0 ** -24
+    for i, (o, L) in enumerate(zip(starts, lens)):
+        S, out = state[slots[i]].double(), []
+        for t in range(o, o + L):
+            x, b, c = rows[t].double().split([inner, groups * n_state, groups * n_state])
+            x, b, c = x.view(heads, vdim), b.view(groups, n_state).repeat_interleave(rep, 0), c.view(groups, n_state).repeat_interleave(rep, 0)
+            S = decay[t][:, None, None] * S + (step[t][:, None] * b)[:, :, None] * x[:, None]
+            out.append((S * c[:, :, None]).sum(1) + (0.0 if skip_d else d.double()[:, None] * x))
+        assert rel(y[o:o + L], torch.stack(out).reshape(L, -1).numpy()) < tol_, i
+        assert rel(dev_state[slots[i]], S.numpy()) < tol_, i
