@@ -1034,6 +1034,32 @@ def test_sample_rows_with_many_equal_logits_at_the_thresholds(ops, vocab):
     assert same >= n - 2
 
 
+@pytest.mark.parametrize("order", ["mixed", "ascending", "few", "one_value"])
+def test_sample_rows_with_the_candidates_found_by_a_bound(ops, order):
+    # ids above a bound are held against each other (mixed: some more than the wanted ones lie above it); where one wave
+    # holds all large ids (ascending), most ids are -inf (few) or all are equal, too many lie above it and the search goes
+    # through the digits
+    g = torch.Generator().manual_seed(66)
+    vocab, top_k = 8192 + 4097, [1, 15, 16, 17, 50, 128, 255, 256]
+    n = len(top_k)
+    logits = torch.randn(n, vocab, generator=g) * 3
+    if order == "ascending":
+        logits = logits.sort(dim=1).values
+    elif order == "few":
+        logits[:, torch.randperm(vocab, generator=g)[:vocab - 40]] = float("-inf")
+    elif order == "one_value":
+        logits[:] = 1.5
+        logits[:, 9000:9003] = torch.tensor([2.0, 1.75, 2.0])
+    rows = logits.double().numpy()
+    for top_p in (1.0, 0.9):
+        for temperature in (0.7, 1.0):
+            u = torch.rand(n, generator=g).tolist()
+            picks = _sample(ops, logits, [temperature] * n, top_k, [top_p] * n, u)
+            for r in range(n):
+                assert np.isfinite(rows[r][picks[r]]), (r, top_k[r])
+                assert _pick_is_right(rows[r], temperature, top_k[r], top_p, u[r], picks[r]), (r, top_k[r])
+
+
 def test_sample_rows_frequencies_and_ties(ops):
     lg = torch.tensor([[2.0, 1.0, 3.0, 3.0, -1.0, 0.5, 2.5, 0.0]])
     n = 4000
