@@ -39,6 +39,27 @@ __device__ __forceinline__ void store_from_float(bf16_t* p, float v) { p->bits =
 
 // GELU with the error function
 __device__ __forceinline__ float gelu_erf(float z) { return 0.5f * z * (1.0f + erff(z * 0.70710678118654752f)); }
+// ... and in its tanh form
+__device__ __forceinline__ float gelu_tanh(float z) {
+    return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
+}
+// xIELU with two numbers worked out by the caller, sp = softplus(p) and sq = 1/2 + softplus(q):
+// z > 0: sp z^2 + z / 2;  z <= 0: sq (exp(z) - 1 - z) + z / 2
+__device__ __forceinline__ float xielu(float z, float sp, float sq) {
+    return (z > 0.f ? sp * z * z : sq * (expm1f(z) - z)) + 0.5f * z;
+}
+// What a product may leave instead of its sums (li_linear_act): 1 max(z, 0)^2, 2 and 3 GELU in its tanh form and with the
+// error function, 4 xIELU with the numbers a0 and a1
+#define LI_ACT_RELU2 1
+#define LI_ACT_GELU_TANH 2
+#define LI_ACT_GELU_ERF 3
+#define LI_ACT_XIELU 4
+__device__ __forceinline__ float activation(float z, int act, float a0, float a1) {
+    if (act == LI_ACT_RELU2) { const float r = fmaxf(z, 0.f); return r * r; }
+    if (act == LI_ACT_GELU_TANH) return gelu_tanh(z);
+    if (act == LI_ACT_GELU_ERF) return gelu_erf(z);
+    return xielu(z, a0, a1);
+}
 
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

@@ -525,10 +525,6 @@ extern "C" int li_relu_squared(const void* x, int x_dtype, void* out, int out_dt
     return li_launch_status();
 }
 
-__device__ __forceinline__ float gelu_tanh(float z) {
-    return 0.5f * z * (1.0f + tanhf(0.7978845608028654f * (z + 0.044715f * z * z * z)));
-}
-
 // out[t, j] = gelu_tanh(a[t, j]) * table[id(t), off + j], j < n; table rows have `row` elements
 template <typename TT, typename TO>
 __global__ void gelu_gate_rows_kernel(const float* __restrict__ a, const int* __restrict__ ids, const int* __restrict__ id_src,
@@ -1337,11 +1333,6 @@ extern "C" int li_stream_sum(const float* x, const int* rows, float* out, int nu
     return li_launch_status();
 }
 
-// xIELU with two numbers worked out by the caller, sp = softplus(p) and sq = 1/2 + softplus(q):
-// z > 0: sp z^2 + z / 2;  z <= 0: sq (exp(z) - 1 - z) + z / 2
-__device__ __forceinline__ float xielu(float z, float sp, float sq) {
-    return (z > 0.f ? sp * z * z : sq * (expm1f(z) - z)) + 0.5f * z;
-}
 template <typename TI, typename TO>
 __global__ void xielu_kernel(const TI* __restrict__ x, TO* __restrict__ out, long n, float sp, float sq) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;

@@ -414,6 +414,8 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
                 v = fminf(v, limit);
                 up = fminf(fmaxf(up, -limit), limit);
                 out[(size_t)row * N + n0 + j] = (up + 1.0f) * (v / (1.0f + expf(-1.702f * v)));
+            } else if (limit < 0.f) {
+                out[(size_t)row * N + n0 + j] = up * gelu_tanh(v);
             } else {
                 out[(size_t)row * N + n0 + j] = up * (v / (1.0f + expf(-v)));
             }
@@ -820,10 +822,12 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
     return up * (gate * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
-// CLAMP: the clamped form, g = min(gate, limit), u = clamp(up, -limit, limit), g sigmoid(1.702 g) (u + 1).
+// CLAMP: the other forms: limit > 0: g = min(gate, limit), u = clamp(up, -limit, limit), g sigmoid(1.702 g) (u + 1);
+// limit < 0: the gate through GELU in its tanh form.
 template <bool CLAMP>
 __device__ __forceinline__ float gated_bf16(float gate, float up, float limit) {
     if constexpr (!CLAMP) return swiglu_bf16(gate, up);
+    if (limit < 0.f) return up * gelu_tanh(gate);
     const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
     const float e = __builtin_amdgcn_exp2f(-1.702f * 1.44269504088896341f * g);
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + e));
@@ -1174,6 +1178,21 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = src[e];
             const size_t o_idx = (size_t)row * NO + col;
+            if constexpr (CLAMP && !SWIGLU) {            // an activation of the sums (its number and its two constants where a norm's factors have theirs)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), nparts, eps, limit);
+                if (col + 8 <= NO && (NO % 8) == 0) {
+                    chunk16 o;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o.w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
+                    *reinterpret_cast<chunk16*>(reinterpret_cast<uint16_t*>(out) + o_idx) = o;
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (col + e < NO) epilogue_store(out, o_idx + e, v[e], nullptr, col + e, 0);
+                }
+                continue;
+            }
             if (col + 8 <= NO && (NO % 8) == 0) {
                 if (bias) {
 #pragma unroll
@@ -1238,6 +1257,21 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit,
     float v = part[i];
     for (int s = 1; s < nsplit; ++s) v += part[(size_t)s * mn + i];
     epilogue_store(out, i, v, bias, (int)(i % N), accumulate);
+}
+
+// out = act(sum over the parts + bias), bfloat16 (see li_linear_act)
+__global__ __launch_bounds__(256) void splitk_reduce_act_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
+                                                                const float* __restrict__ bias, bf16_t* __restrict__ out, int act, float a0, float a1) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= mn) return;
+    float a[8];
+#pragma unroll
+    for (int sp = 0; sp < 8; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + i];      // (all loads at once)
+    float v = a[0];
+#pragma unroll
+    for (int sp = 1; sp < 8; ++sp) v += sp < nsplit ? a[sp] : 0.f;
+    if (bias) v += bias[(int)(i % N)];
+    store_from_float(out + i, activation(v, act, a0, a1));
 }
 
 // The same for the residual sum, one block a row, with the RMS norm of the new sum as a second
@@ -1386,12 +1420,16 @@ struct SkinnyArgs {
     // no statistics of a row, so it is done here and sq_parts stays as it is.
     const float* beta;
     float alpha;
-    // SWIGLU with limit > 0: g = min(gate, limit), u = clamp(up, -limit, limit), out = g sigmoid(1.702 g) (u + 1)
+    // SWIGLU with EPI 1: the other gated forms (see gated_bf16)
     float limit;
+    // EPI 2 (bfloat16 out): out = activation(product + bias, act, a0, a1)
+    int act;
+    float a0, a1;
 };
 #define SK_MAX_PARTS 512            // blocks of a producing product whose sums one consumer adds up
 
-// EPI 1: with SWIGLU the clamped activation, else (float out) the tanh norm of the new sum beside it (SkinnyArgs: beta).
+// EPI 1: with SWIGLU the other gated activations, else (float out) the tanh norm of the new sum beside it (SkinnyArgs: beta).
+// EPI 2: an activation of the sums (SkinnyArgs: act).
 template <int MT, int NT, int WAVES, bool SWIGLU, typename TO, bool ROPE = false, int EPI = 0>
 __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs a) {
     static_assert(!ROPE || (MT <= 2 && !SWIGLU), "the rotary epilogue takes one or two tiles of rows");
@@ -1446,7 +1484,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
     // weights, the rotation's cosines and sines, the page slot) is asked for now, by the wave
     // that will write the results: the answers arrive with the first chunk, and the epilogue
     // waits for no memory.  Never conditional per lane: a place past the end reads the last one.
-    constexpr bool PRE = MT <= 2 && !SWIGLU;        // (wave mt writes row tile mt: thread t of the epilogue is lane t % 64 of wave t / 64)
+    constexpr bool PRE = MT <= 2 && !SWIGLU && EPI != 2;        // (wave mt writes row tile mt: thread t of the epilogue is lane t % 64 of wave t / 64)
     float pre_bias[NT][4], pre_res[NT][4], pre_gamma[NT][4], pre_beta[NT][4], pre_cos[NT][4], pre_sin[NT][4];
     int pre_slot = 0;
     if constexpr (PRE) {
@@ -1612,6 +1650,21 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
         for (int nt = 0; nt < NT; ++nt) red[wave][mt * NT + nt][lane] = acc[mt][nt];
     __syncthreads();
     TO* out = (TO*)a.out;
+    if constexpr (EPI == 2 && !SWIGLU) {
+        // one value a thread at a time, by all waves: an activation is tens of instructions a value, and by the one wave that
+        // writes a row tile elsewhere its values would go through them one after the other
+        for (int v = threadIdx.x; v < MT * NT * 256; v += WAVES * 64) {
+            const int tile = v >> 8, l = (v >> 2) & 63, r = v & 3;
+            const int m = 16 * (tile / NT) + (l & 15), n = n0 + 16 * (tile % NT) + 4 * (l >> 4) + r;
+            if (m >= M || n >= nend) continue;
+            float s = red[0][tile][l][r];
+#pragma unroll
+            for (int wv = 1; wv < WAVES; ++wv) s += red[wv][tile][l][r];
+            if (a.bias) s += a.bias[n];
+            store_from_float(out + (size_t)m * N + n, activation(s, a.act, a.a0, a.a1));
+        }
+        return;
+    }
     for (int t = threadIdx.x; t < MT * 64; t += WAVES * 64) {
         const int mt = t >> 6, l = t & 63;
         const int m = 16 * mt + (l & 15);
@@ -1959,6 +2012,21 @@ static double tile_cost(int bm, int bn, double speed, int M, int N, int K) {
     return rounds * ((K / 64) * (mfma_us > load_us ? mfma_us : load_us) + 2.0);
 }
 
+// Seven tilings for more than 64 rows; the one with the least estimated time is taken (tile_cost).  The two with four
+// waves one above the other take any multiple of 32 columns: 224 or 288 columns cut 3,584 or 4,608 into exactly as many
+// tiles as 2,048 rows need to give every compute unit one.
+static int tiling_of(int M, int N, int K) {
+    static const struct { int bm, bn; double speed; } shape[7] = {{256, 256, 1.0}, {256, 192, 0.95}, {256, 128, 1.0}, {192, 128, 0.95},
+                                                                    {128, 128, 0.8}, {128, 224, 0.9}, {128, 288, 0.9}};
+    int pick = 0;
+    double best = 0.0;
+    for (int i = 0; i < 7; ++i) {
+        const double c = tile_cost(shape[i].bm, shape[i].bn, shape[i].speed, M, N, K);
+        if (i == 0 || c < best) { best = c; pick = i; }
+    }
+    return pick;
+}
+
 // More than 64 rows but so few 128 x 128 tiles that half of the compute units would idle (a narrow
 // matrix with a long K, like the feed-forward's way back at 128 to 512 rows): K is cut into parts
 // here too.  Returns the number of parts, 1 for none.
@@ -2158,17 +2226,7 @@ extern "C" int li_linear(const void* x, const void* w, const float* bias, void* 
                 }
 #define LI_DMA4(BM, BN, BK, NS) (out_dtype == LI_F32 ? launch_dma<BM, BN, BK, NS, false, float, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (float*)out, M, N, K, accumulate, stream) \
                                                 : launch_dma<BM, BN, BK, NS, false, bf16_t, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, accumulate, stream))
-                // Seven tilings; the one with the least estimated time is taken (tile_cost).  The two with four
-                // waves one above the other take any multiple of 32 columns: 224 or 288 columns cut 3,584 or
-                // 4,608 into exactly as many tiles as 2,048 rows need to give every compute unit one.
-                static const struct { int bm, bn; double speed; } shape[7] = {{256, 256, 1.0}, {256, 192, 0.95}, {256, 128, 1.0}, {192, 128, 0.95},
-                                                                                {128, 128, 0.8}, {128, 224, 0.9}, {128, 288, 0.9}};
-                int pick = 0;
-                double best = 0.0;
-                for (int i = 0; i < 7; ++i) {
-                    const double c = tile_cost(shape[i].bm, shape[i].bn, shape[i].speed, M, N, K);
-                    if (i == 0 || c < best) { best = c; pick = i; }
-                }
+                const int pick = tiling_of(M, N, K);
                 switch (pick) {
                 case 0: return LI_DMA(256, 256, 64, 2);
                 case 1: return LI_DMA(256, 192, 64, 2);
@@ -2193,6 +2251,56 @@ extern "C" int li_linear(const void* x, const void* w, const float* bias, void* 
     return li_launch_status();
 }
 
+// out = act(x w^T + bias), bfloat16 throughout, the sums float32 until the activation has been taken: in the epilogue of
+// the kernel that li_linear would take for these sizes, or of the one that adds its parts up.  Without it the sums go to
+// memory in float32 and a kernel of their own reads them again: at a few rows that kernel costs its launch, 5 us a layer,
+// and at 2,048 rows of 8,960 columns the reads and writes of 73 MB (squared ReLU: 15 to 29 us).  Above 64 rows the
+// squared ReLU only: the others are tens of instructions a value, which a tile's four waves take one after the other when
+// the matrix cores are done (xIELU, 2,601 rows of 8,960 columns: product and kernel 96 + 24 us, in the epilogue 183).
+// Returns -1, having done nothing, where it does not take the call.
+extern "C" int li_linear_act(const void* x, const void* w, const float* bias, void* out, int M, int N, int K, int act, float a0,
+                             float a1, void* work, long work_bytes, hipStream_t stream) {
+    if (M <= 0 || N <= 0 || K <= 0 || act < LI_ACT_RELU2 || act > LI_ACT_XIELU) return LI_ERR_SIZE;
+    if (K % 8 || (M > 64 && (K % 64 || act != LI_ACT_RELU2))) return -1;
+#define LI_ACT(BM, BN, NS, WLM) launch_dma<BM, BN, 64, NS, false, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, act, a0, a1)
+    if (M <= 64 && (K % 64 || !mid_rows_take(M, N, K))) {
+        SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, 0.f,
+                     nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
+        a.act = act;
+        a.a0 = a0;
+        a.a1 = a1;
+        launch_skinny<false, bf16_t, 2>(a, stream);
+        return li_launch_status();
+    }
+    const long need = li_linear_work_bytes(M, N, K, LI_BF16);
+    if (need > 0) {                                  // K in parts
+        const size_t mn = (size_t)M * N;
+        const int nsplit = (int)(need / (long)(mn * sizeof(float)));
+        if (!work || work_bytes < need || nsplit > 8) return -1;
+        const int rc = M <= 64
+            ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit)
+            : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
+        if (rc != LI_OK) return rc;
+        splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, act, a0, a1);
+        return li_launch_status();
+    }
+    if (M <= 64) {                                   // (as linear_mid_rows takes them)
+        if ((N + 255) / 256 >= 128) return LI_ACT(64, 256, 3, 2);
+        if ((N + 127) / 128 >= 128) return LI_ACT(64, 128, 4, 2);
+        return -1;
+    }
+    switch (tiling_of(M, N, K)) {
+    case 0: return LI_ACT(256, 256, 2, 2);
+    case 1: return LI_ACT(256, 192, 2, 2);
+    case 2: return LI_ACT(256, 128, 3, 2);
+    case 3: return LI_ACT(192, 128, 3, 2);
+    case 4: return LI_ACT(128, 128, 4, 2);
+    case 5: return LI_ACT(128, 224, 3, 4);
+    default: return LI_ACT(128, 288, 3, 4);
+    }
+#undef LI_ACT
+}
+
 // The same in float32 for up to 64 rows (K a multiple of 4): the few-row product on the float32 matrix cores with
 // the activation in its epilogue.
 extern "C" int li_linear_swiglu_f32(const float* x, const float* w, float* out, int M, int I, int K, float limit, hipStream_t stream) {
@@ -2203,7 +2311,7 @@ extern "C" int li_linear_swiglu_f32(const float* x, const float* w, float* out, 
 
 // out[m, n] = up * gate / (1 + exp(-gate)) with [gate, up] = x w^T, w = [gate; up] of I rows each:
 // the activation as the product's epilogue, so the 2 I columns never go to memory.  bfloat16;
-// K a multiple of 8 for up to 64 rows, a multiple of 64 above.  limit > 0: the clamped form (see gated_bf16).
+// K a multiple of 8 for up to 64 rows, a multiple of 64 above.  limit not zero: the other forms (see gated_bf16).
 // row_parts (may be null): x is the xg of li_linear_residual_norm and these are its sq_parts, nparts of
 // them; every row's result is that of the RMS norm with eps (up to 16 rows).
 extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, int I, int K,
@@ -2244,25 +2352,25 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
             const double c = tile_cost(64, widths[i], 1.0, M, N, K);
             if (pick < 0 || c < best) { best = c; pick = i; }
         }
-#define LI_SW64(BN, NS) (limit > 0.f ? launch_dma<64, BN, 64, NS, true, bf16_t, 2, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, limit) \
+#define LI_SW64(BN, NS) (limit != 0.f ? launch_dma<64, BN, 64, NS, true, bf16_t, 2, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, limit) \
                                      : launch_dma<64, BN, 64, NS, true, bf16_t>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps))
         if (pick == 0) return LI_SW64(256, 3);
         if (pick == 1) return LI_SW64(192, 4);
         if (pick == 2) return LI_SW64(128, 4);
 #undef LI_SW64
     }
-    if (row_parts || (M <= 64 && limit > 0.f)) {
+    if (row_parts || (M <= 64 && limit != 0.f)) {
         if (K % 8) return LI_ERR_SIZE;
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, nullptr, out, M, I, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, row_parts, nparts, eps};
         a.limit = limit;
-        if (limit > 0.f) launch_skinny<true, bf16_t, 1>(a, stream);
+        if (limit != 0.f) launch_skinny<true, bf16_t, 1>(a, stream);
         else launch_skinny<true, bf16_t>(a, stream);
         return li_launch_status();
     }
     if (M <= 64) return li_linear_skinny(x, w, nullptr, out, M, I, K, LI_BF16, 0, 1, stream);
     if (K % 64) return LI_ERR_SIZE;
-#define LI_DMA(BM, BN, BK, NS, WLM) (limit > 0.f ? launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, limit) \
+#define LI_DMA(BM, BN, BK, NS, WLM) (limit != 0.f ? launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, limit) \
                                                  : launch_dma<BM, BN, BK, NS, true, bf16_t, WLM>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream))
     // (a tile's columns are gate and up columns in turn, 32 of each: its width is a multiple of 64)
     // (128 x 320: 160 gate columns in one wave, their ups in the wave beside it; for portions of a few hundred rows,

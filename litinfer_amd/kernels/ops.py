@@ -89,6 +89,7 @@ _SIGNATURES = {
         "li_linear_residual_norm": [P, P, P, P, I, I, I, F, P, P, P],
         "li_linear_then_norm": [P, P, P, P, I, I, I, P, L, F, P, F, P, I],
         "li_linear_tanh_norm": [P, P, P, P, I, I, I, P, L, F, F, P, P, P, I],
+        "li_linear_act": [P, P, P, P, I, I, I, I, F, F, P, L],
         "li_linear_rope_store": [P, P, P, P, I, I, P, P, P, P, P, I, I, I, I, I, P, I, F],
         "li_linear_rope_store_parts": [P, P, P, P, I, I, P, P, P, P, P, I, I, I, I, I, P, L],
     },
@@ -1193,13 +1194,18 @@ def _check_row_scale(what: str, m: int, row_scale: Optional[RowScale]):
     return row_scale.sq_parts.data_ptr(), row_scale.nparts, row_scale.eps
 
 
+GELU_TANH_GATE = -1.0          # as `limit` of linear_swiglu: the gate through GELU in its tanh form
+
+
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, row_scale: Optional[RowScale] = None,
                   limit: float = 0.0) -> None:
     """out[m, n] = up * gate / (1 + exp(-gate)) with [gate, up] = x w^T, w = [gate; up]
     (2 N rows): the activation in the product's epilogue, from the product's float32 sums.
     With `row_scale`, x is the xg of `linear_residual_norm` and the result is that of the norm.  With `limit` > 0 the
-    clamped form: g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)."""
+    clamped form: g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit); with
+    GELU_TANH_GATE: up * gelu_tanh(gate)."""
     _gpu(x, w, out)
+    _chk(limit >= 0 or limit == GELU_TANH_GATE, "linear_swiglu: limit")
     _chk(x.dim() == 2 and w.dim() == 2 and out.dim() == 2, "linear_swiglu: needs matrices")
     m, k = x.shape
     n = out.shape[1]
@@ -1216,6 +1222,41 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, row_scale
     _chk(x.dtype is torch.bfloat16 and out.dtype is torch.bfloat16, "linear_swiglu: x and out must be bfloat16")
     _run("gemm", "li_linear_swiglu", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k,
          *_check_row_scale("linear_swiglu", m, row_scale), float(limit))
+
+
+LINEAR_ACTS = {"relu2": 1, "gelu_tanh": 2, "gelu": 3, "xielu": 4}      # the kernels' numbers (gelu: with the error function)
+
+
+def linear_act(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, act: str,
+               constants=(0.0, 0.0), ws=None) -> bool:
+    """out = act(x w^T + bias) with the activation taken of the product's float32 sums, bfloat16 operands and out; act:
+    "relu2" max(., 0)^2, "gelu_tanh", "gelu" (error function), "xielu" with two constants (see `xielu`).  False, with
+    nothing done, where the product has no such epilogue (the caller then multiplies and activates in two calls)."""
+    _gpu(x, w, bias, out)
+    _chk(x.dim() == 2 and w.dim() == 2 and out.dim() == 2 and act in LINEAR_ACTS, "linear_act: matrices, act")
+    m, k = x.shape
+    n = w.shape[0]
+    _chk(w.shape[1] == k and out.shape == (m, n), "linear_act: shapes do not fit")
+    _chk(x.is_contiguous() and w.is_contiguous() and out.is_contiguous(), "linear_act: contiguous operands")
+    _chk(bias is None or (bias.dtype is torch.float32 and bias.numel() == n and bias.is_contiguous()), "linear_act: bias must be float32 [N]")
+    if not (x.dtype is w.dtype is out.dtype is torch.bfloat16) or (x.data_ptr() | w.data_ptr() | out.data_ptr()) % 16:
+        return False
+    if not m:
+        return True
+    work, work_bytes = 0, 0
+    need = _work_bytes(m, n, k, _DT[x.dtype]) if ws is not None else 0
+    if need:
+        if m <= SKINNY_MAX_ROWS:                    # one size for all row counts of a decode batch: the buffer does not move
+            need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)
+        buf = ws.buffer("gemm.parts", (need // 4,), torch.float32)
+        work, work_bytes = buf.data_ptr(), buf.numel() * 4
+    rc = _fn("gemm", "li_linear_act")(x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(), m, n, k,
+                                      LINEAR_ACTS[act], float(constants[0]), float(constants[1]), work, work_bytes, _stream())
+    if rc == -1:
+        return False
+    if rc != 0:
+        raise RuntimeError(f"li_linear_act: the kernel library refused the call (code {rc}): {_ERRORS.get(rc, 'unknown')}")
+    return True
 
 
 ROPE_STORE_MAX_ROWS = 32

@@ -55,11 +55,18 @@ class Linear:
             return False
         return ops.linear_tanh_norm(x, self.weight, self.bias, out, tanh.alpha, tanh.weight, tanh.bias, xn, ws, factor=factor)
 
+    def with_activation(self, x: torch.Tensor, out: torch.Tensor, act: str, constants=(0.0, 0.0), ws=None) -> bool:
+        """out = act(x W^T + b) in one go, from the product's float32 sums, where the kernels have that (see
+        `ops.linear_act`); False, with nothing done, where not."""
+        if not (x.dtype is self.weight.dtype is out.dtype is torch.bfloat16):
+            return False
+        return ops.linear_act(x, self.weight, self.bias, out, act, constants, ws)
+
     def __call__(self, x: torch.Tensor, out: torch.Tensor, accumulate: bool = False, ws=None,
                  swiglu: bool = False, row_scale=None, factor: float = 1.0, limit: float = 0.0):
         """out = x W^T + b, or out += factor * (...) when `accumulate` (out is float32 then).
         With `swiglu` (only where `takes_swiglu`) W is [gate; up] and out gets
-        up * silu(gate), or with `limit` > 0 the clamped form of `ops.linear_swiglu`; `row_scale` then says that x came out of `add_with_scaling`.  A matrix that is stored in 32-bit is multiplied in
+        up * silu(gate), or with a `limit` that is not zero one of the other forms of `ops.linear_swiglu`; `row_scale` then says that x came out of `add_with_scaling`.  A matrix that is stored in 32-bit is multiplied in
         32-bit also when the activations are bfloat16: they are widened for it,
         exactly."""
         if swiglu:

@@ -27,7 +27,8 @@ class SwiGLUMLP(FeedForward):
             raise ValueError(f"gated feed-forward: activation {self.activation!r} (silu, gelu_tanh or clamped)")
         if (self.activation == "clamped") != (self.limit > 0):
             raise ValueError("gated feed-forward: the clamped activation takes a positive limit, the others none")
-        self.fused = self.activation in ("silu", "clamped")         # the activations that the products have as an epilogue
+        # which of the products' gated epilogues this is (0: silu)
+        self.gate_form = ops.GELU_TANH_GATE if self.activation == "gelu_tanh" else self.limit
         self.names = {"gate": "gate_proj.weight", "up": "up_proj.weight", "down": "down_proj.weight", **(spec.args.get("names") or {})}
         self.gate_up = None
         self.down = None
@@ -51,18 +52,18 @@ class SwiGLUMLP(FeedForward):
     def forward_prenorm(self, norm, residual, xn, ctx):
         # few rows (decoding): the product before the norm may have left its rows scaled by the
         # norm's weights; the gate/up product then applies the rows' factors with its activation
-        sc = residual.scaled_rows(norm) if self.fused else None
+        sc = residual.scaled_rows(norm)
         if sc is not None and self.gate_up.takes_swiglu(sc.rows):
             h = ctx.ws.buffer("mlp.h", (sc.rows.shape[0], self.inter), self.rt.dtype)
-            self.gate_up(sc.rows, h, ws=ctx.ws, swiglu=True, row_scale=sc.scale, limit=self.limit)
+            self.gate_up(sc.rows, h, ws=ctx.ws, swiglu=True, row_scale=sc.scale, limit=self.gate_form)
             return residual.add_linear(self.down, h)
         self.forward(residual.normed(norm, xn), residual, ctx)
 
     def forward(self, xn, residual, ctx):
         t = xn.shape[0]
         h = ctx.ws.buffer("mlp.h", (t, self.inter), self.rt.dtype)
-        if self.fused and self.gate_up.takes_swiglu(xn):
-            self.gate_up(xn, h, ws=ctx.ws, swiglu=True, limit=self.limit)        # few rows: the activation is the epilogue
+        if self.gate_up.takes_swiglu(xn):
+            self.gate_up(xn, h, ws=ctx.ws, swiglu=True, limit=self.gate_form)        # few rows: the activation is the epilogue
         else:
             if self.activation == "silu":
                 gu = ctx.ws.buffer("mlp.gate_up", (t, 2 * self.inter), self.rt.dtype)
@@ -106,11 +107,15 @@ class ReluSquaredMLP(FeedForward):
 
     def forward(self, xn, residual, ctx):
         t = xn.shape[0]
-        u = ctx.ws.buffer("mlp.up32", (t, self.inter), torch.float32)
-        self.up(xn, u, ws=ctx.ws)
         h = ctx.ws.buffer("mlp.h", (t, self.inter), self.rt.dtype)
-        self.activate(u, h)
+        if not self.up.with_activation(xn, h, *self.epilogue(), ws=ctx.ws):
+            u = ctx.ws.buffer("mlp.up32", (t, self.inter), torch.float32)
+            self.up(xn, u, ws=ctx.ws)
+            self.activate(u, h)
         residual.add_linear(self.down, h)
+
+    def epilogue(self):
+        return "relu2", (0.0, 0.0)
 
     def activate(self, u, h):
         ops.relu_squared(u, h)
@@ -151,10 +156,11 @@ class GeluMLP(FeedForward):
 
     def forward(self, xn, residual, ctx):
         t = xn.shape[0]
-        u = ctx.ws.buffer("mlp.up32", (t, self.inter), torch.float32)
-        self.up(xn, u, ws=ctx.ws)
         h = ctx.ws.buffer("mlp.h", (t, self.inter), self.rt.dtype)
-        ops.gelu_tanh(u, h)
+        if not self.up.with_activation(xn, h, "gelu_tanh", ws=ctx.ws):
+            u = ctx.ws.buffer("mlp.up32", (t, self.inter), torch.float32)
+            self.up(xn, u, ws=ctx.ws)
+            ops.gelu_tanh(u, h)
         residual.add_linear(self.down, h)
 
 
@@ -178,6 +184,9 @@ class XieluMLP(ReluSquaredMLP):
         super().load_params(get)
         p, q = torch.nn.functional.softplus(get(self.prefix + self.names["act"]).to(torch.float64)).tolist()
         self.sp, self.sq = p, 0.5 + q
+
+    def epilogue(self):
+        return "xielu", (self.sp, self.sq)
 
     def activate(self, u, h):
         ops.xielu(u, h, self.sp, self.sq)

@@ -163,10 +163,11 @@ class RoutedMLP(FeedForward):
         ops.moe_linear(h, None, self.w_down, plan, max_tiles, yrows, pairs, tile_rows=rows_a_tile)
         shared = None
         if self.shared_inter:
-            u = ws.buffer("mlp.up32", (t, self.shared_inter), torch.float32)
-            self.shared_up(xn, u, ws=ws)
             hs = ws.buffer("mlp.h", (t, self.shared_inter), self.rt.dtype)
-            SHARED_ACTIVATIONS[self.activation](u, hs)
+            if not self.shared_up.with_activation(xn, hs, self.activation, ws=ws):
+                u = ws.buffer("mlp.up32", (t, self.shared_inter), torch.float32)
+                self.shared_up(xn, u, ws=ws)
+                SHARED_ACTIVATIONS[self.activation](u, hs)
             shared = ws.buffer("moe.shared", (t, self.hidden), torch.float32)
             self.shared_down(hs, shared, ws=ws)
         # (a pair whose choice is an identity expert has no row in the plan: the sum takes the token's input for it)

@@ -1259,3 +1259,55 @@ def test_state_space_recurrence_of_long_portions(ops, lens, heads, vdim, n_state
             out.append((S * c[:, :, None]).sum(1) + (0.0 if skip_d else d.double()[:, None] * x))
         assert rel(y[o:o + L], torch.stack(out).reshape(L, -1).numpy()) < tol_, i
         assert rel(dev_state[slots[i]], S.numpy()) < tol_, i
+
+
+@pytest.mark.parametrize("act", ["relu2", "gelu_tanh", "gelu", "xielu"])
+@pytest.mark.parametrize("m,n,k,bias,ws", [
+    (1, 36, 40, True, True),             # the few-row kernel: a chunk that is not whole, columns that fill no tile
+    (8, 9000, 1536, False, True),        # ... many columns
+    (24, 301, 520, True, True),          # ... two tiles of rows
+    (40, 130, 72, True, True),           # 33 to 64 rows, K no multiple of 64: four tiles of rows
+    (50, 300, 1024, True, True),         # K in parts
+    (64, 17000, 128, False, True),       # 64-row tiles of 128 columns
+    (37, 33000, 64, True, True),         # ... and of 256
+    (65, 300, 4096, True, True),         # more rows, K in parts
+    (300, 2053, 192, True, True),        # tiles whose last columns lie past the end, not in 16-byte pieces
+    (1100, 4608, 320, False, True),
+    (2050, 264, 64, True, True),
+])
+def test_linear_with_an_activation_of_its_sums(ops, act, m, n, k, bias, ws):
+    g = torch.Generator().manual_seed(67)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g) * 2 / math.sqrt(k)).to(torch.bfloat16)
+    b = torch.randn(n, generator=g) if bias else None
+    sp, sq = 0.7, 1.3
+    z = x.double() @ w.double().t() + (0 if b is None else b.double())
+    want = {"relu2": lambda: z.clamp(min=0) ** 2, "gelu_tanh": lambda: torch.nn.functional.gelu(z, approximate="tanh"),
+            "gelu": lambda: torch.nn.functional.gelu(z),
+            "xielu": lambda: torch.where(z > 0, sp * z * z, sq * (torch.expm1(z) - z)) + 0.5 * z}[act]()
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    did = ops.linear_act(x.to(DEV), w.to(DEV), None if b is None else b.to(DEV), out, act, (sp, sq), _Lender())
+    assert did == (m <= 64 or act == "relu2")
+    if did:
+        assert rel(out, want.numpy()) < 5e-3                       # the rounding to bfloat16
+        # value by value: half a bfloat16 step of the value, and what the float32 sums of K products lose in the activation's slope
+        slack = want.abs() * 2.0 ** -8 + 8 * math.sqrt(k) * 2.0 ** -24 * (1 + z.abs())
+        assert bool(((out.double().cpu() - want).abs() <= slack).all())
+    else:
+        assert bool(torch.isnan(out.float()).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 100, 72), (9, 8960, 1536), (30, 50, 136), (64, 9000, 256), (200, 333, 128), (1030, 1500, 192)])
+def test_gated_product_with_the_tanh_form_of_gelu(ops, m, n, k):
+    g = torch.Generator().manual_seed(68)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(2 * n, k, generator=g) * 2 / math.sqrt(k)).to(torch.bfloat16)
+    z = x.double() @ w.double().t()
+    want = torch.nn.functional.gelu(z[:, :n], approximate="tanh") * z[:, n:]
+    out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.linear_swiglu(x.to(DEV), w.to(DEV), out, limit=ops.GELU_TANH_GATE)
+    assert rel(out, want.numpy()) < 5e-3
+    if m <= 16:
+        out = torch.full((m, n), float("nan"), device=DEV)
+        ops.linear_swiglu(x.float().to(DEV), w.float().to(DEV), out, limit=ops.GELU_TANH_GATE)
+        assert rel(out, want.numpy()) < 8 * math.sqrt(k) * 2.0 ** -24
