@@ -1045,19 +1045,36 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
 
 // joins the splits of every (token, head) in split order: a block a (token, head)
 // (the parts of a token lie at its place in the list, or, with by_token, at its own number)
+// The first wave takes the splits' maxima and sums side by side and leaves every split's factor in LDS; a column's parts are
+// then asked for eight at a time.  (Maxima, factors and parts split after split were a chain of three loads and an
+// exponential for each: 24 to 48 splits 6.6 to 10 us, now 4.6 to 5.3.)
+#define JOIN_MAX_SPLITS 64
 __global__ void masked_attention_join_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out,
                                              const int* __restrict__ token_list, int nh, int dv, int nsplit, MaExtras ex, int by_token) {
+    __shared__ float fac[JOIN_MAX_SPLITS], sums[JOIN_MAX_SPLITS], top[1];
     const int t = token_list ? token_list[blockIdx.x] : blockIdx.x, head = blockIdx.y;
     const float* base = parts + ((size_t)(by_token ? t : (int)blockIdx.x) * nh + head) * nsplit * (dv + 2);
-    float mm = -INFINITY;
-    for (int x = 0; x < nsplit; ++x) mm = fmaxf(mm, base[(size_t)x * (dv + 2) + dv]);
+    if (threadIdx.x < LI_WAVE) {                       // (at most as many splits as a wave has lanes)
+        const int x = threadIdx.x < nsplit ? threadIdx.x : nsplit - 1;
+        const float m = base[(size_t)x * (dv + 2) + dv], l = base[(size_t)x * (dv + 2) + dv + 1];
+        const float mm = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - mm);
+        fac[threadIdx.x] = f;
+        sums[threadIdx.x] = l * f;
+        if (threadIdx.x == 0) top[0] = mm;
+    }
+    __syncthreads();
+    const float mm = top[0];
+    float ll = 0.f;
+#pragma unroll 8
+    for (int x = 0; x < nsplit; ++x) ll += sums[x];
     for (int d = threadIdx.x; d < dv; d += blockDim.x) {
-        float a = 0.f, ll = 0.f;
-        for (int x = 0; x < nsplit; ++x) {
-            const float* r = base + (size_t)x * (dv + 2);
-            const float f = (r[dv] == -INFINITY) ? 0.f : expf(r[dv] - mm);
-            a += r[d] * f;
-            ll += r[dv + 1] * f;
+        float a = 0.f;
+        for (int x0 = 0; x0 < nsplit; x0 += 8) {
+            float r[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) r[i] = base[(size_t)(x0 + i < nsplit ? x0 + i : nsplit - 1) * (dv + 2) + d];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a = x0 + i < nsplit ? fmaf(r[i], fac[x0 + i], a) : a;
         }
         out[((size_t)t * nh + head) * dv + d].bits = float_to_bf16(a * finish_factor(ll, mm, ex, t, head) * column_gate(ex, t, head, dv, d));
     }
@@ -1135,9 +1152,12 @@ extern "C" int li_masked_attention_single(const float* q, int q_token_stride, in
 // the other.  x and out are addressed by a token stride and a head stride, so that a head's columns may lie inside
 // a wider row.  With `gate`, head h's outputs of token t are multiplied by sigmoid(gate[t * gate_stride + h]), or, with
 // gate_per_column, output j of head h by sigmoid(gate[t * gate_stride + h * n_out + j]).
-// A block takes one head, HL_TOK tokens and 256 outputs: the tokens' inputs lie in LDS as float32, a
-// thread owns an output and reads its matrix row once for all the tokens.  Sums are float32, in the order of k.
+// A block takes one head, TOK tokens (1, 2, 4 or 8, as many as there are) and 64 outputs at a time: the tokens' inputs lie
+// in LDS as float32, four neighbouring threads share an output and read its matrix row once for all the tokens, HL_AHEAD
+// pieces of 16 bytes asked for together (one after the other, and multiplied for eight tokens whatever there were, 12 heads
+// of 128 x 256 took 12.5 us at 2 tokens, of 256 x 128 8.2; now 8.6 and 6.0).  Sums are float32, in the order of k.
 #define HL_TOK 8
+#define HL_AHEAD 8
 
 // Behind a head's n_in inputs may lie `n` more columns that are not multiplied but ROTATED by the token's angles
 // (cos, sin [T, n / 2]) and written behind the head's n_out outputs: pairs of neighbouring columns, or (split)
@@ -1153,28 +1173,28 @@ __device__ __forceinline__ void head_tail_rotate(const TX* __restrict__ src, TO*
     store_from_float(dst + b, fmaf(v, c, __fmul_rn(u, sn)));
 }
 
-template <typename TX, typename TM, typename TO, bool VEC>
+template <typename TX, typename TM, typename TO, bool VEC, int TOK>
 __global__ __launch_bounds__(256) void headwise_linear_kernel(
     const TX* __restrict__ x, long x_token_stride, int x_head_stride, const TM* __restrict__ m, TO* __restrict__ out,
     long o_token_stride, int o_head_stride, int T_, int n_out, int n_in, const float* __restrict__ gate, long gate_stride,
     int gate_per_column, HeadTail tail) {
-    extern __shared__ float xs[];                    // [HL_TOK][n_in]
-    const int h = blockIdx.y, t0 = blockIdx.x * HL_TOK;
-    const int nt = (T_ - t0 < HL_TOK) ? T_ - t0 : HL_TOK;
+    extern __shared__ float xs[];                    // [TOK][n_in]
+    const int h = blockIdx.y, t0 = blockIdx.x * TOK;
+    const int nt = (T_ - t0 < TOK) ? T_ - t0 : TOK;
     if (tail.n > 0 && blockIdx.z == 0)
         for (int u = threadIdx.x; u < nt * (tail.n / 2); u += 256) {
             const int tt = u / (tail.n / 2), i = u % (tail.n / 2);
             head_tail_rotate(x + (size_t)(t0 + tt) * x_token_stride + (size_t)h * x_head_stride + n_in,
                              out + (size_t)(t0 + tt) * o_token_stride + (size_t)h * o_head_stride + n_out, t0 + tt, i, tail);
         }
-    for (int i = threadIdx.x; i < HL_TOK * n_in; i += 256) {
+    for (int i = threadIdx.x; i < TOK * n_in; i += 256) {
         const int tt = i / n_in, k = i % n_in;
         xs[i] = tt < nt ? load_as_float(x + (size_t)(t0 + tt) * x_token_stride + (size_t)h * x_head_stride + k) : 0.f;
     }
     // the heads' gates are asked for before the products, so that they have arrived when the outputs are ready
-    float gf[HL_TOK];
+    float gf[TOK];
 #pragma unroll
-    for (int tt = 0; tt < HL_TOK; ++tt) gf[tt] = gate && !gate_per_column ? gate[(size_t)(t0 + (tt < nt ? tt : 0)) * gate_stride + h] : 0.f;
+    for (int tt = 0; tt < TOK; ++tt) gf[tt] = gate && !gate_per_column ? gate[(size_t)(t0 + (tt < nt ? tt : 0)) * gate_stride + h] : 0.f;
     __syncthreads();
     // four neighbouring threads share an output: each takes every fourth piece of the matrix row
     constexpr int E = VEC ? 16 / (int)sizeof(TM) : 1;
@@ -1182,39 +1202,53 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
     for (int j = blockIdx.z * 64 + (threadIdx.x >> 2); j < n_out + 63; j += gridDim.z * 64) {       // (whole groups of four go round together)
         const bool on = j < n_out;
         const TM* row = m + ((size_t)h * n_out + (on ? j : 0)) * n_in;
-        float acc[HL_TOK];
+        float acc[TOK];
 #pragma unroll
-        for (int tt = 0; tt < HL_TOK; ++tt) acc[tt] = 0.f;
-        for (int k = part * E; k < n_in; k += 4 * E) {
-            float wv[E];
-            if constexpr (VEC) {
-                const uint4 raw = *reinterpret_cast<const uint4*>(row + k);
-                if constexpr (sizeof(TM) == 2) {
-                    const uint32_t r4[4] = {raw.x, raw.y, raw.z, raw.w};
+        for (int tt = 0; tt < TOK; ++tt) acc[tt] = 0.f;
+        if constexpr (VEC) {
+            const int pieces = n_in / E;             // (a whole number; a thread takes the pieces part, part + 4, ...)
+            for (int c0 = part; c0 < pieces; c0 += 4 * HL_AHEAD) {
+                uint4 raw[HL_AHEAD];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        wv[2 * e] = __uint_as_float(r4[e] << 16);
-                        wv[2 * e + 1] = __uint_as_float(r4[e] & 0xffff0000u);
+                for (int u = 0; u < HL_AHEAD; ++u) raw[u] = *reinterpret_cast<const uint4*>(row + (size_t)(c0 + 4 * u < pieces ? c0 + 4 * u : pieces - 1) * E);
+#pragma unroll
+                for (int u = 0; u < HL_AHEAD; ++u) {
+                    const int k = (c0 + 4 * u) * E;
+                    if (k >= n_in) break;
+                    float wv[E];
+                    const uint32_t r4[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
+                    if constexpr (sizeof(TM) == 2) {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            wv[2 * e] = __uint_as_float(r4[e] << 16);
+                            wv[2 * e + 1] = __uint_as_float(r4[e] & 0xffff0000u);
+                        }
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) wv[e] = __uint_as_float(r4[e]);
                     }
-                } else {
-                    wv[0] = __uint_as_float(raw.x); wv[1] = __uint_as_float(raw.y);
-                    wv[2] = __uint_as_float(raw.z); wv[3] = __uint_as_float(raw.w);
+#pragma unroll
+                    for (int e = 0; e < E; ++e)
+#pragma unroll
+                        for (int tt = 0; tt < TOK; ++tt) acc[tt] = fmaf(wv[e], xs[tt * n_in + k + e], acc[tt]);
                 }
-            } else {
-                wv[0] = load_as_float(row + k);
             }
+        } else {
+            for (int k = part; k < n_in; k += 4) {
+                const float wv = load_as_float(row + k);
 #pragma unroll
-            for (int e = 0; e < E; ++e)
-#pragma unroll
-                for (int tt = 0; tt < HL_TOK; ++tt) acc[tt] = fmaf(wv[e], xs[tt * n_in + k + e], acc[tt]);
+                for (int tt = 0; tt < TOK; ++tt) acc[tt] = fmaf(wv, xs[tt * n_in + k], acc[tt]);
+            }
         }
 #pragma unroll
-        for (int tt = 0; tt < HL_TOK; ++tt) {
+        for (int tt = 0; tt < TOK; ++tt) {
             acc[tt] += __shfl_xor(acc[tt], 1, LI_WAVE);
             acc[tt] += __shfl_xor(acc[tt], 2, LI_WAVE);
         }
         if (on && part == 0)
-            for (int tt = 0; tt < nt; ++tt) {
+#pragma unroll
+            for (int tt = 0; tt < TOK; ++tt) {
+                if (tt >= nt) break;
                 const float gv = gate_per_column ? gate[(size_t)(t0 + tt) * gate_stride + (size_t)h * n_out + j] : gf[tt];
                 const float f = gate ? 1.0f / (1.0f + expf(-gv)) : 1.0f;
                 store_from_float(out + (size_t)(t0 + tt) * o_token_stride + (size_t)h * o_head_stride + j, acc[tt] * f);
@@ -1323,18 +1357,22 @@ extern "C" int li_headwise_linear(const void* x, int x_dtype, long x_token_strid
         else if (x_dtype == LI_BF16 && out_dtype == LI_F32) took = headwise_mfma<bf16_t, float>(x, x_token_stride, x_head_stride, m, out, o_token_stride, o_head_stride, T_, nh, n_out, n_in, gate, gate_stride, gate_per_column, tail, stream);
         if (took) return li_launch_status();
     }
-    const int zs = (n_out + 63) / 64;
-    const dim3 grid((T_ + HL_TOK - 1) / HL_TOK, nh, zs < 64 ? zs : 64);
-    const size_t lds = (size_t)HL_TOK * n_in * 4;
+    const int zs = (n_out + 63) / 64, tok = T_ <= 1 ? 1 : T_ <= 2 ? 2 : T_ <= 4 ? 4 : HL_TOK;
+    const dim3 grid((T_ + tok - 1) / tok, nh, zs < 64 ? zs : 64);
+    const size_t lds = (size_t)tok * n_in * 4;
+#define HL_AS(TX, TM, TO, VEC, TOK)                                                                                        \
+    headwise_linear_kernel<TX, TM, TO, VEC, TOK><<<grid, 256, lds, stream>>>(                                              \
+        (const TX*)x, x_token_stride, x_head_stride, (const TM*)m, (TO*)out, o_token_stride, o_head_stride, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail)
 #define HL_GO(TX, TM, TO)                                                                                                  \
     {                                                                                                                      \
         constexpr int E = 16 / sizeof(TM);                                                                                 \
-        if (n_in % E == 0 && ((uintptr_t)m % 16) == 0)                                                                     \
-            headwise_linear_kernel<TX, TM, TO, true><<<grid, 256, lds, stream>>>(                                          \
-                (const TX*)x, x_token_stride, x_head_stride, (const TM*)m, (TO*)out, o_token_stride, o_head_stride, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail); \
-        else                                                                                                               \
-            headwise_linear_kernel<TX, TM, TO, false><<<grid, 256, lds, stream>>>(                                         \
-                (const TX*)x, x_token_stride, x_head_stride, (const TM*)m, (TO*)out, o_token_stride, o_head_stride, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail); \
+        if (n_in % E == 0 && ((uintptr_t)m % 16) == 0) {                                                                   \
+            if (tok == 1) HL_AS(TX, TM, TO, true, 1); else if (tok == 2) HL_AS(TX, TM, TO, true, 2);                       \
+            else if (tok == 4) HL_AS(TX, TM, TO, true, 4); else HL_AS(TX, TM, TO, true, HL_TOK);                           \
+        } else {                                                                                                           \
+            if (tok == 1) HL_AS(TX, TM, TO, false, 1); else if (tok == 2) HL_AS(TX, TM, TO, false, 2);                     \
+            else if (tok == 4) HL_AS(TX, TM, TO, false, 4); else HL_AS(TX, TM, TO, false, HL_TOK);                         \
+        }                                                                                                                  \
         return li_launch_status();                                                                                         \
     }
     if (x_dtype == LI_F32 && m_dtype == LI_F32 && out_dtype == LI_F32) HL_GO(float, float, float)
@@ -1343,5 +1381,6 @@ extern "C" int li_headwise_linear(const void* x, int x_dtype, long x_token_strid
     if (x_dtype == LI_BF16 && m_dtype == LI_BF16 && out_dtype == LI_BF16) HL_GO(bf16_t, bf16_t, bf16_t)
     if (x_dtype == LI_BF16 && m_dtype == LI_BF16 && out_dtype == LI_F32) HL_GO(bf16_t, bf16_t, float)
 #undef HL_GO
+#undef HL_AS
     return LI_ERR_DTYPE;
 }
