@@ -1,11 +1,10 @@
 // out[M, N] = x[M, K] w[N, K]^T (+ bias[N]), or out += accumulate * (x w^T + bias) where the number `accumulate`
 // is not 0 (1 for a plain sum), float32 accumulation.
 //
-// float32 operands: an LDS-tiled FMA kernel (true 32-bit, no reduced-precision
-// matrix mode).  bfloat16 operands: MFMA tiles for 64-wide waves.  For each
-// output element the sum over K runs in an order that depends on K alone, not
-// on M or on the element's place, so a row's result does not depend on which
-// other rows are in the batch.
+// float32 operands: float32 MFMA tiles, and an LDS-tiled FMA kernel where K is no multiple of 4 (true 32-bit, no
+// reduced-precision matrix mode).  bfloat16 operands: MFMA tiles for 64-wide waves.  Within a kernel the sum over K
+// runs in an order that depends on K and the number of parts K is cut into, not on the element's place; which kernel
+// and how many parts follow from M, N and K, so the rows of one call are all summed alike.
 #include "common.h"
 #include <algorithm>
 #include <type_traits>
@@ -166,21 +165,29 @@ __global__ __launch_bounds__(256) void gemm_f32_big_kernel(const float* __restri
 // is not one of the reduced-precision matrix modes), at twice the rate of the vector ALU's FMA and without
 // the operands' way through registers that an 8 x 8 tile a lane needs.  Block tile 128 x 128, four waves
 // two by two, each 64 x 64 = 2 x 2 MFMA tiles; K in steps of 16 (eight MFMAs of two k-values a tile).
-// A stage holds x and w transposed, [k][row] with rows of 128 + 4 floats: lane (row, k) of an MFMA operand
-// reads consecutive words, and the transposing writes of the 16-byte global loads (lane = row / k-quarter)
-// meet no bank twice.  Two stages: the next step's global loads are in registers while this step is
-// multiplied.  K a multiple of 4; rows and columns past the end repeat the last and are not stored.
+// A stage holds the rows of x and w as they lie in memory, 16 k-values (four 16-byte pieces) a row; piece p of row r
+// lies at place p ^ (r / 4 % 4), so that neither the writes (four rows' pieces side by side) nor the reads (a piece
+// each of sixteen rows) meet a bank twice.  Lane (row, k) of an MFMA reads a whole piece, the k-th of a pair, and the
+// MFMA e of a pair multiplies the e-th values of both: k-values e and 4 + e of eight (within a step the order of a
+// sum is the same for every row and column).  Bound by the matrix cores: a wave's 32 MFMAs of a step take 2,048 cycles
+// of its SIMD, so what a wave needs next has to be there when it is done.  The pieces of a half step are read while the
+// other half is multiplied, and global loads are on their way for a whole step: a step 1.06 us where a unit has one block,
+// against 1.21 with transposed stages read word by word as the MFMAs need them (0.87 if a step were its MFMAs alone);
+// 1,024 x 17,920 x 1,536 520 -> 500 us, 2,048 rows 925 -> 890, 128 x 1,536 x 1,536 in one part 128 -> 113.  Steps of 32
+// k-values were no faster (the same time a k-value), and loads straight into LDS were where the blocks fill whole rounds
+// over the chip (1,024 x 3,584 x 18,944 in one part 1,267 -> 1,165) and up to 15 % slower where they do not
+// (2,048 x 1,536 x 8,960 460 -> 540): blocks in lockstep end together, and the next ones pile up on the first unit.
+// K a multiple of 4; rows and columns past the end repeat the last and are not stored.
 // gridDim.z > 1: K is cut into that many parts of `part_steps` steps (the last one shorter), and part z's sums go to
 // the z-th [M, N] matrix behind `out`, without bias (splitk_reduce_kernel adds them up in order; see f32_split_parts).
 #define F32M_BM 128
 #define F32M_BN 128
 #define F32M_BK 16
-#define F32M_LD (F32M_BM + 4)
 __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, const float* __restrict__ w,
                                                              const float* __restrict__ bias, float* __restrict__ out,
                                                              int M, int N, int row_len, float accumulate, int part_steps) {
-    __shared__ float As[2][F32M_BK * F32M_LD];
-    __shared__ float Bs[2][F32M_BK * F32M_LD];
+    __shared__ __align__(16) float As[2][F32M_BM * F32M_BK];
+    __shared__ __align__(16) float Bs[2][F32M_BN * F32M_BK];
     // this block's k-values: [k_first, k_first + K) of rows of row_len
     const int k_first = blockIdx.z * part_steps * F32M_BK;
     const int K = gridDim.z == 1 || blockIdx.z + 1 == gridDim.z ? row_len - k_first : part_steps * F32M_BK;
@@ -188,8 +195,9 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int m0 = blockIdx.y * F32M_BM, n0 = blockIdx.x * F32M_BN;
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    // global loads: thread t takes the k-quarter t % 4 of rows t / 4 and t / 4 + 64 of both tiles
+    // global loads: thread t takes the piece t % 4 of rows t / 4 and t / 4 + 64 of both tiles
     const int lrow = tid >> 2, lkq = tid & 3;
+    const int put = lrow * F32M_BK + 4 * (lkq ^ ((lrow >> 2) & 3));          // (row + 64: 64 rows further on)
     const float* xa[2];
     const float* wb[2];
 #pragma unroll
@@ -213,14 +221,13 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
             if constexpr (!WHOLE) { if (!ok) { ga[h] = floatx4{0.f, 0.f, 0.f, 0.f}; gb[h] = floatx4{0.f, 0.f, 0.f, 0.f}; } }
         }
     };
+    auto fetch_any = [&](int k0) { if (k0 + F32M_BK <= K) fetch(k0, std::true_type{}); else fetch(k0, std::false_type{}); };
     auto stash = [&](int st) {
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                As[st][(4 * lkq + e) * F32M_LD + lrow + 64 * h] = ga[h][e];
-                Bs[st][(4 * lkq + e) * F32M_LD + lrow + 64 * h] = gb[h][e];
-            }
+        for (int h = 0; h < 2; ++h) {
+            *reinterpret_cast<floatx4*>(&As[st][put + 64 * h * F32M_BK]) = ga[h];
+            *reinterpret_cast<floatx4*>(&Bs[st][put + 64 * h * F32M_BK]) = gb[h];
+        }
     };
     floatx16 acc[2][2];
 #pragma unroll
@@ -230,42 +237,62 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 #pragma unroll
             for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
     const int frow = lane & 31, fk = lane >> 5;
-    auto multiply = [&](int st) {
+    floatx4 fa[2][2], fb[2][2];                            // [half of the step][MFMA tile]
+    auto read = [&](int st, auto half_tag) {
+        constexpr int H = decltype(half_tag)::value;
+        const int piece = 4 * ((2 * H + fk) ^ ((frow >> 2) & 3));
 #pragma unroll
-        for (int s2 = 0; s2 < F32M_BK / 2; ++s2) {
-            float a[2], b[2];
+        for (int i = 0; i < 2; ++i) fa[H][i] = *reinterpret_cast<const floatx4*>(&As[st][(wm + 32 * i + frow) * F32M_BK + piece]);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = As[st][(2 * s2 + fk) * F32M_LD + wm + 32 * i + frow];
+        for (int j = 0; j < 2; ++j) fb[H][j] = *reinterpret_cast<const floatx4*>(&Bs[st][(wn + 32 * j + frow) * F32M_BK + piece]);
+    };
+    auto multiply = [&](auto half_tag) {
+        constexpr int H = decltype(half_tag)::value;
 #pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = Bs[st][(2 * s2 + fk) * F32M_LD + wn + 32 * j + frow];
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < 2; ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[H][i][e], fb[H][j][e], acc[i][j], 0, 0, 0);
     };
-    if (K >= F32M_BK) fetch(0, std::true_type{}); else fetch(0, std::false_type{});
+    constexpr std::integral_constant<int, 0> FIRST{};
+    constexpr std::integral_constant<int, 1> SECOND{};
+    fetch_any(0);
     stash(0);
+    if (F32M_BK < K) fetch_any(F32M_BK);
     __syncthreads();
+    read(0, FIRST);
     int st = 0, k0 = 0;
-    // while the step after this one is whole, its loads are neither conditional nor chosen from ...
-    for (; k0 + 2 * F32M_BK <= K; k0 += F32M_BK) {
-        fetch(k0 + F32M_BK, std::true_type{});
-        __builtin_amdgcn_sched_barrier(0);                 // (left to itself the compiler moves the loads down to where their values are stored)
-        multiply(st);
-        stash(st ^ 1);                                     // (the other stage: its readers passed the barrier a step ago)
+    // A step: its second half's pieces are asked for, the first half is multiplied, the next step's values go to the other
+    // stage (whose readers have passed the barrier of the step before), the loads of the step after it start, and behind
+    // the barrier the next step's first half is asked for while the second half is multiplied.
+    // While the step two further on is whole, its loads are neither conditional nor chosen from ...
+    for (; k0 + 3 * F32M_BK <= K; k0 += F32M_BK) {
+        read(st, SECOND);
+        __builtin_amdgcn_sched_barrier(0);                 // (left to itself the compiler moves reads and loads down to where their values are used)
+        multiply(FIRST);
+        stash(st ^ 1);
+        fetch(k0 + 2 * F32M_BK, std::true_type{});
         __syncthreads();
         st ^= 1;
+        read(st, FIRST);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(SECOND);
     }
-    // ... then the last whole step and, where K is no multiple of the step, the one behind it
+    // ... then the steps that are left
     for (; k0 < K; k0 += F32M_BK) {
         const bool more = k0 + F32M_BK < K;
-        if (more) fetch(k0 + F32M_BK, std::false_type{});
-        multiply(st);
-        if (more) stash(st ^ 1);
+        read(st, SECOND);
+        multiply(FIRST);
+        if (more) {
+            stash(st ^ 1);
+            if (k0 + 2 * F32M_BK < K) fetch_any(k0 + 2 * F32M_BK);
+        }
         __syncthreads();
         st ^= 1;
+        if (more) read(st, FIRST);
+        multiply(SECOND);
     }
     // register r of lane l: row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32 of a 32 x 32 tile
 #pragma unroll
@@ -2049,14 +2076,13 @@ static void launch_f32_mfma(const float* x, const float* w, const float* bias, f
 
 // Into how many parts K is cut for the float32 tiles of 128 x 128 (more than 64 rows): a narrow matrix has fewer tiles
 // than the chip has compute units (810 rows against 1,536 columns: 84), and a tile's time is the length of K whatever the
-// others do.  The least estimated time, in microseconds: a step of 16 k-values takes a unit 1.2 us (0.43 TFLOP/s a unit;
-// blocks that share a unit overlap by some 5 %), a block 6 for its start and end, and the parts' sums are written and
-// read again at 5 TB/s by a kernel of its own (4 us).  Measured, one part against the parts taken here: 65 to 128 rows
-// x 1,536 x 8,960 685 -> 60 us (16 parts), 300 rows 683 -> 130 (6), 810 rows 682 -> 227 (6), x 1,536 x 1,536 138 -> 56,
-// 810 x 2,048 x 1,536 135 -> 75 (2), 1,024 x 3,584 x 18,944 1,464 -> 1,107 (8), 2,048 x 3,584 x 3,584 495 -> 452 (4);
-// from some thousand tiles on (810 x 17,920: 980) parts cost what they give, and K stays whole.  The rule is within
-// 6 % of the best number of parts measured at 65 to 4,096 rows against seven matrices (13 % at 128 rows x 1,536 x 1,536
-// and 810 x 4,608 x 3,584).  At most 256 MB of parts.
+// others do.  The least estimated time, in microseconds: a step of 16 k-values counts as 1.2 us of a unit (1.06 measured
+// where blocks do not share units, up to 1.25 where they do), a block 6 for its start and end, and the parts' sums are
+// written and read again at 5 TB/s by a kernel of its own (4 us).  Measured, one part against the parts taken here: 65 to
+// 128 rows x 1,536 x 8,960 597 -> 54 us (16 parts), 300 rows 597 -> 100 (6), 810 rows 598 -> 206 (6), x 1,536 x 1,536
+// 125 -> 51, 810 x 2,048 x 1,536 122 -> 67 (2), 1,024 x 3,584 x 18,944 1,276 -> 1,074 (8), 2,048 x 3,584 x 3,584
+// 463 -> 430 (4); from some thousand tiles on (810 x 17,920: 980) parts cost what they give, and K stays whole.  The rule
+// is within 7 % of the best number of parts measured at 65 to 2,048 rows against seven matrices.  At most 256 MB of parts.
 #define F32_MAX_PARTS 16
 #define F32_PARTS_MAX_BYTES (256l << 20)
 #define F32_PART_MIN_STEPS 6

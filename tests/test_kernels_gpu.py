@@ -194,6 +194,10 @@ def test_linear_with_k_in_parts(ops, m, n, k, out_dtype, bias, acc):
     (810, 1536, 1536, False, 1.0),
     (257, 260, 4096, True, 0.0),             # not accumulating
     (2048, 300, 92, True, 1.0),              # too short a K for parts
+    (65, 4, 4, False, 1.0),                  # a quarter of a step
+    (70, 130, 20, True, 1.0),                # one whole step and a quarter
+    (129, 257, 36, False, 0.5),              # two and a quarter, tiles of one row and one column
+    (200, 96, 52, True, 1.0),                # three and a quarter: the loop's first whole round
 ])
 def test_float32_linear_with_k_in_parts(ops, m, n, k, bias, factor):
     from litinfer_amd.kernels.ops import _work_bytes
