@@ -319,7 +319,7 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 // so a wave keeps many loads in flight: the FMA form held 8 x 8 sums a lane and one piece in flight, and
 // streamed w at 3.2 TB/s.  The eight waves' sums are added in wave order: an order that depends on K alone.
 #define F32RM_WAVES 8
-template <int AHEAD, int TILES, int RT, bool SWIGLU>
+template <int AHEAD, int TILES, int RT, bool SWIGLU, bool PACK = false>
 __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(const float* __restrict__ x,
                                                                               const float* __restrict__ w,
                                                                               const float* __restrict__ bias,
@@ -332,21 +332,29 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
     // SWIGLU: w is [gate; up] of N rows each, the tiles come in pairs (the gate columns n0 + 16 p .. and the
     // up columns of the same outputs), `cols` <= 8 TILES outputs a block, and out [M, N] gets
     // up * gate / (1 + exp(-gate)) from the float32 sums: the 2 N columns never go to memory.
+    // PACK: at most 8 rows and 8 columns a block: an MFMA takes both halves of a piece, k-values 0 .. 15 in its rows and
+    // columns 0 .. 7 and 16 .. 31 in 8 .. 15, so that no lane loads a row or a column that another one has; the two
+    // quarters of the result that pair a half with itself are the sums, the other two are left.  (A matrix of few columns
+    // has few of them a block, six of 1,536 on 256 units: of sixteen lanes' loads ten brought what others had.  3 rows
+    // x 1,536 x 8,960, 55 MB, 22.4 -> 17.3 us.)
     static_assert(!SWIGLU || TILES % 2 == 0, "gate and up tiles in pairs");
+    static_assert(!PACK || (!SWIGLU && TILES == 1 && RT == 1), "one tile");
+    constexpr int UN = PACK ? 1 : 2;                          // loads a piece
     __shared__ float part[F32RM_WAVES][RT * TILES * 256];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (the same for a wave's lanes: its branches are scalar)
     const int c = lane & 15, q = lane >> 4;
+    const int cr = PACK ? c & 7 : c, kq = PACK ? 16 * (c >> 3) + 4 * q : 4 * q;      // a lane's row or column of a tile, its first k-value of a piece
     const int n0 = blockIdx.x * cols;
     const int nend = n0 + cols < N ? n0 + cols : N;
     const float* wrow[TILES];
 #pragma unroll
     for (int t = 0; t < TILES; ++t) {
-        const int col = SWIGLU ? n0 + 16 * (t / 2) + c : n0 + 16 * t + c;
-        wrow[t] = w + ((size_t)(col < nend ? col : nend - 1) + (SWIGLU && (t & 1) ? (size_t)N : 0)) * K + 4 * q;
+        const int col = SWIGLU ? n0 + 16 * (t / 2) + c : n0 + 16 * t + cr;
+        wrow[t] = w + ((size_t)(col < nend ? col : nend - 1) + (SWIGLU && (t & 1) ? (size_t)N : 0)) * K + kq;
     }
     const float* xrow[RT];
 #pragma unroll
-    for (int i = 0; i < RT; ++i) xrow[i] = x + (size_t)(16 * i + c < M ? 16 * i + c : M - 1) * K + 4 * q;
+    for (int i = 0; i < RT; ++i) xrow[i] = x + (size_t)(16 * i + cr < M ? 16 * i + cr : M - 1) * K + kq;
     floatx4 acc[RT][TILES][2];                                // two chains of MFMAs a tile (each waits for its own last result only)
 #pragma unroll
     for (int i = 0; i < RT; ++i)
@@ -357,7 +365,7 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
     // the end reads the row's last 16 bytes and multiplies by zero); the next trip's loads are issued before
     // this trip is multiplied, into the other set of registers.  (Loads that pass the caches by, `nontemporal`,
     // were 10 % slower here, as for the bfloat16 products.)
-    floatx4 wv[2][AHEAD][2][TILES], xv[2][AHEAD][2][RT];
+    floatx4 wv[2][AHEAD][UN][TILES], xv[2][AHEAD][UN][RT];
     constexpr int PIECE = 32 * F32RM_WAVES, TRIP = PIECE * AHEAD;
     // WHOLE: every piece of the trip lies inside K; nothing is then chosen or replaced (a value chosen between what
     // was loaded and zero is waited for at once, and so is the next use of any load behind a conditional one).
@@ -366,10 +374,10 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
 #pragma unroll
         for (int a = 0; a < AHEAD; ++a)
 #pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                const int k = k0 + PIECE * a + 16 * u;                    // + 4 q is in the row pointers
-                const bool ok = WHOLE || k + 4 * q < K;
-                const int at = ok ? k : last - 4 * q;
+            for (int u = 0; u < UN; ++u) {
+                const int k = k0 + PIECE * a + 16 * u;                    // + kq is in the row pointers
+                const bool ok = WHOLE || k + kq < K;
+                const int at = ok ? k : last - kq;
 #pragma unroll
                 for (int t = 0; t < TILES; ++t) wv[buf][a][u][t] = *reinterpret_cast<const floatx4*>(wrow[t] + at);
 #pragma unroll
@@ -387,7 +395,7 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
 #pragma unroll
         for (int a = 0; a < AHEAD; ++a)
 #pragma unroll
-            for (int u = 0; u < 2; ++u)
+            for (int u = 0; u < UN; ++u)
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -433,6 +441,10 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
         float v = part[0][at];
 #pragma unroll
         for (int v2 = 1; v2 < F32RM_WAVES; ++v2) v += part[v2][at];
+        if constexpr (PACK) {                                   // (rows and columns below 8: `row` < M and j < cols)
+#pragma unroll
+            for (int v2 = 0; v2 < F32RM_WAVES; ++v2) v += part[v2][at + 8 * 16 + 8];
+        }
         if constexpr (SWIGLU) {
             float up = part[0][at + 256];
 #pragma unroll
@@ -476,8 +488,9 @@ static int launch_f32_rows(const float* x, const float* w, const float* bias, fl
     const unsigned grid = (unsigned)groups;
     // pieces a trip: a long K keeps four a wave in flight, a short one two (measured: 3,584 columns 136 against
     // 156 us for the 7B's gate/up matrix, 18,944 columns 68.6 against 74.0 us for its way back), a tiny one, and
-    // many rows (whose registers hold the rows' pieces too), one
-#define LI_F32RM(AH, TL, RTV, SW) gemm_f32_rows_mfma_kernel<AH, TL, RTV, SW><<<grid, F32RM_WAVES * 64, 0, stream>>>(x, w, bias, out, M, N, K, accumulate, cols, limit)
+    // many rows (whose registers hold the rows' pieces too), one.  At most 8 rows and 8 columns a block: both halves of a
+    // piece in one load, and so twice the pieces in the same registers (K = 8,960 22.4 -> 17.3 us, K = 1,536 5.5 either way)
+#define LI_F32RM(AH, TL, RTV, ...) gemm_f32_rows_mfma_kernel<AH, TL, RTV, __VA_ARGS__><<<grid, F32RM_WAVES * 64, 0, stream>>>(x, w, bias, out, M, N, K, accumulate, cols, limit)
     const int ahead = rt == 4 ? 1 : K >= 8192 && rt == 1 ? 4 : K >= 32 * F32RM_WAVES * 4 ? 2 : 1;
     if (swiglu) {
         if (rt == 1) { if (ahead == 4) LI_F32RM(4, 2, 1, true); else if (ahead == 2) LI_F32RM(2, 2, 1, true); else LI_F32RM(1, 2, 1, true); }
@@ -487,7 +500,9 @@ static int launch_f32_rows(const float* x, const float* w, const float* bias, fl
     }
     if (rt == 1) {
         if (tiles == 2) { if (ahead == 4) LI_F32RM(4, 2, 1, false); else if (ahead == 2) LI_F32RM(2, 2, 1, false); else LI_F32RM(1, 2, 1, false); }
-        else { if (ahead == 4) LI_F32RM(4, 1, 1, false); else if (ahead == 2) LI_F32RM(2, 1, 1, false); else LI_F32RM(1, 1, 1, false); }
+        else if (M <= 8 && cols <= 8) {
+            if (K >= 8192) LI_F32RM(8, 1, 1, false, true); else if (ahead == 2) LI_F32RM(4, 1, 1, false, true); else LI_F32RM(1, 1, 1, false, true);
+        } else { if (ahead == 4) LI_F32RM(4, 1, 1, false); else if (ahead == 2) LI_F32RM(2, 1, 1, false); else LI_F32RM(1, 1, 1, false); }
     } else if (rt == 2) {
         if (tiles == 2) { if (ahead >= 2) LI_F32RM(2, 2, 2, false); else LI_F32RM(1, 2, 2, false); }
         else { if (ahead >= 2) LI_F32RM(2, 1, 2, false); else LI_F32RM(1, 1, 2, false); }

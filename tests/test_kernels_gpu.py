@@ -218,6 +218,28 @@ def test_float32_linear_with_k_in_parts(ops, m, n, k, bias, factor):
     assert torch.equal(outs[0], outs[2])                       # the parts are added in a fixed order
 
 
+@pytest.mark.parametrize("m,n,k,bias,factor", [
+    (8, 1536, 8960, False, 1.0),             # six columns a block, the longest trips
+    (3, 2048, 1536, True, 0.0),              # eight columns a block
+    (8, 2049, 1540, True, 0.5),              # nine: both halves of a piece one after the other; one piece of a row over
+    (9, 1536, 1536, False, 0.0),             # a row more than both halves of a piece take
+    (1, 5, 4, True, 1.0),                    # one column a block, a single 16-byte piece a row
+    (7, 300, 20, False, 0.0),                # the second half of the only piece is cut
+    (8, 257, 8212, True, 1.0),               # the last piece ends inside its second half
+])
+def test_float32_linear_of_few_rows_and_columns(ops, m, n, k, bias, factor):
+    g = torch.Generator().manual_seed(63)
+    x = torch.randn(m, k, generator=g)
+    w = torch.randn(n, k, generator=g) / math.sqrt(k)
+    b = torch.randn(n, generator=g) if bias else None
+    base = torch.randn(m, n, generator=g)
+    y = x.double().numpy() @ w.double().numpy().T + (0 if b is None else b.double().numpy())
+    y = base.double().numpy() + factor * y if factor else y
+    out = base.to(DEV) if factor else torch.full((m, n), float("nan"), device=DEV)
+    ops.linear(x.to(DEV), w.to(DEV), None if b is None else b.to(DEV), out, bool(factor), factor=factor or 1.0)
+    assert rel(out, y) < 4 * math.sqrt(k) * 2.0 ** -24         # (sums of k float32 products)
+
+
 @pytest.mark.parametrize("m,n,k,bias,taken", [
     (64, 3584, 18944, False, True),      # a decoding batch of 64 at the 7B sizes
     (40, 200, 1024, True, True),
