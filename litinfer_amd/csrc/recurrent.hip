@@ -646,6 +646,7 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
     float* sV = sK + RET_Q * KS;                       // [RET_Q][VB]
     float* pw = sV + RET_Q * VB;                       // [RET_Q + 1]: the powers of the decay (VAR: the tokens' steps)
     __shared__ double cum[VAR ? RET_Q : 1];
+    __shared__ int spoilt_from[VB];                    // the first token whose value of a column is not finite
     const int bx = blockIdx.x, seg = chunk_seg[bx];
     if (seg < 0) return;
     const int first = chunk_idx[bx] * RET_Q, L = q_len[seg];
@@ -671,15 +672,31 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
         if (j < ntok && c < N) k = silu_if4(*reinterpret_cast<const float4*>(xbc + (size_t)(t0 + j) * xbc_stride + inner + (size_t)group * N + c), silu_in);
         *reinterpret_cast<float4*>(sK + j * KS + c) = k;
     }
+    float zeros = 0.f;                                 // NaN once a value is not finite
     for (int x = threadIdx.x; x < RET_Q * (VB / 4); x += 256) {
         const int j = x / (VB / 4), c = 4 * (x % (VB / 4));
         float4 v = float4{0.f, 0.f, 0.f, 0.f};
         if (j < ntok && p0 + c < vdim) v = silu_if4(*reinterpret_cast<const float4*>(xbc + (size_t)(t0 + j) * xbc_stride + (size_t)head * vdim + p0 + c), silu_in);
         *reinterpret_cast<float4*>(sV + j * VB + c) = v;
+        zeros = fmaf(v.x, 0.f, fmaf(v.y, 0.f, fmaf(v.z, 0.f, fmaf(v.w, 0.f, zeros))));
     }
 #pragma unroll
     for (int t = 0; t < NQ; ++t) q[t] = silu_if4(q[t], silu_in);        // (silu(0) = 0)
-    __syncthreads();
+    // A value that is not finite belongs to its column's outputs from its token on.  In the product below it would meet the
+    // zero scores of the tokens before it, and 0 x inf is NaN: it is taken out here, and the outputs from its token on, which
+    // the recurrence leaves infinite or NaN, are written over with NaN.
+    const bool spoilt = __syncthreads_or(!(zeros == 0.f));
+    if (spoilt) {
+        if (threadIdx.x < VB) {
+            int from = RET_Q;
+            for (int j = RET_Q - 1; j >= 0; --j) {
+                float* v = sV + j * VB + threadIdx.x;
+                if (!(*v * 0.f == 0.f)) { *v = 0.f; from = j; }
+            }
+            spoilt_from[threadIdx.x] = from;
+        }
+        __syncthreads();
+    }
     if (it * 32 >= ntok || pc >= vdim) return;
     [[maybe_unused]] const double ci = VAR ? cum[i] : 0.0;
     // VAR: a sum of sixty-four steps of the matrix cores is taken as four (of the products with V: two) side by side, which
@@ -774,6 +791,13 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
                 y[(size_t)(t0 + row) * y_stride + (size_t)head * vdim + p] = v;
             }
         }
+    if (spoilt)
+#pragma unroll
+        for (int pt = 0; pt < PT; ++pt)
+            for (int r = 0; r < 16; ++r) {
+                const int row = it * 32 + 8 * (r >> 2) + 4 * h + (r & 3), p = pc + 32 * pt + ql;
+                if (row < ntok && p < vdim && row >= spoilt_from[p - p0]) y[(size_t)(t0 + row) * y_stride + (size_t)head * vdim + p] = NAN;
+            }
 }
 
 template <int NQ, int PT, bool VAR>

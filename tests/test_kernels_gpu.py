@@ -1287,6 +1287,48 @@ def test_state_space_recurrence_of_long_portions(ops, lens, heads, vdim, n_state
         assert rel(dev_state[slots[i]], S.numpy()) < tol_, i
 
 
+@pytest.mark.parametrize("kind,silu", [("ssm", False), ("fixed", False), ("fixed", True)])
+@pytest.mark.parametrize("vdim,n_state", [(64, 128), (132, 40)])
+def test_recurrence_of_long_portions_keeps_values_that_are_not_finite_to_their_columns_and_later_tokens(ops, kind, silu, vdim, n_state):
+    """Token by token an infinite value reaches its own column's state and outputs from its token on and nothing else: all
+    other outputs and states are, bit for bit, those of the same portion without it."""
+    import types
+    g = torch.Generator().manual_seed(69)
+    R = lambda *s: torch.randn(*s, generator=g)
+    lens, heads, groups = [130, 40, 64], 4, 4
+    n, T, inner = len(lens), sum(lens), heads * vdim
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    ctx = types.SimpleNamespace(num_tokens=T, num_segments=n, max_q_len=max(lens), host_state_slots=np.arange(n, dtype=np.int32),
+                                state_slots=dev([0, 1, 2]), q_start=dev([0, 130, 170]), q_len=dev(lens))
+    state, rows, dt = R(n, heads, n_state, vdim) * 0.3, R(T, inner + 2 * groups * n_state), R(T, heads).to(DEV)
+    bias, a_log, d = (R(heads) - 3.0).to(DEV), torch.rand(heads, generator=g).to(DEV), R(heads).to(DEV)
+    fixed = torch.linspace(0.9, 0.99, heads).to(DEV)
+    bad = [(0, 20, 5, float("inf")), (0, 63, 0, float("-inf")), (0, 64, vdim - 1, float("nan")), (0, 129, inner - 1, float("inf")),
+           (1, 130, 7, float("inf")), (1, 169, 8, float("nan")), (2, 170 + 31, vdim, float("inf")), (2, 170 + 33, vdim, float("inf"))]
+    spoilt = rows.clone()
+    for _, t, col, v in bad:
+        spoilt[t, col] = v
+
+    def run(x):
+        s, y = state.to(DEV), torch.zeros(T, inner, device=DEV)
+        if kind == "ssm":
+            ops.ssm_scan(x.to(DEV), dt, bias, a_log, d, s, ctx, y, heads, vdim, n_state, groups, _Lender())
+        else:
+            ops.ssm_scan(x.to(DEV), None, None, None, None, s, ctx, y, heads, vdim, n_state, groups, _Lender(), fixed_decay=fixed,
+                         fixed_step=0.3, silu_in=silu)
+        return y.cpu(), s.cpu()
+
+    (y0, s0), (y1, s1) = run(rows), run(spoilt)
+    ends = [130, 170, 234]
+    reached, state_reached = torch.zeros(T, inner, dtype=torch.bool), torch.zeros(n, heads, n_state, vdim, dtype=torch.bool)
+    for i, t, col, _ in bad:
+        reached[t:ends[i], col] = True
+        state_reached[i, col // vdim, :, col % vdim] = True
+    assert torch.isfinite(y0).all() and torch.isfinite(s0).all()
+    assert torch.equal(y1[~reached], y0[~reached]) and not torch.isfinite(y1[reached]).any()
+    assert torch.equal(s1[~state_reached], s0[~state_reached]) and not torch.isfinite(s1[state_reached]).any()
+
+
 @pytest.mark.parametrize("act", ["relu2", "gelu_tanh", "gelu", "xielu"])
 @pytest.mark.parametrize("m,n,k,bias,ws", [
     (1, 36, 40, True, True),             # the few-row kernel: a chunk that is not whole, columns that fill no tile
