@@ -498,7 +498,11 @@ __device__ __forceinline__ void ret_chunk_decays(const RetDecay& dc, int t0, int
     if (threadIdx.x >= RET_Q) return;
     const int j = threadIdx.x;
     const float d = j < ntok ? softplus_f32(dc.dt_raw[(size_t)(t0 + j) * dc.dt_stride + head] + dc.dt_bias[head]) : 0.f;
-    double c = (double)(-expf(dc.A_log[head]) * d);
+    // A token whose decay is zero in float32 counts as exp(-128), zero all the same: an infinite exponent would make the
+    // differences of the sums behind it NaN, and a huge one would swallow the exponents of the other tokens.  (NaN stays.)
+    float l = j < ntok ? -expf(dc.A_log[head]) * d : 0.f;
+    l = l < -128.f ? -128.f : l;
+    double c = (double)l;
 #pragma unroll
     for (int o = 1; o < RET_Q; o <<= 1) {
         const double before = __shfl_up(c, o, LI_WAVE);

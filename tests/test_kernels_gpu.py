@@ -1329,6 +1329,50 @@ def test_recurrence_of_long_portions_keeps_values_that_are_not_finite_to_their_c
     assert torch.equal(s1[~state_reached], s0[~state_reached]) and not torch.isfinite(s1[state_reached]).any()
 
 
+@pytest.mark.parametrize("a_log,dt_raw", [
+    (2.0, 100.0),            # a decay of exp(-740): zero in float32
+    (60.0, 3.0),             # an exponent of 1e26, beside which the other tokens' vanish
+    (80.0, 1.0e4),           # ... that overflows
+    (95.0, -2.0),            # a rate that overflows by itself
+])
+def test_state_space_recurrence_of_long_portions_with_decays_of_zero(ops, a_log, dt_raw):
+    """Some tokens multiply the state by zero; the tokens between them decay as usual (heads 1 and 2) or also to zero (head 0)."""
+    import types
+    g = torch.Generator().manual_seed(70)
+    R = lambda *s: torch.randn(*s, generator=g)
+    lens, heads, vdim, n_state, groups = [130, 70, 20], 3, 64, 32, 1
+    n, T, inner = len(lens), sum(lens), heads * vdim
+    starts = [0, 130, 200]
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    ctx = types.SimpleNamespace(num_tokens=T, num_segments=n, max_q_len=max(lens), host_state_slots=np.arange(n, dtype=np.int32),
+                                state_slots=dev([0, 1, 2]), q_start=dev(starts), q_len=dev(lens))
+    state, rows, dt = R(n, heads, n_state, vdim) * 0.3, R(T, inner + 2 * groups * n_state), R(T, heads)
+    bias, rates, d = R(heads) - 3.0, torch.tensor([a_log, 0.5, a_log]), R(heads)
+    for t in (5, 40, 41, 64, 127, 150, 199, 203):
+        dt[t, :] = torch.tensor([dt_raw, 0.1, dt_raw])
+    if a_log > 50:                                             # head 2: exponents near one for the other tokens
+        quiet = torch.ones(T, dtype=torch.bool)
+        quiet[[5, 40, 41, 64, 127, 150, 199, 203]] = False
+        dt[quiet, 2] = -a_log - float(bias[2]) if a_log < 85 else dt[quiet, 2]
+    dev_state, y = state.to(DEV), torch.full((T, inner), float("nan"), device=DEV)
+    ops.ssm_scan(rows.to(DEV), dt.to(DEV), bias.to(DEV), rates.to(DEV), d.to(DEV), dev_state, ctx, y, heads, vdim, n_state, groups, _Lender())
+    raw = (dt + bias).double()
+    step = torch.where(raw > 20, raw, torch.log1p(torch.exp(raw.clamp(max=20))))
+    decay = torch.exp(-rates.double().exp() * step)
+    for i, (o, L) in enumerate(zip(starts, lens)):
+        S, out = state[i].double(), []
+        for t in range(o, o + L):
+            x, b, c = rows[t].double().split([inner, groups * n_state, groups * n_state])
+            x, b, c = x.view(heads, vdim), b.expand(heads, -1), c.expand(heads, -1)
+            S = decay[t][:, None, None] * S + (step[t][:, None] * b)[:, :, None] * x[:, None]
+            out.append((S * c[:, :, None]).sum(1) + d.double()[:, None] * x)
+        want = torch.stack(out)
+        for h in range(heads):                                 # (each head by itself: their sizes differ)
+            got = y[o:o + L].view(L, heads, vdim)[:, h]
+            assert rel(got, want[:, h].numpy()) < 8 * math.sqrt(2 * n_state + 128) * 2.0 ** -24, (i, h)
+            assert rel(dev_state[i, h], S[h].numpy()) < 8 * math.sqrt(2 * n_state + 128) * 2.0 ** -24, (i, h)
+
+
 @pytest.mark.parametrize("act", ["relu2", "gelu_tanh", "gelu", "xielu"])
 @pytest.mark.parametrize("m,n,k,bias,ws", [
     (1, 36, 40, True, True),             # the few-row kernel: a chunk that is not whole, columns that fill no tile
