@@ -480,7 +480,7 @@ static int ssm_launch(int silu_in, A... args) { return silu_in ? ssm_launch_as<N
 // would lose in float32 what the neighbouring tokens, whose factors are near one, need; the factors themselves and all
 // products are float32, as in the recurrence token by token.  48 heads of 64 columns, 128 state values in 8 groups: 2,048
 // tokens 430 us token by token in chunks side by side -> 155 us, 8 portions of 100 tokens 391 -> 97, 65 tokens 176 -> 33;
-// 112 heads, 2,048 tokens 833 -> 318.
+// 112 heads, 2,048 tokens 833 -> 318; 32 heads of 128 columns, 256 values, 400 tokens 218 -> 125.
 #define RET_Q 64               // tokens of a chunk (SSM chunks of the same length are what the host numbers)
 typedef float ret_f32x16 __attribute__((ext_vector_type(16)));
 
@@ -637,6 +637,21 @@ __global__ __launch_bounds__(64) void retention_carry_kernel(float4* __restrict_
     *st = run;
 }
 
+// the sum of chains that ran side by side, in pairs
+template <int C>
+__device__ __forceinline__ ret_f32x16 ret_chain_sum(const ret_f32x16 (&chain)[C]) {
+    static_assert(C == 1 || C % 2 == 0, "pairs");
+    if constexpr (C == 1) return chain[0];
+    else {
+        ret_f32x16 half[C / 2];
+#pragma unroll
+        for (int c = 0; c < C / 2; ++c)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) half[c][r] = chain[2 * c][r] + chain[2 * c + 1][r];
+        return ret_chain_sum(half);
+    }
+}
+
 // NQ: 8-value pieces of a query (N <= 8 NQ); PT: fragments of 32 columns a wave.  The four waves are two query tiles of 32 by two
 // column ranges; a query lies in registers (16-byte pieces 2 t + l / 32 of row l % 32), keys and values in LDS.
 template <int NQ, int PT, bool VAR>
@@ -703,10 +718,11 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
     }
     if (it * 32 >= ntok || pc >= vdim) return;
     [[maybe_unused]] const double ci = VAR ? cum[i] : 0.0;
-    // VAR: a sum of sixty-four steps of the matrix cores is taken as four (of the products with V: two) side by side, which
-    // halves what it loses to rounding: with one, y was 2.4e-7 off the float64 result where the recurrence token by token is
-    // 8.2e-8 off, with these 8.1e-8
-    constexpr int CH = VAR ? 4 : 1, CV = VAR ? 2 : 1;
+    // VAR: the long sums are taken as several side by side, and those of more than 128 state values in four shares one after
+    // the other as well, so that no output is further from the float64 result than the recurrence token by token leaves it
+    // (400 tokens, relative errors of y, token by token / in one chain / so: 48 heads of 64 columns and 128 values
+    // 8.17e-8 / 2.4e-7 / 7.58e-8, 32 heads of 128 and 256 values 8.38e-8 / - / 8.16e-8, with four chains 9.6e-8).
+    constexpr int CH = VAR ? (NQ > 16 ? 4 : 8) : 1, SH = VAR && NQ > 16 ? 4 : 1, CM = VAR ? 4 : 1, CV = VAR ? 2 : 1;
     ret_f32x16 out[PT][CV];
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt)
@@ -715,25 +731,25 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
 #pragma unroll
             for (int r = 0; r < 16; ++r) out[pt][v][r] = 0.f;
     for (int jt = 0; jt <= it; ++jt) {
-        ret_f32x16 part[CH];                           // keys as rows, the wave's queries as columns
-#pragma unroll
-        for (int e = 0; e < CH; ++e)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) part[e][r] = 0.f;
         const float* krow = sK + (jt * 32 + ql) * KS + 4 * h;
+        ret_f32x16 share[SH];                          // keys as rows, the wave's queries as columns
 #pragma unroll
-        for (int t = 0; t < NQ; ++t) {
-            const float4 k = *reinterpret_cast<const float4*>(krow + 8 * t);
-            part[0 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.x, q[t].x, part[0 % CH], 0, 0, 0);
-            part[1 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.y, q[t].y, part[1 % CH], 0, 0, 0);
-            part[2 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.z, q[t].z, part[2 % CH], 0, 0, 0);
-            part[3 % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(k.w, q[t].w, part[3 % CH], 0, 0, 0);
-        }
-        ret_f32x16 sc = part[0];
-        if constexpr (VAR) {
+        for (int s = 0; s < SH; ++s) {
+            ret_f32x16 part[CH];
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sc[r] = (part[0][r] + part[1][r]) + (part[2][r] + part[3][r]);
+            for (int e = 0; e < CH; ++e)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) part[e][r] = 0.f;
+#pragma unroll
+            for (int t = s * (NQ / SH); t < (s + 1) * (NQ / SH); ++t) {
+                const float4 k = *reinterpret_cast<const float4*>(krow + 8 * t);
+                const float ks[4] = {k.x, k.y, k.z, k.w}, qs[4] = {q[t].x, q[t].y, q[t].z, q[t].w};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) part[(4 * t + e) % CH] = __builtin_amdgcn_mfma_f32_32x32x2f32(ks[e], qs[e], part[(4 * t + e) % CH], 0, 0, 0);
+            }
+            share[s] = ret_chain_sum(part);
         }
+        ret_f32x16 sc = ret_chain_sum(share);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int j = jt * 32 + 8 * (r >> 2) + 4 * h + (r & 3), d = i - j;
@@ -753,12 +769,12 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
     int col[PT];
 #pragma unroll
     for (int pt = 0; pt < PT; ++pt) col[pt] = pc + 32 * pt + ql < vdim ? pc + 32 * pt + ql : vdim - 1;     // (a column past the last is not written)
-    ret_f32x16 more[VAR ? PT : 1][VAR ? CH : 1];
+    ret_f32x16 more[VAR ? PT : 1][CM];
     if constexpr (VAR) {
 #pragma unroll
         for (int pt = 0; pt < PT; ++pt)
 #pragma unroll
-            for (int e = 0; e < CH; ++e)
+            for (int e = 0; e < CM; ++e)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) more[pt][e][r] = 0.f;
     }
@@ -777,24 +793,28 @@ __global__ __launch_bounds__(256, VAR && PT == 1 && NQ <= 16 ? 2 : 1) void reten
         for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int pt = 0; pt < PT; ++pt) {
-                if constexpr (VAR) more[pt][e] = __builtin_amdgcn_mfma_f32_32x32x2f32(qs[e], sv[e][pt], more[pt][e], 0, 0, 0);
+                if constexpr (VAR) more[pt][(4 * t + e) % CM] = __builtin_amdgcn_mfma_f32_32x32x2f32(qs[e], sv[e][pt], more[pt][(4 * t + e) % CM], 0, 0, 0);
                 else out[pt][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(qs[e], sv[e][pt], out[pt][0], 0, 0, 0);
             }
     }
 #pragma unroll
-    for (int pt = 0; pt < PT; ++pt)
+    for (int pt = 0; pt < PT; ++pt) {
+        const ret_f32x16 sum = ret_chain_sum(out[pt]);
+        ret_f32x16 begun = sum;
+        if constexpr (VAR) begun = ret_chain_sum(more[pt]);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int row = it * 32 + 8 * (r >> 2) + 4 * h + (r & 3), p = pc + 32 * pt + ql;
             if (row < ntok && p < vdim) {
-                float v = out[pt][0][r];
+                float v = sum[r];
                 if constexpr (VAR) {
-                    v = fmaf(expf((float)cum[row]), (more[pt][0][r] + more[pt][1][r]) + (more[pt][2][r] + more[pt][3][r]), out[pt][0][r] + out[pt][1][r]);
+                    v = fmaf(expf((float)cum[row]), begun[r], v);
                     if (Dw) v = fmaf(Dw[head], sV[row * VB + p - p0], v);
                 }
                 y[(size_t)(t0 + row) * y_stride + (size_t)head * vdim + p] = v;
             }
         }
+    }
     if (spoilt)
 #pragma unroll
         for (int pt = 0; pt < PT; ++pt)
@@ -933,7 +953,10 @@ extern "C" int li_ssm_scan(const float* xbc, long xbc_stride, const float* dt_ra
     const bool aligned = ((uintptr_t)state | (uintptr_t)y | (uintptr_t)carry) % 16 == 0 && y_stride % 4 == 0;
     if (chunked && aligned && Q == RET_Q && N % 4 == 0 && vdim % 4 == 0 && xbc_stride % 4 == 0 && ((uintptr_t)xbc % 16) == 0) {
         const RetDecay dc{fixed_a, fixed_dt, dt_raw, dt_stride, dt_bias, A_log};
-        if (!fixed_a)
+        // Narrow heads with many state values stay token by token (in chunks side by side): a column's sums are spread over
+        // eight or sixteen lanes there, whose short shares lose less than the products' chains (errors of y, 16 columns
+        // and 252 values 7.8e-8 against 8.1e-8 as products, 20 and 128 7.44e-8 / 7.55e-8; at 2 to 3 times the products' time).
+        if (!fixed_a && (vdim > 32 || N <= 32))
             return retention_launch<true>(xbc, xbc_stride, state, slots, q_start, q_len, chunk_tab, carry, decay, y, y_stride, heads, G, vdim, N,
                                           segs, max_chunks, dc, Dw, silu_in, stream);
         if (G == heads && !Dw)

@@ -1252,9 +1252,11 @@ def test_recurrences_of_a_decoding_step(ops, kind, n, heads, vdim, n_state, grou
 
 @pytest.mark.parametrize("lens,heads,vdim,n_state,groups,skip_d", [
     ([65], 6, 64, 128, 2, False),                # a chunk and one token
-    ([64, 1, 130, 7], 4, 20, 100, 4, False),     # one whole chunk, one token, a short last chunk, less than a chunk; values that fill no fragment
+    ([64, 1, 130, 7], 4, 36, 100, 4, False),     # one whole chunk, one token, a short last chunk, less than a chunk; values that fill no fragment
+    ([64, 1, 130, 7], 4, 20, 100, 4, False),     # ... narrow heads with many state values: token by token in chunks
     ([200, 190], 3, 68, 24, 1, True),            # columns over a second block; no term of x
     ([96], 2, 8, 256, 2, False),
+    ([96], 2, 72, 252, 2, False),                # four shares of the state values, the last one cut
     ([70], 4, 6, 30, 2, False),                  # not in 16-byte pieces: token by token in chunks
 ])
 def test_state_space_recurrence_of_long_portions(ops, lens, heads, vdim, n_state, groups, skip_d):
@@ -1371,6 +1373,40 @@ def test_state_space_recurrence_of_long_portions_with_decays_of_zero(ops, a_log,
             got = y[o:o + L].view(L, heads, vdim)[:, h]
             assert rel(got, want[:, h].numpy()) < 8 * math.sqrt(2 * n_state + 128) * 2.0 ** -24, (i, h)
             assert rel(dev_state[i, h], S[h].numpy()) < 8 * math.sqrt(2 * n_state + 128) * 2.0 ** -24, (i, h)
+
+
+@pytest.mark.parametrize("vdim,n_state", [(64, 128), (128, 256), (36, 100), (64, 132), (16, 252), (8, 128), (32, 36), (32, 32)])
+def test_state_space_recurrence_of_long_portions_is_as_exact_as_token_by_token(ops, vdim, n_state):
+    """The rule that takes long portions as matrix products, against the form it replaces (which rows that do not lie in
+    16-byte pieces still take): no further from the float64 result."""
+    import types
+    T, heads, groups = 200, 32, 4
+    inner, width = heads * vdim, heads * vdim + 2 * groups * n_state
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    ctx = types.SimpleNamespace(num_tokens=T, num_segments=1, max_q_len=T, host_state_slots=np.zeros(1, dtype=np.int32),
+                                state_slots=dev([0]), q_start=dev([0]), q_len=dev([T]))
+    g = torch.Generator(device=DEV).manual_seed(71)
+    R = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    rows, dt, state = torch.nn.functional.silu(R(T, width)), R(T, heads), R(1, heads, n_state, vdim) * 0.1
+    bias, a_log, d = R(heads) * 0.1 - 3.0, 2.0 * torch.rand(heads, generator=g, device=DEV), R(heads)
+    step = torch.nn.functional.softplus(dt.double() + bias.double())
+    decay = torch.exp(-a_log.double().exp() * step)
+    x, b, c = rows.double().split([inner, groups * n_state, groups * n_state], dim=1)
+    x = x.view(T, heads, vdim)
+    b, c = (v.view(T, groups, n_state).repeat_interleave(heads // groups, 1) for v in (b, c))
+    S, want = state[0].double(), []
+    for t in range(T):
+        S = decay[t][:, None, None] * S + (step[t][:, None] * b[t])[:, :, None] * x[t][:, None]
+        want.append((S * c[t][:, :, None]).sum(1) + d.double()[:, None] * x[t])
+    want = torch.stack(want).view(T, inner)
+    wide = torch.zeros(T, width + 1, device=DEV)
+    wide[:, :width] = rows
+    errors = []
+    for xbc in (rows, wide[:, :width]):
+        s, y = state.clone(), torch.empty(T, inner, device=DEV)
+        ops.ssm_scan(xbc, dt, bias, a_log, d, s, ctx, y, heads, vdim, n_state, groups, _Lender())
+        errors.append([float((v.double() - w).norm() / w.norm()) for v, w in ((y, want), (s[0], S))])
+    assert all(product <= 1.01 * tokens for product, tokens in zip(*errors)), errors
 
 
 @pytest.mark.parametrize("act", ["relu2", "gelu_tanh", "gelu", "xielu"])
