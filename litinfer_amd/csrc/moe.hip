@@ -616,11 +616,15 @@ __global__ __launch_bounds__(256) void moe_linear_rows_kernel(const bf16_t* __re
 // A decoding step of a batch: few rows an expert, and every tile streams its expert's matrix, so the product is bound by
 // how many bytes of the matrices are on their way.  A block takes a tile and 16 NT outputs; its four waves take K in
 // chunks of 128 in turn, each with the loads of its NEXT chunk (16 bytes a lane, 64 neighbouring bytes of a matrix row an
-// instruction; whole chunks without conditions) in flight while it multiplies one, and add up through LDS in wave order.
+// instruction; whole chunks without conditions) in flight while it multiplies one, and add up through LDS.
 // v_mfma_f32_16x16x32_bf16 has the matrix as the row operand and 16 of the tile's rows as the column operand, so a lane
 // ends with four neighbouring outputs of one row; a tile of more than 16 rows is gone through twice (the block's share
 // of the matrix is in the L2 by then).  The rows are read 256 neighbouring bytes of a row at a time and turned into the
 // operand's order through a piece of LDS of the wave's own, as in the few-row product of a dense layer.
+// The matrix cores lose more on the way to a long sum than the vector ALU (in one chain a wave 1.14e-7 of a result at K =
+// 1,536, 2.0e-7 at 4,736, where the kernel of few rows loses 7.2e-8 and 8.7e-8), so none of their sums is longer than 32
+// k-values: a chunk's four are added in pairs to one of two running sums, and so are the waves' (7.1e-8 and 8.0e-8, in the
+// same time).
 #define MS_CHUNK 128
 template <bool EXT, typename TO, int NT>
 __global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __restrict__ a, long a_stride, const int* __restrict__ row_token,
@@ -646,6 +650,8 @@ __global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __
     }
     const int nfull = K / MS_CHUNK, nchunks = (K + MS_CHUNK - 1) / MS_CHUNK;
     const moe_frag8 zero = {};
+    constexpr std::integral_constant<int, 0> FIRST{};
+    constexpr std::integral_constant<int, 1> SECOND{};
     for (int rc = 0; rc < nr; rc += 16) {
         const bf16_t* xrow[4];                // this lane's rows of x: g + 4 i, the last one repeated past the tile's end
 #pragma unroll
@@ -653,9 +659,11 @@ __global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __
             const int r = r0 + (rc + g + 4 * i < nr ? rc + g + 4 * i : nr - 1);
             xrow[i] = a + (size_t)(row_token ? row_token[r] : r) * a_stride + 8 * r16;
         }
-        moe_f32x4 acc[NT];
+        moe_f32x4 acc[NT][2];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[nt] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+            for (int b = 0; b < 2; ++b) acc[nt][b] = moe_f32x4{0.f, 0.f, 0.f, 0.f};
         moe_frag8 wbuf[2][NT][4], xbuf[2][4];
         auto load_chunk = [&](int c, moe_frag8 (*wd)[4], moe_frag8* xd, auto tail_tag) {
             constexpr bool TAIL = decltype(tail_tag)::value;
@@ -673,18 +681,21 @@ __global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __
                     else wd[nt][j].raw = *reinterpret_cast<const uint4*>(wrow[nt] + kb + 32 * j);
                 }
         };
-        auto multiply = [&](moe_frag8 (*wa)[4], moe_frag8* xd) {
+        auto multiply = [&](moe_frag8 (*wa)[4], moe_frag8* xd, auto buf_tag) {
             __builtin_amdgcn_wave_barrier();  // (a wave's LDS instructions are carried out in order; keep the compiler's too)
 #pragma unroll
             for (int i = 0; i < 4; ++i) *reinterpret_cast<uint4*>(&xs[xslot(g + 4 * i, r16)]) = xd[i].raw;
             __builtin_amdgcn_wave_barrier();
             moe_frag8 xa[4];
+            moe_f32x4 part[NT][4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) xa[j].raw = *reinterpret_cast<const uint4*>(&xs[xslot(r16, g + 4 * j)]);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[nt][j].v, xa[j].v, acc[nt], 0, 0, 0);
+                for (int j = 0; j < 4; ++j) part[nt][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[nt][j].v, xa[j].v, moe_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[nt][decltype(buf_tag)::value] += (part[nt][0] + part[nt][1]) + (part[nt][2] + part[nt][3]);
             __builtin_amdgcn_wave_barrier();
         };
         // Nothing about the loads inside the loop is conditional: it runs while both of a turn's loads exist, and the one or
@@ -694,27 +705,25 @@ __global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __
             load_chunk(c, wbuf[0], xbuf[0], std::false_type{});
             for (; c + 2 * WAVES < nfull; c += 2 * WAVES) {
                 load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
-                multiply(wbuf[0], xbuf[0]);
+                multiply(wbuf[0], xbuf[0], FIRST);
                 load_chunk(c + 2 * WAVES, wbuf[0], xbuf[0], std::false_type{});
-                multiply(wbuf[1], xbuf[1]);
+                multiply(wbuf[1], xbuf[1], SECOND);
             }
             const bool more = c + WAVES < nfull;
             if (more) load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
-            multiply(wbuf[0], xbuf[0]);
-            if (more) multiply(wbuf[1], xbuf[1]);
+            multiply(wbuf[0], xbuf[0], FIRST);
+            if (more) multiply(wbuf[1], xbuf[1], SECOND);
         }
         if (nfull < nchunks && wave == nfull % WAVES) {      // the chunk that K ends in
             load_chunk(nfull, wbuf[0], xbuf[0], std::true_type{});
-            multiply(wbuf[0], xbuf[0]);
+            multiply(wbuf[0], xbuf[0], FIRST);
         }
         if (rc) __syncthreads();              // the sums of the 16 rows before have been read
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) red[wave][nt][lane] = acc[nt];
+        for (int nt = 0; nt < NT; ++nt) red[wave][nt][lane] = acc[nt][0] + acc[nt][1];
         __syncthreads();
         if (wave < NT) {                      // wave nt writes the 16 outputs of column tile nt
-            moe_f32x4 s = red[0][wave][lane];
-#pragma unroll
-            for (int v = 1; v < WAVES; ++v) s += red[v][wave][lane];
+            const moe_f32x4 s = (red[0][wave][lane] + red[1][wave][lane]) + (red[2][wave][lane] + red[3][wave][lane]);
             const int row = rc + r16, col = j0 + 16 * wave + 4 * g;
             if (row < nr && col < n_out)
                 moe_store4<EXT>(out + (size_t)(r0 + row) * out_stride, col, s[0], s[1], s[2], s[3], ep, moe_row_factor<EXT>(ep, r0 + row));

@@ -1193,6 +1193,23 @@ def test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, weigh, g
     assert rel(out, y.numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
 
 
+@pytest.mark.parametrize("k", [128, 512, 1160, 1536, 4736])
+def test_routed_product_of_a_decoding_batch_is_as_exact_as_of_few_rows(ops, k):
+    """No further from the float64 result than the same rows four at a time, which another kernel takes."""
+    g = torch.Generator(device=DEV).manual_seed(72)
+    rows, n_out = 20, 1024
+    a = torch.randn(rows, k, generator=g, device=DEV).to(torch.bfloat16)
+    w = (torch.randn(2, n_out, k, generator=g, device=DEV) / math.sqrt(k)).to(torch.bfloat16)
+    plan = lambda *tiles: torch.tensor([len(tiles), 0, 0, 0] + [v for t in tiles for v in t + (0,)], dtype=torch.int32, device=DEV)
+    batch, few = torch.empty(rows, n_out, device=DEV), torch.empty(rows, n_out, device=DEV)
+    ops.moe_linear(a, None, w, plan((0, 0, 12), (1, 12, 8)), 2, batch, rows)
+    for r in range(0, rows, 4):
+        ops.moe_linear(a[r:r + 4], None, w, plan((int(r >= 12), 0, 4)), 1, few[r:r + 4], 4)
+    want = torch.cat([a[:12].double() @ w[0].double().t(), a[12:].double() @ w[1].double().t()])
+    error = [float((v.double() - want).norm()) for v in (batch, few)]
+    assert error[0] < 1.03 * error[1], error               # (equal ones differ by 1 / sqrt(2 x 20,480) of themselves)
+
+
 def _one_token_batch(n):
     import types
     at = np.arange(n, dtype=np.int32)
