@@ -13,7 +13,8 @@
 #define MOE_NARROW_BYTES (16l << 20)   // a decoding step's tiles against matrices below this size take 64 columns a block: more blocks, filled more evenly (1.5B sizes 38 -> 32 us; 7B sizes 138 against 155 us)
 #define MOE_FEW_ROWS 32        // rows of a step up to which every row may be a matrix-vector product of its own,
 #define MOE_VECTOR_ROWS 4      // ... and up to which it is one also where the kernel that streams the matrices could take them
-#define MOE_STREAM_ROWS_A_TILE 12  // rows a tile, on average, up to which that kernel is taken (see moe_linear_launch)
+#define MOE_STREAM_ROWS 10         // rows an expert, on average, up to which that kernel is taken (see moe_streams),
+#define MOE_STREAM_ROWS_LARGE 12   // ... and against matrices of MOE_NARROW_BYTES and more
 
 // ------------------------------------------------------------------------------------------------ router
 // One block a token.  logits[e] = b[e] + sum_k W[e, k] x[k] in float32 (a wave an expert, in turns); the `top`
@@ -859,6 +860,26 @@ extern "C" int li_moe_linear_big_takes(int a_dtype, int w_dtype, int n_out, int 
     return a_dtype == LI_BF16 && w_dtype == LI_BF16 && K % MB_K == 0 && n_out % 32 == 0;
 }
 
+// Whether a decoding step's product takes the kernel that streams the matrices (max_tiles = rows / MOE_TILE + experts, or
+// fewer where there are fewer rows than that).  It goes through the matrix of a tile of more than 16 rows twice, so the line
+// is drawn by the rows an expert has on average.  Us a product, other kernels (matrix-vector products up to 32 rows, tiles of 32 rows with K
+// in quarters above) / this one, random choices: 16 experts of 2,240 x 1,536 4 rows 8.5 / 8.7, 8 rows 8.9 / 8.6, 32 rows
+// 26.8 / 19.7, 64 rows 30.0 / 19.7 (110 MB: 5.6 TB/s), 128 rows 30.7 / 20.8; 1,536 x 2,240 at 128 rows 27.8 / 20.8, 160 rows
+// 28.4 / 22.1, 192 rows 29.0 / 26.0, 256 rows 30.1 / 34.0; gate and up together (4,480 x 1,536) at 32 rows 40.6 / 35.0; 1,024 x
+// 1,024 at 128 rows 9.2 / 8.2, 160 rows 9.4 / 9.3, 192 rows 9.6 / 10.6; 64 experts of 768 x 1,536 at 640 rows 34.4 / 31.4;
+// 8 experts of 4,736 x 3,584 at 8 rows 29.9 / 28.0, 64 rows 84 / 43, 96 rows 86 / 46; of 3,584 x 4,736 at 10 rows 39.3 /
+// 40.1, 32 rows 58 / 42, 96 rows 57 / 49, 128 rows 59 / 69.
+// Where no more rows than experts bring 15 to 45 MB of rather long matrix rows, most tiles have one row, and the products
+// of few rows are the faster by a little (means of five draws: 128 experts of 768 x 2,048, 6 / 8 / 10 / 12 / 16 rows 6.6 /
+// 7.7 / 8.4 / 9.3 / 11.5 against 7.5 / 8.1 / 8.3 / 10.4 / 11.1 here; 64 of 768 x 1,536 5 / 8 / 12 / 20 rows 6.0 / 6.4 / 7.5 / 10.4 against 4.6 /
+// 6.3 / 7.8 / 9.5; 16 of 2,240 x 1,536 5 / 8 rows 7.9 / 12.1 against 8.3 / 10.8; 64 of 1,536 x 768 12 rows 8.6 against 7.9).
+static bool moe_streams(int rows, int max_tiles, int n_out, int K) {
+    const long experts = max_tiles - rows / MOE_TILE, bytes = 2l * n_out * K, reads = rows * bytes;
+    if (rows <= MOE_VECTOR_ROWS || (rows <= max_tiles && K >= 1280 && reads >= 15000000 && reads <= 45000000)) return false;
+    return rows <= (bytes < MOE_NARROW_BYTES ? MOE_STREAM_ROWS : MOE_STREAM_ROWS_LARGE) * experts;
+}
+extern "C" int li_moe_linear_streams(int rows, int max_tiles, int n_out, int K) { return moe_streams(rows, max_tiles, n_out, K); }
+
 template <bool EXT>
 static int moe_linear_launch(const void* a, int a_dtype, long a_stride, const int* row_token, const void* w, int w_dtype,
                              const int* plan, int max_tiles, void* out, int out_dtype, long out_stride, int n_out, int K, MoeEpilogue ep,
@@ -877,19 +898,12 @@ static int moe_linear_launch(const void* a, int a_dtype, long a_stride, const in
         return li_launch_status();
     }
     if (tile_rows != MOE_TILE) return LI_ERR_SIZE;
-    // A decoding step: each tile streams its expert's matrix.  16 experts, us a product before (matrix-vector products up to
-    // 32 rows, tiles of 32 rows with K in quarters above) and with the kernel that streams, 1.5B sizes (2,240 x 1,536):
-    // 2 rows 6.6 / 6.7, 4 rows 8.5 / 8.7, 8 rows 15.0 / 13.2, 32 rows 23.2 / 19.5, 64 rows 37.8 / 23.3 (110 MB: 4.7 TB/s),
-    // 128 rows 39.0 / 24.7, 256 rows 40.3 / 37; gate and up together (4,480) at 32 rows 42.4 / 33.6; 7B sizes (4,736 x
-    // 3,584) at 2 rows 14.1 / 14.9, 32 rows 81 / 75, 64 rows 146 / 93.5, 256 rows 155 / 136.  Above 16 rows a tile it goes
-    // through the matrix twice, so tiles of more than 12 rows on average stay with the wider ones.  Two column tiles a
-    // block (half the reads of x) from four rows a tile on: 128 rows 25.4 / 24.7, 8 rows 13.2 / 14.3.
     const bool pieces = a_dtype == LI_BF16 && w_dtype == LI_BF16 && K % 8 == 0 && a_stride % 8 == 0 &&
                         ((uintptr_t)a | (uintptr_t)w) % 16 == 0 && (out_dtype == LI_BF16 || out_dtype == LI_F32);
     const int gate2 = ep.act == 2 || ep.act == 3 ? 2 : 1;        // (a store takes four sums: two outputs where they are pairs)
-    if (pieces && rows > MOE_VECTOR_ROWS && rows <= MOE_STREAM_ROWS_A_TILE * (long)max_tiles && n_out % 4 == 0 &&
+    if (pieces && moe_streams(rows, max_tiles, n_out, K) && n_out % 4 == 0 &&
         out_stride % (4 / gate2) == 0 && (uintptr_t)out % (4 / gate2 * (out_dtype == LI_BF16 ? 2 : 4)) == 0 && max_tiles <= 65535) {
-        const bool two = rows >= 4l * max_tiles;
+        const bool two = rows >= 4l * max_tiles;         // two column tiles a block, half the reads of x: 128 rows over 16 experts 25.4 -> 24.7 us, 8 rows 13.2 -> 14.3
         const dim3 grid((n_out + (two ? 31 : 15)) / (two ? 32 : 16), max_tiles);
 #define MS(TO, NT) moe_linear_stream_kernel<EXT, TO, NT><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (TO*)out, out_stride, n_out, K, ep)
         if (out_dtype == LI_BF16) { if (two) MS(bf16_t, 2); else MS(bf16_t, 1); }

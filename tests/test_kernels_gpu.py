@@ -1184,11 +1184,11 @@ def test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, weigh, g
     elif act == 4:
         y = torch.nn.functional.gelu(y)
     plan = torch.tensor([len(tiles), rows, 0, 0] + [v for t in tiles for v in t], dtype=torch.int32)
-    plan = torch.cat([plan, torch.full((8,), -1, dtype=torch.int32)])                  # two tiles that the plan does not have
+    plan = torch.cat([plan, torch.full((16,), -1, dtype=torch.int32)])                 # four tiles that the plan does not have
     out = torch.full((rows, y.shape[1]), float("nan"), dtype=out_dtype, device=DEV)
     wide = torch.zeros(tokens, k + 8, dtype=torch.bfloat16, device=DEV)
     wide[:, :k] = a.to(DEV)
-    ops.moe_linear(wide[:, :k], src.to(torch.int32).to(DEV) if gather else None, w.to(DEV), plan.to(DEV), len(tiles) + 2, out, rows,
+    ops.moe_linear(wide[:, :k], src.to(torch.int32).to(DEV) if gather else None, w.to(DEV), plan.to(DEV), len(tiles) + 4, out, rows,
                    act=act, limit=1.5 if act == 3 else 0.0, row_wt=None if row_wt is None else row_wt.to(DEV))
     assert rel(out, y.numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
 
@@ -1208,6 +1208,19 @@ def test_routed_product_of_a_decoding_batch_is_as_exact_as_of_few_rows(ops, k):
     want = torch.cat([a[:12].double() @ w[0].double().t(), a[12:].double() @ w[1].double().t()])
     error = [float((v.double() - want).norm()) for v in (batch, few)]
     assert error[0] < 1.03 * error[1], error               # (equal ones differ by 1 / sqrt(2 x 20,480) of themselves)
+
+
+@pytest.mark.parametrize("tokens,top,experts,n_out,k,streams", [
+    (1, 4, 16, 2240, 1536, False), (1, 5, 16, 2240, 1536, False), (1, 7, 16, 2240, 1536, True), (1, 5, 16, 1536, 1024, True),
+    (1, 5, 4, 2240, 1536, True), (2, 6, 64, 768, 1536, False), (2, 3, 64, 768, 1536, True), (2, 10, 64, 768, 1536, True),
+    (40, 4, 16, 1536, 2240, True), (41, 4, 16, 1536, 2240, False), (64, 4, 16, 1536, 2240, False),
+    (96, 1, 8, 3584, 4736, True), (97, 1, 8, 3584, 4736, False), (80, 8, 64, 768, 1536, True), (81, 8, 64, 768, 1536, False),
+    (5, 2, 128, 256, 512, True),                 # fewer rows than experts
+])
+def test_which_routed_products_stream_the_matrices(ops, tokens, top, experts, n_out, k, streams):
+    import ctypes
+    takes = ops._lib_fn("moe", "li_moe_linear_streams", [ctypes.c_int] * 4, ctypes.c_int)
+    assert bool(takes(tokens * top, ops.moe_max_tiles(tokens, top, experts), n_out, k)) == streams
 
 
 def _one_token_batch(n):
