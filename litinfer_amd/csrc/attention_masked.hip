@@ -1152,11 +1152,16 @@ extern "C" int li_masked_attention_single(const float* q, int q_token_stride, in
 // the other.  x and out are addressed by a token stride and a head stride, so that a head's columns may lie inside
 // a wider row.  With `gate`, head h's outputs of token t are multiplied by sigmoid(gate[t * gate_stride + h]), or, with
 // gate_per_column, output j of head h by sigmoid(gate[t * gate_stride + h * n_out + j]).
-// A block takes one head, TOK tokens (1, 2, 4 or 8, as many as there are) and 64 outputs at a time: the tokens' inputs lie
-// in LDS as float32, four neighbouring threads share an output and read its matrix row once for all the tokens, HL_AHEAD
-// pieces of 16 bytes asked for together (one after the other, and multiplied for eight tokens whatever there were, 12 heads
-// of 128 x 256 took 12.5 us at 2 tokens, of 256 x 128 8.2; now 8.6 and 6.0).  Sums are float32, in the order of k.
+// A block takes one head, TOK tokens and 64 outputs at a time: the tokens' inputs lie in LDS as float32, four neighbouring
+// threads share an output and read its matrix row once for all the tokens.  Up to HL_FEW tokens a block takes 1, 2 or 4 of
+// them and asks for HL_AHEAD pieces of 16 bytes of the row together; above that it takes 8 and goes piece by piece, which
+// reads the matrix half as often (with pieces ahead, and stores unrolled over the tokens, eight tokens' sums take twice as
+// long).  Us, 8 tokens piece by piece whatever there are / as it is now: 12 heads of 128 x 256, float32, 2 / 8 / 16 tokens
+// 9.8 / 11.2 / 11.2 -> 6.9 / 8.5 / 8.5; 4 of 512 x 520, bfloat16, 8 tokens 20.0 -> 12.1; 28 of 512 x 128, float32, 16 tokens 8.3 -> 7.8;
+// four a block would take 15.5 there instead of 13.2 at 33 tokens, and 58.9 instead of 46.9 at 500 of 4 x 512 x 520.  Sums
+// are float32, in the order of k.
 #define HL_TOK 8
+#define HL_FEW 16
 #define HL_AHEAD 8
 
 // Behind a head's n_in inputs may lie `n` more columns that are not multiplied but ROTATED by the token's angles
@@ -1205,7 +1210,26 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
         float acc[TOK];
 #pragma unroll
         for (int tt = 0; tt < TOK; ++tt) acc[tt] = 0.f;
-        if constexpr (VEC) {
+        auto take = [&](const uint4& raw, int k) {
+            constexpr int PE = 16 / (int)sizeof(TM);
+            float wv[PE];
+            const uint32_t r4[4] = {raw.x, raw.y, raw.z, raw.w};
+            if constexpr (PE == 8) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    wv[2 * e] = __uint_as_float(r4[e] << 16);
+                    wv[2 * e + 1] = __uint_as_float(r4[e] & 0xffff0000u);
+                }
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) wv[e] = __uint_as_float(r4[e]);
+            }
+#pragma unroll
+            for (int e = 0; e < PE; ++e)
+#pragma unroll
+                for (int tt = 0; tt < TOK; ++tt) acc[tt] = fmaf(wv[e], xs[tt * n_in + k + e], acc[tt]);
+        };
+        if constexpr (VEC && TOK < HL_TOK) {
             const int pieces = n_in / E;             // (a whole number; a thread takes the pieces part, part + 4, ...)
             for (int c0 = part; c0 < pieces; c0 += 4 * HL_AHEAD) {
                 uint4 raw[HL_AHEAD];
@@ -1213,26 +1237,12 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
                 for (int u = 0; u < HL_AHEAD; ++u) raw[u] = *reinterpret_cast<const uint4*>(row + (size_t)(c0 + 4 * u < pieces ? c0 + 4 * u : pieces - 1) * E);
 #pragma unroll
                 for (int u = 0; u < HL_AHEAD; ++u) {
-                    const int k = (c0 + 4 * u) * E;
-                    if (k >= n_in) break;
-                    float wv[E];
-                    const uint32_t r4[4] = {raw[u].x, raw[u].y, raw[u].z, raw[u].w};
-                    if constexpr (sizeof(TM) == 2) {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            wv[2 * e] = __uint_as_float(r4[e] << 16);
-                            wv[2 * e + 1] = __uint_as_float(r4[e] & 0xffff0000u);
-                        }
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) wv[e] = __uint_as_float(r4[e]);
-                    }
-#pragma unroll
-                    for (int e = 0; e < E; ++e)
-#pragma unroll
-                        for (int tt = 0; tt < TOK; ++tt) acc[tt] = fmaf(wv[e], xs[tt * n_in + k + e], acc[tt]);
+                    if ((c0 + 4 * u) * E >= n_in) break;
+                    take(raw[u], (c0 + 4 * u) * E);
                 }
             }
+        } else if constexpr (VEC) {
+            for (int k = part * E; k < n_in; k += 4 * E) take(*reinterpret_cast<const uint4*>(row + k), k);
         } else {
             for (int k = part; k < n_in; k += 4) {
                 const float wv = load_as_float(row + k);
@@ -1245,14 +1255,21 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
             acc[tt] += __shfl_xor(acc[tt], 1, LI_WAVE);
             acc[tt] += __shfl_xor(acc[tt], 2, LI_WAVE);
         }
-        if (on && part == 0)
+        auto store = [&](int tt) {
+            const float gv = gate_per_column ? gate[(size_t)(t0 + tt) * gate_stride + (size_t)h * n_out + j] : gf[tt];
+            const float f = gate ? 1.0f / (1.0f + expf(-gv)) : 1.0f;
+            store_from_float(out + (size_t)(t0 + tt) * o_token_stride + (size_t)h * o_head_stride + j, acc[tt] * f);
+        };
+        if (!on || part) continue;
+        if constexpr (TOK < HL_TOK) {
 #pragma unroll
             for (int tt = 0; tt < TOK; ++tt) {
                 if (tt >= nt) break;
-                const float gv = gate_per_column ? gate[(size_t)(t0 + tt) * gate_stride + (size_t)h * n_out + j] : gf[tt];
-                const float f = gate ? 1.0f / (1.0f + expf(-gv)) : 1.0f;
-                store_from_float(out + (size_t)(t0 + tt) * o_token_stride + (size_t)h * o_head_stride + j, acc[tt] * f);
+                store(tt);
             }
+        } else {
+            for (int tt = 0; tt < nt; ++tt) store(tt);
+        }
     }
 }
 
@@ -1357,7 +1374,7 @@ extern "C" int li_headwise_linear(const void* x, int x_dtype, long x_token_strid
         else if (x_dtype == LI_BF16 && out_dtype == LI_F32) took = headwise_mfma<bf16_t, float>(x, x_token_stride, x_head_stride, m, out, o_token_stride, o_head_stride, T_, nh, n_out, n_in, gate, gate_stride, gate_per_column, tail, stream);
         if (took) return li_launch_status();
     }
-    const int zs = (n_out + 63) / 64, tok = T_ <= 1 ? 1 : T_ <= 2 ? 2 : T_ <= 4 ? 4 : HL_TOK;
+    const int zs = (n_out + 63) / 64, tok = T_ <= 1 ? 1 : T_ <= 2 ? 2 : T_ <= HL_FEW ? 4 : HL_TOK;
     const dim3 grid((T_ + tok - 1) / tok, nh, zs < 64 ? zs : 64);
     const size_t lds = (size_t)tok * n_in * 4;
 #define HL_AS(TX, TM, TO, VEC, TOK)                                                                                        \

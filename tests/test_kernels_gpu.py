@@ -1223,6 +1223,26 @@ def test_which_routed_products_stream_the_matrices(ops, tokens, top, experts, n_
     assert bool(takes(tokens * top, ops.moe_max_tiles(tokens, top, experts), n_out, k)) == streams
 
 
+@pytest.mark.parametrize("tokens", [1, 2, 3, 5, 8, 16, 17, 40])        # 1, 2, 4 and 8 tokens a block, whole and cut
+@pytest.mark.parametrize("heads,n_out,n_in", [(3, 70, 520), (2, 130, 256), (2, 64, 264), (1, 5, 36)])      # trips of 256 bfloat16 or 128 float32 inputs, whole, cut and one piece over
+@pytest.mark.parametrize("kind", ["float32", "bfloat16", "to_float32"])
+@pytest.mark.parametrize("gated", [None, "heads", "columns"])
+def test_per_head_products_of_few_tokens(ops, tokens, heads, n_out, n_in, kind, gated):
+    g = torch.Generator().manual_seed(73)
+    dt = torch.float32 if kind == "float32" else torch.bfloat16
+    x = torch.randn(tokens, heads, n_in, generator=g).to(dt)
+    m = (torch.randn(heads, n_out, n_in, generator=g) / math.sqrt(n_in)).to(dt)
+    gate = None if gated is None else torch.randn(tokens, heads * (1 if gated == "heads" else n_out), generator=g)
+    want = (x.double()[:, :, None, :] * m.double()[None]).sum(-1)
+    if gate is not None:
+        want = want * torch.sigmoid(gate.double()).view(tokens, heads, -1)
+    out = torch.full((tokens, heads * n_out), float("nan"), dtype=torch.bfloat16 if kind == "bfloat16" else torch.float32, device=DEV)
+    ops.headwise_linear(x.view(tokens, -1).to(DEV), heads * n_in, n_in, m.to(DEV), out, heads * n_out, n_out, tokens,
+                        gate=None if gate is None else gate.to(DEV), gate_columns=gated == "columns")
+    # sums of n_in exact products (of rounded ones in float32), or the rounding to bfloat16
+    assert rel(out, want.reshape(tokens, -1).numpy()) < (8e-3 if kind == "bfloat16" else 8 * math.sqrt(n_in) * 2.0 ** -24)
+
+
 def _one_token_batch(n):
     import types
     at = np.arange(n, dtype=np.int32)
