@@ -336,7 +336,7 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
     // columns 0 .. 7 and 16 .. 31 in 8 .. 15, so that no lane loads a row or a column that another one has; the two
     // quarters of the result that pair a half with itself are the sums, the other two are left.  (A matrix of few columns
     // has few of them a block, six of 1,536 on 256 units: of sixteen lanes' loads ten brought what others had.  3 rows
-    // x 1,536 x 8,960, 55 MB, 22.4 -> 17.3 us.)
+    // x 1,536 x 8,960, 55 MB, 22.9 -> 14.8 us.)
     static_assert(!SWIGLU || TILES % 2 == 0, "gate and up tiles in pairs");
     static_assert(!PACK || (!SWIGLU && TILES == 1 && RT == 1), "one tile");
     constexpr int UN = PACK ? 1 : 2;                          // loads a piece
@@ -489,7 +489,10 @@ static int launch_f32_rows(const float* x, const float* w, const float* bias, fl
     // pieces a trip: a long K keeps four a wave in flight, a short one two (measured: 3,584 columns 136 against
     // 156 us for the 7B's gate/up matrix, 18,944 columns 68.6 against 74.0 us for its way back), a tiny one, and
     // many rows (whose registers hold the rows' pieces too), one.  At most 8 rows and 8 columns a block: both halves of a
-    // piece in one load, and so twice the pieces in the same registers (K = 8,960 22.4 -> 17.3 us, K = 1,536 5.5 either way)
+    // piece in one load, and four pieces a trip for up to four rows over a long K or one of whole trips, else one (us with
+    // the matrices in memory, halves in turn / packed with one / four: 3 rows x 1,536 x 1,536 5.7 / 5.0 / 5.5, x 1,536 x 8,960
+    // 22.9 / 15.9 / 14.8, x 2,048 x 2,048 6.8 / 6.0 / 5.8, x 2,048 x 1,024 5.0 / 4.5 / 4.3; 4 rows x 1,536 x 4,096 10.7 / 8.6 /
+    // 8.1; 8 rows x 1,536 x 1,536 5.9 / 5.3 / 6.4, x 1,536 x 8,960 24.7 / 17.1 / 18.3)
 #define LI_F32RM(AH, TL, RTV, ...) gemm_f32_rows_mfma_kernel<AH, TL, RTV, __VA_ARGS__><<<grid, F32RM_WAVES * 64, 0, stream>>>(x, w, bias, out, M, N, K, accumulate, cols, limit)
     const int ahead = rt == 4 ? 1 : K >= 8192 && rt == 1 ? 4 : K >= 32 * F32RM_WAVES * 4 ? 2 : 1;
     if (swiglu) {
@@ -501,7 +504,7 @@ static int launch_f32_rows(const float* x, const float* w, const float* bias, fl
     if (rt == 1) {
         if (tiles == 2) { if (ahead == 4) LI_F32RM(4, 2, 1, false); else if (ahead == 2) LI_F32RM(2, 2, 1, false); else LI_F32RM(1, 2, 1, false); }
         else if (M <= 8 && cols <= 8) {
-            if (K >= 8192) LI_F32RM(8, 1, 1, false, true); else if (ahead == 2) LI_F32RM(4, 1, 1, false, true); else LI_F32RM(1, 1, 1, false, true);
+            if (M <= 4 && (K >= 2048 || K % 1024 == 0)) LI_F32RM(4, 1, 1, false, true); else LI_F32RM(1, 1, 1, false, true);
         } else { if (ahead == 4) LI_F32RM(4, 1, 1, false); else if (ahead == 2) LI_F32RM(2, 1, 1, false); else LI_F32RM(1, 1, 1, false); }
     } else if (rt == 2) {
         if (tiles == 2) { if (ahead >= 2) LI_F32RM(2, 2, 2, false); else LI_F32RM(1, 2, 2, false); }

@@ -226,6 +226,9 @@ def test_float32_linear_with_k_in_parts(ops, m, n, k, bias, factor):
     (1, 5, 4, True, 1.0),                    # one column a block, a single 16-byte piece a row
     (7, 300, 20, False, 0.0),                # the second half of the only piece is cut
     (8, 257, 8212, True, 1.0),               # the last piece ends inside its second half
+    (4, 300, 2052, False, 1.0),              # four pieces a trip: one trip and a piece of its own half over
+    (5, 300, 2052, False, 0.0),              # ... a row more: one piece a trip
+    (2, 100, 4096, True, 0.5),
 ])
 def test_float32_linear_of_few_rows_and_columns(ops, m, n, k, bias, factor):
     g = torch.Generator().manual_seed(63)
