@@ -390,10 +390,12 @@ __device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int
 // e_ties = their mass together; not cut: all keys): tp = the largest key c with mass(keys >= c) >=
 // `remaining`, four bits a pass (masses by the next digit); on return `remaining` is what the keys
 // equal to tp have to bring.  m: the maximum that masses are taken against.
-// Digits in which the smallest survivor (`low`: a key that no survivor is below, tau where cut) and the maximum agree are
-// taken as they are, and once a single key is left that agrees with the digits found, it is tp: a digit of which all mass
-// is left changes neither `remaining` nor the choice.  64 rows, top-k 50 with top-p 0.9: rows kernel 40 -> 25 us.
-template <typename Each>
+// Where cut, digits in which tau, which no survivor is below, and the maximum agree are taken as they are; and with LOOK,
+// once a single key is left that agrees with the digits found, it is tp: a digit of which all mass is left changes neither
+// `remaining` nor the choice.  64 rows, top-k 50 with top-p 0.9: rows kernel 40 -> 25 us.  Looking for that key is another
+// pass over `each`, so it is for keys in registers: over the row itself a pass takes as long as the one it may spare (64
+// rows, top-k 300 with top-p 0.95, logits of bfloat16's values: 762 us with it, 635 without).
+template <bool LOOK, typename Each>
 __device__ __forceinline__ void radix_mass(Each&& each, bool cut, uint32_t tau, int ties, float e_ties, float m,
                                            float& remaining, uint32_t& tp, float* work_f, float* tot_f, int* res) {
     tp = 0u;
@@ -435,7 +437,7 @@ __device__ __forceinline__ void radix_mass(Each&& each, bool cut, uint32_t tau, 
         }
         remaining -= above;
         tp |= (uint32_t)d << shift;
-        if (shift > 0 && cut && !(ties > 0 && (tau >> shift) == (tp >> shift))) {
+        if (LOOK && shift > 0 && cut && !(ties > 0 && (tau >> shift) == (tp >> shift))) {
             int left = 0;
             uint32_t one = 0u;
             each([&](float z) {
@@ -650,7 +652,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
             }
             float remaining = p * (zk + e_ties);
             uint32_t tp;
-            radix_mass(each, cut, tau, ties, e_ties, m, remaining, tp, work_f, tot_f, tot_i);
+            radix_mass<true>(each, cut, tau, ties, e_ties, m, remaining, tp, work_f, tot_f, tot_i);
             if (!by_k && total < V && !(tp > tau_c)) exact = false;       // the prefix may go on beyond the candidates
             const int need_p = ties_needed(remaining, tp, m);
             need = (cut && tp == tau) ? min(need, need_p) : need_p;
@@ -723,7 +725,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
             const float e_ties = cut ? (float)ties * expf(key_value(tau) - m) : 0.f;
             float remaining = p * (zk + e_ties);      // mass that the prefix has to reach
             uint32_t tp;
-            radix_mass(each_of_row, cut, tau, ties, e_ties, m, remaining, tp, work_f, tot_f, tot_i);
+            radix_mass<false>(each_of_row, cut, tau, ties, e_ties, m, remaining, tp, work_f, tot_f, tot_i);
             const int need_p = ties_needed(remaining, tp, m);
             need = (cut && tp == tau) ? min(need, need_p) : need_p;
             tau = tp;
