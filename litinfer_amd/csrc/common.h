@@ -54,11 +54,14 @@ __device__ __forceinline__ float xielu(float z, float sp, float sq) {
 #define LI_ACT_GELU_TANH 2
 #define LI_ACT_GELU_ERF 3
 #define LI_ACT_XIELU 4
-__device__ __forceinline__ float activation(float z, int act, float a0, float a1) {
-    if (act == LI_ACT_RELU2) { const float r = fmaxf(z, 0.f); return r * r; }
-    if (act == LI_ACT_GELU_TANH) return gelu_tanh(z);
-    if (act == LI_ACT_GELU_ERF) return gelu_erf(z);
-    return xielu(z, a0, a1);
+// (a product of gate and up columns, li_linear_swiglu: 2 up * GELU(gate), 5 the clamped form with the limit a0; 0 the plain one)
+#define LI_ACT_CLAMPED 5
+struct LiAct { int act; float a0, a1; };
+__device__ __forceinline__ float activation(float z, const LiAct& e) {
+    if (e.act == LI_ACT_RELU2) { const float r = fmaxf(z, 0.f); return r * r; }
+    if (e.act == LI_ACT_GELU_TANH) return gelu_tanh(z);
+    if (e.act == LI_ACT_GELU_ERF) return gelu_erf(z);
+    return xielu(z, e.a0, e.a1);
 }
 
 __device__ __forceinline__ float wave_sum(float v) {

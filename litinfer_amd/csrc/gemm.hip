@@ -324,7 +324,7 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
                                                                               const float* __restrict__ w,
                                                                               const float* __restrict__ bias,
                                                                               float* __restrict__ out, int M, int N, int K,
-                                                                              float accumulate, int cols, float limit) {
+                                                                              float accumulate, int cols, LiAct gated) {
     // TILES: MFMA tiles of 16 columns side by side in a block (`cols` <= 16 TILES): they share the block's
     // loads of x, which come through the same path as w (a matrix of many columns has blocks enough).
     // RT: tiles of 16 rows one above the other (M <= 16 RT): they share the block's loads of w, which is
@@ -449,11 +449,11 @@ __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(co
             float up = part[0][at + 256];
 #pragma unroll
             for (int v2 = 1; v2 < F32RM_WAVES; ++v2) up += part[v2][at + 256];
-            if (limit > 0.f) {                                  // the clamped form (see gated_bf16)
-                v = fminf(v, limit);
-                up = fminf(fmaxf(up, -limit), limit);
+            if (gated.act == LI_ACT_CLAMPED) {                  // (see gated_bf16)
+                v = fminf(v, gated.a0);
+                up = fminf(fmaxf(up, -gated.a0), gated.a0);
                 out[(size_t)row * N + n0 + j] = (up + 1.0f) * (v / (1.0f + expf(-1.702f * v)));
-            } else if (limit < 0.f) {
+            } else if (gated.act == LI_ACT_GELU_TANH) {
                 out[(size_t)row * N + n0 + j] = up * gelu_tanh(v);
             } else {
                 out[(size_t)row * N + n0 + j] = up * (v / (1.0f + expf(-v)));
@@ -470,7 +470,7 @@ static int compute_units();
 
 // swiglu: w is [gate; up] of N rows each and out [M, N] gets the activation (no bias, no accumulation)
 static int launch_f32_rows(const float* x, const float* w, const float* bias, float* out, int M, int N, int K,
-                           float accumulate, hipStream_t stream, bool swiglu = false, float limit = 0.f) {
+                           float accumulate, hipStream_t stream, bool swiglu = false, LiAct gated = {}) {
     // as many blocks as a whole number of rounds over the compute units, each with the same share of the columns;
     // two MFMA tiles side by side where 16 columns a block would not fit one round (they share the loads of x:
     // the 7B's gate/up matrix at 8 rows 136 -> 130 us)
@@ -493,7 +493,7 @@ static int launch_f32_rows(const float* x, const float* w, const float* bias, fl
     // the matrices in memory, halves in turn / packed with one / four: 3 rows x 1,536 x 1,536 5.7 / 5.0 / 5.5, x 1,536 x 8,960
     // 22.9 / 15.9 / 14.8, x 2,048 x 2,048 6.8 / 6.0 / 5.8, x 2,048 x 1,024 5.0 / 4.5 / 4.3; 4 rows x 1,536 x 4,096 10.7 / 8.6 /
     // 8.1; 8 rows x 1,536 x 1,536 5.9 / 5.3 / 6.4, x 1,536 x 8,960 24.7 / 17.1 / 18.3)
-#define LI_F32RM(AH, TL, RTV, ...) gemm_f32_rows_mfma_kernel<AH, TL, RTV, __VA_ARGS__><<<grid, F32RM_WAVES * 64, 0, stream>>>(x, w, bias, out, M, N, K, accumulate, cols, limit)
+#define LI_F32RM(AH, TL, RTV, ...) gemm_f32_rows_mfma_kernel<AH, TL, RTV, __VA_ARGS__><<<grid, F32RM_WAVES * 64, 0, stream>>>(x, w, bias, out, M, N, K, accumulate, cols, gated)
     const int ahead = rt == 4 ? 1 : K >= 8192 && rt == 1 ? 4 : K >= 32 * F32RM_WAVES * 4 ? 2 : 1;
     if (swiglu) {
         if (rt == 1) { if (ahead == 4) LI_F32RM(4, 2, 1, true); else if (ahead == 2) LI_F32RM(2, 2, 1, true); else LI_F32RM(1, 2, 1, true); }
@@ -867,13 +867,13 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
     return up * (gate * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
-// CLAMP: the other forms: limit > 0: g = min(gate, limit), u = clamp(up, -limit, limit), g sigmoid(1.702 g) (u + 1);
-// limit < 0: the gate through GELU in its tanh form.
-template <bool CLAMP>
-__device__ __forceinline__ float gated_bf16(float gate, float up, float limit) {
-    if constexpr (!CLAMP) return swiglu_bf16(gate, up);
-    if (limit < 0.f) return up * gelu_tanh(gate);
-    const float g = fminf(gate, limit), u = fminf(fmaxf(up, -limit), limit);
+// ACT: the other forms: the gate through GELU in its tanh form, or clamped with the limit a0: g = min(gate, a0),
+// u = clamp(up, -a0, a0), g sigmoid(1.702 g) (u + 1).
+template <bool ACT>
+__device__ __forceinline__ float gated_bf16(float gate, float up, const LiAct& ep) {
+    if constexpr (!ACT) return swiglu_bf16(gate, up);
+    if (ep.act == LI_ACT_GELU_TANH) return up * gelu_tanh(gate);
+    const float g = fminf(gate, ep.a0), u = fminf(fmaxf(up, -ep.a0), ep.a0);
     const float e = __builtin_amdgcn_exp2f(-1.702f * 1.44269504088896341f * g);
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + e));
 }
@@ -894,15 +894,15 @@ __device__ __forceinline__ void static_for(F&& f) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"                          \
                  :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(voff), "s"(base) : "memory", "m0")
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, bool CLAMP = false>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, bool ACT = false>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ w,
                                                              const float* __restrict__ bias,
                                                              TO* __restrict__ out, int M, int N, int K,
                                                              float accumulate, int nsplit,
                                                              const float* __restrict__ row_parts, int nparts, float eps,
-                                                             float limit) {
-    // limit: see gated_bf16 (SwiGLU tiles).
+                                                             LiAct ep) {
+    // ACT: the activation `ep`, of gate and up columns (gated_bf16) or of the sums.
     // row_parts (SwiGLU tiles of 64 rows, up to 32 rows of x): x is the xg of li_linear_residual_norm and these
     // are its sq_parts; every row's sums are scaled by 1 / sqrt(sum of the row's parts / K + eps) before the
     // activation, which makes the result that of the RMS norm (the factor of a row does not depend on k).
@@ -1163,7 +1163,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
                 float f = 1.0f;
                 if constexpr (ROWSCALE) f = row_parts ? row_inv[row & 31] : 1.0f;      // (row_parts: M <= 32, so row < 32 here)
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = gated_bf16<CLAMP>(gs[e] * f, us[e] * f, limit);
+                for (int e = 0; e < 8; ++e) v[e] = gated_bf16<ACT>(gs[e] * f, us[e] * f, ep);
                 const size_t o_idx = (size_t)row * NO + col;
                 if (col + 8 <= NO && (NO % 8) == 0) {
                     chunk16 o;
@@ -1204,7 +1204,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
                             uv *= f;
                         }
                     }
-                    band[(8 * (r >> 2) + crow + (r & 3)) * ESTRIDE + 16 * j + ccol] = gated_bf16<CLAMP>(gv, uv, limit);
+                    band[(8 * (r >> 2) + crow + (r & 3)) * ESTRIDE + 16 * j + ccol] = gated_bf16<ACT>(gv, uv, ep);
                 }
         } else {
 #pragma unroll
@@ -1223,9 +1223,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = src[e];
             const size_t o_idx = (size_t)row * NO + col;
-            if constexpr (CLAMP && !SWIGLU) {            // an activation of the sums (its number and its two constants where a norm's factors have theirs)
+            if constexpr (ACT && !SWIGLU) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), nparts, eps, limit);
+                for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), ep);
                 if (col + 8 <= NO && (NO % 8) == 0) {
                     chunk16 o;
 #pragma unroll
@@ -1268,10 +1268,10 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     }
 }
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, bool CLAMP = false>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, bool ACT = false>
 static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* out, int M, int N, int K,
                       float accumulate, hipStream_t stream, int nsplit = 1, const float* row_parts = nullptr,
-                      int nparts = 0, float eps = 0.f, float limit = 0.f) {
+                      int nparts = 0, float eps = 0.f, LiAct ep = {}) {
     if (row_parts && !(SWIGLU && BM == 64 && M <= 32 && nparts > 0)) return LI_ERR_SIZE;
     const long mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
     if (nsplit < 1 || nsplit > 65535 || nsplit > K / BK) return LI_ERR_SIZE;
@@ -1284,12 +1284,12 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
     constexpr int lds_bytes = NSTAGE * (BM + BN) * BK * 2;
     static bool configured = false;
     if (!configured) {
-        if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, WLM, CLAMP>,
+        if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, WLM, ACT>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
             return LI_ERR_LAUNCH;
         configured = true;
     }
-    gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, WLM, CLAMP><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, nsplit, row_parts, nparts, eps, limit);
+    gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, WLM, ACT><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, nsplit, row_parts, nparts, eps, ep);
     return li_launch_status();
 }
 
@@ -1306,7 +1306,7 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit,
 
 // out = act(sum over the parts + bias), bfloat16 (see li_linear_act)
 __global__ __launch_bounds__(256) void splitk_reduce_act_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
-                                                                const float* __restrict__ bias, bf16_t* __restrict__ out, int act, float a0, float a1) {
+                                                                const float* __restrict__ bias, bf16_t* __restrict__ out, LiAct ep) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
     float a[8];
@@ -1316,7 +1316,7 @@ __global__ __launch_bounds__(256) void splitk_reduce_act_kernel(const float* __r
 #pragma unroll
     for (int sp = 1; sp < 8; ++sp) v += sp < nsplit ? a[sp] : 0.f;
     if (bias) v += bias[(int)(i % N)];
-    store_from_float(out + i, activation(v, act, a0, a1));
+    store_from_float(out + i, activation(v, ep));
 }
 
 // The same for the residual sum, one block a row, with the RMS norm of the new sum as a second
@@ -1465,16 +1465,13 @@ struct SkinnyArgs {
     // no statistics of a row, so it is done here and sq_parts stays as it is.
     const float* beta;
     float alpha;
-    // SWIGLU with EPI 1: the other gated forms (see gated_bf16)
-    float limit;
-    // EPI 2 (bfloat16 out): out = activation(product + bias, act, a0, a1)
-    int act;
-    float a0, a1;
+    // SWIGLU with EPI 1: one of the other gated forms (see gated_bf16).  EPI 2 (bfloat16 out): out = activation(product + bias)
+    LiAct ep;
 };
 #define SK_MAX_PARTS 512            // blocks of a producing product whose sums one consumer adds up
 
 // EPI 1: with SWIGLU the other gated activations, else (float out) the tanh norm of the new sum beside it (SkinnyArgs: beta).
-// EPI 2: an activation of the sums (SkinnyArgs: act).
+// EPI 2: an activation of the sums (SkinnyArgs: ep).
 template <int MT, int NT, int WAVES, bool SWIGLU, typename TO, bool ROPE = false, int EPI = 0>
 __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs a) {
     static_assert(!ROPE || (MT <= 2 && !SWIGLU), "the rotary epilogue takes one or two tiles of rows");
@@ -1706,7 +1703,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
 #pragma unroll
             for (int wv = 1; wv < WAVES; ++wv) s += red[wv][tile][l][r];
             if (a.bias) s += a.bias[n];
-            store_from_float(out + (size_t)m * N + n, activation(s, a.act, a.a0, a.a1));
+            store_from_float(out + (size_t)m * N + n, activation(s, a.ep));
         }
         return;
     }
@@ -1769,7 +1766,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
                 const int n = n0 + 4 * (l >> 4) + r;
                 if (n < nend) {
                     const float gv = s[0][r], uv = s[NT - 1][r];
-                    store_from_float(out + (size_t)m * N + n, gated_bf16<EPI == 1>(gv, uv, a.limit));
+                    store_from_float(out + (size_t)m * N + n, gated_bf16<EPI == 1>(gv, uv, a.ep));
                 }
             }
         } else {
@@ -2306,13 +2303,12 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
                              float a1, void* work, long work_bytes, hipStream_t stream) {
     if (M <= 0 || N <= 0 || K <= 0 || act < LI_ACT_RELU2 || act > LI_ACT_XIELU) return LI_ERR_SIZE;
     if (K % 8 || (M > 64 && (K % 64 || act != LI_ACT_RELU2))) return -1;
-#define LI_ACT(BM, BN, NS, WLM) launch_dma<BM, BN, 64, NS, false, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, act, a0, a1)
+    const LiAct ep{act, a0, a1};
+#define LI_ACT(BM, BN, NS, WLM) launch_dma<BM, BN, 64, NS, false, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
     if (M <= 64 && (K % 64 || !mid_rows_take(M, N, K))) {
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
-        a.act = act;
-        a.a0 = a0;
-        a.a1 = a1;
+        a.ep = ep;
         launch_skinny<false, bf16_t, 2>(a, stream);
         return li_launch_status();
     }
@@ -2325,7 +2321,7 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
             ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit)
             : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
         if (rc != LI_OK) return rc;
-        splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, act, a0, a1);
+        splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
         return li_launch_status();
     }
     if (M <= 64) {                                   // (as linear_mid_rows takes them)
@@ -2345,21 +2341,27 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
 #undef LI_ACT
 }
 
-// The same in float32 for up to 64 rows (K a multiple of 4): the few-row product on the float32 matrix cores with
+// The gated forms: 0 the plain one, LI_ACT_GELU_TANH, LI_ACT_CLAMPED with a positive limit.
+static bool gated_form_known(int act, float limit) { return act == 0 || act == LI_ACT_GELU_TANH || (act == LI_ACT_CLAMPED && limit > 0.f); }
+
+// The gated product below in float32 for up to 64 rows (K a multiple of 4): the few-row product on the float32 matrix cores with
 // the activation in its epilogue.
-extern "C" int li_linear_swiglu_f32(const float* x, const float* w, float* out, int M, int I, int K, float limit, hipStream_t stream) {
+extern "C" int li_linear_swiglu_f32(const float* x, const float* w, float* out, int M, int I, int K, int act, float limit, hipStream_t stream) {
+    if (!gated_form_known(act, limit)) return LI_ERR_SIZE;
     if (M <= 0 || M > F32_ROWS_MAX || I <= 0 || K <= 0 || K % 4 || I > 0x3fffffff) return LI_ERR_SIZE;
     if ((((uintptr_t)x | (uintptr_t)w) & 15) != 0) return LI_ERR_SIZE;
-    return launch_f32_rows(x, w, nullptr, out, M, I, K, 0.f, stream, true, limit);
+    return launch_f32_rows(x, w, nullptr, out, M, I, K, 0.f, stream, true, LiAct{act, limit, 0.f});
 }
 
 // out[m, n] = up * gate / (1 + exp(-gate)) with [gate, up] = x w^T, w = [gate; up] of I rows each:
 // the activation as the product's epilogue, so the 2 I columns never go to memory.  bfloat16;
-// K a multiple of 8 for up to 64 rows, a multiple of 64 above.  limit not zero: the other forms (see gated_bf16).
+// K a multiple of 8 for up to 64 rows, a multiple of 64 above.  act, limit: which form (see gated_form_known and gated_bf16).
 // row_parts (may be null): x is the xg of li_linear_residual_norm and these are its sq_parts, nparts of
 // them; every row's result is that of the RMS norm with eps (up to 16 rows).
 extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, int I, int K,
-                                const float* row_parts, int nparts, float eps, float limit, hipStream_t stream) {
+                                const float* row_parts, int nparts, float eps, int act, float limit, hipStream_t stream) {
+    if (!gated_form_known(act, limit)) return LI_ERR_SIZE;
+    const LiAct ep{act, limit, 0.f};
     if (M <= 0 || I <= 0 || K <= 0 || I > 0x3fffffff) return LI_ERR_SIZE;
     const int N = 2 * I;
     if (row_parts && (M > 32 || (K % 8) || nparts <= 0 || nparts > SK_MAX_PARTS || eps < 0.f)) return LI_ERR_SIZE;
@@ -2396,25 +2398,25 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
             const double c = tile_cost(64, widths[i], 1.0, M, N, K);
             if (pick < 0 || c < best) { best = c; pick = i; }
         }
-#define LI_SW64(BN, NS) (limit != 0.f ? launch_dma<64, BN, 64, NS, true, bf16_t, 2, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, limit) \
+#define LI_SW64(BN, NS) (act ? launch_dma<64, BN, 64, NS, true, bf16_t, 2, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, ep) \
                                      : launch_dma<64, BN, 64, NS, true, bf16_t>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps))
         if (pick == 0) return LI_SW64(256, 3);
         if (pick == 1) return LI_SW64(192, 4);
         if (pick == 2) return LI_SW64(128, 4);
 #undef LI_SW64
     }
-    if (row_parts || (M <= 64 && limit != 0.f)) {
+    if (row_parts || (M <= 64 && act)) {
         if (K % 8) return LI_ERR_SIZE;
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, nullptr, out, M, I, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, row_parts, nparts, eps};
-        a.limit = limit;
-        if (limit != 0.f) launch_skinny<true, bf16_t, 1>(a, stream);
+        a.ep = ep;
+        if (act) launch_skinny<true, bf16_t, 1>(a, stream);
         else launch_skinny<true, bf16_t>(a, stream);
         return li_launch_status();
     }
     if (M <= 64) return li_linear_skinny(x, w, nullptr, out, M, I, K, LI_BF16, 0, 1, stream);
     if (K % 64) return LI_ERR_SIZE;
-#define LI_DMA(BM, BN, BK, NS, WLM) (limit != 0.f ? launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, limit) \
+#define LI_DMA(BM, BN, BK, NS, WLM) (act ? launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep) \
                                                  : launch_dma<BM, BN, BK, NS, true, bf16_t, WLM>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream))
     // (a tile's columns are gate and up columns in turn, 32 of each: its width is a multiple of 64)
     // (128 x 320: 160 gate columns in one wave, their ups in the wave beside it; for portions of a few hundred rows,

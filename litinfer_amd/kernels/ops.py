@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 import math
 from ctypes import c_float, c_int, c_long, c_void_p
-from typing import Dict, Optional
+from typing import Dict, Optional, Union
 
 import numpy as np
 import torch
@@ -84,8 +84,8 @@ _SIGNATURES = {
     "gemm": {
         "li_linear": [P, P, P, P, I, I, I, I, I, F, P, L],
         "li_linear_skinny": [P, P, P, P, I, I, I, I, F, I],
-        "li_linear_swiglu": [P, P, P, I, I, I, P, I, F, F],
-        "li_linear_swiglu_f32": [P, P, P, I, I, I, F],
+        "li_linear_swiglu": [P, P, P, I, I, I, P, I, F, I, F],
+        "li_linear_swiglu_f32": [P, P, P, I, I, I, I, F],
         "li_linear_residual_norm": [P, P, P, P, I, I, I, F, P, P, P],
         "li_linear_then_norm": [P, P, P, P, I, I, I, P, L, F, P, F, P, I],
         "li_linear_tanh_norm": [P, P, P, P, I, I, I, P, L, F, F, P, P, P, I],
@@ -1194,18 +1194,24 @@ def _check_row_scale(what: str, m: int, row_scale: Optional[RowScale]):
     return row_scale.sq_parts.data_ptr(), row_scale.nparts, row_scale.eps
 
 
-GELU_TANH_GATE = -1.0          # as `limit` of linear_swiglu: the gate through GELU in its tanh form
+GELU_TANH_GATE = "gelu_tanh"   # in place of a limit of linear_swiglu: the gate through GELU in its tanh form
+
+
+def _gated_form(limit):
+    """The kernels' number of a gated form and its limit."""
+    if limit == GELU_TANH_GATE:
+        return LINEAR_ACTS["gelu_tanh"], 0.0
+    return (5, float(limit)) if limit > 0 else (0, 0.0)
 
 
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, row_scale: Optional[RowScale] = None,
-                  limit: float = 0.0) -> None:
+                  limit: Union[float, str] = 0.0) -> None:
     """out[m, n] = up * gate / (1 + exp(-gate)) with [gate, up] = x w^T, w = [gate; up]
     (2 N rows): the activation in the product's epilogue, from the product's float32 sums.
-    With `row_scale`, x is the xg of `linear_residual_norm` and the result is that of the norm.  With `limit` > 0 the
-    clamped form: g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit); with
-    GELU_TANH_GATE: up * gelu_tanh(gate)."""
+    With `row_scale`, x is the xg of `linear_residual_norm` and the result is that of the norm.  With a `limit` > 0 the
+    clamped form: g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit); with GELU_TANH_GATE in
+    its place up * gelu_tanh(gate)."""
     _gpu(x, w, out)
-    _chk(limit >= 0 or limit == GELU_TANH_GATE, "linear_swiglu: limit")
     _chk(x.dim() == 2 and w.dim() == 2 and out.dim() == 2, "linear_swiglu: needs matrices")
     m, k = x.shape
     n = out.shape[1]
@@ -1217,11 +1223,11 @@ def linear_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, row_scale
         _chk(x.dtype is torch.float32 and out.dtype is torch.float32 and row_scale is None,
              "linear_swiglu: float32 w goes with float32 x and out, and no row scale")
         _chk(x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0, "linear_swiglu: operands must start on 16 bytes")
-        _run("gemm", "li_linear_swiglu_f32", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, float(limit))
+        _run("gemm", "li_linear_swiglu_f32", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k, *_gated_form(limit))
         return
     _chk(x.dtype is torch.bfloat16 and out.dtype is torch.bfloat16, "linear_swiglu: x and out must be bfloat16")
     _run("gemm", "li_linear_swiglu", x.data_ptr(), w.data_ptr(), out.data_ptr(), m, n, k,
-         *_check_row_scale("linear_swiglu", m, row_scale), float(limit))
+         *_check_row_scale("linear_swiglu", m, row_scale), *_gated_form(limit))
 
 
 LINEAR_ACTS = {"relu2": 1, "gelu_tanh": 2, "gelu": 3, "xielu": 4}      # the kernels' numbers (gelu: with the error function)

@@ -3,7 +3,7 @@
 mixers, feed-forwards and the head hold these."""
 from __future__ import annotations
 
-from typing import Optional
+from typing import Optional, Union
 
 import torch
 
@@ -63,12 +63,12 @@ class Linear:
         return ops.linear_act(x, self.weight, self.bias, out, act, constants, ws)
 
     def __call__(self, x: torch.Tensor, out: torch.Tensor, accumulate: bool = False, ws=None,
-                 swiglu: bool = False, row_scale=None, factor: float = 1.0, limit: float = 0.0):
+                 swiglu: bool = False, row_scale=None, factor: float = 1.0, limit: Union[float, str] = 0.0):
         """out = x W^T + b, or out += factor * (...) when `accumulate` (out is float32 then).
         With `swiglu` (only where `takes_swiglu`) W is [gate; up] and out gets
-        up * silu(gate), or with a `limit` that is not zero one of the other forms of `ops.linear_swiglu`; `row_scale` then says that x came out of `add_with_scaling`.  A matrix that is stored in 32-bit is multiplied in
-        32-bit also when the activations are bfloat16: they are widened for it,
-        exactly."""
+        up * silu(gate), or another form by `limit` (see `ops.linear_swiglu`); `row_scale` then says that x came out of
+        `add_with_scaling`.  A matrix that is stored in 32-bit is multiplied in 32-bit also when the activations are
+        bfloat16: they are widened for it, exactly."""
         if swiglu:
             ops.linear_swiglu(x, self.weight, out, row_scale=row_scale, limit=limit)
         elif self.weight.dtype is torch.float32 and x.dtype is not torch.float32:

@@ -27,7 +27,7 @@ class SwiGLUMLP(FeedForward):
             raise ValueError(f"gated feed-forward: activation {self.activation!r} (silu, gelu_tanh or clamped)")
         if (self.activation == "clamped") != (self.limit > 0):
             raise ValueError("gated feed-forward: the clamped activation takes a positive limit, the others none")
-        # which of the products' gated epilogues this is (0: silu)
+        # which of the products' gated epilogues this is (no positive limit: silu)
         self.gate_form = ops.GELU_TANH_GATE if self.activation == "gelu_tanh" else self.limit
         self.names = {"gate": "gate_proj.weight", "up": "up_proj.weight", "down": "down_proj.weight", **(spec.args.get("names") or {})}
         self.gate_up = None

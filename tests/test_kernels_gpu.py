@@ -1512,3 +1512,15 @@ def test_gated_product_with_the_tanh_form_of_gelu(ops, m, n, k):
         out = torch.full((m, n), float("nan"), device=DEV)
         ops.linear_swiglu(x.float().to(DEV), w.float().to(DEV), out, limit=ops.GELU_TANH_GATE)
         assert rel(out, want.numpy()) < 8 * math.sqrt(k) * 2.0 ** -24
+
+
+@pytest.mark.parametrize("limit", [-1.0, -2.5])
+@pytest.mark.parametrize("dtype,m", [(torch.bfloat16, 5), (torch.bfloat16, 40), (torch.bfloat16, 100), (torch.float32, 3)])
+def test_gated_product_takes_a_limit_that_is_not_positive_as_none(ops, dtype, m, limit):
+    g = torch.Generator().manual_seed(74)
+    n, k = 300, 128
+    x, w = torch.randn(m, k, generator=g).to(dtype).to(DEV), (torch.randn(2 * n, k, generator=g) * 2 / math.sqrt(k)).to(dtype).to(DEV)
+    plain, other = torch.empty(m, n, dtype=dtype, device=DEV), torch.empty(m, n, dtype=dtype, device=DEV)
+    ops.linear_swiglu(x, w, plain)
+    ops.linear_swiglu(x, w, other, limit=limit)
+    assert torch.equal(plain, other)
