@@ -168,16 +168,35 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
+def _call(module: str, name: str, args) -> int:
+    if not profiler.enabled:
+        return _fn(module, name)(*args, _stream())
+    rc = []
+
+    def launch():
+        rc.append(_fn(module, name)(*args, _stream()))
+        return rc[0] != _NOT_TAKEN
+    profiler.timed(name[3:], launch, torch.cuda.synchronize)
+    return rc[0]
+
+
 def _run(module: str, name: str, *args) -> None:
-    if profiler.enabled:
-        rc = []
-        profiler.timed(name[3:], lambda: rc.append(_fn(module, name)(*args, _stream())), torch.cuda.synchronize)
-        rc = rc[0]
-    else:
-        rc = _fn(module, name)(*args, _stream())
+    rc = _call(module, name, args)
     if rc != 0:
         raise RuntimeError(f"{name}: the kernel library refused the call (code {rc}): "
                            f"{_ERRORS.get(rc, 'unknown')}")
+
+
+_NOT_TAKEN = -1         # an entry point's answer where it has no kernel for the sizes, with nothing done
+
+
+def _try(module: str, name: str, *args) -> bool:
+    """Like `_run`, but False where the library has no kernel for these sizes."""
+    rc = _call(module, name, args)
+    if rc not in (0, _NOT_TAKEN):
+        raise RuntimeError(f"{name}: the kernel library refused the call (code {rc}): "
+                           f"{_ERRORS.get(rc, 'unknown')}")
+    return rc == 0
 
 
 _ERRORS = {1: "unsupported dtype combination", 2: "unsupported size", 3: "launch failed"}
@@ -1135,14 +1154,9 @@ def linear_then_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tens
     if m <= SKINNY_MAX_ROWS:                # one size for all row counts of a decode batch: the buffer does not move
         need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)
     buf = ws.buffer("gemm.parts", (need // 4,), torch.float32)
-    rc = _fn("gemm", "li_linear_then_norm")(x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(),
-                                             out.data_ptr(), m, n, k, buf.data_ptr(), buf.numel() * 4, float(factor), gamma.data_ptr(),
-                                             float(eps), xn.data_ptr(), _DT[xn.dtype], _stream())
-    if rc == -1:
-        return False
-    if rc != 0:
-        raise RuntimeError(f"li_linear_then_norm: the kernel library refused the call (code {rc}): {_ERRORS.get(rc, 'unknown')}")
-    return True
+    return _try("gemm", "li_linear_then_norm", x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(),
+                out.data_ptr(), m, n, k, buf.data_ptr(), buf.numel() * 4, float(factor), gamma.data_ptr(),
+                float(eps), xn.data_ptr(), _DT[xn.dtype])
 
 
 def linear_tanh_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor, alpha: float,
@@ -1172,14 +1186,9 @@ def linear_tanh_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tens
     _chk(xn.dtype in _DT and xn.shape == (m, n) and xn.is_contiguous(), "linear_tanh_norm: xn must be [M, N]")
     _chk(all(v is None or (v.dtype is torch.float32 and v.numel() == n and v.is_contiguous()) for v in (bias, gamma, beta))
          and factor != 0.0, "linear_tanh_norm: bias, gamma and beta must be float32 [N], the factor not zero")
-    rc = _fn("gemm", "li_linear_tanh_norm")(x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(),
-                                             m, n, k, work, work_bytes, float(factor), float(alpha), gamma.data_ptr(),
-                                             beta.data_ptr(), xn.data_ptr(), _DT[xn.dtype], _stream())
-    if rc == -1:
-        return False
-    if rc != 0:
-        raise RuntimeError(f"li_linear_tanh_norm: the kernel library refused the call (code {rc}): {_ERRORS.get(rc, 'unknown')}")
-    return True
+    return _try("gemm", "li_linear_tanh_norm", x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(),
+                m, n, k, work, work_bytes, float(factor), float(alpha), gamma.data_ptr(),
+                beta.data_ptr(), xn.data_ptr(), _DT[xn.dtype])
 
 
 def _check_row_scale(what: str, m: int, row_scale: Optional[RowScale]):
@@ -1256,13 +1265,8 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], o
             need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)
         buf = ws.buffer("gemm.parts", (need // 4,), torch.float32)
         work, work_bytes = buf.data_ptr(), buf.numel() * 4
-    rc = _fn("gemm", "li_linear_act")(x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(), m, n, k,
-                                      LINEAR_ACTS[act], float(constants[0]), float(constants[1]), work, work_bytes, _stream())
-    if rc == -1:
-        return False
-    if rc != 0:
-        raise RuntimeError(f"li_linear_act: the kernel library refused the call (code {rc}): {_ERRORS.get(rc, 'unknown')}")
-    return True
+    return _try("gemm", "li_linear_act", x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(), m, n, k,
+                LINEAR_ACTS[act], float(constants[0]), float(constants[1]), work, work_bytes)
 
 
 ROPE_STORE_MAX_ROWS = 32
@@ -1329,15 +1333,9 @@ def linear_rope_store_parts(x: torch.Tensor, w: torch.Tensor, bias: Optional[tor
     if m <= SKINNY_MAX_ROWS:                # one size for all row counts of a decode batch: the buffer does not move
         need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)
     buf = ws.buffer("gemm.parts", (need // 4,), torch.float32)
-    rc = _fn("gemm", "li_linear_rope_store_parts")(
-        x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(), m, kk,
-        cos.data_ptr(), sin.data_ptr(), slot_map.data_ptr(), k.data_ptr(), v.data_ptr(), nh, nkv, dh, page_size,
-        k.shape[0], buf.data_ptr(), buf.numel() * 4, _stream())
-    if rc == -1:
-        return False
-    if rc != 0:
-        raise RuntimeError(f"li_linear_rope_store_parts: the kernel library refused the call (code {rc}): {_ERRORS.get(rc, 'unknown')}")
-    return True
+    return _try("gemm", "li_linear_rope_store_parts", x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(), m, kk,
+                cos.data_ptr(), sin.data_ptr(), slot_map.data_ptr(), k.data_ptr(), v.data_ptr(), nh, nkv, dh, page_size,
+                k.shape[0], buf.data_ptr(), buf.numel() * 4)
 
 
 # ----------------------------------------------------------------- attention

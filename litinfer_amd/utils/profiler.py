@@ -43,12 +43,13 @@ class OpProfiler:
         self.calls[key] += 1
 
     def timed(self, name: str, launch, sync) -> None:
-        """Run `launch()` between two waits for the device and record it."""
+        """Run `launch()` between two waits for the device and record it, unless it returns False: nothing was launched."""
         sync()
         t = time.perf_counter()
-        launch()
+        ran = launch()
         sync()
-        self.record(name, time.perf_counter() - t)
+        if ran is not False:
+            self.record(name, time.perf_counter() - t)
 
     def report(self, out=None) -> None:
         if not self.total:

@@ -1524,3 +1524,21 @@ def test_gated_product_takes_a_limit_that_is_not_positive_as_none(ops, dtype, m,
     ops.linear_swiglu(x, w, plain)
     ops.linear_swiglu(x, w, other, limit=limit)
     assert torch.equal(plain, other)
+
+
+def test_the_profiler_sees_products_that_may_not_be_taken(ops, monkeypatch):
+    """A product with an epilogue of its own is a row of the table like any other call; one that is not taken is none."""
+    from litinfer_amd.utils import OpProfiler
+    prof = OpProfiler(False)
+    prof.enabled, prof.phase = True, "decode"
+    monkeypatch.setattr(ops, "profiler", prof)
+    bf16 = lambda *s: torch.randn(*s, device=DEV).to(torch.bfloat16)
+    out = torch.empty(4, 48, dtype=torch.bfloat16, device=DEV)
+    assert ops.linear_act(bf16(4, 64), bf16(48, 64), None, out, "gelu", ws=_Lender())
+    assert not ops.linear_act(bf16(100, 64), bf16(48, 64), None, torch.empty(100, 48, dtype=torch.bfloat16, device=DEV), "gelu", ws=_Lender())
+    m, n, k = 64, 3584, 18944
+    rows, xn = torch.zeros(m, n, device=DEV), torch.empty(m, n, dtype=torch.bfloat16, device=DEV)
+    assert ops.linear_then_norm(bf16(m, k), bf16(n, k), None, rows, torch.ones(n, device=DEV), 1e-6, xn, _Lender())
+    assert ops.linear_tanh_norm(bf16(m, k), bf16(n, k), None, rows, 0.5, torch.ones(n, device=DEV), torch.zeros(n, device=DEV), xn, _Lender())
+    assert dict(prof.calls) == {("decode", name): 1 for name in ("linear_act", "linear_then_norm", "linear_tanh_norm")}
+    assert all(v > 0 for v in prof.total.values())
