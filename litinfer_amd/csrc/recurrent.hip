@@ -598,6 +598,7 @@ __global__ __launch_bounds__(64) void retention_carry_kernel(float4* __restrict_
     const int seg = blockIdx.x, head = blockIdx.y, e = blockIdx.z * 64 + threadIdx.x;
     if (e >= NV4) return;
     const int L = q_len[seg], nch = (L + RET_Q - 1) / RET_Q;
+    if (nch <= 0) return;                              // (a request without tokens has no chunk to ask for, and its state stays)
     const float a = VAR ? 1.f : fixed_a[head], whole = VAR ? 1.f : powf(a, (float)RET_Q), tail = VAR ? 1.f : powf(a, (float)(L - (nch - 1) * RET_Q));
     const float* factors = VAR ? chunk_decay + (size_t)chunk_first[seg] * heads + head : nullptr;
     float4* at = carry + ((size_t)chunk_first[seg] * heads + head) * NV4 + e;

@@ -1384,6 +1384,36 @@ def test_recurrence_of_long_portions_keeps_values_that_are_not_finite_to_their_c
     assert torch.equal(s1[~state_reached], s0[~state_reached]) and not torch.isfinite(s1[state_reached]).any()
 
 
+@pytest.mark.parametrize("kind", ["ssm", "fixed"])
+def test_recurrence_of_long_portions_leaves_requests_without_tokens_alone(ops, kind):
+    """A request that brings no tokens, before, between and behind others: no chunk is its own, its state stays as it was, and
+    the other requests' outputs and states are those of a step without it."""
+    import types
+    g = torch.Generator().manual_seed(72)
+    R = lambda *s: torch.randn(*s, generator=g)
+    heads, vdim, n_state = 3, 36, 20
+    T, inner = 230, heads * vdim
+    dev = lambda a: torch.tensor(a, dtype=torch.int32, device=DEV)
+    state, rows, dt = R(5, heads, n_state, vdim), R(T, inner + 2 * heads * n_state).to(DEV), R(T, heads).to(DEV)
+    bias, a_log, d = R(heads).to(DEV), torch.rand(heads, generator=g).to(DEV), R(heads).to(DEV)
+    fixed = torch.linspace(0.9, 0.99, heads).to(DEV)
+
+    def run(lens, slots):
+        starts = [sum(lens[:i]) for i in range(len(lens))]
+        ctx = types.SimpleNamespace(num_tokens=T, num_segments=len(lens), max_q_len=max(lens), host_state_slots=np.array(slots, dtype=np.int32),
+                                    state_slots=dev(slots), q_start=dev(starts), q_len=dev(lens))
+        s, y = state.to(DEV), torch.zeros(T, inner, device=DEV)
+        if kind == "ssm":
+            ops.ssm_scan(rows, dt, bias, a_log, d, s, ctx, y, heads, vdim, n_state, heads, _Lender())
+        else:
+            ops.ssm_scan(rows, None, None, None, None, s, ctx, y, heads, vdim, n_state, heads, _Lender(), fixed_decay=fixed, fixed_step=0.3)
+        return y.cpu(), s.cpu()
+
+    (y0, s0), (y1, s1) = run([130, 100], [1, 3]), run([0, 130, 0, 100, 0], [0, 1, 2, 3, 4])
+    assert torch.equal(y0, y1) and torch.equal(s0, s1)
+    assert torch.equal(s1[[0, 2, 4]], state[[0, 2, 4]]) and not torch.equal(s1[1], state[1])
+
+
 @pytest.mark.parametrize("a_log,dt_raw", [
     (2.0, 100.0),            # a decay of exp(-740): zero in float32
     (60.0, 3.0),             # an exponent of 1e26, beside which the other tokens' vanish
