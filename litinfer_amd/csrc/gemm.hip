@@ -317,7 +317,9 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 // four k-slots are the k-values k0 + e, k0 + 4 + e, k0 + 8 + e, k0 + 12 + e (the order within a piece does
 // not matter for a sum; it is the same for every row and column).  No vector arithmetic and few registers,
 // so a wave keeps many loads in flight: the FMA form held 8 x 8 sums a lane and one piece in flight, and
-// streamed w at 3.2 TB/s.  The eight waves' sums are added in wave order: an order that depends on K alone.
+// streamed w at 3.2 TB/s.  The eight waves' sums are added in wave order.  The order of a sum is the same for every row and
+// column of a call; it depends on K and on whether the halves of a piece are summed by themselves (PACK: at most 8 rows, and
+// at most 8 columns a block, which follow from N).
 #define F32RM_WAVES 8
 template <int AHEAD, int TILES, int RT, bool SWIGLU, bool PACK = false>
 __global__ __launch_bounds__(F32RM_WAVES * 64) void gemm_f32_rows_mfma_kernel(const float* __restrict__ x,

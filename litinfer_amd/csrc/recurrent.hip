@@ -853,7 +853,9 @@ static int retention_launch(const float* xbc, long xbc_stride, float* state, con
     // (where a head has at most 64 columns, wide blocks would leave two of their four waves without any)
     const int wt = (VAR ? vdim > 64 : N > 64 || vdim > 64) ? 2 : 1, b = 64 * wt;
     const dim3 gs(max_chunks, heads, ((N + b - 1) / b) * ((vdim + b - 1) / b));
-#define RET_STATES(WT_) retention_states_kernel<WT_, VAR><<<gs, 256, 2 * RET_Q * 64 * WT_ * 4, stream>>>(xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry,                                                                                                          heads, groups, vdim, N, dc, chunk_decay, silu_in)
+#define RET_STATES(WT_)                                                                                                   \
+    retention_states_kernel<WT_, VAR><<<gs, 256, 2 * RET_Q * 64 * WT_ * 4, stream>>>(                                     \
+        xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, heads, groups, vdim, N, dc, chunk_decay, silu_in)
     if (wt == 2) RET_STATES(2); else RET_STATES(1);
 #undef RET_STATES
     const int NV4 = N * vdim / 4;
@@ -861,12 +863,16 @@ static int retention_launch(const float* xbc, long xbc_stride, float* state, con
                                                                                        dc.fixed_a, chunk_decay);
     const int pt = !VAR && vdim > 64 ? 2 : 1;          // (VAR: the sums side by side leave no registers for a second fragment of columns)
     const dim3 go(max_chunks, heads, (vdim + 64 * pt - 1) / (64 * pt));
-#define RET_GO(NQ_)                                                                                                                      return pt == 2 ? retention_outputs_launch<NQ_, VAR ? 1 : 2, VAR>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, heads, groups, vdim, N, dc, Dw, silu_in, stream)                    : retention_outputs_launch<NQ_, 1, VAR>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, heads, groups, vdim, N, dc, Dw, silu_in, stream)
+#define RET_AS(NQ_, PT_)                                                                                                  \
+    retention_outputs_launch<NQ_, PT_, VAR>(go, xbc, xbc_stride, q_start, q_len, chunk_seg, chunk_idx, carry, y, y_stride, \
+                                            heads, groups, vdim, N, dc, Dw, silu_in, stream)
+#define RET_GO(NQ_) return pt == 2 ? RET_AS(NQ_, VAR ? 1 : 2) : RET_AS(NQ_, 1)
     if (N <= 32) RET_GO(4);
     if (N <= 64) RET_GO(8);
     if (N <= 128) RET_GO(16);
     RET_GO(32);
 #undef RET_GO
+#undef RET_AS
 }
 
 // The four-columns-a-lane layout for a state of N values a column and heads of vdim columns (a multiple of 4): lanes

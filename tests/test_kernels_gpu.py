@@ -219,7 +219,7 @@ def test_float32_linear_with_k_in_parts(ops, m, n, k, bias, factor):
 
 
 @pytest.mark.parametrize("m,n,k,bias,factor", [
-    (8, 1536, 8960, False, 1.0),             # six columns a block, the longest trips
+    (8, 1536, 8960, False, 1.0),             # six columns a block, the most trips
     (3, 2048, 1536, True, 0.0),              # eight columns a block
     (8, 2049, 1540, True, 0.5),              # nine: both halves of a piece one after the other; one piece of a row over
     (9, 1536, 1536, False, 0.0),             # a row more than both halves of a piece take
