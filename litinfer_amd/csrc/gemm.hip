@@ -869,12 +869,18 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
     return up * (gate * __builtin_amdgcn_rcpf(1.0f + e));
 }
 
-// ACT: the other forms: the gate through GELU in its tanh form, or clamped with the limit a0: g = min(gate, a0),
-// u = clamp(up, -a0, a0), g sigmoid(1.702 g) (u + 1).
-template <bool ACT>
+// ACT: 0, or the other forms: LI_ACT_GELU_TANH, the gate through GELU in its tanh form; LI_ACT_CLAMPED with the limit a0:
+// g = min(gate, a0), u = clamp(up, -a0, a0), g sigmoid(1.702 g) (u + 1); ACT_TOLD, the one of them that `ep` says.  The tiles
+// have an instance each: with both forms' code in one kernel, 2,048 rows of 8,960 clamped outputs took 129.8 us instead of
+// 125.7, 64 rows of 18,944 54.1 instead of 52.7.  The kernel of few rows, bound by its loads, has one for both.
+#define ACT_TOLD (-1)
+template <int ACT>
 __device__ __forceinline__ float gated_bf16(float gate, float up, const LiAct& ep) {
-    if constexpr (!ACT) return swiglu_bf16(gate, up);
-    if (ep.act == LI_ACT_GELU_TANH) return up * gelu_tanh(gate);
+    if constexpr (ACT == 0) return swiglu_bf16(gate, up);
+    if constexpr (ACT == LI_ACT_GELU_TANH) return up * gelu_tanh(gate);
+    if constexpr (ACT == ACT_TOLD) {
+        if (ep.act == LI_ACT_GELU_TANH) return up * gelu_tanh(gate);
+    }
     const float g = fminf(gate, ep.a0), u = fminf(fmaxf(up, -ep.a0), ep.a0);
     const float e = __builtin_amdgcn_exp2f(-1.702f * 1.44269504088896341f * g);
     return (u + 1.0f) * (g * __builtin_amdgcn_rcpf(1.0f + e));
@@ -896,7 +902,7 @@ __device__ __forceinline__ void static_for(F&& f) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"                          \
                  :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(voff), "s"(base) : "memory", "m0")
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, bool ACT = false>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, int ACT = 0>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ w,
                                                              const float* __restrict__ bias,
@@ -904,7 +910,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
                                                              float accumulate, int nsplit,
                                                              const float* __restrict__ row_parts, int nparts, float eps,
                                                              LiAct ep) {
-    // ACT: the activation `ep`, of gate and up columns (gated_bf16) or of the sums.
+    // ACT: an activation, of gate and up columns (see gated_bf16) or of the sums (its number); its constants are in `ep`.
     // row_parts (SwiGLU tiles of 64 rows, up to 32 rows of x): x is the xg of li_linear_residual_norm and these
     // are its sq_parts; every row's sums are scaled by 1 / sqrt(sum of the row's parts / K + eps) before the
     // activation, which makes the result that of the RMS norm (the factor of a row does not depend on k).
@@ -1225,9 +1231,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
 #pragma unroll
             for (int e = 0; e < 8; ++e) v[e] = src[e];
             const size_t o_idx = (size_t)row * NO + col;
-            if constexpr (ACT && !SWIGLU) {
+            if constexpr (ACT != 0 && !SWIGLU) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), ep);
+                for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), LiAct{ACT, ep.a0, ep.a1});
                 if (col + 8 <= NO && (NO % 8) == 0) {
                     chunk16 o;
 #pragma unroll
@@ -1270,7 +1276,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     }
 }
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, bool ACT = false>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, int ACT = 0>
 static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* out, int M, int N, int K,
                       float accumulate, hipStream_t stream, int nsplit = 1, const float* row_parts = nullptr,
                       int nparts = 0, float eps = 0.f, LiAct ep = {}) {
@@ -1319,6 +1325,27 @@ __global__ __launch_bounds__(256) void splitk_reduce_act_kernel(const float* __r
     for (int sp = 1; sp < 8; ++sp) v += sp < nsplit ? a[sp] : 0.f;
     if (bias) v += bias[(int)(i % N)];
     store_from_float(out + i, activation(v, ep));
+}
+
+// The same of one part, four values a thread (GELU, 64 x 20,000 x 1,024, product included: 16.8 us, 18.2 with the kernel above)
+__global__ __launch_bounds__(256) void act_of_sums_kernel(const float* __restrict__ sums, size_t mn, int N, const float* __restrict__ bias,
+                                                          bf16_t* __restrict__ out, LiAct ep) {
+    const size_t i = 4 * ((size_t)blockIdx.x * 256 + threadIdx.x);
+    if (i >= mn) return;
+    float v[4];
+    if (i + 4 <= mn) {
+        const floatx4 a = *reinterpret_cast<const floatx4*>(sums + i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = a[e];
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = i + e < mn ? sums[i + e] : 0.f;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        if (i + e >= mn) continue;
+        store_from_float(out + i + e, activation(v[e] + (bias ? bias[(int)((i + e) % N)] : 0.f), ep));
+    }
 }
 
 // The same for the residual sum, one block a row, with the RMS norm of the new sum as a second
@@ -1768,7 +1795,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
                 const int n = n0 + 4 * (l >> 4) + r;
                 if (n < nend) {
                     const float gv = s[0][r], uv = s[NT - 1][r];
-                    store_from_float(out + (size_t)m * N + n, gated_bf16<EPI == 1>(gv, uv, a.ep));
+                    store_from_float(out + (size_t)m * N + n, gated_bf16<EPI == 1 ? ACT_TOLD : 0>(gv, uv, a.ep));
                 }
             }
         } else {
@@ -2294,19 +2321,30 @@ extern "C" int li_linear(const void* x, const void* w, const float* bias, void* 
     return li_launch_status();
 }
 
+// Bytes of workspace that li_linear_act needs (0: none).
+extern "C" long li_linear_act_work_bytes(int M, int N, int K, int act) {
+    const long parts = li_linear_work_bytes(M, N, K, LI_BF16);
+    if (parts > 0 || act == LI_ACT_RELU2 || M <= 0 || N <= 0 || K <= 0 || K % 64 || !mid_rows_take(M, N, K) || (N + 127) / 128 < 128) return parts;
+    return (long)M * N * (long)sizeof(float);
+}
+
 // out = act(x w^T + bias), bfloat16 throughout, the sums float32 until the activation has been taken: in the epilogue of
 // the kernel that li_linear would take for these sizes, or of the one that adds its parts up.  Without it the sums go to
-// memory in float32 and a kernel of their own reads them again: at a few rows that kernel costs its launch, 5 us a layer,
-// and at 2,048 rows of 8,960 columns the reads and writes of 73 MB (squared ReLU: 15 to 29 us).  Above 64 rows the
-// squared ReLU only: the others are tens of instructions a value, which a tile's four waves take one after the other when
-// the matrix cores are done (xIELU, 2,601 rows of 8,960 columns: product and kernel 96 + 24 us, in the epilogue 183).
+// memory in float32 and a kernel of their own reads them again: at a few rows that kernel costs its launch, some 2 us a layer in
+// a recorded step (8 x 8,960 x 1,536 12.7 -> 10.7 us, 64 rows, K in parts, 17.0 -> 14.3), and at 2,048 rows of 8,960 columns the
+// reads and writes of 73 MB (squared ReLU 93 -> 70 us, of 18,944 x 3,584 327 -> 263; 300 rows of 8,960 23.9 -> 17.7).  Tiles
+// whose K is not in parts take the squared ReLU only, in instances of their own: the others are tens of instructions a value, which
+// a tile's four waves take one after the other when the matrix cores are done (xIELU, 2,601 rows of 8,960 columns: product and
+// kernel 96 + 24 us, in the epilogue 183; GELU, 17 to 48 rows of 18,944 x 3,584 31.7 to 35.9 -> 33.1 to 36.8), and with the
+// code of all four in one kernel the squared ReLU pays too (2,048 rows of 8,960 103 us, 1,000 rows of 18,944 182 -> 223).
+// Up to 64 rows the others' sums go to the lent memory (li_linear_act_work_bytes) and on to act_of_sums_kernel
+// (17 / 48 rows 32.4 / 36.4); above, the caller does the same.
 // Returns -1, having done nothing, where it does not take the call.
 extern "C" int li_linear_act(const void* x, const void* w, const float* bias, void* out, int M, int N, int K, int act, float a0,
                              float a1, void* work, long work_bytes, hipStream_t stream) {
     if (M <= 0 || N <= 0 || K <= 0 || act < LI_ACT_RELU2 || act > LI_ACT_XIELU) return LI_ERR_SIZE;
     if (K % 8 || (M > 64 && (K % 64 || act != LI_ACT_RELU2))) return -1;
     const LiAct ep{act, a0, a1};
-#define LI_ACT(BM, BN, NS, WLM) launch_dma<BM, BN, 64, NS, false, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
     if (M <= 64 && (K % 64 || !mid_rows_take(M, N, K))) {
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
@@ -2314,18 +2352,22 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
         launch_skinny<false, bf16_t, 2>(a, stream);
         return li_launch_status();
     }
-    const long need = li_linear_work_bytes(M, N, K, LI_BF16);
-    if (need > 0) {                                  // K in parts
+    const long need = li_linear_act_work_bytes(M, N, K, act);
+    if (need > 0) {                                  // K in parts, or in one
         const size_t mn = (size_t)M * N;
         const int nsplit = (int)(need / (long)(mn * sizeof(float)));
-        if (!work || work_bytes < need || nsplit > 8) return -1;
-        const int rc = M <= 64
+        if (!work || (uintptr_t)work % 16 || work_bytes < need || nsplit > 8) return -1;
+        const int rc = M <= 64 && nsplit == 1 && (N + 255) / 256 >= 128
+            ? launch_dma<64, 256, 64, 3, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream)
+            : M <= 64
             ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit)
             : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
         if (rc != LI_OK) return rc;
-        splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
+        if (nsplit == 1) act_of_sums_kernel<<<(unsigned)((mn + 1023) / 1024), 256, 0, stream>>>((const float*)work, mn, N, bias, (bf16_t*)out, ep);
+        else splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
         return li_launch_status();
     }
+#define LI_ACT(BM, BN, NS, WLM) launch_dma<BM, BN, 64, NS, false, bf16_t, WLM, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
     if (M <= 64) {                                   // (as linear_mid_rows takes them)
         if ((N + 255) / 256 >= 128) return LI_ACT(64, 256, 3, 2);
         if ((N + 127) / 128 >= 128) return LI_ACT(64, 128, 4, 2);
@@ -2400,12 +2442,13 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
             const double c = tile_cost(64, widths[i], 1.0, M, N, K);
             if (pick < 0 || c < best) { best = c; pick = i; }
         }
-#define LI_SW64(BN, NS) (act ? launch_dma<64, BN, 64, NS, true, bf16_t, 2, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, ep) \
-                                     : launch_dma<64, BN, 64, NS, true, bf16_t>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps))
+#define LI_SW64_AS(BN, NS, ACT) launch_dma<64, BN, 64, NS, true, bf16_t, 2, ACT>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, ep)
+#define LI_SW64(BN, NS) (act == LI_ACT_CLAMPED ? LI_SW64_AS(BN, NS, LI_ACT_CLAMPED) : act ? LI_SW64_AS(BN, NS, LI_ACT_GELU_TANH) : LI_SW64_AS(BN, NS, 0))
         if (pick == 0) return LI_SW64(256, 3);
         if (pick == 1) return LI_SW64(192, 4);
         if (pick == 2) return LI_SW64(128, 4);
 #undef LI_SW64
+#undef LI_SW64_AS
     }
     if (row_parts || (M <= 64 && act)) {
         if (K % 8) return LI_ERR_SIZE;
@@ -2418,8 +2461,8 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
     }
     if (M <= 64) return li_linear_skinny(x, w, nullptr, out, M, I, K, LI_BF16, 0, 1, stream);
     if (K % 64) return LI_ERR_SIZE;
-#define LI_DMA(BM, BN, BK, NS, WLM) (act ? launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, true>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep) \
-                                                 : launch_dma<BM, BN, BK, NS, true, bf16_t, WLM>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream))
+#define LI_DMA_AS(BM, BN, BK, NS, WLM, ACT) launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, ACT>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
+#define LI_DMA(BM, BN, BK, NS, WLM) (act == LI_ACT_CLAMPED ? LI_DMA_AS(BM, BN, BK, NS, WLM, LI_ACT_CLAMPED) : act ? LI_DMA_AS(BM, BN, BK, NS, WLM, LI_ACT_GELU_TANH) : LI_DMA_AS(BM, BN, BK, NS, WLM, 0))
     // (a tile's columns are gate and up columns in turn, 32 of each: its width is a multiple of 64)
     // (128 x 320: 160 gate columns in one wave, their ups in the wave beside it; for portions of a few hundred rows,
     // where no other width comes near whole rounds of the compute units: 512 rows against the 1.5B's 17,920
@@ -2444,6 +2487,7 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
     default: return LI_DMA(128, 320, 64, 2, 2);
     }
 #undef LI_DMA
+#undef LI_DMA_AS
 }
 
 // The packed q/k/v projection of up to 32 rows with the half-split rotary encoding of query and key

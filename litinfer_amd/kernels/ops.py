@@ -168,9 +168,10 @@ def _stream() -> int:
     return torch.cuda.current_stream().cuda_stream
 
 
-def _call(module: str, name: str, args) -> int:
-    if not profiler.enabled:
-        return _fn(module, name)(*args, _stream())
+_NOT_TAKEN = -1         # an entry point's answer where it has no kernel for the sizes, with nothing done
+
+
+def _timed(module: str, name: str, args) -> int:
     rc = []
 
     def launch():
@@ -180,22 +181,21 @@ def _call(module: str, name: str, args) -> int:
     return rc[0]
 
 
+def _refused(name: str, rc: int) -> RuntimeError:
+    return RuntimeError(f"{name}: the kernel library refused the call (code {rc}): {_ERRORS.get(rc, 'unknown')}")
+
+
 def _run(module: str, name: str, *args) -> None:
-    rc = _call(module, name, args)
+    rc = _timed(module, name, args) if profiler.enabled else _fn(module, name)(*args, _stream())
     if rc != 0:
-        raise RuntimeError(f"{name}: the kernel library refused the call (code {rc}): "
-                           f"{_ERRORS.get(rc, 'unknown')}")
-
-
-_NOT_TAKEN = -1         # an entry point's answer where it has no kernel for the sizes, with nothing done
+        raise _refused(name, rc)
 
 
 def _try(module: str, name: str, *args) -> bool:
     """Like `_run`, but False where the library has no kernel for these sizes."""
-    rc = _call(module, name, args)
+    rc = _timed(module, name, args) if profiler.enabled else _fn(module, name)(*args, _stream())
     if rc not in (0, _NOT_TAKEN):
-        raise RuntimeError(f"{name}: the kernel library refused the call (code {rc}): "
-                           f"{_ERRORS.get(rc, 'unknown')}")
+        raise _refused(name, rc)
     return rc == 0
 
 
@@ -1259,7 +1259,7 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], o
     if not m:
         return True
     work, work_bytes = 0, 0
-    need = _work_bytes(m, n, k, _DT[x.dtype]) if ws is not None else 0
+    need = _lib_fn("gemm", "li_linear_act_work_bytes", [c_int] * 4, c_long)(m, n, k, LINEAR_ACTS[act]) if ws is not None else 0
     if need:
         if m <= SKINNY_MAX_ROWS:                    # one size for all row counts of a decode batch: the buffer does not move
             need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)

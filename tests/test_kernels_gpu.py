@@ -1501,6 +1501,7 @@ def test_state_space_recurrence_of_long_portions_is_as_exact_as_token_by_token(o
     (50, 300, 1024, True, True),         # K in parts
     (64, 17000, 128, False, True),       # 64-row tiles of 128 columns
     (37, 33000, 64, True, True),         # ... and of 256
+    (33, 16387, 64, True, True),         # ... whose sums end inside a piece of four
     (65, 300, 4096, True, True),         # more rows, K in parts
     (300, 2053, 192, True, True),        # tiles whose last columns lie past the end, not in 16-byte pieces
     (1100, 4608, 320, False, True),
