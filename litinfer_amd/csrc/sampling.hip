@@ -323,12 +323,15 @@ __device__ __forceinline__ void radix_kth(Each&& each, int kk, uint32_t& tau, in
     need = kk;
 }
 
-// The same tau and need for keys that lie in registers, up to 8 a thread (0: none), in the first `waves` waves.  Eight passes
-// of sixteen counts are long for one block; this takes a bound first.  Every wave finds the ceil(kk / waves)-th largest of its
-// threads' largest keys: at least kk keys are no smaller than the least of these, and in earnest not many more (kk = 50 of
-// 8,192 normal logits: some 150).  They go into a list in LDS, and each is held against all others: the one with fewer than
-// kk keys above it and at least kk no smaller is tau.  False, with nothing done, where the bound leaves fewer than kk keys
-// (a wave without enough of them sets none) or more than SMP_LIST (many equal logits): radix_kth then.
+// The same tau and need for keys that lie in registers, up to 8 a thread (0: none), in the first `waves` waves and, where the
+// last one is cut short, the one behind them.  Eight passes of sixteen counts are long for one block; this takes a bound
+// first.  Each of the `waves` whole waves finds the ceil(kk / waves)-th largest of its threads' largest keys: at least kk keys
+// are no smaller than the least of these, and in earnest not many more (kk = 50 of 8,192 normal logits: some 150; a wave cut
+// short sets no bound: its share of kk would lie far down among its few keys, or it would not have as many; 16 rows of 32,000
+// ids, top-k 200 with top-p 0.9: 73.5 us with its bound, 49.5).  They go into a list in LDS, and each is held against all
+// others: the one with fewer than kk keys above it and at least kk no smaller is tau.  False, with nothing done, where the
+// bound leaves fewer than kk keys (a wave without enough of them sets none) or more than SMP_LIST (many equal logits):
+// radix_kth then.
 // 64 rows of 151,936 ids, top-k 50: tiles kernel 58 -> 45 us (one row 26 -> 13), rows kernel 22 -> 14.
 constexpr int SMP_LIST = 1024;
 __device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int waves, uint32_t& tau, int& need, uint32_t* list, int* work_i, int* res) {
@@ -350,7 +353,7 @@ __device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int
     __syncthreads();
     uint32_t bound = 0xffffffffu;
 #pragma unroll
-    for (int i = 0; i < SMP_WAVES; ++i) bound = min(bound, (uint32_t)work_i[i] - 1u);      // (0, no bound, becomes the largest)
+    for (int i = 0; i < SMP_WAVES; ++i) bound = i < waves ? min(bound, (uint32_t)work_i[i] - 1u) : bound;      // (0, no bound, becomes the largest)
     bound += 1u;
     if (bound == 0u) return false;
     int mine = 0;
@@ -391,10 +394,12 @@ __device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int
 // `remaining`, four bits a pass (masses by the next digit); on return `remaining` is what the keys
 // equal to tp have to bring.  m: the maximum that masses are taken against.
 // Where cut, digits in which tau, which no survivor is below, and the maximum agree are taken as they are; and with LOOK,
-// once a single key is left that agrees with the digits found, it is tp: a digit of which all mass is left changes neither
-// `remaining` nor the choice.  64 rows, top-k 50 with top-p 0.9: rows kernel 40 -> 25 us.  Looking for that key is another
-// pass over `each`, so it is for keys in registers: over the row itself a pass takes as long as the one it may spare (64
-// rows, top-k 300 with top-p 0.95, logits of bfloat16's values: 762 us with it, 635 without).
+// once all keys that agree with the digits found are one key (alone, or several ids of one value), it is tp: a digit of which
+// all mass is left changes neither `remaining` nor the choice.  64 rows, top-k 50 with top-p 0.9: rows kernel 40 -> 25 us.
+// A look takes two barriers, so it is taken where the mass that is left is no more than one key's (two keys so close bring
+// twice the least of them), and once behind the digits of a bfloat16 value, several ids of which there mostly are.  It is
+// for keys in registers: over the row itself a pass takes as long as the one it may spare (64 rows, top-k 300 with top-p
+// 0.95, logits of bfloat16's values: 762 us with it, 635 without).
 template <bool LOOK, typename Each>
 __device__ __forceinline__ void radix_mass(Each&& each, bool cut, uint32_t tau, int ties, float e_ties, float m,
                                            float& remaining, uint32_t& tp, float* work_f, float* tot_f, int* res) {
@@ -438,16 +443,18 @@ __device__ __forceinline__ void radix_mass(Each&& each, bool cut, uint32_t tau, 
         remaining -= above;
         tp |= (uint32_t)d << shift;
         if (LOOK && shift > 0 && cut && !(ties > 0 && (tau >> shift) == (tp >> shift))) {
-            int left = 0;
-            uint32_t one = 0u;
+            const float least = key_value(tp), most = key_value(tp | ((1u << shift) - 1u));
+            if (!(shift == 16 || (most - least < 0.69f && tot_f[d] <= 1.0001f * expf(most - m)))) continue;
+            uint32_t one = 0u;                   // one of the thread's keys that are left (0: it has none; a key above tau is not 0)
+            bool differ = false;
             each([&](float z) {
                 const uint32_t key = sort_key(z);
-                if (key > tau && (key >> shift) == (tp >> shift)) { ++left; one = key; }
+                if (key > tau && (key >> shift) == (tp >> shift)) { differ |= one != 0u && key != one; one = key; }
             });
-            if (__syncthreads_count(left > 0) == 1) {
-                if (left) res[0] = left == 1 ? (int)one : 0;
-                __syncthreads();
-                if (res[0]) { tp = (uint32_t)res[0]; return; }
+            if (one) res[0] = (int)one;          // (any of the threads' keys: the others are held against it)
+            if (__syncthreads_or(one != 0u)) {
+                const uint32_t all = (uint32_t)res[0];
+                if (!__syncthreads_or(differ || (one && one != all))) { tp = all; return; }
             }
         }
     }
@@ -519,7 +526,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_tiles_kernel(
         uint32_t key[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) key[e] = j0 + e < V ? sort_key(z[e]) : 0u;
-        if (!select_kth(key, kc, (in_tile + 8 * LI_WAVE - 1) / (8 * LI_WAVE), tau, need, list, work_i, tot_i))
+        if (!select_kth(key, kc, max(in_tile / (8 * LI_WAVE), 1), tau, need, list, work_i, tot_i))
             radix_kth([&](auto f) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
@@ -632,7 +639,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
         for (int c = 0; c < SMP_CAND_PER_THREAD; ++c) key[c] = have[c] ? sort_key(cz[c]) : 0u;
         const int kk = min(by_k ? k : kc, total);
         const int threads = (slots + C - 1) / C;
-        if (!select_kth(key, kk, (threads + LI_WAVE - 1) / LI_WAVE, tau_c, need_c, list, work_i, tot_i)) radix_kth(each, kk, tau_c, need_c, work_i, tot_i);
+        if (!select_kth(key, kk, max(threads / LI_WAVE, 1), tau_c, need_c, list, work_i, tot_i)) radix_kth(each, kk, tau_c, need_c, work_i, tot_i);
         bool exact = true;
         if (by_k) { cut = true; tau = tau_c; need = need_c; }
         if (by_p) {
@@ -791,10 +798,15 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
         // The tiles' sums are there, each against its tile's own maximum: brought to the row's maximum
         // they give the tile that holds the target; within it the search goes on in the tile's own scale.
         float top = -INFINITY;
-        for (int t = tid & (LI_WAVE - 1); t < ntiles; t += LI_WAVE) top = fmaxf(top, tile_m[t]);
-        top = wave_max(top);
-        for (int t = tid; t < ntiles; t += SMP_NT) tile_sum[t] = tile_s[t] * expf(tile_m[t] - top);
-        __syncthreads();
+        if (ntiles == 1) {                           // (a vocabulary of one tile: nothing to do side by side, 12.1 -> 11.4 us)
+            top = tile_m[0];
+            if (tid == 0) tile_sum[0] = tile_s[0] * expf(tile_m[0] - top);
+        } else {
+            for (int t = tid & (LI_WAVE - 1); t < ntiles; t += LI_WAVE) top = fmaxf(top, tile_m[t]);
+            top = wave_max(top);
+            for (int t = tid; t < ntiles; t += SMP_NT) tile_sum[t] = tile_s[t] * expf(tile_m[t] - top);
+            __syncthreads();
+        }
         if (tid == 0) {
             float total = 0.f;
 #pragma unroll 8

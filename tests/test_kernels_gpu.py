@@ -1063,16 +1063,18 @@ def test_sample_rows_with_many_equal_logits_at_the_thresholds(ops, vocab):
     assert same >= n - 2
 
 
-@pytest.mark.parametrize("order", ["mixed", "ascending", "few", "one_value"])
+@pytest.mark.parametrize("order", ["mixed", "rounded", "ascending", "few", "one_value"])
 def test_sample_rows_with_the_candidates_found_by_a_bound(ops, order):
     # ids above a bound are held against each other (mixed: some more than the wanted ones lie above it); where one wave
     # holds all large ids (ascending), most ids are -inf (few) or all are equal, too many lie above it and the search goes
-    # through the digits
+    # through the digits; of bfloat16's values (rounded) several ids share one, at the threshold of top-p too
     g = torch.Generator().manual_seed(66)
     vocab, top_k = 8192 + 4097, [1, 15, 16, 17, 50, 128, 255, 256]
     n = len(top_k)
     logits = torch.randn(n, vocab, generator=g) * 3
-    if order == "ascending":
+    if order == "rounded":
+        logits = logits.bfloat16().float()
+    elif order == "ascending":
         logits = logits.sort(dim=1).values
     elif order == "few":
         logits[:, torch.randperm(vocab, generator=g)[:vocab - 40]] = float("-inf")
