@@ -877,9 +877,9 @@ __device__ __forceinline__ float swiglu_bf16(float gate, float up) {
 template <int ACT>
 __device__ __forceinline__ float gated_bf16(float gate, float up, const LiAct& ep) {
     if constexpr (ACT == 0) return swiglu_bf16(gate, up);
-    if constexpr (ACT == LI_ACT_GELU_TANH) return up * gelu_tanh(gate);
+    if constexpr (ACT == LI_ACT_GELU_TANH) return up * gelu_tanh_bf16(gate);
     if constexpr (ACT == ACT_TOLD) {
-        if (ep.act == LI_ACT_GELU_TANH) return up * gelu_tanh(gate);
+        if (ep.act == LI_ACT_GELU_TANH) return up * gelu_tanh_bf16(gate);
     }
     const float g = fminf(gate, ep.a0), u = fminf(fmaxf(up, -ep.a0), ep.a0);
     const float e = __builtin_amdgcn_exp2f(-1.702f * 1.44269504088896341f * g);

@@ -1213,6 +1213,19 @@ def _gated_form(limit):
     return (5, float(limit)) if limit > 0 else (0, 0.0)
 
 
+def gelu_gate_as_epilogue(m: int, n: int, k: int, dtype: torch.dtype) -> bool:
+    """Whether up * gelu_tanh(gate) of m rows and n gate and up columns together is better taken in the product's epilogue than
+    by a kernel of its own.  The product with the epilogue is not cut along k; where the product alone would be (few tiles),
+    that is worth more than the float32 columns cost if k is long, and for 33 to 64 rows, whose few-row kernel goes through
+    its rows twice, also if the matrix is large.  Us, two kernels / epilogue, n x k: 48 rows x 6,144 x 1,536 (19 MB) 12.8 / 10.3,
+    8,960 x 1,024 13.2 / 12.6, 8,960 x 1,536 (28 MB) 14.7 / 18.4, 12,000 x 2,048 18.1 / 25.2, 2,048 x 4,096 (17 MB) 11.1 / 20.2; 65 rows
+    x 16,000 x 2,048 27.2 / 20.9, x 3,072 x 2,048 13.3 / 13.6, x 4,096 x 4,096 19.6 / 30.3, x 8,960 x 3,584 23.5 / 29.8; 32 rows
+    x 8,960 x 3,584 19.9 / 21.0."""
+    if dtype is not torch.bfloat16 or not _work_bytes(m, n, k, _DT[dtype]):
+        return True
+    return k <= 2048 and not (32 < m <= SKINNY_MAX_ROWS and 2 * n * k > 20_000_000)
+
+
 def linear_swiglu(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, row_scale: Optional[RowScale] = None,
                   limit: Union[float, str] = 0.0) -> None:
     """out[m, n] = up * gate / (1 + exp(-gate)) with [gate, up] = x w^T, w = [gate; up]

@@ -62,7 +62,8 @@ class SwiGLUMLP(FeedForward):
     def forward(self, xn, residual, ctx):
         t = xn.shape[0]
         h = ctx.ws.buffer("mlp.h", (t, self.inter), self.rt.dtype)
-        if self.gate_up.takes_swiglu(xn):
+        if self.gate_up.takes_swiglu(xn) and (self.gate_form != ops.GELU_TANH_GATE
+                                              or ops.gelu_gate_as_epilogue(t, 2 * self.inter, self.hidden, xn.dtype)):
             self.gate_up(xn, h, ws=ctx.ws, swiglu=True, limit=self.gate_form)        # few rows: the activation is the epilogue
         else:
             if self.activation == "silu":

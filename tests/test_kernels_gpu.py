@@ -1531,6 +1531,16 @@ def test_linear_with_an_activation_of_its_sums(ops, act, m, n, k, bias, ws):
         assert bool(torch.isnan(out.float()).all())
 
 
+def test_where_the_tanh_form_of_gelu_is_the_gated_products_epilogue(ops):
+    """The rule at its lines: a product that is not cut along K always, one that is by the length of K and, for 33 to 64 rows,
+    by the matrix."""
+    takes = lambda m, n, k: ops.gelu_gate_as_epilogue(m, n, k, torch.bfloat16)
+    assert all(takes(m, 8960, 1536) for m in (1, 16, 17, 32, 65, 300, 2048)) and not takes(33, 8960, 1536) and not takes(64, 8960, 1536)
+    assert takes(48, 6144, 1536) and takes(48, 14000, 768) and takes(64, 40000, 1024)
+    assert takes(1, 2048, 4096) and takes(2048, 37888, 3584) and not any(takes(m, 4096, 4096) for m in (33, 64, 65, 128))
+    assert ops.gelu_gate_as_epilogue(48, 8960, 1536, torch.float32)
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 100, 72), (9, 8960, 1536), (30, 50, 136), (64, 9000, 256), (200, 333, 128), (1030, 1500, 192)])
 def test_gated_product_with_the_tanh_form_of_gelu(ops, m, n, k):
     g = torch.Generator().manual_seed(68)
