@@ -902,7 +902,69 @@ __device__ __forceinline__ void static_for(F&& f) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"                          \
                  :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(voff), "s"(base) : "memory", "m0")
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, int ACT = 0>
+// A wave's band of 32 rows of EW sums in LDS (ESTRIDE floats apart) goes to rows row0 .. and columns col0 .. of out: row by row,
+// 8 consecutive columns a lane, so that the stores (and the loads of what is added to) are whole 16-byte pieces.
+// GATED: the band holds results already; ACT otherwise: the activation of sums and bias.
+template <int EW, int ESTRIDE, bool GATED, int ACT, typename TO>
+__device__ __forceinline__ void band_to_memory(const float* band, int row0, int col0, int M, int NO, const float* bias, TO* out,
+                                               float accumulate, const LiAct& ep) {
+    constexpr int LPR = EW / 8, RPP = 64 / LPR;     // lanes that take a row; rows a pass of the wave covers
+    const int lane = threadIdx.x & 63;
+    const int erow = lane / LPR, ecol = (lane % LPR) * 8;      // (where 64 is no multiple of LPR the last lanes idle)
+    const int col = col0 + ecol;
+#pragma unroll
+    for (int pass = 0; pass < (32 + RPP - 1) / RPP; ++pass) {
+        const int row = row0 + RPP * pass + erow;
+        if (erow >= RPP || RPP * pass + erow >= 32 || row >= M || col >= NO) continue;
+        const float* src = &band[(RPP * pass + erow) * ESTRIDE + ecol];
+        float v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = src[e];
+        const size_t o_idx = (size_t)row * NO + col;
+        if constexpr (ACT != 0 && !GATED) {
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), LiAct{ACT, ep.a0, ep.a1});
+            if (col + 8 <= NO && (NO % 8) == 0) {
+                chunk16 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o.w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
+                *reinterpret_cast<chunk16*>(reinterpret_cast<uint16_t*>(out) + o_idx) = o;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (col + e < NO) epilogue_store(out, o_idx + e, v[e], nullptr, col + e, 0);
+            }
+            continue;
+        }
+        if (col + 8 <= NO && (NO % 8) == 0) {
+            if (bias) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] += bias[col + e];
+            }
+            if constexpr (sizeof(TO) == 4) {
+                float4* o = reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + o_idx);
+                if (accumulate != 0.f) {
+                    const float4 a0 = o[0], a1 = o[1];
+                    v[0] = fmaf(accumulate, v[0], a0.x); v[1] = fmaf(accumulate, v[1], a0.y); v[2] = fmaf(accumulate, v[2], a0.z); v[3] = fmaf(accumulate, v[3], a0.w);
+                    v[4] = fmaf(accumulate, v[4], a1.x); v[5] = fmaf(accumulate, v[5], a1.y); v[6] = fmaf(accumulate, v[6], a1.z); v[7] = fmaf(accumulate, v[7], a1.w);
+                }
+                o[0] = float4{v[0], v[1], v[2], v[3]};
+                o[1] = float4{v[4], v[5], v[6], v[7]};
+            } else {
+                chunk16 o;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) o.w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
+                *reinterpret_cast<chunk16*>(reinterpret_cast<uint16_t*>(out) + o_idx) = o;
+            }
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (col + e < NO) epilogue_store(out, o_idx + e, v[e], bias, col + e, accumulate);
+        }
+    }
+}
+
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ w,
                                                              const float* __restrict__ bias,
@@ -916,13 +978,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     // activation, which makes the result that of the RMS norm (the factor of a row does not depend on k).
     // nsplit > 1: a block multiplies one of nsplit parts of K, the y-th, and writes its sums to the y-th
     // [M, N] matrix behind `out` (float, no bias, no accumulation); splitk_reduce_kernel adds them
-    // WLM: waves along the rows of the tile, 2 (two by two) or 4 (each wave 32-row bands over all columns:
-    // BN may then be any multiple of 32, for matrices whose columns no other tile divides into 256 tiles)
-    constexpr int WLN = 4 / WLM;
-    constexpr int WM = BM / WLM, WN = BN / WLN, TM = WM / 32, TN = WN / 32;
-    static_assert(WM % 32 == 0 && WN % 32 == 0 && (WLM == 2 || WLM == 4), "a wave's part of the tile is made of 32 x 32 tiles");
+    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
+    static_assert(WM % 32 == 0 && WN % 32 == 0, "a wave's part of the tile is made of 32 x 32 tiles");
     constexpr bool SWSPLIT = SWIGLU && (TN % 2 == 1);        // gates and ups in different waves (see the rows of w below)
-    static_assert(!SWSPLIT || WLN == 2, "gates in one wave, ups in the wave beside it");
     static_assert(BM % 32 == 0 && BN % 32 == 0 && (BM / 4) % (64 / (BK / 8)) == 0 && (BN / 4) % (64 / (BK / 8)) == 0, "whole load instructions a wave");
     constexpr int CPR = BK / 8, WRAP = 128 / BK;                 // chunks in a row; rows that fill all banks once
     constexpr int RPI = 64 / CPR;                                // rows one load instruction of a wave covers
@@ -931,7 +989,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     constexpr int LPW = IA + IB;                                 // loads a wave issues per step
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave / WLN) * WM, wn = (wave % WLN) * WN;
+    const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
     const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
     int mt, nt, split;
     if (!TileOrder(mtiles).tile(blockIdx.x, mtiles, ntiles, nsplit, mt, nt, split)) return;
@@ -1192,10 +1250,6 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     static_assert(4 * 32 * ESTRIDE * 4 <= NSTAGE * STAGE * 2, "the waves' bands fit the main loop's LDS");
     float* band = reinterpret_cast<float*>(lds) + wave * 32 * ESTRIDE;
     const int ccol = lane & 31, crow = (lane >> 5) * 4;
-    constexpr int LPR = EW / 8, RPP = 64 / LPR;     // lanes a row of the band takes; rows a pass of the wave covers
-    const int erow = lane / LPR, ecol = (lane % LPR) * 8;      // (where 64 is no multiple of LPR the last lanes idle)
-    const int NO = SWIGLU ? N / 2 : N;             // columns of out
-    const int col = (SWIGLU ? (n0 + wn) / 2 : n0 + wn) + ecol;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         __builtin_amdgcn_wave_barrier();
@@ -1222,61 +1276,12 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
                     band[(8 * (r >> 2) + crow + (r & 3)) * ESTRIDE + 32 * j + ccol] = acc[i][j][r];
         }
         __builtin_amdgcn_wave_barrier();
-#pragma unroll
-        for (int pass = 0; pass < (32 + RPP - 1) / RPP; ++pass) {
-            const int row = m0 + wm + 32 * i + RPP * pass + erow;
-            if (erow >= RPP || RPP * pass + erow >= 32 || row >= M || col >= NO) continue;
-            const float* src = &band[(RPP * pass + erow) * ESTRIDE + ecol];
-            float v[8];
-#pragma unroll
-            for (int e = 0; e < 8; ++e) v[e] = src[e];
-            const size_t o_idx = (size_t)row * NO + col;
-            if constexpr (ACT != 0 && !SWIGLU) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = activation(v[e] + (bias && col + e < NO ? bias[col + e] : 0.f), LiAct{ACT, ep.a0, ep.a1});
-                if (col + 8 <= NO && (NO % 8) == 0) {
-                    chunk16 o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) o.w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
-                    *reinterpret_cast<chunk16*>(reinterpret_cast<uint16_t*>(out) + o_idx) = o;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e)
-                        if (col + e < NO) epilogue_store(out, o_idx + e, v[e], nullptr, col + e, 0);
-                }
-                continue;
-            }
-            if (col + 8 <= NO && (NO % 8) == 0) {
-                if (bias) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) v[e] += bias[col + e];
-                }
-                if constexpr (sizeof(TO) == 4) {
-                    float4* o = reinterpret_cast<float4*>(reinterpret_cast<float*>(out) + o_idx);
-                    if (accumulate != 0.f) {
-                        const float4 a0 = o[0], a1 = o[1];
-                        v[0] = fmaf(accumulate, v[0], a0.x); v[1] = fmaf(accumulate, v[1], a0.y); v[2] = fmaf(accumulate, v[2], a0.z); v[3] = fmaf(accumulate, v[3], a0.w);
-                        v[4] = fmaf(accumulate, v[4], a1.x); v[5] = fmaf(accumulate, v[5], a1.y); v[6] = fmaf(accumulate, v[6], a1.z); v[7] = fmaf(accumulate, v[7], a1.w);
-                    }
-                    o[0] = float4{v[0], v[1], v[2], v[3]};
-                    o[1] = float4{v[4], v[5], v[6], v[7]};
-                } else {
-                    chunk16 o;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        o.w[e] = pack2_bf16(v[2 * e], v[2 * e + 1]);
-                    *reinterpret_cast<chunk16*>(reinterpret_cast<uint16_t*>(out) + o_idx) = o;
-                }
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (col + e < NO) epilogue_store(out, o_idx + e, v[e], bias, col + e, accumulate);
-            }
-        }
+        band_to_memory<EW, ESTRIDE, SWIGLU, ACT, TO>(band, m0 + wm + 32 * i, SWIGLU ? (n0 + wn) / 2 : n0 + wn, M, SWIGLU ? N / 2 : N,
+                                                     bias, out, accumulate, ep);
     }
 }
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int WLM = 2, int ACT = 0>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0>
 static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* out, int M, int N, int K,
                       float accumulate, hipStream_t stream, int nsplit = 1, const float* row_parts = nullptr,
                       int nparts = 0, float eps = 0.f, LiAct ep = {}) {
@@ -1292,12 +1297,257 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
     constexpr int lds_bytes = NSTAGE * (BM + BN) * BK * 2;
     static bool configured = false;
     if (!configured) {
-        if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, WLM, ACT>,
+        if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, ACT>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
             return LI_ERR_LAUNCH;
         configured = true;
     }
-    gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, WLM, ACT><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, nsplit, row_parts, nparts, eps, ep);
+    gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, ACT><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, nsplit, row_parts, nparts, eps, ep);
+    return li_launch_status();
+}
+
+// ------------------------------- bfloat16, more than 64 rows: tiles of a block, two by two waves
+// A block of four waves, one a SIMD, makes a tile of BM x BN; a step is 64 k-values, and NSTAGE stages lie in LDS,
+// filled by loads that go straight there.  What bounds it is the time between a load's issue and its arrival (a thousand
+// and more clocks under load): a wave is alone on its SIMD, so whatever it waits for, the matrix cores wait for too.  With
+// whole stages handed back once a step (the form before) 8,192^3 kept the matrix cores busy 60 % of the time at 1.88 GHz.
+// So a stage is handed back in pieces.  A wave's part of the tile is cut in two both ways; each of the four pieces is
+// multiplied for the whole step, in an order in which one operand stays (quarter (0, X), (0, Y), (1, Y), (1, X) of rows
+// and columns, X and Y the halves of the columns, which change places from step to step), and while it is multiplied the
+// operand that the NEXT quarter needs anew is read from LDS, into the registers of the half that is dead by then:
+//     quarter     multiplies    reads                   asks memory for, NSTAGE steps ahead
+//     0           (0, X)        B half Y                A half 0
+//     1           (0, Y)        A half 1                B half X         then a barrier
+//     2           (1, Y)        A half 0, next step     B half Y
+//     3           (1, X)        B half Y, next step     A half 1         then a barrier
+// Half of the stage has been read at each barrier and its place is asked for again at once, so a load has two
+// barriers more than NSTAGE - 1 steps to arrive, the loads are spread evenly over the whole step, and no register
+// holds an operand twice: 128 registers of operands beside the 256 of the sums.
+// Multiplied by v_mfma_f32_16x16x32_bf16: with operands as they are in use the chip is at its power limit here, and this
+// form draws less for the same product than the 32 x 32 x 16 one (a loop of nothing else 1.90 against 1.75 PFLOP/s).
+// The MFMAs are assembly so that a sum stays in its registers: the instruction's result may lie elsewhere, and the compiler
+// made use of that, with some 600 moves between registers a step and spills.  What it then does not see is seen to
+// here: operands come from LDS reads alone, which it waits for as for any use; the same sum comes up again after four
+// MFMAs at least; and before the sums are read behind the loop, two waits of 16 cycles pass.
+// A half's rows of a stage: first those of the waves of the first row (column) of waves, then the others'.
+// ... by the lanes that are told: all, or none (a step past the last asks for nothing, but counts as the others do)
+#define LI_LOAD_TO_LDS_BY(lanes, base, voff, lptr)                                                       \
+    asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\tglobal_load_lds_dwordx4 %1, %2\n\ts_mov_b64 exec, -1"   \
+                 :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(voff), "s"(base), "s"(lanes) : "memory", "m0")
+
+template <int BM, int BN, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0>
+__global__ __launch_bounds__(256) void gemm_bf16_tile_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                              const float* __restrict__ bias, TO* __restrict__ out, int M, int N, int K,
+                                                              float accumulate, LiAct ep) {
+    // ACT: an activation, of gate and up columns (see gated_bf16) or of the sums (its number); its constants are in `ep`
+    constexpr int BK = 64;
+    constexpr int TM = BM / 32, TN = BN / 32;                    // 16-row and 16-column pieces of a wave
+    static_assert(BM % 64 == 0 && BN % 32 == 0 && NSTAGE >= 2, "bands of 32 rows a wave, pieces of 16 columns");
+    static_assert(!SWIGLU || TN % 2 == 0, "gate and up columns in turn, 16 of each");
+    constexpr int WM = 16 * TM, WN = 16 * TN;
+    constexpr int STAGE = (BM + BN) * BK, LPW = TM + TN;         // elements of a stage; loads a wave issues for it
+    // (a set of T pieces a wave is 32 T rows of a stage, 4 T load instructions of 8 rows, T of them a wave's)
+    struct Half { int a0, a1, b0, b1; };
+    constexpr Half T{(TM + 1) / 2, TM / 2, (TN + 1) / 2, TN / 2};
+    constexpr int TA[2] = {T.a0, T.a1}, TB[2] = {T.b0, T.b1};
+    extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wi = wave >> 1, wj = wave & 1;
+    const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
+    int mt, nt, split;
+    if (!TileOrder(mtiles).tile(blockIdx.x, mtiles, ntiles, 1, mt, nt, split)) return;
+    const int m0 = mt * BM, n0 = nt * BN;
+    const int half_n = N / 2;                                    // (SWIGLU: w is [gate; up] of N / 2 rows each)
+
+    // a lane's part of a load: the row of x or w, from the tile's first, as a byte offset that never changes
+    uint32_t ga[TM], gb[TN];
+    const bf16_t* abase = x + (size_t)m0 * K;
+    const bf16_t* bbase = w + (size_t)(SWIGLU ? n0 / 2 : n0) * K;
+    const int sub = lane >> 3;                                   // row of the 8 of an instruction
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int h = i < TA[0] ? 0 : 1, t = TA[h];
+        const int in = (wave * t + (i - h * TA[0])) * 8 + sub;   // row within the half
+        const int row = (in / (16 * t)) * WM + h * TA[0] * 16 + in % (16 * t);
+        const int c = (lane & 7) ^ (in & 7);
+        ga[i] = (uint32_t)(((size_t)(m0 + row < M ? row : M - 1 - m0) * K + 8 * c) * 2);       // rows past the end: the last row
+    }
+#pragma unroll
+    for (int i = 0; i < TN; ++i) {
+        const int h = i < TB[0] ? 0 : 1, t = TB[h];
+        const int in = (wave * t + (i - h * TB[0])) * 8 + sub;
+        const int col = (in / (16 * t)) * WN + h * TB[0] * 16 + in % (16 * t);
+        const int c = (lane & 7) ^ (in & 7);
+        size_t rel = n0 + col < N ? col : N - 1 - n0;
+        if constexpr (SWIGLU) {                                  // 16 gate rows, the 16 up rows of the same outputs, and so on
+            const int o = n0 / 2 + (col / 32) * 16 + col % 16;
+            rel = (size_t)((o < half_n ? o : half_n - 1) - n0 / 2) + (size_t)((col >> 4) & 1) * half_n;
+        }
+        gb[i] = (uint32_t)((rel * K + 8 * c) * 2);
+    }
+    const int nk = K / BK;
+    // a step that there is: all lanes (the loads of a step past the last count like any other, but ask for nothing)
+    auto lanes_of = [&](int t) { return __builtin_amdgcn_readfirstlane((t - nk) >> 31); };
+
+    // loads l of a step: A half 0, B half X, B half Y, A half 1 (X = par), in the order they are issued
+    auto issue_one = [&](auto par_tag, auto l_tag, int stage, int kt, int lanes) {
+        constexpr int X = decltype(par_tag)::value, Y = X ^ 1, l = decltype(l_tag)::value;
+        constexpr bool is_a = l < TA[0] || l >= TA[0] + TB[0] + TB[1], second = l >= TA[0] + TB[X];
+        constexpr int h = is_a ? (l < TA[0] ? 0 : 1) : (second ? Y : X);
+        constexpr int i = is_a ? (h ? l - TA[0] - TB[0] - TB[1] : l) : l - TA[0] - (second ? TB[X] : 0);
+        constexpr int t = is_a ? TA[h] : TB[h], first = is_a ? h * TA[0] : h * TB[0];
+        const bf16_t* base = (is_a ? abase : bbase) + (size_t)kt * BK;
+        const uint32_t off = is_a ? ga[is_a ? first + i : 0] : gb[is_a ? 0 : first + i];
+        uint16_t* to = lds + stage * STAGE + ((is_a ? 0 : BM) + first * 32 + (wave * t + i) * 8) * BK;
+        LI_LOAD_TO_LDS_BY(lanes, base, off, to);
+    };
+    // (the sums start as products of zeros: like this they are in the matrix cores' registers from the first to the last)
+    floatx4 acc[TM][TN];
+    bf16x8 none = {0, 0, 0, 0, 0, 0, 0, 0};
+    asm volatile("s_nop 4" : "+v"(none));                        // (written by the vector ALU: a few cycles before the MFMAs may read it)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %1, 0" : "=a"(acc[i][j]) : "v"(none));
+    bf16x8 af[TM][2], bf[TN][2];                                 // a step's operands: [piece][first or second 32 k-values]
+    // a lane's place in a piece of 16 rows: row lane % 16, the 8 k-values of group lane / 16 (of 4 in 32)
+    const int place0 = (lane & 15) * BK + (((lane >> 4) ^ (lane & 7)) << 3), place1 = place0 ^ 32;
+    auto read_a = [&](int i, int kk, int stage) {
+        const int h = i < TA[0] ? 0 : 1;
+        af[i][kk] = *reinterpret_cast<const bf16x8*>(&lds[stage * STAGE + (h * TA[0] * 32 + wi * TA[h] * 16 + (i - h * TA[0]) * 16) * BK + (kk ? place1 : place0)]);
+    };
+    auto read_b = [&](int j, int kk, int stage) {
+        const int h = j < TB[0] ? 0 : 1;
+        bf[j][kk] = *reinterpret_cast<const bf16x8*>(&lds[stage * STAGE + (BM + h * TB[0] * 32 + wj * TB[h] * 16 + (j - h * TB[0]) * 16) * BK + (kk ? place1 : place0)]);
+    };
+    // (a wave's loads retire in order: allowing the younger ones waits exactly for the oldest; the reads of LDS are done too)
+#define LI_ARRIVED(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x0070)
+#define LI_MEET()                                                                                          \
+    { asm volatile("" ::: "memory"); __builtin_amdgcn_s_barrier(); asm volatile("" ::: "memory"); __builtin_amdgcn_sched_barrier(0); }
+    static_assert((NSTAGE - 1) * LPW <= 63, "vmcnt counts to 63");
+    static_for<NSTAGE>([&](auto t_tag) {                         // (as if issued NSTAGE steps earlier)
+        constexpr int t = decltype(t_tag)::value;
+        const int lanes = lanes_of(t);
+        static_for<LPW>([&](auto l_tag) { issue_one(std::integral_constant<int, (t + NSTAGE) & 1>{}, l_tag, t, t, lanes); });
+    });
+    // Steps are taken two by two: behind an odd number of them comes one of zeros
+    auto zeros = [&](int stage) {
+        for (int i = tid; i < STAGE / 8; i += 256) *reinterpret_cast<uint4*>(&lds[stage * STAGE + 8 * i]) = uint4{0u, 0u, 0u, 0u};
+    };
+    if (nk & 1 && nk < NSTAGE) zeros(nk);
+    LI_ARRIVED((NSTAGE - 1) * LPW);
+    LI_MEET()
+#pragma unroll
+    for (int i = 0; i < TA[0]; ++i) { read_a(i, 0, 0); read_a(i, 1, 0); }
+#pragma unroll
+    for (int j = 0; j < TB[0]; ++j) { read_b(j, 0, 0); read_b(j, 1, 0); }
+    __builtin_amdgcn_s_waitcnt(0xC07F);                          // lgkmcnt(0)
+    LI_MEET()
+    // step kt, X = par (the last one reads a next stage that is not multiplied)
+    auto step = [&](auto par_tag, int kt, int stage, int next) {
+        constexpr int X = decltype(par_tag)::value, Y = X ^ 1;
+        const int lanes = lanes_of(kt + NSTAGE);
+        constexpr int H1 = TA[0] + TB[X], H2 = TB[Y] + TA[1];
+        // quarter q of rows ah and columns bh; reads: half rh of A (or B) from stage rs; loads l0 .. l1 of the step
+        auto quarter = [&](auto ah_t, auto bh_t, auto isa_t, auto rh_t, int rs, auto l0_t, auto l1_t) {
+            constexpr int ah = decltype(ah_t)::value, bh = decltype(bh_t)::value, rh = decltype(rh_t)::value;
+            constexpr bool isa = decltype(isa_t)::value;
+            constexpr int l0 = decltype(l0_t)::value, NL = decltype(l1_t)::value - l0;
+            constexpr int P = TA[ah] * TB[bh], G = 2 * P;        // MFMAs: all pieces for the first 32 k-values, then for the others
+            constexpr int R = 2 * (isa ? TA[rh] : TB[rh]);
+            constexpr int GR = G * 5 / 8 > 0 ? G * 5 / 8 : 1;    // the reads go out before the first five eighths of them
+            static_for<G>([&](auto m_tag) {
+                constexpr int m = decltype(m_tag)::value;
+                constexpr int r0 = m < GR ? (m * R + GR - 1) / GR : R, r1 = m + 1 < GR ? ((m + 1) * R + GR - 1) / GR : R;
+                static_for<r1 - r0>([&](auto r_tag) {
+                    // (the first 32 k-values of all pieces first, as they are multiplied)
+                    constexpr int r = r0 + decltype(r_tag)::value, n = R / 2, p = r % (n > 0 ? n : 1), kk = r / (n > 0 ? n : 1);
+                    if constexpr (isa) read_a(rh * TA[0] + p, kk, rs); else read_b(rh * TB[0] + p, kk, rs);
+                });
+                constexpr int kk = m / P, i = ah * TA[0] + (m % P) / TB[bh], j = bh * TB[0] + (m % P) % TB[bh];
+                asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(af[i][kk]), "v"(bf[j][kk]));
+                constexpr int a = l0 + (m * NL) / G, b = l0 + ((m + 1) * NL) / G;
+                static_for<b - a>([&](auto l_tag) { issue_one(par_tag, std::integral_constant<int, a + decltype(l_tag)::value>{}, stage, kt + NSTAGE, lanes); });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        };
+        constexpr std::integral_constant<int, 0> c0{};
+        constexpr std::integral_constant<int, 1> c1{};
+        constexpr std::integral_constant<int, X> cx{};
+        constexpr std::integral_constant<int, Y> cy{};
+        quarter(c0, cx, std::false_type{}, cy, stage, c0, std::integral_constant<int, H1 / 2>{});
+        quarter(c0, cy, std::true_type{}, c1, stage, std::integral_constant<int, H1 / 2>{}, std::integral_constant<int, H1>{});
+        // A half 0 and B half Y (the next step's X) of the next step: behind them its other loads, whole steps, this step's
+        // first half.  (With an odd number of stages that B half came second among its step's B halves.)
+        LI_ARRIVED((NSTAGE % 2 ? TA[1] : TB[X] + TA[1]) + (NSTAGE - 2) * LPW + H1);
+        LI_MEET()
+        quarter(c1, cy, std::true_type{}, c0, next, std::integral_constant<int, H1>{}, std::integral_constant<int, H1 + H2 / 2>{});
+        quarter(c1, cx, std::false_type{}, cy, next, std::integral_constant<int, H1 + H2 / 2>{}, std::integral_constant<int, LPW>{});
+        if (nk & 1 && kt + NSTAGE == nk) zeros(stage);
+        LI_ARRIVED((NSTAGE - 1) * LPW);
+        LI_MEET()
+    };
+    auto after = [](int s) { return s + 1 == NSTAGE ? 0 : s + 1; };
+    constexpr std::integral_constant<int, 0> even{};
+    constexpr std::integral_constant<int, 1> odd{};
+    int kt = 0, s = 0;
+    do {
+        const int s1 = after(s), s2 = after(s1);
+        step(even, kt, s, s1);
+        step(odd, kt + 1, s1, s2);
+        s = s2;
+        kt += 2;
+    } while (kt < nk);
+#undef LI_ARRIVED
+#undef LI_MEET
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();                               // the main loop's LDS is free now
+    constexpr int EW = SWIGLU ? WN / 2 : WN;       // output columns of a wave
+    constexpr int ESTRIDE = EW + 4;                // floats of a band's row: the four groups of rows of a piece on different banks
+    static_assert(4 * 32 * ESTRIDE * 4 <= NSTAGE * STAGE * 2, "the waves' bands fit the main loop's LDS");
+    float* band = reinterpret_cast<float*>(lds) + wave * 32 * ESTRIDE;
+    const int ccol = lane & 15, crow = (lane >> 4) * 4;
+#pragma unroll
+    for (int i = 0; i < TM; i += 2) {
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int j = 0; j < TN; j += SWIGLU ? 2 : 1)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    float v = acc[i + u][j][r];
+                    if constexpr (SWIGLU) v = gated_bf16<ACT>(v, acc[i + u][j + 1][r], ep);
+                    band[(16 * u + crow + r) * ESTRIDE + (SWIGLU ? 8 : 16) * j + ccol] = v;
+                }
+        __builtin_amdgcn_wave_barrier();
+        band_to_memory<EW, ESTRIDE, SWIGLU, ACT, TO>(band, m0 + wi * WM + 16 * i, (SWIGLU ? n0 / 2 : n0) + wj * EW, M,
+                                                     SWIGLU ? N / 2 : N, SWIGLU ? nullptr : bias, out, SWIGLU ? 0.f : accumulate, ep);
+    }
+}
+
+template <int BM, int BN, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0>
+static int launch_tile(const bf16_t* x, const bf16_t* w, const float* bias, TO* out, int M, int N, int K,
+                       float accumulate, hipStream_t stream, LiAct ep = {}) {
+    const long mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
+    if (K % 64) return LI_ERR_SIZE;
+    const long blocks = TileOrder::blocks(mtiles, ntiles);
+    if (blocks > 0x7fffffffL) return LI_ERR_SIZE;
+    // a lane's byte offset from its tile's first row is kept in 32 bits (the gate and up rows of a
+    // SwiGLU tile lie N / 2 rows apart)
+    const unsigned long long span_rows = SWIGLU ? (unsigned long long)N / 2 + BN : (unsigned long long)(BM > BN ? BM : BN);
+    if (span_rows * (unsigned long long)K * 2ull >= (1ull << 32)) return LI_ERR_SIZE;
+    constexpr int lds_bytes = NSTAGE * (BM + BN) * 64 * 2;
+    static bool configured = false;
+    if (!configured) {
+        if (hipFuncSetAttribute((const void*)gemm_bf16_tile_kernel<BM, BN, NSTAGE, SWIGLU, TO, ACT>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
+            return LI_ERR_LAUNCH;
+        configured = true;
+    }
+    gemm_bf16_tile_kernel<BM, BN, NSTAGE, SWIGLU, TO, ACT><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, ep);
     return li_launch_status();
 }
 
@@ -2083,19 +2333,39 @@ static double tile_cost(int bm, int bn, double speed, int M, int N, int K) {
     return rounds * ((K / 64) * (mfma_us > load_us ? mfma_us : load_us) + 2.0);
 }
 
-// Seven tilings for more than 64 rows; the one with the least estimated time is taken (tile_cost).  The two with four
-// waves one above the other take any multiple of 32 columns: 224 or 288 columns cut 3,584 or 4,608 into exactly as many
-// tiles as 2,048 rows need to give every compute unit one.
-static int tiling_of(int M, int N, int K) {
-    static const struct { int bm, bn; double speed; } shape[7] = {{256, 256, 1.0}, {256, 192, 0.95}, {256, 128, 1.0}, {192, 128, 0.95},
-                                                                    {128, 128, 0.8}, {128, 224, 0.9}, {128, 288, 0.9}};
+// Tiles of more than 64 rows: the one with the least estimated time is taken, in microseconds: rounds of tiles over the compute
+// units (a last round that does not fill the chip counts for 0.3 less than a whole one: the units that run clock higher and
+// have the memory to themselves) x (steps of 64 k-values x `step_us`, and the tile's start and end: 95 ns for 1,024 results
+// and 29 for each byte of theirs that goes to memory or comes from there, of 1,024).  `step_us` as measured with the chip
+// full: tiles up to 128 x 288 and 192 x 192 take in 55 GB/s a compute unit whatever they multiply (what 256 lines of a unit's
+// cache, all on their way, bring at the latency of the lines that come from beyond the L2: the loads straight into LDS alone
+// take 130 GB/s where all of it lies there), the larger ones are bound by the MFMAs at the chip's power limit.
+// Fitted to 400 products, 80 to 6,000 rows x thirteen matrices of 896 to 7,168 rows of 896 to 27,648 and four gated ones up to
+// 55,296 rows: the tile that is taken is within 0.4 % of the best one on average, at worst 15 % (810 x 5,120 x 27,648).
+struct Tiling { int bm, bn; double step_us; };
+static double tile_us(const Tiling& t, int bytes, int M, int N, int K) {
+    const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    const int cu = compute_units();
+    const double filled = (double)tiles / cu, whole = (double)((tiles + cu - 1) / cu);
+    return (filled + 0.7 * (whole - filled)) * (K / 64 * t.step_us + (double)t.bm * t.bn * (9.5e-5 + 2.85e-5 * bytes));
+}
+template <int COUNT>
+static int least_us(const Tiling (&shape)[COUNT], int bytes, int M, int N, int K) {
     int pick = 0;
     double best = 0.0;
-    for (int i = 0; i < 7; ++i) {
-        const double c = tile_cost(shape[i].bm, shape[i].bn, shape[i].speed, M, N, K);
+    for (int i = 0; i < COUNT; ++i) {
+        const double c = tile_us(shape[i], bytes, M, N, K);
         if (i == 0 || c < best) { best = c; pick = i; }
     }
     return pick;
+}
+// The first three are gemm_bf16_dma_kernel's, the others gemm_bf16_tile_kernel's: where a step has few MFMAs, whole stages and one
+// barrier a step are the faster form (128 x 128 x 3,584: 60 us against 64 for 2,048 x 3,584 results, 192 x 128 75 against 79),
+// with more of them the stage handed back in pieces (256 x 256, 8,192^3: 827 -> 726 us; 2,048 x 37,888 x 3,584 gated 483 -> 406).
+static int tiling_of(int M, int N, int K, int bytes) {
+    static const Tiling shape[7] = {{128, 128, 0.50}, {192, 128, 0.61}, {256, 128, 0.75}, {192, 224, 0.965}, {192, 256, 1.083},
+                                    {256, 224, 1.234}, {256, 256, 1.384}};
+    return least_us(shape, bytes, M, N, K);
 }
 
 // More than 64 rows but so few 128 x 128 tiles that half of the compute units would idle (a narrow
@@ -2294,19 +2564,18 @@ extern "C" int li_linear(const void* x, const void* w, const float* bias, void* 
                     else splitk_reduce_kernel<bf16_t><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, accumulate);
                     return li_launch_status();
                 }
-#define LI_DMA4(BM, BN, BK, NS) (out_dtype == LI_F32 ? launch_dma<BM, BN, BK, NS, false, float, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (float*)out, M, N, K, accumulate, stream) \
-                                                : launch_dma<BM, BN, BK, NS, false, bf16_t, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, accumulate, stream))
-                const int pick = tiling_of(M, N, K);
-                switch (pick) {
-                case 0: return LI_DMA(256, 256, 64, 2);
-                case 1: return LI_DMA(256, 192, 64, 2);
+#define LI_TILE(BM, BN, NS) (out_dtype == LI_F32 ? launch_tile<BM, BN, NS, false, float>((const bf16_t*)x, (const bf16_t*)w, bias, (float*)out, M, N, K, accumulate, stream) \
+                                        : launch_tile<BM, BN, NS, false, bf16_t>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, accumulate, stream))
+                switch (tiling_of(M, N, K, out_dtype == LI_BF16 ? 2 : accumulate != 0.f ? 8 : 4)) {
+                case 0: return LI_DMA(128, 128, 64, 4);
+                case 1: return LI_DMA(192, 128, 64, 3);
                 case 2: return LI_DMA(256, 128, 64, 3);
-                case 3: return LI_DMA(192, 128, 64, 3);
-                case 4: return LI_DMA(128, 128, 64, 4);
-                case 5: return LI_DMA4(128, 224, 64, 3);
-                default: return LI_DMA4(128, 288, 64, 3);
+                case 3: return LI_TILE(192, 224, 2);
+                case 4: return LI_TILE(192, 256, 2);
+                case 5: return LI_TILE(256, 224, 2);
+                default: return LI_TILE(256, 256, 2);
                 }
-#undef LI_DMA4
+#undef LI_TILE
             }
 #undef LI_DMA
             return LI_BIG(128, 128, 64);             // K not a multiple of 64: loads staged in registers
@@ -2367,21 +2636,23 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
         else splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
         return li_launch_status();
     }
-#define LI_ACT(BM, BN, NS, WLM) launch_dma<BM, BN, 64, NS, false, bf16_t, WLM, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
+#define LI_ACT(BM, BN, NS) launch_dma<BM, BN, 64, NS, false, bf16_t, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
+#define LI_ACT_TILE(BM, BN, NS) launch_tile<BM, BN, NS, false, bf16_t, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, ep)
     if (M <= 64) {                                   // (as linear_mid_rows takes them)
-        if ((N + 255) / 256 >= 128) return LI_ACT(64, 256, 3, 2);
-        if ((N + 127) / 128 >= 128) return LI_ACT(64, 128, 4, 2);
+        if ((N + 255) / 256 >= 128) return LI_ACT(64, 256, 3);
+        if ((N + 127) / 128 >= 128) return LI_ACT(64, 128, 4);
         return -1;
     }
-    switch (tiling_of(M, N, K)) {
-    case 0: return LI_ACT(256, 256, 2, 2);
-    case 1: return LI_ACT(256, 192, 2, 2);
-    case 2: return LI_ACT(256, 128, 3, 2);
-    case 3: return LI_ACT(192, 128, 3, 2);
-    case 4: return LI_ACT(128, 128, 4, 2);
-    case 5: return LI_ACT(128, 224, 3, 4);
-    default: return LI_ACT(128, 288, 3, 4);
+    switch (tiling_of(M, N, K, 2)) {
+    case 0: return LI_ACT(128, 128, 4);
+    case 1: return LI_ACT(192, 128, 3);
+    case 2: return LI_ACT(256, 128, 3);
+    case 3: return LI_ACT_TILE(192, 224, 2);
+    case 4: return LI_ACT_TILE(192, 256, 2);
+    case 5: return LI_ACT_TILE(256, 224, 2);
+    default: return LI_ACT_TILE(256, 256, 2);
     }
+#undef LI_ACT_TILE
 #undef LI_ACT
 }
 
@@ -2442,7 +2713,7 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
             const double c = tile_cost(64, widths[i], 1.0, M, N, K);
             if (pick < 0 || c < best) { best = c; pick = i; }
         }
-#define LI_SW64_AS(BN, NS, ACT) launch_dma<64, BN, 64, NS, true, bf16_t, 2, ACT>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, ep)
+#define LI_SW64_AS(BN, NS, ACT) launch_dma<64, BN, 64, NS, true, bf16_t, ACT>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, row_parts, nparts, eps, ep)
 #define LI_SW64(BN, NS) (act == LI_ACT_CLAMPED ? LI_SW64_AS(BN, NS, LI_ACT_CLAMPED) : act ? LI_SW64_AS(BN, NS, LI_ACT_GELU_TANH) : LI_SW64_AS(BN, NS, 0))
         if (pick == 0) return LI_SW64(256, 3);
         if (pick == 1) return LI_SW64(192, 4);
@@ -2461,31 +2732,30 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
     }
     if (M <= 64) return li_linear_skinny(x, w, nullptr, out, M, I, K, LI_BF16, 0, 1, stream);
     if (K % 64) return LI_ERR_SIZE;
-#define LI_DMA_AS(BM, BN, BK, NS, WLM, ACT) launch_dma<BM, BN, BK, NS, true, bf16_t, WLM, ACT>((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
-#define LI_DMA(BM, BN, BK, NS, WLM) (act == LI_ACT_CLAMPED ? LI_DMA_AS(BM, BN, BK, NS, WLM, LI_ACT_CLAMPED) : act ? LI_DMA_AS(BM, BN, BK, NS, WLM, LI_ACT_GELU_TANH) : LI_DMA_AS(BM, BN, BK, NS, WLM, 0))
-    // (a tile's columns are gate and up columns in turn, 32 of each: its width is a multiple of 64)
-    // (128 x 320: 160 gate columns in one wave, their ups in the wave beside it; for portions of a few hundred rows,
-    // where no other width comes near whole rounds of the compute units: 512 rows against the 1.5B's 17,920
-    // columns are 224 tiles of it, one round: 45.2 -> 38.7 us.  From four rows of tiles on: with two, 256 rows
-    // against the 7B's 37,888 columns, it measured 107 us against the 101 us of 148 tiles of 256 x 256, which
-    // read w once)
-    static const struct { int bm, bn; double speed; } shape[6] = {{256, 256, 1.0}, {256, 128, 1.0}, {128, 256, 1.0}, {128, 128, 0.8}, {128, 192, 0.9},
-                                                                  {128, 320, 0.9}};
-    int pick = 0;
-    double best = 0.0;
-    for (int i = 0; i < 6; ++i) {
-        if (i == 5 && M <= 3 * 128) continue;
-        const double c = tile_cost(shape[i].bm, shape[i].bn, shape[i].speed, M, N, K);
-        if (i == 0 || c < best) { best = c; pick = i; }
+#define LI_GATED(LAUNCH, ...) LAUNCH((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, __VA_ARGS__)
+#define LI_DMA_AS(BM, BN, NS, ACT) LI_GATED((launch_dma<BM, BN, 64, NS, true, bf16_t, ACT>), 1, nullptr, 0, 0.f, ep)
+#define LI_DMA(BM, BN, NS) (act == LI_ACT_CLAMPED ? LI_DMA_AS(BM, BN, NS, LI_ACT_CLAMPED) : act ? LI_DMA_AS(BM, BN, NS, LI_ACT_GELU_TANH) : LI_DMA_AS(BM, BN, NS, 0))
+#define LI_TILE_AS(BM, BN, NS, ACT) LI_GATED((launch_tile<BM, BN, NS, true, bf16_t, ACT>), ep)
+#define LI_TILE(BM, BN, NS) (act == LI_ACT_CLAMPED ? LI_TILE_AS(BM, BN, NS, LI_ACT_CLAMPED) : act ? LI_TILE_AS(BM, BN, NS, LI_ACT_GELU_TANH) : LI_TILE_AS(BM, BN, NS, 0))
+    // (the first two are gemm_bf16_dma_kernel's, see tiling_of; a tile's columns are gate and up columns in turn.  Wide ones of
+    // 128 rows for steps of a few hundred rows or a few more than a multiple of 256: 1,027 rows against the 1.5B's 17,920 columns
+    // are 504 tiles of 128 x 320, two rounds: 69 -> 58 us)
+    static const Tiling shape[9] = {{128, 128, 0.551}, {128, 256, 0.885}, {128, 192, 0.70}, {128, 320, 1.036}, {128, 384, 1.214},
+                                    {192, 256, 1.087}, {192, 320, 1.314}, {256, 192, 1.075}, {256, 256, 1.378}};
+    switch (least_us(shape, 1, M, N, K)) {
+    case 0: return LI_DMA(128, 128, 4);
+    case 1: return LI_DMA(128, 256, 3);
+    case 2: return LI_TILE(128, 192, 4);
+    case 3: return LI_TILE(128, 320, 2);
+    case 4: return LI_TILE(128, 384, 2);
+    case 5: return LI_TILE(192, 256, 2);
+    case 6: return LI_TILE(192, 320, 2);
+    case 7: return LI_TILE(256, 192, 2);
+    default: return LI_TILE(256, 256, 2);
     }
-    switch (pick) {
-    case 0: return LI_DMA(256, 256, 64, 2, 2);
-    case 1: return LI_DMA(256, 128, 64, 3, 2);
-    case 2: return LI_DMA(128, 256, 64, 3, 2);
-    case 3: return LI_DMA(128, 128, 64, 4, 2);
-    case 4: return LI_DMA(128, 192, 64, 3, 4);
-    default: return LI_DMA(128, 320, 64, 2, 2);
-    }
+#undef LI_TILE
+#undef LI_TILE_AS
+#undef LI_GATED
 #undef LI_DMA
 #undef LI_DMA_AS
 }

@@ -75,8 +75,8 @@ def test_rmsnorm_zero_row_is_zero_not_nan(ops):
     ((9, 18, 4), True, False),
     ((300, 200, 130), True, True), ((256, 128, 64), False, False), ((1000, 333, 1027), True, False),     # the large 32-bit tile
     ((2048, 3584, 128), True, True), ((2000, 4600, 64), True, False),           # tiles of 256 x 128 and 256 x 256, ragged
-    ((1100, 4600, 128), True, True), ((1167, 6627, 128), False, False),         # 192 x 128 and 256 x 192: a last row of tiles with few rows
-    ((585, 3979, 128), True, False), ((779, 6296, 128), False, True)])          # four waves one above the other: 128 x 224 and 128 x 288
+    ((1100, 4600, 128), True, True), ((1167, 6627, 128), False, False),         # tiles of 192 and more: a last row of tiles with few rows
+    ((585, 3979, 128), True, False), ((779, 6296, 128), False, True)])          # columns that few tiles divide
 def test_linear(ops, dtype, mnk, bias, acc):
     m, n, k = mnk
     g = torch.Generator().manual_seed(2)
@@ -94,6 +94,58 @@ def test_linear(ops, dtype, mnk, bias, acc):
     # operands are exact in both dtypes; what differs is the float32 accumulation over K terms
     # (a random-walk error of about sqrt(K) half-ulps) and, for a bfloat16 out, its rounding
     assert rel(out, ref) < (4 * math.sqrt(k) * 2.0 ** -24 if out.dtype is torch.float32 else 5e-3)
+
+
+# Tiles whose stages are handed back in pieces (gemm_bf16_tile_kernel), each one by its sizes: rows and columns past the last, widths
+# that no 16-byte piece divides, and one, an odd number and an even number of steps of 64 k-values.
+@pytest.mark.parametrize("m,n,k,form", [
+    (129, 32771, 64, "residual"), (129, 32776, 192, "bf16"), (769, 20488, 256, "relu2"),               # 192 x 224
+    (641, 14344, 64, "residual"), (385, 20491, 320, "residual"), (705, 14341, 64, "bf16"), (385, 20488, 192, "relu2"),     # 192 x 256
+    (385, 24584, 192, "residual"), (193, 32776, 320, "bf16"), (385, 24589, 128, "residual"),           # 256 x 224
+    (769, 14344, 192, "residual"), (1537, 8200, 448, "residual"),                                      # 256 x 256
+    (129, 8203, 64, "gated"), (130, 8200, 192, "gelu_gate"),                                           # 128 x 192
+    (129, 16388, 320, "gated"), (257, 16388, 64, "clamped"), (300, 16385, 128, "gated"),               # 128 x 320, 192 x 320
+    (385, 10244, 192, "gated"), (385, 10241, 64, "gelu_gate"),                                         # 256 x 192
+    (513, 8200, 320, "gated"), (577, 8200, 64, "gated"), (577, 8203, 192, "clamped"),                  # 192 x 256, 128 x 384
+    (641, 10244, 64, "gelu_gate"), (577, 10241, 192, "gated"), (600, 10244, 448, "clamped")])          # 256 x 256
+def test_linear_in_large_tiles(ops, m, n, k, form):
+    g = torch.Generator(device=DEV).manual_seed(91)
+    gated = form in ("gated", "gelu_gate", "clamped")
+    x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
+    w = (torch.randn((2 if gated else 1) * n, k, generator=g, device=DEV) * 2 / math.sqrt(k)).bfloat16()
+    y = x.double() @ w.double().t()
+    # the float32 sums of K products (a random walk of half-ulps of terms of size y), carried on by slopes of 3 at most
+    slack = 12 * math.sqrt(k) * 2.0 ** -24 * (1 + y.abs())
+    if gated:
+        gate, up = y[:, :n], y[:, n:]
+        slack = (slack[:, :n] + slack[:, n:]) * (1 + gate.abs() + up.abs())
+        limit = {"gated": 0.0, "gelu_gate": ops.GELU_TANH_GATE, "clamped": 1.5}[form]
+        if form == "gated":
+            want = up * gate * torch.sigmoid(gate)
+        elif form == "gelu_gate":
+            want = up * torch.nn.functional.gelu(gate, approximate="tanh")
+        else:
+            gc, uc = gate.clamp(max=1.5), up.clamp(-1.5, 1.5)
+            want = gc * torch.sigmoid(1.702 * gc) * (uc + 1)
+        out = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+        ops.linear_swiglu(x, w, out, limit=limit)
+    else:
+        b = torch.randn(n, generator=g, device=DEV)
+        y = y + b.double()
+        if form == "residual":
+            out = torch.randn(m, n, generator=g, device=DEV)
+            want = out.double() + 0.5 * y
+            ops.linear(x, w, b, out, accumulate=True, factor=0.5)
+        elif form == "bf16":
+            out, want = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV), y
+            ops.linear(x, w, b, out)
+        else:
+            out, want = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV), y.clamp(min=0) ** 2
+            slack = slack * (1 + y.abs())
+            assert ops.linear_act(x, w, b, out, "relu2", (0.0, 0.0), None)
+    if out.dtype is torch.bfloat16:
+        slack = slack + want.abs() * 2.0 ** -8
+    assert bool(((out.double() - want).abs() <= slack).all())
 
 
 @pytest.mark.parametrize("m,n,k,swiglu,out_dtype,bias,acc", [
@@ -294,10 +346,10 @@ def test_linear_into_the_residual_sum_with_its_norm(ops, m, n, k, bias, taken):
     (300, 1000, 192),            # several tiles both ways, ragged edges
     (700, 4700, 256),            # tiles of 256 x 128
     (2048, 18944, 128),          # enough tiles for the largest tiling
-    (97, 7419, 128),             # few rows against many columns: tiles of 128 x 192, four waves one above the other
+    (97, 7419, 128),             # few rows against many columns: tiles of 128 x 192
     (300, 9001, 128),            # tiles of 128 x 256
     (1101, 2500, 192),           # nine rows of tiles: the last XCD's share of the tiles is short
-    (1024, 4800, 192),           # tiles of 128 x 320: 160 gate columns in one wave, their ups in the wave beside it
+    (1024, 4800, 192),           # tiles of 128 x 320
     (2000, 4793, 192),           # the same with ragged edges both ways
 ])
 def test_linear_with_swiglu_epilogue(ops, m, n, k):
