@@ -334,13 +334,14 @@ __device__ __forceinline__ void radix_kth(Each&& each, int kk, uint32_t& tau, in
 // radix_kth then.
 // 64 rows of 151,936 ids, top-k 50: tiles kernel 58 -> 45 us (one row 26 -> 13), rows kernel 22 -> 14.
 constexpr int SMP_LIST = 1024;
-__device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int waves, uint32_t& tau, int& need, uint32_t* list, int* work_i, int* res) {
-    const int tid = threadIdx.x, lane = tid & (LI_WAVE - 1), w = tid / LI_WAVE;
+// the bound, as above (0: none): at least kk of the block's keys are no smaller
+__device__ __forceinline__ uint32_t bound_of_kth(const uint32_t (&key)[8], int kk, int waves, int* work_i) {
+    const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
     uint32_t cur = key[0];
 #pragma unroll
     for (int e = 1; e < 8; ++e) cur = max(cur, key[e]);
     const int rounds = (kk + waves - 1) / waves;
-    if (rounds > LI_WAVE) return false;
+    if (rounds > LI_WAVE) return 0u;
     // the rounds-th largest of the wave's keys, bit by bit, down to the sixteenth (a bound; 0: the wave has fewer)
     uint32_t largest = 0u;
 #pragma unroll
@@ -354,22 +355,24 @@ __device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int
     uint32_t bound = 0xffffffffu;
 #pragma unroll
     for (int i = 0; i < SMP_WAVES; ++i) bound = i < waves ? min(bound, (uint32_t)work_i[i] - 1u) : bound;      // (0, no bound, becomes the largest)
-    bound += 1u;
-    if (bound == 0u) return false;
+    return bound + 1u;
+}
+// put(place, e) for the keys no smaller than the bound, in the order of threads and keys; how many they are is left in res[0] (and is
+// there for all threads behind the next barrier)
+template <typename Put>
+__device__ __forceinline__ void put_from(const uint32_t (&key)[8], uint32_t bound, int* work_i, int* res, Put&& put) {
     int mine = 0;
 #pragma unroll
     for (int e = 0; e < 8; ++e) mine += key[e] >= bound;
     int pos = block_sum_before(mine, work_i);
-    if (tid == SMP_NT - 1) res[0] = pos + mine;
+    if (threadIdx.x == SMP_NT - 1) res[0] = pos + mine;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
-        if (key[e] >= bound) {
-            if (pos < SMP_LIST) list[pos] = key[e];
-            ++pos;
-        }
-    __syncthreads();
-    const int n = res[0];
-    if (n < kk || n > SMP_LIST) return false;
+        if (key[e] >= bound) put(pos++, e);
+}
+// n keys in the list (n at least kk): tau and need
+__device__ __forceinline__ void kth_of_list(uint32_t* list, int n, int kk, uint32_t& tau, int& need, int* res) {
+    const int tid = threadIdx.x;
     if (tid < 4 && n + tid < SMP_LIST) list[n + tid] = 0u;      // (whole pieces of four below)
     __syncthreads();
     if (tid < n) {
@@ -386,6 +389,64 @@ __device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int
     __syncthreads();
     tau = (uint32_t)res[1];
     need = res[2];
+}
+// `tag` gives each key's own number (its id), which goes beside it into list_id; n: the keys in the list
+template <typename Tag>
+__device__ __forceinline__ bool select_kth(const uint32_t (&key)[8], int kk, int waves, uint32_t& tau, int& need, uint32_t* list, int* list_id,
+                                           int& n, int* work_i, int* res, Tag&& tag) {
+    const uint32_t bound = bound_of_kth(key, kk, waves, work_i);
+    if (bound == 0u) return false;
+    put_from(key, bound, work_i, res, [&](int at, int e) {
+        if (at < SMP_LIST) { list[at] = key[e]; list_id[at] = tag(e); }
+    });
+    __syncthreads();
+    n = res[0];
+    if (n < kk || n > SMP_LIST) return false;
+    kth_of_list(list, n, kk, tau, need, res);
+    return true;
+}
+
+// Top-p among the survivors of top-k where these lie in the list: the same tp as radix_mass and what is left of `remaining` =
+// p x (their mass), which is worked out here.  Each key of the list is held against all others: its own mass and that above it
+// (sums of four, in the list's order: they grow with every key that counts, so one key alone has the prefix's end), the
+// one whose mass above is short of `remaining` and whose own reaches it is tp; below them all the keys equal to tau.
+// False, with nothing done, where rounding or masses of zero leave none (radix_mass then).  64 rows of 151,936 ids, top-k 50 with
+// top-p 0.9: rows kernel 25 us with radix passes (up to eight, three barriers each).
+__device__ __forceinline__ bool mass_of_list(const uint32_t* list, int n, uint32_t tau, int ties, float m, float p,
+                                             float& remaining, uint32_t& tp, float* mass, float* res_f, int* res) {
+    const int tid = threadIdx.x;
+    if (tid < ((n + 3) & ~3)) mass[tid] = tid < n && list[tid] > tau ? expf(key_value(list[tid]) - m) : 0.f;
+    if (tid == 0) res[0] = 0;
+    __syncthreads();
+    const float e_ties = (float)ties * expf(key_value(tau) - m);
+    if (tid < n) {
+        const uint32_t own = list[tid];
+        float above[4] = {0.f, 0.f, 0.f, 0.f}, from[4] = {0.f, 0.f, 0.f, 0.f}, all[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+        for (int j = 0; j < n; j += 4) {                // (the list is filled up to whole pieces)
+            const uint4 v = *reinterpret_cast<const uint4*>(list + j);
+            const float4 e = *reinterpret_cast<const float4*>(mass + j);
+            const uint32_t k4[4] = {v.x, v.y, v.z, v.w};
+            const float e4[4] = {e.x, e.y, e.z, e.w};
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                above[u] += k4[u] > own ? e4[u] : 0.f;
+                from[u] += k4[u] >= own ? e4[u] : 0.f;
+                all[u] += e4[u];
+            }
+        }
+        const float g = (above[0] + above[1]) + (above[2] + above[3]), h = (from[0] + from[1]) + (from[2] + from[3]);
+        const float z = (all[0] + all[1]) + (all[2] + all[3]), want = p * (z + e_ties);
+        if (own > tau ? g < want && h >= want : own == tau && z < want && z + e_ties >= want) {
+            res[0] = 1;                                  // (all threads with this key write the same)
+            res[1] = (int)own;
+            res_f[0] = want - (own > tau ? g : z);
+        }
+    }
+    __syncthreads();
+    if (!res[0]) return false;
+    tp = (uint32_t)res[1];
+    remaining = res_f[0];
     return true;
 }
 
@@ -481,7 +542,13 @@ __device__ __forceinline__ int sample_candidates(int k, float p, int V, int ntil
     return (kc <= SMP_KC && (long)kc * ntiles <= (long)SMP_NT * SMP_CAND_PER_THREAD) ? kc : 0;
 }
 
-__global__ __launch_bounds__(SMP_NT) void sample_tiles_kernel(
+// Do SMP_KC candidates of every tile fit the second kernel's registers?  Then a tile may hand over more than kc of them: all that
+// are no smaller than a bound (tile_i: how many).
+__device__ __forceinline__ bool sample_wide(int ntiles) { return ntiles * SMP_KC <= SMP_NT * SMP_CAND_PER_THREAD; }
+
+// (eight waves a SIMD, two blocks a compute unit: with the 71 registers that the compiler would take, one block, 64 greedy rows took
+// 18 us instead of 13)
+__global__ __launch_bounds__(SMP_NT, 8) void sample_tiles_kernel(
     const float* __restrict__ logits, const float* __restrict__ temperature, const int* __restrict__ top_k,
     const float* __restrict__ top_p, float* __restrict__ tile_m, float* __restrict__ tile_s,
     int* __restrict__ tile_i, float* __restrict__ cand_z, int* __restrict__ cand_id, int V) {
@@ -510,15 +577,20 @@ __global__ __launch_bounds__(SMP_NT) void sample_tiles_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) m = fmaxf(m, z[e]);
     m = block_max_f(m, sf);
-    float sum = 0.f;
+    const int k = top_k[r], kc = sample_candidates(k, top_p[r], V, ntiles);
+    if (kc == 0 || !(k > 0 && k < V)) {                        // (behind top-k nothing is taken of the whole row's mass)
+        float sum = 0.f;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) sum += (j0 + e < V && m > -INFINITY) ? expf(z[e] - m) : 0.f;       // (a tile of -inf alone has no mass)
-    sum = block_sum<SMP_NT>(sum, sf);
-    if (tid == 0) { tile_m[slot] = m; tile_s[slot] = sum; }
-    const int kc = sample_candidates(top_k[r], top_p[r], V, ntiles);
+        for (int e = 0; e < 8; ++e) sum += (j0 + e < V && m > -INFINITY) ? expf(z[e] - m) : 0.f;       // (a tile of -inf alone has no mass)
+        sum = block_sum<SMP_NT>(sum, sf);
+        if (tid == 0) tile_s[slot] = sum;
+    }
+    if (tid == 0) tile_m[slot] = m;
     if (kc == 0) return;
-    // the tile's kc largest ids, written in id order
+    // the tile's kc largest ids, written in id order; or, where the second kernel has room for them, all from the bound on: these
+    // hold the kc largest too, and finding exactly those takes as long again
     const int in_tile = min(SMP_TILE, V - tile * SMP_TILE);
+    const size_t base = slot * SMP_KC;
     const bool all = in_tile <= kc;
     uint32_t tau = 0u;
     int need = 0x7fffffff;
@@ -526,12 +598,31 @@ __global__ __launch_bounds__(SMP_NT) void sample_tiles_kernel(
         uint32_t key[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) key[e] = j0 + e < V ? sort_key(z[e]) : 0u;
-        if (!select_kth(key, kc, max(in_tile / (8 * LI_WAVE), 1), tau, need, list, work_i, tot_i))
+        const bool wide = sample_wide(ntiles);
+        const uint32_t bound = bound_of_kth(key, kc, max(in_tile / (8 * LI_WAVE), 1), work_i);
+        bool found = false;
+        if (bound != 0u) {
+            put_from(key, bound, work_i, tot_i, [&](int at, int e) {
+                if (at < SMP_LIST) list[at] = key[e];
+                if (wide && at < SMP_KC) { cand_z[base + at] = z[e]; cand_id[base + at] = j0 + e; }
+            });
+            __syncthreads();
+            const int n = tot_i[0];
+            if (wide && n >= kc && n <= SMP_KC) {
+                if (tid == 0) tile_i[slot] = n;
+                return;
+            }
+            found = n >= kc && n <= SMP_LIST;
+            if (found) kth_of_list(list, n, kc, tau, need, tot_i);
+        }
+        if (!found) {
+            __syncthreads();                            // (tot_i has been read)
             radix_kth([&](auto f) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
                     if (j0 + e < V) f(z[e]);
             }, kc, tau, need, work_i, tot_i);
+        }
     }
     int eq = 0;
 #pragma unroll
@@ -546,7 +637,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_tiles_kernel(
         mine += in[e];
     }
     int pos = block_sum_before(mine, si);
-    const size_t base = slot * SMP_KC;
+    if (tid == SMP_NT - 1) tile_i[slot] = pos + mine;
 #pragma unroll
     for (int e = 0; e < 8; ++e)
         if (in[e]) {
@@ -570,6 +661,8 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     __shared__ float work_f[SMP_WAVES * 16], tot_f[16];
     __shared__ int work_i[SMP_WAVES * 16], tot_i[16];
     __shared__ __align__(16) uint32_t list[SMP_LIST];
+    __shared__ __align__(16) float list_e[SMP_LIST];
+    __shared__ int list_id[SMP_LIST];
     __shared__ float pick_f[3];
     __shared__ int pick_i[1];
     const int r = blockIdx.x, tid = threadIdx.x;
@@ -604,26 +697,48 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
 
     const int kc = sample_candidates(k, p, V, ntiles);
     if (kc > 0) {
-        // ---- among the candidates: slot s = tile * kc + place, ascending ids; thread t has the slots t * C ...
-        const int slots = ntiles * kc, C = (slots + SMP_NT - 1) / SMP_NT;
+        // ---- among the candidates, in ascending ids: thread t has the C of them from t * C on
         float cz[SMP_CAND_PER_THREAD];
         int cid[SMP_CAND_PER_THREAD];
         bool have[SMP_CAND_PER_THREAD];
-        const int total = (ntiles - 1) * kc + min(kc, V - (ntiles - 1) * SMP_TILE);      // candidates in all (kc < SMP_TILE)
+        const int lane = tid & (LI_WAVE - 1);
+        int total, first = 0;                       // candidates in all; those of the tiles before tile `lane` (where the tiles hold different numbers)
+        const bool wide = sample_wide(ntiles);
+        if (wide) {                                 // (up to 32 tiles: a lane each)
+            const int count = lane < ntiles ? tile_i[lane] : 0;
+            int upto = count;
+#pragma unroll
+            for (int o = 1; o < LI_WAVE; o <<= 1) {
+                const int t = __shfl_up(upto, o, LI_WAVE);
+                if (lane >= o) upto += t;
+            }
+            first = upto - count;
+            total = __shfl(upto, LI_WAVE - 1, LI_WAVE);
+        } else {
+            total = (ntiles - 1) * kc + min(kc, V - (ntiles - 1) * SMP_TILE);      // (kc < SMP_TILE)
+        }
+        const int C = (total + SMP_NT - 1) / SMP_NT;
 #pragma unroll
         for (int c = 0; c < SMP_CAND_PER_THREAD; ++c) {
             const int s = tid * C + c;
-            have[c] = false;
+            have[c] = c < C && s < total;
+            int t = 0, i = s;
+            if (wide) {
+                if (c < C) {                        // (the same for all threads) the last tile that begins at s or before it
+                    for (int step = 16; step > 0; step >>= 1)
+                        if (__shfl(first, t + step, LI_WAVE) <= s && t + step < ntiles) t += step;
+                    i = s - __shfl(first, t, LI_WAVE);
+                }
+            } else {
+                t = min(s / kc, ntiles - 1);
+                i = s - t * kc;
+            }
             cz[c] = -INFINITY;
             cid[c] = 0;
-            if (c < C && s < slots) {
-                const int t = s / kc, i = s % kc;
-                if (i < min(kc, V - t * SMP_TILE)) {
-                    const size_t at = ((size_t)r * ntiles + t) * SMP_KC + i;
-                    have[c] = true;
-                    cz[c] = cand_z[at];
-                    cid[c] = cand_id[at];
-                }
+            if (have[c]) {
+                const size_t at = ((size_t)r * ntiles + t) * SMP_KC + i;
+                cz[c] = cand_z[at];
+                cid[c] = cand_id[at];
             }
         }
         auto each = [&](auto f) {
@@ -638,11 +753,65 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
 #pragma unroll
         for (int c = 0; c < SMP_CAND_PER_THREAD; ++c) key[c] = have[c] ? sort_key(cz[c]) : 0u;
         const int kk = min(by_k ? k : kc, total);
-        const int threads = (slots + C - 1) / C;
-        if (!select_kth(key, kk, max(threads / LI_WAVE, 1), tau_c, need_c, list, work_i, tot_i)) radix_kth(each, kk, tau_c, need_c, work_i, tot_i);
-        bool exact = true;
+        const int threads = (total + C - 1) / C;
+        int n = 0;
+        const bool listed = select_kth(key, kk, max(threads / LI_WAVE, 1), tau_c, need_c, list, list_id, n, work_i, tot_i, [&](int e) { return cid[e]; });
+        if (!listed) radix_kth(each, kk, tau_c, need_c, work_i, tot_i);
+        bool exact = true, done = false;
         if (by_k) { cut = true; tau = tau_c; need = need_c; }
-        if (by_p) {
+        if (by_p && by_k && listed) {
+            // (of the candidates equal to tau, which the list holds all, `need` count)
+            float remaining;
+            uint32_t tp;
+            if (mass_of_list(list, n, tau, need, m, p, remaining, tp, list_e, pick_f, tot_i)) {
+                const int need_p = ties_needed(remaining, tp, m);
+                need = tp == tau ? min(need, need_p) : need_p;
+                tau = tp;
+                done = true;
+            }
+        }
+        if (by_k && listed && (done || !by_p)) {
+            // inverse CDF over the survivors in the list, in id order: the first wave alone, a lane the `per` next ones
+            if (tid >= LI_WAVE) return;
+            const int per = (n + LI_WAVE - 1) / LI_WAVE, from = lane * per, to = min(from + per, n);
+            int eq = 0;
+            for (int j = from; j < to; ++j) eq += list[j] == tau;
+            int rank0 = eq;
+#pragma unroll
+            for (int o = 1; o < LI_WAVE; o <<= 1) {
+                const int t = __shfl_up(rank0, o, LI_WAVE);
+                if (lane >= o) rank0 += t;
+            }
+            rank0 -= eq;                            // keys at tau before this lane's
+            auto in = [&](int j, int& rank) { return list[j] > tau || (list[j] == tau && rank++ < need); };
+            float mine = 0.f;
+            bool any = false;
+            for (int j = from, rank = rank0; j < to; ++j)
+                if (in(j, rank)) { mine += expf(key_value(list[j]) - m); any = true; }
+            float upto = mine;
+#pragma unroll
+            for (int o = 1; o < LI_WAVE; o <<= 1) {
+                const float t = __shfl_up(upto, o, LI_WAVE);
+                if (lane >= o) upto += t;
+            }
+            float run = __shfl_up(upto, 1, LI_WAVE);
+            if (lane == 0) run = 0.f;
+            const float target = uniform[r] * __shfl(upto, LI_WAVE - 1, LI_WAVE);
+            const unsigned long long reach = __ballot(any && run + mine >= target), some = __ballot(any);
+            const int chosen = reach ? __ffsll((long long)reach) - 1 : 63 - __clzll((long long)some);      // (else the last one with a survivor)
+            if (lane == chosen) {
+                int pick = -1;
+                for (int j = from, rank = rank0; j < to; ++j) {
+                    if (!in(j, rank)) continue;
+                    pick = list_id[j];
+                    run += expf(key_value(list[j]) - m);
+                    if (run >= target) break;
+                }
+                out[r] = pick;
+            }
+            return;
+        }
+        if (by_p && !done) {
             float zk = 0.f;
             int eq = 0;
             each([&](float z) {

@@ -1143,6 +1143,27 @@ def test_sample_rows_with_the_candidates_found_by_a_bound(ops, order):
                 assert _pick_is_right(rows[r], temperature, top_k[r], top_p, u[r], picks[r]), (r, top_k[r])
 
 
+@pytest.mark.parametrize("vocab", [32 * 8192, 32 * 8192 + 1, 5 * 8192 + 3])
+def test_sample_rows_with_tiles_that_hand_over_different_numbers_of_candidates(ops, vocab):
+    # up to 32 tiles hand over all ids above their own bound, more tiles exactly k of them; here one tile's large ids lie in one wave
+    # (so many above its bound that it hands over k), one has a single value, one next to nothing, the last one is cut short
+    g = torch.Generator().manual_seed(68)
+    top_k = [1, 17, 50, 200, 256, 50]
+    n = len(top_k)
+    logits = torch.randn(n, vocab, generator=g) * 3
+    logits[:, 8192:16384] = logits[:, 8192:16384].sort(dim=1).values
+    logits[:, 16384:24576] = 9.0
+    logits[5, 16384:24576] = 2.0
+    logits[:, 24576:32768 - 20] = float("-inf")
+    rows = logits.double().numpy()
+    for top_p in (1.0, 0.9, 0.05):
+        u = torch.rand(n, generator=g).tolist()
+        u[1] = 0.99999994
+        picks = _sample(ops, logits, [0.8] * n, top_k, [top_p] * n, u)
+        for r in range(n):
+            assert _pick_is_right(rows[r], 0.8, top_k[r], top_p, u[r], picks[r]), (r, top_k[r], top_p)
+
+
 def test_sample_rows_frequencies_and_ties(ops):
     lg = torch.tensor([[2.0, 1.0, 3.0, 3.0, -1.0, 0.5, 2.5, 0.0]])
     n = 4000
