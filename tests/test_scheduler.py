@@ -180,6 +180,12 @@ def test_abort_gives_everything_back():
     assert s.requests[a].finish_reason == "aborted"
 
 
+def test_uniform_numbers_of_many_rows_at_once():
+    from litinfer_amd.sampling.sampler import _uniforms, uniform
+    seeds, counters = [0, 1, -1, 2 ** 63, 2 ** 64 - 1, -2 ** 70, 12345], [0, 2 ** 64 - 1, 3, 7, 2 ** 40, 1, 99]
+    assert _uniforms(seeds, counters).tolist() == [uniform(s, c) for s, c in zip(seeds, counters)]
+
+
 def test_sampling_stream_is_per_request():
     # the k-th draw of a request depends on (seed, k) only
     assert uniform(3, 0) == uniform(3, 0) and uniform(3, 0) != uniform(3, 1) != uniform(4, 1)
