@@ -1307,17 +1307,21 @@ typedef short tr4 __attribute__((ext_vector_type(4)));
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"                        \
                  :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(gptr) : "memory", "m0")
 // P32: the page size divides 32, so a row keeps its place in its page from block to block
-template <int DH, bool P32>
+template <int DH, bool P32, int HEADS>
 __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_kernel(
     const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __restrict__ out,
     const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc, const int* __restrict__ block_table,
     int max_blocks, const int* __restrict__ tiles, const int* __restrict__ q_start,
     const int* __restrict__ q_len, const int* __restrict__ ctx_len, int nh, int nkv, int page_size,
     int num_pages, int window, float scale, int ncu, int ksplit, float* __restrict__ part_acc,
-    float* __restrict__ part_ml) {
+    float* __restrict__ part_ml, int ntiles) {
     // ksplit > 1: the tile's blocks of keys are cut into ksplit runs, blockIdx.z = part of the heads x
     // ksplit + run; a block then leaves its sums, unscaled, in part_acc [token, head, run, dh] and its
     // (maximum, sum) in part_ml, and attention_merge_runs_kernel joins the runs in their order
+    // HEADS: the block's four waves are this many heads of a group (4, 2 or 1) x 4 / HEADS tiles of a segment that follow each
+    // other, all of which read the keys that the block fetches.  Four heads and one tile where the group's heads divide by four;
+    // else waves would have no head and only help to fetch: with 5 heads a group 3 of 8.  The price is that the waves with the
+    // earlier tiles wait while the last one's newest keys are worked on (li_paged_attention_prefill_heads weighs it)
     constexpr int KS = DH / 16;                 // MFMA steps of K Q^T (16 head dimensions each)
     constexpr int HD = DH / 2;                  // head dimensions owned by one lane half
     constexpr int DT = DH / 32;                 // tiles of 32 output dimensions
@@ -1337,20 +1341,32 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     const int round = lin / ncu, pos = lin - round * ncu;
     const int in_round = total - round * ncu < ncu ? total - round * ncu : ncu;
     const int item = round * ncu + ((round & 1) ? in_round - 1 - pos : pos);
-    const int tile = gridDim.x - 1 - item / per_tile;
-    const int s = tiles[tile * 4], t0 = tiles[tile * 4 + 1], nrows = tiles[tile * 4 + 2];
+    // (tiles whose number in the list is the same modulo `abreast` follow each other: with one long segment the blocks that
+    // have nothing to do, see below, come behind the others; dealt among them they left compute units idle: 512 blocks took
+    // 935 us, as long as two rounds)
+    constexpr int abreast = PRE_WAVES / HEADS;          // tiles of a block
+    const int turn = item / per_tile, rows_of_tiles = gridDim.x / abreast;
+    const int tile = (rows_of_tiles - 1 - turn % rows_of_tiles) * abreast + turn / rows_of_tiles;
+    if (tile >= ntiles) return;
+    const int s = tiles[tile * 4], t00 = tiles[tile * 4 + 1], seg0 = q_start[s], seg_rows = q_len[s];
+    if (abreast > 1 && ((t00 - seg0) / 32) % abreast) return;          // (one of the tiles of the block before: before any barrier)
     const int kvh = (item % per_tile) / gridDim.z;      // (the parts of a group of heads are neighbours: they read the same keys)
     const int G = nh / nkv;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int zz = (item % per_tile) % gridDim.z, run = zz % ksplit;
-    const int hw = (zz / ksplit) * PRE_WAVES + wave;    // this wave's head within the group
-    const bool active = hw < G;                         // (idle waves still help to fetch and keep the barriers)
-    const int head = kvh * G + (active ? hw : 0);
+    const int hw = (zz / ksplit) * HEADS + wave % HEADS;              // this wave's head within the group
+    const int behind = 32 * (wave / HEADS);                           // its tile's first row behind the block's first
+    const int left = seg_rows - (t00 - seg0);                         // the segment's rows from the block's first on
+    const bool active = hw < G && behind < left;        // (idle waves still help to fetch and keep the barriers)
+    const int t0 = t00 + (active ? behind : 0);
+    const int nrows = left - (t0 - t00) < 32 ? left - (t0 - t00) : 32;
+    const int head = kvh * G + (hw < G ? hw : 0);
     const int ql = lane & 31, h = lane >> 5;
-    const int p0 = ctx_len[s] - q_len[s] + (t0 - q_start[s]);           // position of the tile's first token
-    const int p_last = p0 + nrows - 1;
-    const int lo0 = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
-    int k_begin = lo0 & ~31, k_end = p_last + 1;
+    const int p00 = ctx_len[s] - seg_rows + (t00 - seg0);               // position of the block's first token,
+    const int p0 = p00 + (t0 - t00), p_last = p0 + nrows - 1;           // of the wave's tile's first and last
+    const int lo0 = (window > 0 && p00 - window + 1 > 0) ? p00 - window + 1 : 0;      // the first key that any of the block's tokens sees,
+    const int lo_tile = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;    // ... the wave's
+    int k_begin = lo0 & ~31, k_end = p00 + (left < 32 * abreast ? left : 32 * abreast);
     int first_key = lo0;
     if (ksplit > 1) {                                   // this run's blocks of 32 keys
         const int all = (k_end - k_begin + 31) / 32, per = (all + ksplit - 1) / ksplit;
@@ -1503,7 +1519,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
         if (jb >= nblk) break;
         const int kb = k_begin + 32 * jb;
         if (jb + 2 < nblk) LI_PRE_FETCH((stage + 2) % NST);
-        if (active) {
+        if (active && (abreast == 1 || (kb <= p_last && kb + 31 >= lo_tile))) {
             // ---- S^T = K Q^T
             f32x16_t sv;
 #pragma unroll
@@ -2095,7 +2111,52 @@ extern "C" int li_paged_attention_prefill_runs(int nseg, const int* q_len, const
     return pick;
 }
 
+// How many heads of a group a block's four waves are (the others are tiles that follow each other): 4, 2 or 1.  q_len, ctx_len: the
+// batch's segments in HOST memory.  The estimate, in blocks of 32 keys: rounds of blocks over the chip (two a compute unit; a last
+// one that does not fill it counts for 0.4 of its rest) x the mean block's keys (those of its last tile) x what a block with so many
+// waves at work takes (measured where a round is full: 395, 460, 508 and 600 us with one to four of them; a wave waits for the
+// others' keys and its own chain either way).  A round that does not fill the chip keeps one tile a block: its time is one block's.
+// 1,999 tokens behind 16,000 keys, us, with four heads a block and as taken here: 32 heads of 32 kv heads 1,540 -> 594, 32 of
+// 16 910 -> 580; 40 of 8 940 -> 909 (a last round of 128 blocks), 2,048 tokens from their start 75 -> 65, 4,096 264 -> 202; 28 of 4
+// heads stay with four (2,048 tokens 55 us).
+extern "C" int li_paged_attention_prefill_heads(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int max_blocks, int window) {
+    if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP) return PRE_WAVES;
+    const int G = nh / nkv;
+    if (G % PRE_WAVES == 0) return PRE_WAVES;
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
+        (void)hipGetLastError();
+        ncu = 256;
+    }
+    const double at_work[PRE_WAVES + 1] = {0.0, 0.66, 0.77, 0.85, 1.0};
+    int pick = PRE_WAVES;
+    double best = 0.0;
+    for (int heads = PRE_WAVES; heads >= 1; heads /= 2) {
+        const int abreast = PRE_WAVES / heads, parts = (G + heads - 1) / heads;
+        long groups = 0, keys = 0;
+        for (int i = 0; i < nseg; ++i) {
+            if (q_len[i] <= 1) continue;
+            for (int a = 0; a < q_len[i]; a += 32 * abreast) {
+                const int p0 = ctx_len[i] - q_len[i] + a, rows = q_len[i] - a < 32 * abreast ? q_len[i] - a : 32 * abreast;
+                const int lo0 = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
+                ++groups;
+                keys += (p0 + rows - (lo0 & ~31) + 31) / 32 + 8;
+            }
+        }
+        if (groups == 0) return PRE_WAVES;
+        const double filled = (double)groups * nkv * parts / (2.0 * ncu), whole = ceil(filled);
+        if (heads == PRE_WAVES && filled <= 1.0) return PRE_WAVES;
+        double waves = 0.0;                                              // (the last of a group's blocks may have fewer heads)
+        for (int b = 0; b < parts; ++b) waves += at_work[(G - b * heads < heads ? G - b * heads : heads) * abreast];
+        const double us = (filled + 0.4 * (whole - filled)) * ((double)keys / groups) * (waves / parts);
+        if (heads == PRE_WAVES) best = 0.97 * us;
+        else if (us < best) { best = us; pick = heads; }
+    }
+    return pick;
+}
+
 // tiles: int [ntiles, 4] = (segment, first token of the tile in the batch, rows <= 32, unused)
+// heads: see li_paged_attention_prefill_heads (4 with runs > 1 and with longer block tables)
 // runs > 1 (see li_paged_attention_prefill_runs): part_acc [tokens, nh, runs, dh] and part_ml
 // [tokens, nh, runs, 2] float32 take the runs' results, which are then joined for the n_merge tokens
 // of merge_tokens (null: the tokens 0 .. n_merge - 1).
@@ -2104,16 +2165,19 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
                                           const int* tiles, int ntiles, const int* q_start, const int* q_len,
                                           const int* ctx_len, int nh, int nkv, int dh, int page_size,
                                           int num_pages, int window, float scale, int runs, float* part_acc,
-                                          float* part_ml, const int* merge_tokens, int n_merge, hipStream_t stream) {
+                                          float* part_ml, const int* merge_tokens, int n_merge, int heads, hipStream_t stream) {
     if (ntiles <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || nkv > 65535 || page_size <= 0 || max_blocks <= 0 ||
         max_blocks > PRE_TABLE_CAP || (long long)max_blocks * page_size > (1ll << 21) || !(scale > 0.f))
         return LI_ERR_SIZE;
     if (runs < 1 || runs > MERGE_RUNS_MAX || (runs > 1 && (!part_acc || !part_ml || n_merge <= 0 || nh > 4 * 65535 || max_blocks > PRE2_TABLE_CAP)))
         return LI_ERR_SIZE;
+    if (heads != PRE_WAVES && ((heads != 1 && heads != 2) || runs > 1 || max_blocks > PRE2_TABLE_CAP)) return LI_ERR_SIZE;
     const int G = nh / nkv;
-    const int parts = (G + PRE_WAVES - 1) / PRE_WAVES;
+    const int parts = (G + heads - 1) / heads;
     if ((long)parts * runs > 65535) return LI_ERR_SIZE;
-    dim3 grid(ntiles, nkv, parts);
+    const int abreast = PRE_WAVES / heads;
+    if (ntiles > 0x7fffffff - PRE_WAVES) return LI_ERR_SIZE;
+    dim3 grid((ntiles + abreast - 1) / abreast * abreast, nkv, parts);
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
         (void)hipGetLastError();
@@ -2122,13 +2186,14 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
 #define LI_PRE(DHV) paged_attention_prefill_mfma_kernel<DHV><<<grid, PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
         tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu)
-#define LI_PRE2(DHV, P32V) paged_attention_prefill_dma_kernel<DHV, P32V><<<grid, PRE_WAVES * 64, 0, stream>>>( \
+#define LI_PRE2_AS(DHV, P32V, HEADSV) paged_attention_prefill_dma_kernel<DHV, P32V, HEADSV><<<grid, PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
-        tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu, runs, part_acc, part_ml)
+        tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu, runs, part_acc, part_ml, ntiles)
+#define LI_PRE2(DHV, P32V) { if (heads == 1) LI_PRE2_AS(DHV, P32V, 1); else if (heads == 2) LI_PRE2_AS(DHV, P32V, 2); else LI_PRE2_AS(DHV, P32V, PRE_WAVES); }
 #define LI_PRE3(DHV, P32V) paged_attention_prefill_split_kernel<DHV, P32V><<<grid, 2 * PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
         tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu)
-    if (runs == 1 && max_blocks <= PRE2_TABLE_CAP && (long)ntiles * nkv * parts <= (long)ncu) {      // at most a block a compute unit: the tile's keys in two halves
+    if (runs == 1 && heads == PRE_WAVES && max_blocks <= PRE2_TABLE_CAP && (long)ntiles * nkv * parts <= (long)ncu) {      // at most a block a compute unit: the tile's keys in two halves
         const bool p32 = 32 % page_size == 0;
         if (dh == 128) { if (p32) LI_PRE3(128, true); else LI_PRE3(128, false); }
         else if (dh == 64) { if (p32) LI_PRE3(64, true); else LI_PRE3(64, false); }
@@ -2137,8 +2202,8 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
     if (max_blocks <= PRE2_TABLE_CAP) {                       // (longer block tables: the form that keeps 8,192 entries in LDS)
         grid.z = parts * runs;
         const bool p32 = 32 % page_size == 0;
-        if (dh == 128) { if (p32) LI_PRE2(128, true); else LI_PRE2(128, false); }
-        else if (dh == 64) { if (p32) LI_PRE2(64, true); else LI_PRE2(64, false); }
+        if (dh == 128) { if (p32) LI_PRE2(128, true) else LI_PRE2(128, false) }
+        else if (dh == 64) { if (p32) LI_PRE2(64, true) else LI_PRE2(64, false) }
         else return LI_ERR_SIZE;
         if (runs > 1) {
             if (li_launch_status() != LI_OK) return LI_ERR_LAUNCH;
@@ -2147,6 +2212,7 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
     } else
     if (dh == 128) LI_PRE(128); else if (dh == 64) LI_PRE(64); else return LI_ERR_SIZE;
 #undef LI_PRE2
+#undef LI_PRE2_AS
 #undef LI_PRE3
 #undef LI_PRE
 #undef LI_PRE_FETCH

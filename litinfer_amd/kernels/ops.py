@@ -95,7 +95,7 @@ _SIGNATURES = {
     },
     "attention": {
         "li_paged_attention": [P, I, P, P, P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, F],
-        "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I],
+        "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I, I],
         "li_paged_attention_prefill_f32": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F],
         "li_paged_attention_decode": [P, I, P, P, P, I, P, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, P],
         "li_decode_run_keys": [P, I, P, P, P, P, I, I, I, I, I, I, I, P],
@@ -154,6 +154,18 @@ def _prefill_runs(host_q_len, host_ctx_len, nh: int, nkv: int, dh: int, max_bloc
         return 1
     return int(f(len(host_q_len), host_q_len.ctypes.data, host_ctx_len.ctypes.data, nh, nkv, dh, max_blocks,
                  int(window), tokens, PREFILL_RUNS_MAX_BYTES))
+
+
+PREFILL_WAVES = 4                      # waves of a block of that kernel: heads of a group, or tiles that follow each other
+
+
+def _prefill_heads(host_q_len, host_ctx_len, nh: int, nkv: int, max_blocks: int, window: int) -> int:
+    """How many heads of a group a block of the prompt portions' kernel takes (the batch's segments as int32 arrays in
+    host memory)."""
+    if (nh // nkv) % PREFILL_WAVES == 0 or host_q_len is None or host_ctx_len is None or host_q_len.dtype != "int32" or host_ctx_len.dtype != "int32":
+        return PREFILL_WAVES
+    f = _lib_fn("attention", "li_paged_attention_prefill_heads", [c_int, c_void_p, c_void_p] + [c_int] * 4, c_int)
+    return int(f(len(host_q_len), host_q_len.ctypes.data, host_ctx_len.ctypes.data, nh, nkv, max_blocks, int(window)))
 
 
 # the current stream's handle without the stream object around it (an op is called some hundred times a
@@ -1575,6 +1587,9 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
         if ws is not None:
             runs = _prefill_runs(getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None), nh, nkv, dh,
                                  meta.max_blocks, window, t)
+        heads = PREFILL_WAVES
+        if runs == 1:
+            heads = _prefill_heads(getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None), nh, nkv, meta.max_blocks, window)
         acc = ml = lst = None
         if runs > 1:
             acc = ws.buffer("attn.runs_acc", (t, nh, runs, dh), torch.float32)
@@ -1585,7 +1600,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
              meta.num_tiles, meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
              nh, nkv, dh, page_size, k.shape[0], int(window), float(scale), runs,
              0 if acc is None else acc.data_ptr(), 0 if ml is None else ml.data_ptr(),
-             0 if lst is None else lst.data_ptr(), n_multi)
+             0 if lst is None else lst.data_ptr(), n_multi, heads)
     elif (n_multi and qkv.dtype is torch.float32 and dh in (64, 128) and meta.num_tiles
             and meta.tile_rows == PREFILL_TILE_ROWS and n_multi == meta.num_multi):
         # the 32-bit path's tiled kernel for portions (other head sizes: the general kernel below)

@@ -643,9 +643,9 @@ def _paged_case(ops, dtype, seg_specs, nh, nkv, dh, page, window, seed, scale_on
     ([(1300, 1300)], 32, 8, 64, 8, 200),
     ([(5000, 300)], 4, 2, 128, 1, 0),                               # a table too long for the kernel that keeps the pages' offsets in LDS
     ([(1500, 400), (9, 9)], 7, 1, 128, 1, 0),                       # one key a page, within its table
-    ([(1100, 1100), (40, 3)], 40, 8, 128, 16, 0),                   # groups of 5 heads: blocks of five waves
-    ([(1100, 1100)], 48, 8, 64, 12, 0),                             # groups of 6: six waves, pages that do not divide a block of keys
-    ([(2100, 2100)], 18, 2, 64, 8, 700),                            # groups of 9: two blocks of five waves, one of them with four heads
+    ([(1100, 1100), (40, 3)], 40, 8, 128, 16, 0),                   # groups of 5 heads
+    ([(1100, 1100)], 48, 8, 64, 12, 0),                             # groups of 6, pages that do not divide a block of keys
+    ([(2100, 2100)], 18, 2, 64, 8, 700),                            # groups of 9
 ])
 def test_paged_attention(ops, dtype, segs, nh, nkv, dh, page, window):
     out, ref = _paged_case(ops, dtype, segs, nh, nkv, dh, page, window, seed=6)
@@ -736,6 +736,31 @@ def test_prompt_portions_behind_long_contexts_with_their_keys_in_runs(ops, segs,
     for far in (5, 1000, 2900):
         out, ref = _paged_case(ops, torch.bfloat16, [(3000, 64)], 28, 4, 128, 16, 0, seed=32, scale_one=far, row=40, ws=_Lender())
         assert rel(out, ref) < 1.5e-2
+
+
+@pytest.mark.parametrize("heads", [1, 2])
+@pytest.mark.parametrize("segs,nh,nkv,dh,page,window", [
+    ([(300, 300), (40, 3), (1, 1), (257, 129), (64, 33)], 5, 1, 128, 16, 0),      # segments that end in any of a block's tiles
+    ([(500, 300), (70, 70), (45, 2)], 6, 2, 128, 12, 0),                          # pages that do not divide a block of keys
+    ([(700, 500), (90, 90), (200, 161)], 3, 3, 64, 8, 50),                        # a window shorter than a block's tiles
+    ([(260, 129)], 14, 2, 64, 64, 100),                                           # one row in a block's second tile or first of the next
+])
+def test_prompt_attention_with_several_tiles_a_block(ops, monkeypatch, segs, nh, nkv, dh, page, window, heads):
+    monkeypatch.setattr(ops, "_prefill_heads", lambda *a: heads)
+    out, ref = _paged_case(ops, torch.bfloat16, segs, nh, nkv, dh, page, window, seed=33)
+    assert rel(out, ref) < 1.5e-2
+    # one far key among the keys that only a later tile of the block sees
+    out, ref = _paged_case(ops, torch.bfloat16, [(1000, 300)], nh, nkv, dh, page, 0, seed=34, scale_one=770, row=90)
+    assert rel(out, ref) < 1.5e-2
+
+
+def test_how_many_heads_a_block_of_prompt_attention_takes(ops):
+    from litinfer_amd.kernels.ops import _prefill_heads
+    heads = lambda new, cached, nh, nkv, window=0, pages=2000: _prefill_heads(np.array(new, dtype=np.int32), np.array(cached, dtype=np.int32) + np.array(new, dtype=np.int32), nh, nkv, pages, window)
+    assert heads([1999], [16000], 40, 8) == 1 and heads([2048], [0], 32, 32) < 4 and heads([2000], [4000], 32, 16) == 2
+    assert heads([1999], [16000], 64, 8) == 4 and heads([1999], [16000], 28, 4) == 4      # whole groups; a chip that is not filled
+    assert heads([990], [517], 40, 8) == 4 and heads([1] * 9, [700] * 9, 32, 32) == 4     # one round; no portion at all
+    assert heads([1999], [16000], 40, 8, pages=5000) == 4                                 # a table for the form without
 
 
 @pytest.mark.parametrize("segs,nh,nkv,dh", [
