@@ -1314,9 +1314,9 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     int max_blocks, const int* __restrict__ tiles, const int* __restrict__ q_start,
     const int* __restrict__ q_len, const int* __restrict__ ctx_len, int nh, int nkv, int page_size,
     int num_pages, int window, float scale, int ncu, int ksplit, float* __restrict__ part_acc,
-    float* __restrict__ part_ml, int ntiles) {
-    // ksplit > 1: the tile's blocks of keys are cut into ksplit runs, blockIdx.z = part of the heads x
-    // ksplit + run; a block then leaves its sums, unscaled, in part_acc [token, head, run, dh] and its
+    float* __restrict__ part_ml, int ntiles, int split_rows) {
+    // ksplit > 1: the blocks of keys of the tiles in the first split_rows x 4 / HEADS places of the list (all, or those that would
+    // be a last round of few blocks) are cut into ksplit runs, one a block; it then leaves its sums, unscaled, in part_acc [token, head, run, dh] and its
     // (maximum, sum) in part_ml, and attention_merge_runs_kernel joins the runs in their order
     // HEADS: the block's four waves are this many heads of a group (4, 2 or 1) x 4 / HEADS tiles of a segment that follow each
     // other, all of which read the keys that the block fetches.  Four heads and one tile where the group's heads divide by four;
@@ -1335,9 +1335,9 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     // the compute units in the order of their numbers, one each and then again from the first unit, and
     // a unit's blocks share it: the work is dealt in a snake (every other round of `ncu` blocks backwards),
     // so that the unit with the longest tile of one round gets the shortest of the next.
-    const int per_tile = gridDim.y * gridDim.z;
-    const int total = gridDim.x * per_tile;
-    const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+    const int G = nh / nkv, parts = (G + HEADS - 1) / HEADS;
+    const int total = gridDim.x;
+    const int lin = blockIdx.x;
     const int round = lin / ncu, pos = lin - round * ncu;
     const int in_round = total - round * ncu < ncu ? total - round * ncu : ncu;
     const int item = round * ncu + ((round & 1) ? in_round - 1 - pos : pos);
@@ -1345,16 +1345,18 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     // have nothing to do, see below, come behind the others; dealt among them they left compute units idle: 512 blocks took
     // 935 us, as long as two rounds)
     constexpr int abreast = PRE_WAVES / HEADS;          // tiles of a block
-    const int turn = item / per_tile, rows_of_tiles = gridDim.x / abreast;
-    const int tile = (rows_of_tiles - 1 - turn % rows_of_tiles) * abreast + turn / rows_of_tiles;
+    const int rows = (ntiles + abreast - 1) / abreast, whole = (rows - split_rows) * abreast * nkv * parts;      // blocks of tiles that are not cut
+    const bool cut = item >= whole;
+    const int cuts = cut ? ksplit : 1, first_row = cut ? 0 : split_rows, these = cut ? split_rows : rows - split_rows;
+    const int per_tile = nkv * parts * cuts, at_item = cut ? item - whole : item, turn = at_item / per_tile, of_tile = at_item % per_tile;
+    const int tile = (first_row + these - 1 - turn % these) * abreast + turn / these;
     if (tile >= ntiles) return;
     const int s = tiles[tile * 4], t00 = tiles[tile * 4 + 1], seg0 = q_start[s], seg_rows = q_len[s];
     if (abreast > 1 && ((t00 - seg0) / 32) % abreast) return;          // (one of the tiles of the block before: before any barrier)
-    const int kvh = (item % per_tile) / gridDim.z;      // (the parts of a group of heads are neighbours: they read the same keys)
-    const int G = nh / nkv;
+    const int kvh = of_tile / (parts * cuts);           // (the parts of a group of heads are neighbours: they read the same keys)
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int zz = (item % per_tile) % gridDim.z, run = zz % ksplit;
-    const int hw = (zz / ksplit) * HEADS + wave % HEADS;              // this wave's head within the group
+    const int zz = of_tile % (parts * cuts), run = zz % cuts;
+    const int hw = (zz / cuts) * HEADS + wave % HEADS;              // this wave's head within the group
     const int behind = 32 * (wave / HEADS);                           // its tile's first row behind the block's first
     const int left = seg_rows - (t00 - seg0);                         // the segment's rows from the block's first on
     const bool active = hw < G && behind < left;        // (idle waves still help to fetch and keep the barriers)
@@ -1368,7 +1370,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     const int lo_tile = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;    // ... the wave's
     int k_begin = lo0 & ~31, k_end = p00 + (left < 32 * abreast ? left : 32 * abreast);
     int first_key = lo0;
-    if (ksplit > 1) {                                   // this run's blocks of 32 keys
+    if (cuts > 1) {                                     // this run's blocks of 32 keys
         const int all = (k_end - k_begin + 31) / 32, per = (all + ksplit - 1) / ksplit;
         const int b0 = run * per, b1 = (run + 1) * per < all ? (run + 1) * per : all;
         if (b0 >= b1) {                                 // no keys for this run: it says so and is done (before any barrier)
@@ -1589,7 +1591,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     }
     if (!active || ql >= nrows) return;
     l += __shfl_xor(l, 32, LI_WAVE);               // (both halves of a query are past the return together)
-    if (ksplit > 1) {
+    if (cuts > 1) {
         const size_t at = ((size_t)(t0 + ql) * nh + head) * ksplit + run;
         if (h == 0) {
             part_ml[at * 2] = m * 0.69314718055994531f;          // (the kernel that joins the runs counts in powers of e)
@@ -2155,8 +2157,61 @@ extern "C" int li_paged_attention_prefill_heads(int nseg, const int* q_len, cons
     return pick;
 }
 
+// Where the blocks fill the chip (two a compute unit) some whole rounds and a few are left, these few take a round of their own, each as
+// long as its chain of keys: their tiles' keys are cut into so many runs that they fill the chip as well.  The tiles in question
+// are the first of the list (the last that are started); *split_tiles takes their number, *split_tokens the tokens of the blocks that
+// begin with one of them and *upto the batch's tokens up to the last of those.  Returns the runs, 1 for none.  A block of 32 keys takes about 1.1 us where two blocks
+// share a unit and 0.7 where one has it alone (1,999 tokens behind 16,000, 40 of 8 heads: 512 blocks 590 us, the other 128 365).
+extern "C" int li_paged_attention_prefill_tail(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh, int max_blocks, int window,
+                                               int heads, long max_bytes, int* split_tiles, int* split_tokens, int* upto) {
+    if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nh > 4 * 65535 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP || !split_tiles || !split_tokens ||
+        !upto || (heads != 1 && heads != 2 && heads != PRE_WAVES)) return 1;
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
+        (void)hipGetLastError();
+        ncu = 256;
+    }
+    const int abreast = PRE_WAVES / heads, parts = (nh / nkv + heads - 1) / heads;
+    const long each = (long)nkv * parts, round = 2l * ncu;
+    long groups = 0;
+    for (int i = 0; i < nseg; ++i)
+        if (q_len[i] > 1) groups += (q_len[i] + 32 * abreast - 1) / (32 * abreast);
+    const long left = groups * each % round;                            // blocks beyond the whole rounds
+    if (groups * each < round || left == 0) return 1;
+    long tile = 0, tail = 0, keys = 0;
+    int tokens = 0, at = 0, last = 0;
+    bool done = false;
+    for (int i = 0; i < nseg && !done; at += q_len[i], ++i) {
+        if (q_len[i] <= 1) continue;
+        for (int a = 0; a < q_len[i] && !done; a += 32, ++tile) {
+            if (tile % abreast == 0 && tail * each >= left) { done = true; break; }      // (whole rows of the list)
+            if ((a / 32) % abreast) continue;                           // (a block goes by its first tile)
+            const int p0 = ctx_len[i] - q_len[i] + a, more = q_len[i] - a < 32 * abreast ? q_len[i] - a : 32 * abreast;
+            const int lo0 = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
+            ++tail;
+            tokens += more;
+            last = at + a + more;
+            keys += (p0 + more - (lo0 & ~31) + 31) / 32;
+        }
+    }
+    if (tail == 0 || tail >= groups) return 1;
+    const long blocks = tail * each;
+    const double mean = (double)keys / tail;
+    int runs = (int)(round / blocks);
+    if (runs > MERGE_RUNS_MAX) runs = MERGE_RUNS_MAX;
+    while (runs > 1 && (mean / runs < 16.0 || (long)last * nh * runs * (dh + 2) * 4 > max_bytes)) --runs;
+    if (runs < 2) return 1;
+    const double alone = 0.7 * mean, cut = 1.1 * (mean / runs + 8.0) + 5.0 + (double)tokens * nh * runs * dh * 8.0 / 6.0e6;
+    if (cut > 0.85 * alone) return 1;
+    *split_tiles = (int)tile;
+    *split_tokens = tokens;
+    *upto = last;
+    return runs;
+}
+
 // tiles: int [ntiles, 4] = (segment, first token of the tile in the batch, rows <= 32, unused)
-// heads: see li_paged_attention_prefill_heads (4 with runs > 1 and with longer block tables)
+// heads: see li_paged_attention_prefill_heads (4 with longer block tables).  split_tiles: the tiles that runs > 1 is for (the first of
+// the list; whole rows of 4 / heads, or all), n_merge then their tokens: see li_paged_attention_prefill_tail
 // runs > 1 (see li_paged_attention_prefill_runs): part_acc [tokens, nh, runs, dh] and part_ml
 // [tokens, nh, runs, 2] float32 take the runs' results, which are then joined for the n_merge tokens
 // of merge_tokens (null: the tokens 0 .. n_merge - 1).
@@ -2165,19 +2220,22 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
                                           const int* tiles, int ntiles, const int* q_start, const int* q_len,
                                           const int* ctx_len, int nh, int nkv, int dh, int page_size,
                                           int num_pages, int window, float scale, int runs, float* part_acc,
-                                          float* part_ml, const int* merge_tokens, int n_merge, int heads, hipStream_t stream) {
+                                          float* part_ml, const int* merge_tokens, int n_merge, int heads, int split_tiles, hipStream_t stream) {
     if (ntiles <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || nkv > 65535 || page_size <= 0 || max_blocks <= 0 ||
         max_blocks > PRE_TABLE_CAP || (long long)max_blocks * page_size > (1ll << 21) || !(scale > 0.f))
         return LI_ERR_SIZE;
     if (runs < 1 || runs > MERGE_RUNS_MAX || (runs > 1 && (!part_acc || !part_ml || n_merge <= 0 || nh > 4 * 65535 || max_blocks > PRE2_TABLE_CAP)))
         return LI_ERR_SIZE;
-    if (heads != PRE_WAVES && ((heads != 1 && heads != 2) || runs > 1 || max_blocks > PRE2_TABLE_CAP)) return LI_ERR_SIZE;
+    if (heads != PRE_WAVES && ((heads != 1 && heads != 2) || max_blocks > PRE2_TABLE_CAP)) return LI_ERR_SIZE;
     const int G = nh / nkv;
     const int parts = (G + heads - 1) / heads;
     if ((long)parts * runs > 65535) return LI_ERR_SIZE;
-    const int abreast = PRE_WAVES / heads;
-    if (ntiles > 0x7fffffff - PRE_WAVES) return LI_ERR_SIZE;
-    dim3 grid((ntiles + abreast - 1) / abreast * abreast, nkv, parts);
+    const int abreast = PRE_WAVES / heads, rows = (int)(((long)ntiles + abreast - 1) / abreast);
+    const int split_rows = runs > 1 ? (split_tiles >= ntiles ? rows : split_tiles / abreast) : 0;
+    if (runs > 1 && (split_tiles <= 0 || (split_tiles < ntiles && split_tiles % abreast))) return LI_ERR_SIZE;
+    const long blocks = ((long)(rows - split_rows) + (long)split_rows * runs) * abreast * nkv * parts;
+    if (blocks > 0x7fffffffl) return LI_ERR_SIZE;
+    dim3 grid(ntiles, nkv, parts);
     int dev = 0, ncu = 0;
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
         (void)hipGetLastError();
@@ -2186,9 +2244,9 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
 #define LI_PRE(DHV) paged_attention_prefill_mfma_kernel<DHV><<<grid, PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
         tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu)
-#define LI_PRE2_AS(DHV, P32V, HEADSV) paged_attention_prefill_dma_kernel<DHV, P32V, HEADSV><<<grid, PRE_WAVES * 64, 0, stream>>>( \
+#define LI_PRE2_AS(DHV, P32V, HEADSV) paged_attention_prefill_dma_kernel<DHV, P32V, HEADSV><<<(unsigned)blocks, PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
-        tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu, runs, part_acc, part_ml, ntiles)
+        tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu, runs, part_acc, part_ml, ntiles, split_rows)
 #define LI_PRE2(DHV, P32V) { if (heads == 1) LI_PRE2_AS(DHV, P32V, 1); else if (heads == 2) LI_PRE2_AS(DHV, P32V, 2); else LI_PRE2_AS(DHV, P32V, PRE_WAVES); }
 #define LI_PRE3(DHV, P32V) paged_attention_prefill_split_kernel<DHV, P32V><<<grid, 2 * PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
@@ -2200,7 +2258,6 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
         else return LI_ERR_SIZE;
     } else
     if (max_blocks <= PRE2_TABLE_CAP) {                       // (longer block tables: the form that keeps 8,192 entries in LDS)
-        grid.z = parts * runs;
         const bool p32 = 32 % page_size == 0;
         if (dh == 128) { if (p32) LI_PRE2(128, true) else LI_PRE2(128, false) }
         else if (dh == 64) { if (p32) LI_PRE2(64, true) else LI_PRE2(64, false) }

@@ -95,7 +95,7 @@ _SIGNATURES = {
     },
     "attention": {
         "li_paged_attention": [P, I, P, P, P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, F],
-        "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I, I],
+        "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I, I, I],
         "li_paged_attention_prefill_f32": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F],
         "li_paged_attention_decode": [P, I, P, P, P, I, P, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, P],
         "li_decode_run_keys": [P, I, P, P, P, P, I, I, I, I, I, I, I, P],
@@ -166,6 +166,19 @@ def _prefill_heads(host_q_len, host_ctx_len, nh: int, nkv: int, max_blocks: int,
         return PREFILL_WAVES
     f = _lib_fn("attention", "li_paged_attention_prefill_heads", [c_int, c_void_p, c_void_p] + [c_int] * 4, c_int)
     return int(f(len(host_q_len), host_q_len.ctypes.data, host_ctx_len.ctypes.data, nh, nkv, max_blocks, int(window)))
+
+
+def _prefill_tail(host_q_len, host_ctx_len, nh: int, nkv: int, dh: int, max_blocks: int, window: int, heads: int):
+    """(runs, tiles, tokens, the batch's tokens up to the last of these): the tiles whose keys are cut where the blocks of a prompt
+    portion would leave a last round of few (runs 1: none)."""
+    if host_q_len is None or host_ctx_len is None or host_q_len.dtype != "int32" or host_ctx_len.dtype != "int32":
+        return 1, 0, 0, 0
+    f = _lib_fn("attention", "li_paged_attention_prefill_tail", [c_int, c_void_p, c_void_p] + [c_int] * 6 + [c_long] + [c_void_p] * 3, c_int)
+    out = (c_int * 3)()
+    at = ctypes.addressof(out)
+    runs = int(f(len(host_q_len), host_q_len.ctypes.data, host_ctx_len.ctypes.data, nh, nkv, dh, max_blocks, int(window), heads,
+                 PREFILL_RUNS_MAX_BYTES, at, at + 4, at + 8))
+    return runs, out[0], out[1], out[2]
 
 
 # the current stream's handle without the stream object around it (an op is called some hundred times a
@@ -1587,20 +1600,23 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
         if ws is not None:
             runs = _prefill_runs(getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None), nh, nkv, dh,
                                  meta.max_blocks, window, t)
-        heads = PREFILL_WAVES
+        heads, cut_tiles, cut_tokens, upto = PREFILL_WAVES, meta.num_tiles, n_multi, t
         if runs == 1:
-            heads = _prefill_heads(getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None), nh, nkv, meta.max_blocks, window)
+            lens = getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None)
+            heads = _prefill_heads(*lens, nh, nkv, meta.max_blocks, window)
+            if ws is not None:
+                runs, cut_tiles, cut_tokens, upto = _prefill_tail(*lens, nh, nkv, dh, meta.max_blocks, window, heads)
         acc = ml = lst = None
         if runs > 1:
-            acc = ws.buffer("attn.runs_acc", (t, nh, runs, dh), torch.float32)
-            ml = ws.buffer("attn.runs_ml", (t, nh, runs, 2), torch.float32)
+            acc = ws.buffer("attn.runs_acc", (upto, nh, runs, dh), torch.float32)
+            ml = ws.buffer("attn.runs_ml", (upto, nh, runs, 2), torch.float32)
             lst = meta.multi_tokens if n_multi < t else None
         _run("attention", "li_paged_attention_prefill", qkv.data_ptr(), qkv.stride(0), out.data_ptr(),
              k.data_ptr(), v.data_ptr(), bt.data_ptr(), meta.max_blocks, meta.tiles.data_ptr(),
              meta.num_tiles, meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
              nh, nkv, dh, page_size, k.shape[0], int(window), float(scale), runs,
              0 if acc is None else acc.data_ptr(), 0 if ml is None else ml.data_ptr(),
-             0 if lst is None else lst.data_ptr(), n_multi, heads)
+             0 if lst is None else lst.data_ptr(), cut_tokens, heads, cut_tiles)
     elif (n_multi and qkv.dtype is torch.float32 and dh in (64, 128) and meta.num_tiles
             and meta.tile_rows == PREFILL_TILE_ROWS and n_multi == meta.num_multi):
         # the 32-bit path's tiled kernel for portions (other head sizes: the general kernel below)

@@ -754,6 +754,29 @@ def test_prompt_attention_with_several_tiles_a_block(ops, monkeypatch, segs, nh,
     assert rel(out, ref) < 1.5e-2
 
 
+@pytest.mark.parametrize("heads,tiles,runs", [(4, 1, 2), (4, 7, 5), (2, 2, 3), (2, 10, 16), (1, 4, 4), (1, 12, 2)])
+def test_prompt_attention_with_the_keys_of_its_first_tiles_in_runs(ops, monkeypatch, heads, tiles, runs):
+    segs = [(700, 300), (1, 1), (90, 70), (400, 40), (257, 129)]                # 10 + 3 + 2 + 5 tiles, a decoding token among them
+    blocks = 128 // heads                                                        # tokens of a block; one goes by its first tile
+    of = [(s, a, min(blocks, q - a)) for s, a, q in [(s, a, q) for s, (_, q) in enumerate(segs) if q > 1 for a in range(0, q, 32)][:tiles] if a % blocks == 0]
+    starts = np.concatenate([[0], np.cumsum([q for _, q in segs])])
+    monkeypatch.setattr(ops, "_prefill_runs", lambda *a: 1)
+    monkeypatch.setattr(ops, "_prefill_heads", lambda *a: heads)
+    monkeypatch.setattr(ops, "_prefill_tail", lambda *a: (runs, tiles, sum(r for _, _, r in of), int(starts[of[-1][0]] + of[-1][1] + of[-1][2])))
+    for nh, nkv, dh, window in ((5, 1, 128, 0), (6, 2, 64, 90)):
+        out, ref = _paged_case(ops, torch.bfloat16, segs, nh, nkv, dh, 16, window, seed=35, ws=_Lender())
+        assert rel(out, ref) < 1.5e-2
+
+
+def test_which_tiles_of_prompt_attention_have_their_keys_in_runs(ops):
+    from litinfer_amd.kernels.ops import _prefill_tail
+    tail = lambda new, cached, nh, nkv, heads: _prefill_tail(np.array(new, dtype=np.int32), np.array(cached, dtype=np.int32) + np.array(new, dtype=np.int32), nh, nkv, 128, 2000, 0, heads)
+    assert tail([1999], [16000], 40, 8, 1) == (3, 16, 512, 512)                   # 640 blocks: 512 and the first four rows of tiles
+    assert tail([1, 1999], [50, 16000], 40, 8, 1) == (3, 16, 512, 513)
+    assert tail([1999], [16000], 40, 8, 4)[0] == 1 and tail([990], [16000], 40, 8, 4)[0] == 1      # a last round that is nearly full; less than one round
+    assert tail([1999], [100], 40, 8, 1)[0] == 1                                  # too few keys
+
+
 def test_how_many_heads_a_block_of_prompt_attention_takes(ops):
     from litinfer_amd.kernels.ops import _prefill_heads
     heads = lambda new, cached, nh, nkv, window=0, pages=2000: _prefill_heads(np.array(new, dtype=np.int32), np.array(cached, dtype=np.int32) + np.array(new, dtype=np.int32), nh, nkv, pages, window)
