@@ -28,12 +28,10 @@ template <> struct RouteVec<float> { static constexpr int N = 4; };
 template <> struct RouteVec<bf16_t> { static constexpr int N = 8; };
 
 // 16 bytes of a matrix row against the row in LDS
-__device__ __forceinline__ float route_dot16(const float* p, const float* xs) {
-    const float4 v = *reinterpret_cast<const float4*>(p);
-    return fmaf(v.x, xs[0], fmaf(v.y, xs[1], fmaf(v.z, xs[2], v.w * xs[3])));
+__device__ __forceinline__ float route_dot16(const uint4 r, const float* xs, const float*) {
+    return fmaf(__uint_as_float(r.x), xs[0], fmaf(__uint_as_float(r.y), xs[1], fmaf(__uint_as_float(r.z), xs[2], __uint_as_float(r.w) * xs[3])));
 }
-__device__ __forceinline__ float route_dot16(const bf16_t* p, const float* xs) {
-    const uint4 r = *reinterpret_cast<const uint4*>(p);
+__device__ __forceinline__ float route_dot16(const uint4 r, const float* xs, const bf16_t*) {
     const uint32_t u[4] = {r.x, r.y, r.z, r.w};
     float s = 0.f;
 #pragma unroll
@@ -44,12 +42,66 @@ __device__ __forceinline__ float route_dot16(const bf16_t* p, const float* xs) {
     return s;
 }
 
+// What a plan is made of (see moe_plan_kernel below); plan null: none.
+struct MoePlanOut { int* plan; int* row_token; int* pair_row; float* row_wt; int* count; int max_tiles, tile_rows, experts; };
+#define MOE_PLAN_EXPERTS 64       // experts up to which the router makes the plan: one a lane
+
+// A wave's fence: what its lanes wrote to LDS is there for its other lanes
+#define LI_WAVE_LDS()                                            \
+    {                                                            \
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   \
+        __builtin_amdgcn_wave_barrier();                         \
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");   \
+    }
+
+// The plan of a decoding step by one wave, behind the router (moe_plan_kernel in a launch of its own is 4 to 5 us, and does less
+// than a microsecond's work for so few pairs).  The choices are read from memory: other blocks wrote them.
+__device__ __forceinline__ void moe_plan_by_wave(const MoePlanOut& p, const int* __restrict__ idx, const float* __restrict__ wt, int pairs, int top, int* cursor) {
+    const int lane = threadIdx.x & 63;
+    cursor[lane] = 0;
+    LI_WAVE_LDS()
+    for (int i = lane; i < pairs; i += 64) {
+        const int e = __hip_atomic_load(idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (e >= 0 && e < p.experts) atomicAdd(&cursor[e], 1);
+    }
+    LI_WAVE_LDS()
+    const int rows = cursor[lane], tiles = (rows + p.tile_rows - 1) / p.tile_rows;       // (lanes past the last expert: none)
+    int rows_upto = rows, tiles_upto = tiles;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(rows_upto, o, LI_WAVE), b = __shfl_up(tiles_upto, o, LI_WAVE);
+        if (lane >= o) { rows_upto += a; tiles_upto += b; }
+    }
+    const int start = rows_upto - rows;
+    for (int i = 0, nt = tiles_upto - tiles; i < tiles && nt < p.max_tiles; ++i, ++nt) {
+        const int r = i * p.tile_rows;
+        int* tile = p.plan + 4 + 4 * nt;
+        tile[0] = lane; tile[1] = start + r; tile[2] = rows - r < p.tile_rows ? rows - r : p.tile_rows; tile[3] = 0;
+    }
+    if (lane == 63) { p.plan[0] = tiles_upto < p.max_tiles ? tiles_upto : p.max_tiles; p.plan[1] = rows_upto; p.plan[2] = p.plan[3] = 0; }
+    cursor[lane] = start;
+    LI_WAVE_LDS()
+    for (int i = lane; i < pairs; i += 64) {
+        const int e = __hip_atomic_load(idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (e >= 0 && e < p.experts) {
+            const int row = atomicAdd(&cursor[e], 1);
+            p.pair_row[i] = row;
+            p.row_token[row] = i / top;
+            if (p.row_wt) p.row_wt[row] = __hip_atomic_load(wt + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        } else {
+            p.pair_row[i] = -1;
+        }
+    }
+}
+
+// Few tokens: what bounds it is a chain of trips to memory (the row, a matrix row, the pick), so a wave asks for its first two
+// matrix rows, where they are short enough to wait in registers, before the token's row has come.
 template <typename TX, typename TW, int NT>
 __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x, long x_stride, const TW* __restrict__ wr,
                                                        const float* __restrict__ br, const TW* __restrict__ wg,
                                                        int* __restrict__ idx, float* __restrict__ wt, float* __restrict__ gate,
                                                        int K, int E, int top, int vec, int mode_flags,
-                                                       const float* __restrict__ corr, int groups, int keep) {
+                                                       const float* __restrict__ corr, int groups, int keep, MoePlanOut po) {
     const int mode = mode_flags & 3;
     const bool group_max = mode_flags & 4, plain_weights = mode_flags & 8;
     extern __shared__ __align__(16) float sm[];        // [K] the row, [E] the logits, [E] the scores, [groups] the groups' scores
@@ -59,15 +111,37 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
     float* gs = sc + E;
     const int t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const TX* row = x + (size_t)t * x_stride;
+    constexpr int VE = RouteVec<TW>::N;
+    constexpr int HELD = 4;                            // pieces of a matrix row that a lane holds
+    const int n_rows = E + (wg ? 1 : 0);
+    const bool held = NT == 1024 && vec && K / VE <= 64 * HELD;
+    uint4 piece[2][HELD];
+    if constexpr (NT == 1024) {
+        if (held) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int e = w + q * (NT / 64) < n_rows ? w + q * (NT / 64) : 0;       // (never conditional: a row past the last reads the first)
+                const TW* wrow = e < E ? wr + (size_t)e * K : wg;
+#pragma unroll
+                for (int i = 0; i < HELD; ++i) {
+                    const int at = lane + 64 * i < K / VE ? lane + 64 * i : 0;
+                    piece[q][i] = *reinterpret_cast<const uint4*>(wrow + (size_t)at * VE);
+                }
+            }
+        }
+    }
     for (int k = threadIdx.x; k < K; k += NT) xs[k] = load_as_float(row + k);
     __syncthreads();
-    constexpr int VE = RouteVec<TW>::N;
-    for (int e = w; e < E + (wg ? 1 : 0); e += NT / 64) {
+    for (int e = w, q = 0; e < n_rows; e += NT / 64, ++q) {
         const TW* wrow = e < E ? wr + (size_t)e * K : wg;
         float s = 0.f;
-        if (vec) {                                     // 16 bytes a lane and turn, several turns on their way
+        if (held && q < 2) {
+#pragma unroll
+            for (int i = 0; i < HELD; ++i)
+                if (lane + 64 * i < K / VE) s += route_dot16(q ? piece[1][i] : piece[0][i], xs + (lane + 64 * i) * VE, (const TW*)nullptr);
+        } else if (vec) {                              // 16 bytes a lane and turn, several turns on their way
 #pragma unroll 4
-            for (int i = lane; i < K / VE; i += 64) s += route_dot16(wrow + (size_t)i * VE, xs + i * VE);
+            for (int i = lane; i < K / VE; i += 64) s += route_dot16(*reinterpret_cast<const uint4*>(wrow + (size_t)i * VE), xs + i * VE, (const TW*)nullptr);
         } else {
             for (int k = lane; k < K; k += 64) s = fmaf(load_as_float(wrow + k), xs[k], s);
         }
@@ -154,12 +228,37 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     }
     if (mode != 0) sum += 1e-20f;
-    if (lane < top) { idx[(size_t)t * top + lane] = mine; wt[(size_t)t * top + lane] = plain_weights ? chosen : chosen / sum; }
+    const float share = plain_weights ? chosen : chosen / sum;
+    if (!po.plan) {
+        if (lane < top) { idx[(size_t)t * top + lane] = mine; wt[(size_t)t * top + lane] = share; }
+        return;
+    }
+    // The choices go through to memory; the block counts itself there, and the one that completes the count makes the plan.
+    // Nobody waits for anybody, and the count is left at zero.
+    if (lane < top) {
+        __hip_atomic_store(idx + (size_t)t * top + lane, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(wt + (size_t)t * top + lane, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if (gridDim.x > 1) {
+        int before = 0;
+        if (lane == 0) before = atomicAdd(po.count, 1);
+        if (__builtin_amdgcn_readfirstlane(before) != (int)gridDim.x - 1) return;
+        if (lane == 0) atomicExch(po.count, 0);
+    }
+    moe_plan_by_wave(po, idx, wt, gridDim.x * top, top, reinterpret_cast<int*>(sm));
 }
 
+// plan (may be null) and what follows: the plan of the step as well (li_moe_plan's, over `experts` of the E router outputs), up to 128
+// tokens and MOE_PLAN_EXPERTS experts; count: an int that is zero before the call and after it.
 extern "C" int li_moe_route(const void* x, int x_dtype, long x_stride, const void* wr, int w_dtype, const float* br, const void* wg,
                             int* idx, float* wt, float* gate, int T, int K, int E, int top, int mode, const float* corr,
-                            int groups, int keep, hipStream_t stream) {
+                            int groups, int keep, int* plan, int max_tiles, int* row_token, int* pair_row, int tile_rows, float* row_wt,
+                            int experts, int* count, hipStream_t stream) {
+    if (plan && (T > 128 || experts <= 0 || experts > MOE_PLAN_EXPERTS || experts > E || K < 64 || max_tiles <= 0 || !row_token || !pair_row || !count ||
+                 (tile_rows != MOE_TILE && tile_rows != MOE_BIG_TILE && tile_rows != MOE_HUGE_TILE)))
+        return LI_ERR_SIZE;
+    const MoePlanOut po{plan, row_token, pair_row, row_wt, count, max_tiles, tile_rows, experts};
     if (T <= 0 || K <= 0 || E <= 0 || top <= 0 || top > E || top > 64 || x_stride < K || (wg && !gate) || mode < 0 || mode > 15 || (mode & 3) == 3 ||
         groups <= 0 || keep <= 0 || keep > groups || E % groups || (size_t)(K + 2 * E + groups + 4) * 4 > 60000)
         return LI_ERR_SIZE;
@@ -171,8 +270,8 @@ extern "C" int li_moe_route(const void* x, int x_dtype, long x_stride, const voi
     // few tokens: sixteen waves share a token's experts, so that a wave has one or two rows to go through
 #define MR(TX, TW)                                                                                                                \
     {                                                                                                                             \
-        if (T <= 128) moe_route_kernel<TX, TW, 1024><<<T, 1024, lds, stream>>>((const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, K, E, top, vec, mode, corr, groups, keep); \
-        else moe_route_kernel<TX, TW, 256><<<T, 256, lds, stream>>>((const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, K, E, top, vec, mode, corr, groups, keep);           \
+        if (T <= 128) moe_route_kernel<TX, TW, 1024><<<T, 1024, lds, stream>>>((const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, K, E, top, vec, mode, corr, groups, keep, po); \
+        else moe_route_kernel<TX, TW, 256><<<T, 256, lds, stream>>>((const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, K, E, top, vec, mode, corr, groups, keep, po);       \
     }
     if (x_dtype == LI_F32 && w_dtype == LI_F32) MR(float, float)
     else if (x_dtype == LI_BF16 && w_dtype == LI_BF16) MR(bf16_t, bf16_t)

@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import math
+from dataclasses import dataclass
 from ctypes import c_float, c_int, c_long, c_void_p
 from typing import Dict, Optional, Union
 
@@ -69,7 +70,7 @@ _SIGNATURES = {
         "li_gated_group_norm": [P, L, P, L, P, F, P, I, L, I, I, I, I],
     },
     "moe": {
-        "li_moe_route": [P, I, L, P, I, P, P, P, P, P, I, I, I, I, I, P, I, I],
+        "li_moe_route": [P, I, L, P, I, P, P, P, P, P, I, I, I, I, I, P, I, I, P, I, P, P, I, P, I, P],
         "li_moe_plan": [P, I, I, I, P, I, P, P, I, P, P],
         "li_moe_linear": [P, I, L, P, P, I, P, I, P, I, L, I, I, I, F, I, I, P],
         "li_moe_combine": [P, L, P, L, P, P, P, P, L, I, I, I, P, I, P, I, L, F, F, P, P, P, I],
@@ -1966,17 +1967,49 @@ def moe_max_tiles(tokens: int, top: int, experts: int, tile_rows: int = MOE_TILE
     return min(pairs, pairs // tile_rows + experts)
 
 
+@dataclass
+class MoePlan:
+    """Room for the plan of a step (see `moe_plan`) and what it goes by."""
+    experts: int
+    plan: torch.Tensor                      # int32 [4 + 4 * max_tiles]
+    row_token: torch.Tensor                 # int32 [pairs]
+    pair_row: torch.Tensor                  # int32 [pairs]
+    tile_rows: int
+    row_wt: Optional[torch.Tensor] = None   # float32 [pairs]
+    count: Optional[torch.Tensor] = None    # int32 [1], zero: the router's blocks count themselves there and leave it zero
+
+
+MOE_ROUTE_PLAN_TOKENS, MOE_ROUTE_PLAN_EXPERTS = 128, 64
+
+
+def moe_route_takes_plan(t: int, experts: int, hidden: int) -> bool:
+    """Whether `moe_route` makes the plan too: a decoding step's few pairs, by the wave that made the last choice."""
+    return 0 < t <= MOE_ROUTE_PLAN_TOKENS and experts <= MOE_ROUTE_PLAN_EXPERTS and hidden >= 64
+
+
+def _check_plan(what: str, t: int, top: int, p: MoePlan) -> int:
+    _gpu(p.plan, p.row_token, p.pair_row, p.row_wt)
+    _chk(p.row_wt is None or (p.row_wt.dtype is torch.float32 and p.row_wt.is_contiguous() and p.row_wt.numel() >= t * top), f"{what}: row_wt")
+    max_tiles = moe_max_tiles(t, top, p.experts, p.tile_rows)
+    _chk(p.tile_rows in (MOE_TILE_ROWS, MOE_BIG_TILE_ROWS, MOE_HUGE_TILE_ROWS), f"{what}: tiles of 32, 64 or 128 rows")
+    _chk(all(v.dtype is torch.int32 and v.is_contiguous() for v in (p.plan, p.row_token, p.pair_row))
+         and p.plan.numel() >= 4 + 4 * max_tiles and p.row_token.numel() >= t * top and p.pair_row.numel() >= t * top and p.experts <= 8000,
+         f"{what}: int32 arrays of the step's sizes")
+    return max_tiles
+
+
 def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], gate_row: Optional[torch.Tensor],
               idx: torch.Tensor, wt: torch.Tensor, gate: Optional[torch.Tensor], scores: str = "softmax_chosen",
               correction: Optional[torch.Tensor] = None, groups: int = 1, keep_groups: int = 1,
-              group_score: str = "top2_sum", normalize: bool = True) -> None:
+              group_score: str = "top2_sum", normalize: bool = True, plan: Optional[MoePlan] = None) -> None:
     """idx [T, top] int32: the experts with the largest logits x router^T + bias (float32 sums; the lower index wins a
     tie); wt [T, top] float32: softmax over the chosen logits; gate [T] = sigmoid(x . gate_row) where a row is given.
     With scores = "sigmoid" an expert's score is sigmoid(logit); the choice goes by score + correction[e], and only
     among the experts of the `keep_groups` groups (of experts / groups neighbours each) whose two largest choice
     values have the largest sum (`group_score` = "max": whose largest choice value is largest); wt = the chosen scores
     over their sum (+ 1e-20), or, with `normalize` False, the chosen scores themselves.  scores = "softmax": the same
-    with an expert's score = the softmax over ALL logits."""
+    with an expert's score = the softmax over ALL logits.  With a `plan` (where `moe_route_takes_plan`) the same launch makes what
+    `moe_plan` makes of idx."""
     _gpu(x, router, bias, gate_row, idx, wt, gate, correction)
     t, k = x.shape
     e, top = router.shape[0], idx.shape[1]
@@ -1993,12 +2026,19 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
     _chk((gate_row is None) == (gate is None) and (gate_row is None or (gate_row.dtype is router.dtype and gate_row.numel() == k
          and gate_row.is_contiguous() and gate.dtype is torch.float32 and gate.numel() == t and gate.is_contiguous())), "moe_route: gate")
     _chk((k + 2 * e + groups + 4) * 4 <= 60000, "moe_route: the row and the logits must fit 60 KB of LDS")
+    made = (0, 0, 0, 0, 0, 0, 0, 0)
+    if plan is not None:
+        max_tiles = _check_plan("moe_route", t, top, plan)
+        _gpu(plan.count)
+        _chk(moe_route_takes_plan(t, plan.experts, k) and plan.experts <= e and plan.count.dtype is torch.int32 and plan.count.numel() > 0, "moe_route: plan")
+        made = (plan.plan.data_ptr(), max_tiles, plan.row_token.data_ptr(), plan.pair_row.data_ptr(), int(plan.tile_rows),
+                0 if plan.row_wt is None else plan.row_wt.data_ptr(), plan.experts, plan.count.data_ptr())
     if t:
         _run("moe", "li_moe_route", x.data_ptr(), _DT[x.dtype], x.stride(0), router.data_ptr(), _DT[router.dtype],
              0 if bias is None else bias.data_ptr(), 0 if gate_row is None else gate_row.data_ptr(), idx.data_ptr(), wt.data_ptr(),
              0 if gate is None else gate.data_ptr(), t, k, e, top,
              mode | (4 if group_score == "max" else 0) | (0 if normalize or mode == 0 else 8), 0 if correction is None else correction.data_ptr(),
-             int(groups), int(keep_groups))
+             int(groups), int(keep_groups), *made)
 
 
 def moe_plan(idx: torch.Tensor, experts: int, plan: torch.Tensor, row_token: torch.Tensor, pair_row: torch.Tensor,
@@ -2006,15 +2046,11 @@ def moe_plan(idx: torch.Tensor, experts: int, plan: torch.Tensor, row_token: tor
     """Sorts the (token, choice) pairs by expert.  plan int32 [4 + 4 * max_tiles]: the number of tiles, then (expert,
     first row, rows, 0) a tile; row_token [pairs]: the token of a sorted row; pair_row [pairs]: the row of a pair;
     row_wt [pairs] float32 (with wt [T, top]): the weight of a sorted row's pair.  Returns max_tiles."""
-    _gpu(idx, plan, row_token, pair_row, wt, row_wt)
-    _chk(row_wt is None or (wt is not None and all(v.dtype is torch.float32 and v.is_contiguous() and v.numel() >= idx.numel()
-                                                   for v in (wt, row_wt))), "moe_plan: wt, row_wt")
+    _gpu(idx, wt)
     t, top = idx.shape
-    max_tiles = moe_max_tiles(t, top, experts, tile_rows)
-    _chk(tile_rows in (MOE_TILE_ROWS, MOE_BIG_TILE_ROWS, MOE_HUGE_TILE_ROWS), "moe_plan: tiles of 32, 64 or 128 rows")
-    _chk(all(x.dtype is torch.int32 and x.is_contiguous() for x in (idx, plan, row_token, pair_row))
-         and plan.numel() >= 4 + 4 * max_tiles and row_token.numel() >= t * top and pair_row.numel() >= t * top and experts <= 8000,
-         "moe_plan: int32 arrays of the step's sizes")
+    _chk(idx.dtype is torch.int32 and idx.is_contiguous() and (row_wt is None or (wt is not None and wt.dtype is torch.float32 and wt.is_contiguous()
+                                                                                   and wt.numel() >= idx.numel())), "moe_plan: idx, wt")
+    max_tiles = _check_plan("moe_plan", t, top, MoePlan(experts, plan, row_token, pair_row, tile_rows, row_wt))
     if t:
         _run("moe", "li_moe_plan", idx.data_ptr(), t, top, experts, plan.data_ptr(), max_tiles, row_token.data_ptr(), pair_row.data_ptr(),
              int(tile_rows), 0 if wt is None else wt.data_ptr(), 0 if row_wt is None else row_wt.data_ptr())

@@ -143,9 +143,6 @@ class RoutedMLP(FeedForward):
         idx = ws.buffer("moe.idx", (t, top), torch.int32)
         wt = ws.buffer("moe.wt", (t, top), torch.float32)
         gate = ws.buffer("moe.gate", (t,), torch.float32) if self.gate_row is not None else None
-        ops.moe_route(xn, self.router, self.router_b, self.gate_row, idx, wt, gate, scores=self.scores,
-                      correction=self.correction, groups=self.groups, keep_groups=self.keep_groups,
-                      group_score=self.group_score, normalize=self.normalize)
         # (a prompt's portion gives every expert hundreds of rows: larger tiles then, for the kernel that stages them in LDS)
         n_first = self.w_up.shape[1]
         rows_a_tile = ops.moe_tile_rows(t, top, self.experts, xn.dtype, self.w_up.dtype,
@@ -155,7 +152,14 @@ class RoutedMLP(FeedForward):
         row_token = ws.buffer("moe.row_token", (pairs,), torch.int32)
         pair_row = ws.buffer("moe.pair_row", (pairs,), torch.int32)
         row_wt = ws.buffer("moe.row_wt", (pairs,), torch.float32) if self.weigh_input else None
-        ops.moe_plan(idx, self.experts, plan, row_token, pair_row, rows_a_tile, wt=wt if self.weigh_input else None, row_wt=row_wt)
+        count = ws.buffer("moe.count", (1,), torch.int32, zero=True)         # (asked for by every step: a recorded one finds it)
+        with_plan = ops.moe_route_takes_plan(t, self.experts, self.hidden)
+        ops.moe_route(xn, self.router, self.router_b, self.gate_row, idx, wt, gate, scores=self.scores,
+                      correction=self.correction, groups=self.groups, keep_groups=self.keep_groups,
+                      group_score=self.group_score, normalize=self.normalize,
+                      plan=ops.MoePlan(self.experts, plan, row_token, pair_row, rows_a_tile, row_wt, count) if with_plan else None)
+        if not with_plan:
+            ops.moe_plan(idx, self.experts, plan, row_token, pair_row, rows_a_tile, wt=wt if self.weigh_input else None, row_wt=row_wt)
         h = ws.buffer("moe.h", (pairs, self.inter), self.rt.dtype)
         ops.moe_linear(xn, row_token, self.w_up, plan, max_tiles, h, pairs, act=ACTIVATIONS[self.activation],
                        tile_rows=rows_a_tile, limit=self.limit, row_wt=row_wt)

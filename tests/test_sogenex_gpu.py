@@ -471,6 +471,45 @@ def test_equal_router_logits_take_the_lower_expert():
     assert np.allclose(wt.cpu().numpy(), e / e.sum(), atol=1e-6)
 
 
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,K,n_router,experts,top,tile_rows", [
+    (1, 64, 2, 2, 1, 32), (1, 1536, 16, 16, 2, 32), (2, 72, 5, 3, 2, 32), (33, 1536, 20, 16, 6, 32), (128, 2049, 64, 64, 8, 64), (100, 300, 70, 1, 2, 32),
+    (128, 520, 17, 16, 3, 32)])
+def test_the_routers_launch_makes_the_plan_too(dt, T, K, n_router, experts, top, tile_rows):
+    """The plan beside the choices (by the block that counts itself last) holds what moe_plan makes of the choices of a launch
+    without it; twice, with the count left at zero in between."""
+    from litinfer_amd.kernels import ops
+    assert ops.moe_route_takes_plan(T, experts, K) and not ops.moe_route_takes_plan(129, experts, K) and not ops.moe_route_takes_plan(T, 65, K)
+    dtype, pairs = getattr(torch, dt), T * top
+    count = torch.zeros(1, dtype=torch.int32, device=DEV)
+    for seed in (1, 2):
+        g = torch.Generator().manual_seed(seed)
+        x, router = torch.randn(T, K, generator=g).to(dtype).to(DEV), torch.randn(n_router, K, generator=g).to(dtype).to(DEV)
+        gate_row = torch.randn(K, generator=g).to(dtype).to(DEV)
+        new = lambda *shape, d=torch.int32: torch.full(shape, -7, dtype=d, device=DEV)
+        idx, wt, gate = new(T, top), new(T, top, d=torch.float32), new(T, d=torch.float32)
+        ops.moe_route(x, router, None, gate_row, idx, wt, gate, scores="sigmoid")
+        tiles = ops.moe_max_tiles(T, top, experts, tile_rows)
+        plan, row_token, pair_row, row_wt = new(4 + 4 * tiles), new(pairs), new(pairs), new(pairs, d=torch.float32)
+        ops.moe_plan(idx, experts, plan, row_token, pair_row, tile_rows, wt=wt, row_wt=row_wt)
+        i2, w2, g2 = new(T, top), new(T, top, d=torch.float32), new(T, d=torch.float32)
+        p2 = ops.MoePlan(experts, new(4 + 4 * tiles), new(pairs), new(pairs), tile_rows, new(pairs, d=torch.float32), count)
+        ops.moe_route(x, router, None, gate_row, i2, w2, g2, scores="sigmoid", plan=p2)
+        assert torch.equal(idx, i2) and torch.equal(wt, w2) and torch.equal(gate, g2) and count.item() == 0
+        n, rows = plan[0].item(), plan[1].item()
+        assert torch.equal(plan[:4 + 4 * n], p2.plan[:4 + 4 * n]) and torch.equal(pair_row < 0, p2.pair_row < 0)
+        # which of an expert's rows a pair gets is open: every pair's row lies in its expert's tiles, holds its token and weight
+        expert_of = torch.zeros(max(rows, 1), dtype=torch.int32)
+        for e, r0, nr, _ in p2.plan[4:4 + 4 * n].view(-1, 4).tolist():
+            expert_of[r0:r0 + nr] = e
+        at, flat = p2.pair_row.cpu().long(), i2.cpu().view(-1)
+        have = at >= 0
+        assert torch.equal(at[have].sort().values, torch.arange(rows)) and torch.equal(have, flat < experts)
+        assert torch.equal(expert_of[at[have]], flat[have])
+        assert torch.equal(p2.row_token.cpu()[at[have]], (torch.arange(pairs) // top).int()[have])
+        assert torch.equal(p2.row_wt.cpu()[at[have]], w2.cpu().view(-1)[have])
+
+
 def test_difference_of_two_maps_and_its_norm():
     from litinfer_amd.kernels import ops
     rng = np.random.default_rng(2)
