@@ -827,6 +827,10 @@ __device__ __forceinline__ void unpack8(const uint4 raw, float* f) {
     f[6] = __uint_as_float(raw.w << 16); f[7] = __uint_as_float(raw.w & 0xffff0000u);
 }
 
+// Two maps over the same values (differential attention) in one launch: blocks from n tokens on are the second map's, whose queries
+// lie q_off floats further on and whose keys in kc; every block leaves parts, also without splits.  n 0: one map.
+struct MaSecond { const bf16_t* kc; long q_off; int n; };
+
 template <int NPK, int NPV, int RH, int U>
 __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     const float* __restrict__ q, int q_token_stride, int q_head_stride, bf16_t* __restrict__ out,
@@ -834,11 +838,14 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     const int* __restrict__ block_table, int max_blocks, const int* __restrict__ token_list,
     const int* __restrict__ seg_of_token, const int* __restrict__ q_start, const int* __restrict__ q_len,
     const int* __restrict__ ctx_len, int nh, int nkv, int dk, int dv, int page_size, int num_pages, int window,
-    int keep_first, float softcap, float scale, MaExtras ex, int tab_cap, int pshift, int nsplit, float* __restrict__ parts) {
+    int keep_first, float softcap, float scale, MaExtras ex, int tab_cap, int pshift, int nsplit, float* __restrict__ parts, MaSecond second) {
     extern __shared__ float join[];                 // [4 waves][RH][dv + 2], then tab_cap table entries
     int* tab = (int*)(join + (size_t)4 * RH * (dv + 2));
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, g = lane >> 3, j = lane & 7;
-    const int t = token_list ? token_list[blockIdx.x] : blockIdx.x, kvh = blockIdx.y;
+    const bool other = second.n > 0 && (int)blockIdx.x >= second.n;
+    const int ti = (int)blockIdx.x - (other ? second.n : 0);
+    const int t = token_list ? token_list[ti] : ti, kvh = blockIdx.y;
+    if (other) { q += second.q_off; kc = second.kc; }
     const int rep = nh / nkv, hfirst = (blockIdx.z / nsplit) * RH, sp = blockIdx.z % nsplit;
     const int nheads = rep - hfirst < RH ? rep - hfirst : RH;
     const int s = seg_of_token[t];
@@ -1033,7 +1040,7 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
             ll += r[dv + 1] * f;
         }
         const int head = kvh * rep + hfirst + hh;
-        if (nsplit == 1) {
+        if (nsplit == 1 && second.n == 0) {
             out[((size_t)t * nh + head) * dv + d].bits = float_to_bf16(a * finish_factor(ll, mm, ex, t, head) * column_gate(ex, t, head, dv, d));
         } else {                                    // this split's sums, maximum and sum of weights: joined by the kernel behind
             float* part = parts + (((size_t)blockIdx.x * nh + head) * nsplit + sp) * (dv + 2);
@@ -1080,6 +1087,63 @@ __global__ void masked_attention_join_kernel(const float* __restrict__ parts, bf
     }
 }
 
+// The same for two maps: both joined, their difference a1 - lambda a2 and its norm over the head's columns, times `mult` (what
+// diff_combine_kernel does, here without the maps' rounding between).  A block of two waves a (token, head), a wave the factors of one
+// map's splits.  Bound by the launches: a step's five kernels of 4 to 8 us, each waiting for the one before it, are two (an answer of
+// a model with such layers 12.35 -> 11.83 ms).
+#define JOIN_DIFF_COLUMNS 2         // columns a thread holds: dv up to 256, the most that the kernel before it has
+__global__ __launch_bounds__(128) void masked_attention_join_diff_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out, int n, int nh, int dv, int nsplit,
+                                                                         float lambda, float eps, float mult) {
+    __shared__ float fac[2][JOIN_MAX_SPLITS], sums[2][JOIN_MAX_SPLITS], squares[2];
+    const int t = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const size_t map = (size_t)n * nh * nsplit * (dv + 2);
+    const float* base = parts + ((size_t)t * nh + head) * nsplit * (dv + 2);
+    {
+        const float* mine = base + w * map + (size_t)(lane < nsplit ? lane : nsplit - 1) * (dv + 2) + dv;
+        const float m = mine[0], l = mine[1];
+        const float mm = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - mm);
+        fac[w][lane] = f;
+        sums[w][lane] = l * f;
+    }
+    __syncthreads();
+    float inv[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+        float ll = 0.f;
+#pragma unroll 8
+        for (int x = 0; x < nsplit; ++x) ll += sums[q][x];
+        inv[q] = ll != 0.f ? 1.0f / ll : 0.f;
+    }
+    float o[JOIN_DIFF_COLUMNS], ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < JOIN_DIFF_COLUMNS; ++c) {
+        const int d = threadIdx.x + 128 * c;
+        o[c] = 0.f;
+        if (d >= dv) continue;
+        float a[2] = {0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            for (int x0 = 0; x0 < nsplit; x0 += 8) {
+                float r[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) r[i] = base[q * map + (size_t)(x0 + i < nsplit ? x0 + i : nsplit - 1) * (dv + 2) + d];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) a[q] = x0 + i < nsplit ? fmaf(r[i], fac[q][x0 + i], a[q]) : a[q];
+            }
+        o[c] = fmaf(-lambda, a[1] * inv[1], a[0] * inv[0]);
+        ss = fmaf(o[c], o[c], ss);
+    }
+    ss = wave_sum(ss);
+    if (lane == 0) squares[w] = ss;
+    __syncthreads();
+    const float f = mult / sqrtf((squares[0] + squares[1]) / (float)dv + eps);
+#pragma unroll
+    for (int c = 0; c < JOIN_DIFF_COLUMNS; ++c) {
+        const int d = threadIdx.x + 128 * c;
+        if (d < dv) out[((size_t)t * nh + head) * dv + d].bits = float_to_bf16(o[c] * f);
+    }
+}
+
 // 1 if the kernel for single tokens takes these sizes (bfloat16 cache and output)
 extern "C" int li_masked_attention_single_takes(int dk, int dv) {
     const int npk = (dk + 63) / 64, npv = (dv + 63) / 64;
@@ -1094,12 +1158,12 @@ extern "C" int li_masked_attention_single_blocks(int n_tokens, int nh, int nkv, 
     return n_tokens * nkv * ((rep + rh - 1) / rh);
 }
 
-extern "C" int li_masked_attention_single(const float* q, int q_token_stride, int q_head_stride, void* out, const void* kc,
+static int single_launch(const float* q, int q_token_stride, int q_head_stride, void* out, const void* kc,
                                           const void* vc, int k_row, int v_row, const int* block_table, int max_blocks,
                                           const int* token_list, int n_tokens, const int* seg_of_token, const int* q_start,
                                           const int* q_len, const int* ctx_len, int nh, int nkv, int dk, int dv, int page_size,
                                           int num_pages, int window, int keep_first, float softcap, float scale, const float* sink, const float* gate, long gate_stride, int gate_per_column, const float* slopes, int chunk,
-                                          int nsplit, float* parts, long parts_floats, hipStream_t stream) {
+                                          int nsplit, float* parts, long parts_floats, const MaSecond& second, float lambda, float eps, float mult, hipStream_t stream) {
     if (chunk < 0 || (chunk > 0 && keep_first > 0)) return LI_ERR_SIZE;
     const MaExtras ex{sink, gate, gate_stride, gate_per_column, slopes, chunk};
     if (n_tokens <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || nkv > 65535 || dk > k_row || dv > v_row || page_size <= 0 ||
@@ -1108,8 +1172,10 @@ extern "C" int li_masked_attention_single(const float* q, int q_token_stride, in
         return LI_ERR_SIZE;
     const int rep = nh / nkv, npk = (dk + 63) / 64, npv = (dv + 63) / 64;
     const int rh = (npk + npv > 6) ? (rep >= 2 ? 2 : 1) : (rep >= 4 && (rep % 4 == 0 || rep % 4 == 3 || rep > 8)) ? 4 : rep >= 2 ? 2 : 1;
-    if (nsplit < 1 || nsplit > 64 || (nsplit > 1 && (!parts || parts_floats < (long)n_tokens * nh * nsplit * (dv + 2)))) return LI_ERR_SIZE;
-    const dim3 grid(n_tokens, nkv, ((rep + rh - 1) / rh) * nsplit);
+    const int maps = second.n ? 2 : 1;
+    if (nsplit < 1 || nsplit > 64 || ((nsplit > 1 || maps > 1) && (!parts || parts_floats < (long)maps * n_tokens * nh * nsplit * (dv + 2)))) return LI_ERR_SIZE;
+    if (n_tokens > 0x3fffffff) return LI_ERR_SIZE;
+    const dim3 grid(maps * n_tokens, nkv, ((rep + rh - 1) / rh) * nsplit);
     // room for the pages of one query's visible keys: the window's and the kept ones, or the whole table's width
     const long reach = window > 0 && (chunk <= 0 || window < chunk) ? window : chunk;      // (0: no bound)
     long cap = reach > 0 ? reach / page_size + 3 + (keep_first + page_size - 1) / page_size : (long)max_blocks;
@@ -1122,9 +1188,11 @@ extern "C" int li_masked_attention_single(const float* q, int q_token_stride, in
     masked_attention_single_kernel<K, V, R, UU><<<grid, 256, lds, stream>>>(                                                \
         q, q_token_stride, q_head_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, k_row, v_row, block_table,    \
         max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, nh, nkv, dk, dv, page_size, num_pages, window,       \
-        keep_first, softcap, scale, ex, tab_cap, pshift, nsplit, parts)
+        keep_first, softcap, scale, ex, tab_cap, pshift, nsplit, parts, second)
 #define MS_JOIN                                                                                                             \
-    if (nsplit > 1)                                                                                                         \
+    if (maps > 1)                                                                                                           \
+        masked_attention_join_diff_kernel<<<dim3(n_tokens, nh), 128, 0, stream>>>(parts, (bf16_t*)out, n_tokens, nh, dv, nsplit, lambda, eps, mult); \
+    else if (nsplit > 1)                                                                                                         \
         masked_attention_join_kernel<<<dim3(n_tokens, nh), dv >= 256 ? 256 : 128, 0, stream>>>(parts, (bf16_t*)out, token_list, nh, dv, nsplit, ex);
 #define MS_SMALL(K, V)                                                                                                      \
     if (npk == K && npv == V) {                                                                                             \
@@ -1145,6 +1213,30 @@ extern "C" int li_masked_attention_single(const float* q, int q_token_stride, in
 #undef MS_SMALL
 #undef MS_LARGE
     return LI_ERR_SIZE;
+}
+
+extern "C" int li_masked_attention_single(const float* q, int q_token_stride, int q_head_stride, void* out, const void* kc,
+                                          const void* vc, int k_row, int v_row, const int* block_table, int max_blocks,
+                                          const int* token_list, int n_tokens, const int* seg_of_token, const int* q_start,
+                                          const int* q_len, const int* ctx_len, int nh, int nkv, int dk, int dv, int page_size,
+                                          int num_pages, int window, int keep_first, float softcap, float scale, const float* sink, const float* gate, long gate_stride, int gate_per_column, const float* slopes, int chunk,
+                                          int nsplit, float* parts, long parts_floats, hipStream_t stream) {
+    return single_launch(q, q_token_stride, q_head_stride, out, kc, vc, k_row, v_row, block_table, max_blocks, token_list, n_tokens, seg_of_token,
+                         q_start, q_len, ctx_len, nh, nkv, dk, dv, page_size, num_pages, window, keep_first, softcap, scale, sink, gate, gate_stride, gate_per_column, slopes, chunk, nsplit, parts, parts_floats, MaSecond{nullptr, 0, 0}, 0.f, 0.f, 0.f, stream);
+}
+
+// Differential attention of single tokens: out = mult * o / sqrt(mean(o^2) + eps) over a head's columns, o = (the map of q and kc) - lambda *
+// (the map of the queries q_off floats further on and k2), both over the values vc.  parts: 2 n_tokens nh nsplit (dv + 2) floats.
+extern "C" int li_masked_attention_single_pair(const float* q, int q_token_stride, int q_head_stride, long q_off, void* out, const void* kc, const void* k2,
+                                               const void* vc, int k_row, int v_row, const int* block_table, int max_blocks,
+                                               int n_tokens, const int* seg_of_token, const int* q_start,
+                                               const int* q_len, const int* ctx_len, int nh, int nkv, int dk, int dv, int page_size,
+                                               int num_pages, int window, int keep_first, float softcap, float scale, int nsplit, float* parts,
+                                               long parts_floats, float lambda, float eps, float mult, hipStream_t stream) {
+    if (!k2 || (uintptr_t)k2 % 16 || q_off % 4 || n_tokens <= 0 || dv > 128 * JOIN_DIFF_COLUMNS) return LI_ERR_SIZE;
+    return single_launch(q, q_token_stride, q_head_stride, out, kc, vc, k_row, v_row, block_table, max_blocks, nullptr, n_tokens, seg_of_token,
+                         q_start, q_len, ctx_len, nh, nkv, dk, dv, page_size, num_pages, window, keep_first, softcap, scale, nullptr, nullptr, 0, 0,
+                         nullptr, 0, nsplit, parts, parts_floats, MaSecond{(const bf16_t*)k2, q_off, n_tokens}, lambda, eps, mult, stream);
 }
 
 // ------------------------------------------------------------------------------------------- per-head products

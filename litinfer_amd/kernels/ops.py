@@ -77,6 +77,7 @@ _SIGNATURES = {
     },
     "attention_masked": {
         "li_masked_attention": [P, I, I, P, I, P, P, I, I, I, P, I, P, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, P, L, I, P, I, I],
+        "li_masked_attention_single_pair": [P, I, I, L, P, P, P, P, I, I, P, I, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F, I, P, L, F, F, F],
         "li_masked_attention_single": [P, I, I, P, P, P, I, I, P, I, P, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, P, L, I, P, I, I, P, L],
         "li_masked_attention_heads": [P, I, I, P, P, P, I, I, P, I, P, I, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, P, L, I, P, I, I, P, L],
         "li_masked_attention_tiles": [P, I, I, P, P, P, I, I, P, I, P, I, P, P, P, I, I, I, I, I, I, I, I, F, F, P, P, L, I, P, I, I, P, L, P, I, I],
@@ -928,6 +929,39 @@ MASKED_HEADS_MIN = 4          # query heads a kv head from which rows of up to 3
 MASKED_HEADS_MIN_PAIRS = 48   # for at least so many (token, head) pairs a kv head
 MASKED_HEADS_MIN_LONG = 24    # ... and from which longer rows do, for at least MASKED_HEADS_MIN_WORK (token, head) pairs a kv head
 MASKED_HEADS_MIN_WORK = 1024
+
+
+def masked_attention_difference(q: torch.Tensor, q_token_stride: int, q_head_stride: int, q_offset: int, out: torch.Tensor, k1: torch.Tensor,
+                                k2: torch.Tensor, v: torch.Tensor, meta, nh: int, nkv: int, dk: int, dv: int, page_size: int, window: int,
+                                keep_first: int, softcap: float, scale: float, lam: float, eps: float, mult: float, ws) -> bool:
+    """A decoding step of differential attention in two launches: `masked_attention` of q over k1 and of the queries q_offset floats
+    further on over k2, both with the values v, and `diff_combine` of the two.  False, with nothing done, where the kernel for single
+    tokens does not have the sizes or the step holds more than single tokens."""
+    t = out.shape[0]
+    if (not t or meta.num_single != t or meta.num_multi or ws is None or not masked_single_takes(dk, dv)
+            or not k1.dtype is k2.dtype is v.dtype is out.dtype is torch.bfloat16 or k1.shape[3] % 8 or v.shape[3] % 8
+            or q_token_stride % 4 or q_head_stride % 4 or q_offset % 4 or q.data_ptr() % 16
+            or (masked_tiles_take(dk, dv) and _heads_kernel_pays(t, nh // nkv, dk, dv))):
+        return False
+    _gpu(q, out, k1, k2, v, meta.block_table)
+    _chk(q.dtype is torch.float32 and q.is_contiguous() and q_offset >= 0
+         and q.numel() >= (t - 1) * q_token_stride + q_offset + (nh - 1) * q_head_stride + dk, "masked_attention_difference: q")
+    _chk(out.shape == (t, nh * dv) and out.is_contiguous(), "masked_attention_difference: out")
+    _chk(k1.dim() == 4 and v.dim() == 4 and k1.shape[:3] == (k1.shape[0], nkv, page_size) and k2.shape == k1.shape and v.shape[:3] == k1.shape[:3]
+         and k1.shape[3] >= dk and v.shape[3] >= dv and k1.is_contiguous() and k2.is_contiguous() and v.is_contiguous()
+         and (k1.data_ptr() | k2.data_ptr() | v.data_ptr()) % 16 == 0, "masked_attention_difference: cache")
+    _chk(nh % nkv == 0 and meta.num_tokens == t and meta.block_table.shape == (meta.num_segments, meta.max_blocks), "masked_attention_difference: batch")
+    bound = window + keep_first if window else meta.max_blocks * page_size
+    # (the splits of `masked_attention`, of twice as many blocks)
+    blocks = 2 * _single_blocks(t, nh, nkv, dk, dv)
+    nsplit = max(1, min(_compute_units(q.device) * (1 if -(-dk // 64) + -(-dv // 64) > 6 else 2) // blocks, bound // 128, 32))
+    parts = ws.buffer("masked_attention.parts", (2 * t * nh * nsplit * (dv + 2),), torch.float32)
+    _run("attention_masked", "li_masked_attention_single_pair", q.data_ptr(), int(q_token_stride), int(q_head_stride), int(q_offset), out.data_ptr(),
+         k1.data_ptr(), k2.data_ptr(), v.data_ptr(), k1.shape[3], v.shape[3], meta.block_table.data_ptr(), meta.max_blocks, t,
+         meta.seg_of_token.data_ptr(), meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(), nh, nkv, dk, dv, page_size,
+         k1.shape[0], int(window), int(keep_first), float(softcap or 0.0), float(scale), nsplit, parts.data_ptr(), parts.numel(), float(lam), float(eps),
+         float(mult))
+    return True
 
 
 def _heads_kernel_pays(n: int, rep: int, dk: int, dv: int) -> bool:

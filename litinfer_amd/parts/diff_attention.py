@@ -97,13 +97,17 @@ class DiffAttention(Mixer):
                                   (2 * nq + 2 * nk, self.nkv, self.dv, v)], ctx.slot_map(cache.group), cache.page_size)
         meta = ctx.attention_meta(cache.group)
         flat = qkv.view(-1)
+        o = ctx.ws.buffer("attn.out", (t, self.nh * self.dv), self.rt.dtype)
+        if ops.masked_attention_difference(flat, width, self.dk, nq, o, k1, k2, v, meta, self.nh, self.nkv, self.dk, self.dv, cache.page_size,
+                                           self.window, self.keep_first, self.softcap, self.scale, self.lam, self.eps, 1.0 - self.diff, ctx.ws):
+            residual.add_linear(self.out, o)                # (a decoding step, at the sizes its kernel has)
+            return
         maps = []
         for m, keys in enumerate((k1, k2)):
             a = ctx.ws.buffer(f"diff_attn.map{m}", (t, self.nh * self.dv), self.rt.dtype)
             ops.masked_attention(flat[m * nq:], width, self.dk, a, keys, v, meta, self.nh, self.nkv, self.dk, self.dv,
                                  cache.page_size, self.window, self.keep_first, self.softcap, self.scale, ws=ctx.ws)
             maps.append(a)
-        o = ctx.ws.buffer("attn.out", (t, self.nh * self.dv), self.rt.dtype)
         ops.diff_combine(maps[0], maps[1], self.lam, self.eps, 1.0 - self.diff, o, self.dv)
         residual.add_linear(self.out, o)
 

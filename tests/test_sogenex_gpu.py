@@ -13,6 +13,7 @@ import torch
 
 import helpers
 import plain_sogenex as plain
+import plain_tovasun
 import schedules
 import sogenex_cases as cases
 
@@ -521,6 +522,61 @@ def test_difference_of_two_maps_and_its_norm():
         ops.diff_combine(torch.tensor(a1, dtype=torch.float32, device=DEV), torch.tensor(a2, dtype=torch.float32, device=DEV),
                          0.37, 1e-5, 0.8, out, dv)
         assert np.abs(out.cpu().numpy() - ref).max() < 1e-5
+
+
+@pytest.mark.parametrize("ctxs,nh,nkv,dk,dv,page,window,keep,cap", [
+    ([700, 90, 3, 41, 1], 12, 2, 128, 128, 16, 200, 4, 30.0),       # two splits, some of them empty
+    ([40], 3, 3, 64, 64, 8, 0, 0, 0.0),                             # no splits: parts all the same
+    ([3000, 5, 129], 4, 2, 64, 128, 16, 0, 0, 0.0),
+    ([1500, 100], 5, 1, 320, 256, 16, 1024, 0, 0.0),                # long rows: two columns a thread
+    ([260, 17] * 40, 6, 2, 64, 128, 32, 100, 40, 0.0),              # many tokens
+])
+def test_difference_of_two_maps_in_a_decoding_step(ctxs, nh, nkv, dk, dv, page, window, keep, cap):
+    from litinfer_amd.engine.workspace import Workspace
+    from litinfer_amd.kernels import ops
+    from litinfer_amd.engine.batch import AttentionMeta
+    g = torch.Generator().manual_seed(dk + nh)
+    n, scale = len(ctxs), dk ** -0.5
+    pages = [-(-c // page) for c in ctxs]
+    ids, width = torch.randperm(sum(pages) + 3, generator=g), max(pages)
+    tab, caches, at = torch.zeros(n, width, dtype=torch.int32), [], 0
+    for d in (dk, dk, dv):
+        caches.append(torch.randn(len(ids), nkv, page, d, generator=g).to(torch.bfloat16))
+    for i, p in enumerate(pages):
+        tab[i, :p] = ids[at:at + p].int()
+        at += p
+    q = torch.randn(n, 2 * nh * dk + 8, generator=g)
+    one, ctx = np.ones(n, dtype=np.int32), np.asarray(ctxs, dtype=np.int32)
+    first = np.arange(n, dtype=np.int32)
+    dev = lambda a: torch.from_numpy(a).to(DEV)
+    meta = AttentionMeta(block_table=tab.to(DEV), max_blocks=width, seg_of_token=dev(first), q_start=dev(first), q_len=dev(one), ctx_len=dev(ctx),
+                         num_segments=n, num_tokens=n, max_q_len=1, max_ctx_len=int(ctx.max()), host_q_start=first, host_q_len=one,
+                         host_ctx_len=ctx, num_single=n, num_multi=0)
+    ws, (k1, k2, v), qd = Workspace(DEV), [c.to(DEV) for c in caches], q.to(DEV)
+    out = torch.empty(n, nh * dv, dtype=torch.bfloat16, device=DEV)
+    args = (nh, nkv, dk, dv, page, window, keep, cap, scale)
+    assert ops.masked_attention_difference(qd.view(-1), q.shape[1], dk, nh * dk, out, k1, k2, v, meta, *args, 0.37, 1e-5, 0.8, ws)
+    # against 64 bits, the maps not rounded between: the result's own rounding to bfloat16 (half of 2^-8) and the maps' sums in float32
+    ref = np.zeros((n, nh, dv))
+    for i, c in enumerate(ctxs):
+        rows = [np.repeat(cc[tab[i, :pages[i]].long()].double().transpose(1, 2).reshape(-1, nkv, cc.shape[3])[:c].numpy(), nh // nkv, axis=1)
+                for cc in caches]
+        a = [plain_tovasun.masked_softmax_attention(q[i:i + 1, m * nh * dk:(m + 1) * nh * dk].double().numpy().reshape(1, nh, dk), rows[m], rows[2], scale,
+                                            window, keep, cap or None, q_pos=np.arange(c - 1, c), k_pos=np.arange(c)) for m in (0, 1)]
+        ref[i] = plain.rms((np.asarray(a[0]) - 0.37 * np.asarray(a[1])).reshape(nh, dv), 1e-5) * 0.8
+    got = out.float().cpu().numpy().reshape(n, nh, dv)
+    assert np.all(np.abs(got - ref) <= 2 ** -8 * np.abs(ref) + 1e-4 * np.abs(ref).max())
+    # ... and the three launches it replaces, which round the maps
+    maps = []
+    for m, keys in enumerate((k1, k2)):
+        maps.append(torch.empty_like(out))
+        ops.masked_attention(qd.view(-1)[m * nh * dk:], q.shape[1], dk, maps[m], keys, v, meta, *args, ws=ws)
+    three = torch.empty_like(out)
+    ops.diff_combine(maps[0], maps[1], 0.37, 1e-5, 0.8, three, dv)
+    assert np.abs(three.float().cpu().numpy().reshape(n, nh, dv) - ref).max() < 2e-2 * np.abs(ref).max()
+    # not a decoding step, or no kernel for its sizes: nothing is done
+    meta.num_single, meta.num_multi = n - 1, 1
+    assert not ops.masked_attention_difference(qd.view(-1), q.shape[1], dk, nh * dk, out, k1, k2, v, meta, *args, 0.37, 1e-5, 0.8, ws)
 
 
 def test_position_vector_and_capped_logits():
