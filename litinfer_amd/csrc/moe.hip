@@ -1117,3 +1117,123 @@ extern "C" int li_moe_combine(float* x, long x_stride, const float* yrows, long 
 #undef MC
     return li_launch_status();
 }
+
+// The same for few tokens, with the RMS norms on its two sides: with w1, the sum's own norm b / sqrt(mean(b^2) + eps1) * w1 joins x; with xn,
+// the row that x's next reader takes is left there: the norm of the new x with w2 and eps2 or, without w2, the new x itself.  One block a
+// token, its row in registers.  Bound by trips to memory one behind the other and by launches: the choices are read a lane each and
+// everything that hangs on none of them is asked for with them, so there are two trips (a trip a choice, the norms' weights behind their
+// sums: 7.0 us, now 4.9).  One token of 1,536: sum and norm 3.8 + 3.3 us and the gap between them, now 4.9 in all (an answer of
+// a model with such layers 11.83 -> 11.74 ms); 8 tokens with w1, the branch cleared, the sum and the norms 4.6 + 4.7 + 4.7 us, now 6.2 (an
+// answer 14.33 -> 14.15).  From 256 tokens on the sum alone is spread over more blocks than one a row and the norms read their rows with
+// 16 bytes a lane; the launches are then the smaller part.
+#define MOE_NORM_NT 1024
+#define MOE_NORM_COLUMNS 4          // of a thread: rows of up to 4,096
+#define MOE_NORM_CHOICES 8          // rows asked for at a time
+#define MOE_NORM_MAX_TOKENS 255
+
+extern "C" int li_moe_combine_norm_takes(int T, int H) { return T > 0 && T <= MOE_NORM_MAX_TOKENS && H > 0 && H <= MOE_NORM_NT * MOE_NORM_COLUMNS; }
+
+template <typename TI, typename TO>
+__global__ __launch_bounds__(MOE_NORM_NT) void moe_combine_norm_kernel(
+    float* x, const float* __restrict__ yrows, long y_stride, const int* __restrict__ pair_row, const float* __restrict__ wt,
+    const float* __restrict__ gate, const float* __restrict__ shared_out, long s_stride, int H, int top, const int* __restrict__ idx, int experts,
+    const TI* ident, long i_stride, float factor, const float* __restrict__ w1, float eps1, const float* __restrict__ w2, float eps2, TO* xn) {
+    __shared__ float red[MOE_NORM_NT / LI_WAVE];
+    const int t = blockIdx.x;
+    float* xr = x + (size_t)t * H;                     // (x, ident and xn may be one tensor's rows: a thread has read its columns before it writes them)
+    float v[MOE_NORM_COLUMNS] = {}, was[MOE_NORM_COLUMNS], sh[MOE_NORM_COLUMNS] = {}, g1[MOE_NORM_COLUMNS] = {}, g2[MOE_NORM_COLUMNS] = {}, own[MOE_NORM_COLUMNS] = {};
+    const float g = shared_out && gate ? gate[t] : 1.f;
+    // (a thread's columns beyond the row read its last one again, and add nothing; whole turns beyond it are left out)
+#define MOE_COLUMN(i) const int j = threadIdx.x + i * MOE_NORM_NT, jj = j < H ? j : H - 1; if (i * MOE_NORM_NT >= H) continue
+    const int lane = threadIdx.x & (LI_WAVE - 1);
+    int my_row = -1;
+    float my_f = 0.f;
+    for (int c0 = 0; c0 < top; c0 += MOE_NORM_CHOICES) {
+        if (c0 % LI_WAVE == 0) {                       // the next 64 choices, a lane each: one trip to memory, not one a choice
+            const int c = c0 + lane < top ? c0 + lane : top - 1;
+            const size_t p = (size_t)t * top + c;
+            my_row = pair_row[p];
+            const int choice = (ident ? idx : pair_row)[p];
+            my_f = (wt ? wt : yrows)[wt ? p : 0];
+            if (c0 == 0) {                             // what hangs on no choice is asked for before the first rows are waited for
+#pragma unroll
+                for (int i = 0; i < MOE_NORM_COLUMNS; ++i) {
+                    MOE_COLUMN(i);
+                    was[i] = xr[jj];
+                    if (shared_out) sh[i] = shared_out[(size_t)t * s_stride + jj];
+                    if (ident) own[i] = load_as_float(ident + (size_t)t * i_stride + jj);
+                    if (w1) g1[i] = w1[jj];
+                    if (w2) g2[i] = w2[jj];
+                }
+            }
+            if (!wt) my_f = 1.f;
+            if (my_row < 0) my_row = ident && choice >= experts ? -2 : -1;       // -2: an identity expert, the token's input row
+            if (c0 + lane >= top) my_row = -1;
+        }
+        int row[MOE_NORM_CHOICES];
+        float f[MOE_NORM_CHOICES], y[MOE_NORM_COLUMNS][MOE_NORM_CHOICES];
+#pragma unroll
+        for (int c = 0; c < MOE_NORM_CHOICES; ++c) {
+            row[c] = __builtin_amdgcn_readlane(my_row, (c0 + c) % LI_WAVE);
+            f[c] = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(my_f), (c0 + c) % LI_WAVE));
+        }
+#pragma unroll
+        for (int i = 0; i < MOE_NORM_COLUMNS; ++i) {
+            MOE_COLUMN(i);
+#pragma unroll
+            for (int c = 0; c < MOE_NORM_CHOICES; ++c) y[i][c] = yrows[(size_t)(row[c] < 0 ? 0 : row[c]) * y_stride + jj];
+        }
+#pragma unroll
+        for (int i = 0; i < MOE_NORM_COLUMNS; ++i) {
+            if (i * MOE_NORM_NT >= H) continue;
+#pragma unroll
+            for (int c = 0; c < MOE_NORM_CHOICES; ++c)
+                if (row[c] != -1) v[i] = fmaf(f[c], row[c] == -2 ? own[i] : y[i][c], v[i]);
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < MOE_NORM_COLUMNS; ++i) {
+        MOE_COLUMN(i);
+        if (shared_out) v[i] = fmaf(g, sh[i], v[i]);
+        if (j < H) ss += v[i] * v[i];
+    }
+    float inv = 1.f;
+    if (w1) inv = 1.0f / sqrtf(block_sum<MOE_NORM_NT>(ss, red) / (float)H + eps1);
+    float s2 = 0.f;
+#pragma unroll
+    for (int i = 0; i < MOE_NORM_COLUMNS; ++i) {
+        MOE_COLUMN(i);
+        v[i] = w1 ? was[i] + v[i] * inv * g1[i] : fmaf(factor, v[i], was[i]);
+        if (j >= H) continue;
+        xr[j] = v[i];
+        s2 += v[i] * v[i];
+    }
+    if (!xn) return;
+    float inv2 = 1.f;
+    if (w2) inv2 = 1.0f / sqrtf(block_sum<MOE_NORM_NT>(s2, red) / (float)H + eps2);
+#pragma unroll
+    for (int i = 0; i < MOE_NORM_COLUMNS; ++i) {
+        MOE_COLUMN(i);
+        if (j < H) store_from_float(xn + (size_t)t * H + j, w2 ? v[i] * inv2 * g2[i] : v[i]);
+    }
+#undef MOE_COLUMN
+}
+
+extern "C" int li_moe_combine_norm(float* x, const float* yrows, long y_stride, const int* pair_row, const float* wt, const float* gate,
+                                   const float* shared_out, long s_stride, int T, int H, int top, const int* idx, int experts, const void* ident,
+                                   int ident_dtype, long i_stride, float factor, const float* w1, float eps1, const float* w2, float eps2,
+                                   void* xn, int xn_dtype, hipStream_t stream) {
+    if (!li_moe_combine_norm_takes(T, H) || top <= 0 || y_stride < H || (shared_out && s_stride < H) ||
+        (ident && (!idx || i_stride < H || experts < 0)) || (w2 && !xn) || (w1 && factor != 1.0f))
+        return LI_ERR_SIZE;
+#define MC(TI, TO)                                                                                                                    \
+    moe_combine_norm_kernel<TI, TO><<<T, MOE_NORM_NT, 0, stream>>>(x, yrows, y_stride, pair_row, wt, gate, shared_out, s_stride, H, top, \
+                                                                   idx, experts, (const TI*)ident, i_stride, factor, w1, eps1, w2, eps2, (TO*)xn)
+    const bool ib = ident && ident_dtype == LI_BF16, ob = xn && xn_dtype == LI_BF16;
+    if ((ident && !ib && ident_dtype != LI_F32) || (xn && !ob && xn_dtype != LI_F32)) return LI_ERR_DTYPE;
+    if (ib) { if (ob) MC(bf16_t, bf16_t); else MC(bf16_t, float); }
+    else { if (ob) MC(float, bf16_t); else MC(float, float); }
+#undef MC
+    return li_launch_status();
+}

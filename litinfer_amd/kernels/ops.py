@@ -73,6 +73,7 @@ _SIGNATURES = {
         "li_moe_route": [P, I, L, P, I, P, P, P, P, P, I, I, I, I, I, P, I, I, P, I, P, P, I, P, I, P],
         "li_moe_plan": [P, I, I, I, P, I, P, P, I, P, P],
         "li_moe_linear": [P, I, L, P, P, I, P, I, P, I, L, I, I, I, F, I, I, P],
+        "li_moe_combine_norm": [P, P, L, P, P, P, P, L, I, I, I, P, I, P, I, L, F, P, F, P, F, P, I],
         "li_moe_combine": [P, L, P, L, P, P, P, P, L, I, I, I, P, I, P, I, L, F, F, P, P, P, I],
     },
     "attention_masked": {
@@ -2148,3 +2149,48 @@ def moe_combine(x: torch.Tensor, yrows: torch.Tensor, pair_row: torch.Tensor, wt
              _DT[identity_rows.dtype] if identity_rows is not None else 0, 0 if identity_rows is None else identity_rows.stride(0),
              float(factor), float(alpha), 0 if gamma is None else gamma.data_ptr(), 0 if beta is None else beta.data_ptr(),
              0 if xn is None else xn.data_ptr(), 0 if xn is None else _DT[xn.dtype])
+
+
+def moe_combine_takes_norms(x: torch.Tensor) -> bool:
+    """Whether `moe_combine_norm` has the sizes of x [T, H] (few tokens) and x lies where its kernel runs."""
+    f = _fn_cache.get(("moe", "li_moe_combine_norm_takes"))
+    if f is None:
+        if not x.is_cuda:
+            return False
+        f = build.load("moe").li_moe_combine_norm_takes
+        f.argtypes, f.restype = [c_int, c_int], c_int
+        _fn_cache[("moe", "li_moe_combine_norm_takes")] = f
+    return x.is_cuda and x.is_contiguous() and bool(f(x.shape[0], x.shape[1]))
+
+
+def moe_combine_norm(x: torch.Tensor, yrows: torch.Tensor, pair_row: torch.Tensor, wt: Optional[torch.Tensor], gate: Optional[torch.Tensor],
+                     shared_out: Optional[torch.Tensor], idx: Optional[torch.Tensor] = None, experts: int = 0,
+                     identity_rows: Optional[torch.Tensor] = None, top: int = 0, factor: float = 1.0, before=None, after=None,
+                     rows: Optional[torch.Tensor] = None) -> None:
+    """`moe_combine` with the RMS norms on its two sides, where `moe_combine_takes_norms`: with `before` = (weight, eps) that norm of the
+    sum joins x (factor 1); `rows` [T, H] receives what x's next reader takes: the norm `after` = (weight, eps) of the new x, or the new x
+    itself in rows' type."""
+    _gpu(x, yrows, pair_row, wt, gate, shared_out, idx, identity_rows, rows)
+    t, h = x.shape
+    top = wt.shape[1] if wt is not None else int(top)
+    _chk(x.dtype is torch.float32 and x.is_contiguous() and yrows.dtype is torch.float32 and _rows_ok(yrows) and yrows.shape == (t * top, h)
+         and pair_row.dtype is torch.int32 and pair_row.numel() >= t * top and top > 0
+         and (wt is None or (wt.dtype is torch.float32 and wt.is_contiguous() and wt.shape[0] == t)), "moe_combine_norm: x [T, H], yrows [T * top, H], pair_row, wt")
+    _chk(shared_out is None or (shared_out.dtype is torch.float32 and _rows_ok(shared_out) and shared_out.shape == (t, h)
+                                and (gate is None or (gate.dtype is torch.float32 and gate.numel() == t))), "moe_combine_norm: shared")
+    _chk(identity_rows is None or (idx is not None and idx.dtype is torch.int32 and idx.is_contiguous() and idx.shape == (t, top)
+                                   and identity_rows.dtype in _DT and _rows_ok(identity_rows) and identity_rows.shape == (t, h)
+                                   and experts >= 0), "moe_combine_norm: identity experts")
+    _chk(rows is None or (rows.dtype in _DT and rows.shape == (t, h) and rows.is_contiguous()), "moe_combine_norm: rows")
+    for norm in (before, after):
+        if norm is not None:
+            _gpu(norm[0])
+            _chk(norm[0].dtype is torch.float32 and norm[0].numel() == h and norm[0].is_contiguous(), "moe_combine_norm: a norm's weight")
+    _run("moe", "li_moe_combine_norm", x.data_ptr(), yrows.data_ptr(), yrows.stride(0), pair_row.data_ptr(), 0 if wt is None else wt.data_ptr(),
+         0 if gate is None else gate.data_ptr(), 0 if shared_out is None else shared_out.data_ptr(),
+         0 if shared_out is None else shared_out.stride(0), t, h, top,
+         0 if identity_rows is None else idx.data_ptr(), int(experts), 0 if identity_rows is None else identity_rows.data_ptr(),
+         _DT[identity_rows.dtype] if identity_rows is not None else 0, 0 if identity_rows is None else identity_rows.stride(0), float(factor),
+         0 if before is None else before[0].data_ptr(), 0.0 if before is None else float(before[1]),
+         0 if after is None else after[0].data_ptr(), 0.0 if after is None else float(after[1]),
+         0 if rows is None else rows.data_ptr(), 0 if rows is None else _DT[rows.dtype])

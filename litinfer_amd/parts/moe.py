@@ -175,9 +175,11 @@ class RoutedMLP(FeedForward):
             shared = ws.buffer("moe.shared", (t, self.hidden), torch.float32)
             self.shared_down(hs, shared, ws=ws)
         # (a pair whose choice is an identity expert has no row in the plan: the sum takes the token's input for it)
-        residual.add_by(lambda x, factor, tanh_norm: ops.moe_combine(
-            x, yrows, pair_row, None if self.weigh_input else wt, gate, shared, idx=idx if self.identity else None,
-            experts=self.experts, identity_rows=xn if self.identity else None, top=top, factor=factor, tanh_norm=tanh_norm))
+        rows = (yrows, pair_row, None if self.weigh_input else wt, gate, shared)
+        how = dict(idx=idx if self.identity else None, experts=self.experts, identity_rows=xn if self.identity else None, top=top)
+        residual.add_by(lambda x, factor, tanh_norm: ops.moe_combine(x, *rows, factor=factor, tanh_norm=tanh_norm, **how),
+                        lambda x, factor, before, after, out: ops.moe_combine_norm(x, *rows, factor=factor, before=before, after=after, rows=out, **how),
+                        ops.moe_combine_takes_norms)
 
 
 class RoutedReluSquaredMLP(RoutedMLP):

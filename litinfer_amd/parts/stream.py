@@ -79,11 +79,19 @@ class ResidualStream:
                 return
         linear(h, self.x, accumulate=True, ws=self.ws, factor=self.factor)
 
-    def add_by(self, add) -> None:
+    def add_by(self, add, add_normed=None, takes_norms=None) -> None:
         """For a sublayer whose own kernel adds into the stream: `add(x, factor, tanh_norm)` adds factor * (its output) to
         the float32 sum x and, where `tanh_norm` = (alpha, weight, bias, rows) is given, leaves that norm of the new sum in
-        rows (the norm through which the stream is read next, if it is an elementwise one)."""
+        rows (the norm through which the stream is read next, if it is an elementwise one).  A sublayer whose kernel can take the RMS
+        norms on its two sides as well, where `takes_norms(x)`, gives `add_normed(x, factor, before, after, rows)`: the norm `before` =
+        (weight, eps) of its output joins the sum, if there is one, and `rows` receives the norm `after` of the new sum, or the sum itself."""
         norm, self._scaled, self._normed = self.next_norm, None, None
+        scaling = norm.as_scaling() if norm is not None else None
+        if scaling is not None and add_normed is not None and takes_norms(self.x):
+            rows = self.ws.buffer("stream.normed_rows", self.x.shape, self.ws_dtype)
+            add_normed(self.x, self.factor, None, (scaling.weight, scaling.eps), rows)
+            self._normed = (norm, rows)
+            return
         tanh = norm.as_tanh() if norm is not None else None
         if tanh is None:
             return add(self.x, self.factor, None)
@@ -128,11 +136,20 @@ class ResidualStream:
             raise NotImplementedError("add_normed: the norm behind a sublayer must be an RMS norm with weights")
         if self.factor != 1.0:
             raise NotImplementedError("add_normed: a factor on the sublayers' outputs goes with the pre-norm arrangements")
-        y2, factors = None, (1.0, 1.0)
+        y2, factors, add_to = None, (1.0, 1.0), None
         if isinstance(y, BranchStream):
-            y, y2, factors = y.outputs()
+            add_to = y.take_waiting(self.x)
+            if add_to is None:
+                y, y2, factors = y.outputs()
         self._scaled = self._normed = None
         nxt = next_norm.as_scaling() if next_norm is not None else None
+        if add_to is not None:                       # the sublayer's own kernel joins, norms included
+            rows = None
+            if nxt is not None or (next_plain and self.ws_dtype is not self.x.dtype):
+                rows = self.ws.buffer("stream.normed_rows", self.x.shape, self.ws_dtype)
+                self._normed = (next_norm if nxt is not None else _PLAIN, rows)
+            add_to(self.x, 1.0, (scaling.weight, scaling.eps), None if nxt is None else (nxt.weight, nxt.eps), rows)
+            return
         if nxt is None and not (next_plain and self.ws_dtype is not self.x.dtype):
             ops.rmsnorm_add(y, scaling.weight, scaling.eps, self.x, y2=y2, factors=factors)
             return
@@ -153,12 +170,14 @@ class BranchStream(ResidualStream):
     def __init__(self, y: torch.Tensor, ws):
         super().__init__(y, ws)
         self._fresh = True
+        self._waiting = None                 # an output that its sublayer's kernel can still add, normed, to the residual sum: add_by's arguments
         self.second = None                   # a second output beside this one (a BranchStream with a factor of its own)
 
     def fork(self, name: str) -> "BranchStream":
         """A second output beside this one, for a sublayer made of two that are added with factors."""
         if self.second is not None:
             raise NotImplementedError("a branch holds at most two outputs")
+        self._settle()
         self.second = BranchStream(self.ws.buffer(name, self.x.shape, torch.float32), self.ws)
         return self.second
 
@@ -171,17 +190,39 @@ class BranchStream(ResidualStream):
         return self.result(), self.second.result(), (self.factor, self.second.factor)
 
     def tensor(self) -> torch.Tensor:
+        self._settle()
         if self._fresh:
             self.x.zero_()
             self._fresh = False
         return self.x
 
+    def total(self) -> torch.Tensor:
+        return self.tensor()
+
     def add_linear(self, linear, h: torch.Tensor) -> None:
+        self._settle()
         linear(h, self.x, accumulate=not self._fresh, ws=self.ws)
         self._fresh = False
 
-    def add_by(self, add) -> None:
+    def add_by(self, add, add_normed=None, takes_norms=None) -> None:
+        self._settle()
+        if add_normed is not None and self._fresh and self.second is None and takes_norms(self.x):
+            self._waiting = (add, add_normed)
+            return
         add(self.tensor(), 1.0, None)        # (a branch's factor is applied when it joins)
+
+    def _settle(self) -> None:
+        """An output that waits is written here after all."""
+        if self._waiting is not None:
+            add, self._waiting = self._waiting[0], None
+            add(self.tensor(), 1.0, None)
+
+    def take_waiting(self, x: torch.Tensor):
+        """The `add_normed` of the only output of this branch, if it waits for the sum x that it joins; whoever takes it runs it."""
+        if self._waiting is None or self.second is not None or self.factor != 1.0 or x.shape != self.x.shape or not x.is_contiguous():
+            return None
+        take, self._waiting = self._waiting[1], None
+        return take
 
     def result(self) -> torch.Tensor:
         return self.tensor()

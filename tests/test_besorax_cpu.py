@@ -269,3 +269,36 @@ def test_a_stream_with_a_factor():
             return object()
     with pytest.raises(NotImplementedError):
         s.add_normed(N(), x)
+
+
+def test_an_output_that_waits_for_the_norm_behind_its_branch():
+    from types import SimpleNamespace
+    from litinfer_amd.parts.stream import BranchStream
+    add = lambda x, factor, tanh_norm: x.add_(3.0, alpha=factor)
+    joined = lambda x, factor, before, after, rows: x.add_(100.0)
+    yes, no = (lambda x: True), (lambda x: False)
+    new = lambda: BranchStream(torch.full((2, 3), 9.0), SimpleNamespace(buffer=lambda name, shape, dt: torch.zeros(shape, dtype=dt)))
+    b = new()
+    b.add_by(add, joined, yes)
+    x = torch.ones(2, 3)
+    b.take_waiting(x)(x, 1.0, None, None, None)              # taken: the branch itself stays untouched
+    assert torch.all(x == 101) and b.take_waiting(x) is None
+    for use in (lambda b: b.result(), lambda b: b.total(), lambda b: b.tensor(), lambda b: b.outputs()[0]):
+        b = new()
+        b.add_by(add, joined, yes)
+        assert torch.all(use(b) == 3) and b.take_waiting(x) is None and torch.all(b.result() == 3)      # written after all, once
+    b = new()
+    b.add_by(add, joined, yes)
+    b.add_by(add, joined, yes)                               # a second addition: both written
+    assert b.take_waiting(x) is None and torch.all(b.result() == 6)
+    b = new()
+    b.add_by(add, joined, yes)
+    b.fork("other")
+    assert b.take_waiting(x) is None and torch.all(b.outputs()[0] == 3)
+    b = new()
+    b.add_by(add, joined, no)
+    assert b.take_waiting(x) is None and torch.all(b.result() == 3)
+    b = new()
+    b.factor = 0.5                                           # (applied when the branch joins)
+    b.add_by(add, joined, yes)
+    assert b.take_waiting(x) is None and torch.all(b.result() == 3)

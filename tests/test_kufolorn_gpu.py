@@ -676,3 +676,55 @@ def test_float32_products_whose_rows_are_shorter_than_a_step_of_the_kernel(M, N,
     ops.linear(_f32(x), _f32(w), _f32(b), out, False)
     want = x @ w.T + b
     assert np.abs(out.cpu().numpy() - want).max() < 1e-5 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,H,top,identity,shared,gated,weights", [
+    (1, 1536, 8, False, True, False, True), (8, 1536, 12, True, False, False, True), (255, 70, 1, False, False, False, False),
+    (3, 4096, 9, True, True, True, True), (17, 1025, 16, False, True, True, True), (2, 1024, 3, True, False, False, False), (2, 96, 70, True, True, True, True)])
+def test_the_sum_of_experts_with_the_norms_on_its_two_sides(T, H, top, identity, shared, gated, weights, dt):
+    from litinfer_amd.kernels import ops
+    rng = np.random.default_rng(H + top)
+    experts, out_dt = 7, torch.float32 if dt == "float32" else torch.bfloat16
+    idx = rng.integers(0, experts + 3, size=(T, top)).astype(np.int32)
+    pair_row = rng.permutation(T * top).astype(np.int32)
+    pair_row[(idx >= experts).reshape(-1)] = -1
+    x, y, wt, gate, sh = (rng.normal(size=n).astype(np.float32) for n in ((T, H), (T * top, H), (T, top), (T,), (T, H)))
+    w1, w2 = (1 + 0.1 * rng.normal(size=(2, H))).astype(np.float32)
+    ident = torch.tensor(rng.normal(size=(T, H)), dtype=torch.float32).to(out_dt)
+    dev = lambda a: torch.from_numpy(a).to(DEV)
+    s = np.zeros((T, H))
+    for t in range(T):
+        for c in range(top):
+            f, r = float(wt[t, c]) if weights else 1.0, pair_row[t * top + c]
+            s[t] += f * y[r].astype(np.float64) if r >= 0 else f * ident[t].double().numpy() if identity else 0.0
+        if shared:
+            s[t] += (float(gate[t]) if gated else 1.0) * sh[t].astype(np.float64)
+    rms = lambda v, w, eps: v / np.sqrt((v ** 2).mean(axis=1, keepdims=True) + eps) * w.astype(np.float64)
+    assert ops.moe_combine_takes_norms(dev(x)) and not ops.moe_combine_takes_norms(torch.zeros(256, 8, device=DEV))
+    assert not ops.moe_combine_takes_norms(torch.zeros(2, 4097, device=DEV)) and not ops.moe_combine_takes_norms(torch.zeros(2, 8))
+    args = (dev(y), dev(pair_row), dev(wt) if weights else None, dev(gate) if gated else None, dev(sh) if shared else None)
+    how = dict(idx=dev(idx) if identity else None, experts=experts, identity_rows=ident.to(DEV) if identity else None, top=top)
+    # sums of top + 1 terms and of H squares in float32, then the result's own rounding
+    tol = 4e-6 * np.sqrt(top + 8)
+    for before, after, leaves, factor in ((None, w2, True, 0.3), (w1, w2, True, 1.0), (w1, None, True, 1.0), (w1, None, False, 1.0)):
+        new = x + (rms(s, w1, 1e-5) if before is not None else factor * s)
+        xd, rows = dev(x), torch.full((T, H), 7.0, dtype=out_dt, device=DEV)
+        # (the reader's rows may be left where the identity experts' rows lie)
+        at = how["identity_rows"].clone() if identity else rows
+        ops.moe_combine_norm(xd, *args, **{**how, "identity_rows": at if identity else None}, factor=factor,
+                             before=None if before is None else (dev(w1), 1e-5), after=None if after is None else (dev(w2), 1e-6),
+                             rows=at if leaves else None)
+        assert np.abs(xd.cpu().numpy() - new).max() <= tol * np.abs(new).max()
+        if leaves:
+            want = rms(new, w2, 1e-6) if after is not None else new
+            err = np.abs(at.float().cpu().numpy() - want)
+            assert np.all(err <= (2 ** -8 * np.abs(want) if out_dt is torch.bfloat16 else 0) + 2 * tol * np.abs(want).max())
+        # the launches that it replaces
+        x3, b, rows3 = dev(x), torch.zeros(T, H, device=DEV), torch.empty_like(rows)
+        if before is None:
+            ops.moe_combine(x3, *args, **how, factor=factor)
+        else:
+            ops.moe_combine(b, *args, **how)
+            ops.rmsnorm_add(b, dev(w1), 1e-5, x3)
+        assert np.abs((x3 - xd).cpu().numpy()).max() <= tol * np.abs(new).max()
