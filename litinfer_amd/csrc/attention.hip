@@ -1902,9 +1902,13 @@ __global__ __launch_bounds__(2 * PRE_WAVES * 64) void paged_attention_prefill_sp
 // ------------------------------------------------ portions of prompts, float32
 // The true 32-bit path's kernel for prompts, on the float32 matrix cores (v_mfma_f32_32x32x2_f32: float32
 // operands, products and sums; no
-// operand is rounded to a shorter format).  A block takes a tile of up to 32 tokens and one kv head; its four
-// waves are query heads of that kv head (blockIdx.z picks which four), so a block of 32 keys is fetched once,
-// into LDS, for all of them.  As in the bfloat16 kernel a wave works on the TRANSPOSED scores S^T = K Q^T: in
+// operand is rounded to a shorter format).  A block takes a tile of up to 32 tokens and one kv head; its waves
+// are HEADS query heads of that kv head (blockIdx.z picks which), so a block of 32 keys is fetched once,
+// into LDS, for all of them, in NG groups that take every NG-th block of keys and join their sums at the end.
+// Bound by the float32 matrix cores of the compute units that have a block: one head's 32 keys are 8,192 cycles of
+// a SIMD's, and a portion of a prompt is few tiles, the last as long as all its keys.  So few tiles go to more units,
+// fewer heads and more groups of keys a block (810 tokens, 12 of 2 heads: 111 us with four heads a block, 83 with
+// two groups beside that, 53 with one head and four groups).  As in the bfloat16 kernel a wave works on the TRANSPOSED scores S^T = K Q^T: in
 // the result a lane holds 16 keys of ITS query (register r: key 8 (r / 4) + 4 (l / 32) + r % 4), so the softmax
 // is arithmetic inside a lane plus one exchange with lane l ^ 32, and those registers are the column operand
 // of O^T = V^T P^T as they are: MFMA step s takes register s, i.e. the keys 8 (s / 4) + s % 4 (lane half 0)
@@ -1912,8 +1916,9 @@ __global__ __launch_bounds__(2 * PRE_WAVES * 64) void paged_attention_prefill_sp
 // scores the two k-slots of an MFMA are the head's two halves: lane half h multiplies the dimensions
 // (DH / 2) h + s, which it keeps of its query in registers and reads of the keys in 16-byte pieces.
 typedef float f32x16m_t __attribute__((ext_vector_type(16)));
-template <int DH>
-__global__ __launch_bounds__(256) void paged_attention_prefill_f32_mfma_kernel(
+typedef float f32x4m_t __attribute__((ext_vector_type(4)));
+template <int DH, int HEADS, int NG>
+__global__ __launch_bounds__(64 * HEADS * NG) void paged_attention_prefill_f32_mfma_kernel(
     const float* __restrict__ q, int q_row_stride, float* __restrict__ out,
     const float* __restrict__ kc, const float* __restrict__ vc, const int* __restrict__ block_table,
     int max_blocks, const int* __restrict__ tiles, const int* __restrict__ q_start,
@@ -1921,16 +1926,19 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_f32_mfma_kernel(
     int num_pages, int window, float scale) {
     constexpr int RS = DH + 4;                      // row stride in LDS
     constexpr int C4 = DH / 4;                      // float4 pieces of a row
-    constexpr int PER = PF_T * C4 / 256;            // pieces of K (and of V) a thread fetches per block of keys
+    constexpr int NT = 64 * HEADS, PER = PF_T * C4 / NT;            // pieces of K (and of V) a thread fetches per block of keys
     constexpr int HD = DH / 2, DT = DH / 32;
-    static_assert(PER * 256 == PF_T * C4, "head sizes 64 and 128");
-    __shared__ __attribute__((aligned(16))) float Ks[PF_T * RS];
-    __shared__ __attribute__((aligned(16))) float Vs[PF_T * RS];
+    static_assert(PER * NT == PF_T * C4, "head sizes 64 and 128");
+    extern __shared__ __attribute__((aligned(16))) float f32_lds[];          // a group's keys and values, group after group; at the end the last groups' sums
+    static_assert((NG - 1) * HEADS * (DT * 16 + 2) * 64 <= NG * 2 * PF_T * RS, "the sums fit where the keys were");
+    const int grp = threadIdx.x / NT;
+    float* Ks = f32_lds + grp * 2 * PF_T * RS;
+    float* Vs = Ks + PF_T * RS;
     const int tile = gridDim.x - 1 - blockIdx.x, kvh = blockIdx.y;           // (the longest tiles of a segment first)
     const int s = tiles[tile * 4], t0 = tiles[tile * 4 + 1], nrows = tiles[tile * 4 + 2];
     const int G = nh / nkv;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int hw = blockIdx.z * 4 + wave;
+    const int tid = threadIdx.x % NT, lane = tid & 63, wave = tid >> 6;
+    const int hw = blockIdx.z * HEADS + wave;
     const bool active = hw < G;                     // (idle waves still help to fetch and keep the barriers)
     const int head = kvh * G + (active ? hw : 0);
     const int ql = lane & 31, h = lane >> 5;
@@ -1949,25 +1957,25 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_f32_mfma_kernel(
             qf[4 * c] = v.x; qf[4 * c + 1] = v.y; qf[4 * c + 2] = v.z; qf[4 * c + 3] = v.w;
         }
     }
-    float4 kreg[PER], vreg[PER];
+    f32x4m_t kreg[PER], vreg[PER];                  // (float4, a struct, went through scratch memory here: every fetch was waited for at once)
     auto fetch = [&](int kb) {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int ci = tid + 256 * i, key = kb + ci / C4, c = ci % C4;
+            const int ci = tid + NT * i, key = kb + ci / C4, c = ci % C4;
             const int kk = key < k_end ? key : k_end - 1;                    // (masked below; the address stays inside the request)
-            int page = table[kk / page_size];
+            int page = table[kk / page_size];       // (a shift where it would do, behind a branch, made the whole form 10 to 30 % slower)
             page = page < 0 ? 0 : (page >= num_pages ? num_pages - 1 : page);
             const size_t off = (((size_t)page * nkv + kvh) * page_size + kk % page_size) * DH + 4 * c;
-            kreg[i] = *reinterpret_cast<const float4*>(kc + off);
-            vreg[i] = *reinterpret_cast<const float4*>(vc + off);
+            kreg[i] = *reinterpret_cast<const f32x4m_t*>(kc + off);
+            vreg[i] = *reinterpret_cast<const f32x4m_t*>(vc + off);
         }
     };
     auto stash = [&]() {
 #pragma unroll
         for (int i = 0; i < PER; ++i) {
-            const int ci = tid + 256 * i, key = ci / C4, c = ci % C4;
-            *reinterpret_cast<float4*>(&Ks[key * RS + 4 * c]) = kreg[i];
-            *reinterpret_cast<float4*>(&Vs[key * RS + 4 * c]) = vreg[i];
+            const int ci = tid + NT * i, key = ci / C4, c = ci % C4;
+            *reinterpret_cast<f32x4m_t*>(&Ks[key * RS + 4 * c]) = kreg[i];
+            *reinterpret_cast<f32x4m_t*>(&Vs[key * RS + 4 * c]) = vreg[i];
         }
     };
     const int pq = p0 + (ql < nrows ? ql : nrows - 1);       // last visible key of this lane's query
@@ -1978,13 +1986,14 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_f32_mfma_kernel(
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
     float m = -INFINITY, l = 0.f;
-    fetch(k_begin);
-    for (int kb = k_begin; kb < k_end; kb += PF_T) {
+    fetch(k_begin + PF_T * grp);                    // (a group's blocks: every NG-th; every group makes as many turns, the barriers are all threads')
+    for (int k0 = k_begin; k0 < k_end; k0 += PF_T * NG) {
+        const int kb = k0 + PF_T * grp;
         __syncthreads();                            // the block before is done with K and V
         stash();
         __syncthreads();
-        if (kb + PF_T < k_end) fetch(kb + PF_T);    // on its way while this block is worked on
-        if (!active) continue;
+        if (k0 + PF_T * NG < k_end) fetch(kb + PF_T * NG);   // on its way while this block is worked on
+        if (!active || kb >= k_end) continue;
         // ---- S^T = K Q^T
         f32x16m_t sv;
 #pragma unroll
@@ -2025,6 +2034,34 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_f32_mfma_kernel(
             }
         }
     }
+    if constexpr (NG > 1) {                         // the other groups' sums join the first's
+        constexpr int ONE = (DT * 16 + 2) * 64;     // a wave's sums, maxima and sums of weights
+        __syncthreads();
+        if (grp > 0) {
+            float* mrg = f32_lds + (size_t)((grp - 1) * HEADS + wave) * ONE;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mrg[(dt * 16 + r) * 64 + lane] = acc[dt][r];
+            mrg[DT * 16 * 64 + lane] = m;
+            mrg[(DT * 16 + 1) * 64 + lane] = l;
+        }
+        __syncthreads();
+        if (grp > 0) return;
+        for (int g = 0; g < NG - 1; ++g) {
+            const float* mrg = f32_lds + (size_t)(g * HEADS + wave) * ONE;
+            const float m1 = mrg[DT * 16 * 64 + lane], l1 = mrg[(DT * 16 + 1) * 64 + lane];
+            const float mn = fmaxf(m, m1);
+            const float a0 = (m == -INFINITY) ? 0.f : expf(m - mn);    // (a group that saw no key brings nothing)
+            const float a1 = (m1 == -INFINITY) ? 0.f : expf(m1 - mn);
+            l = l * a0 + l1 * a1;
+            m = mn;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[dt][r] = acc[dt][r] * a0 + mrg[(dt * 16 + r) * 64 + lane] * a1;
+        }
+    }
     if (!active || ql >= nrows) return;
     l += __shfl_xor(l, 32, LI_WAVE);               // (both halves of a query are past the return together)
     const float inv = l != 0.f ? 1.0f / l : 0.f;
@@ -2037,6 +2074,15 @@ __global__ __launch_bounds__(256) void paged_attention_prefill_f32_mfma_kernel(
                 float4{acc[dt][4 * rg] * inv, acc[dt][4 * rg + 1] * inv, acc[dt][4 * rg + 2] * inv, acc[dt][4 * rg + 3] * inv};
 }
 
+static int compute_units() {
+    int dev = 0, ncu = 0;
+    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
+        (void)hipGetLastError();
+        ncu = 256;
+    }
+    return ncu;
+}
+
 extern "C" int li_paged_attention_prefill_f32(const void* q, int q_row_stride, void* out, const void* kc,
                                               const void* vc, const int* block_table, int max_blocks,
                                               const int* tiles, int ntiles, const int* q_start, const int* q_len,
@@ -2045,13 +2091,25 @@ extern "C" int li_paged_attention_prefill_f32(const void* q, int q_row_stride, v
     if (ntiles <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || nh > 65535 || page_size <= 0 || max_blocks <= 0 ||
         num_pages <= 0 || !(scale > 0.f) || (q_row_stride % 4))
         return LI_ERR_SIZE;
-    if (nkv > 65535 || (nh / nkv + 3) / 4 > 65535) return LI_ERR_SIZE;
-    dim3 grid(ntiles, nkv, (nh / nkv + 3) / 4);
-#define LI_PF(DHV) paged_attention_prefill_f32_mfma_kernel<DHV><<<grid, 256, 0, stream>>>( \
-        (const float*)q, q_row_stride, (float*)out, (const float*)kc, (const float*)vc, block_table, max_blocks, \
+    if (nkv > 65535 || nh / nkv > 65535) return LI_ERR_SIZE;
+    const long group = nh / nkv, pairs = (long)ntiles * nkv, ncu = compute_units();
+    // Heads of a block x groups of its keys: as many blocks as the compute units take at about one time, the more the better while
+    // they last.  us, float32, (1 x 4, 2 x 2, 4 x 2, 4 x 1), 12 of 2 heads of 128: 810 new tokens 80, 84, 131, 143 (324 blocks of
+    // one head, 162 of two); 200 behind 7,800 738, 762, 1,206, 1,336; 2,000 407, 281, 311, 345 (756, 378, 126); 28 of 4 heads: 400
+    // tokens 60, 48, 71, 74 (364, 208, 104); 1,000 379, 202, 161, 177 (896, 512, 256); 2,000 behind 4,000 3,477, 2,155, 1,808, 1,750.
+    const int form = 3 * pairs * group <= 4 * ncu ? 1 : 2 * pairs * ((group + 1) / 2) <= 3 * ncu ? 2 : pairs * ((group + 3) / 4) <= ncu ? 3 : 4;
+#define LI_PF1(DHV, HEADS, NG)                                                                                                     \
+    paged_attention_prefill_f32_mfma_kernel<DHV, HEADS, NG><<<dim3(ntiles, nkv, (group + HEADS - 1) / HEADS), 64 * HEADS * NG,      \
+                                                              (size_t)NG * 2 * PF_T * (DHV + 4) * sizeof(float), stream>>>(          \
+        (const float*)q, q_row_stride, (float*)out, (const float*)kc, (const float*)vc, block_table, max_blocks,                     \
         tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale)
+#define LI_PF(DHV)                                                                                                                 \
+    do {                                                                                                                           \
+        if (form == 1) LI_PF1(DHV, 1, 4); else if (form == 2) LI_PF1(DHV, 2, 2); else if (form == 3) LI_PF1(DHV, 4, 2); else LI_PF1(DHV, 4, 1); \
+    } while (0)
     if (dh == 128) LI_PF(128); else if (dh == 64) LI_PF(64); else return LI_ERR_SIZE;
 #undef LI_PF
+#undef LI_PF1
     return li_launch_status();
 }
 

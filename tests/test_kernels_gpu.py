@@ -768,6 +768,20 @@ def test_prompt_attention_with_the_keys_of_its_first_tiles_in_runs(ops, monkeypa
         assert rel(out, ref) < 1.5e-2
 
 
+@pytest.mark.parametrize("segs,nh,nkv,dh,page,window", [
+    # one head, four groups: as few as one block of keys, so that groups have none; a window that begins inside a block of keys
+    ([(2, 2), (32, 32), (33, 33), (64, 5), (65, 2), (1, 1)], 6, 2, 128, 16, 0), ([(700, 500), (90, 90), (200, 161)], 3, 3, 128, 8, 50),
+    ([(500, 300), (70, 70), (97, 2)], 5, 1, 64, 12, 0),
+    # two heads, two groups: whole pairs of heads and a wave without one
+    ([(400, 400), (33, 33)], 28, 4, 128, 16, 0), ([(990, 990), (300, 40)], 12, 2, 64, 8, 100),
+    # four heads, two groups, with idle waves; and one group
+    ([(960, 960), (31, 2)], 28, 4, 64, 16, 0), ([(1056, 1056)], 32, 16, 64, 16, 0), ([(990, 990), (300, 40)], 24, 12, 128, 16, 100),
+])
+def test_prompt_attention_in_32_bits_with_its_keys_over_groups_of_waves(ops, segs, nh, nkv, dh, page, window):
+    out, ref = _paged_case(ops, torch.float32, segs, nh, nkv, dh, page, window, seed=36)
+    assert rel(out, ref) < 5e-6                     # float32 sums of up to some thousand terms: 2^-24 times the square root of their number
+
+
 def test_which_tiles_of_prompt_attention_have_their_keys_in_runs(ops):
     from litinfer_amd.kernels.ops import _prefill_tail
     tail = lambda new, cached, nh, nkv, heads: _prefill_tail(np.array(new, dtype=np.int32), np.array(cached, dtype=np.int32) + np.array(new, dtype=np.int32), nh, nkv, 128, 2000, 0, heads)
