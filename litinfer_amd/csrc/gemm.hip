@@ -852,8 +852,9 @@ __global__ __launch_bounds__(256) void gemm_bf16_big_kernel(const bf16_t* __rest
 // younger steps to stay outstanding waits exactly for the oldest step, and the
 // barrier after it makes that true for the loads of all four waves.
 // Needs K to be a multiple of the step (a load cannot be masked to zeros).  A step is 64
-// columns, so that a row of a stage is one whole 128-byte line of the caches.  Tiles: 256 x 256
-// with two stages, 256 x 128 with three, 128 x 128 with four (what fits the 160 KB of LDS).
+// columns, so that a row of a stage is one whole 128-byte line of the caches.  Tiles of 64 rows, 128 x
+// 128, 192 x 128, 256 x 128 and (gated) 128 x 256 with two to four stages (what fits the 160 KB of LDS);
+// larger tiles are `gemm_bf16_tile_kernel`'s.
 #define LI_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x0F70)
 #define LI_LOAD_TO_LDS(gptr, lptr)                                                                        \
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gptr),              \
@@ -2321,9 +2322,8 @@ extern "C" int li_linear_rope_store_parts(const void* x, const void* w, const fl
 // above the other the LDS reads take nearly as long as the MFMAs), and takes in about 50 GB/s, rows
 // of x that other units read too included: with few rows of x a tile waits for its part of w, and
 // wide tiles read x less often.  A last round that does not fill the chip counts for less than a
-// whole one: the units that run clock higher.  Fitted to measurements of all tilings at 128 to
-// 8,192 rows of the 1.5B and 7B layer shapes: the tiling it takes is within 4 % of the best one
-// there, but for the 7B's way back from the feed-forward at 4,096 rows and more (10 %).
+// whole one: the units that run clock higher.  Chooses among the widths of the gated product's 64-row tiles alone; tiles of more
+// rows go by `tiling_of`, whose steps are measured ones.
 static double tile_cost(int bm, int bn, double speed, int M, int N, int K) {
     const long tiles = (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn);
     const int cu = compute_units();

@@ -332,7 +332,8 @@ __device__ __forceinline__ void radix_kth(Each&& each, int kk, uint32_t& tau, in
 // others: the one with fewer than kk keys above it and at least kk no smaller is tau.  False, with nothing done, where the
 // bound leaves fewer than kk keys (a wave without enough of them sets none) or more than SMP_LIST (many equal logits):
 // radix_kth then.
-// 64 rows of 151,936 ids, top-k 50: tiles kernel 58 -> 45 us (one row 26 -> 13), rows kernel 22 -> 14.
+// 64 rows of 151,936 ids, top-k 50: tiles kernel 58 -> 45 us (one row 26 -> 13), rows kernel 22 -> 14.  Both are shorter since a tile hands
+// over all that it listed (below): top-k with top-p 44 + 25 -> 24 + 19.
 constexpr int SMP_LIST = 1024;
 // the bound, as above (0: none): at least kk of the block's keys are no smaller
 __device__ __forceinline__ uint32_t bound_of_kth(const uint32_t (&key)[8], int kk, int waves, int* work_i) {
