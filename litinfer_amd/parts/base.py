@@ -277,6 +277,7 @@ class Mixer(Part):
 
 class FeedForward(Part):
     category = "feed_forward"
+    adds_once = False          # the forward adds to its stream once, as the last thing it does, and by `add_by`
 
     def forward(self, xn, residual, ctx) -> None:
         raise NotImplementedError

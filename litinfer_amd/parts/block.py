@@ -123,13 +123,13 @@ class SandwichBlock(Block):
         stream.next_norm, stream.next_plain = None, False
         xn = self._read(stream, self.norm1, ctx)
         y = ctx.ws.buffer("block.branch", stream.shape, torch.float32)
-        branch = BranchStream(y, ctx.ws)
+        branch = BranchStream(y, ctx.ws, waits=False)
         self.mixer.forward(xn, branch, ctx, cache)
         last = self.ffn is None and self.token_input is None
         if self.ffn is not None:
             stream.add_normed(self.norm1b, branch, self.norm2, next_plain=self.norm2 is None)
             xn = self._read(stream, self.norm2, ctx)
-            branch = BranchStream(y, ctx.ws)
+            branch = BranchStream(y, ctx.ws, waits=getattr(self.ffn, "adds_once", False))
             self.ffn.forward(xn, branch, ctx)
             last = self.token_input is None
             stream.add_normed(self.norm2b, branch, after if last else None, next_plain=last and after_plain)
@@ -253,12 +253,12 @@ class HyperBlock(Block):
         after = stream.next_norm                   # who reads the streams after this block
         xn = stream.read(self.reader1, ctx.ws.buffer("block.xn", stream.shape, self.rt.dtype))
         y = ctx.ws.buffer("block.branch", stream.shape, torch.float32)
-        branch = BranchStream(y, ctx.ws)
+        branch = BranchStream(y, ctx.ws, waits=False)
         self.mixer.forward(xn, branch, ctx, cache)
         stream.write(branch, self.mix1, self.out1, self.reader2 if self.ffn is not None else after)
         if self.ffn is not None:
             xn = stream.read(self.reader2, ctx.ws.buffer("block.xn", stream.shape, self.rt.dtype))
-            branch = BranchStream(y, ctx.ws)
+            branch = BranchStream(y, ctx.ws, waits=False)
             self.ffn.forward(xn, branch, ctx)
             stream.write(branch, self.mix2, self.out2, after)
         stream.next_norm = None

@@ -115,6 +115,10 @@ class RoutedMLP(FeedForward):
                 out[s + n["shared_gate"]] = ParamSpec((1, self.hidden))
         return out
 
+    @property
+    def adds_once(self):
+        return type(self).forward is RoutedMLP.forward       # (a part made of this one may add again, through the same buffers)
+
     def batch_needs(self):
         return BatchNeeds(row_tile=self.shared_down.row_tile() if self.shared_down is not None else 1)
 

@@ -165,11 +165,14 @@ class ResidualStream:
 class BranchStream(ResidualStream):
     """What ONE sublayer puts out, for arrangements that treat it (norm it, gate it) before it joins the
     residual stream: the mixer or feed-forward is handed this in the stream's place, and its first
-    `add_linear` writes instead of adding."""
+    `add_linear` writes instead of adding.  With `waits` an output that its sublayer's kernel can still add, normed, to the
+    residual sum is left to that kernel, which then reads what the sublayer's forward left in its buffers: for a sublayer
+    that adds once, at the end of its forward (`FeedForward.adds_once`), and nothing else."""
 
-    def __init__(self, y: torch.Tensor, ws):
+    def __init__(self, y: torch.Tensor, ws, waits: bool = True):
         super().__init__(y, ws)
         self._fresh = True
+        self._may_wait = waits
         self._waiting = None                 # an output that its sublayer's kernel can still add, normed, to the residual sum: add_by's arguments
         self.second = None                   # a second output beside this one (a BranchStream with a factor of its own)
 
@@ -178,7 +181,7 @@ class BranchStream(ResidualStream):
         if self.second is not None:
             raise NotImplementedError("a branch holds at most two outputs")
         self._settle()
-        self.second = BranchStream(self.ws.buffer(name, self.x.shape, torch.float32), self.ws)
+        self.second = BranchStream(self.ws.buffer(name, self.x.shape, torch.float32), self.ws, waits=False)
         return self.second
 
     def outputs(self):
@@ -206,7 +209,7 @@ class BranchStream(ResidualStream):
 
     def add_by(self, add, add_normed=None, takes_norms=None) -> None:
         self._settle()
-        if add_normed is not None and self._fresh and self.second is None and takes_norms(self.x):
+        if self._may_wait and add_normed is not None and self._fresh and self.second is None and takes_norms(self.x):
             self._waiting = (add, add_normed)
             return
         add(self.tensor(), 1.0, None)        # (a branch's factor is applied when it joins)
@@ -226,6 +229,18 @@ class BranchStream(ResidualStream):
 
     def result(self) -> torch.Tensor:
         return self.tensor()
+
+    def gather(self, rows: torch.Tensor, out: torch.Tensor) -> None:
+        self._settle()
+        super().gather(rows, out)
+
+    def normed(self, norm, out: torch.Tensor) -> torch.Tensor:
+        self._settle()
+        return super().normed(norm, out)
+
+    def rounded(self, out: torch.Tensor) -> torch.Tensor:
+        self._settle()
+        return super().rounded(out)
 
 
 class StreamReader:

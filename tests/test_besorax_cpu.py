@@ -302,3 +302,49 @@ def test_an_output_that_waits_for_the_norm_behind_its_branch():
     b.factor = 0.5                                           # (applied when the branch joins)
     b.add_by(add, joined, yes)
     assert b.take_waiting(x) is None and torch.all(b.result() == 3)
+
+
+def test_only_a_lone_sums_output_waits_for_the_norm_behind_its_branch():
+    """A feed-forward that adds twice, its second output through the buffer of the first: both are summed, as they were."""
+    from types import SimpleNamespace
+    from litinfer_amd.parts.block import SandwichBlock
+    from litinfer_amd.parts.moe import RoutedMLP
+    from litinfer_amd.parts.stream import BranchStream
+    bufs = {}
+    ws = SimpleNamespace(buffer=lambda name, shape, dt: bufs.setdefault(name, torch.full(shape, 9.0, dtype=dt)))
+    norm = object()
+
+    class Twice:
+        def forward(self, xn, residual, ctx):
+            for v in (1.0, 2.0):
+                rows = ctx.ws.buffer("rows", (2, 3), torch.float32).fill_(v)
+                residual.add_by(lambda x, factor, tanh_norm: x.add_(rows, alpha=factor),
+                                lambda x, factor, before, after, out: x.add_(rows), lambda x: True)
+
+    class Stream:
+        shape, next_norm, next_plain, got = (2, 3), None, False, []
+
+        def normed(self, norm, out):
+            return out
+
+        def add_normed(self, norm, branch, *a, **kw):
+            take = branch.take_waiting(torch.zeros(2, 3))
+            self.got.append(branch.result().clone() if take is None else take)
+    block = SandwichBlock.__new__(SandwichBlock)
+    block.rt = SimpleNamespace(dtype=torch.float32)
+    block.norm1 = block.norm1b = block.norm2 = block.norm2b = norm
+    block.mixer = SimpleNamespace(forward=lambda xn, branch, ctx, cache: branch.tensor())
+    block.ffn, block.token_input = Twice(), None
+    block.forward(Stream(), SimpleNamespace(ws=ws), None)
+    assert torch.all(Stream.got[0] == 0) and torch.all(Stream.got[1] == 3)
+
+    class Wrapped(RoutedMLP):                                # (calls the part's forward as often as it likes)
+        def forward(self, xn, residual, ctx):
+            pass
+    assert RoutedMLP.__new__(RoutedMLP).adds_once and not Wrapped.__new__(Wrapped).adds_once
+    # whoever reads the branch as a stream finds an output that waited
+    norms = SimpleNamespace(forward=lambda x, out: out.copy_(x))
+    for read in (lambda b, out: b.normed(norms, out), lambda b, out: b.rounded(out)):
+        b = BranchStream(torch.full((2, 3), 9.0), ws)
+        b.add_by(lambda x, factor, tanh_norm: x.add_(5.0), lambda *a: None, lambda x: True)
+        assert torch.all(read(b, torch.empty(2, 3)) == 5.0)
