@@ -313,3 +313,19 @@ def test_unequal_pools_admission_waits_and_preemption_frees_the_windowed_group()
     # both tight: preemption happens and nothing is lost
     e, s, got = run([9, 5])
     assert got == want
+
+
+def test_an_event_is_recorded_by_a_torch_without_the_short_way_to_its_stream(monkeypatch):
+    import torch
+    from litinfer_amd.utils import pinned
+    recorded = []
+
+    class Event:
+        def record(self, *stream):
+            recorded.append(stream)
+    monkeypatch.setattr(torch.cuda, "Event", Event)
+    for name, module in (("_cuda_getCurrentStream", "_current_stream"), ("_cuda_getDevice", "_current_device")):
+        with monkeypatch.context() as m:
+            m.delattr(torch._C, name, raising=False)
+            m.setattr(pinned, module, None, raising=False)
+            assert isinstance(pinned.record_event(), Event) and recorded.pop() == ()
