@@ -184,6 +184,26 @@ def _prefill_tail(host_q_len, host_ctx_len, nh: int, nkv: int, dh: int, max_bloc
     return runs, out[0], out[1], out[2]
 
 
+def _prefill_plan(meta, nh: int, nkv: int, dh: int, window: int, lent: bool):
+    """(runs, heads a block, tiles whose keys are cut into the runs, their tokens, the batch's tokens up to the last of these) for
+    the prompt portions of a step, `lent`: with a workspace for the runs' results.  Looked up once a step for all layers with
+    these numbers (three calls into the library each: 6 us a layer, more than a small portion's kernel has to wait for)."""
+    key = ("prefill_plan", nh, nkv, dh, int(window), lent)
+    plan = meta.extra.get(key)
+    if plan is None:
+        lens, t = (getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None)), meta.num_tokens
+        # few tiles against long contexts: the tiles' keys in runs, joined by the kernel that joins the
+        # decode attention's (the library says how many; their results take room in the workspace)
+        runs = _prefill_runs(*lens, nh, nkv, dh, meta.max_blocks, window, t) if lent else 1
+        heads, cut_tiles, cut_tokens, upto = PREFILL_WAVES, meta.num_tiles, meta.num_multi, t
+        if runs == 1:
+            heads = _prefill_heads(*lens, nh, nkv, meta.max_blocks, window)
+            if lent:
+                runs, cut_tiles, cut_tokens, upto = _prefill_tail(*lens, nh, nkv, dh, meta.max_blocks, window, heads)
+        plan = meta.extra[key] = runs, heads, cut_tiles, cut_tokens, upto
+    return plan
+
+
 # the current stream's handle without the stream object around it (an op is called some hundred times a
 # step, and the object's way through torch's Python layers took a quarter of a step's host time)
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -1630,18 +1650,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
     # positions by the page size in float, exact below 2^21 keys; longer tables take the general kernel
     if (n_multi and qkv.dtype is torch.bfloat16 and dh in (64, 128) and meta.num_tiles
             and meta.tile_rows == PREFILL_TILE_ROWS and n_multi == meta.num_multi and meta.max_blocks <= 8192 and meta.max_blocks * page_size <= 1 << 21):
-        # few tiles against long contexts: the tiles' keys in runs, joined by the kernel that joins the
-        # decode attention's (the library says how many; their results take room in the workspace)
-        runs = 1
-        if ws is not None:
-            runs = _prefill_runs(getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None), nh, nkv, dh,
-                                 meta.max_blocks, window, t)
-        heads, cut_tiles, cut_tokens, upto = PREFILL_WAVES, meta.num_tiles, n_multi, t
-        if runs == 1:
-            lens = getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None)
-            heads = _prefill_heads(*lens, nh, nkv, meta.max_blocks, window)
-            if ws is not None:
-                runs, cut_tiles, cut_tokens, upto = _prefill_tail(*lens, nh, nkv, dh, meta.max_blocks, window, heads)
+        runs, heads, cut_tiles, cut_tokens, upto = _prefill_plan(meta, nh, nkv, dh, window, ws is not None)
         acc = ml = lst = None
         if runs > 1:
             acc = ws.buffer("attn.runs_acc", (upto, nh, runs, dh), torch.float32)

@@ -53,3 +53,36 @@ def test_the_decode_kernels_float_quotient_is_the_page_of_every_key():
         inv = np.float32(1.0) / np.float32(page)
         blk = ((keys.astype(np.float32) + half) * inv).astype(np.int64)
         assert np.array_equal(blk, keys // page), page
+
+
+def test_prompt_attention_is_planned_once_a_step(monkeypatch):
+    """A step's layers share what the library says of its portions; another window or step asks again."""
+    from types import SimpleNamespace
+    import torch
+    from litinfer_amd.engine.batch import AttentionMeta
+    asked = []
+    for name, says in (("_prefill_runs", 1), ("_prefill_heads", 2), ("_prefill_tail", (3, 2, 64, 64))):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, says=says: (asked.append(name), says)[1])
+    sent = []
+    monkeypatch.setattr(ops, "_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "_run", lambda *a: sent.append(a))
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32)
+    t, nh, nkv, dh, page = 70, 6, 2, 64, 16
+
+    def step():
+        return AttentionMeta(block_table=torch.zeros(1, 5, dtype=torch.int32), max_blocks=5, seg_of_token=torch.zeros(t, dtype=torch.int32),
+                             q_start=ints(0), q_len=ints(t), ctx_len=ints(t), num_segments=1, num_tokens=t, max_q_len=t, max_ctx_len=t,
+                             host_q_start=np.zeros(1, np.int32), host_q_len=np.full(1, t, np.int32), host_ctx_len=np.full(1, t, np.int32),
+                             num_single=0, num_multi=t, tiles=torch.zeros(3, 4, dtype=torch.int32), num_tiles=3, tile_rows=32)
+    cache = torch.zeros(8, nkv, page, dh, dtype=torch.bfloat16)
+    q = torch.zeros(t, nh * dh, dtype=torch.bfloat16)
+    ws = SimpleNamespace(buffer=lambda name, shape, dt, zero=False: torch.zeros(shape, dtype=dt))
+    call = lambda meta, window: ops.paged_attention(q, torch.empty_like(q), cache, cache.clone(), meta, nh, nkv, dh, page, window, 0.1, ws=ws)
+    first = step()
+    for _ in range(28):
+        call(first, 0)
+    assert asked == ["_prefill_runs", "_prefill_heads", "_prefill_tail"]
+    assert len(sent) == 28 and all(s[1] == "li_paged_attention_prefill" and s[-7] == 3 and s[-3:] == (64, 2, 2) for s in sent)
+    call(first, 40)
+    call(step(), 0)
+    assert len(asked) == 9
