@@ -8,6 +8,10 @@
 // division are float32 (online softmax); the output is rounded once.
 #include "common.h"
 #include <math.h>
+#include <exception>
+#include <functional>
+#include <queue>
+#include <vector>
 
 #define ATT_MAX_DH 256
 
@@ -2171,66 +2175,65 @@ extern "C" int li_paged_attention_prefill_runs(int nseg, const int* q_len, const
     return pick;
 }
 
-// How many heads of a group a block's four waves are (the others are tiles that follow each other): 4, 2 or 1.  q_len, ctx_len: the
-// batch's segments in HOST memory.  The estimate, in blocks of 32 keys: rounds of blocks over the chip (two a compute unit; a last
-// one that does not fill it counts for 0.4 of its rest) x the mean block's keys (those of its last tile) x what a block with so many
-// waves at work takes (measured where a round is full: 395, 460, 508 and 600 us with one to four of them; a wave waits for the
-// others' keys and its own chain either way).  A round that does not fill the chip keeps one tile a block: its time is one block's.
-// 1,999 tokens behind 16,000 keys, us, with four heads a block and as taken here: 32 heads of 32 kv heads 1,540 -> 594, 32 of
-// 16 910 -> 580; 40 of 8 940 -> 909 (a last round of 128 blocks), 2,048 tokens from their start 75 -> 65, 4,096 264 -> 202; 28 of 4
-// heads stay with four (2,048 tokens 55 us).
-extern "C" int li_paged_attention_prefill_heads(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int max_blocks, int window) {
-    if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP) return PRE_WAVES;
-    const int G = nh / nkv;
-    if (G % PRE_WAVES == 0) return PRE_WAVES;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
-        (void)hipGetLastError();
-        ncu = 256;
-    }
-    const double at_work[PRE_WAVES + 1] = {0.0, 0.66, 0.77, 0.85, 1.0};
-    int pick = PRE_WAVES;
-    double best = 0.0;
-    for (int heads = PRE_WAVES; heads >= 1; heads /= 2) {
-        const int abreast = PRE_WAVES / heads, parts = (G + heads - 1) / heads;
-        long groups = 0, keys = 0;
-        for (int i = 0; i < nseg; ++i) {
-            if (q_len[i] <= 1) continue;
-            for (int a = 0; a < q_len[i]; a += 32 * abreast) {
-                const int p0 = ctx_len[i] - q_len[i] + a, rows = q_len[i] - a < 32 * abreast ? q_len[i] - a : 32 * abreast;
-                const int lo0 = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
-                ++groups;
-                keys += (p0 + rows - (lo0 & ~31) + 31) / 32 + 8;
+// When the blocks of a prompt portion's launch are done, in units of a block of 32 keys with all four waves at work: `longest`, where each is
+// started in the kernel's order as one of the compute units' places (two a unit) comes free, and `mean`, what a place has to
+// do on average.  A block has its keys and 7 more for its start and end, times what one with so many waves at work takes (one of four keeps a
+// unit busy for three quarters of the time of four: a wave waits for the others' keys and its own chain either way).
+// The kv heads' blocks are alike, so one of them stands for all, on so many fewer places.  `runs` and `split_tiles`: as the kernel's.
+struct PrefillTime { double longest, mean; long blocks; };
+static PrefillTime prefill_time(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int window, int heads, int runs, long split_tiles) {
+    static const double at_work[PRE_WAVES + 1] = {0.0, 0.72, 0.84, 0.93, 1.0};
+    struct Tile { int segment, row; };
+    std::vector<Tile> tiles;
+    for (int i = 0; i < nseg; ++i)
+        if (q_len[i] > 1)
+            for (int a = 0; a < q_len[i]; a += 32) tiles.push_back(Tile{i, a});
+    const int G = nh / nkv, abreast = PRE_WAVES / heads, parts = (G + heads - 1) / heads;
+    const long ntiles = (long)tiles.size(), rows = (ntiles + abreast - 1) / abreast;
+    const long split_rows = runs > 1 ? (split_tiles >= ntiles ? rows : split_tiles / abreast) : 0;
+    const long places = 2l * compute_units() / nkv > 1 ? 2l * compute_units() / nkv : 1;
+    std::priority_queue<double, std::vector<double>, std::greater<double>> free_at(std::greater<double>(), std::vector<double>((size_t)places, 0.0));
+    PrefillTime r{0.0, 0.0, 0};
+    for (int cut = 0; cut < 2; ++cut) {
+        const long first = cut ? 0 : split_rows, these = cut ? split_rows : rows - split_rows;
+        const int cuts = cut ? runs : 1;
+        for (long turn = 0; turn < these * abreast; ++turn) {
+            const long tile = (first + these - 1 - turn % these) * abreast + turn / these;
+            if (tile >= ntiles || (tiles[tile].row / 32) % abreast) continue;
+            const int i = tiles[tile].segment, a = tiles[tile].row, p0 = ctx_len[i] - q_len[i] + a;
+            const int more = q_len[i] - a < 32 * abreast ? q_len[i] - a : 32 * abreast;
+            const int lo0 = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
+            const int keys = (p0 + more - (lo0 & ~31) + 31) / 32, per = (keys + cuts - 1) / cuts;
+            for (int part = 0; part < parts; ++part) {
+                const double waves = at_work[(G - part * heads < heads ? G - part * heads : heads) * ((more + 31) / 32)];
+                for (int run = 0; run < cuts; ++run) {
+                    const int left = keys - run * per, mine = left < 0 ? 0 : left < per ? left : per;
+                    const double end = free_at.top() + (mine + 7) * waves;
+                    free_at.pop();
+                    free_at.push(end);
+                    r.longest = end > r.longest ? end : r.longest;
+                    r.mean += (mine + 7) * waves / places;
+                    ++r.blocks;
+                }
             }
         }
-        if (groups == 0) return PRE_WAVES;
-        const double filled = (double)groups * nkv * parts / (2.0 * ncu), whole = ceil(filled);
-        if (heads == PRE_WAVES && filled <= 1.0) return PRE_WAVES;
-        double waves = 0.0;                                              // (the last of a group's blocks may have fewer heads)
-        for (int b = 0; b < parts; ++b) waves += at_work[(G - b * heads < heads ? G - b * heads : heads) * abreast];
-        const double us = (filled + 0.4 * (whole - filled)) * ((double)keys / groups) * (waves / parts);
-        if (heads == PRE_WAVES) best = 0.97 * us;
-        else if (us < best) { best = us; pick = heads; }
     }
-    return pick;
+    r.blocks *= nkv;
+    return r;
 }
 
 // Where the blocks fill the chip (two a compute unit) some whole rounds and a few are left, these few take a round of their own, each as
 // long as its chain of keys: their tiles' keys are cut into so many runs that they fill the chip as well.  The tiles in question
 // are the first of the list (the last that are started); *split_tiles takes their number, *split_tokens the tokens of the blocks that
-// begin with one of them and *upto the batch's tokens up to the last of those.  Returns the runs, 1 for none.  A block of 32 keys takes about 1.1 us where two blocks
-// share a unit and 0.7 where one has it alone (1,999 tokens behind 16,000, 40 of 8 heads: 512 blocks 590 us, the other 128 365).
-extern "C" int li_paged_attention_prefill_tail(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh, int max_blocks, int window,
-                                               int heads, long max_bytes, int* split_tiles, int* split_tokens, int* upto) {
-    if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nh > 4 * 65535 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP || !split_tiles || !split_tokens ||
-        !upto || (heads != 1 && heads != 2 && heads != PRE_WAVES)) return 1;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
-        (void)hipGetLastError();
-        ncu = 256;
-    }
+// begin with one of them and *upto the batch's tokens up to the last of those.  Returns the runs, 1 for none.  Only where the last block
+// is then done, the runs joined, 5 % earlier: segments of different lengths do not run in rounds, and a first tile's few keys
+// gain nothing.  103 batches of one to five segments in seven head layouts, where rounds alone would cut: 26 were 3 to 14 % slower for it; with
+// the ends of all blocks worked out none is by more than 2 %, and 40 are cut, 12 % faster on average (1,999 tokens behind 16,000, 40 of 8
+// heads: 909 -> 812 us; 290 tokens behind 2,048 and 2,048 from their start, 28 of 4: 84.8 -> 79.0).
+static int prefill_tail(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh, int window, int heads, long max_bytes, const PrefillTime& whole,
+                        PrefillTime* with, int* split_tiles, int* split_tokens, int* upto) {
     const int abreast = PRE_WAVES / heads, parts = (nh / nkv + heads - 1) / heads;
-    const long each = (long)nkv * parts, round = 2l * ncu;
+    const long each = (long)nkv * parts, round = 2l * compute_units();
     long groups = 0;
     for (int i = 0; i < nseg; ++i)
         if (q_len[i] > 1) groups += (q_len[i] + 32 * abreast - 1) / (32 * abreast);
@@ -2253,18 +2256,66 @@ extern "C" int li_paged_attention_prefill_tail(int nseg, const int* q_len, const
         }
     }
     if (tail == 0 || tail >= groups) return 1;
-    const long blocks = tail * each;
     const double mean = (double)keys / tail;
-    int runs = (int)(round / blocks);
+    int runs = (int)(round / (tail * each));
     if (runs > MERGE_RUNS_MAX) runs = MERGE_RUNS_MAX;
     while (runs > 1 && (mean / runs < 16.0 || (long)last * nh * runs * (dh + 2) * 4 > max_bytes)) --runs;
     if (runs < 2) return 1;
-    const double alone = 0.7 * mean, cut = 1.1 * (mean / runs + 8.0) + 5.0 + (double)tokens * nh * runs * dh * 8.0 / 6.0e6;
-    if (cut > 0.85 * alone) return 1;
+    *with = prefill_time(nseg, q_len, ctx_len, nh, nkv, window, heads, runs, tile);
+    // (the runs' results are written and read again by a launch of their own; a block of keys takes about 1.1 us)
+    const double joining = (5.0 + (double)tokens * nh * runs * dh * 8.0 / 6.0e6) / 1.1;
+    with->longest += joining;
+    with->mean += joining;
+    if (with->longest > 0.95 * whole.longest) return 1;
     *split_tiles = (int)tile;
     *split_tokens = tokens;
     *upto = last;
     return runs;
+}
+
+extern "C" int li_paged_attention_prefill_tail(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh, int max_blocks, int window,
+                                               int heads, long max_bytes, int* split_tiles, int* split_tokens, int* upto) {
+    if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nh > 4 * 65535 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP || !split_tiles || !split_tokens ||
+        !upto || (heads != 1 && heads != 2 && heads != PRE_WAVES)) return 1;
+    try {
+        PrefillTime with;
+        const PrefillTime whole = prefill_time(nseg, q_len, ctx_len, nh, nkv, window, heads, 1, 0);
+        return prefill_tail(nseg, q_len, ctx_len, nh, nkv, dh, window, heads, max_bytes, whole, &with, split_tiles, split_tokens, upto);
+    } catch (const std::exception&) {                    // (no memory for the list of tiles: nothing is cut)
+        return 1;
+    }
+}
+
+// How many heads of a group a block's four waves are (the others are tiles that follow each other): 4, 2 or 1.  q_len, ctx_len: the
+// batch's segments in HOST memory; max_bytes: room for runs of the last round's keys (0: none), which may follow (above).  By the ends of
+// the blocks: half of the last one's and half of what a place has to do on average, since a unit with one block left works faster; fewer
+// heads for a clear gain (10 %) alone.  A round that does not fill the chip keeps one tile a block: its time is one block's.
+// 1,503 batches of one to five segments with heads of 128, in eleven layouts whose groups do not divide by four: in 13 % less time on average
+// than with four heads a block, 21 are slower by more than 3 %, at worst 13 %; by the mean block's time alone 89 were, at worst 56 %: the
+// longest segment's blocks in a round of their own.  Heads of 64 stay with four: 143 batches took 1 % longer with what that picked, at worst 25 %.
+// 1,999 tokens behind 16,000 keys, us, with four heads a block and as taken here: 32 heads of 32 kv heads 1,540 -> 594, 32 of
+// 16 910 -> 580; 40 of 8 940 -> 909 (812 with the runs); 2,048 tokens from their start 75 -> 65, 4,096 264 -> 202; 28 of 4
+// heads stay with four (2,048 tokens 55 us).
+extern "C" int li_paged_attention_prefill_heads(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh, int max_blocks, int window, long max_bytes) {
+    if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nh > 4 * 65535 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP) return PRE_WAVES;
+    if ((nh / nkv) % PRE_WAVES == 0 || dh != 128) return PRE_WAVES;
+    try {
+        int pick = PRE_WAVES;
+        double best = 0.0;
+        for (int heads = PRE_WAVES; heads >= 1; heads /= 2) {
+            const PrefillTime whole = prefill_time(nseg, q_len, ctx_len, nh, nkv, window, heads, 1, 0);
+            if (heads == PRE_WAVES && whole.blocks <= 2l * compute_units()) return PRE_WAVES;
+            PrefillTime with = whole;
+            int tiles, tokens, upto;
+            if (max_bytes <= 0 || prefill_tail(nseg, q_len, ctx_len, nh, nkv, dh, window, heads, max_bytes, whole, &with, &tiles, &tokens, &upto) == 1) with = whole;
+            const double time = 0.5 * (with.longest + with.mean);
+            if (heads == PRE_WAVES) best = 0.9 * time;
+            else if (time < (pick == PRE_WAVES ? 1.0 : 0.98) * best) { best = time; pick = heads; }
+        }
+        return pick;
+    } catch (const std::exception&) {
+        return PRE_WAVES;
+    }
 }
 
 // tiles: int [ntiles, 4] = (segment, first token of the tile in the batch, rows <= 32, unused)

@@ -162,13 +162,14 @@ def _prefill_runs(host_q_len, host_ctx_len, nh: int, nkv: int, dh: int, max_bloc
 PREFILL_WAVES = 4                      # waves of a block of that kernel: heads of a group, or tiles that follow each other
 
 
-def _prefill_heads(host_q_len, host_ctx_len, nh: int, nkv: int, max_blocks: int, window: int) -> int:
+def _prefill_heads(host_q_len, host_ctx_len, nh: int, nkv: int, max_blocks: int, window: int, dh: int = 128, lent: bool = True) -> int:
     """How many heads of a group a block of the prompt portions' kernel takes (the batch's segments as int32 arrays in
-    host memory)."""
+    host memory); `lent`: the last round's keys may be cut into runs."""
     if (nh // nkv) % PREFILL_WAVES == 0 or host_q_len is None or host_ctx_len is None or host_q_len.dtype != "int32" or host_ctx_len.dtype != "int32":
         return PREFILL_WAVES
-    f = _lib_fn("attention", "li_paged_attention_prefill_heads", [c_int, c_void_p, c_void_p] + [c_int] * 4, c_int)
-    return int(f(len(host_q_len), host_q_len.ctypes.data, host_ctx_len.ctypes.data, nh, nkv, max_blocks, int(window)))
+    f = _lib_fn("attention", "li_paged_attention_prefill_heads", [c_int, c_void_p, c_void_p] + [c_int] * 5 + [c_long], c_int)
+    return int(f(len(host_q_len), host_q_len.ctypes.data, host_ctx_len.ctypes.data, nh, nkv, dh, max_blocks, int(window),
+                 PREFILL_RUNS_MAX_BYTES if lent else 0))
 
 
 def _prefill_tail(host_q_len, host_ctx_len, nh: int, nkv: int, dh: int, max_blocks: int, window: int, heads: int):
@@ -197,7 +198,7 @@ def _prefill_plan(meta, nh: int, nkv: int, dh: int, window: int, lent: bool):
         runs = _prefill_runs(*lens, nh, nkv, dh, meta.max_blocks, window, t) if lent else 1
         heads, cut_tiles, cut_tokens, upto = PREFILL_WAVES, meta.num_tiles, meta.num_multi, t
         if runs == 1:
-            heads = _prefill_heads(*lens, nh, nkv, meta.max_blocks, window)
+            heads = _prefill_heads(*lens, nh, nkv, meta.max_blocks, window, dh, lent)
             if lent:
                 runs, cut_tiles, cut_tokens, upto = _prefill_tail(*lens, nh, nkv, dh, meta.max_blocks, window, heads)
         plan = meta.extra[key] = runs, heads, cut_tiles, cut_tokens, upto
