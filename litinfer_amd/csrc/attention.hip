@@ -2087,21 +2087,31 @@ static int compute_units() {
     return ncu;
 }
 
+// Heads of a block x groups of its keys (1: 1 x 4, 2: 2 x 2, 3: 4 x 2, 4: 4 x 1): as many blocks as the compute units take at about one
+// time, the more the better while they last.  us, float32, (1 x 4, 2 x 2, 4 x 2, 4 x 1), 12 of 2 heads of 128: 810 new tokens 80, 84, 131,
+// 143 (324 blocks of one head, 162 of two); 200 behind 7,800 738, 762, 1,206, 1,336; 2,000 407, 281, 311, 345 (756, 378, 126); 28 of 4
+// heads: 400 tokens 60, 48, 71, 74 (364, 208, 104); 1,000 379, 202, 161, 177 (896, 512, 256); 2,000 behind 4,000 3,477, 2,155, 1,808, 1,750.
+// With one block of keys (max_keys: the longest context; 0: not known) further groups have nothing to add but their join: 10.1 -> 11.6 us.
+// And one head's four groups of 128 columns fill a unit's LDS, so more blocks than units are two rounds, which pay from three
+// blocks of keys on: 320 blocks, contexts of 64 17.5 -> 21.9 us, of 96 24.1 -> 22.0, of 128 30.8 -> 22.3.
+extern "C" int li_paged_attention_prefill_f32_form(int ntiles, int nh, int nkv, int dh, int max_keys) {
+    if (nkv <= 0) return 4;
+    const long group = nh / nkv, pairs = (long)ntiles * nkv, ncu = compute_units();
+    if (max_keys > 0 && max_keys <= PF_T) return 4;
+    if (3 * pairs * group <= 4 * ncu) return max_keys > 0 && max_keys <= 2 * PF_T && dh == 128 && pairs * group > ncu ? 4 : 1;
+    return 2 * pairs * ((group + 1) / 2) <= 3 * ncu ? 2 : pairs * ((group + 3) / 4) <= ncu ? 3 : 4;
+}
+
 extern "C" int li_paged_attention_prefill_f32(const void* q, int q_row_stride, void* out, const void* kc,
                                               const void* vc, const int* block_table, int max_blocks,
                                               const int* tiles, int ntiles, const int* q_start, const int* q_len,
                                               const int* ctx_len, int nh, int nkv, int dh, int page_size,
-                                              int num_pages, int window, float scale, hipStream_t stream) {
+                                              int num_pages, int window, float scale, int max_keys, hipStream_t stream) {
     if (ntiles <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || nh > 65535 || page_size <= 0 || max_blocks <= 0 ||
         num_pages <= 0 || !(scale > 0.f) || (q_row_stride % 4))
         return LI_ERR_SIZE;
     if (nkv > 65535 || nh / nkv > 65535) return LI_ERR_SIZE;
-    const long group = nh / nkv, pairs = (long)ntiles * nkv, ncu = compute_units();
-    // Heads of a block x groups of its keys: as many blocks as the compute units take at about one time, the more the better while
-    // they last.  us, float32, (1 x 4, 2 x 2, 4 x 2, 4 x 1), 12 of 2 heads of 128: 810 new tokens 80, 84, 131, 143 (324 blocks of
-    // one head, 162 of two); 200 behind 7,800 738, 762, 1,206, 1,336; 2,000 407, 281, 311, 345 (756, 378, 126); 28 of 4 heads: 400
-    // tokens 60, 48, 71, 74 (364, 208, 104); 1,000 379, 202, 161, 177 (896, 512, 256); 2,000 behind 4,000 3,477, 2,155, 1,808, 1,750.
-    const int form = 3 * pairs * group <= 4 * ncu ? 1 : 2 * pairs * ((group + 1) / 2) <= 3 * ncu ? 2 : pairs * ((group + 3) / 4) <= ncu ? 3 : 4;
+    const int group = nh / nkv, form = li_paged_attention_prefill_f32_form(ntiles, nh, nkv, dh, max_keys);
 #define LI_PF1(DHV, HEADS, NG)                                                                                                     \
     paged_attention_prefill_f32_mfma_kernel<DHV, HEADS, NG><<<dim3(ntiles, nkv, (group + HEADS - 1) / HEADS), 64 * HEADS * NG,      \
                                                               (size_t)NG * 2 * PF_T * (DHV + 4) * sizeof(float), stream>>>(          \

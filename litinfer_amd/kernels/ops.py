@@ -99,7 +99,7 @@ _SIGNATURES = {
     "attention": {
         "li_paged_attention": [P, I, P, P, P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, F],
         "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I, I, I],
-        "li_paged_attention_prefill_f32": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F],
+        "li_paged_attention_prefill_f32": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I],
         "li_paged_attention_decode": [P, I, P, P, P, I, P, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, P],
         "li_decode_run_keys": [P, I, P, P, P, P, I, I, I, I, I, I, I, P],
     },
@@ -203,6 +203,15 @@ def _prefill_plan(meta, nh: int, nkv: int, dh: int, window: int, lent: bool):
                 runs, cut_tiles, cut_tokens, upto = _prefill_tail(*lens, nh, nkv, dh, meta.max_blocks, window, heads)
         plan = meta.extra[key] = runs, heads, cut_tiles, cut_tokens, upto
     return plan
+
+
+def _prefill_keys(meta) -> int:
+    """The longest context among a step's portions (0: not known); looked up once a step."""
+    keys = meta.extra.get("prefill_keys")
+    if keys is None:
+        q, c = getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None)
+        keys = meta.extra["prefill_keys"] = 0 if q is None or c is None else min(int(c[q > 1].max(initial=0)), 1 << 30)
+    return keys
 
 
 # the current stream's handle without the stream object around it (an op is called some hundred times a
@@ -1669,7 +1678,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
         _run("attention", "li_paged_attention_prefill_f32", qkv.data_ptr(), qkv.stride(0), out.data_ptr(),
              k.data_ptr(), v.data_ptr(), bt.data_ptr(), meta.max_blocks, meta.tiles.data_ptr(),
              meta.num_tiles, meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
-             nh, nkv, dh, page_size, k.shape[0], int(window), float(scale))
+             nh, nkv, dh, page_size, k.shape[0], int(window), float(scale), _prefill_keys(meta))
     elif n_multi:
         lst = meta.multi_tokens if n_multi < t else None
         _run("attention", "li_paged_attention", qkv.data_ptr(), qkv.stride(0), out.data_ptr(),

@@ -114,3 +114,16 @@ def test_keys_of_the_first_tiles_are_cut_only_where_the_last_block_is_done_earli
         for heads in (4, 2, 1):
             runs, tiles, tokens, upto = tail(segs, 6, 2, heads)
             assert runs == 1 or (0 < tokens <= upto <= sum(q for _, q in segs) and tiles % (4 // heads) == 0)
+
+
+def test_groups_of_keys_of_the_32_bit_prompt_attention():
+    """Heads x groups of a block (1: one head in four groups ... 4: four heads in one): no further groups for a single block of keys, nor
+    two rounds of blocks for two."""
+    import ctypes
+    f = ops._lib_fn("attention", "li_paged_attention_prefill_f32_form", [ctypes.c_int] * 5, ctypes.c_int)
+    assert [f(1, 28, 4, 128, keys) for keys in (2, 32, 33, 200, 0)] == [4, 4, 1, 1, 1]
+    assert [f(8, 40, 8, 128, keys) for keys in (2, 64, 65, 0)] == [4, 4, 1, 1]          # 320 blocks of one head: more than units
+    assert [f(6, 40, 8, 128, keys) for keys in (2, 64)] == [4, 1]                       # 240: not more
+    assert [f(8, 40, 8, 64, keys) for keys in (32, 64)] == [4, 1]                       # two blocks of 64 columns share a unit
+    assert [f(13, 28, 4, 128, 400), f(32, 28, 4, 128, 1000), f(63, 28, 4, 128, 2000)] == [2, 3, 4]
+    assert f(13, 28, 4, 128, 20) == f(32, 28, 4, 128, 20) == 4
