@@ -2113,13 +2113,22 @@ extern "C" int li_paged_attention_prefill_f32(const void* q, int q_row_stride, v
     if (nkv > 65535 || nh / nkv > 65535) return LI_ERR_SIZE;
     const int group = nh / nkv, form = li_paged_attention_prefill_f32_form(ntiles, nh, nkv, dh, max_keys);
 #define LI_PF1(DHV, HEADS, NG)                                                                                                     \
-    paged_attention_prefill_f32_mfma_kernel<DHV, HEADS, NG><<<dim3(ntiles, nkv, (group + HEADS - 1) / HEADS), 64 * HEADS * NG,      \
-                                                              (size_t)NG * 2 * PF_T * (DHV + 4) * sizeof(float), stream>>>(          \
-        (const float*)q, q_row_stride, (float*)out, (const float*)kc, (const float*)vc, block_table, max_blocks,                     \
-        tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale)
+    {                                                                                                                              \
+        constexpr int lds_bytes = NG * 2 * PF_T * (DHV + 4) * (int)sizeof(float);                                                   \
+        static bool configured = lds_bytes <= 64 * 1024;         /* (up to 135 KB) */                                               \
+        if (!configured) {                                                                                                         \
+            if (hipFuncSetAttribute((const void*)paged_attention_prefill_f32_mfma_kernel<DHV, HEADS, NG>,                           \
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)                           \
+                return LI_ERR_LAUNCH;                                                                                              \
+            configured = true;                                                                                                     \
+        }                                                                                                                          \
+        paged_attention_prefill_f32_mfma_kernel<DHV, HEADS, NG><<<dim3(ntiles, nkv, (group + HEADS - 1) / HEADS), 64 * HEADS * NG, lds_bytes, stream>>>( \
+            (const float*)q, q_row_stride, (float*)out, (const float*)kc, (const float*)vc, block_table, max_blocks,                 \
+            tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale);                                          \
+    }
 #define LI_PF(DHV)                                                                                                                 \
     do {                                                                                                                           \
-        if (form == 1) LI_PF1(DHV, 1, 4); else if (form == 2) LI_PF1(DHV, 2, 2); else if (form == 3) LI_PF1(DHV, 4, 2); else LI_PF1(DHV, 4, 1); \
+        if (form == 1) LI_PF1(DHV, 1, 4) else if (form == 2) LI_PF1(DHV, 2, 2) else if (form == 3) LI_PF1(DHV, 4, 2) else LI_PF1(DHV, 4, 1)       \
     } while (0)
     if (dh == 128) LI_PF(128); else if (dh == 64) LI_PF(64); else return LI_ERR_SIZE;
 #undef LI_PF
@@ -2141,11 +2150,7 @@ extern "C" int li_paged_attention_prefill_f32(const void* q, int q_row_stride, v
 extern "C" int li_paged_attention_prefill_runs(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh,
                                                int max_blocks, int window, int tokens, long max_bytes) {
     if (nseg <= 0 || !q_len || !ctx_len || nh <= 0 || nh > 4 * 65535 || nkv <= 0 || nh % nkv || max_blocks > PRE2_TABLE_CAP) return 1;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
-        (void)hipGetLastError();
-        ncu = 256;
-    }
+    const int ncu = compute_units();
     long ntiles = 0, work = 0;
     int len = 0;                                                        // the longest tile's blocks of keys
     for (int i = 0; i < nseg; ++i) {
@@ -2355,11 +2360,7 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
     const long blocks = ((long)(rows - split_rows) + (long)split_rows * runs) * abreast * nkv * parts;
     if (blocks > 0x7fffffffl) return LI_ERR_SIZE;
     dim3 grid(ntiles, nkv, parts);
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu <= 0) {
-        (void)hipGetLastError();
-        ncu = 256;
-    }
+    const int ncu = compute_units();
 #define LI_PRE(DHV) paged_attention_prefill_mfma_kernel<DHV><<<grid, PRE_WAVES * 64, 0, stream>>>( \
         (const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc, (const bf16_t*)vc, block_table, max_blocks, \
         tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, scale, ncu)
