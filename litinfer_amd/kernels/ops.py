@@ -2037,8 +2037,16 @@ MOE_ROUTE_PLAN_TOKENS, MOE_ROUTE_PLAN_EXPERTS = 128, 64
 
 
 def moe_route_takes_plan(t: int, experts: int, hidden: int) -> bool:
-    """Whether `moe_route` makes the plan too: a decoding step's few pairs, by the wave that made the last choice."""
+    """Whether `moe_route` can make the plan too: a decoding step's few pairs, by the wave that made the last choice."""
     return 0 < t <= MOE_ROUTE_PLAN_TOKENS and experts <= MOE_ROUTE_PLAN_EXPERTS and hidden >= 64
+
+
+def moe_route_plan_pays(t: int, experts: int, hidden: int) -> bool:
+    """Whether it should.  One wave lists all pairs, 64 a trip to memory, while the plan's own launch has more; with few experts
+    the router itself has little for the other blocks to do meanwhile.  us, both in one launch against two, rows of 2,048: 1 token of
+    16 experts 6.5 / 7.9, 64 tokens 8.6 / 9.3, 96 9.6 / 9.4, 128 10.4 / 9.5; 64 tokens of 60 experts, 10 each, 20.8 / 22.7, 96 23.9 /
+    22.9; of 8 experts 32 tokens 7.6 / 8.0, 48 8.3 / 8.0, 128 10.5 / 8.4."""
+    return moe_route_takes_plan(t, experts, hidden) and t <= (64 if experts >= 16 else 32)
 
 
 def _check_plan(what: str, t: int, top: int, p: MoePlan) -> int:

@@ -157,7 +157,7 @@ class RoutedMLP(FeedForward):
         pair_row = ws.buffer("moe.pair_row", (pairs,), torch.int32)
         row_wt = ws.buffer("moe.row_wt", (pairs,), torch.float32) if self.weigh_input else None
         count = ws.buffer("moe.count", (1,), torch.int32, zero=True)         # (asked for by every step: a recorded one finds it)
-        with_plan = ops.moe_route_takes_plan(t, self.experts, self.hidden)
+        with_plan = ops.moe_route_plan_pays(t, self.experts, self.hidden)
         ops.moe_route(xn, self.router, self.router_b, self.gate_row, idx, wt, gate, scores=self.scores,
                       correction=self.correction, groups=self.groups, keep_groups=self.keep_groups,
                       group_score=self.group_score, normalize=self.normalize,

@@ -348,3 +348,31 @@ def test_only_a_lone_sums_output_waits_for_the_norm_behind_its_branch():
         b = BranchStream(torch.full((2, 3), 9.0), ws)
         b.add_by(lambda x, factor, tanh_norm: x.add_(5.0), lambda *a: None, lambda x: True)
         assert torch.all(read(b, torch.empty(2, 3)) == 5.0)
+
+
+def _routed(monkeypatch, experts, hidden, top):
+    """A routed feed-forward whose kernels only say that they were called."""
+    from types import SimpleNamespace
+    from litinfer_amd.kernels import ops
+    from litinfer_amd.parts.moe import RoutedMLP
+    called = []
+    for name in ("moe_route", "moe_plan", "moe_linear"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, **kw: called.append((name, kw)))
+    monkeypatch.setattr(ops, "moe_tile_rows", lambda *a: 32)
+    part = RoutedMLP.__new__(RoutedMLP)
+    for k, v in dict(experts=experts, top=top, hidden=hidden, inter=96, w_up=torch.zeros(1, 192, 1), router=None, router_b=None, gate_row=None, scores="sigmoid",
+                     correction=None, groups=1, keep_groups=1, group_score="max", normalize=True, weigh_input=False, w_down=None, activation="swiglu",
+                     limit=0.0, shared_inter=0, identity=0, rt=SimpleNamespace(dtype=torch.float32)).items():
+        setattr(part, k, v)
+    ctx = SimpleNamespace(ws=SimpleNamespace(buffer=lambda name, shape, dt, zero=False: torch.zeros(shape, dtype=dt)))
+    return part, ctx, called
+
+
+@pytest.mark.parametrize("experts,top,tokens,together", [(16, 2, 1, True), (16, 2, 64, True), (16, 2, 65, False), (60, 10, 96, False), (64, 8, 128, False),
+                                                         (8, 2, 32, True), (8, 2, 48, False), (65, 2, 1, False)])
+def test_which_steps_have_the_plan_made_by_the_router(monkeypatch, experts, top, tokens, together):
+    from types import SimpleNamespace
+    part, ctx, called = _routed(monkeypatch, experts, 128, top)
+    part.forward(torch.zeros(tokens, 128), SimpleNamespace(add_by=lambda *a: None), ctx)
+    assert [n for n, _ in called] == ["moe_route"] + ([] if together else ["moe_plan"]) + ["moe_linear"] * 2
+    assert (called[0][1]["plan"] is not None) is together
