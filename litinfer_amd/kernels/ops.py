@@ -2190,6 +2190,18 @@ def moe_combine_takes_norms(x: torch.Tensor) -> bool:
     return x.is_cuda and x.is_contiguous() and bool(f(x.shape[0], x.shape[1]))
 
 
+def moe_combine_norm_pays(x: torch.Tensor, before: bool, top: int) -> bool:
+    """Whether it should take them: always with the norm in front (three launches become one, at worst 1.36 times as fast); with
+    the norm behind alone up to rows of 2,048, which one block's threads hold in two columns each.  Longer rows have the two launches'
+    more blocks against them: 8 tokens of 4,096, 1 / 2 / 4 / 6 / 8 / 10 choices, 0.80 / 0.81 / 0.88 / 0.92 / 0.97 / 0.71 times as fast, of 2,880
+    0.88 / 0.91 / 0.98 / 1.02 / 1.10 / 0.82; from 128 tokens on the sum alone fills the chip either way (0.97 to 1.47 with two choices and
+    more)."""
+    if not moe_combine_takes_norms(x):
+        return False
+    t, h = x.shape
+    return before or h <= 2048 or (t >= 128 and top > 1) or (h <= 3072 and 5 <= top <= 8)
+
+
 def moe_combine_norm(x: torch.Tensor, yrows: torch.Tensor, pair_row: torch.Tensor, wt: Optional[torch.Tensor], gate: Optional[torch.Tensor],
                      shared_out: Optional[torch.Tensor], idx: Optional[torch.Tensor] = None, experts: int = 0,
                      identity_rows: Optional[torch.Tensor] = None, top: int = 0, factor: float = 1.0, before=None, after=None,

@@ -183,7 +183,7 @@ class RoutedMLP(FeedForward):
         how = dict(idx=idx if self.identity else None, experts=self.experts, identity_rows=xn if self.identity else None, top=top)
         residual.add_by(lambda x, factor, tanh_norm: ops.moe_combine(x, *rows, factor=factor, tanh_norm=tanh_norm, **how),
                         lambda x, factor, before, after, out: ops.moe_combine_norm(x, *rows, factor=factor, before=before, after=after, rows=out, **how),
-                        ops.moe_combine_takes_norms)
+                        lambda x, before=True: ops.moe_combine_norm_pays(x, before, top))
 
 
 class RoutedReluSquaredMLP(RoutedMLP):

@@ -83,11 +83,11 @@ class ResidualStream:
         """For a sublayer whose own kernel adds into the stream: `add(x, factor, tanh_norm)` adds factor * (its output) to
         the float32 sum x and, where `tanh_norm` = (alpha, weight, bias, rows) is given, leaves that norm of the new sum in
         rows (the norm through which the stream is read next, if it is an elementwise one).  A sublayer whose kernel can take the RMS
-        norms on its two sides as well, where `takes_norms(x)`, gives `add_normed(x, factor, before, after, rows)`: the norm `before` =
+        norms on its two sides as well, where `takes_norms(x)` (`takes_norms(x, False)`: the one behind alone), gives `add_normed(x, factor, before, after, rows)`: the norm `before` =
         (weight, eps) of its output joins the sum, if there is one, and `rows` receives the norm `after` of the new sum, or the sum itself."""
         norm, self._scaled, self._normed = self.next_norm, None, None
         scaling = norm.as_scaling() if norm is not None else None
-        if scaling is not None and add_normed is not None and takes_norms(self.x):
+        if scaling is not None and add_normed is not None and takes_norms(self.x, False):
             rows = self.ws.buffer("stream.normed_rows", self.x.shape, self.ws_dtype)
             add_normed(self.x, self.factor, None, (scaling.weight, scaling.eps), rows)
             self._normed = (norm, rows)

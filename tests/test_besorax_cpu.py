@@ -376,3 +376,23 @@ def test_which_steps_have_the_plan_made_by_the_router(monkeypatch, experts, top,
     part.forward(torch.zeros(tokens, 128), SimpleNamespace(add_by=lambda *a: None), ctx)
     assert [n for n, _ in called] == ["moe_route"] + ([] if together else ["moe_plan"]) + ["moe_linear"] * 2
     assert (called[0][1]["plan"] is not None) is together
+
+
+@pytest.mark.parametrize("tokens,hidden,top,alone", [(1, 2048, 2, True), (8, 2048, 10, True), (8, 2049, 2, False), (8, 2880, 8, True), (8, 3073, 8, False),
+                                                     (64, 4096, 4, False), (127, 4096, 10, False), (128, 4096, 10, True), (128, 4096, 1, False)])
+def test_which_sums_of_experts_take_the_norm_behind_them(monkeypatch, tokens, hidden, top, alone):
+    """With a norm in front and one behind always; with the one behind alone where that is the faster."""
+    from types import SimpleNamespace
+    from litinfer_amd.kernels import ops
+    from litinfer_amd.parts.stream import BranchStream, ResidualStream
+    part, ctx, called = _routed(monkeypatch, 16, hidden, top)
+    monkeypatch.setattr(ops, "moe_combine_takes_norms", lambda x: True)
+    for name in ("moe_combine", "moe_combine_norm"):
+        monkeypatch.setattr(ops, name, lambda *a, name=name, **kw: called.append((name, kw)))
+    stream = ResidualStream(torch.zeros(tokens, hidden), ctx.ws)
+    stream.next_norm = SimpleNamespace(as_scaling=lambda: SimpleNamespace(weight=None, eps=1e-6), as_tanh=lambda: None)
+    part.forward(torch.zeros(tokens, hidden), stream, ctx)
+    assert called[-1][0] == ("moe_combine_norm" if alone else "moe_combine") and (stream._normed is not None) is alone
+    branch = BranchStream(torch.zeros(tokens, hidden), ctx.ws)
+    part.forward(torch.zeros(tokens, hidden), branch, ctx)
+    assert branch.take_waiting(stream.x) is not None
