@@ -852,9 +852,8 @@ __global__ __launch_bounds__(256) void gemm_bf16_big_kernel(const bf16_t* __rest
 // younger steps to stay outstanding waits exactly for the oldest step, and the
 // barrier after it makes that true for the loads of all four waves.
 // Needs K to be a multiple of the step (a load cannot be masked to zeros).  A step is 64
-// columns, so that a row of a stage is one whole 128-byte line of the caches.  Tiles of 64 rows, 128 x
-// 128, 192 x 128, 256 x 128 and (gated) 128 x 256 with two to four stages (what fits the 160 KB of LDS);
-// larger tiles are `gemm_bf16_tile_kernel`'s.
+// columns, so that a row of a stage is one whole 128-byte line of the caches.  Two to four stages (what fits the
+// 160 KB of LDS); which tiles are this kernel's and which `gemm_bf16_tile_kernel`'s: `tiling_of`, `gated_tiling_of`.
 #define LI_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x0F70)
 #define LI_LOAD_TO_LDS(gptr, lptr)                                                                        \
     __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gptr),              \
@@ -965,7 +964,7 @@ __device__ __forceinline__ void band_to_memory(const float* band, int row0, int 
     }
 }
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0, int WLM = 2>
 __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __restrict__ x,
                                                              const bf16_t* __restrict__ w,
                                                              const float* __restrict__ bias,
@@ -979,9 +978,13 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     // activation, which makes the result that of the RMS norm (the factor of a row does not depend on k).
     // nsplit > 1: a block multiplies one of nsplit parts of K, the y-th, and writes its sums to the y-th
     // [M, N] matrix behind `out` (float, no bias, no accumulation); splitk_reduce_kernel adds them
-    constexpr int WM = BM / 2, WN = BN / 2, TM = WM / 32, TN = WN / 32;
-    static_assert(WM % 32 == 0 && WN % 32 == 0, "a wave's part of the tile is made of 32 x 32 tiles");
+    // WLM: waves along the rows of the tile, 2 (two by two) or 4 (each wave 32-row bands over all columns:
+    // BN may then be any multiple of 32, for matrices whose columns no other tile divides into whole rounds)
+    constexpr int WLN = 4 / WLM;
+    constexpr int WM = BM / WLM, WN = BN / WLN, TM = WM / 32, TN = WN / 32;
+    static_assert(WM % 32 == 0 && WN % 32 == 0 && (WLM == 2 || WLM == 4), "a wave's part of the tile is made of 32 x 32 tiles");
     constexpr bool SWSPLIT = SWIGLU && (TN % 2 == 1);        // gates and ups in different waves (see the rows of w below)
+    static_assert(!SWSPLIT || WLN == 2, "gates in one wave, ups in the wave beside it");
     static_assert(BM % 32 == 0 && BN % 32 == 0 && (BM / 4) % (64 / (BK / 8)) == 0 && (BN / 4) % (64 / (BK / 8)) == 0, "whole load instructions a wave");
     constexpr int CPR = BK / 8, WRAP = 128 / BK;                 // chunks in a row; rows that fill all banks once
     constexpr int RPI = 64 / CPR;                                // rows one load instruction of a wave covers
@@ -990,7 +993,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     constexpr int LPW = IA + IB;                                 // loads a wave issues per step
     extern __shared__ __attribute__((aligned(16))) uint16_t lds[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * WM, wn = (wave & 1) * WN;
+    const int wm = (wave / WLN) * WM, wn = (wave % WLN) * WN;
     const int mtiles = (M + BM - 1) / BM, ntiles = (N + BN - 1) / BN;
     int mt, nt, split;
     if (!TileOrder(mtiles).tile(blockIdx.x, mtiles, ntiles, nsplit, mt, nt, split)) return;
@@ -1282,7 +1285,7 @@ __global__ __launch_bounds__(256) void gemm_bf16_dma_kernel(const bf16_t* __rest
     }
 }
 
-template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0>
+template <int BM, int BN, int BK, int NSTAGE, bool SWIGLU, typename TO, int ACT = 0, int WLM = 2>
 static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* out, int M, int N, int K,
                       float accumulate, hipStream_t stream, int nsplit = 1, const float* row_parts = nullptr,
                       int nparts = 0, float eps = 0.f, LiAct ep = {}) {
@@ -1298,12 +1301,12 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
     constexpr int lds_bytes = NSTAGE * (BM + BN) * BK * 2;
     static bool configured = false;
     if (!configured) {
-        if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, ACT>,
+        if (hipFuncSetAttribute((const void*)gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, ACT, WLM>,
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes) != hipSuccess)
             return LI_ERR_LAUNCH;
         configured = true;
     }
-    gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, ACT><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, nsplit, row_parts, nparts, eps, ep);
+    gemm_bf16_dma_kernel<BM, BN, BK, NSTAGE, SWIGLU, TO, ACT, WLM><<<(unsigned)blocks, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate, nsplit, row_parts, nparts, eps, ep);
     return li_launch_status();
 }
 
@@ -2334,38 +2337,55 @@ static double tile_cost(int bm, int bn, double speed, int M, int N, int K) {
 }
 
 // Tiles of more than 64 rows: the one with the least estimated time is taken, in microseconds: rounds of tiles over the compute
-// units (a last round that does not fill the chip counts for 0.3 less than a whole one: the units that run clock higher and
-// have the memory to themselves) x (steps of 64 k-values x `step_us`, and the tile's start and end: 95 ns for 1,024 results
-// and 29 for each byte of theirs that goes to memory or comes from there, of 1,024).  `step_us` as measured with the chip
-// full: tiles up to 128 x 288 and 192 x 192 take in 55 GB/s a compute unit whatever they multiply (what 256 lines of a unit's
-// cache, all on their way, bring at the latency of the lines that come from beyond the L2: the loads straight into LDS alone
-// take 130 GB/s where all of it lies there), the larger ones are bound by the MFMAs at the chip's power limit.
-// Fitted to 400 products, 80 to 6,000 rows x thirteen matrices of 896 to 7,168 rows of 896 to 27,648 and four gated ones up to
-// 55,296 rows: the tile that is taken is within 0.4 % of the best one on average, at worst 15 % (810 x 5,120 x 27,648).
-struct Tiling { int bm, bn; double step_us; };
-static double tile_us(const Tiling& t, int bytes, int M, int N, int K) {
+// units (a last round that does not fill the chip counts for less than a whole one: the units that run clock higher and have the memory
+// to themselves) x (steps of 64 k-values x `step_us`, and the tile's start and end: `ends_us` and `byte_us` for each byte of its results
+// that goes to memory or comes from there).  `pieces`: gemm_bf16_tile_kernel's, whose steps go two by two; the others are
+// gemm_bf16_dma_kernel's.  Where a step has few MFMAs, whole stages and one barrier a step are the faster form (128 x 128 x 3,584: 60 us
+// against 64 for 2,048 x 3,584 results; 128 x 192 of 4 waves one above the other 12 % before the same tile in pieces, gated, on average), and
+// so they are where K is a few steps (3,330 rows against 12,288 gated columns of 64: 26 us against 43); with more MFMAs and
+// steps the stage handed back in pieces (256 x 256, 8,192^3: 827 -> 726 us; 2,048 x 37,888 x 3,584 gated 483 -> 406).
+// All tiles up to 128 x 288 and 192 x 192 that were timed take in 55 GB/s a compute unit whatever they multiply (what 256 lines of a unit's
+// cache, all on their way, bring at the latency of the lines that come from beyond the L2: the loads straight into LDS alone take 130 GB/s
+// where all of it lies there); the larger ones are bound by the MFMAs at the chip's power limit.
+// The numbers are fitted to 804 products and 880 gated ones, 65 to 6,000 rows x 512 to 28,000 columns x 64 to 19,200, half of them layers'
+// matrices, each timed in every tile: what is taken is within 0.4 % of the best tile on average, and 1 % of them are more than 3 % behind
+// the best that any rule took before (at worst 20 %: 162 x 14,752 x 3,392, 2,501 x 2,176 x 384 gated).
+struct Tiling { int bm, bn; bool pieces; double step_us, ends_us; };
+struct Fit { double byte_us, rest; };        // rest: what a last round's idle units count for
+static double tile_us(const Tiling& t, const Fit& f, int bytes, int M, int N, int K) {
     const long tiles = (long)((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
     const int cu = compute_units();
     const double filled = (double)tiles / cu, whole = (double)((tiles + cu - 1) / cu);
-    return (filled + 0.7 * (whole - filled)) * (K / 64 * t.step_us + (double)t.bm * t.bn * (9.5e-5 + 2.85e-5 * bytes));
+    const int steps = t.pieces ? (K / 64 + 1) / 2 * 2 : K / 64;
+    return (filled + f.rest * (whole - filled)) * (steps * t.step_us + t.ends_us + (double)t.bm * t.bn * f.byte_us * bytes);
 }
 template <int COUNT>
-static int least_us(const Tiling (&shape)[COUNT], int bytes, int M, int N, int K) {
+static int least_us(const Tiling (&shape)[COUNT], const Fit& f, int bytes, int M, int N, int K) {
     int pick = 0;
     double best = 0.0;
     for (int i = 0; i < COUNT; ++i) {
-        const double c = tile_us(shape[i], bytes, M, N, K);
+        const double c = tile_us(shape[i], f, bytes, M, N, K);
         if (i == 0 || c < best) { best = c; pick = i; }
     }
     return pick;
 }
-// The first three are gemm_bf16_dma_kernel's, the others gemm_bf16_tile_kernel's: where a step has few MFMAs, whole stages and one
-// barrier a step are the faster form (128 x 128 x 3,584: 60 us against 64 for 2,048 x 3,584 results, 192 x 128 75 against 79),
-// with more of them the stage handed back in pieces (256 x 256, 8,192^3: 827 -> 726 us; 2,048 x 37,888 x 3,584 gated 483 -> 406).
-static int tiling_of(int M, int N, int K, int bytes) {
-    static const Tiling shape[7] = {{128, 128, 0.50}, {192, 128, 0.61}, {256, 128, 0.75}, {192, 224, 0.965}, {192, 256, 1.083},
-                                    {256, 224, 1.234}, {256, 256, 1.384}};
-    return least_us(shape, bytes, M, N, K);
+static const Tiling plain_tiles[9] = {{128, 128, false, 0.523, 1.48}, {192, 128, false, 0.630, 2.22}, {256, 128, false, 0.787, 2.61},
+                                      {128, 224, false, 0.801, 2.45}, {256, 256, false, 1.434, 3.58}, {192, 224, true, 0.993, 3.47},
+                                      {192, 256, true, 1.106, 3.40}, {256, 224, true, 1.223, 5.43}, {256, 256, true, 1.393, 4.33}};
+static int tiling_of(int M, int N, int K, int bytes) { return least_us(plain_tiles, Fit{2.884e-5, 0.617}, bytes, M, N, K); }
+// (a tile's columns are gate and up columns in turn.  Wide ones of 128 rows for steps of a few hundred rows or a few more than a multiple
+// of 256: 1,027 rows against the 1.5B's 17,920 columns are 504 tiles of 128 x 320, two rounds: 69 -> 58 us)
+static const Tiling gated_tiles[10] = {{128, 128, false, 0.584, 1.98}, {128, 256, false, 0.869, 2.32}, {128, 192, false, 0.648, 2.62},
+                                       {256, 128, false, 0.832, 3.80}, {256, 256, false, 1.478, 3.70}, {128, 320, true, 0.988, 3.12},
+                                       {192, 256, true, 1.096, 3.10}, {192, 320, true, 1.289, 4.67}, {256, 192, true, 1.075, 3.82},
+                                       {256, 256, true, 1.377, 4.09}};
+static int gated_tiling_of(int M, int N, int K) { return least_us(gated_tiles, Fit{2.051e-5, 0.748}, 1, M, N, K); }
+
+// The tile of a product of more than 64 rows, K a multiple of 64, that is not cut along K: rows x 65,536 + columns, negative in pieces.
+// `bytes` of a result that move (float32 8 where it is added to, else 4; bfloat16 2); gated: N is both halves' columns, bytes does not matter.
+extern "C" int li_linear_tile(int gated, int M, int N, int K, int bytes) {
+    const Tiling& t = gated ? gated_tiles[gated_tiling_of(M, N, K)] : plain_tiles[tiling_of(M, N, K, bytes)];
+    return (t.pieces ? -1 : 1) * (t.bm * 65536 + t.bn);
 }
 
 // More than 64 rows but so few 128 x 128 tiles that half of the compute units would idle (a narrow
@@ -2566,15 +2586,20 @@ extern "C" int li_linear(const void* x, const void* w, const float* bias, void* 
                 }
 #define LI_TILE(BM, BN, NS) (out_dtype == LI_F32 ? launch_tile<BM, BN, NS, false, float>((const bf16_t*)x, (const bf16_t*)w, bias, (float*)out, M, N, K, accumulate, stream) \
                                         : launch_tile<BM, BN, NS, false, bf16_t>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, accumulate, stream))
+#define LI_DMA4(BM, BN, NS) (out_dtype == LI_F32 ? launch_dma<BM, BN, 64, NS, false, float, 0, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (float*)out, M, N, K, accumulate, stream) \
+                                        : launch_dma<BM, BN, 64, NS, false, bf16_t, 0, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, accumulate, stream))
                 switch (tiling_of(M, N, K, out_dtype == LI_BF16 ? 2 : accumulate != 0.f ? 8 : 4)) {
                 case 0: return LI_DMA(128, 128, 64, 4);
                 case 1: return LI_DMA(192, 128, 64, 3);
                 case 2: return LI_DMA(256, 128, 64, 3);
-                case 3: return LI_TILE(192, 224, 2);
-                case 4: return LI_TILE(192, 256, 2);
-                case 5: return LI_TILE(256, 224, 2);
+                case 3: return LI_DMA4(128, 224, 3);
+                case 4: return LI_DMA(256, 256, 64, 2);
+                case 5: return LI_TILE(192, 224, 2);
+                case 6: return LI_TILE(192, 256, 2);
+                case 7: return LI_TILE(256, 224, 2);
                 default: return LI_TILE(256, 256, 2);
                 }
+#undef LI_DMA4
 #undef LI_TILE
             }
 #undef LI_DMA
@@ -2637,6 +2662,7 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
         return li_launch_status();
     }
 #define LI_ACT(BM, BN, NS) launch_dma<BM, BN, 64, NS, false, bf16_t, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
+#define LI_ACT4(BM, BN, NS) launch_dma<BM, BN, 64, NS, false, bf16_t, LI_ACT_RELU2, 4>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)
 #define LI_ACT_TILE(BM, BN, NS) launch_tile<BM, BN, NS, false, bf16_t, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, ep)
     if (M <= 64) {                                   // (as linear_mid_rows takes them)
         if ((N + 255) / 256 >= 128) return LI_ACT(64, 256, 3);
@@ -2647,12 +2673,15 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
     case 0: return LI_ACT(128, 128, 4);
     case 1: return LI_ACT(192, 128, 3);
     case 2: return LI_ACT(256, 128, 3);
-    case 3: return LI_ACT_TILE(192, 224, 2);
-    case 4: return LI_ACT_TILE(192, 256, 2);
-    case 5: return LI_ACT_TILE(256, 224, 2);
+    case 3: return LI_ACT4(128, 224, 3);
+    case 4: return LI_ACT(256, 256, 2);
+    case 5: return LI_ACT_TILE(192, 224, 2);
+    case 6: return LI_ACT_TILE(192, 256, 2);
+    case 7: return LI_ACT_TILE(256, 224, 2);
     default: return LI_ACT_TILE(256, 256, 2);
     }
 #undef LI_ACT_TILE
+#undef LI_ACT4
 #undef LI_ACT
 }
 
@@ -2733,24 +2762,20 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
     if (M <= 64) return li_linear_skinny(x, w, nullptr, out, M, I, K, LI_BF16, 0, 1, stream);
     if (K % 64) return LI_ERR_SIZE;
 #define LI_GATED(LAUNCH, ...) LAUNCH((const bf16_t*)x, (const bf16_t*)w, nullptr, (bf16_t*)out, M, N, K, 0.f, stream, __VA_ARGS__)
-#define LI_DMA_AS(BM, BN, NS, ACT) LI_GATED((launch_dma<BM, BN, 64, NS, true, bf16_t, ACT>), 1, nullptr, 0, 0.f, ep)
-#define LI_DMA(BM, BN, NS) (act == LI_ACT_CLAMPED ? LI_DMA_AS(BM, BN, NS, LI_ACT_CLAMPED) : act ? LI_DMA_AS(BM, BN, NS, LI_ACT_GELU_TANH) : LI_DMA_AS(BM, BN, NS, 0))
+#define LI_DMA_AS(BM, BN, NS, WLM, ACT) LI_GATED((launch_dma<BM, BN, 64, NS, true, bf16_t, ACT, WLM>), 1, nullptr, 0, 0.f, ep)
+#define LI_DMA(BM, BN, NS, WLM) (act == LI_ACT_CLAMPED ? LI_DMA_AS(BM, BN, NS, WLM, LI_ACT_CLAMPED) : act ? LI_DMA_AS(BM, BN, NS, WLM, LI_ACT_GELU_TANH) : LI_DMA_AS(BM, BN, NS, WLM, 0))
 #define LI_TILE_AS(BM, BN, NS, ACT) LI_GATED((launch_tile<BM, BN, NS, true, bf16_t, ACT>), ep)
 #define LI_TILE(BM, BN, NS) (act == LI_ACT_CLAMPED ? LI_TILE_AS(BM, BN, NS, LI_ACT_CLAMPED) : act ? LI_TILE_AS(BM, BN, NS, LI_ACT_GELU_TANH) : LI_TILE_AS(BM, BN, NS, 0))
-    // (the first two are gemm_bf16_dma_kernel's, see tiling_of; a tile's columns are gate and up columns in turn.  Wide ones of
-    // 128 rows for steps of a few hundred rows or a few more than a multiple of 256: 1,027 rows against the 1.5B's 17,920 columns
-    // are 504 tiles of 128 x 320, two rounds: 69 -> 58 us)
-    static const Tiling shape[9] = {{128, 128, 0.551}, {128, 256, 0.885}, {128, 192, 0.70}, {128, 320, 1.036}, {128, 384, 1.214},
-                                    {192, 256, 1.087}, {192, 320, 1.314}, {256, 192, 1.075}, {256, 256, 1.378}};
-    switch (least_us(shape, 1, M, N, K)) {
-    case 0: return LI_DMA(128, 128, 4);
-    case 1: return LI_DMA(128, 256, 3);
-    case 2: return LI_TILE(128, 192, 4);
-    case 3: return LI_TILE(128, 320, 2);
-    case 4: return LI_TILE(128, 384, 2);
-    case 5: return LI_TILE(192, 256, 2);
-    case 6: return LI_TILE(192, 320, 2);
-    case 7: return LI_TILE(256, 192, 2);
+    switch (gated_tiling_of(M, N, K)) {
+    case 0: return LI_DMA(128, 128, 4, 2);
+    case 1: return LI_DMA(128, 256, 3, 2);
+    case 2: return LI_DMA(128, 192, 3, 4);
+    case 3: return LI_DMA(256, 128, 3, 2);
+    case 4: return LI_DMA(256, 256, 2, 2);
+    case 5: return LI_TILE(128, 320, 2);
+    case 6: return LI_TILE(192, 256, 2);
+    case 7: return LI_TILE(192, 320, 2);
+    case 8: return LI_TILE(256, 192, 2);
     default: return LI_TILE(256, 256, 2);
     }
 #undef LI_TILE

@@ -1,6 +1,7 @@
 """Host-side bounds that keep kernels inside their tables, checked against the kernels'
 own arithmetic redone in Python."""
 import numpy as np
+import pytest
 
 from litinfer_amd.kernels import ops
 
@@ -127,3 +128,19 @@ def test_groups_of_keys_of_the_32_bit_prompt_attention():
     assert [f(8, 40, 8, 64, keys) for keys in (32, 64)] == [4, 1]                       # two blocks of 64 columns share a unit
     assert [f(13, 28, 4, 128, 400), f(32, 28, 4, 128, 1000), f(63, 28, 4, 128, 2000)] == [2, 3, 4]
     assert f(13, 28, 4, 128, 20) == f(32, 28, 4, 128, 20) == 4
+
+
+@pytest.mark.parametrize("gated,m,n,k,result_bytes,tile", [
+    # wide matrices of a few hundred rows (97 -> 128 us without these tiles, 48 -> 61), narrow gated ones (148 -> 169)
+    (0, 257, 17472, 8000, 2, (128, 224, False)), (0, 380, 18944, 3584, 2, (128, 224, False)), (1, 2012, 2304, 896, 1, (128, 192, False)),
+    (1, 1699, 2688, 16768, 1, (128, 192, False)),
+    # a single step of 64 k-values, which a tile in pieces doubles (26 -> 43)
+    (1, 3330, 12288, 64, 1, (256, 256, False)),
+    # the layers' products of a prompt
+    (1, 2048, 37888, 3584, 1, (256, 256, True)), (0, 8192, 8192, 8192, 8, (256, 256, True)),
+])
+def test_tiles_of_products(gated, m, n, k, result_bytes, tile):
+    import ctypes
+    f = ops._lib_fn("gemm", "li_linear_tile", [ctypes.c_int] * 5, ctypes.c_int)
+    got = f(gated, m, n, k, result_bytes)
+    assert (abs(got) >> 16, abs(got) & 65535, got < 0) == tile

@@ -74,8 +74,8 @@ def test_rmsnorm_zero_row_is_zero_not_nan(ops):
     ((1, 1000, 3584), True, False), ((16, 70, 260), True, True), ((40, 19, 100), False, True),      # few rows in 32-bit
     ((9, 18, 4), True, False),
     ((300, 200, 130), True, True), ((256, 128, 64), False, False), ((1000, 333, 1027), True, False),     # the large 32-bit tile
-    ((2048, 3584, 128), True, True), ((2000, 4600, 64), True, False),           # tiles of 256 x 128 and 256 x 256, ragged
-    ((1100, 4600, 128), True, True), ((1167, 6627, 128), False, False),         # tiles of 192 and more: a last row of tiles with few rows
+    ((2048, 3584, 128), True, True), ((2000, 4600, 64), True, False),           # large tiles, ragged
+    ((1100, 4600, 128), True, True), ((1167, 6627, 128), False, False),         # a last row of tiles with few rows
     ((585, 3979, 128), True, False), ((779, 6296, 128), False, True)])          # columns that few tiles divide
 def test_linear(ops, dtype, mnk, bias, acc):
     m, n, k = mnk
@@ -96,19 +96,57 @@ def test_linear(ops, dtype, mnk, bias, acc):
     assert rel(out, ref) < (4 * math.sqrt(k) * 2.0 ** -24 if out.dtype is torch.float32 else 5e-3)
 
 
-# Tiles whose stages are handed back in pieces (gemm_bf16_tile_kernel), each one by its sizes: rows and columns past the last, widths
-# that no 16-byte piece divides, and one, an odd number and an even number of steps of 64 k-values.
+# Tiles of many rows: rows and columns past the last, widths that no 16-byte piece divides, and one, an odd number and an even number of
+# steps of 64 k-values (which tile each takes, and every tile in its steady state: test_every_tile_of_a_product).
 @pytest.mark.parametrize("m,n,k,form", [
-    (129, 32771, 64, "residual"), (129, 32776, 192, "bf16"), (769, 20488, 256, "relu2"),               # 192 x 224
-    (641, 14344, 64, "residual"), (385, 20491, 320, "residual"), (705, 14341, 64, "bf16"), (385, 20488, 192, "relu2"),     # 192 x 256
-    (385, 24584, 192, "residual"), (193, 32776, 320, "bf16"), (385, 24589, 128, "residual"),           # 256 x 224
-    (769, 14344, 192, "residual"), (1537, 8200, 448, "residual"),                                      # 256 x 256
-    (129, 8203, 64, "gated"), (130, 8200, 192, "gelu_gate"),                                           # 128 x 192
-    (129, 16388, 320, "gated"), (257, 16388, 64, "clamped"), (300, 16385, 128, "gated"),               # 128 x 320, 192 x 320
-    (385, 10244, 192, "gated"), (385, 10241, 64, "gelu_gate"),                                         # 256 x 192
-    (513, 8200, 320, "gated"), (577, 8200, 64, "gated"), (577, 8203, 192, "clamped"),                  # 192 x 256, 128 x 384
-    (641, 10244, 64, "gelu_gate"), (577, 10241, 192, "gated"), (600, 10244, 448, "clamped")])          # 256 x 256
+    (129, 32771, 64, "residual"), (129, 32776, 192, "bf16"), (769, 20488, 256, "relu2"),
+    (641, 14344, 64, "residual"), (385, 20491, 320, "residual"), (705, 14341, 64, "bf16"), (385, 20488, 192, "relu2"),
+    (385, 24584, 192, "residual"), (193, 32776, 320, "bf16"), (385, 24589, 128, "residual"),
+    (769, 14344, 192, "residual"), (1537, 8200, 448, "residual"),
+    (129, 8203, 64, "gated"), (130, 8200, 192, "gelu_gate"),
+    (129, 16388, 320, "gated"), (257, 16388, 64, "clamped"), (300, 16385, 128, "gated"),
+    (385, 10244, 192, "gated"), (385, 10241, 64, "gelu_gate"),
+    (513, 8200, 320, "gated"), (577, 8200, 64, "gated"), (577, 8203, 192, "clamped"),
+    (641, 10244, 64, "gelu_gate"), (577, 10241, 192, "gated"), (600, 10244, 448, "clamped")])
 def test_linear_in_large_tiles(ops, m, n, k, form):
+    _product_is_right(ops, m, n, k, form)
+
+
+# Every tile of more than 64 rows that `tiling_of` and `gated_tiling_of` know, with each of its epilogues: more steps of 64 k-values than
+# stages, an odd and an even number of them (so that stages are filled again while the loop runs, and the step of zeros behind an odd number
+# takes the place of one that was in use), ragged both ways.  "pieces": stages handed back in pieces (gemm_bf16_tile_kernel).
+@pytest.mark.parametrize("bm,bn,how,m,n,k,form", [
+    (128, 128, "whole", 129, 8067, 448, "bf16"),
+    (192, 128, "whole", 129, 16387, 320, "residual"), (192, 128, "whole", 129, 16392, 448, "relu2"),
+    (256, 128, "whole", 385, 14339, 320, "residual"), (256, 128, "whole", 193, 16387, 512, "bf16"),
+    (128, 224, "whole", 193, 16387, 320, "residual"), (128, 224, "whole", 257, 16387, 512, "bf16"), (128, 224, "whole", 257, 16392, 448, "relu2"),
+    (256, 256, "whole", 641, 16387, 320, "residual"), (256, 256, "whole", 577, 16387, 384, "bf16"), (256, 256, "whole", 577, 16392, 448, "relu2"),
+    (192, 224, "pieces", 385, 16387, 320, "residual"), (192, 224, "pieces", 257, 19075, 384, "bf16"), (192, 224, "pieces", 385, 16392, 448, "relu2"),
+    (192, 256, "pieces", 385, 19075, 384, "residual"), (192, 256, "pieces", 577, 14339, 320, "bf16"), (192, 256, "pieces", 385, 19080, 448, "relu2"),
+    (256, 224, "pieces", 641, 16387, 384, "residual"), (256, 224, "pieces", 385, 21763, 832, "residual"),
+    (256, 224, "pieces", 577, 16387, 768, "bf16"), (256, 224, "pieces", 385, 21768, 1216, "relu2"),
+    (256, 256, "pieces", 577, 19075, 1536, "residual"), (256, 256, "pieces", 577, 19075, 3520, "bf16"), (256, 256, "pieces", 577, 19080, 1536, "relu2"),
+    (128, 128, "gated", 300, 1003, 448, "clamped"),
+    (128, 192, "gated", 129, 8195, 320, "gated"), (128, 192, "gated", 130, 8195, 384, "gelu_gate"), (128, 192, "gated", 129, 8200, 448, "clamped"),
+    (128, 256, "gated", 257, 8195, 320, "gated"), (128, 256, "gated", 257, 8195, 384, "gelu_gate"), (128, 256, "gated", 257, 8200, 448, "clamped"),
+    (256, 128, "gated", 641, 5379, 320, "gated"), (256, 128, "gated", 641, 5379, 512, "gelu_gate"), (256, 128, "gated", 641, 5384, 448, "clamped"),
+    (256, 256, "gated", 641, 8195, 320, "gated"), (256, 256, "gated", 385, 9283, 64, "gelu_gate"), (256, 256, "gated", 641, 8200, 448, "clamped"),
+    (128, 320, "gated pieces", 385, 8195, 320, "gated"), (128, 320, "gated pieces", 385, 8195, 384, "gelu_gate"), (128, 320, "gated pieces", 385, 8200, 448, "clamped"),
+    (192, 256, "gated pieces", 513, 8195, 320, "gated"), (192, 256, "gated pieces", 513, 8195, 384, "gelu_gate"), (192, 256, "gated pieces", 513, 8200, 448, "clamped"),
+    (192, 320, "gated pieces", 769, 6531, 384, "gated"), (192, 320, "gated pieces", 1025, 6531, 320, "gelu_gate"), (192, 320, "gated pieces", 1025, 6536, 448, "clamped"),
+    (256, 192, "gated pieces", 385, 10883, 320, "gated"), (256, 192, "gated pieces", 385, 10883, 384, "gelu_gate"), (256, 192, "gated pieces", 385, 10888, 448, "clamped"),
+    (256, 256, "gated pieces", 577, 8195, 384, "gated"), (256, 256, "gated pieces", 1537, 4483, 1600, "gelu_gate"), (256, 256, "gated pieces", 577, 8200, 512, "clamped")])
+def test_every_tile_of_a_product(ops, bm, bn, how, m, n, k, form):
+    import ctypes
+    gated = how.startswith("gated")
+    tile = ops._lib_fn("gemm", "li_linear_tile", [ctypes.c_int] * 5, ctypes.c_int)
+    units = torch.cuda.get_device_properties(0).multi_processor_count
+    if units == 256:                                          # (the sizes are for that many)
+        assert tile(int(gated), m, 2 * n if gated else n, k, 8 if form == "residual" else 2) == (-1 if "pieces" in how else 1) * (bm * 65536 + bn)
+    _product_is_right(ops, m, n, k, form)
+
+
+def _product_is_right(ops, m, n, k, form):
     g = torch.Generator(device=DEV).manual_seed(91)
     gated = form in ("gated", "gelu_gate", "clamped")
     x = torch.randn(m, k, generator=g, device=DEV).bfloat16()
@@ -344,13 +382,13 @@ def test_linear_into_the_residual_sum_with_its_norm(ops, m, n, k, bias, taken):
     (65, 32, 64),                # one tile, one step of K
     (100, 200, 128),             # an output width that is no multiple of 32
     (300, 1000, 192),            # several tiles both ways, ragged edges
-    (700, 4700, 256),            # tiles of 256 x 128
+    (700, 4700, 256),            # (which tiles the larger ones take, and every tile there is: test_every_tile_of_a_product)
     (2048, 18944, 128),          # enough tiles for the largest tiling
-    (97, 7419, 128),             # few rows against many columns: tiles of 128 x 192
-    (300, 9001, 128),            # tiles of 128 x 256
-    (1101, 2500, 192),           # nine rows of tiles: the last XCD's share of the tiles is short
-    (1024, 4800, 192),           # tiles of 128 x 320
-    (2000, 4793, 192),           # the same with ragged edges both ways
+    (97, 7419, 128),             # few rows against many columns
+    (300, 9001, 128),
+    (1101, 2500, 192),           # several rows of tiles: the last XCD's share of the tiles is short
+    (1024, 4800, 192),
+    (2000, 4793, 192),           # ragged edges both ways
 ])
 def test_linear_with_swiglu_epilogue(ops, m, n, k):
     g = torch.Generator().manual_seed(14)
