@@ -13,6 +13,7 @@ from __future__ import annotations
 import ctypes
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -20,7 +21,7 @@ import tempfile
 import threading
 import time
 from pathlib import Path
-from typing import Dict, List, Optional
+from typing import Callable, Dict, List, Optional
 
 CSRC = Path(__file__).resolve().parent.parent / "csrc"
 ARCH = "gfx950"
@@ -123,15 +124,68 @@ def find_built(module: str) -> Optional[Path]:
     return None
 
 
+def tile_kernel_faults(assembly: str) -> List[str]:
+    """What is wrong with the instances of `gemm_bf16_tile_kernel` in the compiler's assembly (nothing, normally).  Their MFMAs are
+    inline assembly, so the compiler does not wait for a sum before it moves or spills one: that is sound only while it does
+    neither between the first MFMA and the two waits of 16 cycles behind the last, and while no MFMA's operand is written by the vector
+    ALU right before it.  A build for which that does not hold would compute wrong sums without an error."""
+    faults, name, body = [], None, []
+    for line in assembly.split("\n"):
+        head = re.match(r"(_Z\S*gemm_bf16_tile_kernel\S*):", line)
+        if head:
+            name, body = head[1], []
+        elif name is not None:
+            body.append(line.split(";")[0].strip())
+            if ".end_amdhsa_kernel" in line:
+                faults += [f"{name}: {f}" for f in _tile_body_faults(body)]
+                name = None
+    if name is not None or "gemm_bf16_tile_kernel" not in assembly:
+        faults.append("no whole instance of gemm_bf16_tile_kernel in the assembly")
+    return faults
+
+
+def _tile_body_faults(body: List[str]) -> List[str]:
+    def registers(operand: str, kind: str):
+        m = re.fullmatch(kind + r"(?:(\d+)|\[(\d+):(\d+)\])", operand)
+        return set() if not m else {int(m[1])} if m[1] else set(range(int(m[2]), int(m[3]) + 1))
+
+    code = [x for x in body if x and not x.startswith((".", ";")) and not x.endswith(":")]
+    mfma = [i for i, x in enumerate(code) if x.startswith("v_mfma")]
+    if not mfma:
+        return ["no MFMA"]
+    out = []
+    if not any(x.split()[-1] == "0" for x in body if x.startswith(".amdhsa_private_segment_fixed_size")) or any("scratch_" in x for x in code):
+        out.append("registers spilled to scratch")
+    waits = [i for i in range(mfma[-1], len(code) - 1) if code[i] == code[i + 1] == "s_nop 15"]
+    if not waits:
+        return out + ["no wait behind the last MFMA"]
+    for i in range(mfma[0], waits[0]):
+        if not code[i].startswith("v_mfma") and re.search(r"\ba(?:\d+|\[\d+:\d+\])", code[i]):
+            out.append(f"a sum moves while MFMAs may be in flight: {code[i]}")
+        elif code[i].startswith("v_") and not code[i].startswith("v_mfma"):
+            written = registers(code[i].split(None, 1)[1].split(",")[0].strip(), "v") if " " in code[i] or "\t" in code[i] else set()
+            for x in code[i + 1:i + 5]:
+                if x.startswith("v_mfma") and any(written & registers(o.strip(), "v") for o in x.split(None, 1)[1].split(",")[1:3]):
+                    out.append(f"an operand written right before its MFMA: {code[i]}")
+    return out
+
+
+# module -> what is wrong with its assembly
+CHECKS: Dict[str, Callable[[str], List[str]]] = {"gemm": tile_kernel_faults}
+
+
 def compile_module(module: str, verbose: bool = True) -> Path:
-    """Compile the module's source under csrc/ now, whether or not a build exists."""
+    """Compile the module's source under csrc/ now, whether or not a build exists.  A module with a check of its assembly
+    is refused if the check finds anything."""
     src = _source(module)
     if not src.exists():
         raise KernelBuildError(f"no source {src}")
     out_dir = _writable_dir()
     out = out_dir / lib_name(module)
     tmp = out_dir / f".{out.name}.{os.getpid()}.tmp"
-    cmd = [_hipcc(), *_flags(module), f"-I{CSRC}", str(src), "-o", str(tmp)]
+    keep = Path(tempfile.mkdtemp(prefix=f"li_{module}-")) if module in CHECKS else None      # (the assembly, beside what is built)
+    target = tmp if keep is None else keep / out.name
+    cmd = [_hipcc(), *_flags(module), f"-I{CSRC}", *([] if keep is None else ["-save-temps=obj"]), str(src), "-o", str(target)]
     env = dict(os.environ)
     env.setdefault("HOME", tempfile.gettempdir())     # hipcc wants a HOME it can look into
     t0 = time.time()
@@ -146,9 +200,21 @@ def compile_module(module: str, verbose: bool = True) -> Path:
             if verbose:
                 print(f"[litinfer_amd]   ... still compiling {src.name} "
                       f"({time.time() - t0:.0f} s)", file=sys.stderr, flush=True)
-    if proc.returncode != 0:
+    try:
+        if proc.returncode != 0:
+            raise KernelBuildError(f"hipcc failed on {src.name}:\n{log}")
+        if keep is not None:
+            faults = [f for a in keep.glob(f"*{ARCH}*.s") for f in CHECKS[module](a.read_text())] if any(keep.glob(f"*{ARCH}*.s")) else ["no assembly to check"]
+            if faults:
+                raise KernelBuildError(f"{src.name}: this compiler's code is not sound:\n" + "\n".join(faults[:20]))
+            shutil.copyfile(target, tmp)
+            shutil.copymode(target, tmp)
+    except BaseException:
         tmp.unlink(missing_ok=True)
-        raise KernelBuildError(f"hipcc failed on {src.name}:\n{log}")
+        raise
+    finally:
+        if keep is not None:
+            shutil.rmtree(keep, ignore_errors=True)
     os.replace(tmp, out)
     for old in out_dir.glob(f"li_{module}-*.so"):
         if old != out:
