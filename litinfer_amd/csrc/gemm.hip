@@ -1379,15 +1379,18 @@ static int launch_dma(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
 //     1           (0, Y)        A half 1                B half X         then a barrier
 //     2           (1, Y)        A half 0, next step     B half Y
 //     3           (1, X)        B half Y, next step     A half 1         then a barrier
-// Half of the stage has been read at each barrier and its place is asked for again at once, so a load has two
-// barriers more than NSTAGE - 1 steps to arrive, the loads are spread evenly over the whole step, and no register
-// holds an operand twice: 128 registers of operands beside the 256 of the sums.
+// Half of the stage has been read at each barrier and its place is asked for again at once: the loads are spread evenly over the
+// whole step, and no register holds an operand twice: 128 registers of operands beside the 256 of the sums.  What step kt
+// asks for is step kt + NSTAGE's.  Of that, A half 0 and the B half that is multiplied first are waited for in the middle of step
+// kt + NSTAGE - 1, the rest at its end.  So A half 0 and, with an even number of stages, B half X have NSTAGE - 1 steps and up to half a
+// step more to arrive, B half Y the same from the middle on, A half 1 NSTAGE - 1 steps and the rest of its quarter.
 // Multiplied by v_mfma_f32_16x16x32_bf16: with operands as they are in use the chip is at its power limit here, and this
 // form draws less for the same product than the 32 x 32 x 16 one (a loop of nothing else 1.90 against 1.75 PFLOP/s).
 // The MFMAs are assembly so that a sum stays in its registers: the instruction's result may lie elsewhere, and the compiler
 // made use of that, with some 600 moves between registers a step and spills.  What it then does not see is seen to
 // here: operands come from LDS reads alone, which it waits for as for any use; the same sum comes up again after four
-// MFMAs at least; and before the sums are read behind the loop, two waits of 16 cycles pass.
+// MFMAs at least; and before the sums are read behind the loop, two waits of 16 cycles pass.  The build looks the assembly
+// of every instance through and refuses one in which a sum is moved or spilled before that.
 // A half's rows of a stage: first those of the waves of the first row (column) of waves, then the others'.
 // ... by the lanes that are told: all, or none (a step past the last asks for nothing, but counts as the others do)
 #define LI_LOAD_TO_LDS_BY(lanes, base, voff, lptr)                                                       \
