@@ -132,24 +132,37 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
     }
     for (int k = threadIdx.x; k < K; k += NT) xs[k] = load_as_float(row + k);
     __syncthreads();
-    for (int e = w, q = 0; e < n_rows; e += NT / 64, ++q) {
-        const TW* wrow = e < E ? wr + (size_t)e * K : wg;
-        float s = 0.f;
-        if (held && q < 2) {
-#pragma unroll
-            for (int i = 0; i < HELD; ++i)
-                if (lane + 64 * i < K / VE) s += route_dot16(q ? piece[1][i] : piece[0][i], xs + (lane + 64 * i) * VE, (const TW*)nullptr);
-        } else if (vec) {                              // 16 bytes a lane and turn, several turns on their way
-#pragma unroll 4
-            for (int i = lane; i < K / VE; i += 64) s += route_dot16(*reinterpret_cast<const uint4*>(wrow + (size_t)i * VE), xs + i * VE, (const TW*)nullptr);
-        } else {
-            for (int k = lane; k < K; k += 64) s = fmaf(load_as_float(wrow + k), xs[k], s);
-        }
+    auto have = [&](int e, float s) {                  // a row's product, in parts by lane
         s = wave_sum(s);
         if (lane == 0) {
             if (e < E) lg[e] = s + (br ? br[e] : 0.f);
             else gate[t] = 1.0f / (1.0f + expf(-s));
         }
+    };
+    int e = w;
+    if constexpr (NT == 1024) {                        // (rows of their own: asked for in the loop below, they made every other row 0.2 us longer)
+        if (held) {
+#pragma unroll
+            for (int q = 0; q < 2; ++q, e += NT / 64) {
+                if (e >= n_rows) break;
+                float s = 0.f;
+#pragma unroll
+                for (int i = 0; i < HELD; ++i)
+                    if (lane + 64 * i < K / VE) s += route_dot16(piece[q][i], xs + (lane + 64 * i) * VE, (const TW*)nullptr);
+                have(e, s);
+            }
+        }
+    }
+    for (; e < n_rows; e += NT / 64) {
+        const TW* wrow = e < E ? wr + (size_t)e * K : wg;
+        float s = 0.f;
+        if (vec) {                                     // 16 bytes a lane and turn, several turns on their way
+#pragma unroll 4
+            for (int i = lane; i < K / VE; i += 64) s += route_dot16(*reinterpret_cast<const uint4*>(wrow + (size_t)i * VE), xs + i * VE, (const TW*)nullptr);
+        } else {
+            for (int k = lane; k < K; k += 64) s = fmaf(load_as_float(wrow + k), xs[k], s);
+        }
+        have(e, s);
     }
     __syncthreads();
     if (w != 0) return;
