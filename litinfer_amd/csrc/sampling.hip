@@ -536,7 +536,7 @@ __device__ __forceinline__ int ties_needed(float remaining, uint32_t tp, float m
 // With top-k <= SMP_KC the candidates hold all survivors (kc = k).  With top-p alone kc = SMP_KC_P
 // and the second kernel checks that the prefix ends above the kc-th largest id of the row, whose
 // betters are all among the candidates; otherwise it reads the row.  0: no candidates.
-constexpr int SMP_KC = 256, SMP_KC_P = 128, SMP_CAND_PER_THREAD = 8;        // (SMP_KC <= 16 * LI_WAVE and 8 keys a thread: select_kth)
+constexpr int SMP_KC = 256, SMP_KC_P = 128, SMP_CAND_PER_THREAD = 8, SMP_WIDE_TILES = 512;        // (SMP_KC <= 16 * LI_WAVE and 8 keys a thread: select_kth)
 __device__ __forceinline__ int sample_candidates(int k, float p, int V, int ntiles) {
     if (sample_unfiltered(k, p, V)) return 0;
     const int kc = (k > 0 && k < V) ? k : SMP_KC_P;
@@ -544,8 +544,12 @@ __device__ __forceinline__ int sample_candidates(int k, float p, int V, int ntil
 }
 
 // Do SMP_KC candidates of every tile fit the second kernel's registers?  Then a tile may hand over more than kc of them: all that
-// are no smaller than a bound (tile_i: how many).
-__device__ __forceinline__ bool sample_wide(int ntiles) { return ntiles * SMP_KC <= SMP_NT * SMP_CAND_PER_THREAD; }
+// are no smaller than a bound (tile_i: how many).  With top-p alone the second kernel goes through all candidates pass after pass, and
+// twice as many cost more than the tiles save unless these are many (p 0.9, exactly kc / all from the bound: one row of 151,936 ids 52 / 57.5
+// us, 16 62 / 68, 64 92 / 87, 256 219 / 177; 64 of 32,000 51 / 53, 256 78 / 77).
+__device__ __forceinline__ bool sample_wide(int k, int V, int rows, int ntiles) {
+    return ntiles * SMP_KC <= SMP_NT * SMP_CAND_PER_THREAD && ((k > 0 && k < V) || rows * ntiles > SMP_WIDE_TILES);
+}
 
 // (eight waves a SIMD, two blocks a compute unit: with the 71 registers that the compiler would take, one block, 64 greedy rows took
 // 18 us instead of 13)
@@ -599,7 +603,7 @@ __global__ __launch_bounds__(SMP_NT, 8) void sample_tiles_kernel(
         uint32_t key[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) key[e] = j0 + e < V ? sort_key(z[e]) : 0u;
-        const bool wide = sample_wide(ntiles);
+        const bool wide = sample_wide(k, V, gridDim.y, ntiles);
         const uint32_t bound = bound_of_kth(key, kc, max(in_tile / (8 * LI_WAVE), 1), work_i);
         bool found = false;
         if (bound != 0u) {
@@ -704,7 +708,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
         bool have[SMP_CAND_PER_THREAD];
         const int lane = tid & (LI_WAVE - 1);
         int total, first = 0;                       // candidates in all; those of the tiles before tile `lane` (where the tiles hold different numbers)
-        const bool wide = sample_wide(ntiles);
+        const bool wide = sample_wide(k, V, gridDim.x, ntiles);
         if (wide) {                                 // (up to 32 tiles: a lane each)
             const int count = lane < ntiles ? tile_i[lane] : 0;
             int upto = count;

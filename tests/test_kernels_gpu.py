@@ -1758,3 +1758,22 @@ def test_the_profiler_sees_products_that_may_not_be_taken(ops, monkeypatch):
     assert ops.linear_tanh_norm(bf16(m, k), bf16(n, k), None, rows, 0.5, torch.ones(n, device=DEV), torch.zeros(n, device=DEV), xn, _Lender())
     assert dict(prof.calls) == {("decode", name): 1 for name in ("linear_act", "linear_then_norm", "linear_tanh_norm")}
     assert all(v > 0 for v in prof.total.values())
+
+
+@pytest.mark.parametrize("vocab", [5 * 8192 + 3, 32 * 8192])
+def test_top_p_alone_hands_over_exactly_its_candidates_or_all_above_a_bound(ops, vocab):
+    # the latter from 513 tiles of rows on; the same rows in a step of few and in one of many, a prefix within the candidates and one
+    # beyond them (flat rows), ties at the threshold
+    few, many = 8, -(-513 // -(-vocab // 8192))
+    g = torch.Generator().manual_seed(71)
+    logits = torch.randn(many, vocab, generator=g) * 6
+    logits[1] *= 0.1
+    logits[2] = (logits[2] * 2).round() / 2
+    logits[3, 100:] = -60.0
+    rows = logits[:few].double().numpy()
+    for top_p in (0.9, 0.3, 0.999):
+        u = torch.rand(many, generator=g).tolist()
+        a = _sample(ops, logits[:few], [0.8] * few, [0] * few, [top_p] * few, u[:few])
+        b = _sample(ops, logits, [0.8] * many, [0] * many, [top_p] * many, u)
+        for r in range(few):
+            assert _pick_is_right(rows[r], 0.8, 0, top_p, u[r], a[r]) and _pick_is_right(rows[r], 0.8, 0, top_p, u[r], b[r]), (r, top_p)
