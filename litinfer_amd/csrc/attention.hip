@@ -2243,7 +2243,7 @@ static PrefillTime prefill_time(int nseg, const int* q_len, const int* ctx_len, 
 // begin with one of them and *upto the batch's tokens up to the last of those.  Returns the runs, 1 for none.  Only where the last block
 // is then done, the runs joined, 5 % earlier: segments of different lengths do not run in rounds, and a first tile's few keys
 // gain nothing.  103 batches of one to five segments in seven head layouts, where rounds alone would cut: 26 were 3 to 14 % slower for it; with
-// the ends of all blocks worked out none is by more than 2 %, and 40 are cut, 12 % faster on average (1,999 tokens behind 16,000, 40 of 8
+// the ends of all blocks worked out none is by more than 2.3 %, and 40 are cut, in 12 % less time on average (1,999 tokens behind 16,000, 40 of 8
 // heads: 909 -> 812 us; 290 tokens behind 2,048 and 2,048 from their start, 28 of 4: 84.8 -> 79.0).
 static int prefill_tail(int nseg, const int* q_len, const int* ctx_len, int nh, int nkv, int dh, int window, int heads, long max_bytes, const PrefillTime& whole,
                         PrefillTime* with, int* split_tiles, int* split_tokens, int* upto) {
