@@ -1663,7 +1663,8 @@ __global__ __launch_bounds__(256) void act_of_sums_kernel(const float* __restric
 // The same for the residual sum, one block a row, with the RMS norm of the new sum as a second
 // result: out[m, :] += factor * (sum of the parts + bias) (float32), xn[m, :] = gamma * out[m, :] /
 // sqrt(mean(out[m, :]^2) + eps).  A row is kept in registers (N <= NT * PER).
-template <typename TN, int NT, int PER>
+// THERE: the sum is in `out` already, and its norm alone is written (nsplit does not matter).
+template <typename TN, int NT, int PER, bool THERE = false>
 __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                  const float* __restrict__ bias, float* __restrict__ out,
                                                                  float factor, const float* __restrict__ gamma, float eps,
@@ -1676,7 +1677,9 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
     for (int i = 0; i < PER; ++i) {
         const int n = threadIdx.x + i * NT;
         v[i] = 0.f;
-        if (n < N) {
+        if constexpr (THERE) {
+            if (n < N) v[i] = out[row + n];
+        } else if (n < N) {
             // all loads at once (a part past the last reads the first and is not added): the block is
             // one of few and must not wait for memory part after part
             float a[8];
@@ -1771,6 +1774,7 @@ static int launch_big(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
 // the bias, rotates query and key heads by the row's angles (float32 tables), writes the
 // queries to out and keys and values straight into their page slots (and to out as well).
 #define SK_CHUNK 128
+#define SK_MAX_PARTS 512            // blocks of a producing product whose sums one consumer adds up
 
 struct SkinnyArgs {
     const bf16_t* x;        // [M, K]
@@ -1808,230 +1812,103 @@ struct SkinnyArgs {
     float alpha;
     // SWIGLU with EPI 1: one of the other gated forms (see gated_bf16).  EPI 2 (bfloat16 out): out = activation(product + bias)
     LiAct ep;
+    unsigned half_magic;    // with ROPE: see skinny_head
 };
-#define SK_MAX_PARTS 512            // blocks of a producing product whose sums one consumer adds up
 
-// EPI 1: with SWIGLU the other gated activations, else (float out) the tanh norm of the new sum beside it (SkinnyArgs: beta).
-// EPI 2: an activation of the sums (SkinnyArgs: ep).
-template <int MT, int NT, int WAVES, bool SWIGLU, typename TO, bool ROPE = false, int EPI = 0>
-__global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs a) {
-    static_assert(!ROPE || (MT <= 2 && !SWIGLU), "the rotary epilogue takes one or two tiles of rows");
-    static_assert(MT <= WAVES, "wave mt writes the results of row tile mt");
-    __shared__ floatx4 red[WAVES][MT * NT][64];
-    __shared__ float part_sums[WAVES * 64];          // [group of threads][row]: the rows' sums of squares, a share a group
-    // rows that the shares of the sums of squares are kept for, a block and a step: 16 up to 16 rows, else 32
-    // (the products on both sides of a norm see the same M)
-    constexpr int RP = MT <= 1 ? 16 : 32;
-    const int M = a.M, N = a.N, K = a.K;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (the same for a wave's lanes: its branches are scalar)
-    const int g = lane >> 4, r16 = lane & 15;
-    const int per_block = a.cols > 0 ? a.cols : (ROPE ? 8 : 16) * (SWIGLU ? 1 : NT);
-    const int n0 = blockIdx.x * per_block;                  // first column (with ROPE: first pair) of this block
-    const int half = a.dh / 2;
-    const int total = ROPE ? (a.nh + 2 * a.nkv) * half : N;
-    const int nend = n0 + per_block < total ? n0 + per_block : total;     // one past its last
-    const bf16_t* wrow[NT];
+// The head that rotation pair p belongs to: p / (dh / 2) by a product with 2^32 / (dh / 2) rounded up (exact below 2^32 / (dh / 2) pairs)
+__device__ __forceinline__ int skinny_head(const SkinnyArgs& a, int p) { return (int)__umulhi((unsigned)p, a.half_magic); }
+
+// Rows that the shares of the sums of squares are kept for, a block and a step: 16 up to 16 rows, else 32 (the products on both sides of a
+// norm see the same M, up to 32; with more rows nobody asks)
+template <int MT> constexpr int SKINNY_PLACES = MT <= 1 ? 16 : 32;
+
+// All of a kernel's arguments in one trip to memory: asked for where they are used they are two or three, one behind the other (0.1 to
+// 0.5 us of a launch whose matrix takes 1 to 3).
+template <bool ROPE>
+__device__ __forceinline__ void skinny_arguments(const SkinnyArgs& a) {
+    asm volatile("" ::"s"(a.x), "s"(a.w), "s"(a.out), "s"(a.bias), "s"(a.M), "s"(a.N), "s"(a.K), "s"(a.cols), "s"(a.row_parts), "s"(a.nparts), "s"(a.accumulate));
+    if constexpr (ROPE) asm volatile("" ::"s"(a.cos), "s"(a.sin), "s"(a.slot_map), "s"(a.kc), "s"(a.vc), "s"(a.nh), "s"(a.nkv), "s"(a.dh), "s"(a.half_magic));
+    else asm volatile("" ::"s"(a.gamma), "s"(a.xg), "s"(a.sq_parts));
+}
+
+// The rows' sums of squares from the shares that the blocks of the product before the norm left.  Thread t asks for four rows (a quad) of
+// parts t / quads, t / quads + G, ..; the loads are conditional on the wave's own count only, into registers that nothing else writes (a
+// share set to zero first made the compiler wait for the first load before it issued the second).
+template <int RP, int WAVES>
+struct RowShares {
+    static constexpr int QUADS = RP / 4, G = WAVES * 64 / QUADS, PER = SK_MAX_PARTS / G;
+    floatx4 v[PER];
+    __device__ __forceinline__ void ask(const float* parts, int nparts) {
+        const int q = threadIdx.x / QUADS, r = 4 * (threadIdx.x % QUADS);
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-        int row;
-        if (SWIGLU) row = ((n0 + r16 < nend) ? n0 + r16 : nend - 1) + nt * N;      // gate row, up row
-        else if (ROPE) {                                    // rows 0..7 of a tile: first members of 8 pairs, 8..15: their partners
-            int p = n0 + 8 * nt + (r16 & 7);
-            p = p < nend ? p : nend - 1;
-            row = (p / half) * a.dh + p % half + (r16 < 8 ? 0 : half);
-        } else row = (n0 + 16 * nt + r16 < nend) ? n0 + 16 * nt + r16 : nend - 1;    // rows past the end repeat the last
-        wrow[nt] = a.w + (size_t)row * K;
+        for (int i = 0; i < PER; ++i)
+            if (i * G < nparts) {
+                const int p = q + i * G;
+                v[i] = *reinterpret_cast<const floatx4*>(parts + (size_t)(p < nparts ? p : nparts - 1) * RP + r);
+            }
     }
-    // x is read with whole rows of a chunk contiguous over 16 lanes (lane l: row l / 16 + 4 i,
-    // piece l % 16), which costs the load path a quarter of what reading it in the MFMA's
-    // operand order would, and is turned into that order through a piece of LDS of the wave's own.
-    // (With 64 rows that piece of LDS would be too large; then x is read in operand order.)
-    constexpr bool XLDS = MT <= 2;
-    constexpr int XR = MT * 4;                      // 16-byte pieces of x per lane and chunk
-    __shared__ __attribute__((aligned(16))) uint16_t xs_all[XLDS ? WAVES : 1][XLDS ? MT * 16 * 128 : 8];
-    uint16_t* xs = xs_all[XLDS ? wave : 0];
-    const int xl_row = lane >> 4, xl_piece = lane & 15;
-    // piece p of row r lies at position p ^ (r % 16): the 16 rows a fragment read touches fall
-    // into 16 different positions, so into all banks
-    auto xslot = [](int row, int piece) { return row * 128 + ((piece ^ (row & 15)) << 3); };
-    floatx4 acc[MT][NT];
+    // each wave's sum of every row to sums[wave][row]
+    __device__ __forceinline__ void add(int nparts, float (*sums)[RP]) {
+        const int q = threadIdx.x / QUADS, lane = threadIdx.x & 63;
+        floatx4 mine = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+        for (int i = 0; i < PER; ++i)
+            if (q + i * G < nparts) mine += v[i];
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
-    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
-    const int nchunks = (K + SK_CHUNK - 1) / SK_CHUNK;
-    const int nfull = K / SK_CHUNK;                    // whole chunks
-
-    // What the epilogue adds to or multiplies with the sums (bias, the residual sum, a norm's
-    // weights, the rotation's cosines and sines, the page slot) is asked for now, by the wave
-    // that will write the results: the answers arrive with the first chunk, and the epilogue
-    // waits for no memory.  Never conditional per lane: a place past the end reads the last one.
-    constexpr bool PRE = MT <= 2 && !SWIGLU && EPI != 2;        // (wave mt writes row tile mt: thread t of the epilogue is lane t % 64 of wave t / 64)
-    float pre_bias[NT][4], pre_res[NT][4], pre_gamma[NT][4], pre_beta[NT][4], pre_cos[NT][4], pre_sin[NT][4];
-    int pre_slot = 0;
-    if constexpr (PRE) {
-        if (wave < MT) {
-            const int m = 16 * wave + (lane & 15) < M ? 16 * wave + (lane & 15) : M - 1;
-            if constexpr (ROPE) {
-                const bool second = (lane >> 4) >= 2;
-                pre_slot = a.slot_map[m];
+        for (int o = QUADS; o < 64; o <<= 1)
 #pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        int p = n0 + 8 * nt + 4 * ((lane >> 4) & 1) + r;
-                        p = p < nend ? p : nend - 1;
-                        const int head = p / half, j = p % half;
-                        pre_bias[nt][r] = a.bias ? a.bias[head * a.dh + (second ? half + j : j)] : 0.f;
-                        pre_cos[nt][r] = a.cos[(size_t)m * half + j];
-                        pre_sin[nt][r] = a.sin[(size_t)m * half + j];
-                    }
-            } else {
-#pragma unroll
-                for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        const int n = n0 + 16 * nt + 4 * (lane >> 4) + r;
-                        const int nc = n < nend ? n : nend - 1;
-                        pre_bias[nt][r] = a.bias ? a.bias[nc] : 0.f;
-                        pre_gamma[nt][r] = a.gamma ? a.gamma[nc] : 0.f;
-                        if constexpr (EPI == 1) pre_beta[nt][r] = a.beta[nc];
-                        if constexpr (sizeof(TO) == 4)
-                            pre_res[nt][r] = a.accumulate != 0.f ? reinterpret_cast<const float*>(a.out)[(size_t)m * N + nc] : 0.f;
-                        else pre_res[nt][r] = 0.f;
-                    }
-            }
-        }
+            for (int e = 0; e < 4; ++e) mine[e] += __shfl_xor(mine[e], o, 64);
+        if (lane < QUADS) *reinterpret_cast<floatx4*>(&sums[threadIdx.x >> 6][4 * lane]) = mine;
     }
+};
 
-    // The memory counter of a wave retires loads in the order they were issued, so waiting for
-    // a chunk's x pieces also waits for every load issued before them.  All loads of a chunk (W
-    // and x) are therefore issued together, one chunk ahead of their use: when chunk c is
-    // multiplied, exactly the loads of chunk c + WAVES are still in flight.  (With 64 rows the x
-    // pieces do not fit a second buffer; then a chunk is loaded and used in one go and the other
-    // waves of the compute unit cover the latency.)
-    constexpr bool AHEAD = MT <= 2;
-    constexpr int NBUF = AHEAD ? 2 : 1;
-    bf16x8 wbuf[NBUF][NT][4], xbuf[NBUF][XR];
-    // No load of a whole chunk is conditional, and none is replaced by zeros: a load under a branch makes the
-    // compiler wait for every load in flight at the next use of any (found in this kernel's code: s_waitcnt
-    // vmcnt(0) before each multiplication, right behind the loads of the chunk after it, so that nothing was in
-    // flight while a wave multiplied), and a value chosen between what was loaded and zero is waited for at once.
-    // A row of x past the last is read from the last row (its sums are not written).  Only the last chunk of a K
-    // that is no multiple of the chunk has k-values to leave out: it is taken by itself, behind the loop (TAIL).
-    auto load_chunk = [&](int c, bf16x8 (*wd)[4], bf16x8* xd, auto tail_tag) {
-        constexpr bool TAIL = decltype(tail_tag)::value;
-        const int kb = c * SK_CHUNK;
+// What the epilogue adds to or multiplies with the sums (bias, the residual sum, a norm's weights, the rotation's cosines and sines, the
+// page slot), asked for by the wave that will write the results (wave mt row tile mt: thread t of the epilogue is lane t % 64 of wave
+// t / 64) before it has them to add: the epilogue waits for no memory.  Never conditional per lane: a place past the end reads the last one.
+template <bool SWIGLU, int EPI> constexpr bool SKINNY_PRE = !SWIGLU && EPI != 2;
+template <int NT> struct SkinnyPre { float bias[NT][4], res[NT][4], gamma[NT][4], beta[NT][4], cos[NT][4], sin[NT][4]; int slot; };
+
+template <int NT, typename TO, bool ROPE, int EPI>
+__device__ __forceinline__ void skinny_ask(const SkinnyArgs& a, SkinnyPre<NT>& pre, int n0, int nend, int mt, int lane) {
+    const int m = 16 * mt + (lane & 15) < a.M ? 16 * mt + (lane & 15) : a.M - 1;
+    if constexpr (ROPE) {
+        const bool second = (lane >> 4) >= 2;
+        const int half = a.dh / 2;
+        pre.slot = a.slot_map[m];
 #pragma unroll
-        for (int i = 0; i < XR; ++i) {
-            int m, kk;
-            if constexpr (XLDS) { m = xl_row + 4 * i; kk = kb + 8 * xl_piece; }
-            else { m = 16 * (i >> 2) + r16; kk = kb + 8 * g + 32 * (i & 3); }       // operand order: row 16 mt + r16, pieces g + 4 j
-            const bf16_t* row = a.x + (size_t)(m < M ? m : M - 1) * K;
-            if constexpr (TAIL) xd[i] = kk < K ? *reinterpret_cast<const bf16x8*>(row + kk) : zero;
-            else xd[i] = *reinterpret_cast<const bf16x8*>(row + kk);
-        }
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int kk = kb + 8 * g + 32 * j;
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt) {
-                if constexpr (TAIL) wd[nt][j] = kk < K ? *reinterpret_cast<const bf16x8*>(wrow[nt] + kk) : zero;
-                else wd[nt][j] = *reinterpret_cast<const bf16x8*>(wrow[nt] + kk);
+            for (int r = 0; r < 4; ++r) {
+                int p = n0 + 8 * nt + 4 * ((lane >> 4) & 1) + r;
+                p = p < nend ? p : nend - 1;
+                const int head = skinny_head(a, p), j = p - head * half;
+                pre.bias[nt][r] = a.bias ? a.bias[head * a.dh + (second ? half + j : j)] : 0.f;
+                pre.cos[nt][r] = a.cos[(size_t)m * half + j];
+                pre.sin[nt][r] = a.sin[(size_t)m * half + j];
             }
-        }
-    };
-    auto multiply = [&](bf16x8 (*wa)[4], bf16x8* xd) {
-        if constexpr (XLDS) {
-            __builtin_amdgcn_wave_barrier();        // a wave's LDS operations run in order; keep the compiler's too
-#pragma unroll
-            for (int i = 0; i < XR; ++i)
-                *reinterpret_cast<bf16x8*>(&xs[xslot(xl_row + 4 * i, xl_piece)]) = xd[i];
-            __builtin_amdgcn_wave_barrier();
-        }
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            bf16x8 xa[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if constexpr (XLDS) xa[j] = *reinterpret_cast<const bf16x8*>(&xs[xslot(16 * mt + r16, g + 4 * j)]);
-                else xa[j] = xd[4 * mt + j];
-            }
-#pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[nt][j], xa[j], acc[mt][nt], 0, 0, 0);
-        }
-        __builtin_amdgcn_wave_barrier();
-    };
-    if constexpr (AHEAD) {
-        if (wave < nfull) load_chunk(wave, wbuf[0], xbuf[0], std::false_type{});
-        // the rows' sums of squares: thread t adds the parts t / 16, t / 16 + G, ... of row t % 16 in
-        // that order; the epilogue adds the G sums in theirs.  The loads are issued together, behind
-        // those of the first chunk, only as many rounds as there are parts, and never conditional
-        // within a round (a part past the end reads the last one).  They are added up behind the
-        // loads of the second chunk: the wait for them is the wait the first multiplication has anyway.
-        constexpr int G = WAVES * 64 / RP, PER = SK_MAX_PARTS / G;
-        float part[PER];
-        if (a.row_parts) {
-            const int m = threadIdx.x % RP, q = threadIdx.x / RP;
-#pragma unroll
-            for (int i = 0; i < PER; ++i) {
-                part[i] = 0.f;
-                if (i * G < a.nparts) {
-                    const int p = q + i * G;
-                    part[i] = a.row_parts[(size_t)(p < a.nparts ? p : a.nparts - 1) * RP + m];
-                }
-            }
-        }
-        if (wave + WAVES < nfull) load_chunk(wave + WAVES, wbuf[1], xbuf[1], std::false_type{});
-        if (a.row_parts) {
-            const int m = threadIdx.x % RP, q = threadIdx.x / RP;
-            float mine = 0.f;
-#pragma unroll
-            for (int i = 0; i < PER; ++i) mine += (q + i * G < a.nparts) ? part[i] : 0.f;
-            part_sums[q * RP + m] = mine;
-        }
-        // (the first turn is written out: its loads of the second chunk stand above, before the parts are added up)
-        if (wave < nfull) multiply(wbuf[0], xbuf[0]);
-        if (wave + WAVES < nfull) {
-            if (wave + 2 * WAVES < nfull) load_chunk(wave + 2 * WAVES, wbuf[0], xbuf[0], std::false_type{});
-            multiply(wbuf[1], xbuf[1]);
-            // Two chunks a turn (buffer numbers are constants).  Inside the loop nothing about the loads is
-            // conditional: where a path with loads and one without meet, the compiler's count of the loads in
-            // flight is the smaller one, and the next wait is for all of them.  So the loop runs while both of
-            // a turn's loads exist, and the one or two chunks that are left are taken behind it.
-            int c = wave + 2 * WAVES;
-            for (; c + 2 * WAVES < nfull; c += 2 * WAVES) {
-                load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
-                multiply(wbuf[0], xbuf[0]);
-                load_chunk(c + 2 * WAVES, wbuf[0], xbuf[0], std::false_type{});
-                multiply(wbuf[1], xbuf[1]);
-            }
-            if (c < nfull) {
-                const bool more = c + WAVES < nfull;
-                if (more) load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
-                multiply(wbuf[0], xbuf[0]);
-                if (more) multiply(wbuf[1], xbuf[1]);
-            }
-        }
     } else {
-        for (int c = wave; c < nfull; c += WAVES) {
-            load_chunk(c, wbuf[0], xbuf[0], std::false_type{});
-            multiply(wbuf[0], xbuf[0]);
-        }
-    }
-    if (nfull < nchunks && wave == nfull % WAVES) {     // the chunk that K ends in
-        load_chunk(nfull, wbuf[0], xbuf[0], std::true_type{});
-        multiply(wbuf[0], xbuf[0]);
-    }
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
+        for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) red[wave][mt * NT + nt][lane] = acc[mt][nt];
-    __syncthreads();
+            for (int r = 0; r < 4; ++r) {
+                const int n = n0 + 16 * nt + 4 * (lane >> 4) + r;
+                const int nc = n < nend ? n : nend - 1;
+                pre.bias[nt][r] = a.bias ? a.bias[nc] : 0.f;
+                pre.gamma[nt][r] = a.gamma ? a.gamma[nc] : 0.f;
+                if constexpr (EPI == 1) pre.beta[nt][r] = a.beta[nc];
+                if constexpr (sizeof(TO) == 4)
+                    pre.res[nt][r] = a.accumulate != 0.f ? reinterpret_cast<const float*>(a.out)[(size_t)m * a.N + nc] : 0.f;
+                else pre.res[nt][r] = 0.f;
+            }
+    }
+}
+
+// The waves' sums (red[wave][row tile, column tile][lane], as the MFMAs leave them) added in wave order, and what follows; row_squares(m):
+// the sum of row m's squares where the rows are those of li_linear_residual_norm.
+template <int MT, int NT, int WAVES, bool SWIGLU, typename TO, bool ROPE, int EPI, typename RowSquares>
+__device__ __forceinline__ void skinny_finish(const SkinnyArgs& a, floatx4 (*red)[MT * NT][64], const SkinnyPre<NT>& pre, int n0, int nend, RowSquares row_squares) {
+    constexpr int RP = SKINNY_PLACES<MT>;
+    const int M = a.M, N = a.N, half = a.dh / 2;
     TO* out = (TO*)a.out;
     if constexpr (EPI == 2 && !SWIGLU) {
         // one value a thread at a time, by all waves: an activation is tens of instructions a value, and by the one wave that
@@ -2062,18 +1939,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
                 s[nt][0] += o[0]; s[nt][1] += o[1]; s[nt][2] += o[2]; s[nt][3] += o[3];
             }
         }
-        if (AHEAD && a.row_parts) {
-            float sq = part_sums[m % RP];
-#pragma unroll
-            for (int q = 1; q < WAVES * 64 / RP; ++q) sq += part_sums[q * RP + m % RP];
-            const float inv = 1.0f / sqrtf(sq / (float)K + a.eps);
+        if ((SWIGLU || ROPE) && a.row_parts) {
+            const float inv = 1.0f / sqrtf(row_squares(m) / (float)a.K + a.eps);
 #pragma unroll
             for (int nt = 0; nt < NT; ++nt) { s[nt][0] *= inv; s[nt][1] *= inv; s[nt][2] *= inv; s[nt][3] *= inv; }
         }
         if constexpr (ROPE) {
             const int dh = a.dh;
             const bool second = (l >> 4) >= 2;                       // this lane holds the pairs' second members
-            const int slot = pre_slot;                               // (thread t is lane l of wave mt, which asked for these)
+            const int slot = pre.slot;                               // (thread t is lane l of wave mt, which asked for these: skinny_ask)
             const int page = slot / a.page_size, in_page = slot - page * a.page_size;
             const bool page_ok = page >= 0 && page < a.num_pages;
 #pragma unroll
@@ -2081,15 +1955,15 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int p = n0 + 8 * nt + 4 * ((l >> 4) & 1) + r;  // the pair's number among all heads' pairs
-                    float own = s[nt][r] + pre_bias[nt][r];
+                    float own = s[nt][r] + pre.bias[nt][r];
                     const float other = __shfl_xor(own, 32, 64);
                     if (p >= nend) continue;                         // (lanes l and l ^ 32 share p: the exchange above is done by both)
-                    const int head = p / half, j = p - head * half;
+                    const int head = skinny_head(a, p), j = p - head * half;
                     const int d = second ? half + j : j;
                     const int col = head * dh + d;
                     float v = own;
                     if (head < a.nh + a.nkv) {
-                        const float c = pre_cos[nt][r], sn = pre_sin[nt][r];
+                        const float c = pre.cos[nt][r], sn = pre.sin[nt][r];
                         v = second ? own * c + other * sn : own * c - other * sn;
                     }
                     const uint16_t bits = float_to_bf16(v);
@@ -2112,7 +1986,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
             }
         } else {
             [[maybe_unused]] const float factor = a.accumulate != 0.f ? a.accumulate : 1.0f;
-            if constexpr (sizeof(TO) == 4 && MT <= 2) {
+            if constexpr (sizeof(TO) == 4) {
                 if (a.xg) {                          // the sum goes out three ways (see SkinnyArgs)
                     float sq = 0.f;
 #pragma unroll
@@ -2122,10 +1996,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
                             const int n = n0 + 16 * nt + 4 * (l >> 4) + r;
                             if (n < nend) {
                                 const size_t idx = (size_t)m * N + n;
-                                const float v = fmaf(factor, s[nt][r] + pre_bias[nt][r], pre_res[nt][r]);
+                                const float v = fmaf(factor, s[nt][r] + pre.bias[nt][r], pre.res[nt][r]);
                                 reinterpret_cast<float*>(out)[idx] = v;
-                                a.xg[idx].bits = float_to_bf16(EPI == 1 ? fmaf(tanhf(a.alpha * v), pre_gamma[nt][r], pre_beta[nt][r])
-                                                                        : pre_gamma[nt][r] * v);
+                                a.xg[idx].bits = float_to_bf16(EPI == 1 ? fmaf(tanhf(a.alpha * v), pre.gamma[nt][r], pre.beta[nt][r])
+                                                                        : pre.gamma[nt][r] * v);
                                 sq += v * v;
                             }
                         }
@@ -2143,11 +2017,299 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs
                 for (int r = 0; r < 4; ++r) {
                     const int n = n0 + 16 * nt + 4 * (l >> 4) + r;
                     if (n >= nend) continue;
-                    if constexpr (PRE) store_from_float(out + (size_t)m * N + n, fmaf(factor, s[nt][r] + pre_bias[nt][r], pre_res[nt][r]));
+                    if constexpr (SKINNY_PRE<SWIGLU, EPI>) store_from_float(out + (size_t)m * N + n, fmaf(factor, s[nt][r] + pre.bias[nt][r], pre.res[nt][r]));
                     else epilogue_store(out, (size_t)m * N + n, s[nt][r], a.bias, n, a.accumulate);
                 }
         }
     }
+}
+
+// EPI 1: with SWIGLU the other gated activations, else (float out) the tanh norm of the new sum beside it (SkinnyArgs: beta).
+// EPI 2: an activation of the sums (SkinnyArgs: ep).
+template <int MT, int NT, int WAVES, bool SWIGLU, typename TO, bool ROPE = false, int EPI = 0>
+__global__ __launch_bounds__(WAVES * 64) void gemm_bf16_skinny_kernel(SkinnyArgs a) {
+    static_assert(!(ROPE && SWIGLU) && MT <= 4, "up to four tiles of rows");
+    static_assert(MT <= WAVES, "wave mt writes the results of row tile mt");
+    // k-values a chunk: with three or four tiles of rows half as many, so that two chunks of x still fit the registers
+    constexpr int CH = MT <= 2 ? SK_CHUNK : SK_CHUNK / 2;
+    // x by wave, and the waves' sums, which with three or four tiles of rows take the same place behind the loop
+    constexpr int XS = MT * 16 * CH, XS_BYTES = WAVES * XS * 2, RED_BYTES = WAVES * MT * NT * 64 * 16;
+    constexpr bool SAME_PLACE = MT > 2;
+    __shared__ __attribute__((aligned(16))) char xs_all[SAME_PLACE && RED_BYTES > XS_BYTES ? RED_BYTES : XS_BYTES];
+    __shared__ floatx4 red_own[SAME_PLACE ? 1 : WAVES][MT * NT][64];
+    floatx4 (*red)[MT * NT][64] = SAME_PLACE ? reinterpret_cast<floatx4 (*)[MT * NT][64]>(xs_all) : red_own;
+    constexpr int RP = SKINNY_PLACES<MT>;
+    __shared__ float part_sums[WAVES * 64];          // [group of threads][row]: the rows' sums of squares, a share a group
+    skinny_arguments<ROPE>(a);
+    const int M = a.M, N = a.N, K = a.K;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // (the same for a wave's lanes: its branches are scalar)
+    const int g = lane >> 4, r16 = lane & 15;
+    const int per_block = a.cols > 0 ? a.cols : (ROPE ? 8 : 16) * (SWIGLU ? 1 : NT);
+    const int n0 = blockIdx.x * per_block;                  // first column (with ROPE: first pair) of this block
+    const int half = a.dh / 2;
+    const int total = ROPE ? (a.nh + 2 * a.nkv) * half : N;
+    const int nend = n0 + per_block < total ? n0 + per_block : total;     // one past its last
+    const bf16_t* wrow[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        int row;
+        if (SWIGLU) row = ((n0 + r16 < nend) ? n0 + r16 : nend - 1) + nt * N;      // gate row, up row
+        else if (ROPE) {                                    // rows 0..7 of a tile: first members of 8 pairs, 8..15: their partners
+            int p = n0 + 8 * nt + (r16 & 7);
+            p = p < nend ? p : nend - 1;
+            const int head = skinny_head(a, p);
+            row = head * a.dh + p - head * half + (r16 < 8 ? 0 : half);
+        } else row = (n0 + 16 * nt + r16 < nend) ? n0 + 16 * nt + r16 : nend - 1;    // rows past the end repeat the last
+        wrow[nt] = a.w + (size_t)row * K;
+    }
+    // x is read with whole rows of a chunk contiguous over 16 (8) lanes (lane l: row l / 16 + 4 i,
+    // piece l % 16), which costs the load path a quarter of what reading it in the MFMA's
+    // operand order would, and is turned into that order through a piece of LDS of the wave's own.
+    constexpr int XP = CH / 8, XROWS = 64 / XP;     // 16-byte pieces of a row's chunk; rows a load of the wave covers
+    constexpr int XR = MT * 16 / XROWS;             // 16-byte pieces of x per lane and chunk
+    constexpr int WJ = CH / 32;                     // ... and of a tile of w
+    uint16_t* xs = reinterpret_cast<uint16_t*>(xs_all) + wave * XS;
+    const int xl_row = lane / XP, xl_piece = lane % XP;
+    // piece p of row r lies at position p ^ (r % 16) (r % 8): the 16 rows a fragment read touches fall
+    // into different positions, so into all banks
+    auto xslot = [](int row, int piece) { return row * CH + ((piece ^ (row & (XP - 1))) << 3); };
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+    const int nchunks = (K + CH - 1) / CH;
+    const int nfull = K / CH;                          // whole chunks
+
+    SkinnyPre<NT> pre;
+    if (SKINNY_PRE<SWIGLU, EPI> && wave < MT) skinny_ask<NT, TO, ROPE, EPI>(a, pre, n0, nend, wave, lane);
+
+    // The memory counter of a wave retires loads in the order they were issued, so waiting for
+    // a chunk's x pieces also waits for every load issued before them.  All loads of a chunk (W
+    // and x) are therefore issued together, one chunk ahead of their use: when chunk c is
+    // multiplied, exactly the loads of chunk c + WAVES are still in flight.
+    bf16x8 wbuf[2][NT][WJ], xbuf[2][XR];
+    // No load of a whole chunk is conditional, and none is replaced by zeros: a load under a branch makes the
+    // compiler wait for every load in flight at the next use of any (found in this kernel's code: s_waitcnt
+    // vmcnt(0) before each multiplication, right behind the loads of the chunk after it, so that nothing was in
+    // flight while a wave multiplied), and a value chosen between what was loaded and zero is waited for at once.
+    // A row of x past the last is read from the last row (its sums are not written).  Only the last chunk of a K
+    // that is no multiple of the chunk has k-values to leave out: it is taken by itself, behind the loop (TAIL).
+    auto load_chunk = [&](int c, bf16x8 (*wd)[WJ], bf16x8* xd, auto tail_tag) {
+        constexpr bool TAIL = decltype(tail_tag)::value;
+        const int kb = c * CH;
+#pragma unroll
+        for (int i = 0; i < XR; ++i) {
+            const int m = xl_row + XROWS * i, kk = kb + 8 * xl_piece;
+            const bf16_t* row = a.x + (size_t)(m < M ? m : M - 1) * K;
+            if constexpr (TAIL) xd[i] = kk < K ? *reinterpret_cast<const bf16x8*>(row + kk) : zero;
+            else xd[i] = *reinterpret_cast<const bf16x8*>(row + kk);
+        }
+#pragma unroll
+        for (int j = 0; j < WJ; ++j) {
+            const int kk = kb + 8 * g + 32 * j;
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                if constexpr (TAIL) wd[nt][j] = kk < K ? *reinterpret_cast<const bf16x8*>(wrow[nt] + kk) : zero;
+                else wd[nt][j] = *reinterpret_cast<const bf16x8*>(wrow[nt] + kk);
+            }
+        }
+    };
+    auto multiply = [&](bf16x8 (*wa)[WJ], bf16x8* xd) {
+        __builtin_amdgcn_wave_barrier();            // a wave's LDS operations run in order; keep the compiler's too
+#pragma unroll
+        for (int i = 0; i < XR; ++i)
+            *reinterpret_cast<bf16x8*>(&xs[xslot(xl_row + XROWS * i, xl_piece)]) = xd[i];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            bf16x8 xa[WJ];
+#pragma unroll
+            for (int j = 0; j < WJ; ++j) xa[j] = *reinterpret_cast<const bf16x8*>(&xs[xslot(16 * mt + r16, g + 4 * j)]);
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int j = 0; j < WJ; ++j)
+                    acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa[nt][j], xa[j], acc[mt][nt], 0, 0, 0);
+        }
+        __builtin_amdgcn_wave_barrier();
+    };
+    if (wave < nfull) load_chunk(wave, wbuf[0], xbuf[0], std::false_type{});
+    // the rows' sums of squares: thread t adds the parts t / RP, t / RP + G, ... of row t % RP in that order; the epilogue adds the G sums in
+    // theirs.  The loads are issued together, behind those of the first chunk, only as many rounds as there are parts, and never conditional
+    // within a round (a part past the end reads the last one).  A part set to zero first makes the compiler wait for the first load before it
+    // issues the second: the packed projection, one round of blocks, is the faster without (8 rows of 4,608 x 3,584 10.4 -> 9.9 us), the gated
+    // product, whose blocks come several to a unit, with it (8 rows of 37,888 x 3,584 50.9 / 50.4).  They are added up behind the loads of the second chunk: the wait for them is the wait the first multiplication has
+    // anyway.  (Exchanges between lanes in place of the G sums: 13.1 -> 13.7 us for 17,920 x 1,536, whose blocks come three to a unit.)
+    constexpr int G = WAVES * 64 / RP, PER = SK_MAX_PARTS / G;
+    [[maybe_unused]] float part[PER];
+    [[maybe_unused]] const int part_m = threadIdx.x % RP, part_q = threadIdx.x / RP;
+    if constexpr (SWIGLU || ROPE)
+        if (a.row_parts) {
+#pragma unroll
+            for (int i = 0; i < PER; ++i) {
+                if constexpr (SWIGLU) part[i] = 0.f;
+                if (i * G < a.nparts) {
+                    const int p = part_q + i * G;
+                    part[i] = a.row_parts[(size_t)(p < a.nparts ? p : a.nparts - 1) * RP + part_m];
+                }
+            }
+        }
+    if (wave + WAVES < nfull) load_chunk(wave + WAVES, wbuf[1], xbuf[1], std::false_type{});
+    if constexpr (SWIGLU || ROPE)
+        if (a.row_parts) {
+            float mine = 0.f;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) mine += (part_q + i * G < a.nparts) ? part[i] : 0.f;
+            part_sums[part_q * RP + part_m] = mine;
+        }
+    // (the first turn is written out: its loads of the second chunk stand above, before the parts are added up)
+    if (wave < nfull) multiply(wbuf[0], xbuf[0]);
+    if (wave + WAVES < nfull) {
+        if (wave + 2 * WAVES < nfull) load_chunk(wave + 2 * WAVES, wbuf[0], xbuf[0], std::false_type{});
+        multiply(wbuf[1], xbuf[1]);
+        // Two chunks a turn (buffer numbers are constants).  Inside the loop nothing about the loads is
+        // conditional: where a path with loads and one without meet, the compiler's count of the loads in
+        // flight is the smaller one, and the next wait is for all of them.  So the loop runs while both of
+        // a turn's loads exist, and the one or two chunks that are left are taken behind it.
+        int c = wave + 2 * WAVES;
+        for (; c + 2 * WAVES < nfull; c += 2 * WAVES) {
+            load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
+            multiply(wbuf[0], xbuf[0]);
+            load_chunk(c + 2 * WAVES, wbuf[0], xbuf[0], std::false_type{});
+            multiply(wbuf[1], xbuf[1]);
+        }
+        if (c < nfull) {
+            const bool more = c + WAVES < nfull;
+            if (more) load_chunk(c + WAVES, wbuf[1], xbuf[1], std::false_type{});
+            multiply(wbuf[0], xbuf[0]);
+            if (more) multiply(wbuf[1], xbuf[1]);
+        }
+    }
+    if (nfull < nchunks && wave == nfull % WAVES) {     // the chunk that K ends in
+        load_chunk(nfull, wbuf[0], xbuf[0], std::true_type{});
+        multiply(wbuf[0], xbuf[0]);
+    }
+    if constexpr (SAME_PLACE) __syncthreads();
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) red[wave][mt * NT + nt][lane] = acc[mt][nt];
+    __syncthreads();
+    skinny_finish<MT, NT, WAVES, SWIGLU, TO, ROPE, EPI>(a, red, pre, n0, nend, [&](int m) {
+        float sq = part_sums[m];
+#pragma unroll
+        for (int q = 1; q < WAVES * 64 / RP; ++q) sq += part_sums[q * RP + m];
+        return sq;
+    });
+}
+
+// Up to 4 rows and K a multiple of 64: the same product where launch, first load and drain are as long as the matrix itself (1 to 30 MB).
+// A block's eight waves take K in runs that follow each other (units of 64 k-values), and a wave asks for all it multiplies before it waits
+// for anything: the shares of the rows' sums of squares, its part of x (the rows that there are, not sixteen), its part of w, then the
+// epilogue's operands.  No load waits behind another one's answer and none is repeated to fill a tile of rows; a branch of the wave's own
+// (which units there are) is around loads whose registers nobody else writes, so the compiler puts no wait at its end.  D units at a time: 4
+// or 10 at once (K up to 2,048 or 5,120), or, LOOP, rounds of 4 whose loads are on their way while the round before is multiplied.
+// In a chain of recorded launches over different matrices, the kernel above against this one (us, one row; an empty launch is 1.6): 896 x 896
+// 3.3 -> 3.0, 896 x 4,864 6.8 -> 5.5, 1,536 x 1,536 4.0 -> 3.6, 1,536 x 4,480 6.7 -> 5.8, 1,536 x 8,960 10.5 -> 8.3, 2,048 x 11,008 13.6 -> 11.6,
+// 8,240 x 1,536 9.3 -> 7.0; q/k/v with rotation and page write 896 5.0 -> 4.5, 1,536 5.8 -> 5.1.
+#define FR_WAVES 8
+template <typename TO, bool ROPE, int EPI, int D, bool LOOP, int XI>
+__global__ __launch_bounds__(FR_WAVES * 64) void gemm_bf16_rows_kernel(SkinnyArgs a, int log_rows) {
+    // x of a round by wave: [unit][row][8 pieces of 16 bytes], rows a power of two (1 << log_rows; rows past the last repeat it), XI loads of
+    // 64 pieces
+    __shared__ __attribute__((aligned(16))) uint16_t xs_all[FR_WAVES][XI * 512];
+    skinny_arguments<ROPE>(a);
+    asm volatile("" ::"s"(log_rows));
+    __shared__ floatx4 red[FR_WAVES][1][64];
+    __shared__ __attribute__((aligned(16))) float part_sums[FR_WAVES][16];
+    const int M = a.M, N = a.N, K = a.K;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int g = lane >> 4, r16 = lane & 15;
+    const int n0 = blockIdx.x * a.cols, half = a.dh / 2, total = ROPE ? (a.nh + 2 * a.nkv) * half : N;
+    const int nend = n0 + a.cols < total ? n0 + a.cols : total;
+    const int units = K / 64, base = units / FR_WAVES, extra = units % FR_WAVES;
+    const int u0 = wave * base + (wave < extra ? wave : extra), n = base + (wave < extra ? 1 : 0);
+    [[maybe_unused]] RowShares<16, FR_WAVES> shares;
+    if constexpr (ROPE)
+        if (a.row_parts) shares.ask(a.row_parts, a.nparts);
+    uint16_t* xs = xs_all[wave];
+    bf16x8 xb[XI];
+    auto ask_x = [&](int first) {
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int f = (lane + 64 * i) >> 3, row = f & ((1 << log_rows) - 1);
+            int u = first + (f >> log_rows);
+            u = u < n ? u : n - 1;
+            xb[i] = *reinterpret_cast<const bf16x8*>(a.x + (size_t)(row < M ? row : M - 1) * K + 64 * (u0 + u) + 8 * (lane & 7));
+        }
+    };
+    auto put_x = [&]() {
+        __builtin_amdgcn_wave_barrier();            // a wave's LDS operations run in order; keep the compiler's too
+#pragma unroll
+        for (int i = 0; i < XI; ++i)
+            *reinterpret_cast<bf16x8*>(xs + (lane + 64 * i) * 8) = xb[i];
+        __builtin_amdgcn_wave_barrier();
+    };
+    int row;
+    if (ROPE) {                                     // rows 0..7 of a tile: first members of 8 pairs, 8..15: their partners
+        int p = n0 + (r16 & 7);
+        p = p < nend ? p : nend - 1;
+        const int head = skinny_head(a, p);
+        row = head * a.dh + p - head * half + (r16 < 8 ? 0 : half);
+    } else row = (n0 + r16 < nend) ? n0 + r16 : nend - 1;
+    const bf16_t* wrow = a.w + (size_t)row * K + 64 * u0 + 8 * g;
+    bf16x8 wb[D][2];
+    auto ask_w = [&](int u, int d) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) wb[d][j] = *reinterpret_cast<const bf16x8*>(wrow + 64 * u + 32 * j);
+    };
+    if (n > 0) {
+        ask_x(0);
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (d < n) ask_w(d, d);
+    }
+    SkinnyPre<1> pre;
+    if (SKINNY_PRE<false, EPI> && wave == 0) skinny_ask<1, TO, ROPE, EPI>(a, pre, n0, nend, 0, lane);
+    if constexpr (ROPE)                   // added up while w is on its way
+        if (a.row_parts) shares.add(a.nparts, part_sums);
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    const int xrow = r16 & ((1 << log_rows) - 1);
+    auto multiply = [&](int d) {
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const bf16x8 xa = *reinterpret_cast<const bf16x8*>(xs + ((((d << log_rows) + xrow) << 3) + g + 4 * j) * 8);
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[d][j], xa, acc, 0, 0, 0);
+        }
+    };
+    if (n > 0) {
+        int i = 0;
+        if constexpr (LOOP) {
+            for (; i + D < n; i += D) {             // (a unit past the last asks for the last again: at most three a wave)
+                put_x();
+                ask_x(i + D);
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    multiply(d);
+                    ask_w(i + D + d < n ? i + D + d : n - 1, d);
+                }
+            }
+        }
+        put_x();
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (i + d < n) multiply(d);
+    }
+    red[wave][0][lane] = acc;
+    __syncthreads();
+    skinny_finish<1, 1, FR_WAVES, false, TO, ROPE, EPI>(a, red, pre, n0, nend, [&](int m) {
+        float sq = part_sums[0][m];
+#pragma unroll
+        for (int q = 1; q < FR_WAVES; ++q) sq += part_sums[q][m];
+        return sq;
+    });
 }
 
 // Compute units of the current device (256 where it cannot be asked).
@@ -2167,11 +2329,12 @@ static int compute_units() {
 // tile): a compute unit takes in what its blocks ask for at a rate of its own, far below its share of
 // the memory's rate times the number of units, so the time of such a product is that of the unit with the
 // most blocks.  Every unit therefore gets one block and every block the same number of columns (at
-// most two tiles' worth, at least half a tile's), not whole tiles.
+// most two tiles' worth, at least a quarter of a tile's), not whole tiles.  (At least a quarter, where a half was: 896 x 4,864 at one row
+// 6.05 -> 5.53 us with twice the blocks.)
 static int balanced_per_block(int total, int unit) {
     const int cu = compute_units();
     int per = (total + cu - 1) / cu;
-    per = per < unit / 2 ? unit / 2 : per;
+    per = per < unit / 4 ? unit / 4 : per;
     return per > 2 * unit ? 0 : per;
 }
 
@@ -2187,9 +2350,45 @@ static int balanced_round_cols(int total, int unit) {
     return (int)(per > unit ? unit : per);
 }
 
+// Whether a product of few rows goes to gemm_bf16_rows_kernel (columns: the matrix's rows).  Not from five rows on, where all blocks' reading of
+// x bounds both and the kernel above, whose loads of x are whole rows of a chunk, is as fast or faster (us, 5 rows: 896 x 896 3.5 / 3.6, 8 rows:
+// 2,048 x 11,008 13.7 / 14.9); nor against a wide matrix of long rows, where its chunks, which the eight waves take in turns, read w in longer
+// pieces (one row: 3,584 x 3,584 7.1 / 8.0, 5,120 x 5,120 12.1 / 13.9).  The gated product stays with it too: its blocks come two and more to a
+// compute unit, where this kernel's registers leave room for fewer (17,920 x 1,536 13.1 / 14.5).
+#define ROWS_KERNEL_M 4
+static bool rows_kernel_takes(int M, long columns, int K) {
+    return M <= ROWS_KERNEL_M && K % 64 == 0 && (K <= 2048 || columns <= 2048);
+}
+
+template <typename TO, bool ROPE, int EPI>
+static void launch_rows(const SkinnyArgs& a, int blocks, hipStream_t stream) {
+    const int log_rows = a.M <= 1 ? 0 : a.M <= 2 ? 1 : 2;
+    const int n = (a.K / 64 + FR_WAVES - 1) / FR_WAVES;              // a wave's units
+#define LI_FR(D, LOOP, X2, X4)                                                                                                          \
+    {                                                                                                                                   \
+        if (log_rows <= 1) gemm_bf16_rows_kernel<TO, ROPE, EPI, D, LOOP, X2><<<blocks, FR_WAVES * 64, 0, stream>>>(a, log_rows);        \
+        else gemm_bf16_rows_kernel<TO, ROPE, EPI, D, LOOP, X4><<<blocks, FR_WAVES * 64, 0, stream>>>(a, log_rows);                      \
+    }
+    if (n <= 4) LI_FR(4, false, 1, 2)
+    else if constexpr (!ROPE) {
+        if (n <= 10) LI_FR(10, false, 3, 5)
+        else LI_FR(4, true, 1, 2)
+    }
+#undef LI_FR
+}
+
 template <bool SWIGLU, typename TO, int EPI = 0>
 static void launch_skinny(SkinnyArgs a, hipStream_t stream) {
     const int M = a.M, N = a.N;
+    if constexpr (!SWIGLU) {
+        // (a sum into out comes out of one kernel whether or not its shares of the rows' squares are asked for, whose number goes with the
+        // columns alone: li_residual_norm_parts)
+        if (rows_kernel_takes(M, N, a.K) && (a.accumulate == 0.f || N <= 4096)) {
+            a.cols = N <= 4096 ? balanced_per_block(N, 16) : balanced_round_cols(N, 16);
+            launch_rows<TO, false, EPI>(a, (N + a.cols - 1) / a.cols, stream);
+            return;
+        }
+    }
 #define LI_SK(MT, NT, WV) gemm_bf16_skinny_kernel<MT, NT, WV, SWIGLU, TO, false, EPI><<<(N + 16 * (SWIGLU ? 1 : NT) - 1) / (16 * (SWIGLU ? 1 : NT)), WV * 64, 0, stream>>>(a)
     if constexpr (SWIGLU) {
         a.cols = balanced_round_cols(N, 16);
@@ -2209,8 +2408,12 @@ static void launch_skinny(SkinnyArgs a, hipStream_t stream) {
         const int per = a.cols ? a.cols : 16, blocks = (N + per - 1) / per;
         if (per > 16) gemm_bf16_skinny_kernel<2, 2, 4, false, TO, false, EPI><<<blocks, 4 * 64, 0, stream>>>(a);
         else gemm_bf16_skinny_kernel<2, 1, 4, false, TO, false, EPI><<<blocks, 4 * 64, 0, stream>>>(a);
-    } else {
-        LI_SK(4, 2, 8);
+    } else {                                                // 33 to 64 rows: rows up to 48 are three tiles
+        a.cols = balanced_per_block(N, 16);
+        const int per = a.cols ? a.cols : 16, blocks = (N + per - 1) / per;
+        if (per > 16) gemm_bf16_skinny_kernel<4, 2, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
+        else if (M <= 48) gemm_bf16_skinny_kernel<3, 1, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
+        else gemm_bf16_skinny_kernel<4, 1, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
     }
 #undef LI_SK
 }
@@ -2227,6 +2430,33 @@ extern "C" int li_linear_skinny(const void* x, const void* w, const float* bias,
     else if (out_dtype == LI_BF16) launch_skinny<false, bf16_t>(a, stream);
     else if (out_dtype == LI_F32) launch_skinny<false, float>(a, stream);
     else return LI_ERR_DTYPE;
+    return li_launch_status();
+}
+
+// The packed projection of up to 64 rows, rotated and written into its pages (SkinnyArgs: ROPE).
+static int launch_skinny_rope(SkinnyArgs a, hipStream_t stream) {
+    const int M = a.M, pairs = a.N / 2, half = a.dh / 2;
+    if ((unsigned long long)pairs * half >= (1ull << 32)) return LI_ERR_SIZE;
+    a.half_magic = (unsigned)(((1ull << 32) + half - 1) / half);
+    if (rows_kernel_takes(M, a.N, a.K) && a.K <= 2048 && pairs <= 8l * compute_units()) {
+        const int even = (pairs + compute_units() - 1) / compute_units();
+        a.cols = even < 3 ? 3 : even;                   // (576 pairs of 896: 3 a block 4.47 us, 4 4.66, 2 4.90)
+        launch_rows<bf16_t, true, 0>(a, (pairs + a.cols - 1) / a.cols, stream);
+        return li_launch_status();
+    }
+    a.cols = balanced_per_block(pairs, 8);
+    const int per = a.cols ? a.cols : 8, blocks = (pairs + per - 1) / per;
+    if (M <= 16) {
+        if (per > 8) gemm_bf16_skinny_kernel<1, 2, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
+        else gemm_bf16_skinny_kernel<1, 1, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
+    } else if (M > 32) {
+        if (per > 8) gemm_bf16_skinny_kernel<4, 2, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
+        else if (M <= 48) gemm_bf16_skinny_kernel<3, 1, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
+        else gemm_bf16_skinny_kernel<4, 1, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
+    } else {                                            // (two tiles of rows: four waves, as for the plain product)
+        if (per > 8) gemm_bf16_skinny_kernel<2, 2, 4, false, bf16_t, true><<<blocks, 4 * 64, 0, stream>>>(a);
+        else gemm_bf16_skinny_kernel<2, 1, 4, false, bf16_t, true><<<blocks, 4 * 64, 0, stream>>>(a);
+    }
     return li_launch_status();
 }
 
@@ -2285,6 +2515,17 @@ extern "C" int li_few_rows_preferred(int M, long N, long K) {
     return bytes <= FEW_ROWS_TWO_TILES_BYTES && (K <= FEW_ROWS_TWO_TILES_LONG_K || bytes <= FEW_ROWS_TWO_TILES_LONG_K_BYTES);
 }
 
+// 33 to 64 rows against a small matrix of short rows: three or four tiles of rows a block of the few-row kernel, K whole, rather than the
+// 64-row tiles with K in parts, whose sums go to memory and to a kernel that adds them up.  Every block reads all of x, so the line lies at the
+// length of a row.  Us, in parts / whole, with the norm behind it, and with the rotation and the page write: 48 rows of 1,536 x 1,536 10.1 / 9.2
+// and 9.5 / 6.2, 64 of 2,048 x 1,536 11.6 / 11.0 and 10.4 / 8.1, 64 of 896 x 896 11.7 / 8.1 and 11.0 / 6.0, 48 of 2,048 x 2,048 11.4 / 10.9 and
+// 10.8 / 8.1; 64 of 2,048 x 2,048 with the norm 11.8 / 12.4, of 3,584 x 3,584 15.8 / 18.
+#define FOUR_TILES_K 2048         // up to 48 rows,
+#define FOUR_TILES_LAST_K 1536    // above
+extern "C" int li_four_tiles_preferred(int M, long N, long K) {
+    return M > FEW_ROWS_TWO_TILES && M <= 64 && K % 8 == 0 && K <= (M <= 48 ? FOUR_TILES_K : FOUR_TILES_LAST_K) && N <= 16l * compute_units();
+}
+
 static bool mid_rows_take(int M, int N, int K) {
     return !li_few_rows_preferred(M, N, K) && M <= 64;
 }
@@ -2292,7 +2533,7 @@ static bool mid_rows_take(int M, int N, int K) {
 static int linear_mid_rows(const bf16_t* x, const bf16_t* w, const float* bias, void* out, int M, int N,
                            int K, int out_dtype, float accumulate, void* work, long work_bytes,
                            hipStream_t stream) {
-    if (!mid_rows_take(M, N, K) || K % 64 || (out_dtype != LI_F32 && out_dtype != LI_BF16)) return -1;
+    if (!mid_rows_take(M, N, K) || li_four_tiles_preferred(M, N, K) || K % 64 || (out_dtype != LI_F32 && out_dtype != LI_BF16)) return -1;
 #define LI_MID(BN, NS, TO, dst, b, acc, split) launch_dma<64, BN, 64, NS, false, TO>(x, w, b, (TO*)(dst), M, N, K, acc, stream, split)
     if ((N + 255) / 256 >= 128)
         return out_dtype == LI_F32 ? LI_MID(256, 3, float, out, bias, accumulate, 1) : LI_MID(256, 3, bf16_t, out, bias, accumulate, 1);
@@ -2351,7 +2592,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_rope_store_kernel(
     }
 }
 
-// Returns -1, having done nothing, where li_linear would not cut this product along K.
+// Up to 64 rows of some products take the few-row kernel with its epilogue (li_four_tiles_preferred), without parts and without `work`.
+// Returns -1, having done nothing, where neither that is the case nor li_linear would cut this product along K.
 extern "C" int li_linear_rope_store_parts(const void* x, const void* w, const float* bias, void* out, int M, int K,
                                           const float* cos, const float* sin, const int* slot_map, void* kc, void* vc,
                                           int nh, int nkv, int dh, int page_size, int num_pages,
@@ -2360,6 +2602,10 @@ extern "C" int li_linear_rope_store_parts(const void* x, const void* w, const fl
         (long)(nh + 2 * nkv) * dh > 0x7fffffffL)
         return LI_ERR_SIZE;
     const int N = (nh + 2 * nkv) * dh;
+    if (dh % 16 == 0 && li_four_tiles_preferred(M, N, K))                // (K whole: nothing to add up)
+        return launch_skinny_rope(SkinnyArgs{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, 0, cos, sin, slot_map,
+                                             (bf16_t*)kc, (bf16_t*)vc, nh, nkv, dh, page_size, num_pages,
+                                             nullptr, nullptr, nullptr, nullptr, 0, 0.f}, stream);
     if (li_few_rows_preferred(M, N, K) || K % 64) return -1;
     const long need = li_linear_work_bytes(M, N, K, LI_BF16);            // (0 where li_linear would not cut this product)
     if (need <= 0 || !work || work_bytes < need) return -1;
@@ -2531,6 +2777,17 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
     const size_t mn = (size_t)M * N;
     const int nsplit = (int)(need / (long)(mn * sizeof(float)));
     if (nsplit > 8) return -1;                      // (the adding-up kernel takes up to 8 parts)
+    if (li_four_tiles_preferred(M, N, K)) {         // K whole: the sum, then its norm
+        const int rc = li_linear_skinny(x, w, bias, out, M, N, K, LI_F32, factor, 0, stream);
+        if (rc != LI_OK) return rc;
+        if (xn_dtype == LI_BF16)
+            splitk_reduce_norm_kernel<bf16_t, REDUCE_NORM_NT, REDUCE_NORM_PER, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
+                nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (bf16_t*)xn);
+        else
+            splitk_reduce_norm_kernel<float, REDUCE_NORM_NT, REDUCE_NORM_PER, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
+                nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (float*)xn);
+        return li_launch_status();
+    }
     const int rc = M <= 64
         ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit)
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit);
@@ -2545,13 +2802,13 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
 }
 
 // out += factor * (x w^T + bias) (float32: the residual sum) and xn = tanh(alpha * out) * gamma + beta in one go: in the
-// epilogue of the few-row kernel (up to 32 rows, bfloat16 xn), or, where li_linear would cut K into parts, in the kernel
+// epilogue of the few-row kernel (up to 32 rows, or 64 against a small matrix; bfloat16 xn), or, where li_linear would cut K into parts, in the kernel
 // that adds the parts up.  Returns -1, having done nothing, where neither is the case.
 extern "C" int li_linear_tanh_norm(const void* x, const void* w, const float* bias, float* out, int M, int N, int K,
                                    void* work, long work_bytes, float factor, float alpha, const float* gamma,
                                    const float* beta, void* xn, int xn_dtype, hipStream_t stream) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 8 || factor == 0.f || !gamma || !beta || !xn || (xn_dtype != LI_BF16 && xn_dtype != LI_F32)) return -1;
-    if (M <= 32 && li_few_rows_preferred(M, N, K)) {
+    if ((M <= 32 && li_few_rows_preferred(M, N, K)) || (xn_dtype == LI_BF16 && li_four_tiles_preferred(M, N, K))) {
         if (xn_dtype != LI_BF16) return -1;
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, factor,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, gamma, (bf16_t*)xn, nullptr, nullptr, 0, 0.f};
@@ -2697,7 +2954,7 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
     if (M <= 0 || N <= 0 || K <= 0 || act < LI_ACT_RELU2 || act > LI_ACT_XIELU) return LI_ERR_SIZE;
     if (K % 8 || (M > 64 && (K % 64 || act != LI_ACT_RELU2))) return -1;
     const LiAct ep{act, a0, a1};
-    if (M <= 64 && (K % 64 || !mid_rows_take(M, N, K))) {
+    if (M <= 64 && (K % 64 || !mid_rows_take(M, N, K) || li_four_tiles_preferred(M, N, K))) {
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
         a.ep = ep;
@@ -2759,7 +3016,7 @@ extern "C" int li_linear_swiglu_f32(const float* x, const float* w, float* out, 
 // the activation as the product's epilogue, so the 2 I columns never go to memory.  bfloat16;
 // K a multiple of 8 for up to 64 rows, a multiple of 64 above.  act, limit: which form (see gated_form_known and gated_bf16).
 // row_parts (may be null): x is the xg of li_linear_residual_norm and these are its sq_parts, nparts of
-// them; every row's result is that of the RMS norm with eps (up to 16 rows).
+// them; every row's result is that of the RMS norm with eps (up to 32 rows).
 extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, int I, int K,
                                 const float* row_parts, int nparts, float eps, int act, float limit, hipStream_t stream) {
     if (!gated_form_known(act, limit)) return LI_ERR_SIZE;
@@ -2860,15 +3117,5 @@ extern "C" int li_linear_rope_store(const void* x, const void* w, const float* b
                  (bf16_t*)kc, (bf16_t*)vc, nh, nkv, dh, page_size, num_pages,
                  nullptr, nullptr, nullptr, row_parts, row_parts ? nparts : 0, eps};
     if (row_parts && (nparts <= 0 || nparts > SK_MAX_PARTS || eps < 0.f)) return LI_ERR_SIZE;
-    const int pairs = N / 2;
-    a.cols = balanced_per_block(pairs, 8);
-    const int per = a.cols ? a.cols : 8, blocks = (pairs + per - 1) / per;
-    if (M <= 16) {
-        if (per > 8) gemm_bf16_skinny_kernel<1, 2, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
-        else gemm_bf16_skinny_kernel<1, 1, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
-    } else {                                            // (two tiles of rows: four waves, as for the plain product)
-        if (per > 8) gemm_bf16_skinny_kernel<2, 2, 4, false, bf16_t, true><<<blocks, 4 * 64, 0, stream>>>(a);
-        else gemm_bf16_skinny_kernel<2, 1, 4, false, bf16_t, true><<<blocks, 4 * 64, 0, stream>>>(a);
-    }
-    return li_launch_status();
+    return launch_skinny_rope(a, stream);
 }

@@ -1170,6 +1170,11 @@ def few_rows_preferred(m: int, n: int, k: int) -> bool:
     return bool(f(int(m), int(n), int(k)))
 
 
+def four_tiles_preferred(m: int, n: int, k: int) -> bool:
+    """Whether 33 to 64 rows against a matrix [n, k] take the few-row kernels too (the library's rule)."""
+    return bool(_lib_fn("gemm", "li_four_tiles_preferred", [c_int, c_long, c_long], c_int)(int(m), int(n), int(k)))
+
+
 class RowScale:
     """What the product after a fused RMS norm needs beside its rows: the shares of the rows' sums
     of squares [nparts * R] float32 (R = 16 for up to 16 rows, 32 above) and the norm's eps."""
@@ -1413,16 +1418,17 @@ def linear_rope_store(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Ten
 def linear_rope_store_parts(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                             nh: int, nkv: int, dh: int, cos: torch.Tensor, sin: torch.Tensor,
                             slot_map: torch.Tensor, k: torch.Tensor, v: torch.Tensor, page_size: int, ws) -> bool:
-    """The same result as `linear_rope_store` for the rows of a large decoding batch, where the
-    packed projection is cut along K anyway: the kernel that adds the parts up rotates and writes
-    the pages.  Returns False, having done nothing, where `linear` would not cut this product."""
+    """The same result as `linear_rope_store` for the rows of a large decoding batch: 33 to 64 rows against a small matrix
+    (`four_tiles_preferred`) in the product's epilogue, else, where the packed projection is cut along K anyway, in the kernel
+    that adds the parts up.  Returns False, having done nothing, where neither is the case."""
     _gpu(x, w, bias, out, cos, sin, slot_map, k, v)
     if ws is None or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16 or 2 * cos.shape[1] != dh:
         return False
     m, kk = x.shape
     n = (nh + 2 * nkv) * dh
-    need = _work_bytes(m, n, kk, _DT[x.dtype])
-    if not need:
+    whole = dh % 16 == 0 and four_tiles_preferred(m, n, kk)
+    need = 0 if whole else _work_bytes(m, n, kk, _DT[x.dtype])
+    if not need and not whole:
         return False
     _chk(w.shape == (n, kk) and out.shape == (m, n), "linear_rope_store_parts: shapes do not fit")
     _chk(x.is_contiguous() and w.is_contiguous() and out.is_contiguous(), "linear_rope_store_parts: contiguous operands")
@@ -1434,12 +1440,12 @@ def linear_rope_store_parts(x: torch.Tensor, w: torch.Tensor, bias: Optional[tor
          and sin.dtype is torch.float32 and cos.is_contiguous() and sin.is_contiguous(), "linear_rope_store_parts: tables")
     _chk(slot_map.dtype is torch.int32 and slot_map.numel() == m and slot_map.is_contiguous(),
          "linear_rope_store_parts: slot_map")
-    if m <= SKINNY_MAX_ROWS:                # one size for all row counts of a decode batch: the buffer does not move
+    if need and m <= SKINNY_MAX_ROWS:       # one size for all row counts of a decode batch: the buffer does not move
         need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)
-    buf = ws.buffer("gemm.parts", (need // 4,), torch.float32)
+    buf = ws.buffer("gemm.parts", (need // 4,), torch.float32) if need else None
     return _try("gemm", "li_linear_rope_store_parts", x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(), out.data_ptr(), m, kk,
                 cos.data_ptr(), sin.data_ptr(), slot_map.data_ptr(), k.data_ptr(), v.data_ptr(), nh, nkv, dh, page_size,
-                k.shape[0], buf.data_ptr(), buf.numel() * 4)
+                k.shape[0], 0 if buf is None else buf.data_ptr(), 0 if buf is None else buf.numel() * 4)
 
 
 # ----------------------------------------------------------------- attention

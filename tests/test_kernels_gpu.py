@@ -333,6 +333,84 @@ def test_float32_linear_of_few_rows_and_columns(ops, m, n, k, bias, factor):
     assert rel(out, y) < 4 * math.sqrt(k) * 2.0 ** -24         # (sums of k float32 products)
 
 
+@pytest.mark.parametrize("m", [1, 2, 3, 4])
+@pytest.mark.parametrize("n,k", [
+    (5, 64), (200, 448),                 # fewer units of 64 than waves: some waves have none
+    (897, 512), (1536, 2048),            # up to four units a wave, a ragged last block; the longest rows of a wide matrix
+    (5000, 1088), (9000, 192),           # more columns than a round of blocks
+    (300, 2112), (70, 5120),             # five to ten units a wave at once
+    (33, 5184), (300, 8960),             # ... and in rounds of four: a last round of one unit, of two
+])
+def test_products_of_one_to_four_rows(ops, m, n, k):
+    g = torch.Generator().manual_seed(81)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g) / math.sqrt(k)).to(torch.bfloat16)
+    b, base = torch.randn(n, generator=g), torch.randn(m, n, generator=g)
+    y = x.double().numpy() @ w.double().numpy().T + b.double().numpy()
+    bound = 4 * math.sqrt(k) * 2.0 ** -24                       # sums of k float32 products
+    plain = torch.full((m, n), float("nan"), device=DEV)
+    ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), plain)
+    assert rel(plain, y) < bound
+    added = base.to(DEV)
+    ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), added, True, factor=0.5)
+    assert rel(added, base.double().numpy() + 0.5 * y) < bound
+    short = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), short)
+    assert rel(short, y) < 2.0 ** -8
+    if n % 8 == 0:
+        assert ops.linear_act(x.to(DEV), w.to(DEV), b.to(DEV), short, "relu2")
+        assert rel(short, np.maximum(y, 0) ** 2) < 2.0 ** -8
+    # a value that is not finite stays with its row
+    x[m - 1, k - 1] = float("inf")
+    ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), plain)
+    assert rel(plain[:m - 1], y[:m - 1]) < bound if m > 1 else True
+    assert not torch.isfinite(plain[m - 1]).any()
+
+
+@pytest.mark.parametrize("m", [33, 48, 49, 64])
+@pytest.mark.parametrize("n,k", [(64, 512), (1536, 1536), (1100, 1032), (4096, 1024), (2048, 2048)])      # the last one up to 48 rows only
+def test_products_of_33_to_64_rows_against_small_matrices(ops, m, n, k):
+    assert ops.four_tiles_preferred(m, n, k) == (m <= 48 or k <= 1536)
+    g = torch.Generator().manual_seed(82)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g) / math.sqrt(k)).to(torch.bfloat16)
+    b, base = torch.randn(n, generator=g), torch.randn(m, n, generator=g) * torch.logspace(-2, 2, m)[:, None]
+    gamma, beta, eps = torch.rand(n, generator=g) + 0.5, torch.randn(n, generator=g), 1e-5
+    y = base.double().numpy() + x.double().numpy() @ w.double().numpy().T + b.double().numpy()
+    bound = 4 * math.sqrt(k) * 2.0 ** -24
+    alone, xn = base.to(DEV), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), alone, True, ws=_Lender())
+    for i in range(m):
+        assert rel(alone[i], y[i]) < bound, i
+    out = base.to(DEV)
+    if ops.linear_then_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, gamma.to(DEV), eps, xn, _Lender()):
+        assert torch.equal(out, alone)
+        ref = plain_impl.rms_norm(y, gamma.double().numpy(), eps)
+        for i in range(m):
+            assert rel(xn[i], ref[i]) < 8e-3, i
+    out = base.to(DEV)
+    if ops.linear_tanh_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, 0.7, gamma.to(DEV), beta.to(DEV), xn, _Lender()):
+        assert rel(out, y) < bound and rel(xn, np.tanh(0.7 * y) * gamma.double().numpy() + beta.double().numpy()) < 8e-3
+    # the packed projection with rotary encoding and page write, in one launch
+    if n % 64 == 0 and n >= 256:
+        nkv, dh, page = 1, 64, 16
+        nh = n // dh - 2
+        pos = torch.randint(0, 3000, (m,), generator=g, dtype=torch.int32)
+        slots = torch.randperm(5 * page, generator=g)[:m].to(torch.int32)
+        cos, sin = torch.empty(m, dh // 2, device=DEV), torch.empty(m, dh // 2, device=DEV)
+        ops.rope_table(pos.to(DEV), 1e6, dh, cos, sin)
+        kc = torch.zeros((5, nkv, page, dh), dtype=torch.bfloat16, device=DEV)
+        vc, q = torch.zeros_like(kc), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert ops.linear_rope_store_parts(x.to(DEV), w.to(DEV), b.to(DEV), q, nh, nkv, dh, cos, sin, slots.to(DEV), kc, vc, page, _Lender())
+        yq = (y - base.double().numpy()).reshape(m, nh + 2 * nkv, dh)
+        ref = np.concatenate([plain_impl.rope_neox(yq[:, :nh + nkv], pos.numpy(), 1e6), yq[:, nh + nkv:]], axis=1)
+        assert rel(q, ref.reshape(m, n)) < 5e-3
+        qv = q.cpu().view(m, nh + 2 * nkv, dh)
+        for i in range(m):
+            sl = int(slots[i])
+            assert torch.equal(kc[sl // page, :, sl % page].cpu(), qv[i, nh:nh + nkv]) and torch.equal(vc[sl // page, :, sl % page].cpu(), qv[i, nh + nkv:])
+
+
 @pytest.mark.parametrize("m,n,k,bias,taken", [
     (64, 3584, 18944, False, True),      # a decoding batch of 64 at the 7B sizes
     (40, 200, 1024, True, True),
