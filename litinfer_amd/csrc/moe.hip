@@ -3,9 +3,7 @@
 // the products of every tile's rows with its expert's matrix, and the weighted sum back into the stream.
 // Nothing here returns to the host: the numbers of rows an expert gets stay on the device, and the launches are
 // sized by what a step can have at most.
-#include "common.h"
-
-#include <type_traits>
+#include "few_rows.h"
 
 #define MOE_TILE 32            // rows of one expert that a tile holds
 #define MOE_BIG_TILE 64        // ... where experts get hundreds of rows each (a prompt's portion): the tiles of the LDS kernel,
@@ -27,7 +25,17 @@ template <typename T> struct RouteVec;
 template <> struct RouteVec<float> { static constexpr int N = 4; };
 template <> struct RouteVec<bf16_t> { static constexpr int N = 8; };
 
-// 16 bytes of a matrix row against the row in LDS
+// 16 bytes of a matrix row against the row in LDS, or against 16 bytes of it (the same additions in the same order)
+__device__ __forceinline__ float route_dot16(const uint4 r, const uint4 x) {
+    const uint32_t u[4] = {r.x, r.y, r.z, r.w}, v[4] = {x.x, x.y, x.z, x.w};
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        s = fmaf(__uint_as_float(u[i] << 16), __uint_as_float(v[i] << 16), s);
+        s = fmaf(__uint_as_float(u[i] & 0xffff0000u), __uint_as_float(v[i] & 0xffff0000u), s);
+    }
+    return s;
+}
 __device__ __forceinline__ float route_dot16(const uint4 r, const float* xs, const float*) {
     return fmaf(__uint_as_float(r.x), xs[0], fmaf(__uint_as_float(r.y), xs[1], fmaf(__uint_as_float(r.z), xs[2], __uint_as_float(r.w) * xs[3])));
 }
@@ -44,6 +52,7 @@ __device__ __forceinline__ float route_dot16(const uint4 r, const float* xs, con
 
 // What a plan is made of (see moe_plan_kernel below); plan null: none.
 struct MoePlanOut { int* plan; int* row_token; int* pair_row; float* row_wt; int* count; int max_tiles, tile_rows, experts; };
+#define MOE_PLAN_HELD 4
 #define MOE_PLAN_EXPERTS 64       // experts up to which the router makes the plan: one a lane
 
 // A wave's fence: what its lanes wrote to LDS is there for its other lanes
@@ -60,7 +69,19 @@ __device__ __forceinline__ void moe_plan_by_wave(const MoePlanOut& p, const int*
     const int lane = threadIdx.x & 63;
     cursor[lane] = 0;
     LI_WAVE_LDS()
-    for (int i = lane; i < pairs; i += 64) {
+    // the first 256 choices and weights wait in registers: one trip to memory
+    int held[MOE_PLAN_HELD];
+    float held_wt[MOE_PLAN_HELD];
+#pragma unroll
+    for (int q = 0; q < MOE_PLAN_HELD; ++q) {
+        const int i = lane + 64 * q < pairs ? lane + 64 * q : 0;
+        held[q] = __hip_atomic_load(idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        held_wt[q] = __hip_atomic_load(wt + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int q = 0; q < MOE_PLAN_HELD; ++q)
+        if (lane + 64 * q < pairs && held[q] >= 0 && held[q] < p.experts) atomicAdd(&cursor[held[q]], 1);
+    for (int i = lane + 64 * MOE_PLAN_HELD; i < pairs; i += 64) {
         const int e = __hip_atomic_load(idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (e >= 0 && e < p.experts) atomicAdd(&cursor[e], 1);
     }
@@ -81,45 +102,74 @@ __device__ __forceinline__ void moe_plan_by_wave(const MoePlanOut& p, const int*
     if (lane == 63) { p.plan[0] = tiles_upto < p.max_tiles ? tiles_upto : p.max_tiles; p.plan[1] = rows_upto; p.plan[2] = p.plan[3] = 0; }
     cursor[lane] = start;
     LI_WAVE_LDS()
-    for (int i = lane; i < pairs; i += 64) {
-        const int e = __hip_atomic_load(idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    auto place = [&](int i, int e, float weight) {
         if (e >= 0 && e < p.experts) {
             const int row = atomicAdd(&cursor[e], 1);
             p.pair_row[i] = row;
             p.row_token[row] = i / top;
-            if (p.row_wt) p.row_wt[row] = __hip_atomic_load(wt + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (p.row_wt) p.row_wt[row] = weight;
         } else {
             p.pair_row[i] = -1;
         }
-    }
+    };
+#pragma unroll
+    for (int q = 0; q < MOE_PLAN_HELD; ++q)
+        if (lane + 64 * q < pairs) place(lane + 64 * q, held[q], held_wt[q]);
+    for (int i = lane + 64 * MOE_PLAN_HELD; i < pairs; i += 64)
+        place(i, __hip_atomic_load(idx + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), __hip_atomic_load(wt + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
 }
 
-// Few tokens: what bounds it is a chain of trips to memory (the row, a matrix row, the pick), so a wave asks for its first two
-// matrix rows, where they are short enough to wait in registers, before the token's row has come.
+// Few tokens: what bounds it is a chain of trips to memory (the row, a matrix row, the pick, the plan), so a wave asks for its first
+// matrix rows, where they are short enough to wait in registers, before the token's row has come; up to 64 outputs are picked at once, and
+// one token's plan is made of what the wave knows (8 tokens, 16 outputs, 4 choices 12.0 -> 10.0 us).
+template <typename TX, typename TW>
+struct MoeRoute {
+    const TX* x;
+    long x_stride;
+    const TW* wr;
+    const float* br;
+    const TW* wg;
+    int* idx;
+    float* wt;
+    float* gate;
+    int T, K, E, top, vec, mode_flags;
+    const float* corr;
+    int groups, keep;
+    MoePlanOut po;
+};
+
 template <typename TX, typename TW, int NT>
-__global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x, long x_stride, const TW* __restrict__ wr,
-                                                       const float* __restrict__ br, const TW* __restrict__ wg,
-                                                       int* __restrict__ idx, float* __restrict__ wt, float* __restrict__ gate,
-                                                       int K, int E, int top, int vec, int mode_flags,
-                                                       const float* __restrict__ corr, int groups, int keep, MoePlanOut po) {
-    const int mode = mode_flags & 3;
-    const bool group_max = mode_flags & 4, plain_weights = mode_flags & 8;
-    extern __shared__ __align__(16) float sm[];        // [K] the row, [E] the logits, [E] the scores, [groups] the groups' scores
+__device__ __forceinline__ void moe_route_token(const MoeRoute<TX, TW>& a, const int t, float* sm) {
+    const TX* __restrict__ x = a.x;
+    const TW* __restrict__ wr = a.wr;
+    const TW* __restrict__ wg = a.wg;
+    const float* __restrict__ br = a.br;
+    const float* __restrict__ corr = a.corr;
+    int* __restrict__ idx = a.idx;
+    float* __restrict__ wt = a.wt;
+    float* __restrict__ gate = a.gate;
+    const long x_stride = a.x_stride;
+    const int K = a.K, E = a.E, top = a.top, vec = a.vec, groups = a.groups, keep = a.keep;
+    const MoePlanOut& po = a.po;
+    const int mode = a.mode_flags & 3;
+    const bool group_max = a.mode_flags & 4, plain_weights = a.mode_flags & 8;
+    // sm: [K] the row, [E] the logits, [E] the scores, [groups] the groups' scores
     float* xs = sm;
     float* lg = sm + ((K + 3) & ~3);
     float* sc = lg + E;
     float* gs = sc + E;
-    const int t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const TX* row = x + (size_t)t * x_stride;
     constexpr int VE = RouteVec<TW>::N;
     constexpr int HELD = 4;                            // pieces of a matrix row that a lane holds
     const int n_rows = E + (wg ? 1 : 0);
-    const bool held = NT == 1024 && vec && K / VE <= 64 * HELD;
-    uint4 piece[2][HELD];
-    if constexpr (NT == 1024) {
+    const bool held = NT >= 512 && (vec & 1) && K / VE <= 64 * HELD;
+    constexpr int FIRST = NT >= 1024 ? 2 : 3;          // matrix rows that a wave asks for at once
+    uint4 piece[FIRST][HELD];
+    if constexpr (NT >= 512) {
         if (held) {
 #pragma unroll
-            for (int q = 0; q < 2; ++q) {
+            for (int q = 0; q < FIRST; ++q) {
                 const int e = w + q * (NT / 64) < n_rows ? w + q * (NT / 64) : 0;       // (never conditional: a row past the last reads the first)
                 const TW* wrow = e < E ? wr + (size_t)e * K : wg;
 #pragma unroll
@@ -130,39 +180,51 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
             }
         }
     }
-    for (int k = threadIdx.x; k < K; k += NT) xs[k] = load_as_float(row + k);
-    __syncthreads();
-    auto have = [&](int e, float s) {                  // a row's product, in parts by lane
-        s = wave_sum(s);
+    // Where row and matrix are bfloat16 and a wave holds all its matrix rows, every wave reads the row for itself beside them: it does not
+    // pass through LDS, and nobody waits for anybody before the logits are there.
+    const bool direct = sizeof(TX) == 2 && sizeof(TW) == 2 && held && (vec & 2) && n_rows <= FIRST * (NT / 64);
+    [[maybe_unused]] uint4 xp[HELD];
+    if (direct) {
+#pragma unroll
+        for (int i = 0; i < HELD; ++i) xp[i] = *reinterpret_cast<const uint4*>(row + (lane + 64 * i < K / VE ? lane + 64 * i : 0) * VE);
+    } else {
+        for (int k = threadIdx.x; k < K; k += NT) xs[k] = load_as_float(row + k);
+        __syncthreads();
+    }
+    auto have = [&](int e, float s) {                  // a row's product
         if (lane == 0) {
             if (e < E) lg[e] = s + (br ? br[e] : 0.f);
             else gate[t] = 1.0f / (1.0f + expf(-s));
         }
     };
     int e = w;
-    if constexpr (NT == 1024) {                        // (rows of their own: asked for in the loop below, they made every other row 0.2 us longer)
+    if constexpr (NT >= 512) {                         // (rows of their own: asked for in the loop below, they made every other row 0.2 us longer)
         if (held) {
+            float s[FIRST];
 #pragma unroll
-            for (int q = 0; q < 2; ++q, e += NT / 64) {
-                if (e >= n_rows) break;
-                float s = 0.f;
+            for (int q = 0; q < FIRST; ++q) {
+                s[q] = 0.f;
 #pragma unroll
                 for (int i = 0; i < HELD; ++i)
-                    if (lane + 64 * i < K / VE) s += route_dot16(piece[q][i], xs + (lane + 64 * i) * VE, (const TW*)nullptr);
-                have(e, s);
+                    if (lane + 64 * i < K / VE) s[q] += direct ? route_dot16(piece[q][i], xp[i]) : route_dot16(piece[q][i], xs + (lane + 64 * i) * VE, (const TW*)nullptr);
             }
+#pragma unroll
+            for (int q = 0; q < FIRST; ++q) s[q] = wave_sum(s[q]);
+#pragma unroll
+            for (int q = 0; q < FIRST; ++q, e += NT / 64)
+                if (e < n_rows) have(e, s[q]);
         }
     }
     for (; e < n_rows; e += NT / 64) {
         const TW* wrow = e < E ? wr + (size_t)e * K : wg;
         float s = 0.f;
-        if (vec) {                                     // 16 bytes a lane and turn, several turns on their way
+        if (vec & 1) {                                 // 16 bytes a lane and turn, several turns on their way
 #pragma unroll 4
             for (int i = lane; i < K / VE; i += 64) s += route_dot16(*reinterpret_cast<const uint4*>(wrow + (size_t)i * VE), xs + i * VE, (const TW*)nullptr);
         } else {
             for (int k = lane; k < K; k += 64) s = fmaf(load_as_float(wrow + k), xs[k], s);
         }
-        have(e, s);
+        have(e, wave_sum(s));
     }
     __syncthreads();
     if (w != 0) return;
@@ -214,9 +276,34 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         }
     }
-    // wave 0 picks: `top` rounds of a maximum over the logits that are left
     float chosen = 0.f, mx = 0.f, sum = 0.f;
     int mine = -1;
+    unsigned long long taken = 0;                      // (up to 64 router outputs: those that were chosen)
+    if (E <= 64) {
+        // An output a lane: its place is the number of those that go before it (a larger value, or an equal one and a lower number), all
+        // places at once, where rounds of a maximum took twelve exchanges between lanes a choice.  The values are compared as whole
+        // numbers of the same order (both zeros the same; what is no number before all others), so every place is some output's.
+        const float v = lane < E ? lg[lane] + 0.f : 0.f;
+        uint32_t key = __float_as_uint(v);
+        key = v != v ? 0xffffffffu : key & 0x80000000u ? ~key : key | 0x80000000u;
+        int place = 0;
+        for (int o = 0; o < E; ++o) {
+            const uint32_t other = __builtin_amdgcn_readlane(key, o);
+            place += other > key || (other == key && o < lane) ? 1 : 0;
+        }
+        if (lane >= E) place = 64;
+        taken = __ballot(place < top);
+        const float score = mode != 0 && lane < E ? sc[lane] : 0.f;
+        mx = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), __ffsll((long long)__ballot(place == 0)) - 1));
+        const float ex = mode != 0 ? score : expf(v - mx);
+        for (int r = 0; r < top; ++r) {
+            const int from = __ffsll((long long)__ballot(place == r)) - 1;
+            const float one = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(ex), from));
+            sum += one;
+            if (lane == r) { mine = from; chosen = one; }
+        }
+    } else
+    // wave 0 picks: `top` rounds of a maximum over the logits that are left
     for (int r = 0; r < top; ++r) {
         float best = -INFINITY;
         int bi = 0x7fffffff;
@@ -246,6 +333,25 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
         if (lane < top) { idx[(size_t)t * top + lane] = mine; wt[(size_t)t * top + lane] = share; }
         return;
     }
+    if (a.T == 1 && E <= 64) {
+        // one token's plan: a tile of one row for every expert that was chosen, from what the lanes know
+        if (lane < top) { idx[lane] = mine; wt[lane] = share; }
+        taken &= po.experts < 64 ? (1ull << po.experts) - 1 : ~0ull;
+        const int n = __popcll(taken);
+        if (lane < top) {
+            const bool real = mine < po.experts;
+            const int at = __popcll(taken & ((1ull << (mine & 63)) - 1));
+            po.pair_row[lane] = real ? at : -1;
+            if (real) {
+                po.row_token[at] = 0;
+                if (po.row_wt) po.row_wt[at] = share;
+                int* tile = po.plan + 4 + 4 * at;
+                if (at < po.max_tiles) { tile[0] = mine; tile[1] = at; tile[2] = 1; tile[3] = 0; }
+            }
+        }
+        if (lane == 63) { po.plan[0] = n < po.max_tiles ? n : po.max_tiles; po.plan[1] = n; po.plan[2] = po.plan[3] = 0; }
+        return;
+    }
     // The choices go through to memory; the block counts itself there, and the one that completes the count makes the plan.
     // Nobody waits for anybody, and the count is left at zero.
     if (lane < top) {
@@ -253,13 +359,19 @@ __global__ __launch_bounds__(NT) void moe_route_kernel(const TX* __restrict__ x,
         __hip_atomic_store(wt + (size_t)t * top + lane, share, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    if (gridDim.x > 1) {
+    if (a.T > 1) {
         int before = 0;
         if (lane == 0) before = atomicAdd(po.count, 1);
-        if (__builtin_amdgcn_readfirstlane(before) != (int)gridDim.x - 1) return;
+        if (__builtin_amdgcn_readfirstlane(before) != a.T - 1) return;
         if (lane == 0) atomicExch(po.count, 0);
     }
-    moe_plan_by_wave(po, idx, wt, gridDim.x * top, top, reinterpret_cast<int*>(sm));
+    moe_plan_by_wave(po, idx, wt, a.T * top, top, reinterpret_cast<int*>(sm));
+}
+
+template <typename TX, typename TW, int NT>
+__global__ __launch_bounds__(NT) void moe_route_kernel(MoeRoute<TX, TW> a) {
+    extern __shared__ __align__(16) float sm[];
+    moe_route_token<TX, TW, NT>(a, blockIdx.x, sm);
 }
 
 // plan (may be null) and what follows: the plan of the step as well (li_moe_plan's, over `experts` of the E router outputs), up to 128
@@ -279,12 +391,13 @@ extern "C" int li_moe_route(const void* x, int x_dtype, long x_stride, const voi
     const size_t lds = (size_t)(((K + 3) & ~3) + 2 * E + groups) * 4;
     // whole 16-byte pieces of every matrix row (the gate row included)
     const int ve = w_dtype == LI_F32 ? 4 : 8;
-    const int vec = K % ve == 0 && ((uintptr_t)wr % 16) == 0 && (!wg || ((uintptr_t)wg % 16) == 0);
+    const int vec = (K % ve == 0 && ((uintptr_t)wr % 16) == 0 && (!wg || ((uintptr_t)wg % 16) == 0)) | (x_dtype == LI_BF16 && x_stride % 8 == 0 && (uintptr_t)x % 16 == 0) << 1;
     // few tokens: sixteen waves share a token's experts, so that a wave has one or two rows to go through
 #define MR(TX, TW)                                                                                                                \
     {                                                                                                                             \
-        if (T <= 128) moe_route_kernel<TX, TW, 1024><<<T, 1024, lds, stream>>>((const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, K, E, top, vec, mode, corr, groups, keep, po); \
-        else moe_route_kernel<TX, TW, 256><<<T, 256, lds, stream>>>((const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, K, E, top, vec, mode, corr, groups, keep, po);       \
+        const MoeRoute<TX, TW> a{(const TX*)x, x_stride, (const TW*)wr, br, (const TW*)wg, idx, wt, gate, T, K, E, top, vec, mode, corr, groups, keep, po}; \
+        if (T <= 128) moe_route_kernel<TX, TW, 1024><<<T, 1024, lds, stream>>>(a);                                               \
+        else moe_route_kernel<TX, TW, 256><<<T, 256, lds, stream>>>(a);                                                          \
     }
     if (x_dtype == LI_F32 && w_dtype == LI_F32) MR(float, float)
     else if (x_dtype == LI_BF16 && w_dtype == LI_BF16) MR(bf16_t, bf16_t)
@@ -637,22 +750,83 @@ __global__ __launch_bounds__(256) void moe_linear_wide_kernel(const TA* __restri
 // rows, so the product is a matrix-vector product a row.  A wave owns four outputs and walks their matrix rows in
 // 16-byte pieces, 64 lanes side by side along K (a kilobyte of a row at a time, all four rows' pieces asked for
 // together), against up to four of the tile's rows at a time; sums in float32, lanes added up at the end.
+// Up to MOE_VECTOR_ROWS rows a wave owns two (twice the blocks, spread more evenly over the compute units), and a tile's one row against
+// matrices of up to MR_HELD pieces a lane is one trip to memory: all of the wave's pieces are asked for before any is multiplied.
+// (Two rows of 2,240 x 1,536 7.9 -> 5.9 us, of 1,536 x 2,240 8.4 -> 6.1, an empty launch being 1.6.)
 #define MR_OUT 4
+#define MR_OUT_FEW 2
 #define MR_ROWS 4
+#define MR_HELD 5
 
-template <bool EXT, typename TO>
-__global__ __launch_bounds__(256) void moe_linear_rows_kernel(const bf16_t* __restrict__ a, long a_stride, const int* __restrict__ row_token,
-                                                              const bf16_t* __restrict__ w, const int* __restrict__ plan,
-                                                              TO* __restrict__ out, long out_stride, int n_out, int K, MoeEpilogue ep) {
-    const int tile = blockIdx.y;              // (columns first: neighbouring blocks go to different XCDs, and each XCD gets a share of every expert)
-    if (tile >= plan[0]) return;
-    const int e = plan[4 + 4 * tile], r0 = plan[5 + 4 * tile], nr = plan[6 + 4 * tile];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int j0 = (blockIdx.x * 4 + wv) * MR_OUT;
-    if (j0 >= n_out) return;
-    const bf16_t* wrow[MR_OUT];
+// The operands of a product by tile, bfloat16 rows and matrices
+template <typename TO>
+struct MoeLinear { const bf16_t* a; long a_stride; const int* row_token; const bf16_t* w; const int* plan; TO* out; long out_stride; int n_out, K; MoeEpilogue ep; };
+
+template <bool EXT, typename TO, int OUT>
+__device__ __forceinline__ void moe_linear_rows_wave(const MoeLinear<TO>& p, const int tile, const int j0) {
+    const bf16_t* __restrict__ a = p.a;
+    const bf16_t* __restrict__ w = p.w;
+    const int* __restrict__ plan = p.plan;
+    const int* __restrict__ row_token = p.row_token;
+    TO* __restrict__ out = p.out;
+    const long a_stride = p.a_stride, out_stride = p.out_stride;
+    const int n_out = p.n_out, K = p.K;
+    const MoeEpilogue& ep = p.ep;
+    const int tiles = plan[0], e = plan[4 + 4 * tile], r0 = plan[5 + 4 * tile], nr = plan[6 + 4 * tile];      // (one trip: a tile past the last has its place)
+    asm volatile("" ::"s"(tiles), "s"(e), "s"(r0), "s"(nr));
+    const int lane = threadIdx.x & 63;
+    if (tile >= tiles || j0 >= n_out) return;
+    const bf16_t* wrow[OUT];
 #pragma unroll
-    for (int j = 0; j < MR_OUT; ++j) wrow[j] = w + ((size_t)e * n_out + (j0 + j < n_out ? j0 + j : n_out - 1)) * K;
+    for (int j = 0; j < OUT; ++j) wrow[j] = w + ((size_t)e * n_out + (j0 + j < n_out ? j0 + j : n_out - 1)) * K;
+    // what becomes of one row's sums, in lane 0
+    auto finish = [&](int row, const float (*acc)[MR_ROWS], int r) {
+        TO* orow = out + (size_t)row * out_stride;
+        const float factor = moe_row_factor<EXT>(ep, row);
+        if (moe_is_gated(ep.act)) {                    // (gate, up) pairs: n_out is even and j0 a multiple of OUT
+#pragma unroll
+            for (int j = 0; j < OUT; j += 2)
+                if (j0 + j < n_out) store_from_float(orow + ((j0 + j) >> 1), moe_gated(acc[j][r] * factor, acc[j + 1][r] * factor, ep.act, ep.limit));
+            return;
+        }
+#pragma unroll
+        for (int j = 0; j < OUT; ++j)
+            if (j0 + j < n_out) store_from_float(orow + j0 + j, moe_act1<EXT>(acc[j][r] * factor, ep.act));
+    };
+    if (nr == 1 && K <= MR_HELD * 512) {               // one row: all the wave multiplies is asked for at once
+        const int at = (row_token ? row_token[r0] : r0), last = K / 8 - 1;
+        const bf16_t* xrow = a + (size_t)at * a_stride;
+        uint4 wp[MR_HELD][OUT], xp[MR_HELD];
+#pragma unroll
+        for (int i = 0; i < MR_HELD; ++i) {
+            if (64 * i > last) continue;               // (the wave's own question, and nothing else writes these registers: no wait at its end)
+            const int c = lane + 64 * i < last ? lane + 64 * i : last;
+#pragma unroll
+            for (int j = 0; j < OUT; ++j) wp[i][j] = *reinterpret_cast<const uint4*>(wrow[j] + 8 * c);
+            xp[i] = *reinterpret_cast<const uint4*>(xrow + 8 * c);
+        }
+        float acc[OUT][MR_ROWS];
+#pragma unroll
+        for (int j = 0; j < OUT; ++j) acc[j][0] = 0.f;
+#pragma unroll
+        for (int i = 0; i < MR_HELD; ++i) {
+            if (64 * i > last) continue;
+            const bool mine = lane + 64 * i <= last;
+#pragma unroll
+            for (int j = 0; j < OUT; ++j) {
+                const uint32_t u[4] = {wp[i][j].x, wp[i][j].y, wp[i][j].z, wp[i][j].w}, v[4] = {xp[i].x, xp[i].y, xp[i].z, xp[i].w};
+                float s = acc[j][0];
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    s = fmaf(__uint_as_float(u[q] & 0xffff0000u), __uint_as_float(v[q] & 0xffff0000u), fmaf(__uint_as_float(u[q] << 16), __uint_as_float(v[q] << 16), s));
+                acc[j][0] = mine ? s : acc[j][0];
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < OUT; ++j) acc[j][0] = wave_sum(acc[j][0]);
+        if (lane == 0) finish(r0, acc, 0);
+        return;
+    }
     for (int rc = 0; rc < nr; rc += MR_ROWS) {
         const bf16_t* xrow[MR_ROWS];
 #pragma unroll
@@ -660,24 +834,24 @@ __global__ __launch_bounds__(256) void moe_linear_rows_kernel(const bf16_t* __re
             const int row = r0 + (rc + r < nr ? rc + r : nr - 1);
             xrow[r] = a + (size_t)(row_token ? row_token[row] : row) * a_stride;
         }
-        float acc[MR_OUT][MR_ROWS];
+        float acc[OUT][MR_ROWS];
 #pragma unroll
-        for (int j = 0; j < MR_OUT; ++j)
+        for (int j = 0; j < OUT; ++j)
 #pragma unroll
             for (int r = 0; r < MR_ROWS; ++r) acc[j][r] = 0.f;
         // the next turn's pieces of the matrix rows are on their way while this one's are multiplied (past the end: the last
         // turn's again, not used); a load is not moved past the empty statement behind it
-        uint4 wp[MR_OUT], wn[MR_OUT];
+        uint4 wp[OUT], wn[OUT];
         const int i_last = K / 8 - 1;
 #pragma unroll
-        for (int j = 0; j < MR_OUT; ++j) wp[j] = *reinterpret_cast<const uint4*>(wrow[j] + 8 * (lane < i_last ? lane : i_last));
+        for (int j = 0; j < OUT; ++j) wp[j] = *reinterpret_cast<const uint4*>(wrow[j] + 8 * (lane < i_last ? lane : i_last));
         for (int i = lane; i < K / 8; i += 64) {
             uint4 xp[MR_ROWS];
 #pragma unroll
             for (int r = 0; r < MR_ROWS; ++r) xp[r] = *reinterpret_cast<const uint4*>(xrow[r] + 8 * i);
             const int in = i + 64 < i_last ? i + 64 : i_last;
 #pragma unroll
-            for (int j = 0; j < MR_OUT; ++j) wn[j] = *reinterpret_cast<const uint4*>(wrow[j] + 8 * in);
+            for (int j = 0; j < OUT; ++j) wn[j] = *reinterpret_cast<const uint4*>(wrow[j] + 8 * in);
             asm volatile("" ::: "memory");
             float xf[MR_ROWS][8];
 #pragma unroll
@@ -687,7 +861,7 @@ __global__ __launch_bounds__(256) void moe_linear_rows_kernel(const bf16_t* __re
                 for (int q = 0; q < 4; ++q) { xf[r][2 * q] = __uint_as_float(u[q] << 16); xf[r][2 * q + 1] = __uint_as_float(u[q] & 0xffff0000u); }
             }
 #pragma unroll
-            for (int j = 0; j < MR_OUT; ++j) {
+            for (int j = 0; j < OUT; ++j) {
                 const uint32_t u[4] = {wp[j].x, wp[j].y, wp[j].z, wp[j].w};
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
@@ -697,33 +871,25 @@ __global__ __launch_bounds__(256) void moe_linear_rows_kernel(const bf16_t* __re
                 }
             }
 #pragma unroll
-            for (int j = 0; j < MR_OUT; ++j) wp[j] = wn[j];
+            for (int j = 0; j < OUT; ++j) wp[j] = wn[j];
         }
 #pragma unroll
-        for (int j = 0; j < MR_OUT; ++j)
+        for (int j = 0; j < OUT; ++j)
 #pragma unroll
             for (int r = 0; r < MR_ROWS; ++r)
                 if (rc + r < nr) acc[j][r] = wave_sum(acc[j][r]);
         if (lane == 0) {
 #pragma unroll
-            for (int r = 0; r < MR_ROWS; ++r) {
-                if (rc + r >= nr) continue;
-                TO* orow = out + (size_t)(r0 + rc + r) * out_stride;
-                const float factor = moe_row_factor<EXT>(ep, r0 + rc + r);
-                if (moe_is_gated(ep.act)) {            // (gate, up) pairs: n_out is even and j0 a multiple of 4
-#pragma unroll
-                    for (int j = 0; j < MR_OUT; j += 2)
-                        if (j0 + j < n_out) store_from_float(orow + ((j0 + j) >> 1), moe_gated(acc[j][r] * factor, acc[j + 1][r] * factor, ep.act, ep.limit));
-                    continue;
-                }
-#pragma unroll
-                for (int j = 0; j < MR_OUT; ++j) {
-                    if (j0 + j >= n_out) continue;
-                    store_from_float(orow + j0 + j, moe_act1<EXT>(acc[j][r] * factor, ep.act));
-                }
-            }
+            for (int r = 0; r < MR_ROWS; ++r)
+                if (rc + r < nr) finish(r0 + rc + r, acc, r);
         }
     }
+}
+
+template <bool EXT, typename TO, int OUT>
+__global__ __launch_bounds__(256) void moe_linear_rows_kernel(MoeLinear<TO> p) {
+    // (columns first: neighbouring blocks go to different XCDs, and each XCD gets a share of every expert)
+    moe_linear_rows_wave<EXT, TO, OUT>(p, blockIdx.y, (blockIdx.x * 4 + (threadIdx.x >> 6)) * OUT);
 }
 
 // A decoding step of a batch: few rows an expert, and every tile streams its expert's matrix, so the product is bound by
@@ -745,8 +911,9 @@ __global__ __launch_bounds__(256) void moe_linear_stream_kernel(const bf16_t* __
                                                                 TO* __restrict__ out, long out_stride, int n_out, int K, MoeEpilogue ep) {
     constexpr int WAVES = 4;
     const int tile = blockIdx.y;              // (columns first: see the kernel of few rows)
-    if (tile >= plan[0]) return;
-    const int e = plan[4 + 4 * tile], r0 = plan[5 + 4 * tile], nr = plan[6 + 4 * tile];
+    const int tiles = plan[0], e = plan[4 + 4 * tile], r0 = plan[5 + 4 * tile], nr = plan[6 + 4 * tile];      // (one trip: see the kernel of few rows)
+    asm volatile("" ::"s"(tiles), "s"(e), "s"(r0), "s"(nr));
+    if (tile >= tiles) return;
     __shared__ moe_f32x4 red[WAVES][NT][64];
     __shared__ __attribute__((aligned(16))) uint16_t xs_all[WAVES][16 * MS_CHUNK];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -1025,11 +1192,12 @@ static int moe_linear_launch(const void* a, int a_dtype, long a_stride, const in
     }
     // a handful of rows in all: a matrix-vector product a row
     if (rows <= MOE_FEW_ROWS && pieces) {
-        const dim3 grid((n_out + 4 * MR_OUT - 1) / (4 * MR_OUT), max_tiles);
-        if (out_dtype == LI_BF16)
-            moe_linear_rows_kernel<EXT, bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (bf16_t*)out, out_stride, n_out, K, ep);
-        else
-            moe_linear_rows_kernel<EXT, float><<<grid, 256, 0, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (float*)out, out_stride, n_out, K, ep);
+        const int wave_out = rows <= MOE_VECTOR_ROWS ? MR_OUT_FEW : MR_OUT;
+        const dim3 grid((n_out + 4 * wave_out - 1) / (4 * wave_out), max_tiles);
+#define MF(TO, OUT) moe_linear_rows_kernel<EXT, TO, OUT><<<grid, 256, 0, stream>>>(MoeLinear<TO>{(const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (TO*)out, out_stride, n_out, K, ep})
+        if (out_dtype == LI_BF16) { if (wave_out == MR_OUT) MF(bf16_t, MR_OUT); else MF(bf16_t, MR_OUT_FEW); }
+        else { if (wave_out == MR_OUT) MF(float, MR_OUT); else MF(float, MR_OUT_FEW); }
+#undef MF
         return li_launch_status();
     }
     if (w_dtype == LI_BF16 && K % 16 == 0 && n_out % 32 == 0 && a_stride % 8 == 0 && out_stride % 4 == 0 &&
@@ -1077,6 +1245,110 @@ extern "C" int li_moe_linear(const void* a, int a_dtype, long a_stride, const in
     if (act == 4 || row_wt)
         return moe_linear_launch<true>(a, a_dtype, a_stride, row_token, w, w_dtype, plan, max_tiles, out, out_dtype, out_stride, n_out, K, ep, tile_rows, rows, stream);
     return moe_linear_launch<false>(a, a_dtype, a_stride, row_token, w, w_dtype, plan, max_tiles, out, out_dtype, out_stride, n_out, K, ep, tile_rows, rows, stream);
+}
+
+// ------------------------------------------------------------------------------- the shared expert beside the routed ones
+// A decoding step's shared expert hangs on none of the router's choices, yet its two products were launches of their own behind the routed
+// ones: 5 to 9 us each, in which the chip waits for a first load and a drain.  Its first product goes with the router, which is a block a token
+// and leaves the chip idle, and its second with the routed experts' first: blocks of 512 threads, of which some take one and the rest the
+// other.  Which form the product beside takes (see few_rows.h): up to 4 rows rows_product, up to 16 and 32 one and two tiles of rows of
+// skinny_product, eight waves a block.
+// Left out of a recorded step (us, 16 experts of 2,240 x 1,536, a shared one of 4,480): one token, router 8.2 and first product 4.8 apart,
+// 8.0 together; routed 7.9 and shared 5.9 apart, 8.9 together; 32 tokens, router 8.8 and first product 9.2 apart, 10.9 together.  The second
+// pair only for rows few enough for the kernel of few rows: in blocks of 512 threads the streaming kernel had too few of them on a
+// unit (32 tokens, 23.5 and 8.2 apart, 37.1 together).
+#define MOE_BESIDE_NT 512
+#define MOE_BESIDE_ROWS 32
+enum { BESIDE_ROWS = 0, BESIDE_ONE_TILE = 1, BESIDE_TWO_TILES = 2 };
+template <int FORM> constexpr int beside_lds() {
+    return FORM == BESIDE_ROWS ? fr_lds_bytes(2) : FORM == BESIDE_ONE_TILE ? SkinnyLds<1, 1, 8, SK_CHUNK>::BYTES : SkinnyLds<2, 1, 8, SK_CHUNK / 2>::BYTES;
+}
+template <int FORM, typename TO, int EPI>
+__device__ __forceinline__ void beside_product(const SkinnyArgs& a, int log_rows, int block, char* lds) {
+    if constexpr (FORM == BESIDE_ROWS) rows_product<TO, false, EPI, 4, true, 2>(a, log_rows, block, lds);
+    else if constexpr (FORM == BESIDE_ONE_TILE) skinny_product<1, 1, 8, false, TO, false, EPI, SK_CHUNK>(a, block, lds);
+    else skinny_product<2, 1, 8, false, TO, false, EPI, SK_CHUNK / 2>(a, block, lds);
+}
+
+template <int FORM>
+__global__ __launch_bounds__(MOE_BESIDE_NT) void moe_route_beside_kernel(MoeRoute<bf16_t, bf16_t> r, SkinnyArgs a, int log_rows) {
+    extern __shared__ __align__(16) float sm[];
+    if ((int)blockIdx.x < r.T) moe_route_token<bf16_t, bf16_t, MOE_BESIDE_NT>(r, blockIdx.x, sm);
+    else beside_product<FORM, bf16_t, 2>(a, log_rows, blockIdx.x - r.T, reinterpret_cast<char*>(sm));
+}
+
+template <int FORM, bool EXT>
+__global__ __launch_bounds__(MOE_BESIDE_NT) void moe_linear_beside_kernel(MoeLinear<bf16_t> p, SkinnyArgs a, int log_rows, int blocks_beside, int col_blocks) {
+    __shared__ __attribute__((aligned(16))) char lds[beside_lds<FORM>()];
+    if ((int)blockIdx.x < blocks_beside) return beside_product<FORM, float, 0>(a, log_rows, blockIdx.x, lds);
+    const int b = blockIdx.x - blocks_beside, tile = b / col_blocks, cb = b - tile * col_blocks;
+    moe_linear_rows_wave<EXT, bf16_t, MR_OUT_FEW>(p, tile, (cb * (MOE_BESIDE_NT / 64) + (threadIdx.x >> 6)) * MR_OUT_FEW);
+}
+
+// The product beside: x [T, K] w [N, K]^T; the form, the columns a block takes and the blocks.  False where it takes none.
+static bool beside_form(SkinnyArgs& a, const void* x, const void* w, void* out, int T, int N, int K, int& form, int& blocks, int& log_rows) {
+    if (T <= 0 || T > MOE_BESIDE_ROWS || N <= 0 || K <= 0 || K % 8 || ((uintptr_t)x | (uintptr_t)w) % 16 || (uintptr_t)out % 4) return false;
+    form = T <= ROWS_KERNEL_M && K % 64 == 0 ? BESIDE_ROWS : T <= 16 ? BESIDE_ONE_TILE : BESIDE_TWO_TILES;
+    a = SkinnyArgs{(const bf16_t*)x, (const bf16_t*)w, nullptr, out, T, N, K, 0.f};
+    a.cols = balanced_round_cols(N, 16);
+    blocks = (N + a.cols - 1) / a.cols;
+    log_rows = T <= 1 ? 0 : T <= 2 ? 1 : 2;
+    return true;
+}
+
+// li_moe_route for bfloat16 rows and router of up to 32 tokens, and hs[t, n] = act(sum_k x[t, k] w[n, k]) (bfloat16, act as li_linear_act's)
+// in the same launch.  Returns -1, having done nothing, where it does not take the call.
+extern "C" int li_moe_route_beside(const void* x, const void* wr, const float* br, const void* wg, int* idx, float* wt, float* gate, int T, int K,
+                                   int E, int top, int mode, const float* corr, int groups, int keep, int* plan, int max_tiles, int* row_token,
+                                   int* pair_row, int tile_rows, float* row_wt, int experts, int* count, const void* w, void* hs, int N, int act,
+                                   hipStream_t stream) {
+    if (plan && (T > 128 || experts <= 0 || experts > MOE_PLAN_EXPERTS || experts > E || K < 64 || max_tiles <= 0 || !row_token || !pair_row || !count ||
+                 (tile_rows != MOE_TILE && tile_rows != MOE_BIG_TILE && tile_rows != MOE_HUGE_TILE)))
+        return LI_ERR_SIZE;
+    if (T <= 0 || K <= 0 || E <= 0 || top <= 0 || top > E || top > 64 || (wg && !gate) || mode < 0 || mode > 15 || (mode & 3) == 3 ||
+        groups <= 0 || keep <= 0 || keep > groups || E % groups || (size_t)(K + 2 * E + groups + 4) * 4 > 60000)
+        return LI_ERR_SIZE;
+    if ((mode & 3) != 0 && (long)top > (long)keep * (E / groups)) return LI_ERR_SIZE;
+    SkinnyArgs a;
+    int form, blocks, log_rows;
+    if (act < LI_ACT_RELU2 || act > LI_ACT_GELU_ERF || !beside_form(a, x, w, hs, T, N, K, form, blocks, log_rows)) return -1;
+    a.ep = LiAct{act, 0.f, 0.f};
+    const int vec = (K % 8 == 0 && ((uintptr_t)wr % 16) == 0 && (!wg || ((uintptr_t)wg % 16) == 0)) | 2;      // (K % 8 and x's alignment: beside_form)
+    const MoeRoute<bf16_t, bf16_t> r{(const bf16_t*)x, K, (const bf16_t*)wr, br, (const bf16_t*)wg, idx, wt, gate, T, K, E, top, vec, mode, corr, groups, keep,
+                                     MoePlanOut{plan, row_token, pair_row, row_wt, count, max_tiles, tile_rows, experts}};
+    const size_t mine = (size_t)(((K + 3) & ~3) + 2 * E + groups) * 4;
+#define RB(FORM)                                                                                                                  \
+    {                                                                                                                             \
+        const size_t his = beside_lds<FORM>(), lds = mine > his ? mine : his;                                                     \
+        moe_route_beside_kernel<FORM><<<T + blocks, MOE_BESIDE_NT, lds, stream>>>(r, a, log_rows);                                \
+    }
+    if (form == BESIDE_ROWS) RB(BESIDE_ROWS) else if (form == BESIDE_ONE_TILE) RB(BESIDE_ONE_TILE) else RB(BESIDE_TWO_TILES)
+#undef RB
+    return li_launch_status();
+}
+
+// li_moe_linear for bfloat16 rows, matrices and results in tiles of MOE_TILE rows, at most MOE_VECTOR_ROWS rows, and y[t, n] = sum_k x[t, k] w2[n, k] (float32, t < T) in the
+// same launch.  Returns -1, having done nothing, where it does not take the call (other forms of the routed product among it).
+extern "C" int li_moe_linear_beside(const void* a, long a_stride, const int* row_token, const void* w, const int* plan, int max_tiles, void* out,
+                                    long out_stride, int n_out, int K, int act, float limit, int rows, const float* row_wt, const void* x,
+                                    const void* w2, float* y, int T, int N2, int K2, hipStream_t stream) {
+    const bool gated = act == 2 || act == 3;
+    if (max_tiles <= 0 || n_out <= 0 || K <= 0 || a_stride < K || act < 0 || act > 4 || out_stride < (gated ? n_out / 2 : n_out) || (gated && (n_out & 1)))
+        return LI_ERR_SIZE;
+    SkinnyArgs s;
+    int form, blocks, log_rows;
+    if (T > ROWS_KERNEL_M || K % 8 || a_stride % 8 || ((uintptr_t)a | (uintptr_t)w) % 16 || !beside_form(s, x, w2, y, T, N2, K2, form, blocks, log_rows)) return -1;
+    if (rows > MOE_VECTOR_ROWS) return -1;
+    const int block_cols = MOE_BESIDE_NT / 64 * MR_OUT_FEW, col_blocks = (n_out + block_cols - 1) / block_cols;
+    const MoeLinear<bf16_t> p{(const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (bf16_t*)out, out_stride, n_out, K, MoeEpilogue{act, limit, row_wt}};
+    if ((long)col_blocks * max_tiles + blocks > 0x7fffffffL) return -1;
+    const unsigned grid = (unsigned)(blocks + col_blocks * max_tiles);
+#define LB2(FORM, EXT) moe_linear_beside_kernel<FORM, EXT><<<grid, MOE_BESIDE_NT, 0, stream>>>(p, s, log_rows, blocks, col_blocks)
+#define LB(FORM) { if (act == 4 || row_wt) LB2(FORM, true); else LB2(FORM, false); }
+    if (form == BESIDE_ROWS) LB(BESIDE_ROWS) else LB(BESIDE_ONE_TILE)       // (so few rows: at most 4 tokens)
+#undef LB
+#undef LB2
+    return li_launch_status();
 }
 
 // ----------------------------------------------------------------------------------------------- the sum

@@ -71,6 +71,8 @@ _SIGNATURES = {
     },
     "moe": {
         "li_moe_route": [P, I, L, P, I, P, P, P, P, P, I, I, I, I, I, P, I, I, P, I, P, P, I, P, I, P],
+        "li_moe_route_beside": [P, P, P, P, P, P, P, I, I, I, I, I, P, I, I, P, I, P, P, I, P, I, P, P, P, I, I],
+        "li_moe_linear_beside": [P, L, P, P, P, I, P, L, I, I, I, F, I, P, P, P, P, I, I, I],
         "li_moe_plan": [P, I, I, I, P, I, P, P, I, P, P],
         "li_moe_linear": [P, I, L, P, P, I, P, I, P, I, L, I, I, I, F, I, I, P],
         "li_moe_combine_norm": [P, P, L, P, P, P, P, L, I, I, I, P, I, P, I, L, F, P, F, P, F, P, I],
@@ -2040,6 +2042,8 @@ class MoePlan:
 
 
 MOE_ROUTE_PLAN_TOKENS, MOE_ROUTE_PLAN_EXPERTS = 128, 64
+MOE_BESIDE_ROWS = 32         # tokens up to which the shared expert's first product goes in the router's launch,
+MOE_BESIDE_PAIRS = 4         # ... and rows of the routed product up to which its second goes in that one's
 
 
 def moe_route_takes_plan(t: int, experts: int, hidden: int) -> bool:
@@ -2069,7 +2073,7 @@ def _check_plan(what: str, t: int, top: int, p: MoePlan) -> int:
 def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor], gate_row: Optional[torch.Tensor],
               idx: torch.Tensor, wt: torch.Tensor, gate: Optional[torch.Tensor], scores: str = "softmax_chosen",
               correction: Optional[torch.Tensor] = None, groups: int = 1, keep_groups: int = 1,
-              group_score: str = "top2_sum", normalize: bool = True, plan: Optional[MoePlan] = None) -> None:
+              group_score: str = "top2_sum", normalize: bool = True, plan: Optional[MoePlan] = None, beside=None) -> bool:
     """idx [T, top] int32: the experts with the largest logits x router^T + bias (float32 sums; the lower index wins a
     tie); wt [T, top] float32: softmax over the chosen logits; gate [T] = sigmoid(x . gate_row) where a row is given.
     With scores = "sigmoid" an expert's score is sigmoid(logit); the choice goes by score + correction[e], and only
@@ -2077,7 +2081,8 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
     values have the largest sum (`group_score` = "max": whose largest choice value is largest); wt = the chosen scores
     over their sum (+ 1e-20), or, with `normalize` False, the chosen scores themselves.  scores = "softmax": the same
     with an expert's score = the softmax over ALL logits.  With a `plan` (where `moe_route_takes_plan`) the same launch makes what
-    `moe_plan` makes of idx."""
+    `moe_plan` makes of idx.  `beside` = (w [N, K], out [T, N], activation): a product of the same rows that may go in the same launch,
+    out = act(x w^T); returns whether it did."""
     _gpu(x, router, bias, gate_row, idx, wt, gate, correction)
     t, k = x.shape
     e, top = router.shape[0], idx.shape[1]
@@ -2101,12 +2106,24 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
         _chk(moe_route_takes_plan(t, plan.experts, k) and plan.experts <= e and plan.count.dtype is torch.int32 and plan.count.numel() > 0, "moe_route: plan")
         made = (plan.plan.data_ptr(), max_tiles, plan.row_token.data_ptr(), plan.pair_row.data_ptr(), int(plan.tile_rows),
                 0 if plan.row_wt is None else plan.row_wt.data_ptr(), plan.experts, plan.count.data_ptr())
+    if beside is not None and 0 < t <= MOE_BESIDE_ROWS:
+        w, out, act = beside
+        _gpu(w, out)
+        n = w.shape[0]
+        _chk(w.shape == (n, k) and w.is_contiguous() and out.shape == (t, n) and out.is_contiguous() and act in LINEAR_ACTS, "moe_route: beside")
+        if (x.dtype is router.dtype is w.dtype is out.dtype is torch.bfloat16 and x.is_contiguous()
+                and _try("moe", "li_moe_route_beside", x.data_ptr(), router.data_ptr(), 0 if bias is None else bias.data_ptr(),
+                         0 if gate_row is None else gate_row.data_ptr(), idx.data_ptr(), wt.data_ptr(), 0 if gate is None else gate.data_ptr(), t, k, e, top,
+                         mode | (4 if group_score == "max" else 0) | (0 if normalize or mode == 0 else 8), 0 if correction is None else correction.data_ptr(),
+                         int(groups), int(keep_groups), *made, w.data_ptr(), out.data_ptr(), n, LINEAR_ACTS[act])):
+            return True
     if t:
         _run("moe", "li_moe_route", x.data_ptr(), _DT[x.dtype], x.stride(0), router.data_ptr(), _DT[router.dtype],
              0 if bias is None else bias.data_ptr(), 0 if gate_row is None else gate_row.data_ptr(), idx.data_ptr(), wt.data_ptr(),
              0 if gate is None else gate.data_ptr(), t, k, e, top,
              mode | (4 if group_score == "max" else 0) | (0 if normalize or mode == 0 else 8), 0 if correction is None else correction.data_ptr(),
              int(groups), int(keep_groups), *made)
+    return False
 
 
 def moe_plan(idx: torch.Tensor, experts: int, plan: torch.Tensor, row_token: torch.Tensor, pair_row: torch.Tensor,
@@ -2127,12 +2144,14 @@ def moe_plan(idx: torch.Tensor, experts: int, plan: torch.Tensor, row_token: tor
 
 def moe_linear(a: torch.Tensor, row_token: Optional[torch.Tensor], w: torch.Tensor, plan: torch.Tensor, max_tiles: int,
                out: torch.Tensor, rows: int, act: int = 0, tile_rows: int = MOE_TILE_ROWS, limit: float = 0.0,
-               row_wt: Optional[torch.Tensor] = None) -> None:
+               row_wt: Optional[torch.Tensor] = None, beside=None) -> bool:
     """out[row] = act(W[expert of the row's tile] a[src(row)]) for the sorted rows of the plan; src(row) = row_token[row]
     where given (rows gathered from tokens), else the row.  w [experts, n_out, K]; act 1: max(., 0)^2; act 2: the
     matrix rows are (gate, up) pairs, out[row, j] = silu(W[2j] a) * (W[2j + 1] a) and out has n_out / 2 columns; act 3:
     the same pairs with g = min(gate, limit), u = clamp(up, -limit, limit) and out = g sigmoid(1.702 g) (u + 1);
-    act 4: gelu (with the error function).  `row_wt` (float32, a number a sorted row) multiplies the row of a."""
+    act 4: gelu (with the error function).  `row_wt` (float32, a number a sorted row) multiplies the row of a.
+    `beside` = (x [T, K2], w2 [N2, K2], y [T, N2] float32): another product that may go in the same launch, y = x w2^T; returns whether
+    it did."""
     _gpu(a, row_token, w, plan, out, row_wt)
     e, n_out, k = w.shape
     gated = act in (2, 3)
@@ -2144,10 +2163,22 @@ def moe_linear(a: torch.Tensor, row_token: Optional[torch.Tensor], w: torch.Tens
          "moe_linear: a [*, K], w [E, n_out, K], out [rows, n_out]")
     _chk(plan.dtype is torch.int32 and plan.numel() >= 4 + 4 * max_tiles and (row_token is not None or a.shape[0] >= rows)
          and (row_token is None or (row_token.dtype is torch.int32 and row_token.numel() >= rows)), "moe_linear: plan, rows")
+    if beside is not None and 0 < rows <= MOE_BESIDE_PAIRS and 0 < beside[0].shape[0] and tile_rows == MOE_TILE_ROWS:
+        x, w2, y = beside
+        _gpu(x, w2, y)
+        t, k2 = x.shape
+        n2 = w2.shape[0]
+        _chk(w2.shape == (n2, k2) and w2.is_contiguous() and x.is_contiguous() and y.shape == (t, n2) and y.is_contiguous(), "moe_linear: beside")
+        if (a.dtype is w.dtype is out.dtype is x.dtype is w2.dtype is torch.bfloat16 and y.dtype is torch.float32
+                and _try("moe", "li_moe_linear_beside", a.data_ptr(), a.stride(0), 0 if row_token is None else row_token.data_ptr(), w.data_ptr(),
+                         plan.data_ptr(), int(max_tiles), out.data_ptr(), out.stride(0), n_out, k, int(act), float(limit), int(rows),
+                         0 if row_wt is None else row_wt.data_ptr(), x.data_ptr(), w2.data_ptr(), y.data_ptr(), t, n2, k2)):
+            return True
     if rows:
         _run("moe", "li_moe_linear", a.data_ptr(), _DT[a.dtype], a.stride(0), 0 if row_token is None else row_token.data_ptr(),
              w.data_ptr(), _DT[w.dtype], plan.data_ptr(), int(max_tiles), out.data_ptr(), _DT[out.dtype], out.stride(0), n_out, k, int(act),
              float(limit), int(tile_rows), int(rows), 0 if row_wt is None else row_wt.data_ptr())
+    return False
 
 
 def moe_combine(x: torch.Tensor, yrows: torch.Tensor, pair_row: torch.Tensor, wt: Optional[torch.Tensor], gate: Optional[torch.Tensor],

@@ -158,25 +158,27 @@ class RoutedMLP(FeedForward):
         row_wt = ws.buffer("moe.row_wt", (pairs,), torch.float32) if self.weigh_input else None
         count = ws.buffer("moe.count", (1,), torch.int32, zero=True)         # (asked for by every step: a recorded one finds it)
         with_plan = ops.moe_route_plan_pays(t, self.experts, self.hidden)
-        ops.moe_route(xn, self.router, self.router_b, self.gate_row, idx, wt, gate, scores=self.scores,
-                      correction=self.correction, groups=self.groups, keep_groups=self.keep_groups,
-                      group_score=self.group_score, normalize=self.normalize,
-                      plan=ops.MoePlan(self.experts, plan, row_token, pair_row, rows_a_tile, row_wt, count) if with_plan else None)
+        # (a decoding step: the shared expert's products, which hang on no choice, go in the launches of the router and of the first routed product)
+        hs = ws.buffer("mlp.h", (t, self.shared_inter), self.rt.dtype) if self.shared_inter else None
+        up_done = ops.moe_route(xn, self.router, self.router_b, self.gate_row, idx, wt, gate, scores=self.scores,
+                                correction=self.correction, groups=self.groups, keep_groups=self.keep_groups,
+                                group_score=self.group_score, normalize=self.normalize,
+                                plan=ops.MoePlan(self.experts, plan, row_token, pair_row, rows_a_tile, row_wt, count) if with_plan else None,
+                                beside=(self.shared_up.weight, hs, self.activation) if self.shared_inter else None)
         if not with_plan:
             ops.moe_plan(idx, self.experts, plan, row_token, pair_row, rows_a_tile, wt=wt if self.weigh_input else None, row_wt=row_wt)
         h = ws.buffer("moe.h", (pairs, self.inter), self.rt.dtype)
-        ops.moe_linear(xn, row_token, self.w_up, plan, max_tiles, h, pairs, act=ACTIVATIONS[self.activation],
-                       tile_rows=rows_a_tile, limit=self.limit, row_wt=row_wt)
+        shared = ws.buffer("moe.shared", (t, self.hidden), torch.float32) if self.shared_inter else None
+        down_done = ops.moe_linear(xn, row_token, self.w_up, plan, max_tiles, h, pairs, act=ACTIVATIONS[self.activation],
+                                   tile_rows=rows_a_tile, limit=self.limit, row_wt=row_wt,
+                                   beside=(hs, self.shared_down.weight, shared) if up_done else None)
         yrows = ws.buffer("moe.y", (pairs, self.hidden), torch.float32)
         ops.moe_linear(h, None, self.w_down, plan, max_tiles, yrows, pairs, tile_rows=rows_a_tile)
-        shared = None
-        if self.shared_inter:
-            hs = ws.buffer("mlp.h", (t, self.shared_inter), self.rt.dtype)
-            if not self.shared_up.with_activation(xn, hs, self.activation, ws=ws):
-                u = ws.buffer("mlp.up32", (t, self.shared_inter), torch.float32)
-                self.shared_up(xn, u, ws=ws)
-                SHARED_ACTIVATIONS[self.activation](u, hs)
-            shared = ws.buffer("moe.shared", (t, self.hidden), torch.float32)
+        if self.shared_inter and not up_done and not self.shared_up.with_activation(xn, hs, self.activation, ws=ws):
+            u = ws.buffer("mlp.up32", (t, self.shared_inter), torch.float32)
+            self.shared_up(xn, u, ws=ws)
+            SHARED_ACTIVATIONS[self.activation](u, hs)
+        if self.shared_inter and not down_done:
             self.shared_down(hs, shared, ws=ws)
         # (a pair whose choice is an identity expert has no row in the plan: the sum takes the token's input for it)
         rows = (yrows, pair_row, None if self.weigh_input else wt, gate, shared)

@@ -596,3 +596,54 @@ def test_position_vector_and_capped_logits():
     u = torch.linspace(-3, 3, 11, device=DEV)
     ops.scale_softcap(u, 2.0, 0.0)
     assert torch.allclose(u, torch.linspace(-6, 6, 11, device=DEV))
+
+
+@pytest.mark.parametrize("T,K,n_router,experts,top,n_out,inter,shared,act", [
+    (1, 1536, 16, 16, 2, 2240, 2240, 4480, "relu2"), (1, 72, 20, 16, 6, 44, 24, 40, "gelu"), (1, 2560, 64, 64, 2, 36, 2568, 64, "relu2"),
+    (2, 64, 5, 3, 2, 20, 32, 128, "gelu"), (4, 1088, 33, 33, 1, 34, 64, 1088, "relu2"), (5, 1536, 16, 16, 2, 68, 64, 200, "gelu"),
+    (16, 520, 8, 8, 2, 48, 96, 520, "relu2"), (17, 136, 4, 4, 2, 100, 64, 1160, "gelu"), (32, 1536, 16, 16, 2, 1536, 96, 2240, "relu2")])
+def test_the_shared_expert_beside_the_routed_ones(T, K, n_router, experts, top, n_out, inter, shared, act):
+    """Choices, weights, plan, the routed product and both products of the shared expert from the two common launches, against launches
+    of their own (the shared expert's also against float64); the few tokens' choices against the choice in float64."""
+    from litinfer_amd.kernels import ops
+    from litinfer_amd.parts.moe import ACTIVATIONS
+    g = torch.Generator().manual_seed(T * 1000 + K)
+    draw = lambda *shape: (torch.randn(*shape, generator=g) / shape[-1] ** 0.5).to(torch.bfloat16).to(DEV)
+    x, router, gate_row = torch.randn(T, K, generator=g).to(torch.bfloat16).to(DEV), draw(n_router, K), draw(K)
+    w, up, down, corr = draw(experts, n_out, K), draw(shared, K), draw(inter, shared), torch.randn(n_router, generator=g).to(DEV) / 8
+    pairs, tiles = T * top, ops.moe_max_tiles(T, top, experts, 32)
+    count = torch.zeros(1, dtype=torch.int32, device=DEV)
+    got = []
+    for beside in (False, True, True):
+        new = lambda *shape, d=torch.int32: torch.full(shape, -7, dtype=d, device=DEV)
+        idx, wt, gate = new(T, top), new(T, top, d=torch.float32), new(T, d=torch.float32)
+        plan = ops.MoePlan(experts, new(4 + 4 * tiles), new(pairs), new(pairs), 32, new(pairs, d=torch.float32), count)
+        hs, y, h = new(T, shared, d=torch.bfloat16), new(T, inter, d=torch.float32), new(pairs, n_out, d=torch.bfloat16)
+        args = dict(scores="sigmoid", correction=corr)
+        took = ops.moe_route(x, router, None, gate_row, idx, wt, gate, plan=plan if beside else None, beside=(up, hs, act) if beside else None, **args)
+        if not beside:
+            ops.moe_plan(idx, experts, plan.plan, plan.row_token, plan.pair_row, 32, wt=wt, row_wt=plan.row_wt)
+            assert ops.linear_act(x, up, None, hs, act)
+        took2 = ops.moe_linear(x, plan.row_token, w, plan.plan, tiles, h, pairs, act=ACTIVATIONS[act], row_wt=plan.row_wt, beside=(hs, down, y) if beside else None)
+        assert took is beside and took2 in (beside, False) and count.item() == 0
+        if not took2:
+            ops.linear(hs, down, None, y)
+        at = plan.pair_row.cpu().long().view(-1)
+        rows = torch.where((at >= 0)[:, None], h.float().cpu()[at.clamp(min=0)], torch.zeros(()))
+        n = plan.plan[0].item()
+        got.append([idx, wt, gate, plan.plan[:4 + 4 * n], at >= 0, rows, hs.float(), y])
+    for mine in got[1:]:
+        for a, b in zip(got[0][:6], mine[:6]):
+            assert torch.equal(a, b)
+        hs, y = mine[6:]
+        z = x.double() @ up.double().T
+        ref = torch.relu(z) ** 2 if act == "relu2" else torch.nn.functional.gelu(z)
+        # a bfloat16 result: half a unit in 2^-8, and the sum's own error through the activation (slope at most 2 |z| + 2)
+        assert torch.all((hs.double() - ref).abs() <= 2 ** -8 * ref.abs() + K * 2 ** -24 * (2 * z.abs() + 2) * (x.double().abs() @ up.double().abs().T))
+        z = hs.double() @ down.double().T
+        assert torch.all((y.double() - z).abs() <= shared * 2 ** -24 * (hs.double().abs() @ down.double().abs().T))
+    logits = x.double() @ router.double().T
+    score = torch.sigmoid(logits) + corr.double()
+    best = score.sort(dim=1, descending=True)
+    clear = (best.values[:, :top] - best.values[:, 1:top + 1] > 1e-5).all(1) if n_router > top else torch.ones(T, dtype=torch.bool, device=DEV)
+    assert torch.equal(got[1][0].long()[clear], best.indices[:, :top][clear]) and clear.any()
