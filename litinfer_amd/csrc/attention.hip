@@ -117,8 +117,7 @@ __device__ __forceinline__ void unpack16(const u32x4& r, float* f) {
 // Sum over the LPK lanes that share a key; every one of them gets the total.
 // Steps within a row of 16 lanes are DPP moves inside the vector ALU (swap
 // neighbours, swap pairs, mirror the half row, mirror the row), which keep
-// their place in the instruction stream; only steps across rows go through
-// the LDS crossbar.
+// their place in the instruction stream; steps across rows are swaps of rows.
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float v) {
     return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
@@ -130,8 +129,8 @@ __device__ __forceinline__ float group_sum(float v) {
     if constexpr (LPK >= 4) v = dpp_add<0x4E>(v);      // quad_perm [2,3,0,1]
     if constexpr (LPK >= 8) v = dpp_add<0x141>(v);     // row_half_mirror
     if constexpr (LPK >= 16) v = dpp_add<0x140>(v);    // row_mirror
-    if constexpr (LPK >= 32) v += __shfl_xor(v, 16, LI_WAVE);
-    if constexpr (LPK >= 64) v += __shfl_xor(v, 32, LI_WAVE);
+    if constexpr (LPK >= 32) v = lane_xor_add(v, 16);
+    if constexpr (LPK >= 64) v = lane_xor_add(v, 32);
     return v;
 }
 
@@ -252,10 +251,10 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
         for (int o = LPK; o < 64; o <<= 1) {
 #pragma unroll
             for (int h = 0; h < GB; ++h) {
-                const float mo = __shfl_xor(m[h], o, LI_WAVE), lo2 = __shfl_xor(l[h], o, LI_WAVE);
+                const float mo = lane_xor(m[h], o), lo2 = lane_xor(l[h], o);
                 float ao[E];
 #pragma unroll
-                for (int j = 0; j < E; ++j) ao[j] = __shfl_xor(acc[h][j], o, LI_WAVE);
+                for (int j = 0; j < E; ++j) ao[j] = lane_xor(acc[h][j], o);
                 softmax_merge(m[h], l[h], acc[h], E, mo, lo2, ao);
             }
         }

@@ -69,16 +69,49 @@ __device__ __forceinline__ float activation(float z, const LiAct& e) {
     return xielu(z, e.a0, e.a1);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = LI_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, LI_WAVE);
-    return v;
+// Exchanges between the lanes of a wave inside the vector ALU.  __shfl_xor goes through the LDS crossbar: sixty cycles and more a step, in a
+// chain of six for a sum over a wave, behind which every other LDS access waits; a DPP move (within rows of 16 lanes) or v_permlane16/32_swap
+// (between them) is an instruction of a few.  In launches whose work is one row or a few this chain is a good part of the time.
+// All lanes of a row (o < 16) or of the wave have to take part.
+template <int CTRL>
+__device__ __forceinline__ int dpp_mov(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true); }
+// v of lane l ^ o; o a constant once the caller's loop is unrolled: 1, 2, 4, 8, 16 or 32
+__device__ __forceinline__ int lane_xor(int v, const int o) {
+    if (o == 1) return dpp_mov<0xB1>(v);                       // quad_perm [1,0,3,2]
+    if (o == 2) return dpp_mov<0x4E>(v);                       // quad_perm [2,3,0,1]
+    if (o == 4) return dpp_mov<0x141>(dpp_mov<0x1B>(v));       // quad_perm [3,2,1,0], then row_half_mirror: l ^ 3 ^ 7
+    if (o == 8) return dpp_mov<0x128>(v);                      // row_ror:8
+    // (the swap leaves the even rows' (the lower half's) values in every lane of one result, the others' in the other)
+    const bool upper = (__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0)) & o) != 0;
+    if (o == 16) { const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false); return upper ? r[0] : r[1]; }
+    const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return upper ? r[0] : r[1];
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = LI_WAVE / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, LI_WAVE));
-    return v;
+__device__ __forceinline__ float lane_xor(float v, const int o) { return __int_as_float(lane_xor(__float_as_int(v), o)); }
+// v + lane_xor(v, o), max(v, lane_xor(v, o)): no choice between the swap's results
+template <typename Op>
+__device__ __forceinline__ float lane_xor_with(float v, const int o, Op op) {
+    if (o < 16) return op(v, lane_xor(v, o));
+    const uint32_t u = __float_as_uint(v);
+    if (o == 16) { const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false); return op(__uint_as_float(r[0]), __uint_as_float(r[1])); }
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    return op(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
+__device__ __forceinline__ float lane_xor_add(float v, const int o) { return lane_xor_with(v, o, [](float a, float b) { return a + b; }); }
+__device__ __forceinline__ float lane_xor_max(float v, const int o) { return lane_xor_with(v, o, [](float a, float b) { return fmaxf(a, b); }); }
+
+// Over the wave, in the order 32, 16, 8, 4, 2, 1.  (Once the values repeat every eight lanes, a rotation of the row by 4 brings lane l ^ 4's.)
+template <typename Op>
+__device__ __forceinline__ float wave_with(float v, Op op) {
+    v = lane_xor_with(v, 32, op);
+    v = lane_xor_with(v, 16, op);
+    v = op(v, __int_as_float(dpp_mov<0x128>(__float_as_int(v))));
+    v = op(v, __int_as_float(dpp_mov<0x124>(__float_as_int(v))));
+    v = op(v, __int_as_float(dpp_mov<0x122>(__float_as_int(v))));
+    return op(v, __int_as_float(dpp_mov<0x121>(__float_as_int(v))));
+}
+__device__ __forceinline__ float wave_sum(float v) { return wave_with(v, [](float a, float b) { return a + b; }); }
+__device__ __forceinline__ float wave_max(float v) { return wave_with(v, [](float a, float b) { return fmaxf(a, b); }); }
 
 // Sum over a block of NT threads (NT a multiple of 64, at most 1024); every
 // thread gets the result.  The order of additions depends on NT only.

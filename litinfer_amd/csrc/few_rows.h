@@ -151,7 +151,7 @@ struct RowShares {
 #pragma unroll
         for (int o = QUADS; o < 64; o <<= 1)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) mine[e] += __shfl_xor(mine[e], o, 64);
+            for (int e = 0; e < 4; ++e) mine[e] = lane_xor_add(mine[e], o);
         if (lane < QUADS) *reinterpret_cast<floatx4*>(&sums[threadIdx.x >> 6][4 * lane]) = mine;
     }
 };

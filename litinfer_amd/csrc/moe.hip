@@ -313,8 +313,8 @@ __device__ __forceinline__ void moe_route_token(const MoeRoute<TX, TW>& a, const
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o, LI_WAVE);
-            const int oi = __shfl_xor(bi, o, LI_WAVE);
+            const float ob = lane_xor(best, o);
+            const int oi = lane_xor(bi, o);
             if (oi != 0x7fffffff && (bi == 0x7fffffff || ob > best || (ob == best && oi < bi))) { best = ob; bi = oi; }
         }
         if (r == 0) mx = best;

@@ -220,7 +220,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_kernel(
             if (MODE == 0) {
                 float yv = (y0 + y1) + (y2 + y3);
 #pragma unroll
-                for (int o = 1; o < NS; o <<= 1) yv += __shfl_xor(yv, o, LI_WAVE);
+                for (int o = 1; o < NS; o <<= 1) yv = lane_xor_add(yv, o);
                 if (s == 0 && p < vdim) y[(size_t)(t0 + b0 + tt) * y_stride + (size_t)head * vdim + p] = fmaf(Dh, xv, yv);
             } else {
                 prod *= a;
@@ -354,10 +354,10 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
             if (MODE == 0) {
 #pragma unroll
                 for (int o = 1; o < NS; o <<= 1) {
-                    yv.x += __shfl_xor(yv.x, o, LI_WAVE);
-                    yv.y += __shfl_xor(yv.y, o, LI_WAVE);
-                    yv.z += __shfl_xor(yv.z, o, LI_WAVE);
-                    yv.w += __shfl_xor(yv.w, o, LI_WAVE);
+                    yv.x = lane_xor_add(yv.x, o);
+                    yv.y = lane_xor_add(yv.y, o);
+                    yv.z = lane_xor_add(yv.z, o);
+                    yv.w = lane_xor_add(yv.w, o);
                 }
                 if (s == 0 && cols)
                     *reinterpret_cast<float4*>(y + (size_t)(t0 + b0 + tt) * y_stride + (size_t)head * vdim + p) =
@@ -1120,8 +1120,8 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
             }
 #pragma unroll
             for (int o = 1; o < 16; o <<= 1) {
-                sk += __shfl_xor(sk, o, LI_WAVE);
-                sq += __shfl_xor(sq, o, LI_WAVE);
+                sk = lane_xor_add(sk, o);
+                sq = lane_xor_add(sq, o);
             }
             const float ik = 1.0f / sqrtf(sk + 1e-6f), iq = q_scale / sqrtf(sq + 1e-6f);
             for (int n = part; n < NP; n += 16) {
