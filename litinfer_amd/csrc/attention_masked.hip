@@ -425,7 +425,7 @@ __global__ __launch_bounds__(NW * 64) void masked_attention_tile_kernel(
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sv[r]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, LI_WAVE));
+            mx = lane_xor_max(mx, 32);
             const float mn = fmaxf(m, mx);
             const float ms = (mn == -INFINITY) ? 0.f : mn;                    // a query may see no key of this block
             const float alpha = (m == -INFINITY) ? 1.f : fast_exp(m - ms);    // (m = -inf: nothing summed yet)
@@ -651,7 +651,7 @@ __global__ __launch_bounds__(64) void masked_attention_heads_kernel(
             }
 #pragma unroll
             for (int r = 0; r < 16; ++r) mx = fmaxf(mx, sv[r]);
-            mx = fmaxf(mx, __shfl_xor(mx, 32, LI_WAVE));
+            mx = lane_xor_max(mx, 32);
             const float mn = fmaxf(m, mx);
             const float ms = (mn == -INFINITY) ? 0.f : mn;                    // a query may see no key of this block
             const float alpha = (m == -INFINITY) ? 1.f : fast_exp(m - ms);    // (m = -inf: nothing summed yet)
@@ -804,8 +804,12 @@ extern "C" int li_masked_attention_heads(const float* q, int q_token_stride, int
 // takes one (token, kv head) and RH query heads of that kv head, so that a row is read once for all of them.  A
 // key's row is spread over 8 lanes, 16 bytes a lane and piece (lane j holds the pieces j, j + 8, ...): a wave takes
 // 8 keys at a time, the block 32, and U such rounds are in flight.  Every group of 8 lanes keeps a running
-// (maximum, sum, sums of values) per head over its keys; the groups of a wave are joined by a butterfly, the waves
+// (maximum, sum, sums of values) per head over its keys; the groups of a wave are joined by halves, the waves
 // through LDS in wave order.
+// Few keys a block: bound by the wave's own instructions (there is one a SIMD) and by a chain of trips to memory (the token's request, its
+// length, its pages, the rows).  The join by halves, a last round that asks for nothing and q and pages asked for ahead: 12 heads on 2 of 128
+// columns, 2 requests, a call with the splits' join (us): one key, one split 9.0 -> 5.9; 1,300 keys, 16 splits 13.5 -> 10.5; 12 on 1 of 256
+// 17.0 -> 12.9; 32 requests of 90 keys, 320 columns shared 13.5 -> 9.5.
 // the sum over a group of 8 neighbouring lanes, in every lane of the group, by lane moves inside the vector ALU
 // (quad_perm [1,0,3,2], quad_perm [2,3,0,1], row_half_mirror) instead of three trips through LDS
 __device__ __forceinline__ float dpp_move(float v, const int ctrl) {
@@ -849,19 +853,35 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     const int rep = nh / nkv, hfirst = (blockIdx.z / nsplit) * RH, sp = blockIdx.z % nsplit;
     const int nheads = rep - hfirst < RH ? rep - hfirst : RH;
     const int s = seg_of_token[t];
+    const int* table = block_table + (size_t)s * max_blocks;
+    // (what does not hang on the position is on its way before the position is known: the heads of q, and, where every key is visible and
+    // the room holds the whole table, the table)
+    float4 qraw[RH][NPK][2];
+#pragma unroll
+    for (int hh = 0; hh < RH; ++hh) {
+        const float* qrow = q + (size_t)t * q_token_stride + (size_t)(kvh * rep + hfirst + (hh < nheads ? hh : 0)) * q_head_stride;
+#pragma unroll
+        for (int c = 0; c < NPK; ++c) {
+            const int d0 = 8 * (j + 8 * c) < dk ? 8 * (j + 8 * c) : 0;
+            qraw[hh][c][0] = *reinterpret_cast<const float4*>(qrow + d0);
+            qraw[hh][c][1] = *reinterpret_cast<const float4*>(qrow + d0 + 4);
+        }
+    }
+    const bool whole = window <= 0 && ex.chunk <= 0 && max_blocks <= tab_cap;
+    if (whole)
+        for (int i = threadIdx.x; i < max_blocks; i += 256) tab[i] = table[i];
     const int p = ctx_len[s] - q_len[s] + (t - q_start[s]);
     const int lo = lower_edge(p, window, ex.chunk);
     const int n_first = keep_first < lo ? keep_first : lo;
     const int n_all = n_first + (p - lo + 1);
     // this block's share of the visible keys (split sp of nsplit)
     const int i_begin = (int)((long)n_all * sp / nsplit), n_keys = (int)((long)n_all * (sp + 1) / nsplit);
-    const int* table = block_table + (size_t)s * max_blocks;
     // the pages of the visible keys in LDS (the window's blocks, then the kept first blocks), so that a key's row
     // costs no trip to memory before its own; a table too long for the room given is read where it lies
     const int b_lo = pshift >= 0 ? lo >> pshift : lo / page_size, b_hi = pshift >= 0 ? p >> pshift : p / page_size;
     const int nb_w = b_hi - b_lo + 1, nb_k = n_first > 0 ? (n_first - 1) / page_size + 1 : 0;
     const bool in_lds = nb_w + nb_k <= tab_cap;
-    if (in_lds) {
+    if (in_lds && !whole) {
         for (int i = threadIdx.x; i < nb_w; i += 256) tab[i] = table[b_lo + i];
         for (int i = threadIdx.x; i < nb_k; i += 256) tab[nb_w + i] = table[i];
     }
@@ -870,15 +890,12 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     float qr[RH][NPK][8];
 #pragma unroll
     for (int hh = 0; hh < RH; ++hh) {
-        const float* qrow = q + (size_t)t * q_token_stride + (size_t)(kvh * rep + hfirst + (hh < nheads ? hh : 0)) * q_head_stride;
 #pragma unroll
         for (int c = 0; c < NPK; ++c) {
-            const int d0 = 8 * (j + 8 * c);
-            const bool on = d0 < dk && hh < nheads;
-            const float4 a = on ? *reinterpret_cast<const float4*>(qrow + d0) : float4{0.f, 0.f, 0.f, 0.f};
-            const float4 b = on ? *reinterpret_cast<const float4*>(qrow + d0 + 4) : float4{0.f, 0.f, 0.f, 0.f};
-            qr[hh][c][0] = a.x; qr[hh][c][1] = a.y; qr[hh][c][2] = a.z; qr[hh][c][3] = a.w;
-            qr[hh][c][4] = b.x; qr[hh][c][5] = b.y; qr[hh][c][6] = b.z; qr[hh][c][7] = b.w;
+            const bool on = 8 * (j + 8 * c) < dk && hh < nheads;
+            const float4 a = qraw[hh][c][0], b = qraw[hh][c][1];
+            qr[hh][c][0] = on ? a.x : 0.f; qr[hh][c][1] = on ? a.y : 0.f; qr[hh][c][2] = on ? a.z : 0.f; qr[hh][c][3] = on ? a.w : 0.f;
+            qr[hh][c][4] = on ? b.x : 0.f; qr[hh][c][5] = on ? b.y : 0.f; qr[hh][c][6] = on ? b.z : 0.f; qr[hh][c][7] = on ? b.w : 0.f;
         }
     }
     float acc[RH][NPV][8];
@@ -894,7 +911,7 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     const float inv_cap = softcap > 0.f ? 1.0f / softcap : 0.f;
     // the rows of a round's keys (a key past the last: row 0, read and not used) and their pieces; the next round's
     // are asked for before this round's are used, without a condition (a load under a condition would make every
-    // later use wait for all loads)
+    // later use wait for all loads); the last round is taken behind the loop, which asks for nothing
     size_t ro[U];
     bool ok[U];
     int kpos[U];                                    // the keys' positions
@@ -927,13 +944,7 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     }
     MS_ROWS(i_begin, ro, ok, kpos)
     MS_FETCH(ro, kp, vp)
-    for (int i0 = i_begin; i0 < n_keys; i0 += 32 * U) {
-        size_t ro2[U];
-        bool ok2[U];
-        int kpos2[U];
-        uint4 kp2[U][NPK], vp2[U][NPV];
-        MS_ROWS(i0 + 32 * U, ro2, ok2, kpos2)
-        MS_FETCH(ro2, kp2, vp2)
+    auto round = [&]() {
         float sc[U][RH];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -982,6 +993,15 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
                 for (int e = 0; e < 8; ++e) acc[hh][c][e] = a8[e];
             }
         }
+    };
+    for (int i0 = i_begin; i0 + 32 * U < n_keys; i0 += 32 * U) {
+        size_t ro2[U];
+        bool ok2[U];
+        int kpos2[U];
+        uint4 kp2[U][NPK], vp2[U][NPV];
+        MS_ROWS(i0 + 32 * U, ro2, ok2, kpos2)
+        MS_FETCH(ro2, kp2, vp2)
+        round();
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             ok[u] = ok2[u];
@@ -992,42 +1012,52 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
             for (int c = 0; c < NPV; ++c) vp[u][c] = vp2[u][c];
         }
     }
+    round();
 #undef MS_ROWS
 #undef MS_FETCH
-    // the groups of a wave
+    // The groups of a wave: the maximum over them, every group's sums scaled to it once, and the sums added up by halves: a lane keeps
+    // one half of what it holds and gets its partner's part of that half, so that at the end each lane has NPV columns of its own.
+    // (Joined pair by pair, every step rescaled all columns of both sides: some 400 instructions a head, four cycles each.)
 #pragma unroll
-    for (int off = 8; off < 64; off <<= 1) {
+    for (int hh = 0; hh < RH; ++hh) {
+        float* mine = join + (size_t)(w * RH + hh) * (dv + 2);
+        float mw = m[hh];
 #pragma unroll
-        for (int hh = 0; hh < RH; ++hh) {
-            const float m2 = __shfl_xor(m[hh], off, LI_WAVE), l2 = __shfl_xor(l[hh], off, LI_WAVE);
-            const float mn = fmaxf(m[hh], m2);
-            const float f1 = (m[hh] == -INFINITY) ? 0.f : expf(m[hh] - mn), f2 = (m2 == -INFINITY) ? 0.f : expf(m2 - mn);
-            l[hh] = l[hh] * f1 + l2 * f2;
-            m[hh] = mn;
+        for (int off = 8; off < 64; off <<= 1) mw = lane_xor_max(mw, off);
+        const float f = m[hh] == -INFINITY ? 0.f : expf(m[hh] - mw);
+        float lw = l[hh] * f;
 #pragma unroll
-            for (int c = 0; c < NPV; ++c)
+        for (int off = 8; off < 64; off <<= 1) lw = lane_xor_add(lw, off);
+        if (lane == 0) { mine[dv] = mw; mine[dv + 1] = lw; }
+        float v[8 * NPV];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[hh][c][e] = acc[hh][c][e] * f1 + __shfl_xor(acc[hh][c][e], off, LI_WAVE) * f2;
+        for (int x = 0; x < 8 * NPV; ++x) v[x] = acc[hh][x / 8][x % 8] * f;
+#pragma unroll
+        for (int x = 0; x < 4 * NPV; ++x) {         // lanes 32 and up: the second half
+            const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[x]), __float_as_uint(v[x + 4 * NPV]), false, false);
+            v[x] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
         }
-    }
-    // the waves
-    if (g == 0) {
 #pragma unroll
-        for (int hh = 0; hh < RH; ++hh) {
-            float* mine = join + (size_t)(w * RH + hh) * (dv + 2);
-            if (j == 0) { mine[dv] = m[hh]; mine[dv + 1] = l[hh]; }
+        for (int x = 0; x < 2 * NPV; ++x) {         // the second of two rows of 16: the second half
+            const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[x]), __float_as_uint(v[x + 2 * NPV]), false, false);
+            v[x] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        }
+        const bool second8 = lane & 8;
 #pragma unroll
-            for (int c = 0; c < NPV; ++c) {
-                const int d0 = 8 * (j + 8 * c);
-                if (d0 < dv)
+        for (int x = 0; x < NPV; ++x) v[x] = (second8 ? v[x + NPV] : v[x]) + lane_xor(second8 ? v[x] : v[x + NPV], 8);
+        const int x0 = (lane >= 32 ? 4 * NPV : 0) + (lane & 16 ? 2 * NPV : 0) + (second8 ? NPV : 0);
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) mine[d0 + e] = acc[hh][c][e];
-            }
+        for (int x = 0; x < NPV; ++x) {
+            const int d = 8 * (j + 8 * ((x0 + x) >> 3)) + ((x0 + x) & 7);
+            if (d < dv) mine[d] = v[x];
         }
     }
     __syncthreads();
     for (int idx = threadIdx.x; idx < nheads * dv; idx += 256) {
-        const int hh = idx / dv, d = idx % dv;
+        int hh = 0, d = idx;
+#pragma unroll
+        for (int x = 1; x < RH; ++x)
+            if (d >= dv) { d -= dv; ++hh; }
         float mm = -INFINITY;
 #pragma unroll
         for (int x = 0; x < 4; ++x) mm = fmaxf(mm, join[(size_t)(x * RH + hh) * (dv + 2) + dv]);
@@ -1344,8 +1374,8 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
         }
 #pragma unroll
         for (int tt = 0; tt < TOK; ++tt) {
-            acc[tt] += __shfl_xor(acc[tt], 1, LI_WAVE);
-            acc[tt] += __shfl_xor(acc[tt], 2, LI_WAVE);
+            acc[tt] = lane_xor_add(acc[tt], 1);
+            acc[tt] = lane_xor_add(acc[tt], 2);
         }
         auto store = [&](int tt) {
             const float gv = gate_per_column ? gate[(size_t)(t0 + tt) * gate_stride + (size_t)h * n_out + j] : gf[tt];

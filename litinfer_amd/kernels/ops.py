@@ -952,14 +952,16 @@ def masked_attention(q: torch.Tensor, q_token_stride: int, q_head_stride: int, o
     general(None, t)
 
 
-# Single tokens on the matrix cores (the heads of a kv head as a tile's columns) or on the vector ALU.  Measured on
-# 8 / 64 / 256 requests of 1,028 visible keys (us a call, vector against matrix cores): rows of 128 + 128 columns,
-# 28 heads on 4 kv heads 46/20, 84/49, 324/127; 12 on 2: 19/19, 36/33, 152/107; rows of 320 columns shared by keys and
-# values (a compressed cache), 28 heads: 28/38, 144/112, 494/396; 12 heads: 21/36, 74/107, 225/381 (there one wave
-# stages 36 KB a block of keys by itself, which sets its time whatever the heads).
-# One and two requests: 28 on 4: 25/24, 24/24; 12 on 2: 19/23, 18/23; the long rows 20/40.
+# Single tokens on the matrix cores (the heads of a kv head as a tile's columns) or on the vector ALU.  Us a call, vector against matrix
+# cores, at 60 / 300 / 1,028 / 4,000 visible keys of a table half as wide again.  Rows of 128 + 128 columns, 28 heads on 4 kv heads: 4 requests
+# 8/10, 12/14, 20/16, 30/25; 8 requests 8/10, 12/13, 26/18, 44/32; 32 requests 9/11, 27/17, 49/31, 116/79.  12 on 2, where the vector kernel
+# takes two heads a block: 8 requests 6/10, 9/13, 12/15, 23/25; 16 requests 6/10, 11/13, 15/17, 32/32; 32 requests 6/11, 14/15, 24/22, 56/48;
+# 64 requests 8/11, 15/17, 33/31.  8 on 2: 8 requests 8/10, 11/13, 13/15, 25/25; 16 requests 8/10, 12/13, 20/17, 34/32.  Rows of 320 columns shared by
+# keys and values (a compressed cache), 12 heads: 8 requests 7/31, 12/34, 17/36, 33/76; 28 heads: 32 requests 13/32, 29/40, 71/77, 228/218;
+# 64 requests 25/33, 56/62, 139/115 (there one wave stages 36 KB a block of keys by itself, which sets its time whatever the heads).
 MASKED_HEADS_MIN = 4          # query heads a kv head from which rows of up to 384 columns (keys + values) take the matrix cores,
-MASKED_HEADS_MIN_PAIRS = 48   # for at least so many (token, head) pairs a kv head
+MASKED_HEADS_MIN_PAIRS = 48   # for at least so many (token, head) pairs a kv head, or
+MASKED_HEADS_MIN_PAIRS_BY_TWO = 193       # ... so many where the vector kernel takes the heads by two (more, smaller blocks),
 MASKED_HEADS_MIN_LONG = 24    # ... and from which longer rows do, for at least MASKED_HEADS_MIN_WORK (token, head) pairs a kv head
 MASKED_HEADS_MIN_WORK = 1024
 
@@ -999,7 +1001,8 @@ def masked_attention_difference(q: torch.Tensor, q_token_stride: int, q_head_str
 
 def _heads_kernel_pays(n: int, rep: int, dk: int, dv: int) -> bool:
     if dk + dv <= 384:
-        return rep >= MASKED_HEADS_MIN and n * rep >= MASKED_HEADS_MIN_PAIRS
+        by_two = not (rep % 4 in (0, 3) or rep > 8)                  # (the heads a block of the vector kernel takes: 4, or 2)
+        return rep >= MASKED_HEADS_MIN and n * rep >= (MASKED_HEADS_MIN_PAIRS_BY_TWO if by_two else MASKED_HEADS_MIN_PAIRS)
     return rep >= MASKED_HEADS_MIN_LONG and n * rep >= MASKED_HEADS_MIN_WORK
 
 
