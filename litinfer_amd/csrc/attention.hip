@@ -99,6 +99,7 @@ template <> struct raw16<bf16_t> { static constexpr int E = 8; };
 template <> struct raw16<float> { static constexpr int E = 4; };
 
 struct __attribute__((aligned(16))) u32x4 { uint32_t w[4]; };
+struct __attribute__((aligned(8))) u32x2 { uint32_t w[2]; };
 
 template <typename T, int E>
 __device__ __forceinline__ void unpack16(const u32x4& r, float* f) {
@@ -601,14 +602,20 @@ extern "C" int li_decode_run_keys(const int* token_list, int n_tokens, const int
 // `done[token * nkv + kv head]` after its results have been made visible to the device, and the block that
 // finds the count complete sets it back to 0 (the array is zero before the first call and after every
 // call).  Nobody waits for anybody.
-template <int WAVES> struct DecodeJoin {
+template <int WAVES, int DH> struct DecodeJoin {
     float ml[WAVES][16][2];                       // per wave and head of the pass: maximum, sum
-    float acc[WAVES][16][ATT_MAX_DH / 2];         // per wave and head: the unscaled output (DH <= 128)
+    float acc[WAVES][16][DH];                     // per wave and head: the unscaled output
     int last;
 };
-template <> struct DecodeJoin<1> { int last; };
+template <int DH> struct DecodeJoin<1, DH> { int last; };
 
-template <typename T, int DH, int WAVES>
+#define DEC_WHOLE_TABLE 64       // pages up to which a wave asks for a request's whole table before it knows the request's length
+
+// ALIGNED: no window and pages of a multiple of 8 keys, so that 8 (4) keys from a multiple of 8 (4) lie in one page and their rows behind each
+// other: one look at the table for the rows of a lane's values instead of 8 (a quarter of a step's instructions).
+// With that, heads of 64 in pieces of four dimensions (half the permutations and products of P V), the quotients in float32 and the trips
+// saved at the start (the request's number, a short table): 14 heads on 2 of 64, one request of 300 keys 6.9 -> 5.9 us, of one key 4.5 -> 3.4.
+template <typename T, int DH, int WAVES, bool ALIGNED>
 __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel(
     const T* __restrict__ q, int q_row_stride, T* __restrict__ out,
     const T* __restrict__ kc, const T* __restrict__ vc, const int* __restrict__ block_table,
@@ -620,16 +627,17 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     static_assert(DH <= ATT_MAX_DH / 2, "the join buffer holds head sizes up to 128");
     constexpr bool F32 = sizeof(T) == 4;        // float32: v_mfma_f32_16x16x4f32 on float32 operands
     constexpr int KS = DH / 32;                 // bfloat16: MFMA steps of Q K^T
-    constexpr int NS = (DH + 127) / 128;        // bfloat16: slabs of 128 output dimensions
+    constexpr int VE = DH >= 128 ? 8 : 4;       // bfloat16: a lane's neighbouring output dimensions,
+    constexpr int NS = DH / (16 * VE);          // ... in slabs of 16 lanes
     constexpr int QD = DH / 4;                  // head dimensions owned by one lane group in Q K^T
     constexpr int KJ = QD / 4;                  // float32: 16-byte pieces of those
     constexpr int NP = (DH + 63) / 64;          // float32: slabs of 64 output dimensions
     // the output's registers: acc[i] holds, for the lane's four heads, dimension dim_of(i) (below)
-    constexpr int NACC = F32 ? 4 * NP : 8 * NS;
+    constexpr int NACC = F32 ? 4 * NP : VE * NS;
     constexpr int PSTRIDE = F32 ? 36 : 40;      // elements per row of P in LDS (32 keys + pad; rows 16-byte aligned)
     __shared__ __attribute__((aligned(16))) T p_lds_all[WAVES][16 * PSTRIDE];
     __shared__ int pages_all[WAVES][DEC_TABLE_CAP];
-    __shared__ DecodeJoin<WAVES> join;
+    __shared__ DecodeJoin<WAVES, DH> join;
     const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     T* p_lds = p_lds_all[wave];
     int* pages = pages_all[wave];
@@ -653,11 +661,19 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     const int split = quad * WAVES + wave;
     const int t = token_list ? token_list[ti] : ti;
     const int G = nh / nkv;
-    const int s = seg_of_token[t];
-    const int p = ctx_len[s] - q_len[s] + (t - q_start[s]);
+    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
+    // (seg_of_token null: token t is request t's only one, which saves a trip)
+    const int s = seg_of_token ? seg_of_token[t] : t;
+    // The block table of this split goes to LDS first: a page number fetched from global
+    // memory in the loop would make every wait for it a wait for all loads issued before.
+    const bool whole = max_blocks <= DEC_WHOLE_TABLE;
+    if (whole)
+        for (int i = lane; i < max_blocks; i += 64) pages[i] = block_table[(size_t)s * max_blocks + i];
+    const int p = seg_of_token ? ctx_len[s] - q_len[s] + (t - q_start[s]) : ctx_len[t] - 1;
     const int lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
     const int nkeys = p - lo + 1;
-    int per = (((nkeys + nruns_all - 1) / nruns_all) + 31) & ~31;
+    // (the quotient as below in row_of: exact, the keys and the 64 runs at most being fewer than 2^22)
+    int per = ((int)(((float)(nkeys + nruns_all - 1) + 0.5f) * (1.0f / (float)nruns_all)) + 31) & ~31;
     if (run_keys) {
         // one run length for the whole batch (decode_run_keys_kernel): never shorter than this token's keys
         // need to fit the runs, never longer than the runs the host sized the page table in LDS for
@@ -670,14 +686,11 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     }
     const int k_begin = lo + split * per;
     const int k_end = (k_begin + per < p + 1) ? k_begin + per : p + 1;
-    const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
-    auto dim_of = [&](int i) -> int { return F32 ? 64 * (i >> 2) + 4 * c + (i & 3) : 128 * (i >> 3) + 8 * c + (i & 7); };
-    // The block table of this split goes to LDS first: a page number fetched from global
-    // memory in the loop would make every wait for it a wait for all loads issued before.
+    auto dim_of = [&](int i) -> int { return F32 ? 64 * (i >> 2) + 4 * c + (i & 3) : 16 * VE * (i / VE) + VE * c + i % VE; };
     const float inv_page = 1.0f / (float)page_size;
     const float scale2 = scale * 1.44269504088896341f;  // scores in units of log 2: the exponentials are the instruction's own
-    const int first_block = k_begin / page_size;
-    if (k_begin < k_end) {
+    const int first_block = whole ? 0 : k_begin / page_size;
+    if (!whole && k_begin < k_end) {
         const int nblocks = (k_end - 1) / page_size - first_block + 1;       // the host keeps this <= DEC_TABLE_CAP
         const int* table = block_table + (size_t)s * max_blocks + first_block;
         for (int i = lane; i < nblocks && i < DEC_TABLE_CAP; i += 64) pages[i] = table[i];
@@ -697,6 +710,14 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
         ok = ok && page >= 0 && page < num_pages;
         page = page < 0 ? 0 : (page >= num_pages ? num_pages - 1 : page);
         return (((size_t)page * nkv + kvh) * page_size + in_page) * DH;
+    };
+    // the rows of N keys from `key` on, a multiple of N: row i at the result + min(i, upto) * DH (a key past the last repeats it)
+    auto rows_of = [&](int key, const int N, int& upto) -> size_t {
+        const int last = (k_end - 1) & ~(N - 1);
+        const int first = key < last ? key : last;
+        upto = k_end - 1 - first;
+        bool ok;
+        return row_of(first, ok);
     };
 
     for (int h0 = 0; h0 < G; h0 += 16) {
@@ -724,18 +745,24 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
                         kf[tt][j].raw = *reinterpret_cast<const u32x4*>(kc + off + QD * g + 8 * j);
                 }
             };
-            // V rows of this lane: keys kb + 8g + i, dimensions 128 ns + 8c ..  Two sets of registers
+            // V rows of this lane: keys kb + 8g + i, dimensions 16 VE ns + VE c ..  Two sets of registers
             // take turns, so that the values of the NEXT block are in flight while this one is worked on
-            u32x4 va[NS][8], vb[NS][8];
-#define LI_DEC_LOAD_V(kbv, dst)                                                                      \
-            _Pragma("unroll") for (int i = 0; i < 8; ++i) {                                              \
-                bool ok_;                                                                                \
-                const size_t off_ = row_of((kbv) + 8 * g + i, ok_);                                      \
-                _Pragma("unroll") for (int ns = 0; ns < NS; ++ns) {                                      \
-                    const int d_ = 128 * ns + 8 * c;                                                     \
-                    dst[ns][i] = *reinterpret_cast<const u32x4*>(vc + off_ + (d_ < DH ? d_ : DH - 8));   \
-                }                                                                                        \
-            }
+            typedef std::conditional_t<VE == 8, u32x4, u32x2> piece_t;
+            piece_t va[NS][8], vb[NS][8];
+            auto load_v = [&](int kb, piece_t (*dst)[8]) {
+                [[maybe_unused]] int upto;
+                [[maybe_unused]] size_t base;
+                if constexpr (ALIGNED) base = rows_of(kb + 8 * g, 8, upto);
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    size_t off;
+                    if constexpr (ALIGNED) off = base + (i < upto ? i : upto) * DH;
+                    else { bool ok; off = row_of(kb + 8 * g + i, ok); }
+#pragma unroll
+                    for (int ns = 0; ns < NS; ++ns) dst[ns][i] = *reinterpret_cast<const piece_t*>(vc + off + 16 * VE * ns + VE * c);
+                }
+            };
+#define LI_DEC_LOAD_V(kbv, dst) load_v(kbv, dst);
 #define LI_DEC_STEP(kbv, vcur, vnext, more)                                                             \
             {                                                                                            \
                 /* ---- S = Q K^T */                                                                     \
@@ -773,13 +800,13 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
                 pa.raw = *reinterpret_cast<const u32x4*>(&p_lds[c * PSTRIDE + 8 * g]);                   \
                 /* ---- O = alpha O + P V */                                                             \
                 _Pragma("unroll") for (int ns = 0; ns < NS; ++ns) {                                      \
-                    _Pragma("unroll") for (int jj = 0; jj < 8; ++jj) {                                   \
+                    _Pragma("unroll") for (int jj = 0; jj < VE; ++jj) {                                  \
                         frag8 vf;                                                                        \
                         _Pragma("unroll") for (int ii = 0; ii < 4; ++ii)                                 \
                             vf.raw.w[ii] = __builtin_amdgcn_perm(vcur[ns][2 * ii + 1].w[jj >> 1], vcur[ns][2 * ii].w[jj >> 1], \
                                                                  (jj & 1) ? 0x07060302u : 0x05040100u);  \
-                        _Pragma("unroll") for (int r = 0; r < 4; ++r) acc[8 * ns + jj][r] *= alpha[r];        \
-                        acc[8 * ns + jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa.v, vf.v, acc[8 * ns + jj], 0, 0, 0); \
+                        _Pragma("unroll") for (int r = 0; r < 4; ++r) acc[VE * ns + jj][r] *= alpha[r];       \
+                        acc[VE * ns + jj] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa.v, vf.v, acc[VE * ns + jj], 0, 0, 0); \
                     }                                                                                    \
                 }                                                                                        \
             }
@@ -826,15 +853,20 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
             // V rows of this lane: keys kb + 16 tt + 4 g + s, dimensions 64 n + 4 c ..; two sets of registers in turn
             f32x4_t va[2][4][NP], vb[2][4][NP];
 #define LI_DEC_LOAD_V(kbv, dst)                                                                      \
-            _Pragma("unroll") for (int tt = 0; tt < 2; ++tt)                                         \
+            _Pragma("unroll") for (int tt = 0; tt < 2; ++tt) {                                       \
+                [[maybe_unused]] int upto_;                                                          \
+                [[maybe_unused]] size_t base_;                                                       \
+                if constexpr (ALIGNED) base_ = rows_of((kbv) + 16 * tt + 4 * g, 4, upto_);           \
                 _Pragma("unroll") for (int s_ = 0; s_ < 4; ++s_) {                                   \
-                    bool ok_;                                                                        \
-                    const size_t off_ = row_of((kbv) + 16 * tt + 4 * g + s_, ok_);                   \
+                    size_t off_;                                                                     \
+                    if constexpr (ALIGNED) off_ = base_ + (s_ < upto_ ? s_ : upto_) * DH;            \
+                    else { bool ok_; off_ = row_of((kbv) + 16 * tt + 4 * g + s_, ok_); }             \
                     _Pragma("unroll") for (int n = 0; n < NP; ++n) {                                 \
                         const int d_ = 64 * n + 4 * c;                                               \
                         dst[tt][s_][n] = *reinterpret_cast<const f32x4_t*>(vc + off_ + (d_ < DH ? d_ : DH - 4)); \
                     }                                                                                \
-                }
+                }                                                                                    \
+            }
 #define LI_DEC_STEP(kbv, vcur, vnext, more)                                                             \
             {                                                                                        \
                 f32x4_t sv[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};          \
@@ -2446,26 +2478,26 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
     if (li_decode_split_blocks(max_blocks, page_size, window, nsplit) > DEC_TABLE_CAP) return LI_ERR_SIZE;
     if (dh != 128 && dh != 64) return LI_ERR_SIZE;
     if ((long)max_blocks * page_size > (1L << 21) || page_size > (1 << 16)) return LI_ERR_SIZE;   // (the kernel's key / page_size)
-    if (nsplit == 1) {
-        dim3 grid(n_tokens, nkv, 1);
-#define LI_DM(DHV) paged_attention_decode_mfma_kernel<T, DHV, 1><<<grid, 64, 0, stream>>>( \
+    const bool aligned = window <= 0 && page_size % 8 == 0;
+    const bool listed = run_keys != nullptr && nsplit > 1;
+    if (listed && (n_tokens > RUN_KEYS_MAX_TOKENS || nsplit > 0x7fff)) return LI_ERR_SIZE;
+#define LI_DM4(DHV, W, AL, BLOCKS) paged_attention_decode_mfma_kernel<T, DHV, W, AL><<<grid, 64 * W, 0, stream>>>( \
         q, q_row_stride, out, kc, vc, block_table, max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, \
-        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, 1, nullptr, n_tokens, nullptr)
-        if (dh == 128) LI_DM(128); else LI_DM(64);
-#undef LI_DM
+        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, BLOCKS, listed ? run_keys : nullptr, n_tokens, done)
+#define LI_DM(W, BLOCKS)                                                                                     \
+    {                                                                                                        \
+        if (dh == 128) { if (aligned) LI_DM4(128, W, true, BLOCKS); else LI_DM4(128, W, false, BLOCKS); }    \
+        else { if (aligned) LI_DM4(64, W, true, BLOCKS); else LI_DM4(64, W, false, BLOCKS); }                \
+    }
+    if (nsplit == 1) {
+        const dim3 grid(n_tokens, nkv, 1);
+        LI_DM(1, 1)
         return li_launch_status();
     }
-    const bool listed = run_keys != nullptr;
-    if (listed && (n_tokens > RUN_KEYS_MAX_TOKENS || nsplit > 0x7fff)) return LI_ERR_SIZE;
     if (use_mfma == 2) {
         if (!part_acc || !part_ml) return LI_ERR_SIZE;
-        dim3 grid(listed ? n_tokens * nsplit : n_tokens, nkv, listed ? 1 : nsplit);
-#define LI_DM(DHV) paged_attention_decode_mfma_kernel<T, DHV, 1><<<grid, 64, 0, stream>>>( \
-        q, q_row_stride, out, kc, vc, block_table, max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, \
-        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, nsplit, listed ? run_keys : nullptr, n_tokens, \
-        nullptr)
-        if (dh == 128) LI_DM(128); else LI_DM(64);
-#undef LI_DM
+        const dim3 grid(listed ? n_tokens * nsplit : n_tokens, nkv, listed ? 1 : nsplit);
+        LI_DM(1, nsplit)
         dim3 g2(n_tokens, nh);
         attention_merge_kernel<T><<<g2, 128, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit,
                                                           listed ? run_keys + 2 : nullptr);
@@ -2475,12 +2507,10 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
     const int quads = nsplit / LI_DECODE_QUAD;
     if (quads > 1 && (!done || !part_acc || !part_ml)) return LI_ERR_SIZE;
     if ((long)n_tokens * quads > 0x7fffffffL) return LI_ERR_SIZE;
-    dim3 grid(listed ? n_tokens * quads : n_tokens, nkv, listed ? 1 : quads);
-#define LI_DM(DHV) paged_attention_decode_mfma_kernel<T, DHV, LI_DECODE_QUAD><<<grid, 64 * LI_DECODE_QUAD, 0, stream>>>( \
-        q, q_row_stride, out, kc, vc, block_table, max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, \
-        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, quads, listed ? run_keys : nullptr, n_tokens, done)
-    if (dh == 128) LI_DM(128); else LI_DM(64);
+    const dim3 grid(listed ? n_tokens * quads : n_tokens, nkv, listed ? 1 : quads);
+    LI_DM(LI_DECODE_QUAD, quads)
 #undef LI_DM
+#undef LI_DM4
     return li_launch_status();
 }
 

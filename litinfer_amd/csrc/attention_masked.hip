@@ -517,8 +517,8 @@ __global__ __launch_bounds__(64) void masked_attention_heads_kernel(
     __shared__ __attribute__((aligned(16))) uint16_t Vt[DV * MT_VS];      // [value column][key place, permuted]
     __shared__ int rows[3][32];                                           // the cache row of each key place of three blocks in turn, -1: none
     const int t = token_list ? token_list[blockIdx.x] : blockIdx.x, kvh = blockIdx.y;
-    const int s = seg_of_token[t];
-    const int p0 = ctx_len[s] - q_len[s] + (t - q_start[s]);              // the token's position
+    const int s = seg_of_token ? seg_of_token[t] : t;      // (null: token t is request t's only one)
+    const int p0 = seg_of_token ? ctx_len[s] - q_len[s] + (t - q_start[s]) : ctx_len[t] - 1;      // the token's position
     const int p_last = p0;
     const int lo_min = lower_edge(p0, window, ex.chunk);
     const int n_first = keep_first < lo_min ? keep_first : lo_min;
@@ -852,7 +852,7 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     if (other) { q += second.q_off; kc = second.kc; }
     const int rep = nh / nkv, hfirst = (blockIdx.z / nsplit) * RH, sp = blockIdx.z % nsplit;
     const int nheads = rep - hfirst < RH ? rep - hfirst : RH;
-    const int s = seg_of_token[t];
+    const int s = seg_of_token ? seg_of_token[t] : t;      // (null: token t is request t's only one)
     const int* table = block_table + (size_t)s * max_blocks;
     // (what does not hang on the position is on its way before the position is known: the heads of q, and, where every key is visible and
     // the room holds the whole table, the table)
@@ -870,7 +870,7 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     const bool whole = window <= 0 && ex.chunk <= 0 && max_blocks <= tab_cap;
     if (whole)
         for (int i = threadIdx.x; i < max_blocks; i += 256) tab[i] = table[i];
-    const int p = ctx_len[s] - q_len[s] + (t - q_start[s]);
+    const int p = seg_of_token ? ctx_len[s] - q_len[s] + (t - q_start[s]) : ctx_len[t] - 1;
     const int lo = lower_edge(p, window, ex.chunk);
     const int n_first = keep_first < lo ? keep_first : lo;
     const int n_all = n_first + (p - lo + 1);

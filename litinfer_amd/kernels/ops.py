@@ -901,7 +901,7 @@ def masked_attention(q: torch.Tensor, q_token_stride: int, q_head_stride: int, o
             return _run("attention_masked", "li_masked_attention_heads", q.data_ptr(), int(q_token_stride),
                         int(q_head_stride), out.data_ptr(), k.data_ptr(), v.data_ptr(), k.shape[3], v.shape[3],
                         meta.block_table.data_ptr(), meta.max_blocks, 0 if token_list is None else token_list.data_ptr(), n,
-                        meta.seg_of_token.data_ptr(), meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
+                        _seg_of_token(meta), meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
                         nh, nkv, dk, dv, page_size, k.shape[0], int(window), int(keep_first), float(softcap or 0.0),
                         float(scale), *fin, nsplit, parts, parts_n)
         if not (fast and masked_single_takes(dk, dv)):
@@ -919,7 +919,7 @@ def masked_attention(q: torch.Tensor, q_token_stride: int, q_head_stride: int, o
             parts, parts_n = buf.data_ptr(), buf.numel()
         _run("attention_masked", "li_masked_attention_single", q.data_ptr(), int(q_token_stride), int(q_head_stride),
              out.data_ptr(), k.data_ptr(), v.data_ptr(), k.shape[3], v.shape[3], meta.block_table.data_ptr(), meta.max_blocks,
-             0 if token_list is None else token_list.data_ptr(), n, meta.seg_of_token.data_ptr(), meta.q_start.data_ptr(),
+             0 if token_list is None else token_list.data_ptr(), n, _seg_of_token(meta), meta.q_start.data_ptr(),
              meta.q_len.data_ptr(), meta.ctx_len.data_ptr(), nh, nkv, dk, dv, page_size, k.shape[0], int(window),
              int(keep_first), float(softcap or 0.0), float(scale), *fin, nsplit, parts, parts_n)
 
@@ -993,7 +993,7 @@ def masked_attention_difference(q: torch.Tensor, q_token_stride: int, q_head_str
     parts = ws.buffer("masked_attention.parts", (2 * t * nh * nsplit * (dv + 2),), torch.float32)
     _run("attention_masked", "li_masked_attention_single_pair", q.data_ptr(), int(q_token_stride), int(q_head_stride), int(q_offset), out.data_ptr(),
          k1.data_ptr(), k2.data_ptr(), v.data_ptr(), k1.shape[3], v.shape[3], meta.block_table.data_ptr(), meta.max_blocks, t,
-         meta.seg_of_token.data_ptr(), meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(), nh, nkv, dk, dv, page_size,
+         _seg_of_token(meta), meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(), nh, nkv, dk, dv, page_size,
          k1.shape[0], int(window), int(keep_first), float(softcap or 0.0), float(scale), nsplit, parts.data_ptr(), parts.numel(), float(lam), float(eps),
          float(mult))
     return True
@@ -1485,7 +1485,42 @@ _decode_single_waves = False
 _DECODE_FILLS = 0.7
 
 
-def decode_splits(pairs: int, keys: int, simds: int = _DEC_WAVES, quad: int = DECODE_QUAD) -> int:
+
+
+def _seg_of_token(meta, takes: bool = True) -> int:
+    """The device array of the tokens' requests, or 0 (where the kernel takes that) if token t is request t's only one for every t: the
+    kernel then knows without a trip to memory."""
+    if not takes or not meta.num_single == meta.num_tokens == meta.num_segments:
+        return meta.seg_of_token.data_ptr()
+    in_order = meta.extra.get("in_order")
+    if in_order is None:
+        qs, ql = getattr(meta, "host_q_start", None), getattr(meta, "host_q_len", None)
+        in_order = meta.extra["in_order"] = bool(qs is not None and ql is not None and len(qs) == len(ql) == meta.num_segments
+                                                 and np.array_equal(qs, np.arange(len(qs))) and (np.asarray(ql) == 1).all())
+    return 0 if in_order else meta.seg_of_token.data_ptr()
+
+
+def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int):
+    """Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of
+    four runs a (token, kv head), which joins them itself and needs no list of runs; a pair of least lengths, runs of their own and the
+    kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan.
+    A run of 32 keys is a step, whose instructions (bfloat16, 0.9 us) or matrix products (float32, 1.8 us: six heads in tiles of 16) are
+    what it takes, and the second kernel with its trips to memory is 3 us.  Us a call, before / now:
+    bfloat16, 12 heads on 2 of 128, a table of 208 keys, 1 / 64 / 128 requests 8.3 / 10.0 / 13.2 -> 6.4 / 7.3 / 8.9; contexts of 30 to 300, 64 / 128
+    requests 11.0 / 15.2 -> 8.4 / 9.5, 3 requests 7.7 / 7.5; of 50 to 500, 3 requests 8.3 / 9.6 (so not there), 64 12.7 / 10.7; of 100 to 1,000,
+    16 / 64 / 128 requests 10.1 / 14.0, 16.7 / 16.0, 25.4 / 20.0.  Few requests of heads of 128, tables of 592 / 704 / 832 keys:
+    the four runs of a block 9.3 / 9.9 / 11.1 (1 request), 9.8 / 10.3 / 11.3 (16), runs of 64 keys and more 8.1 / 8.1 / 8.3, 9.1 / 9.4 / 9.7 (496 keys, 8 kv
+    heads: 7.7 / 7.9, so not there).
+    float32, 1 request of 150 / 300 / 600 / 1,000 keys 13.4 / 14.7 / 21.5 / 17.0 -> 8.8 / 9.0 / 11.4 / 12.5, 16 requests 14.2 / 15.2 / 26.0 / 20.2 -> 9.7 /
+    10.8 / 14.2 / 17.1; 3 of 50 to 500 keys 12.1 -> 10.0; up to 96 keys one run is the faster (7.8 / 8.5); 64 requests of 300 18.3 / 18.9."""
+    if dtype is torch.bfloat16:
+        if 128 < keys <= min(max(448, 10 * pairs), 1280):
+            return DECODE_QUAD
+        return (64,) if dh == 128 and quads == DECODE_QUAD and 512 < keys <= 1024 and pairs <= 32 else None
+    return (32, 64) if keys > 96 and (pairs <= 16 or (pairs <= 64 and keys <= 1280)) else None
+
+
+def decode_splits(pairs: int, keys: int, simds: int = _DEC_WAVES, quad: int = DECODE_QUAD, least: int = 128) -> int:
     """Into how many runs the keys of a decoding token are cut.  Every (token, kv head) pair and
     run is one wave, and a SIMD holds one wave of this kernel: the waves go over the SIMDs in
     rounds, each as long as a run (plus a wave's start and end, about 24 keys' time), so the
@@ -1493,7 +1528,7 @@ def decode_splits(pairs: int, keys: int, simds: int = _DEC_WAVES, quad: int = DE
     keys and at least 128 where the keys allow; every run costs the join a little (4 keys' time).
     The runs come in blocks of `quad` waves (a block joins its runs itself), so their number is 1
     or a multiple of `quad`.  Few pairs: as many runs as fill the SIMDs once."""
-    most = max(1, min(-(-keys // 128), DECODE_MAX_SPLITS))
+    most = max(1, min(-(-keys // least), DECODE_MAX_SPLITS))
     best, best_cost = 1, None
     for ns in [1] + list(range(quad, most + 1, quad)):
         run = (-(-keys // ns) + 31) & ~31
@@ -1618,6 +1653,16 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
                 quad = 1
                 planned = decode_splits(n_single * nkv, keys, simds, quad)
                 nsplit = _ragged_splits(planned, meta, window, quad)
+            runs = None if _decode_single_waves else _short_runs(n_single * nkv, keys, dh, qkv.dtype, nsplit if quad > 1 else 0)
+            if runs == DECODE_QUAD:
+                quad = nsplit = planned = DECODE_QUAD
+            elif runs is not None:
+                quad = 1
+                for least in runs:                     # (contexts that differ: the longer runs, the second number)
+                    planned = decode_splits(n_single * nkv, keys, simds, quad, least)
+                    nsplit = _ragged_splits(planned, meta, window, quad)
+                    if nsplit == planned:
+                        break
             # a split's pages must fit the kernel's copy of the block table
             while nsplit <= DECODE_MAX_SPLITS and decode_split_blocks(meta.max_blocks, page_size, window, nsplit) > DECODE_TABLE_CAP:
                 nsplit += 1 if nsplit < quad else quad
@@ -1661,7 +1706,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
                 meta.extra[key] = run_keys
         _run("attention", "li_paged_attention_decode", qkv.data_ptr(), qkv.stride(0), out.data_ptr(),
              k.data_ptr(), v.data_ptr(), _DT[qkv.dtype], bt.data_ptr(), meta.max_blocks,
-             0 if lst is None else lst.data_ptr(), n_single, meta.seg_of_token.data_ptr(),
+             0 if lst is None else lst.data_ptr(), n_single, _seg_of_token(meta, mfma),
              meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
              0 if acc is None else acc.data_ptr(), 0 if ml is None else ml.data_ptr(),
              nh, nkv, dh, page_size, k.shape[0], int(window), float(scale), nsplit,

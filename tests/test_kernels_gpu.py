@@ -769,6 +769,31 @@ def test_paged_attention(ops, dtype, segs, nh, nkv, dh, page, window):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("ctx,nh,nkv,dh,page,pad", [
+    ([1, 7, 8, 31, 32, 33, 95, 96], 14, 2, 64, 16, False), ([97, 128, 129], 6, 1, 64, 8, False), ([144] * 2, 12, 2, 128, 12, False),      # four runs a block, one
+    ([449, 450], 12, 2, 128, 16, False), ([513, 640, 700], 7, 1, 128, 16, False), ([700] * 3, 12, 2, 128, 8, False),       # runs of 64 keys and more
+    ([61, 300, 15], 12, 2, 128, 24, False), ([200, 9], 20, 1, 64, 16, False),                     # runs of 32 (float32); 20 heads: two passes
+    ([257, 130, 8], 5, 1, 128, 1, True), ([260 * 16 - 3, 4], 4, 1, 64, 16, False)])               # tables beyond the pages that are asked for ahead
+def test_single_tokens_of_few_keys(ops, dtype, ctx, nh, nkv, dh, page, pad):
+    """A request a token, in order, at the edges of the cuts of short contexts; a portion among them (then the tokens come by a
+    list) must not change what a token gets, and neither the requests' number passed or left out."""
+    from litinfer_amd.engine.workspace import Workspace
+    segs = [(c, 1) for c in ctx]
+    ws = Workspace(DEV)
+    out, ref = _paged_case(ops, dtype, segs, nh, nkv, dh, page, 0, seed=8, ws=ws, pad_pow2=pad)
+    assert rel(out, ref) < tol(dtype, 3e-6, 1.5e-2)
+    told, was = [], ops._seg_of_token
+    try:
+        ops._seg_of_token = lambda meta, takes=True: told.append(was(meta, takes)) or meta.seg_of_token.data_ptr()
+        by_list, _ = _paged_case(ops, dtype, segs, nh, nkv, dh, page, 0, seed=8, ws=ws, pad_pow2=pad)
+    finally:
+        ops._seg_of_token = was
+    assert told == [0] and torch.equal(out, by_list)
+    out, ref = _paged_case(ops, dtype, segs[:1] + [(40, 5)] + segs[1:], nh, nkv, dh, page, 0, seed=9, ws=ws, pad_pow2=pad)
+    assert rel(out, ref) < tol(dtype, 3e-6, 1.5e-2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("far", [3, 1000, 1999])
 def test_a_far_key_stands_out_in_a_decode_batch_of_unequal_contexts(ops, far, dtype):
     # contexts of 2,000 to 5,000 keys: the batch gets one run length and a list of its runs; one key of every
