@@ -6,6 +6,7 @@
 // runs in an order that depends on K and the number of parts K is cut into, not on the element's place; which kernel
 // and how many parts follow from M, N and K, so the rows of one call are all summed alike.
 #include "few_rows.h"
+#include "lds_loads.h"
 #include <algorithm>
 #include <type_traits>
 #include <utility>
@@ -842,27 +843,6 @@ __global__ __launch_bounds__(256) void gemm_bf16_big_kernel(const bf16_t* __rest
 // Needs K to be a multiple of the step (a load cannot be masked to zeros).  A step is 64
 // columns, so that a row of a stage is one whole 128-byte line of the caches.  Two to four stages (what fits the
 // 160 KB of LDS); which tiles are this kernel's and which `gemm_bf16_tile_kernel`'s: `tiling_of`, `gated_tiling_of`.
-#define LI_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 0xF) | (((n) >> 4) << 14) | 0x0F70)
-#define LI_LOAD_TO_LDS(gptr, lptr)                                                                        \
-    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(gptr),              \
-                                     (__attribute__((address_space(3))) void*)(lptr), 16, 0, 0)
-
-// f(std::integral_constant<int, 0>) ... f(std::integral_constant<int, N - 1>)
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-    (f(std::integral_constant<int, I>{}), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-    static_for_impl(f, std::make_integer_sequence<int, N>{});
-}
-
-// The same load with its address as (scalar base) + (32-bit offset of the lane): no address
-// arithmetic in vector registers.  M0 carries the LDS address, as in the compiler's own form.
-#define LI_LOAD_TO_LDS_AT(base, voff, lptr)                                                              \
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"                          \
-                 :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(voff), "s"(base) : "memory", "m0")
-
 // A wave's band of 32 rows of EW sums in LDS (ESTRIDE floats apart) goes to rows row0 .. and columns col0 .. of out: row by row,
 // 8 consecutive columns a lane, so that the stores (and the loads of what is added to) are whole 16-byte pieces.
 // GATED: the band holds results already; ACT otherwise: the activation of sums and bias.

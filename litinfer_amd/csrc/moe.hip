@@ -4,6 +4,7 @@
 // Nothing here returns to the host: the numbers of rows an expert gets stay on the device, and the launches are
 // sized by what a step can have at most.
 #include "few_rows.h"
+#include "lds_loads.h"
 
 #define MOE_TILE 32            // rows of one expert that a tile holds
 #define MOE_BIG_TILE 64        // ... where experts get hundreds of rows each (a prompt's portion): the tiles of the LDS kernel,
@@ -1135,6 +1136,167 @@ __global__ __launch_bounds__(256) void moe_linear_lds_kernel(const bf16_t* __res
 }
 
 // 1 if tiles of MOE_BIG_TILE rows have a kernel for these operands
+// Many rows an expert and K a multiple of 64: the same tiles with the loads going straight into LDS, two stages of 64 k-values in turn.  A
+// block takes a tile of 64 RF rows and 64 CF outputs, its four waves two by two; a lane's row of a matrix instruction is an output, its column
+// a row of the tile, and the k-values come in the order of the kernel above: the sums are the same bit for bit.
+// A stage holds the rows' and the matrix's pieces of 16 bytes, piece c of row r at place c ^ (r / 2 % 8) of the row's eight: the reads of 32
+// lanes fall into all banks.  The loads of the step ahead are issued one by one between the matrix instructions (back to back they
+// would hold the wave until the address unit has taken them); in the middle of a step's last group the wave waits for them and meets the
+// others.  Two blocks share a compute unit and cover each other's waits and the trips to memory before a block's first load; with three or
+// four stages and one block, or stages of 32 k-values and three blocks, the large cases took 10 to 20 % longer.
+// What it was bound by is the way from memory into the XCDs' L2 (some 9 TB/s were asked for): see the order of the blocks.
+// us, the kernel above / this one with its order of blocks / with the order below, random choices: 4,096 rows, 16 experts of 2,240 x 1,536 78.9 / 57.0 /
+// 50.7 (42.6 with 192 outputs a block), of 1,536 x 2,240 76.1 / 64.4 / 42.4; 8,000 rows, 14 of 4,480 x 1,536 203 / 162 / 154, of 1,536 x 2,240 125 /
+// 92 / 78; 4,096 rows, 8 of 9,472 x 3,584 487 / 404 / 390 (358); tiles of 64 rows: 2,048 rows, 16 of 2,240 x 1,536 54.6 / 43.0 / 31.7.
+#define MD_K 64
+#define MD_STAGES 2
+template <bool EXT, typename TO, int RF, int CF>
+__global__ __launch_bounds__(256) void moe_linear_dma_kernel(const bf16_t* __restrict__ a, long a_stride, const int* __restrict__ row_token,
+                                                             const bf16_t* __restrict__ w, const int* __restrict__ plan,
+                                                             TO* __restrict__ out, long out_stride, int n_out, int K, MoeEpilogue ep) {
+    constexpr int BK = MD_K, NSTAGE = MD_STAGES, ROWS = 64 * RF, COLS = 64 * CF, PP = BK / 8, WRAP = 128 / BK, RPI = 64 / PP, IA = ROWS / 4 / RPI, IW = COLS / 4 / RPI, LPW = IA + IW, STAGE = (ROWS + COLS) * BK, KS = BK / 16, GM = CF * RF;
+    extern __shared__ __align__(16) uint16_t stages[];
+    // Blocks go to the eight XCDs in turn.  Each XCD gets an eighth of the tiles, against all columns, and goes through them columns outside: its
+    // tiles' rows stay in its L2, and an expert's matrix comes into one or two of them, not into all.
+    const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3, tiles = plan[0];
+    const int t0 = (int)((long)xcd * tiles >> 3), mine = (int)((long)(xcd + 1) * tiles >> 3) - t0;
+    if (mine <= 0) return;
+    const int cb = idx / mine, tile = t0 + (idx - cb * mine);
+    if (cb * COLS >= n_out) return;
+    const int e = plan[4 + 4 * tile], r0 = plan[5 + 4 * tile], nr = plan[6 + 4 * tile];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ql = lane & 31, h2 = lane >> 5;
+    const int j0 = cb * COLS;
+    // this lane's part of a step: an instruction covers eight rows, lane l row l / 8, place l % 8
+    const bf16_t* ga[IA];
+    const bf16_t* gw[IW];
+#pragma unroll
+    for (int i = 0; i < IA; ++i) {
+        const int row = (ROWS / 4) * wv + RPI * i + lane / PP, c = (lane % PP) ^ ((row / WRAP) & (PP - 1));
+        const int r = r0 + (row < nr ? row : nr - 1);
+        ga[i] = a + (size_t)(row_token ? row_token[r] : r) * a_stride + 8 * c;
+    }
+#pragma unroll
+    for (int i = 0; i < IW; ++i) {
+        const int row = (COLS / 4) * wv + RPI * i + lane / PP, c = (lane % PP) ^ ((row / WRAP) & (PP - 1));
+        gw[i] = w + ((size_t)e * n_out + (j0 + row < n_out ? j0 + row : n_out - 1)) * K + 8 * c;
+    }
+    // load i of the wave's LPW of a step: its rows' first, then the matrix's
+    auto issue_one = [&](int kt, int i) {
+        uint16_t* st = stages + (kt % NSTAGE) * STAGE;
+        if (i < IA) LI_LOAD_TO_LDS_FROM(ga[i] + (size_t)kt * BK, st + ((ROWS / 4) * wv + RPI * i) * BK);
+        else LI_LOAD_TO_LDS_FROM(gw[i - IA] + (size_t)kt * BK, st + ROWS * BK + ((COLS / 4) * wv + RPI * (i - IA)) * BK);
+    };
+    const int nk = K / BK;
+    const int wr = wv >> 1, wc = wv & 1;               // the wave's 32 RF rows and 64 outputs
+    moe_f32x16 acc[RF][CF];
+#pragma unroll
+    for (int rf = 0; rf < RF; ++rf)
+#pragma unroll
+        for (int cf = 0; cf < CF; ++cf)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) acc[rf][cf][i] = 0.f;
+#pragma unroll
+    for (int p = 0; p < NSTAGE - 1; ++p)
+        if (p < nk)
+#pragma unroll
+            for (int i = 0; i < LPW; ++i) issue_one(p, i);
+    moe_frag8 fa[2][RF], fw[2][CF];
+    auto read = [&](int kt, int ks, int buf) {
+        const uint16_t* as = stages + (kt % NSTAGE) * STAGE;
+        const uint16_t* ws = as + ROWS * BK;
+#pragma unroll
+        for (int rf = 0; rf < RF; ++rf) {
+            const int row = 32 * RF * wr + 32 * rf + ql;
+            fa[buf][rf].raw = *reinterpret_cast<const uint4*>(&as[row * BK + (((2 * ks + h2) ^ ((row / WRAP) & (PP - 1))) << 3)]);
+        }
+#pragma unroll
+        for (int cf = 0; cf < CF; ++cf) {
+            const int row = 32 * CF * wc + 32 * cf + ql;
+            fw[buf][cf].raw = *reinterpret_cast<const uint4*>(&ws[row * BK + (((2 * ks + h2) ^ ((row / WRAP) & (PP - 1))) << 3)]);
+        }
+    };
+    auto multiply = [&](int buf, int m) {
+        acc[m / CF][m % CF] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[buf][m % CF].v, fa[buf][m / CF].v, acc[m / CF][m % CF], 0, 0, 0);
+    };
+    // the loads of steps that may stay in flight: `younger` of them
+    auto arrived = [&](int younger) {
+        if (younger >= 2) LI_VMCNT(2 * LPW); else if (younger == 1) LI_VMCNT(LPW); else LI_VMCNT(0);
+        __builtin_amdgcn_s_waitcnt(0xC07F);            // (lgkmcnt(0): this wave's reads of the stage that is given back are done)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    static_assert(NSTAGE <= 4, "at most two steps stay in flight behind the one that is waited for");
+    arrived((nk < NSTAGE - 1 ? nk : NSTAGE - 1) - 1);
+    read(0, 0, 0);
+    // LOADS: the step NSTAGE - 1 further on exists, and its loads are issued
+    auto step = [&](int kt, auto loads_tag) {
+        constexpr bool LOADS = decltype(loads_tag)::value;
+        static_for<KS - 1>([&](auto ks_tag) {
+            constexpr int ks = decltype(ks_tag)::value;
+            constexpr int l0 = LPW * ks / (KS - 1), l1 = LPW * (ks + 1) / (KS - 1);
+            read(kt, ks + 1, (ks + 1) & 1);
+            static_for<GM>([&](auto m_tag) {
+                constexpr int m = decltype(m_tag)::value;
+                multiply(ks & 1, m);
+                if constexpr (LOADS) {
+#pragma unroll
+                    for (int l = l0 + m * (l1 - l0) / GM; l < l0 + (m + 1) * (l1 - l0) / GM; ++l) issue_one(kt + NSTAGE - 1, l);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        });
+        constexpr int BL = (KS - 1) & 1;
+#pragma unroll
+        for (int m = 0; m < GM / 2; ++m) multiply(BL, m);
+        if (kt + 1 < nk) {
+            arrived(LOADS ? NSTAGE - 2 : (nk - 2 - kt < NSTAGE - 2 ? nk - 2 - kt : NSTAGE - 2));
+            read(kt + 1, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int m = GM / 2; m < GM; ++m) multiply(BL, m);
+    };
+    int kt = 0;
+    for (; kt + NSTAGE - 1 < nk; ++kt) step(kt, std::true_type{});
+    for (; kt < nk; ++kt) step(kt, std::false_type{});
+#pragma unroll
+    for (int rf = 0; rf < RF; ++rf) {
+        const int row = 32 * RF * wr + 32 * rf + ql;
+        if (row >= nr) continue;
+        TO* orow = out + (size_t)(r0 + row) * out_stride;
+        const float factor = moe_row_factor<EXT>(ep, r0 + row);
+#pragma unroll
+        for (int cf = 0; cf < CF; ++cf) {
+            if (j0 + 32 * CF * wc + 32 * cf >= n_out) continue;
+#pragma unroll
+            for (int rg = 0; rg < 4; ++rg)             // registers 4 rg .. 4 rg + 3: outputs 32 cf + 8 rg + 4 h2 ..
+                moe_store4<EXT>(orow, j0 + 32 * CF * wc + 32 * cf + 8 * rg + 4 * h2, acc[rf][cf][4 * rg], acc[rf][cf][4 * rg + 1],
+                                acc[rf][cf][4 * rg + 2], acc[rf][cf][4 * rg + 3], ep, factor);
+        }
+    }
+}
+// Outputs a block, 128 or 192, for tiles of 128 rows: by the rounds of two blocks a compute unit that they take (the tiles from the
+// choices' average: half a tile an expert is not full, and a twentieth more; 192 outputs read the rows less often, a twentieth in their favour).
+static bool moe_dma_wide(int rows, int max_tiles, int n_out) {
+    const float experts = (float)(max_tiles - rows / MOE_HUGE_TILE), tiles = 1.05f * ((float)rows / MOE_HUGE_TILE + 0.5f * experts);
+    const float slots = 2.f * compute_units();
+    return 0.95f * 3.f * ceilf(tiles * ((n_out + 191) / 192) / slots) < 2.f * ceilf(tiles * ((n_out + 127) / 128) / slots);
+}
+
+template <bool EXT, typename TO, int RF, int CF>
+static int launch_moe_dma(hipStream_t stream, const void* a, long a_stride, const int* row_token, const void* w, const int* plan, void* out,
+                          long out_stride, int n_out, int K, const MoeEpilogue& ep, int max_tiles) {
+    constexpr int COLS = 64 * CF, lds = MD_STAGES * (64 * RF + COLS) * MD_K * 2;
+    const dim3 grid((unsigned)((long)((max_tiles + 7) / 8) * ((n_out + COLS - 1) / COLS) * 8));
+    if constexpr (lds > 65536) {
+        static const hipError_t ready = hipFuncSetAttribute((const void*)moe_linear_dma_kernel<EXT, TO, RF, CF>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        if (ready != hipSuccess) return LI_ERR_LAUNCH;
+    }
+    moe_linear_dma_kernel<EXT, TO, RF, CF><<<grid, 256, lds, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (TO*)out, out_stride,
+                                                                           n_out, K, ep);
+    return li_launch_status();
+}
+
 extern "C" int li_moe_linear_big_takes(int a_dtype, int w_dtype, int n_out, int K) {
     return a_dtype == LI_BF16 && w_dtype == LI_BF16 && K % MB_K == 0 && n_out % 32 == 0;
 }
@@ -1170,6 +1332,15 @@ static int moe_linear_launch(const void* a, int a_dtype, long a_stride, const in
         const dim3 line((unsigned)((((long)max_tiles * ((n_out + MB_COLS - 1) / MB_COLS) + 63) / 64) * 64));
 #define ML(TO, RF) moe_linear_lds_kernel<EXT, TO, RF><<<line, 256, 0, stream>>>((const bf16_t*)a, a_stride, row_token, (const bf16_t*)w, plan, (TO*)out, out_stride, n_out, K, ep, max_tiles)
         const bool huge = tile_rows == MOE_HUGE_TILE;
+        if (K % MD_K == 0 && (out_dtype == LI_BF16 || out_dtype == LI_F32)) {
+#define MD(TO, RF, CF) return launch_moe_dma<EXT, TO, RF, CF>(stream, a, a_stride, row_token, w, plan, out, out_stride, n_out, K, ep, max_tiles)
+            const bool wide = huge && moe_dma_wide(rows, max_tiles, n_out);
+            if (out_dtype == LI_BF16) { if (!huge) MD(bf16_t, 1, 2); if (wide) MD(bf16_t, 2, 3); MD(bf16_t, 2, 2); }
+            if (!huge) MD(float, 1, 2);
+            if (wide) MD(float, 2, 3);
+            MD(float, 2, 2);
+#undef MD
+        }
         if (out_dtype == LI_BF16) { if (huge) ML(bf16_t, 2); else ML(bf16_t, 1); }
         else if (out_dtype == LI_F32) { if (huge) ML(float, 2); else ML(float, 1); }
         else return LI_ERR_DTYPE;

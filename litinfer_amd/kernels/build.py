@@ -35,7 +35,7 @@ FLAGS = ["-O3", "-std=c++17", "-shared", "-fPIC", f"--offload-arch={ARCH}",
 MODULE_FLAGS = {"attention": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                 # the products' loads into LDS are inline assembly that sets M0 and says so in its clobber
                 # list, which the compiler remarks upon for every instance
-                "gemm": ["-Wno-inline-asm"]}
+                "gemm": ["-Wno-inline-asm"], "moe": ["-Wno-inline-asm"]}
 
 MODULES = ("elementwise", "gemm", "attention", "attention_masked", "recurrent", "moe", "sampling", "host")     # what the models need
 # measuring kernels of the benchmark (a streaming read, a copy, a matrix-core loop): built with the

@@ -1474,6 +1474,50 @@ def test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, weigh, g
     assert rel(out, y.numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
 
 
+@pytest.mark.parametrize("counts,tile,n_out,k,act,weigh,gather,out_dtype", [
+    ([1, 64, 0, 65, 63], 64, 32, 64, 0, False, True, torch.float32),           # one step of k; a quarter of a block's outputs
+    ([130, 5, 200], 64, 160, 192, 2, False, True, torch.bfloat16),             # three steps, pairs of gate and up
+    ([1, 128, 0, 129, 127], 128, 96, 128, 4, True, True, torch.bfloat16),      # two steps, weights on the input
+    ([300, 3], 128, 288, 320, 3, False, False, torch.float32),
+    ([70, 200, 1], 128, 224, 96, 1, False, True, torch.float32),               # k no multiple of 64: the kernel that stages through registers
+    ([400, 390, 410, 401, 399, 380, 420, 400], 128, 2208, 64, 0, False, True, torch.float32),      # 192 outputs a block, the last half full
+    ([129] * 3, 128, 1056, 576, 2, False, True, torch.bfloat16)])              # fewer tiles than XCDs
+def test_routed_product_of_many_rows_an_expert(ops, counts, tile, n_out, k, act, weigh, gather, out_dtype):
+    """As of a decoding batch, in the tiles of a prompt's portion; places of the plan behind its last tile hold anything."""
+    g = torch.Generator(device=DEV).manual_seed(64)
+    rows, E = sum(counts), len(counts)
+    tokens = rows if not gather else rows + 3
+    wide = torch.randn(tokens, k + 8, generator=g, device=DEV).to(torch.bfloat16)       # rows with a stride of their own
+    a = wide[:, :k]
+    w = (torch.randn(E, n_out, k, generator=g, device=DEV) / math.sqrt(k) * 2).to(torch.bfloat16)
+    src = torch.randperm(tokens, generator=g, device=DEV)[:rows] if gather else torch.arange(rows, device=DEV)
+    row_wt = torch.rand(rows, generator=g, device=DEV) + 0.5 if weigh else None
+    tiles, r, ref = [], 0, []
+    for e, n in enumerate(counts):
+        tiles += [(e, r + o, min(tile, n - o), 0) for o in range(0, n, tile)]
+        y = a[src[r:r + n]].double() @ w[e].double().t().contiguous()
+        ref.append(y * row_wt[r:r + n, None].double() if weigh else y)
+        r += n
+    y = torch.cat(ref)
+    if act == 1:
+        y = y.clamp(min=0) ** 2
+    elif act == 2:
+        y = torch.nn.functional.silu(y[:, 0::2]) * y[:, 1::2]
+    elif act == 3:
+        gate, up = y[:, 0::2].clamp(max=1.5), y[:, 1::2].clamp(-1.5, 1.5)
+        y = gate * torch.sigmoid(1.702 * gate) * (up + 1.0)
+    elif act == 4:
+        y = torch.nn.functional.gelu(y)
+    most = rows // tile + E
+    plan = torch.full((4 + 4 * most,), 1 << 20, dtype=torch.int32)
+    plan[:4 + 4 * len(tiles)] = torch.tensor([len(tiles), rows, 0, 0] + [v for t in tiles for v in t], dtype=torch.int32)
+    out = torch.full((rows, y.shape[1]), float("nan"), dtype=out_dtype, device=DEV)
+    for _ in range(2):
+        ops.moe_linear(a, src.to(torch.int32) if gather else None, w, plan.to(DEV), most, out, rows, act=act, tile_rows=tile,
+                       limit=1.5 if act == 3 else 0.0, row_wt=row_wt)
+        assert rel(out, y.cpu().numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
+
+
 @pytest.mark.parametrize("k", [128, 512, 1160, 1536, 4736])
 def test_routed_product_of_a_decoding_batch_is_as_exact_as_of_few_rows(ops, k):
     """No further from the float64 result than the same rows four at a time, which another kernel takes."""
