@@ -768,6 +768,26 @@ def test_paged_attention(ops, dtype, segs, nh, nkv, dh, page, window):
     assert rel(out, ref) < tol(dtype, 3e-6, 1.5e-2)
 
 
+@pytest.mark.parametrize("taps,C,slots,bias", [(2, 5, [2], True), (3, 256, [0, 3], False), (4, 300, [4, 1, 0], True), (5, 257, [1, 2], True)])
+def test_convolution_of_one_token_a_request(ops, taps, C, slots, bias):
+    """A decoding step's outputs and moved tails (bit for bit), also of 5 taps, which the general kernel takes; other slots' tails stay."""
+    from types import SimpleNamespace
+    g = torch.Generator().manual_seed(taps * 100 + C)
+    T = len(slots)
+    wide, w, b, tail = torch.randn(T, C + 8, generator=g), torch.randn(C, taps, generator=g), torch.randn(C, generator=g), torch.randn(6, taps - 1, C, generator=g)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(num_tokens=T, num_segments=T, max_q_len=1, seg_of_token=i32(list(range(T))), q_start=i32(list(range(T))), q_len=i32([1] * T),
+                          state_slots=i32(slots), host_state_slots=np.array(slots, np.int32), host_q_len=np.ones(T, np.int32), host_q_start=np.arange(T, dtype=np.int32))
+    dev_tail, out = tail.to(DEV), torch.empty(T, C, device=DEV)
+    ops.causal_conv_silu(wide.to(DEV)[:, 4:4 + C], w.to(DEV), b.to(DEV) if bias else None, dev_tail, ctx, out)
+    seen = torch.cat([tail[slots], wide[:, None, 4:4 + C]], dim=1)
+    z = (seen.double() * w.t().double()).sum(1) + (b.double() if bias else 0.0)
+    assert (out.cpu().double() - z * torch.sigmoid(z)).abs().max() < 16 * taps * 2 ** -24 * (seen.abs() * w.t().abs()).sum(1).max()
+    moved = tail.clone()
+    moved[slots] = seen[:, 1:]
+    assert torch.equal(dev_tail.cpu(), moved)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("ctx,nh,nkv,dh,page,pad", [
     ([1, 7, 8, 31, 32, 33, 95, 96], 14, 2, 64, 16, False), ([97, 128, 129], 6, 1, 64, 8, False), ([144] * 2, 12, 2, 128, 12, False),      # four runs a block, one
