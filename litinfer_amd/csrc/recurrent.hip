@@ -1811,13 +1811,22 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
     const int t = blockIdx.x, c0 = blockIdx.y * gs;
     const float* yr = y + (size_t)t * y_stride + c0;
     const float* zr = z + (size_t)t * z_stride + c0;
-    float v[PER], gt[PER];
+    float v[PER], gt[PER], ry[PER], rz[PER], rw[PER];
     float ss = 0.f;
+    // (rows and weights are asked for together; a column past the group is its last one again, and counts for nothing)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        if (i * 256 >= gs) continue;
+        const int j = threadIdx.x + i * 256, jj = j < gs ? j : gs - 1;
+        ry[i] = yr[jj];
+        rz[i] = zr[jj];
+        rw[i] = w ? w[c0 + jj] : 1.f;
+    }
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int j = threadIdx.x + i * 256;
         float g = 0.f, sg = 0.f;
-        if (j < gs) { const float zz = zr[j]; sg = (gate_after == 2 ? 1.0f : zz) / (1.0f + expf(-zz)); g = gate_after ? yr[j] : yr[j] * sg; }
+        if (j < gs) { sg = (gate_after == 2 ? 1.0f : rz[i]) / (1.0f + expf(-rz[i])); g = gate_after ? ry[i] : ry[i] * sg; }
         v[i] = g;
         gt[i] = gate_after ? sg : 1.f;
         ss += g * g;
@@ -1832,7 +1841,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(const float* __re
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int j = threadIdx.x + i * 256;
-        if (j < gs) store_from_float(o + j, (w ? w[c0 + j] : 1.f) * v[i] * inv * gt[i]);
+        if (j < gs) store_from_float(o + j, rw[i] * v[i] * inv * gt[i]);
     }
     for (int j = threadIdx.x + PER * 256; j < gs; j += 256) {
         const float zz = zr[j], sg = (gate_after == 2 ? 1.0f : zz) / (1.0f + expf(-zz)), g = gate_after ? yr[j] : yr[j] * sg;
@@ -1853,15 +1862,23 @@ __global__ __launch_bounds__(256) void gated_group_norm_wave_kernel(const float*
     const int c0 = (int)(unit % groups) * gs;
     const float* yr = y + t * y_stride + c0;
     const float* zr = z + t * z_stride + c0;
-    float v[4], gt[4];
+    float v[4], gt[4], ry[4], rz[4], rw[4];
     float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (64 * i >= gs) continue;
+        const int j = lane + 64 * i, jj = j < gs ? j : gs - 1;
+        ry[i] = yr[jj];
+        rz[i] = zr[jj];
+        rw[i] = w ? w[c0 + jj] : 1.f;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int j = lane + 64 * i;
         v[i] = 0.f; gt[i] = 1.f;
         if (j < gs) {
-            const float zz = zr[j], sg = (gate_after == 2 ? 1.0f : zz) / (1.0f + expf(-zz));
-            v[i] = gate_after ? yr[j] : yr[j] * sg;
+            const float sg = (gate_after == 2 ? 1.0f : rz[i]) / (1.0f + expf(-rz[i]));
+            v[i] = gate_after ? ry[i] : ry[i] * sg;
             if (gate_after) gt[i] = sg;
         }
         ss = fmaf(v[i], v[i], ss);
@@ -1871,7 +1888,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_wave_kernel(const float*
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int j = lane + 64 * i;
-        if (j < gs) store_from_float(o + j, (w ? w[c0 + j] : 1.f) * v[i] * inv * gt[i]);
+        if (j < gs) store_from_float(o + j, rw[i] * v[i] * inv * gt[i]);
     }
 }
 

@@ -768,6 +768,47 @@ def test_paged_attention(ops, dtype, segs, nh, nkv, dh, page, window):
     assert rel(out, ref) < tol(dtype, 3e-6, 1.5e-2)
 
 
+@pytest.mark.parametrize("T,nh,nkv,dk,dv,rot,split,norm,store", [
+    (1, 1, 1, 2, 1, 2, False, True, True), (3, 16, 2, 64, 48, 64, True, True, True),          # a unit; two units a thread, all pairs
+    (2, 12, 2, 128, 128, 64, True, True, True), (2, 17, 3, 128, 128, 4, False, True, True),       # 1,024 threads, their units; one head too many for them
+    (5, 8, 8, 32, 32, 0, False, True, True), (2, 3, 1, 40, 257, 8, True, False, True), (4, 24, 1, 64, 64, 32, True, True, False)])
+def test_query_and_key_norms_of_short_and_long_rows(ops, T, nh, nkv, dk, dv, rot, split, norm, store):
+    """At and around the units a thread holds; float32 in the page cache, against float64 (a sum of n squares and a few roundings)."""
+    g = torch.Generator().manual_seed(dk * 7 + nh)
+    nq, nk, page = nh * dk, nkv * dk, 4
+    rows = torch.randn(T, nq + nk + nkv * dv + 3, generator=g)
+    wq, wk = 1 + torch.randn(nq, generator=g) / 8, 1 + torch.randn(nk, generator=g) / 8
+    ang = torch.rand(T, max(rot // 2, 1), generator=g) * 6
+    cos, sin = ang.cos(), ang.sin()
+    slots = torch.randperm(3 * page, generator=g)[:T].to(torch.int32)
+    gpu = lambda x: x.to(DEV)
+    d = gpu(rows)
+    kc, vc = torch.full((3, nkv, page, dk), 7.0, device=DEV), torch.full((3, nkv, page, dv), 7.0, device=DEV)
+    ops.qk_norm_pairs_store(d, nh, nkv, dk, dv, rot, gpu(wq) if norm else None, gpu(wk) if norm else None, 1e-5, gpu(cos[:, :rot // 2].contiguous()),
+                            gpu(sin[:, :rot // 2].contiguous()), gpu(slots) if store else None, kc if store else None, vc if store else None, page, half_split=split)
+
+    def ref(x, w, heads):
+        x = x.double()
+        y = x / (x.square().mean(1, keepdim=True) + 1e-5).sqrt() * w.double() if norm else x
+        y, half = y.view(T, heads, dk).clone(), rot // 2
+        i = torch.arange(half)
+        a, b = (i, i + half) if split else (2 * i, 2 * i + 1)
+        c, s_ = cos[:, None, :half].double(), sin[:, None, :half].double()
+        u, v = y[..., a], y[..., b]
+        y[..., a], y[..., b] = u * c - v * s_, u * s_ + v * c
+        return y
+    bound = (nq + 16) * 2 ** -24 * 6
+    assert (d.cpu()[:, :nq].double() - ref(rows[:, :nq], wq, nh).reshape(T, nq)).abs().max() < bound
+    assert torch.equal(d.cpu()[:, nq:], rows[:, nq:])
+    k, v = kc.cpu().transpose(1, 2).reshape(-1, nkv, dk), vc.cpu().transpose(1, 2).reshape(-1, nkv, dv)
+    other = torch.ones(3 * page, dtype=torch.bool)
+    if store:
+        other[slots.long()] = False
+        assert (k[slots.long()].double() - ref(rows[:, nq:nq + nk], wk, nkv)).abs().max() < bound
+        assert torch.equal(v[slots.long()], rows[:, nq + nk:nq + nk + nkv * dv].reshape(T, nkv, dv))
+    assert (k[other] == 7.0).all() and (v[other] == 7.0).all()
+
+
 @pytest.mark.parametrize("taps,C,slots,bias", [(2, 5, [2], True), (3, 256, [0, 3], False), (4, 300, [4, 1, 0], True), (5, 257, [1, 2], True)])
 def test_convolution_of_one_token_a_request(ops, taps, C, slots, bias):
     """A decoding step's outputs and moved tails (bit for bit), also of 5 taps, which the general kernel takes; other slots' tails stay."""
