@@ -1554,6 +1554,30 @@ static int launch_tile(const bf16_t* x, const bf16_t* w, const float* bias, TO* 
     return li_launch_status();
 }
 
+// The sum of up to MID_PARTS parts, in their order.  All loads at once (a part past the last reads the first and is not added): the kernels
+// that add up have few blocks and must not wait for memory part after part.  FEW: up to 64 rows, which alone have more than 8 parts; where
+// there are many rows the question alone made a step of 1,027 tokens 4 % longer.
+#define MID_PARTS 16
+template <bool FEW>
+__device__ __forceinline__ float parts_sum(const float* __restrict__ part, int nsplit, size_t mn, size_t at) {
+    float a[8];
+    [[maybe_unused]] float b[8];
+#pragma unroll
+    for (int sp = 0; sp < 8; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + at];
+    if (FEW && nsplit > 8) {
+#pragma unroll
+        for (int sp = 0; sp < 8; ++sp) b[sp] = part[(size_t)(8 + sp < nsplit ? 8 + sp : 0) * mn + at];
+    }
+    float t = a[0];
+#pragma unroll
+    for (int sp = 1; sp < 8; ++sp) t += sp < nsplit ? a[sp] : 0.f;
+    if (FEW && nsplit > 8) {
+#pragma unroll
+        for (int sp = 0; sp < 8; ++sp) t += 8 + sp < nsplit ? b[sp] : 0.f;
+    }
+    return t;
+}
+
 // out (+)= sum over the parts, in the order of the parts, + bias
 template <typename TO>
 __global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
@@ -1566,16 +1590,12 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit,
 }
 
 // out = act(sum over the parts + bias), bfloat16 (see li_linear_act)
+template <bool FEW>
 __global__ __launch_bounds__(256) void splitk_reduce_act_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                 const float* __restrict__ bias, bf16_t* __restrict__ out, LiAct ep) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
-    float a[8];
-#pragma unroll
-    for (int sp = 0; sp < 8; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + i];      // (all loads at once)
-    float v = a[0];
-#pragma unroll
-    for (int sp = 1; sp < 8; ++sp) v += sp < nsplit ? a[sp] : 0.f;
+    float v = parts_sum<FEW>(part, nsplit, mn, i);
     if (bias) v += bias[(int)(i % N)];
     store_from_float(out + i, activation(v, ep));
 }
@@ -1605,7 +1625,7 @@ __global__ __launch_bounds__(256) void act_of_sums_kernel(const float* __restric
 // result: out[m, :] += factor * (sum of the parts + bias) (float32), xn[m, :] = gamma * out[m, :] /
 // sqrt(mean(out[m, :]^2) + eps).  A row is kept in registers (N <= NT * PER).
 // THERE: the sum is in `out` already, and its norm alone is written (nsplit does not matter).
-template <typename TN, int NT, int PER, bool THERE = false>
+template <typename TN, int NT, int PER, bool FEW, bool THERE = false>
 __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                  const float* __restrict__ bias, float* __restrict__ out,
                                                                  float factor, const float* __restrict__ gamma, float eps,
@@ -1613,7 +1633,11 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
     __shared__ float red[NT / LI_WAVE];
     const size_t row = (size_t)blockIdx.x * N;
     float v[PER];
+    [[maybe_unused]] float g[PER];
     float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i)                       // (few rows: the norm's weights come with the parts, not behind the sum of squares)
+        if (FEW && i * NT < N) g[i] = gamma[(int)threadIdx.x + i * NT < N ? threadIdx.x + i * NT : N - 1];
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int n = threadIdx.x + i * NT;
@@ -1621,15 +1645,8 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
         if constexpr (THERE) {
             if (n < N) v[i] = out[row + n];
         } else if (n < N) {
-            // all loads at once (a part past the last reads the first and is not added): the block is
-            // one of few and must not wait for memory part after part
-            float a[8];
-#pragma unroll
-            for (int sp = 0; sp < 8; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + row + n];
             const float o = out[row + n];
-            float t = a[0];
-#pragma unroll
-            for (int sp = 1; sp < 8; ++sp) t += sp < nsplit ? a[sp] : 0.f;
+            float t = parts_sum<FEW>(part, nsplit, mn, row + n);
             if (bias) t += bias[n];
             t = fmaf(factor, t, o);
             out[row + n] = t;
@@ -1642,13 +1659,13 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int n = threadIdx.x + i * NT;
-        if (n < N) store_from_float(xn + row + n, gamma[n] * v[i] * inv);
+        if (n < N) store_from_float(xn + row + n, (FEW ? g[i] : gamma[n]) * v[i] * inv);
     }
 }
 
 // The same with a tanh norm, which takes no statistics of a row: out += factor * (sum of the parts + bias) (float32),
 // xn = tanh(alpha * out) * gamma + beta, element by element.
-template <typename TN>
+template <typename TN, bool FEW>
 __global__ __launch_bounds__(256) void splitk_reduce_tanh_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                  const float* __restrict__ bias, float* __restrict__ out,
                                                                  float factor, float alpha, const float* __restrict__ gamma,
@@ -1656,13 +1673,8 @@ __global__ __launch_bounds__(256) void splitk_reduce_tanh_kernel(const float* __
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
     const int n = (int)(i % N);
-    float a[8];
-#pragma unroll
-    for (int sp = 0; sp < 8; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + i];      // (all loads at once, as above)
     const float o = out[i], g = gamma[n], b = beta[n];
-    float t = a[0];
-#pragma unroll
-    for (int sp = 1; sp < 8; ++sp) t += sp < nsplit ? a[sp] : 0.f;
+    float t = parts_sum<FEW>(part, nsplit, mn, i);
     if (bias) t += bias[n];
     t = fmaf(factor, t, o);
     out[i] = t;
@@ -1840,6 +1852,15 @@ extern "C" int li_four_tiles_preferred(int M, long N, long K) {
     return M > FEW_ROWS_TWO_TILES && M <= 64 && K % 8 == 0 && K <= (M <= 48 ? FOUR_TILES_K : FOUR_TILES_LAST_K) && N <= 16l * compute_units();
 }
 
+// Parts of K for up to 64 rows and fewer than 128 tiles of 128 columns: blocks for every compute unit, at least 8 steps a part.  (Up to MID_PARTS,
+// where 8 were: 64 x 1,536 x 8,960, 12 tiles, with the norm 17.5 -> 15.2 us.)
+static int mid_parts(int N, int K) {
+    int nsplit = 256 / ((N + 127) / 128);
+    if (nsplit > MID_PARTS) nsplit = MID_PARTS;
+    if (nsplit > K / 64 / 8) nsplit = K / 64 / 8;
+    return nsplit;
+}
+
 static bool mid_rows_take(int M, int N, int K) {
     return !li_few_rows_preferred(M, N, K) && M <= 64;
 }
@@ -1854,9 +1875,7 @@ static int linear_mid_rows(const bf16_t* x, const bf16_t* w, const float* bias, 
     const int tiles = (N + 127) / 128;
     if (tiles >= 128)
         return out_dtype == LI_F32 ? LI_MID(128, 4, float, out, bias, accumulate, 1) : LI_MID(128, 4, bf16_t, out, bias, accumulate, 1);
-    int nsplit = 256 / tiles;
-    if (nsplit > 8) nsplit = 8;
-    if (nsplit > K / 64 / 8) nsplit = K / 64 / 8;              // at least 8 steps a part
+    const int nsplit = mid_parts(N, K);
     const size_t mn = (size_t)M * N;
     if (nsplit < 2 || !work || (size_t)work_bytes < (size_t)nsplit * mn * sizeof(float)) return -1;
     const int rc = LI_MID(128, 4, float, work, nullptr, 0, nsplit);
@@ -2066,11 +2085,7 @@ extern "C" long li_linear_work_bytes(int M, int N, int K, int in_dtype) {
     int nsplit = 1;
     if (M <= 64) {
         const int tiles = (N + 127) / 128;
-        if (tiles < 128) {
-            nsplit = 256 / tiles;
-            if (nsplit > 8) nsplit = 8;
-            if (nsplit > K / 64 / 8) nsplit = K / 64 / 8;
-        }
+        if (tiles < 128) nsplit = mid_parts(N, K);
     } else {
         nsplit = split_parts_many_rows(M, N, K);
     }
@@ -2090,15 +2105,15 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
     if (need <= 0 || !work || work_bytes < need) return -1;
     const size_t mn = (size_t)M * N;
     const int nsplit = (int)(need / (long)(mn * sizeof(float)));
-    if (nsplit > 8) return -1;                      // (the adding-up kernel takes up to 8 parts)
+    if (nsplit > MID_PARTS) return -1;
     if (li_four_tiles_preferred(M, N, K)) {         // K whole: the sum, then its norm
         const int rc = li_linear_skinny(x, w, bias, out, M, N, K, LI_F32, factor, 0, stream);
         if (rc != LI_OK) return rc;
         if (xn_dtype == LI_BF16)
-            splitk_reduce_norm_kernel<bf16_t, REDUCE_NORM_NT, REDUCE_NORM_PER, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
+            splitk_reduce_norm_kernel<bf16_t, REDUCE_NORM_NT, REDUCE_NORM_PER, true, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
                 nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (bf16_t*)xn);
         else
-            splitk_reduce_norm_kernel<float, REDUCE_NORM_NT, REDUCE_NORM_PER, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
+            splitk_reduce_norm_kernel<float, REDUCE_NORM_NT, REDUCE_NORM_PER, true, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
                 nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (float*)xn);
         return li_launch_status();
     }
@@ -2106,12 +2121,11 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
         ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit)
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit);
     if (rc != LI_OK) return rc;
-    if (xn_dtype == LI_BF16)
-        splitk_reduce_norm_kernel<bf16_t, REDUCE_NORM_NT, REDUCE_NORM_PER><<<M, REDUCE_NORM_NT, 0, stream>>>(
-            (const float*)work, nsplit, mn, N, bias, out, factor, gamma, eps, (bf16_t*)xn);
-    else
-        splitk_reduce_norm_kernel<float, REDUCE_NORM_NT, REDUCE_NORM_PER><<<M, REDUCE_NORM_NT, 0, stream>>>(
-            (const float*)work, nsplit, mn, N, bias, out, factor, gamma, eps, (float*)xn);
+#define LI_RN(TN, FEW) splitk_reduce_norm_kernel<TN, REDUCE_NORM_NT, REDUCE_NORM_PER, FEW><<<M, REDUCE_NORM_NT, 0, stream>>>( \
+        (const float*)work, nsplit, mn, N, bias, out, factor, gamma, eps, (TN*)xn)
+    if (xn_dtype == LI_BF16) { if (M <= 64) LI_RN(bf16_t, true); else LI_RN(bf16_t, false); }
+    else { if (M <= 64) LI_RN(float, true); else LI_RN(float, false); }
+#undef LI_RN
     return li_launch_status();
 }
 
@@ -2135,16 +2149,16 @@ extern "C" int li_linear_tanh_norm(const void* x, const void* w, const float* bi
     if (need <= 0 || !work || work_bytes < need) return -1;
     const size_t mn = (size_t)M * N;
     const int nsplit = (int)(need / (long)(mn * sizeof(float)));
-    if (nsplit > 8) return -1;                      // (the adding-up kernel takes up to 8 parts)
+    if (nsplit > MID_PARTS) return -1;
     const int rc = M <= 64
         ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit)
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
     if (rc != LI_OK) return rc;
     const unsigned blocks = (unsigned)((mn + 255) / 256);
-    if (xn_dtype == LI_BF16)
-        splitk_reduce_tanh_kernel<bf16_t><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, out, factor, alpha, gamma, beta, (bf16_t*)xn);
-    else
-        splitk_reduce_tanh_kernel<float><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, out, factor, alpha, gamma, beta, (float*)xn);
+#define LI_RT(TN, FEW) splitk_reduce_tanh_kernel<TN, FEW><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, out, factor, alpha, gamma, beta, (TN*)xn)
+    if (xn_dtype == LI_BF16) { if (M <= 64) LI_RT(bf16_t, true); else LI_RT(bf16_t, false); }
+    else { if (M <= 64) LI_RT(float, true); else LI_RT(float, false); }
+#undef LI_RT
     return li_launch_status();
 }
 
@@ -2279,7 +2293,7 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
     if (need > 0) {                                  // K in parts, or in one
         const size_t mn = (size_t)M * N;
         const int nsplit = (int)(need / (long)(mn * sizeof(float)));
-        if (!work || (uintptr_t)work % 16 || work_bytes < need || nsplit > 8) return -1;
+        if (!work || (uintptr_t)work % 16 || work_bytes < need || nsplit > MID_PARTS) return -1;
         const int rc = M <= 64 && nsplit == 1 && (N + 255) / 256 >= 128
             ? launch_dma<64, 256, 64, 3, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream)
             : M <= 64
@@ -2287,7 +2301,8 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
             : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
         if (rc != LI_OK) return rc;
         if (nsplit == 1) act_of_sums_kernel<<<(unsigned)((mn + 1023) / 1024), 256, 0, stream>>>((const float*)work, mn, N, bias, (bf16_t*)out, ep);
-        else splitk_reduce_act_kernel<<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
+        else if (M <= 64) splitk_reduce_act_kernel<true><<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
+        else splitk_reduce_act_kernel<false><<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
         return li_launch_status();
     }
 #define LI_ACT(BM, BN, NS) launch_dma<BM, BN, 64, NS, false, bf16_t, LI_ACT_RELU2>((const bf16_t*)x, (const bf16_t*)w, bias, (bf16_t*)out, M, N, K, 0.f, stream, 1, nullptr, 0, 0.f, ep)

@@ -1065,7 +1065,7 @@ def headwise_linear(x: torch.Tensor, x_token_stride: int, x_head_stride: int, m:
 
 # ---------------------------------------------------------------------- gemm
 SKINNY_MAX_ROWS = 64
-SPLITK_MAX_PARTS = 8
+SPLITK_MAX_PARTS = 16
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
