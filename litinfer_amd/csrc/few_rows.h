@@ -645,8 +645,7 @@ static int compute_units() {
 // most blocks.  Every unit therefore gets one block and every block the same number of columns (at
 // most two tiles' worth, at least a quarter of a tile's), not whole tiles.  (At least a quarter, where a half was: 896 x 4,864 at one row
 // 6.05 -> 5.53 us with twice the blocks.)
-static int balanced_per_block(int total, int unit) {
-    const int cu = compute_units();
+static int balanced_per_block(int total, int unit, int cu) {
     int per = (total + cu - 1) / cu;
     per = per < unit / 4 ? unit / 4 : per;
     return per > 2 * unit ? 0 : per;
@@ -656,8 +655,7 @@ static int balanced_per_block(int total, int unit) {
 // the units with one block more than the others set the time when the matrix is small.  The columns a
 // block takes are therefore cut down until the last round is as full as the others: as many rounds as
 // whole tiles would need, and equal shares of the columns within them (at least half a tile's).
-static int balanced_round_cols(int total, int unit) {
-    const long cu = compute_units();
+static int balanced_round_cols(int total, int unit, long cu) {
     const long rounds = (total + unit * cu - 1) / (unit * cu);
     long per = (total + rounds * cu - 1) / (rounds * cu);
     per = per < unit / 2 ? unit / 2 : per;
@@ -673,9 +671,19 @@ static int balanced_round_cols(int total, int unit) {
 static bool rows_kernel_takes(int M, long columns, int K) {
     return M <= ROWS_KERNEL_M && K % 64 == 0 && (K <= 2048 || columns <= 2048);
 }
+// Columns a block of it takes on cu compute units, 1 to 16: a block has one tile of 16.  One block a unit where that is enough for them, else
+// whole rounds of blocks.  0: the product is the kernel's above, which has blocks of two tiles.  into_sum: out is added to; such a sum comes
+// out of one kernel whether or not its shares of the rows' squares are asked for, whose number goes with the columns alone (li_residual_norm_parts)
+static int rows_kernel_cols(int M, int N, int K, bool into_sum, int cu) {
+    if (!rows_kernel_takes(M, N, K)) return 0;
+    if (N <= 16l * cu) return balanced_per_block(N, 16, cu);
+    return into_sum ? 0 : balanced_round_cols(N, 16, cu);
+}
 
 template <typename TO, bool ROPE, int EPI>
-static void launch_rows(const SkinnyArgs& a, int blocks, hipStream_t stream) {
+static int launch_rows(const SkinnyArgs& a, int total, hipStream_t stream) {
+    if (a.cols < 1 || a.cols > (ROPE ? 8 : 16)) return LI_ERR_SIZE;      // (a block writes one tile)
+    const int blocks = (total + a.cols - 1) / a.cols;
     const int log_rows = a.M <= 1 ? 0 : a.M <= 2 ? 1 : 2;
     const int n = (a.K / 64 + FR_WAVES - 1) / FR_WAVES;              // a wave's units
 #define LI_FR(D, LOOP, X2, X4)                                                                                                          \
@@ -687,6 +695,7 @@ static void launch_rows(const SkinnyArgs& a, int blocks, hipStream_t stream) {
     else if constexpr (!ROPE) {
         if (n <= 10) LI_FR(10, false, 3, 5)
         else LI_FR(4, true, 1, 2)
-    }
+    } else return LI_ERR_SIZE;
 #undef LI_FR
+    return li_launch_status();
 }

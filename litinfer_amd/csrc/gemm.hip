@@ -1704,20 +1704,15 @@ static int launch_big(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
 
 
 template <bool SWIGLU, typename TO, int EPI = 0>
-static void launch_skinny(SkinnyArgs a, hipStream_t stream) {
-    const int M = a.M, N = a.N;
+static int launch_skinny(SkinnyArgs a, hipStream_t stream) {
+    const int M = a.M, N = a.N, cu = compute_units();
     if constexpr (!SWIGLU) {
-        // (a sum into out comes out of one kernel whether or not its shares of the rows' squares are asked for, whose number goes with the
-        // columns alone: li_residual_norm_parts)
-        if (rows_kernel_takes(M, N, a.K) && (a.accumulate == 0.f || N <= 4096)) {
-            a.cols = N <= 4096 ? balanced_per_block(N, 16) : balanced_round_cols(N, 16);
-            launch_rows<TO, false, EPI>(a, (N + a.cols - 1) / a.cols, stream);
-            return;
-        }
+        a.cols = rows_kernel_cols(M, N, a.K, a.accumulate != 0.f, cu);
+        if (a.cols > 0) return launch_rows<TO, false, EPI>(a, N, stream);
     }
 #define LI_SK(MT, NT, WV) gemm_bf16_skinny_kernel<MT, NT, WV, SWIGLU, TO, false, EPI><<<(N + 16 * (SWIGLU ? 1 : NT) - 1) / (16 * (SWIGLU ? 1 : NT)), WV * 64, 0, stream>>>(a)
     if constexpr (SWIGLU) {
-        a.cols = balanced_round_cols(N, 16);
+        a.cols = balanced_round_cols(N, 16, cu);
         const int blocks = (N + a.cols - 1) / a.cols;
         if (M <= 16) gemm_bf16_skinny_kernel<1, 2, 4, true, TO, false, EPI><<<blocks, 4 * 64, 0, stream>>>(a);
         else if (M <= 32) gemm_bf16_skinny_kernel<2, 2, 4, true, TO, false, EPI><<<blocks, 4 * 64, 0, stream>>>(a);
@@ -1725,23 +1720,24 @@ static void launch_skinny(SkinnyArgs a, hipStream_t stream) {
     } else if (N >= 8192) {                                 // many columns: many blocks, two tiles share each piece of x
         if (M <= 16) LI_SK(1, 2, 4); else if (M <= 32) LI_SK(2, 2, 4); else LI_SK(4, 2, 8);
     } else if (M <= 16) {                                   // few columns: a block a compute unit, eight waves split K
-        a.cols = balanced_per_block(N, 16);
+        a.cols = balanced_per_block(N, 16, cu);
         const int per = a.cols ? a.cols : 16, blocks = (N + per - 1) / per;
         if (per > 16) gemm_bf16_skinny_kernel<1, 2, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
         else gemm_bf16_skinny_kernel<1, 1, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
     } else if (M <= 32) {
-        a.cols = balanced_per_block(N, 16);
+        a.cols = balanced_per_block(N, 16, cu);
         const int per = a.cols ? a.cols : 16, blocks = (N + per - 1) / per;
         if (per > 16) gemm_bf16_skinny_kernel<2, 2, 4, false, TO, false, EPI><<<blocks, 4 * 64, 0, stream>>>(a);
         else gemm_bf16_skinny_kernel<2, 1, 4, false, TO, false, EPI><<<blocks, 4 * 64, 0, stream>>>(a);
     } else {                                                // 33 to 64 rows: rows up to 48 are three tiles
-        a.cols = balanced_per_block(N, 16);
+        a.cols = balanced_per_block(N, 16, cu);
         const int per = a.cols ? a.cols : 16, blocks = (N + per - 1) / per;
         if (per > 16) gemm_bf16_skinny_kernel<4, 2, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
         else if (M <= 48) gemm_bf16_skinny_kernel<3, 1, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
         else gemm_bf16_skinny_kernel<4, 1, 8, false, TO, false, EPI><<<blocks, 8 * 64, 0, stream>>>(a);
     }
 #undef LI_SK
+    return li_launch_status();
 }
 
 // Few rows (M <= 64), bfloat16, K a multiple of 8.  swiglu: w has 2 N rows ([gate; up]).
@@ -1752,25 +1748,23 @@ extern "C" int li_linear_skinny(const void* x, const void* w, const float* bias,
     if (swiglu && (bias || accumulate || out_dtype != LI_BF16)) return LI_ERR_DTYPE;
     SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, accumulate,
                  nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
-    if (swiglu) launch_skinny<true, bf16_t>(a, stream);
-    else if (out_dtype == LI_BF16) launch_skinny<false, bf16_t>(a, stream);
-    else if (out_dtype == LI_F32) launch_skinny<false, float>(a, stream);
-    else return LI_ERR_DTYPE;
-    return li_launch_status();
+    if (swiglu) return launch_skinny<true, bf16_t>(a, stream);
+    if (out_dtype == LI_BF16) return launch_skinny<false, bf16_t>(a, stream);
+    if (out_dtype == LI_F32) return launch_skinny<false, float>(a, stream);
+    return LI_ERR_DTYPE;
 }
 
 // The packed projection of up to 64 rows, rotated and written into its pages (SkinnyArgs: ROPE).
 static int launch_skinny_rope(SkinnyArgs a, hipStream_t stream) {
-    const int M = a.M, pairs = a.N / 2, half = a.dh / 2;
+    const int M = a.M, pairs = a.N / 2, half = a.dh / 2, cu = compute_units();
     if ((unsigned long long)pairs * half >= (1ull << 32)) return LI_ERR_SIZE;
     a.half_magic = (unsigned)(((1ull << 32) + half - 1) / half);
-    if (rows_kernel_takes(M, a.N, a.K) && a.K <= 2048 && pairs <= 8l * compute_units()) {
-        const int even = (pairs + compute_units() - 1) / compute_units();
+    if (rows_kernel_takes(M, a.N, a.K) && a.K <= 2048 && pairs <= 8l * cu) {
+        const int even = (pairs + cu - 1) / cu;
         a.cols = even < 3 ? 3 : even;                   // (576 pairs of 896: 3 a block 4.47 us, 4 4.66, 2 4.90)
-        launch_rows<bf16_t, true, 0>(a, (pairs + a.cols - 1) / a.cols, stream);
-        return li_launch_status();
+        return launch_rows<bf16_t, true, 0>(a, pairs, stream);
     }
-    a.cols = balanced_per_block(pairs, 8);
+    a.cols = balanced_per_block(pairs, 8, cu);
     const int per = a.cols ? a.cols : 8, blocks = (pairs + per - 1) / per;
     if (M <= 16) {
         if (per > 8) gemm_bf16_skinny_kernel<1, 2, 8, false, bf16_t, true><<<blocks, 8 * 64, 0, stream>>>(a);
@@ -1792,8 +1786,12 @@ static int launch_skinny_rope(SkinnyArgs a, hipStream_t stream) {
 // blocks, i.e. of parts.
 extern "C" int li_residual_norm_parts(int N) {
     int per = 32;                                      // as launch_skinny tiles the columns of few rows
-    if (N < 8192) { per = balanced_per_block(N, 16); per = per ? per : 16; }
+    if (N < 8192) { per = balanced_per_block(N, 16, compute_units()); per = per ? per : 16; }
     return (N + per - 1) / per;
+}
+// Columns a block of the kernel of one to four rows takes on a device of cu compute units, 0 where it does not take the product
+extern "C" int li_rows_kernel_cols(int M, int N, int K, int into_sum, int cu) {
+    return M > 0 && N > 0 && K > 0 && cu > 0 ? rows_kernel_cols(M, N, K, into_sum != 0, cu) : 0;
 }
 
 extern "C" int li_linear_residual_norm(const void* x, const void* w, const float* bias, float* out, int M, int N,
@@ -1802,8 +1800,7 @@ extern "C" int li_linear_residual_norm(const void* x, const void* w, const float
     if (li_residual_norm_parts(N) > SK_MAX_PARTS) return LI_ERR_SIZE;
     SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, factor,
                  nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, gamma, (bf16_t*)xg, sq_parts, nullptr, 0, 0.f};
-    launch_skinny<false, float>(a, stream);
-    return li_launch_status();
+    return launch_skinny<false, float>(a, stream);
 }
 
 // Between 13 and 64 rows (a large decoding batch) the product is still bound by streaming W, but
@@ -2142,8 +2139,7 @@ extern "C" int li_linear_tanh_norm(const void* x, const void* w, const float* bi
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, gamma, (bf16_t*)xn, nullptr, nullptr, 0, 0.f};
         a.beta = beta;
         a.alpha = alpha;
-        launch_skinny<false, float, 1>(a, stream);
-        return li_launch_status();
+        return launch_skinny<false, float, 1>(a, stream);
     }
     const long need = li_linear_work_bytes(M, N, K, LI_BF16);
     if (need <= 0 || !work || work_bytes < need) return -1;
@@ -2286,8 +2282,7 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, bias, out, M, N, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, nullptr, 0, 0.f};
         a.ep = ep;
-        launch_skinny<false, bf16_t, 2>(a, stream);
-        return li_launch_status();
+        return launch_skinny<false, bf16_t, 2>(a, stream);
     }
     const long need = li_linear_act_work_bytes(M, N, K, act);
     if (need > 0) {                                  // K in parts, or in one
@@ -2399,9 +2394,7 @@ extern "C" int li_linear_swiglu(const void* x, const void* w, void* out, int M, 
         SkinnyArgs a{(const bf16_t*)x, (const bf16_t*)w, nullptr, out, M, I, K, 0.f,
                      nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0, 0, 0, nullptr, nullptr, nullptr, row_parts, nparts, eps};
         a.ep = ep;
-        if (act) launch_skinny<true, bf16_t, 1>(a, stream);
-        else launch_skinny<true, bf16_t>(a, stream);
-        return li_launch_status();
+        return act ? launch_skinny<true, bf16_t, 1>(a, stream) : launch_skinny<true, bf16_t>(a, stream);
     }
     if (M <= 64) return li_linear_skinny(x, w, nullptr, out, M, I, K, LI_BF16, 0, 1, stream);
     if (K % 64) return LI_ERR_SIZE;

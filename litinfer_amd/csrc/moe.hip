@@ -1461,7 +1461,7 @@ static bool beside_form(SkinnyArgs& a, const void* x, const void* w, void* out, 
     if (T <= 0 || T > MOE_BESIDE_ROWS || N <= 0 || K <= 0 || K % 8 || ((uintptr_t)x | (uintptr_t)w) % 16 || (uintptr_t)out % 4) return false;
     form = T <= ROWS_KERNEL_M && K % 64 == 0 ? BESIDE_ROWS : T <= 16 ? BESIDE_ONE_TILE : BESIDE_TWO_TILES;
     a = SkinnyArgs{(const bf16_t*)x, (const bf16_t*)w, nullptr, out, T, N, K, 0.f};
-    a.cols = balanced_round_cols(N, 16);
+    a.cols = balanced_round_cols(N, 16, compute_units());
     blocks = (N + a.cols - 1) / a.cols;
     log_rows = T <= 1 ? 0 : T <= 2 ? 1 : 2;
     return true;

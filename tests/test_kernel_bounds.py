@@ -144,3 +144,22 @@ def test_tiles_of_products(gated, m, n, k, result_bytes, tile):
     f = ops._lib_fn("gemm", "li_linear_tile", [ctypes.c_int] * 5, ctypes.c_int)
     got = f(gated, m, n, k, result_bytes)
     assert (abs(got) >> 16, abs(got) & 65535, got < 0) == tile
+
+
+@pytest.mark.parametrize("units", [1, 32, 64, 128, 256, 304])
+def test_columns_a_block_of_the_kernel_of_one_to_four_rows(units):
+    """A block of that kernel writes one tile of 16 columns, however many compute units the device has: with more columns a block
+    some would never be written.  A sum takes as many blocks as its shares of the rows' squares are counted by."""
+    f = ops._lib_fn("gemm", "li_rows_kernel_cols", [ops.c_int] * 5, ops.c_int)
+    taken = 0
+    for n in [1, 15, 16, 17, 896, 1152, 1536, 2048, 3072, 3584, 4095, 4096, 4097, 4608, 4864, 4865, 8240, 17920, 151936, 16 * units, 16 * units + 1]:
+        for k in (64, 896, 2048, 2112, 11008, 100):
+            for m in (1, 2, 4, 5):
+                for into_sum in (0, 1):
+                    cols = f(m, n, k, into_sum, units)
+                    fits = m <= 4 and k % 64 == 0 and (k <= 2048 or n <= 2048) and (n <= 16 * units or not into_sum)
+                    assert (1 <= cols <= 16) if fits else cols == 0, (m, n, k, into_sum, units, cols)
+                    if fits and n <= 16 * units:
+                        assert cols == max(4, -(-n // units))
+                    taken += fits
+    assert taken
