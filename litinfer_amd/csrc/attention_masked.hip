@@ -909,9 +909,11 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
             for (int e = 0; e < 8; ++e) acc[hh][c][e] = 0.f;
     }
     const float inv_cap = softcap > 0.f ? 1.0f / softcap : 0.f;
-    // the rows of a round's keys (a key past the last: row 0, read and not used) and their pieces; the next round's
+    // the rows of a round's keys and their pieces; a place past the last key stands for the last key once more, whose weight there is 0: the
+    // row of another request, or a page never written, could hold infinities, and 0 times those is no number.  The next round's
     // are asked for before this round's are used, without a condition (a load under a condition would make every
-    // later use wait for all loads); the last round is taken behind the loop, which asks for nothing
+    // later use wait for all loads); the last round is taken behind the loop, which asks for nothing, and not where the block's share has no key
+    const int i_last = n_keys > 0 ? n_keys - 1 : 0;
     size_t ro[U];
     bool ok[U];
     int kpos[U];                                    // the keys' positions
@@ -923,13 +925,14 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     _Pragma("unroll") for (int u = 0; u < U; ++u) {                                                                  \
         const int i = (I0) + 32 * u + 8 * w + g;                                                                     \
         OK[u] = i < n_keys;                                                                                          \
-        const int ii = OK[u] ? i : 0;                                                                                \
+        const int ii = OK[u] ? i : i_last;                                                                           \
         const int key = visible_key(ii, n_first, lo);                                                                \
         KPOS[u] = key;                                                                                               \
         const int blk = pshift >= 0 ? key >> pshift : key / page_size;                                               \
         const int page = in_lds ? tab[ii < n_first ? nb_w + blk : blk - b_lo] : table[blk];                          \
-        OK[u] = OK[u] && page >= 0 && page < num_pages;                                                              \
-        RO[u] = OK[u] ? (size_t)(page * nkv + kvh) * page_size + (key - blk * page_size) : 0;                        \
+        const bool there = page >= 0 && page < num_pages;                                                            \
+        OK[u] = OK[u] && there;                                                                                      \
+        RO[u] = there ? (size_t)(page * nkv + kvh) * page_size + (key - blk * page_size) : 0;                        \
     }
 #define MS_FETCH(RO, KP, VP)                                                                                         \
     _Pragma("unroll") for (int u = 0; u < U; ++u) {                                                                  \
@@ -1012,7 +1015,7 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
             for (int c = 0; c < NPV; ++c) vp[u][c] = vp2[u][c];
         }
     }
-    round();
+    if (i_begin < n_keys) round();
 #undef MS_ROWS
 #undef MS_FETCH
     // The groups of a wave: the maximum over them, every group's sums scaled to it once, and the sums added up by halves: a lane keeps

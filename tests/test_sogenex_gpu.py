@@ -579,6 +579,51 @@ def test_difference_of_two_maps_in_a_decoding_step(ctxs, nh, nkv, dk, dv, page, 
     assert not ops.masked_attention_difference(qd.view(-1), q.shape[1], dk, nh * dk, out, k1, k2, v, meta, *args, 0.37, 1e-5, 0.8, ws)
 
 
+@pytest.mark.parametrize("fill", [float("inf"), float("nan")])
+@pytest.mark.parametrize("nh,nkv,dk,dv,window,keep", [(12, 2, 128, 128, 0, 0), (12, 12, 64, 64, 0, 0), (4, 1, 320, 256, 0, 0), (8, 2, 64, 128, 40, 3)])
+def test_rows_that_are_not_the_request_s_own_do_not_reach_it(nh, nkv, dk, dv, window, keep, fill):
+    """Page 0 belongs to nobody here and holds no numbers, nor do the places behind every request's last key: single tokens with fewer
+    keys than the table is cut into splits, and with rounds that are not full, give what they give with zeros there."""
+    from litinfer_amd.engine.batch import AttentionMeta
+    from litinfer_amd.engine.workspace import Workspace
+    from litinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(nh + dk)
+    page, width, ctxs = 16, 256, [1, 2, 17, 33, 250, 1100, 4096]
+    n, pages = len(ctxs), [-(-c // 16) for c in ctxs]
+    ids = 1 + torch.randperm(sum(pages), generator=g)
+    tab, at = torch.full((n, width), -1, dtype=torch.int32), 0
+    own = torch.zeros(len(ids) + 1, 1, page, 1, dtype=torch.bool)
+    for i, p in enumerate(pages):
+        tab[i, :p] = ids[at:at + p].int()
+        for b in range(p):
+            own[ids[at + b], 0, :min(page, ctxs[i] - b * page)] = True
+        at += p
+    pools = [torch.randn(len(own), nkv, page, d, generator=g).to(torch.bfloat16) for d in (dk, dk, dv)]
+    q = torch.randn(n, 2 * nh * dk, generator=g).to(DEV)
+    one, ctx, first = np.ones(n, dtype=np.int32), np.asarray(ctxs, dtype=np.int32), np.arange(n, dtype=np.int32)
+    dev = lambda a: torch.from_numpy(a).to(DEV)
+    meta = AttentionMeta(block_table=tab.to(DEV), max_blocks=width, seg_of_token=dev(first), q_start=dev(first), q_len=dev(one), ctx_len=dev(ctx),
+                         num_segments=n, num_tokens=n, max_q_len=1, max_ctx_len=int(ctx.max()), host_q_start=first, host_q_len=one,
+                         host_ctx_len=ctx, num_single=n, num_multi=0)
+    args, was = (nh, nkv, dk, dv, page, window, keep, 0.0, dk ** -0.5), ops._heads_kernel_pays
+    got = []
+    for value in (0.0, fill):
+        k1, k2, v = [torch.where(own, x, torch.tensor(value, dtype=x.dtype)).to(DEV) for x in pools]
+        outs = []
+        try:
+            for heads in (False, True):
+                ops._heads_kernel_pays = lambda *a: heads
+                outs.append(torch.empty(n, nh * dv, dtype=torch.bfloat16, device=DEV))
+                ops.masked_attention(q.view(-1), q.shape[1], dk, outs[-1], k1, v, meta, *args, ws=Workspace(DEV))
+        finally:
+            ops._heads_kernel_pays = was
+        outs.append(torch.empty(n, nh * dv, dtype=torch.bfloat16, device=DEV))
+        assert ops.masked_attention_difference(q.view(-1), q.shape[1], dk, nh * dk, outs[-1], k1, k2, v, meta, *args, 0.37, 1e-5, 0.8, Workspace(DEV))
+        got.append(outs)
+    for a, b in zip(*got):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, b)
+
+
 def test_position_vector_and_capped_logits():
     from litinfer_amd.kernels import ops
     for H in (96, 7):
