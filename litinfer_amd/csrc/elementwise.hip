@@ -477,7 +477,9 @@ __global__ __launch_bounds__(NT) void rmsnorm_add_kernel(const float* __restrict
     const float* yr2 = y2 ? y2 + (size_t)blockIdx.x * H : nullptr;
     float* xr = x + (size_t)blockIdx.x * H;
     float ss = 0.f;
-    if (H <= RA_HELD * NT) {                           // short rows: a thread's columns wait in registers, all asked for at once (8 x 1,536 3.8 -> 3.2 us)
+    // Short rows: a thread's columns wait in registers, all asked for at once (8 x 1,536 3.8 -> 3.2 us).  Not where there are thousands and most
+    // threads have no column of their own, whose loads are then what the chip is busy with (2,048 x 64 3.6 -> 3.9).
+    if (H <= RA_HELD * NT && (2 * H > NT || gridDim.x <= 1024)) {
         float b[RA_HELD], u[RA_HELD], r[RA_HELD], g[RA_HELD], g2[RA_HELD];
 #pragma unroll
         for (int i = 0; i < RA_HELD; ++i) {
@@ -661,13 +663,14 @@ extern "C" int li_rope_pairs_apply(void* x, int dtype, int row_stride, int n_hea
 // norms the WHOLE query projection and the WHOLE key projection (all heads at once, before they are split) and
 // rotates pairs of columns (neighbours, or with half_split column i and column i + rotary_dim / 2): q is normed and rotated in place (it stays float32), k is normed, rotated and
 // written to its page slot, v is copied to its page slot.  wq / wk null: no norm.  One block a token.
-template <typename T, int NT>
+template <typename T, int NT, bool NORMED>
 __global__ __launch_bounds__(NT) void qk_norm_pairs_store_kernel(
     float* __restrict__ qkv, int row_stride, int nh, int nkv, int dk, int dv, int rotary_dim,
     const float* __restrict__ wq, const float* __restrict__ wk, float eps,
     const float* __restrict__ cosv, const float* __restrict__ sinv, const int* __restrict__ slot_map,
     T* __restrict__ kc, T* __restrict__ vc, int page_size, int store, int half_split) {
     __shared__ float red[NT / LI_WAVE];
+    if constexpr (!NORMED) wq = wk = nullptr;
     const int t = blockIdx.x, half = rotary_dim / 2;
     float* q = qkv + (size_t)t * row_stride;
     float* k = q + (size_t)nh * dk;
@@ -675,9 +678,10 @@ __global__ __launch_bounds__(NT) void qk_norm_pairs_store_kernel(
     const int nq = nh * dk, nk = nkv * dk;
     float inv_q = 1.f, inv_k = 1.f;
     const int units = half + (dk - rotary_dim);            // per head: the pairs, then the columns that are not rotated
-    if (nh * units <= 2 * NT && nkv * units <= NT && nkv * dv <= NT) {
-        // A short row (a decoding step): a thread holds two units of q, one of k and one of v with all that belongs to them, asked for at once
-        // (sum after sum and part after part, each with its own trip to weights and angles: 8 tokens of 12 heads of 128 8.3 -> 3.8 us).
+    if (NORMED && nh * units <= 2 * NT && nkv * units <= NT && nkv * dv <= NT) {
+        // A short row (a decoding step) with a norm: a thread holds two units of q, one of k and one of v with all that belongs to them, asked for
+        // at once (sum after sum and part after part, each with its own trip to weights and angles: 8 tokens of 12 heads of 128 8.3 -> 3.8 us).
+        // Without one the loops below are independent as they stand, and there is nothing to wait for (2.9 us, here 3.8; 28 heads 3.3, 4.0).
         __shared__ float red2[NT / LI_WAVE];
         struct Unit { int j, j2, i; bool on, pair; float a, b, wa, wb, c, s; } un[3];
         const int slot = store ? slot_map[t] : 0;
@@ -811,17 +815,20 @@ extern "C" int li_qk_norm_pairs_store(float* qkv, int row_stride, int nh, int nk
         return LI_ERR_SIZE;
     // few rows (a decoding step): 1024 threads a row, so that the one row is gone through with the least latency
     const bool wide = T < 256 && nh * dk > 1024;
-#define LI_QK(TC)                                                                                                            \
-    {                                                                                                                        \
-        if (wide) qk_norm_pairs_store_kernel<TC, 1024><<<T, 1024, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, \
-                                                                              cosv, sinv, slot_map, (TC*)kc, (TC*)vc, page_size, store, half_split); \
-        else qk_norm_pairs_store_kernel<TC, 256><<<T, 256, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps,  \
-                                                                        cosv, sinv, slot_map, (TC*)kc, (TC*)vc, page_size, store, half_split);  \
+#define LI_QKN(TC, NT, NORMED)                                                                                                              \
+    qk_norm_pairs_store_kernel<TC, NT, NORMED><<<T, NT, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, cosv, sinv, \
+                                                                     slot_map, (TC*)kc, (TC*)vc, page_size, store, half_split)
+#define LI_QK(TC)                                                                            \
+    {                                                                                        \
+        if (wq || wk) { if (wide) LI_QKN(TC, 1024, true); else LI_QKN(TC, 256, true); }      \
+        else if (wide) LI_QKN(TC, 1024, false);                                              \
+        else LI_QKN(TC, 256, false);                                                         \
     }
     if (cache_dtype == LI_F32) LI_QK(float)
     else if (cache_dtype == LI_BF16) LI_QK(bf16_t)
     else return LI_ERR_DTYPE;
 #undef LI_QK
+#undef LI_QKN
     return li_launch_status();
 }
 
