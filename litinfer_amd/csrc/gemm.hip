@@ -1554,29 +1554,35 @@ static int launch_tile(const bf16_t* x, const bf16_t* w, const float* bias, TO* 
     return li_launch_status();
 }
 
-// The sum of up to MID_PARTS parts, in their order.  All loads at once (a part past the last reads the first and is not added): the kernels
-// that add up have few blocks and must not wait for memory part after part.  FEW: up to 64 rows, which alone have more than 8 parts; where
-// there are many rows the question alone made a step of 1,027 tokens 4 % longer.
+// The sum of up to PARTS_HELD parts, or with MORE up to MID_PARTS, in their order.  All loads at once (a part past the last reads the first and
+// is not added): the kernels that add up have few blocks and must not wait for memory part after part.  MORE goes by the number of parts, not
+// by the rows: the question inside the kernel made a step of 1,027 tokens 4 % longer, and one of 33 to 64 rows with 8 parts and fewer 2 to 3 %.
+#define PARTS_HELD 8
 #define MID_PARTS 16
-template <bool FEW>
-__device__ __forceinline__ float parts_sum(const float* __restrict__ part, int nsplit, size_t mn, size_t at) {
-    float a[8];
-    [[maybe_unused]] float b[8];
+template <bool MORE>
+struct Parts {
+    float a[PARTS_HELD], b[MORE ? PARTS_HELD : 1];
+    // (asked for before what else a kernel needs, whose addresses take a division: a tanh norm of 33 to 64 rows 2 to 4 % longer the other way)
+    __device__ __forceinline__ void ask(const float* __restrict__ part, int nsplit, size_t mn, size_t at) {
 #pragma unroll
-    for (int sp = 0; sp < 8; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + at];
-    if (FEW && nsplit > 8) {
+        for (int sp = 0; sp < PARTS_HELD; ++sp) a[sp] = part[(size_t)(sp < nsplit ? sp : 0) * mn + at];
+        if constexpr (MORE) {
 #pragma unroll
-        for (int sp = 0; sp < 8; ++sp) b[sp] = part[(size_t)(8 + sp < nsplit ? 8 + sp : 0) * mn + at];
+            for (int sp = 0; sp < PARTS_HELD; ++sp) b[sp] = part[(size_t)(PARTS_HELD + sp < nsplit ? PARTS_HELD + sp : 0) * mn + at];
+        }
     }
-    float t = a[0];
+    __device__ __forceinline__ float sum(int nsplit) const {
+        float t = a[0];
 #pragma unroll
-    for (int sp = 1; sp < 8; ++sp) t += sp < nsplit ? a[sp] : 0.f;
-    if (FEW && nsplit > 8) {
+        for (int sp = 1; sp < PARTS_HELD; ++sp) t += sp < nsplit ? a[sp] : 0.f;
+        if constexpr (MORE) {
 #pragma unroll
-        for (int sp = 0; sp < 8; ++sp) t += 8 + sp < nsplit ? b[sp] : 0.f;
+            for (int sp = 0; sp < PARTS_HELD; ++sp) t += PARTS_HELD + sp < nsplit ? b[sp] : 0.f;
+        }
+        return t;
     }
-    return t;
-}
+};
+static_assert(MID_PARTS == 2 * PARTS_HELD, "every part that a product is cut into is added up");
 
 // out (+)= sum over the parts, in the order of the parts, + bias
 template <typename TO>
@@ -1590,12 +1596,14 @@ __global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit,
 }
 
 // out = act(sum over the parts + bias), bfloat16 (see li_linear_act)
-template <bool FEW>
+template <bool MORE>
 __global__ __launch_bounds__(256) void splitk_reduce_act_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                 const float* __restrict__ bias, bf16_t* __restrict__ out, LiAct ep) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
-    float v = parts_sum<FEW>(part, nsplit, mn, i);
+    Parts<MORE> parts;
+    parts.ask(part, nsplit, mn, i);
+    float v = parts.sum(nsplit);
     if (bias) v += bias[(int)(i % N)];
     store_from_float(out + i, activation(v, ep));
 }
@@ -1625,7 +1633,7 @@ __global__ __launch_bounds__(256) void act_of_sums_kernel(const float* __restric
 // result: out[m, :] += factor * (sum of the parts + bias) (float32), xn[m, :] = gamma * out[m, :] /
 // sqrt(mean(out[m, :]^2) + eps).  A row is kept in registers (N <= NT * PER).
 // THERE: the sum is in `out` already, and its norm alone is written (nsplit does not matter).
-template <typename TN, int NT, int PER, bool FEW, bool THERE = false>
+template <typename TN, int NT, int PER, bool FEW, bool MORE, bool THERE = false>
 __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                  const float* __restrict__ bias, float* __restrict__ out,
                                                                  float factor, const float* __restrict__ gamma, float eps,
@@ -1645,8 +1653,10 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
         if constexpr (THERE) {
             if (n < N) v[i] = out[row + n];
         } else if (n < N) {
+            Parts<MORE> parts;
+            parts.ask(part, nsplit, mn, row + n);
             const float o = out[row + n];
-            float t = parts_sum<FEW>(part, nsplit, mn, row + n);
+            float t = parts.sum(nsplit);
             if (bias) t += bias[n];
             t = fmaf(factor, t, o);
             out[row + n] = t;
@@ -1665,16 +1675,18 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
 
 // The same with a tanh norm, which takes no statistics of a row: out += factor * (sum of the parts + bias) (float32),
 // xn = tanh(alpha * out) * gamma + beta, element by element.
-template <typename TN, bool FEW>
+template <typename TN, bool MORE>
 __global__ __launch_bounds__(256) void splitk_reduce_tanh_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                  const float* __restrict__ bias, float* __restrict__ out,
                                                                  float factor, float alpha, const float* __restrict__ gamma,
                                                                  const float* __restrict__ beta, TN* __restrict__ xn) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     if (i >= mn) return;
+    Parts<MORE> parts;
+    parts.ask(part, nsplit, mn, i);
     const int n = (int)(i % N);
     const float o = out[i], g = gamma[n], b = beta[n];
-    float t = parts_sum<FEW>(part, nsplit, mn, i);
+    float t = parts.sum(nsplit);
     if (bias) t += bias[n];
     t = fmaf(factor, t, o);
     out[i] = t;
@@ -2030,7 +2042,7 @@ static int split_parts_many_rows(int M, int N, int K) {
     const long tiles = (long)((M + 127) / 128) * ((N + 127) / 128);
     if (tiles >= 128) return 1;
     int nsplit = (int)(256 / tiles);
-    if (nsplit > 8) nsplit = 8;
+    if (nsplit > PARTS_HELD) nsplit = PARTS_HELD;
     if (nsplit > K / 64 / 8) nsplit = K / 64 / 8;              // at least 8 steps a part
     return nsplit < 2 ? 1 : nsplit;
 }
@@ -2107,10 +2119,10 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
         const int rc = li_linear_skinny(x, w, bias, out, M, N, K, LI_F32, factor, 0, stream);
         if (rc != LI_OK) return rc;
         if (xn_dtype == LI_BF16)
-            splitk_reduce_norm_kernel<bf16_t, REDUCE_NORM_NT, REDUCE_NORM_PER, true, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
+            splitk_reduce_norm_kernel<bf16_t, REDUCE_NORM_NT, REDUCE_NORM_PER, true, false, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
                 nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (bf16_t*)xn);
         else
-            splitk_reduce_norm_kernel<float, REDUCE_NORM_NT, REDUCE_NORM_PER, true, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
+            splitk_reduce_norm_kernel<float, REDUCE_NORM_NT, REDUCE_NORM_PER, true, false, true><<<M, REDUCE_NORM_NT, 0, stream>>>(
                 nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (float*)xn);
         return li_launch_status();
     }
@@ -2118,10 +2130,10 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
         ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit)
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit);
     if (rc != LI_OK) return rc;
-#define LI_RN(TN, FEW) splitk_reduce_norm_kernel<TN, REDUCE_NORM_NT, REDUCE_NORM_PER, FEW><<<M, REDUCE_NORM_NT, 0, stream>>>( \
+#define LI_RN(TN, FEW, MORE) splitk_reduce_norm_kernel<TN, REDUCE_NORM_NT, REDUCE_NORM_PER, FEW, MORE><<<M, REDUCE_NORM_NT, 0, stream>>>( \
         (const float*)work, nsplit, mn, N, bias, out, factor, gamma, eps, (TN*)xn)
-    if (xn_dtype == LI_BF16) { if (M <= 64) LI_RN(bf16_t, true); else LI_RN(bf16_t, false); }
-    else { if (M <= 64) LI_RN(float, true); else LI_RN(float, false); }
+    if (xn_dtype == LI_BF16) { if (nsplit > PARTS_HELD) LI_RN(bf16_t, true, true); else if (M <= 64) LI_RN(bf16_t, true, false); else LI_RN(bf16_t, false, false); }
+    else { if (nsplit > PARTS_HELD) LI_RN(float, true, true); else if (M <= 64) LI_RN(float, true, false); else LI_RN(float, false, false); }
 #undef LI_RN
     return li_launch_status();
 }
@@ -2151,9 +2163,9 @@ extern "C" int li_linear_tanh_norm(const void* x, const void* w, const float* bi
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
     if (rc != LI_OK) return rc;
     const unsigned blocks = (unsigned)((mn + 255) / 256);
-#define LI_RT(TN, FEW) splitk_reduce_tanh_kernel<TN, FEW><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, out, factor, alpha, gamma, beta, (TN*)xn)
-    if (xn_dtype == LI_BF16) { if (M <= 64) LI_RT(bf16_t, true); else LI_RT(bf16_t, false); }
-    else { if (M <= 64) LI_RT(float, true); else LI_RT(float, false); }
+#define LI_RT(TN, MORE) splitk_reduce_tanh_kernel<TN, MORE><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, out, factor, alpha, gamma, beta, (TN*)xn)
+    if (xn_dtype == LI_BF16) { if (nsplit > PARTS_HELD) LI_RT(bf16_t, true); else LI_RT(bf16_t, false); }
+    else { if (nsplit > PARTS_HELD) LI_RT(float, true); else LI_RT(float, false); }
 #undef LI_RT
     return li_launch_status();
 }
@@ -2296,7 +2308,7 @@ extern "C" int li_linear_act(const void* x, const void* w, const float* bias, vo
             : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0.f, stream, nsplit);
         if (rc != LI_OK) return rc;
         if (nsplit == 1) act_of_sums_kernel<<<(unsigned)((mn + 1023) / 1024), 256, 0, stream>>>((const float*)work, mn, N, bias, (bf16_t*)out, ep);
-        else if (M <= 64) splitk_reduce_act_kernel<true><<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
+        else if (nsplit > PARTS_HELD) splitk_reduce_act_kernel<true><<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
         else splitk_reduce_act_kernel<false><<<(unsigned)((mn + 255) / 256), 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, ep);
         return li_launch_status();
     }

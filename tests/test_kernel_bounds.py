@@ -163,3 +163,15 @@ def test_columns_a_block_of_the_kernel_of_one_to_four_rows(units):
                         assert cols == max(4, -(-n // units))
                     taken += fits
     assert taken
+
+
+def test_products_are_cut_into_no_more_parts_than_are_added_up():
+    """The kernels that add up the parts of K hold sixteen, and eight above 64 rows; a rope or plain sum counts as far as it is told."""
+    most = {True: 0, False: 0}
+    for m in (17, 33, 48, 64, 65, 128, 300, 1000):
+        for n in (8, 64, 128, 896, 1536, 2048, 3584, 4608, 8192):
+            for k in (64, 512, 1024, 1536, 4096, 8960, 18944, 65536):
+                need = ops._work_bytes(m, n, k, ops._DT[ops.torch.bfloat16])
+                assert need % (4 * m * n) == 0
+                most[m <= 64] = max(most[m <= 64], need // (4 * m * n))
+    assert most[True] == ops.SPLITK_MAX_PARTS == 16 and most[False] == 8

@@ -768,6 +768,33 @@ def test_paged_attention(ops, dtype, segs, nh, nkv, dh, page, window):
     assert rel(out, ref) < tol(dtype, 3e-6, 1.5e-2)
 
 
+@pytest.mark.parametrize("m,n,k,parts", [(33, 200, 4096, 8), (64, 136, 4608, 9), (40, 300, 7744, 15), (64, 264, 9024, 16), (65, 264, 9024, 8)])
+def test_products_of_many_parts_and_what_follows_them(ops, m, n, k, parts):
+    """K in up to sixteen parts (eight above 64 rows): every kernel that adds them up adds all of them."""
+    assert ops._work_bytes(m, n, k, ops._DT[torch.bfloat16]) == 4 * m * n * parts
+    g = torch.Generator().manual_seed(83)
+    x = torch.randn(m, k, generator=g).to(torch.bfloat16)
+    w = (torch.randn(n, k, generator=g) / math.sqrt(k)).to(torch.bfloat16)
+    b, base = torch.randn(n, generator=g), torch.randn(m, n, generator=g)
+    gamma, beta, eps = torch.rand(n, generator=g) + 0.5, torch.randn(n, generator=g), 1e-5
+    y = x.double().numpy() @ w.double().numpy().T + b.double().numpy()
+    total, bound = base.double().numpy() + y, 4 * math.sqrt(k) * 2.0 ** -24
+    dev = [v.to(DEV) for v in (x, w, b)]
+    alone = base.to(DEV)
+    ops.linear(*dev, alone, True, ws=_Lender())
+    assert rel(alone, total) < bound
+    for dtype, near in ((torch.bfloat16, 2.0 ** -8), (torch.float32, 2 * bound)):
+        xn, out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV), base.to(DEV)
+        assert ops.linear_then_norm(*dev, out, gamma.to(DEV), eps, xn, _Lender())
+        assert torch.equal(out, alone) and rel(xn, plain_impl.rms_norm(total, gamma.double().numpy(), eps)) < near
+        xn, out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV), base.to(DEV)
+        assert ops.linear_tanh_norm(*dev, out, 0.7, gamma.to(DEV), beta.to(DEV), xn, _Lender())
+        assert torch.equal(out, alone) and rel(xn, np.tanh(0.7 * total) * gamma.double().numpy() + beta.double().numpy()) < near
+    act = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert ops.linear_act(*dev, act, "relu2", ws=_Lender())
+    assert rel(act, np.maximum(y, 0) ** 2) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("T,nh,nkv,dk,dv,rot,split,norm,store", [
     (1, 1, 1, 2, 1, 2, False, True, True), (3, 16, 2, 64, 48, 64, True, True, True),          # a unit; two units a thread, all pairs
     (2, 12, 2, 128, 128, 64, True, True, True), (2, 17, 3, 128, 128, 4, False, True, True),       # 1,024 threads, their units; one head too many for them
