@@ -1584,7 +1584,17 @@ struct Parts {
 };
 static_assert(MID_PARTS == 2 * PARTS_HELD, "every part that a product is cut into is added up");
 
-// out (+)= sum over the parts, in the order of the parts, + bias
+// out (+)= sum over the parts, in the order of the parts, + bias: of few rows (all parts at once; one after another they were a chain of trips to
+// memory: 33 to 64 rows of 2,048 x 11,008, 16 parts, product included, 18.4 -> 15.9 us, of 896 x 4,864, 8 parts, 11.1 -> 9.9), and of many
+template <typename TO, bool MORE>
+__global__ __launch_bounds__(256) void splitk_reduce_few_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
+                                                                const float* __restrict__ bias, TO* __restrict__ out, float accumulate) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= mn) return;
+    Parts<MORE> parts;
+    parts.ask(part, nsplit, mn, i);
+    epilogue_store(out, i, parts.sum(nsplit), bias, (int)(i % N), accumulate);
+}
 template <typename TO>
 __global__ void splitk_reduce_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                      const float* __restrict__ bias, TO* __restrict__ out, float accumulate) {
@@ -1862,12 +1872,13 @@ extern "C" int li_four_tiles_preferred(int M, long N, long K) {
 }
 
 // Parts of K for up to 64 rows and fewer than 128 tiles of 128 columns: blocks for every compute unit, at least 8 steps a part.  (Up to MID_PARTS,
-// where 8 were: 64 x 1,536 x 8,960, 12 tiles, with the norm 17.5 -> 15.2 us.)
+// where 8 were: 64 x 1,536 x 8,960, 12 tiles, with the norm 17.5 -> 15.2 us.  Nine to eleven are a few units more for another part's sums through
+// memory: 3,584 x 18,944, 28 tiles, 33 to 64 rows with a tanh norm 30.9 us in eight, 31.7 in nine; 896 x 4,864, seven tiles, 9.8 and 9.7.)
 static int mid_parts(int N, int K) {
     int nsplit = 256 / ((N + 127) / 128);
     if (nsplit > MID_PARTS) nsplit = MID_PARTS;
     if (nsplit > K / 64 / 8) nsplit = K / 64 / 8;
-    return nsplit;
+    return nsplit > PARTS_HELD && nsplit < 12 ? PARTS_HELD : nsplit;
 }
 
 static bool mid_rows_take(int M, int N, int K) {
@@ -1891,8 +1902,10 @@ static int linear_mid_rows(const bf16_t* x, const bf16_t* w, const float* bias, 
     if (rc != LI_OK) return rc;
 #undef LI_MID
     const unsigned blocks = (unsigned)((mn + 255) / 256);
-    if (out_dtype == LI_F32) splitk_reduce_kernel<float><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (float*)out, accumulate);
-    else splitk_reduce_kernel<bf16_t><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (bf16_t*)out, accumulate);
+#define LI_RS(TO, MORE) splitk_reduce_few_kernel<TO, MORE><<<blocks, 256, 0, stream>>>((const float*)work, nsplit, mn, N, bias, (TO*)out, accumulate)
+    if (out_dtype == LI_F32) { if (nsplit > PARTS_HELD) LI_RS(float, true); else LI_RS(float, false); }
+    else { if (nsplit > PARTS_HELD) LI_RS(bf16_t, true); else LI_RS(bf16_t, false); }
+#undef LI_RS
     return li_launch_status();
 }
 

@@ -768,7 +768,7 @@ def test_paged_attention(ops, dtype, segs, nh, nkv, dh, page, window):
     assert rel(out, ref) < tol(dtype, 3e-6, 1.5e-2)
 
 
-@pytest.mark.parametrize("m,n,k,parts", [(33, 200, 4096, 8), (64, 136, 4608, 9), (40, 300, 7744, 15), (64, 264, 9024, 16), (65, 264, 9024, 8)])
+@pytest.mark.parametrize("m,n,k,parts", [(33, 200, 4096, 8), (64, 136, 5888, 8), (64, 136, 6144, 12), (40, 300, 7744, 15), (64, 264, 9024, 16), (65, 264, 9024, 8)])
 def test_products_of_many_parts_and_what_follows_them(ops, m, n, k, parts):
     """K in up to sixteen parts (eight above 64 rows): every kernel that adds them up adds all of them."""
     assert ops._work_bytes(m, n, k, ops._DT[torch.bfloat16]) == 4 * m * n * parts
@@ -780,9 +780,10 @@ def test_products_of_many_parts_and_what_follows_them(ops, m, n, k, parts):
     y = x.double().numpy() @ w.double().numpy().T + b.double().numpy()
     total, bound = base.double().numpy() + y, 4 * math.sqrt(k) * 2.0 ** -24
     dev = [v.to(DEV) for v in (x, w, b)]
-    alone = base.to(DEV)
+    alone, short = base.to(DEV), torch.full((m, n), float("nan"), dtype=torch.bfloat16, device=DEV)
     ops.linear(*dev, alone, True, ws=_Lender())
-    assert rel(alone, total) < bound
+    ops.linear(*dev, short, ws=_Lender())
+    assert rel(alone, total) < bound and rel(short, y) < 2.0 ** -8
     for dtype, near in ((torch.bfloat16, 2.0 ** -8), (torch.float32, 2 * bound)):
         xn, out = torch.full((m, n), float("nan"), dtype=dtype, device=DEV), base.to(DEV)
         assert ops.linear_then_norm(*dev, out, gamma.to(DEV), eps, xn, _Lender())
