@@ -2128,7 +2128,7 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
     const size_t mn = (size_t)M * N;
     const int nsplit = (int)(need / (long)(mn * sizeof(float)));
     if (nsplit > MID_PARTS) return -1;
-    if (li_four_tiles_preferred(M, N, K)) {         // K whole: the sum, then its norm
+    if (factor != 0.f && li_four_tiles_preferred(M, N, K)) {      // K whole: the sum, then its norm (0 is that kernel's word for writing, not adding)
         const int rc = li_linear_skinny(x, w, bias, out, M, N, K, LI_F32, factor, 0, stream);
         if (rc != LI_OK) return rc;
         if (xn_dtype == LI_BF16)

@@ -411,6 +411,17 @@ def test_products_of_33_to_64_rows_against_small_matrices(ops, m, n, k):
             assert torch.equal(kc[sl // page, :, sl % page].cpu(), qv[i, nh:nh + nkv]) and torch.equal(vc[sl // page, :, sl % page].cpu(), qv[i, nh + nkv:])
 
 
+@pytest.mark.parametrize("m,n,k", [(48, 1536, 1536), (64, 4096, 1024), (64, 3584, 3584)])      # K whole, twice, and in parts
+def test_norm_behind_a_product_that_counts_for_nothing(ops, m, n, k):
+    g = torch.Generator().manual_seed(83)
+    x, w = torch.randn(m, k, generator=g).to(torch.bfloat16), torch.randn(n, k, generator=g).to(torch.bfloat16)
+    base, gamma = torch.randn(m, n, generator=g), torch.rand(n, generator=g) + 0.5
+    out, xn = base.to(DEV), torch.full((m, n), float("nan"), dtype=torch.float32, device=DEV)
+    assert ops.linear_then_norm(x.to(DEV), w.to(DEV), None, out, gamma.to(DEV), 1e-5, xn, _Lender(), factor=0.0)
+    assert torch.equal(out.cpu(), base)
+    assert rel(xn, plain_impl.rms_norm(base.double().numpy(), gamma.double().numpy(), 1e-5)) < 4 * math.sqrt(n) * 2.0 ** -24
+
+
 @pytest.mark.parametrize("m,n,k,bias,taken", [
     (64, 3584, 18944, False, True),      # a decoding batch of 64 at the 7B sizes
     (40, 200, 1024, True, True),
