@@ -1862,9 +1862,9 @@ extern "C" int li_few_rows_preferred(int M, long N, long K) {
 
 // 33 to 64 rows against a small matrix of short rows: three or four tiles of rows a block of the few-row kernel, K whole, rather than the
 // 64-row tiles with K in parts, whose sums go to memory and to a kernel that adds them up.  Every block reads all of x, so the line lies at the
-// length of a row.  Us, in parts / whole, with the norm behind it, and with the rotation and the page write: 48 rows of 1,536 x 1,536 10.1 / 9.2
-// and 9.5 / 6.2, 64 of 2,048 x 1,536 11.6 / 11.0 and 10.4 / 8.1, 64 of 896 x 896 11.7 / 8.1 and 11.0 / 6.0, 48 of 2,048 x 2,048 11.4 / 10.9 and
-// 10.8 / 8.1; 64 of 2,048 x 2,048 with the norm 11.8 / 12.4, of 3,584 x 3,584 15.8 / 18.
+// length of a row.  Us, in parts / whole, with the norm behind it, and with the rotation and the page write: 48 rows of 1,536 x 1,536 10.2 / 8.8
+// and 9.5 / 6.2, 64 of 2,048 x 1,536 11.1 / 9.8 and 10.4 / 8.1, 48 of 2,048 x 2,048 10.8 / 9.3 and 10.8 / 8.1; 64 of 2,048 x 2,048 with the norm
+// 11.8 / 12.4, of 3,584 x 3,584 15.8 / 18.  64 of 896 x 896, too short for parts: in one and the norm's own kernel 11.6 / 7.8, and 11.0 / 6.0.
 #define FOUR_TILES_K 2048         // up to 48 rows,
 #define FOUR_TILES_LAST_K 1536    // above
 extern "C" int li_four_tiles_preferred(int M, long N, long K) {
@@ -2097,7 +2097,9 @@ static int f32_split_parts(int M, int N, int K) {
     return pick;
 }
 
-// Bytes of workspace with which li_linear cuts this product along K (0: it would not).
+// Bytes of workspace with which this product is cut along K (0: it is not).  The products of li_four_tiles_preferred have a number too: li_linear
+// and what it shares their epilogues with leave K whole there and need none of it, but a tanh norm into float32 and a rotation of heads that are no
+// multiple of 16 columns cut them.
 extern "C" long li_linear_work_bytes(int M, int N, int K, int in_dtype) {
     if (in_dtype == LI_F32) {
         const int parts = N > 0 && K > 0 ? f32_split_parts(M, N, K) : 1;
@@ -2116,18 +2118,15 @@ extern "C" long li_linear_work_bytes(int M, int N, int K, int in_dtype) {
 
 // out += factor * (x w^T + bias) (float32 out: the residual sum) and xn = the RMS norm of the new out with weights
 // gamma, where li_linear would cut K into parts anyway: the kernel that adds the parts up then has
-// whole rows in its hands.  xn is bfloat16 (xn_dtype LI_BF16) or float32.  Returns -1, having done
-// nothing, where the product is not cut (the caller then multiplies and norms in two calls).
+// whole rows in its hands.  Also for the products of li_four_tiles_preferred: K whole, then the norm's kernel, which reads the sum again; no
+// `work`.  xn is bfloat16 (xn_dtype LI_BF16) or float32.  Returns -1, having done
+// nothing, where neither is the case (the caller then multiplies and norms in two calls).
 extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bias, float* out, int M, int N, int K,
                                    void* work, long work_bytes, float factor, const float* gamma, float eps, void* xn,
                                    int xn_dtype, hipStream_t stream) {
     if (N <= 0 || K <= 0 || (K % 64) || li_few_rows_preferred(M, N, K) || !gamma || !xn || eps < 0.f) return -1;
     if (N > REDUCE_NORM_NT * REDUCE_NORM_PER || (xn_dtype != LI_BF16 && xn_dtype != LI_F32)) return -1;
-    const long need = li_linear_work_bytes(M, N, K, LI_BF16);
-    if (need <= 0 || !work || work_bytes < need) return -1;
     const size_t mn = (size_t)M * N;
-    const int nsplit = (int)(need / (long)(mn * sizeof(float)));
-    if (nsplit > MID_PARTS) return -1;
     if (factor != 0.f && li_four_tiles_preferred(M, N, K)) {      // K whole: the sum, then its norm (0 is that kernel's word for writing, not adding)
         const int rc = li_linear_skinny(x, w, bias, out, M, N, K, LI_F32, factor, 0, stream);
         if (rc != LI_OK) return rc;
@@ -2139,6 +2138,10 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
                 nullptr, 0, mn, N, nullptr, out, 0.f, gamma, eps, (float*)xn);
         return li_launch_status();
     }
+    const long need = li_linear_work_bytes(M, N, K, LI_BF16);
+    if (need <= 0 || !work || work_bytes < need) return -1;
+    const int nsplit = (int)(need / (long)(mn * sizeof(float)));
+    if (nsplit > MID_PARTS) return -1;
     const int rc = M <= 64
         ? launch_dma<64, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit)
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit);

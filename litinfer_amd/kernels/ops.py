@@ -1092,7 +1092,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: 
          "linear: bias must be float32 [N]")
     if m:
         work, work_bytes = 0, 0
-        if ws is not None and (not few_rows_preferred(m, n, k) if x.dtype is torch.bfloat16 else m > SKINNY_MAX_ROWS):
+        if ws is not None and (not (few_rows_preferred(m, n, k) or four_tiles_preferred(m, n, k)) if x.dtype is torch.bfloat16 else m > SKINNY_MAX_ROWS):
             # too few tiles to fill the chip: the library cuts k into parts if it is lent room for their sums
             need = _work_bytes(m, n, k, _DT[x.dtype])
             if need:
@@ -1176,8 +1176,8 @@ def few_rows_preferred(m: int, n: int, k: int) -> bool:
 
 
 def four_tiles_preferred(m: int, n: int, k: int) -> bool:
-    """Whether 33 to 64 rows against a matrix [n, k] take the few-row kernels too (the library's rule)."""
-    return bool(_lib_fn("gemm", "li_four_tiles_preferred", [c_int, c_long, c_long], c_int)(int(m), int(n), int(k)))
+    """Whether 33 to 64 rows against a matrix [n, k] take the few-row kernels too (the library's rule): k whole, no memory lent."""
+    return m <= SKINNY_MAX_ROWS and bool(_lib_fn("gemm", "li_four_tiles_preferred", [c_int, c_long, c_long], c_int)(int(m), int(n), int(k)))
 
 
 class RowScale:
@@ -1234,16 +1234,17 @@ def linear_residual_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.
 def linear_then_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], out: torch.Tensor,
                      gamma: torch.Tensor, eps: float, xn: torch.Tensor, ws, factor: float = 1.0) -> bool:
     """out += factor * (x w^T + bias) (float32) and xn = gamma * out / sqrt(mean(out^2) + eps), in the kernel
-    that adds up the parts of a product cut along K.  Returns False, having done nothing, where
-    `linear` would not cut this product (then multiply and norm in two calls)."""
+    that adds up the parts of a product cut along K, or behind a product of 33 to 64 rows against a small matrix
+    (`four_tiles_preferred`).  Returns False, having done nothing, where neither is the case (then multiply and norm in two calls)."""
     _gpu(x, w, bias, out, gamma, xn)
     if ws is None or x.dtype is not torch.bfloat16 or w.dtype is not torch.bfloat16:
         return False
     _chk(x.dim() == 2 and w.dim() == 2, "linear_then_norm: needs matrices")
     m, k = x.shape
     n = w.shape[0]
-    need = _work_bytes(m, n, k, _DT[x.dtype])
-    if not need:
+    whole = factor != 0.0 and four_tiles_preferred(m, n, k)
+    need = 0 if whole else _work_bytes(m, n, k, _DT[x.dtype])
+    if not need and not whole:
         return False
     _chk(w.shape == (n, k) and x.is_contiguous() and w.is_contiguous(), "linear_then_norm: contiguous [M, K] and [N, K]")
     _chk(out.dtype is torch.float32 and out.shape == (m, n) and out.is_contiguous(), "linear_then_norm: out must be float32 [M, N]")
@@ -1252,11 +1253,11 @@ def linear_then_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tens
          "linear_then_norm: bias must be float32 [N]")
     _chk(gamma.dtype is torch.float32 and gamma.shape == (n,) and gamma.is_contiguous() and eps >= 0,
          "linear_then_norm: gamma must be float32 [N], eps not negative")
-    if m <= SKINNY_MAX_ROWS:                # one size for all row counts of a decode batch: the buffer does not move
+    if need and m <= SKINNY_MAX_ROWS:       # one size for all row counts of a decode batch: the buffer does not move
         need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)
-    buf = ws.buffer("gemm.parts", (need // 4,), torch.float32)
+    buf = ws.buffer("gemm.parts", (need // 4,), torch.float32) if need else None
     return _try("gemm", "li_linear_then_norm", x.data_ptr(), w.data_ptr(), 0 if bias is None else bias.data_ptr(),
-                out.data_ptr(), m, n, k, buf.data_ptr(), buf.numel() * 4, float(factor), gamma.data_ptr(),
+                out.data_ptr(), m, n, k, 0 if buf is None else buf.data_ptr(), 0 if buf is None else buf.numel() * 4, float(factor), gamma.data_ptr(),
                 float(eps), xn.data_ptr(), _DT[xn.dtype])
 
 
@@ -1274,7 +1275,7 @@ def linear_tanh_norm(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tens
     if not m:
         return False
     work, work_bytes = 0, 0
-    if not (m <= RESIDUAL_NORM_MAX_ROWS and few_rows_preferred(m, n, k) and xn.dtype is torch.bfloat16):
+    if not (xn.dtype is torch.bfloat16 and ((m <= RESIDUAL_NORM_MAX_ROWS and few_rows_preferred(m, n, k)) or (k % 64 == 0 and four_tiles_preferred(m, n, k)))):
         need = _work_bytes(m, n, k, _DT[x.dtype]) if ws is not None else 0
         if not need:
             return False
@@ -1373,7 +1374,9 @@ def linear_act(x: torch.Tensor, w: torch.Tensor, bias: Optional[torch.Tensor], o
     if not m:
         return True
     work, work_bytes = 0, 0
-    need = _lib_fn("gemm", "li_linear_act_work_bytes", [c_int] * 4, c_long)(m, n, k, LINEAR_ACTS[act]) if ws is not None else 0
+    need = 0
+    if ws is not None and not four_tiles_preferred(m, n, k):
+        need = _lib_fn("gemm", "li_linear_act_work_bytes", [c_int] * 4, c_long)(m, n, k, LINEAR_ACTS[act])
     if need:
         if m <= SKINNY_MAX_ROWS:                    # one size for all row counts of a decode batch: the buffer does not move
             need = max(need, SPLITK_MAX_PARTS * SKINNY_MAX_ROWS * n * 4)

@@ -234,7 +234,10 @@ def test_linear_skinny_with_fused_swiglu(ops, m, n, k, swiglu, out_dtype, bias, 
 
 class _Lender:
     """Stands in for the engine's workspace."""
+    made = 0
+
     def buffer(self, name, shape, dtype, zero=False):
+        self.made += 1
         return (torch.zeros if zero else torch.empty)(*shape, dtype=dtype, device=DEV)
 
 
@@ -382,15 +385,25 @@ def test_products_of_33_to_64_rows_against_small_matrices(ops, m, n, k):
     ops.linear(x.to(DEV), w.to(DEV), b.to(DEV), alone, True, ws=_Lender())
     for i in range(m):
         assert rel(alone[i], y[i]) < bound, i
-    out = base.to(DEV)
-    if ops.linear_then_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, gamma.to(DEV), eps, xn, _Lender()):
+    # with a norm behind it: wherever K has whole steps (the last product above 48 rows in parts), and where not, nothing is touched;
+    # K whole takes no lent memory
+    out, lent = base.to(DEV), _Lender()
+    if k % 64:
+        assert not ops.linear_then_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, gamma.to(DEV), eps, xn, lent)
+        assert not ops.linear_tanh_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, 0.7, gamma.to(DEV), beta.to(DEV), xn, lent)
+        assert torch.equal(out.cpu(), base) and torch.isnan(xn.float()).all()
+    else:
+        assert ops.linear_then_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, gamma.to(DEV), eps, xn, lent)
         assert torch.equal(out, alone)
         ref = plain_impl.rms_norm(y, gamma.double().numpy(), eps)
         for i in range(m):
             assert rel(xn[i], ref[i]) < 8e-3, i
-    out = base.to(DEV)
-    if ops.linear_tanh_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, 0.7, gamma.to(DEV), beta.to(DEV), xn, _Lender()):
+        out, xn = base.to(DEV), torch.full_like(xn, float("nan"))
+        assert ops.linear_tanh_norm(x.to(DEV), w.to(DEV), b.to(DEV), out, 0.7, gamma.to(DEV), beta.to(DEV), xn, lent)
         assert rel(out, y) < bound and rel(xn, np.tanh(0.7 * y) * gamma.double().numpy() + beta.double().numpy()) < 8e-3
+        short = torch.empty_like(xn)
+        assert ops.linear_act(x.to(DEV), w.to(DEV), b.to(DEV), short, "relu2", ws=lent)
+        assert bool(lent.made) == (not ops.four_tiles_preferred(m, n, k))
     # the packed projection with rotary encoding and page write, in one launch
     if n % 64 == 0 and n >= 256:
         nkv, dh, page = 1, 64, 16
