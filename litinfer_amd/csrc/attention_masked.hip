@@ -1184,10 +1184,15 @@ extern "C" int li_masked_attention_single_takes(int dk, int dv) {
     return (npk <= 2 && npv <= 2) || (npk == 3 && npv == 2) || (npk == 4 && npv == 4) || (npk == 5 && npv == 4) || (npk == 4 && npv == 3);
 }
 
+// Query heads of a kv head that a block takes: four where they fill most blocks and the registers hold them, else two
+static bool heads_by_four(int rep) { return rep >= 4 && (rep % 4 == 0 || rep % 4 == 3 || rep > 8); }
+static int single_heads(int rep, int npk, int npv) { return npk + npv <= 6 && heads_by_four(rep) ? 4 : rep >= 2 ? 2 : 1; }
+extern "C" int li_masked_attention_single_by_four(int rep) { return heads_by_four(rep); }
+
 // blocks that a call launches per split (the host sizes the number of splits by it)
 extern "C" int li_masked_attention_single_blocks(int n_tokens, int nh, int nkv, int dk, int dv) {
     const int rep = nh / nkv, npk = (dk + 63) / 64, npv = (dv + 63) / 64;
-    const int rh = (npk + npv > 6) ? (rep >= 2 ? 2 : 1) : (rep >= 4 && (rep % 4 == 0 || rep % 4 == 3 || rep > 8)) ? 4 : rep >= 2 ? 2 : 1;
+    const int rh = single_heads(rep, npk, npv);
     return n_tokens * nkv * ((rep + rh - 1) / rh);
 }
 
@@ -1204,7 +1209,7 @@ static int single_launch(const float* q, int q_token_stride, int q_head_stride, 
         q_head_stride % 4 || ((uintptr_t)q | (uintptr_t)kc | (uintptr_t)vc) % 16 || !li_masked_attention_single_takes(dk, dv))
         return LI_ERR_SIZE;
     const int rep = nh / nkv, npk = (dk + 63) / 64, npv = (dv + 63) / 64;
-    const int rh = (npk + npv > 6) ? (rep >= 2 ? 2 : 1) : (rep >= 4 && (rep % 4 == 0 || rep % 4 == 3 || rep > 8)) ? 4 : rep >= 2 ? 2 : 1;
+    const int rh = single_heads(rep, npk, npv);
     const int maps = second.n ? 2 : 1;
     if (nsplit < 1 || nsplit > 64 || ((nsplit > 1 || maps > 1) && (!parts || parts_floats < (long)maps * n_tokens * nh * nsplit * (dv + 2)))) return LI_ERR_SIZE;
     if (n_tokens > 0x3fffffff) return LI_ERR_SIZE;

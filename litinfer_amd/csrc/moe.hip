@@ -1430,6 +1430,9 @@ extern "C" int li_moe_linear(const void* a, int a_dtype, long a_stride, const in
 // unit (32 tokens, 23.5 and 8.2 apart, 37.1 together).
 #define MOE_BESIDE_NT 512
 #define MOE_BESIDE_ROWS 32
+// Tokens up to which li_moe_route_beside takes a call, and rows of the routed product up to which li_moe_linear_beside does
+extern "C" int li_moe_route_beside_rows() { return MOE_BESIDE_ROWS; }
+extern "C" int li_moe_linear_beside_rows() { return MOE_VECTOR_ROWS; }
 enum { BESIDE_ROWS = 0, BESIDE_ONE_TILE = 1, BESIDE_TWO_TILES = 2 };
 template <int FORM> constexpr int beside_lds() {
     return FORM == BESIDE_ROWS ? fr_lds_bytes(2) : FORM == BESIDE_ONE_TILE ? SkinnyLds<1, 1, 8, SK_CHUNK>::BYTES : SkinnyLds<2, 1, 8, SK_CHUNK / 2>::BYTES;

@@ -1001,8 +1001,10 @@ def masked_attention_difference(q: torch.Tensor, q_token_stride: int, q_head_str
 
 def _heads_kernel_pays(n: int, rep: int, dk: int, dv: int) -> bool:
     if dk + dv <= 384:
-        by_two = not (rep % 4 in (0, 3) or rep > 8)                  # (the heads a block of the vector kernel takes: 4, or 2)
-        return rep >= MASKED_HEADS_MIN and n * rep >= (MASKED_HEADS_MIN_PAIRS_BY_TWO if by_two else MASKED_HEADS_MIN_PAIRS)
+        if rep < MASKED_HEADS_MIN or n * rep < MASKED_HEADS_MIN_PAIRS:
+            return False
+        by_four = _lib_fn("attention_masked", "li_masked_attention_single_by_four", [c_int], c_int)(rep)      # (the heads a block of the vector kernel takes)
+        return bool(by_four) or n * rep >= MASKED_HEADS_MIN_PAIRS_BY_TWO
     return rep >= MASKED_HEADS_MIN_LONG and n * rep >= MASKED_HEADS_MIN_WORK
 
 
@@ -2093,8 +2095,16 @@ class MoePlan:
 
 
 MOE_ROUTE_PLAN_TOKENS, MOE_ROUTE_PLAN_EXPERTS = 128, 64
-MOE_BESIDE_ROWS = 32         # tokens up to which the shared expert's first product goes in the router's launch,
-MOE_BESIDE_PAIRS = 4         # ... and rows of the routed product up to which its second goes in that one's
+
+
+def moe_route_beside_rows() -> int:
+    """Tokens up to which the shared expert's first product goes in the router's launch (the library's limit)."""
+    return _lib_fn("moe", "li_moe_route_beside_rows", [], c_int)()
+
+
+def moe_linear_beside_rows() -> int:
+    """Rows of the routed product up to which the shared expert's second product goes in its launch (the library's limit)."""
+    return _lib_fn("moe", "li_moe_linear_beside_rows", [], c_int)()
 
 
 def moe_route_takes_plan(t: int, experts: int, hidden: int) -> bool:
@@ -2157,7 +2167,7 @@ def moe_route(x: torch.Tensor, router: torch.Tensor, bias: Optional[torch.Tensor
         _chk(moe_route_takes_plan(t, plan.experts, k) and plan.experts <= e and plan.count.dtype is torch.int32 and plan.count.numel() > 0, "moe_route: plan")
         made = (plan.plan.data_ptr(), max_tiles, plan.row_token.data_ptr(), plan.pair_row.data_ptr(), int(plan.tile_rows),
                 0 if plan.row_wt is None else plan.row_wt.data_ptr(), plan.experts, plan.count.data_ptr())
-    if beside is not None and 0 < t <= MOE_BESIDE_ROWS:
+    if beside is not None and 0 < t <= moe_route_beside_rows():
         w, out, act = beside
         _gpu(w, out)
         n = w.shape[0]
@@ -2214,7 +2224,7 @@ def moe_linear(a: torch.Tensor, row_token: Optional[torch.Tensor], w: torch.Tens
          "moe_linear: a [*, K], w [E, n_out, K], out [rows, n_out]")
     _chk(plan.dtype is torch.int32 and plan.numel() >= 4 + 4 * max_tiles and (row_token is not None or a.shape[0] >= rows)
          and (row_token is None or (row_token.dtype is torch.int32 and row_token.numel() >= rows)), "moe_linear: plan, rows")
-    if beside is not None and 0 < rows <= MOE_BESIDE_PAIRS and 0 < beside[0].shape[0] and tile_rows == MOE_TILE_ROWS:
+    if beside is not None and 0 < rows <= moe_linear_beside_rows() and 0 < beside[0].shape[0] and tile_rows == MOE_TILE_ROWS:
         x, w2, y = beside
         _gpu(x, w2, y)
         t, k2 = x.shape
