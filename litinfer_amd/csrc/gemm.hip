@@ -1722,8 +1722,57 @@ static int launch_big(const bf16_t* x, const bf16_t* w, const float* bias, TO* o
     }
     gemm_bf16_big_kernel<BM, BN, BK, TO><<<grid, 256, lds_bytes, stream>>>(x, w, bias, out, M, N, K, accumulate);
     return li_launch_status();
-}// ------------------------------------------------- bfloat16, few rows (decode): few_rows.h
+}
 
+// ------------------------------------------------- bfloat16, few rows (decode): few_rows.h
+// Up to 16 rows against a matrix of few columns (or rotation pairs: `unit` is 16 columns or 8 pairs a
+// tile): a compute unit takes in what its blocks ask for at a rate of its own, far below its share of
+// the memory's rate times the number of units, so the time of such a product is that of the unit with the
+// most blocks.  Every unit therefore gets one block and every block the same number of columns (at
+// most two tiles' worth, at least a quarter of a tile's), not whole tiles.  (At least a quarter, where a half was: 896 x 4,864 at one row
+// 6.05 -> 5.53 us with twice the blocks.)
+static int balanced_per_block(int total, int unit, int cu) {
+    int per = (total + cu - 1) / cu;
+    per = per < unit / 4 ? unit / 4 : per;
+    return per > 2 * unit ? 0 : per;
+}
+
+// Whether a product of few rows goes to gemm_bf16_rows_kernel (columns: the matrix's rows).  Not from five rows on, where all blocks' reading of
+// x bounds both and gemm_bf16_skinny_kernel, whose loads of x are whole rows of a chunk, is as fast or faster (us, 5 rows: 896 x 896 3.5 / 3.6, 8 rows:
+// 2,048 x 11,008 13.7 / 14.9); nor against a wide matrix of long rows, where its chunks, which the eight waves take in turns, read w in longer
+// pieces (one row: 3,584 x 3,584 7.1 / 8.0, 5,120 x 5,120 12.1 / 13.9).  The gated product stays with it too: its blocks come two and more to a
+// compute unit, where this kernel's registers leave room for fewer (17,920 x 1,536 13.1 / 14.5).
+static bool rows_kernel_takes(int M, long columns, int K) {
+    return M <= ROWS_KERNEL_M && K % 64 == 0 && (K <= 2048 || columns <= 2048);
+}
+// Columns a block of it takes on cu compute units, 1 to 16: a block has one tile of 16.  One block a unit where that is enough for them, else
+// whole rounds of blocks.  0: the product is gemm_bf16_skinny_kernel's, which has blocks of two tiles.  into_sum: out is added to; such a sum comes
+// out of one kernel whether or not its shares of the rows' squares are asked for, whose number goes with the columns alone (li_residual_norm_parts)
+static int rows_kernel_cols(int M, int N, int K, bool into_sum, int cu) {
+    if (!rows_kernel_takes(M, N, K)) return 0;
+    if (N <= 16l * cu) return balanced_per_block(N, 16, cu);
+    return into_sum ? 0 : balanced_round_cols(N, 16, cu);
+}
+
+template <typename TO, bool ROPE, int EPI>
+static int launch_rows(const SkinnyArgs& a, int total, hipStream_t stream) {
+    if (a.cols < 1 || a.cols > (ROPE ? 8 : 16)) return LI_ERR_SIZE;      // (a block writes one tile)
+    const int blocks = (total + a.cols - 1) / a.cols;
+    const int log_rows = a.M <= 1 ? 0 : a.M <= 2 ? 1 : 2;
+    const int n = (a.K / 64 + FR_WAVES - 1) / FR_WAVES;              // a wave's units
+#define LI_FR(D, LOOP, X2, X4)                                                                                                          \
+    {                                                                                                                                   \
+        if (log_rows <= 1) gemm_bf16_rows_kernel<TO, ROPE, EPI, D, LOOP, X2><<<blocks, FR_WAVES * 64, 0, stream>>>(a, log_rows);        \
+        else gemm_bf16_rows_kernel<TO, ROPE, EPI, D, LOOP, X4><<<blocks, FR_WAVES * 64, 0, stream>>>(a, log_rows);                      \
+    }
+    if (n <= 4) LI_FR(4, false, 1, 2)
+    else if constexpr (!ROPE) {
+        if (n <= 10) LI_FR(10, false, 3, 5)
+        else LI_FR(4, true, 1, 2)
+    } else return LI_ERR_SIZE;
+#undef LI_FR
+    return li_launch_status();
+}
 
 template <bool SWIGLU, typename TO, int EPI = 0>
 static int launch_skinny(SkinnyArgs a, hipStream_t stream) {
@@ -1831,11 +1880,12 @@ extern "C" int li_linear_residual_norm(const void* x, const void* w, const float
 // 64 rows with the loads straight into LDS, and, where the matrix has too few such tiles to fill
 // the chip, K cut into parts whose sums go to `work` and are added up in a fixed order, by kernels
 // that also do what follows the product (the norm of the new residual sum, the rotary encoding
-// and the page write), which the few-row kernel does in its epilogue for up to 16 rows only.
+// and the page write), which the few-row kernel does in its epilogue.
 // Measured on the 7B layer sizes, a decode step of 17 / 24 / 32 requests: 4.57 / 4.95 / 5.33 ms
 // against 4.90 / 5.33 / 5.84 ms with the few-row kernel up to 32 rows.  Returns -1 when it does
 // not take the call.
-// The few-row kernel takes up to 16 rows with its fused epilogues.  Up to 12 rows it is the faster one for
+// The few-row kernel with its epilogues (a norm between two products up to 32 rows, the rotation and the page write up to 64) against those tiles.
+// Up to 12 rows, one tile of rows, it is the faster one for
 // every product but the largest gate/up matrices (li_linear_swiglu); at 13 to 16 rows the tiles with K in
 // parts are faster where the matrix is large (at 13 rows the 7B's way back from the feed-forward, 136 MB:
 // 29.8 us with its adding-up kernel against 33.5 us; its q/k/v, 33 MB: 11.8 against 9.2 us; the whole step
