@@ -1511,18 +1511,25 @@ def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int):
     kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan.
     A run of 32 keys is a step, whose instructions (bfloat16, 0.9 us) or matrix products (float32, 1.8 us: six heads in tiles of 16) are
     what it takes, and the second kernel with its trips to memory is 3 us.  Us a call, before / now:
-    bfloat16, 12 heads on 2 of 128, a table of 208 keys, 1 / 64 / 128 requests 8.3 / 10.0 / 13.2 -> 6.4 / 7.3 / 8.9; contexts of 30 to 300, 64 / 128
-    requests 11.0 / 15.2 -> 8.4 / 9.5, 3 requests 7.7 / 7.5; of 50 to 500, 3 requests 8.3 / 9.6 (so not there), 64 12.7 / 10.7; of 100 to 1,000,
-    16 / 64 / 128 requests 10.1 / 14.0, 16.7 / 16.0, 25.4 / 20.0.  Few requests of heads of 128, tables of 592 / 704 / 832 keys:
-    the four runs of a block 9.3 / 9.9 / 11.1 (1 request), 9.8 / 10.3 / 11.3 (16), runs of 64 keys and more 8.1 / 8.1 / 8.3, 9.1 / 9.4 / 9.7 (496 keys, 8 kv
-    heads: 7.7 / 7.9, so not there).
-    float32, 1 request of 150 / 300 / 600 / 1,000 keys 13.4 / 14.7 / 21.5 / 17.0 -> 8.8 / 9.0 / 11.4 / 12.5, 16 requests 14.2 / 15.2 / 26.0 / 20.2 -> 9.7 /
-    10.8 / 14.2 / 17.1; 3 of 50 to 500 keys 12.1 -> 10.0; up to 96 keys one run is the faster (7.8 / 8.5); 64 requests of 300 18.3 / 18.9."""
+    bfloat16, beside portions, whose tables are as wide as they must be: 12 heads on 2 of 128, a table of 208 keys, 1 / 64 / 128 requests
+    8.3 / 10.0 / 13.2 -> 6.4 / 7.3 / 8.9; contexts of 30 to 300, 64 / 128 requests 11.0 / 15.2 -> 8.4 / 9.5, 3 requests 7.7 / 7.5; of 50 to 500, 3
+    requests 8.3 / 9.6 (so not there), 64 12.7 / 10.7; of 100 to 1,000, 16 / 64 / 128 requests 10.1 / 14.0, 16.7 / 16.0, 25.4 / 20.0.  Few requests of
+    heads of 128, tables of 592 / 704 / 832 keys: the four runs of a block 9.3 / 9.9 / 11.1 (1 request), 9.8 / 10.3 / 11.3 (16), runs of 64 keys and more
+    8.1 / 8.1 / 8.3, 9.1 / 9.4 / 9.7 (496 keys, 8 kv heads: 7.7 / 7.9, so not there).  Recorded steps, whose tables are 256, 512 or 1,024 keys wide, contexts of
+    three quarters of that / spread from a tenth of it on: 14 heads on 2 of 64, 1 request 8.1 -> 5.2 at 256, 64 requests 9.7 / 10.0 -> 6.0 / 6.2, 6.8 /
+    10.9 -> 7.0 / 7.6, 11.7 / 13.1 -> 9.7 / 10.4; 12 on 2 of 128, 1 request 8.3 -> 6.6 at 256, 64 requests 10.0 / 10.9 -> 7.7 / 8.1, 9.3 / 12.6 -> 9.4 / 10.1,
+    15.7 / 16.1 -> 15.7 / 14.6.
+    float32, tables and contexts likewise: 12 heads on 2 of 128, 1 request 13.5, 15.4, 13.9 -> 8.7, 11.1, 11.9, 16 requests 14.3 / 12.6, 16.5 / 12.9, 15.5 / 14.6 -> 9.5 /
+    10.3, 12.4 / 11.4, 14.1 / 13.8; 14 on 2 of 64, 1 request 10.7, 8.6 (its whole table 10.4), 11.0 -> 7.8, 9.1 (9.2), 9.6, 16 requests 10.6 / 10.2, 9.2 / 10.8,
+    11.7 / 11.8 -> 7.7 / 9.0, 9.8 / 9.9, 11.1 / 12.2.  Not beyond 1,024 keys (2,048, 8 requests: 15.9 / 15.1 against 16.3 / 15.4, heads of 64 12.2 / 12.6 against
+    12.6 / 14.3; 1 request 14.6 / 15.0).  32 requests: 128 columns at 832 keys 25.2 / 16.1 -> 17.4 / 15.5, at 1,024 20.4 / 18.3 against 19.2 / 20.6; 64 columns at 304 keys
+    12.0 / 11.8 -> 9.9 / 10.3, at 400 9.2 / 11.8 against 10.4 / 10.6, at 512 9.5 / 11.9 against 11.3 / 11.4.  Up to 96 keys one run is the faster (7.8 / 8.5)."""
     if dtype is torch.bfloat16:
         if 128 < keys <= min(max(448, 10 * pairs), 1280):
             return DECODE_QUAD
         return (64,) if dh == 128 and quads == DECODE_QUAD and 512 < keys <= 1024 and pairs <= 32 else None
-    return (32, 64) if keys > 96 and (pairs <= 16 or (pairs <= 64 and keys <= 1280)) else None
+    most = 1024 if pairs <= 32 else 0 if pairs > 64 else 1023 if dh == 128 else 320
+    return (32, 64) if 96 < keys <= most else None
 
 
 def decode_splits(pairs: int, keys: int, simds: int = _DEC_WAVES, quad: int = DECODE_QUAD, least: int = 128) -> int:

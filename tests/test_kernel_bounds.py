@@ -175,3 +175,10 @@ def test_products_are_cut_into_no_more_parts_than_are_added_up():
                 assert need % (4 * m * n) == 0
                 most[m <= 64] = max(most[m <= 64], need // (4 * m * n))
     assert most[True] == ops.SPLITK_MAX_PARTS == 16 and most[False] == 8
+
+
+@pytest.mark.parametrize("pairs,dh,ends", [(2, 64, 1024), (32, 64, 1024), (32, 128, 1024), (33, 64, 320), (64, 128, 1008), (64, 64, 320), (65, 128, 0)])
+def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh, ends):
+    """Beyond these widths runs of 32 keys and the kernel that joins them took longer than the ordinary cut."""
+    for keys in range(16, 8192, 16):
+        assert (ops._short_runs(pairs, keys, dh, ops.torch.float32, 4) is not None) == (96 < keys <= ends), keys
