@@ -277,7 +277,10 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_kernel(
 // slice holds NR state values of each of its four columns.  A value of B_t or C_t read from LDS then serves four
 // state elements instead of one, and the state comes from and goes to memory in 16-byte pieces.  A wave is 256 / NS
 // columns of one head.  Modes, chunks and blocks as above.
-template <int NR, int NS, int MODE, bool SILU>
+// ONE: every request brings one token, whose decay comes with it (a decoding step).  Its values come in one trip with the state, each asked for before any
+// is used and none under a lane's condition (what is not the state's is blanked behind), and so do the arguments: 48 heads of 64 x 128, one
+// request 8.7 -> 8.3 us.  An instance of its own: the others would wait for the state before they stage their tokens.
+template <int NR, int NS, int MODE, bool SILU, bool ONE>
 __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
     const float* __restrict__ xbc, long xbc_stride, const float* __restrict__ dt_raw, long dt_stride,
     const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dw,
@@ -291,15 +294,16 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
     float* sX = sC + SSM_TB * NP;                      // [SSM_WAVES][SSM_TB][PW]
     float* sDt = sX + SSM_WAVES * SSM_TB * PW;         // [SSM_WAVES][SSM_TB]
     float* sA = sDt + SSM_WAVES * SSM_TB;              // [SSM_WAVES][SSM_TB]
-    // (the arguments in one trip, not a few at a time where the code first wants them)
-    asm volatile("" ::"s"(xbc), "s"(xbc_stride), "s"(dt_raw), "s"(dt_stride), "s"(dt_bias), "s"(A_log), "s"(Dw), "s"(state), "s"(slots), "s"(q_start), "s"(q_len));
-    asm volatile("" ::"s"(chunk_seg), "s"(carry), "s"(y), "s"(y_stride), "s"(heads), "s"(vdim), "s"(N), "s"(G), "s"(Q), "s"(fixed_a), "s"(fixed_dt));
+    if constexpr (ONE) {
+        asm volatile("" ::"s"(xbc), "s"(xbc_stride), "s"(dt_raw), "s"(dt_stride), "s"(dt_bias), "s"(A_log), "s"(Dw), "s"(state), "s"(slots), "s"(q_start), "s"(q_len));
+        asm volatile("" ::"s"(chunk_seg), "s"(carry), "s"(y), "s"(y_stride), "s"(heads), "s"(vdim), "s"(N), "s"(G), "s"(Q), "s"(fixed_a), "s"(fixed_dt));
+    }
     const int bx = blockIdx.x;
     const int seg = chunk_seg ? chunk_seg[bx] : bx;
     if (seg < 0) return;
     const int c = chunk_seg ? chunk_idx[bx] : 0;
     const int L = q_len[seg], start = q_start[seg], slot = slots[seg], first = c * Q;
-    asm volatile("" ::"s"(L), "s"(start), "s"(slot));
+    if constexpr (ONE) asm volatile("" ::"s"(L), "s"(start), "s"(slot));
     if (first >= L) return;
     const int ntok = (L - first < Q) ? L - first : Q;
     const bool last = first + ntok >= L;
@@ -322,8 +326,8 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
 #pragma unroll
         for (int r = 0; r < NR; ++r) {
             const int n = s * NR + r;
-            // (never conditional, and what is not the state's is blanked when all has been asked for)
-            S[r] = *reinterpret_cast<const float4*>(src + (size_t)(n < N ? n : N - 1) * vdim + (cols ? p : 0));
+            if constexpr (ONE) S[r] = *reinterpret_cast<const float4*>(src + (size_t)(n < N ? n : N - 1) * vdim + (cols ? p : 0));
+            else S[r] = (n < N && cols) ? *reinterpret_cast<const float4*>(src + (size_t)n * vdim + p) : float4{0.f, 0.f, 0.f, 0.f};
         }
     } else {
 #pragma unroll
@@ -331,11 +335,9 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
     }
     float prod = 1.f;
     const float Dh = (MODE == 0 && active && Dw) ? Dw[head] : 0.f;
-    // One token (a decoding step): its values come in one trip with the state, each asked for before any is used.  (48 heads of 64 x 128, one request 8.7 -> 8.3 us.)
     constexpr int BI = (NP + 64 * SSM_WAVES - 1) / (64 * SSM_WAVES), XI = (PW + 63) / 64;
     [[maybe_unused]] float oB[BI], oC[BI], oX[XI], oDt, oBias, oRate;
-    const bool one = MODE == 0 && ntok == 1;
-    if (one) {
+    if constexpr (ONE) {
         const float* row = xbc + (size_t)t0 * xbc_stride;
 #pragma unroll
         for (int i = 0; i < BI; ++i) {
@@ -348,11 +350,9 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
             const int pp = pbase + lane + 64 * i;
             oX[i] = row[(size_t)head * vdim + (pp < vdim ? pp : vdim - 1)];
         }
-        oDt = fixed_a ? 0.f : dt_raw[(size_t)t0 * dt_stride + head];
-        oBias = fixed_a ? 0.f : dt_bias[head];
-        oRate = (fixed_a ? fixed_a : A_log)[head];
-    }
-    if (MODE == 0) {
+        oDt = dt_raw[(size_t)t0 * dt_stride + head];
+        oBias = dt_bias[head];
+        oRate = A_log[head];
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             if (!(s * NR + r < N && cols)) S[r] = float4{0.f, 0.f, 0.f, 0.f};
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
     for (int b0 = 0; b0 < ntok; b0 += SSM_TB) {
         __syncthreads();
         const int nt = (ntok - b0 < SSM_TB) ? ntok - b0 : SSM_TB;          // (one in a decoding step: what is staged for the others would be waited for)
-        if (one) {
+        if constexpr (ONE) {
 #pragma unroll
             for (int i = 0; i < BI; ++i) {
                 const int n = threadIdx.x + 64 * SSM_WAVES * i;
@@ -370,9 +370,9 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
             for (int i = 0; i < XI; ++i)
                 if (lane + 64 * i < PW) sX[w * SSM_TB * PW + lane + 64 * i] = pbase + lane + 64 * i < vdim ? silu_if<SILU>(oX[i]) : 0.f;
             if (lane == 0) {
-                const float d = fixed_a ? fixed_dt : softplus_f32(oDt + oBias);
+                const float d = softplus_f32(oDt + oBias);
                 sDt[w * SSM_TB] = d;
-                sA[w * SSM_TB] = fixed_a ? oRate : expf(-expf(oRate) * d);
+                sA[w * SSM_TB] = expf(-expf(oRate) * d);
             }
         } else
         for (int i = threadIdx.x; i < nt * NP; i += 64 * SSM_WAVES) {
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void ssm_scan_quad_kernel(
             sB[i] = ok ? silu_if<SILU>(row[0]) : 0.f;
             sC[i] = ok ? silu_if<SILU>(row[(size_t)G * N]) : 0.f;
         }
-        if (active && !one) {
+        if (active && !ONE) {
             for (int i = lane; i < nt * PW; i += 64) {
                 const int tt = i / PW, pp = pbase + i % PW;
                 const bool ok = pp < vdim;
@@ -505,13 +505,19 @@ template <int NR, int NS, bool QUAD, bool SILU>
 static int ssm_launch_as(const float* xbc, long xbc_stride, const float* dt_raw, long dt_stride, const float* dt_bias,
                       const float* A_log, const float* Dw, float* state, const int* slots, const int* q_start, const int* q_len,
                       int* chunk_tab, float* carry, float* decay, float* y, long y_stride, int heads, int vdim, int N, int G,
-                      int Q, int segs, int max_chunks, bool chunked, const float* fixed_a, float fixed_dt, hipStream_t stream) {
+                      int Q, int segs, int max_chunks, bool chunked, const float* fixed_a, float fixed_dt, bool one, hipStream_t stream) {
     constexpr int NP = NR * NS, PW = (QUAD ? 256 : 64) / NS;
     const size_t lds = (size_t)(2 * SSM_TB * NP + SSM_WAVES * SSM_TB * PW + 2 * SSM_WAVES * SSM_TB) * sizeof(float);
-#define SSM_KERNEL(MODE_) (QUAD ? ssm_scan_quad_kernel<(QUAD ? NR : 4), (QUAD ? NS : 2), MODE_, SILU> : ssm_scan_kernel<(QUAD ? 16 : NR), (QUAD ? 1 : NS), MODE_, SILU>)
+#define SSM_KERNEL(MODE_) (QUAD ? ssm_scan_quad_kernel<(QUAD ? NR : 4), (QUAD ? NS : 2), MODE_, SILU, false> : ssm_scan_kernel<(QUAD ? 16 : NR), (QUAD ? 1 : NS), MODE_, SILU>)
     const int hpg = heads / G, PS = (vdim + PW - 1) / PW, U = hpg * PS, ublocks = (U + SSM_WAVES - 1) / SSM_WAVES;
     if (!chunked) {
         const dim3 grid(segs, G * ublocks);
+        if constexpr (QUAD)
+            if (one && !fixed_a) {
+                ssm_scan_quad_kernel<NR, NS, 0, SILU, true><<<grid, 64 * SSM_WAVES, lds, stream>>>(xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log, Dw,
+                    state, slots, q_start, q_len, nullptr, nullptr, nullptr, nullptr, y, y_stride, heads, vdim, N, G, Q, fixed_a, fixed_dt);
+                return li_launch_status();
+            }
         SSM_KERNEL(0)<<<grid, 64 * SSM_WAVES, lds, stream>>>(xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log, Dw,
             state, slots, q_start, q_len, nullptr, nullptr, nullptr, nullptr, y, y_stride, heads, vdim, N, G, Q, fixed_a, fixed_dt);
         return li_launch_status();
@@ -1053,7 +1059,7 @@ extern "C" int li_ssm_scan(const float* xbc, long xbc_stride, const float* dt_ra
 #define SSM_QUAD(NR_, NS_)                                                                                                \
     if (qr == NR_ && qs == NS_)                                                                                           \
         return ssm_launch<NR_, NS_, true>(silu_in, xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log, Dw, state, slots, q_start, q_len, \
-                                          chunk_tab, carry, decay, y, y_stride, heads, vdim, N, G, Q, segs, max_chunks, chunked, fixed_a, fixed_dt, stream);
+                                          chunk_tab, carry, decay, y, y_stride, heads, vdim, N, G, Q, segs, max_chunks, chunked, fixed_a, fixed_dt, max_q_len == 1, stream);
         SSM_QUAD(4, 2) SSM_QUAD(8, 2) SSM_QUAD(16, 2) SSM_QUAD(32, 2)
         SSM_QUAD(4, 4) SSM_QUAD(8, 4) SSM_QUAD(16, 4) SSM_QUAD(32, 4)
         SSM_QUAD(4, 8) SSM_QUAD(8, 8) SSM_QUAD(16, 8) SSM_QUAD(32, 8)
@@ -1063,7 +1069,7 @@ extern "C" int li_ssm_scan(const float* xbc, long xbc_stride, const float* dt_ra
 #define SSM_GO(NR_, NS_)                                                                                                  \
     if (nr == NR_ && ns == NS_)                                                                                           \
         return ssm_launch<NR_, NS_, false>(silu_in, xbc, xbc_stride, dt_raw, dt_stride, dt_bias, A_log, Dw, state, slots, q_start, q_len,    \
-                                    chunk_tab, carry, decay, y, y_stride, heads, vdim, N, G, Q, segs, max_chunks, chunked, fixed_a, fixed_dt, stream);
+                                    chunk_tab, carry, decay, y, y_stride, heads, vdim, N, G, Q, segs, max_chunks, chunked, fixed_a, fixed_dt, max_q_len == 1, stream);
     SSM_GO(16, 1) SSM_GO(32, 1) SSM_GO(64, 1) SSM_GO(128, 1)
     SSM_GO(16, 2) SSM_GO(32, 2) SSM_GO(64, 2) SSM_GO(128, 2)
     SSM_GO(16, 4) SSM_GO(32, 4) SSM_GO(64, 4)
@@ -1107,7 +1113,7 @@ template <int NS> __device__ __forceinline__ float lanes_sum(float v) {
 //   MODE 0: the recurrence itself from that state, with the outputs; the last chunk leaves the request's state.
 // A portion of at most Q tokens (a decoding step) is MODE 0 alone, from the request's state.
 
-template <int NR, int NS, int CW, int MODE>
+template <int NR, int NS, int CW, int MODE, bool ONE = false>
 __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
     const float* __restrict__ xkq, long x_stride, const float* __restrict__ ba, long ba_stride,
     const float* __restrict__ dt_bias, const float* __restrict__ A_log, float* __restrict__ state,
@@ -1121,14 +1127,16 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
     float* sX = sQ + DR_TB * NP;                       // [SSM_WAVES][DR_TB][PW]
     float* sBeta = sX + SSM_WAVES * DR_TB * PW;        // [SSM_WAVES][DR_TB]
     float* sG = sBeta + SSM_WAVES * DR_TB;             // [SSM_WAVES][DR_TB]
-    asm volatile("" ::"s"(xkq), "s"(x_stride), "s"(ba), "s"(ba_stride), "s"(dt_bias), "s"(A_log), "s"(state), "s"(slots), "s"(q_start), "s"(q_len));      // (in one trip)
-    asm volatile("" ::"s"(chunk_seg), "s"(carry), "s"(y), "s"(y_stride), "s"(heads), "s"(vdim), "s"(N), "s"(G), "s"(Q), "s"(q_scale));
+    if constexpr (ONE) {                               // (see ssm_scan_quad_kernel)
+        asm volatile("" ::"s"(xkq), "s"(x_stride), "s"(ba), "s"(ba_stride), "s"(dt_bias), "s"(A_log), "s"(state), "s"(slots), "s"(q_start), "s"(q_len));      // (in one trip)
+        asm volatile("" ::"s"(chunk_seg), "s"(carry), "s"(y), "s"(y_stride), "s"(heads), "s"(vdim), "s"(N), "s"(G), "s"(Q), "s"(q_scale));
+    }
     const int bx = blockIdx.x;
     const int seg = chunk_seg ? chunk_seg[bx] : bx;
     if (seg < 0) return;
     const int c = chunk_seg ? chunk_idx[bx] : 0;
     const int L = q_len[seg], start = q_start[seg], slot = slots[seg], first = c * Q;
-    asm volatile("" ::"s"(L), "s"(start), "s"(slot));
+    if constexpr (ONE) asm volatile("" ::"s"(L), "s"(start), "s"(slot));
     if (first >= L) return;
     const int ntok = chunk_seg ? ((L - first < Q) ? L - first : Q) : L;
     const bool last = first + ntok >= L;
@@ -1156,19 +1164,19 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
 #pragma unroll
             for (int cc = 0; cc < CW; ++cc) S[r][cc] = (is_p && n == p + cc) ? 1.f : 0.f;
         } else if constexpr (CW == 4) {
-            // (never conditional, and what is not the state's is blanked when all has been asked for)
-            const float4 v4 = *reinterpret_cast<const float4*>(src + (size_t)(n < N ? n : N - 1) * vdim + (p < vdim ? p : 0));
+            float4 v4;
+            if constexpr (ONE) v4 = *reinterpret_cast<const float4*>(src + (size_t)(n < N ? n : N - 1) * vdim + (p < vdim ? p : 0));
+            else v4 = (active && n < N && p < vdim) ? *reinterpret_cast<const float4*>(src + (size_t)n * vdim + p) : float4{0.f, 0.f, 0.f, 0.f};
             S[r][0] = v4.x; S[r][1] = v4.y; S[r][2] = v4.z; S[r][3] = v4.w;
         } else {
 #pragma unroll
             for (int cc = 0; cc < CW; ++cc) S[r][cc] = (active && n < N && p + cc < vdim) ? src[(size_t)n * vdim + p + cc] : 0.f;
         }
     }
-    // One token (a decoding step): its values come in one trip with the state, each asked for before any is used.  (12 heads of 128 x 128, 8 requests 11.5 -> 11.0 us.)
+    // (12 heads of 128 x 128, 8 requests 11.5 -> 11.0 us)
     constexpr int BI = (NP + 64 * SSM_WAVES - 1) / (64 * SSM_WAVES), XI = (PW + 63) / 64;
     [[maybe_unused]] float oK[BI], oQ[BI], oX[XI], oBeta, oDt, oBias, oRate;
-    const bool one = MODE == 0 && ntok == 1;
-    if (one) {
+    if constexpr (ONE) {
         const float* row = xkq + (size_t)t0 * x_stride;
 #pragma unroll
         for (int i = 0; i < BI; ++i) {
@@ -1186,7 +1194,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
         oBias = dt_bias[head];
         oRate = A_log[head];
     }
-    if constexpr (MODE == 0 && CW == 4) {
+    if constexpr (ONE && CW == 4) {
 #pragma unroll
         for (int r = 0; r < NR; ++r)
             if (!(active && s * NR + r < N && p < vdim)) S[r][0] = S[r][1] = S[r][2] = S[r][3] = 0.f;
@@ -1194,7 +1202,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
     for (int b0 = 0; b0 < ntok; b0 += DR_TB) {
         __syncthreads();
         const int nt = (ntok - b0 < DR_TB) ? ntok - b0 : DR_TB;
-        if (one) {
+        if constexpr (ONE) {
 #pragma unroll
             for (int i = 0; i < BI; ++i) {
                 const int n = threadIdx.x + 64 * SSM_WAVES * i;
@@ -1215,7 +1223,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
             sK[i] = ok ? row[0] : 0.f;
             sQ[i] = ok ? row[(size_t)G * N] : 0.f;
         }
-        if (active && !one) {
+        if (active && !ONE) {
             for (int i = lane; i < nt * PW; i += 64) {
                 const int tt = i / PW, pp = pbase + i % PW;
                 const bool ok = !is_p && pp < vdim;
@@ -1445,11 +1453,17 @@ template <int NR, int NS, int CW>
 static int delta_launch(const float* xkq, long x_stride, const float* ba, long ba_stride, const float* dt_bias, const float* A_log,
                         float* state, const int* slots, const int* q_start, const int* q_len, int* chunk_tab, float* carry,
                         float* pmat, float* y, long y_stride, int heads, int vdim, int N, int G, int Q, float q_scale, int segs,
-                        int max_chunks, bool chunked, hipStream_t stream) {
+                        int max_chunks, bool chunked, bool one, hipStream_t stream) {
     constexpr int NP = NR * NS, PW = 64 * CW / NS;
     const size_t lds = (size_t)(2 * DR_TB * NP + SSM_WAVES * DR_TB * PW + 2 * SSM_WAVES * DR_TB) * sizeof(float);
     const int hpg = heads / G, PSV = (vdim + PW - 1) / PW, PSP = (N + PW - 1) / PW;
     const int ub0 = (hpg * PSV + SSM_WAVES - 1) / SSM_WAVES, ub1 = (hpg * (PSV + PSP) + SSM_WAVES - 1) / SSM_WAVES;
+    if (!chunked && one) {
+        delta_scan_kernel<NR, NS, CW, 0, true><<<dim3(segs, G * ub0), 64 * SSM_WAVES, lds, stream>>>(
+            xkq, x_stride, ba, ba_stride, dt_bias, A_log, state, slots, q_start, q_len, nullptr, nullptr, nullptr, nullptr,
+            y, y_stride, heads, vdim, N, G, Q, q_scale);
+        return li_launch_status();
+    }
     if (!chunked) {
         delta_scan_kernel<NR, NS, CW, 0><<<dim3(segs, G * ub0), 64 * SSM_WAVES, lds, stream>>>(
             xkq, x_stride, ba, ba_stride, dt_bias, A_log, state, slots, q_start, q_len, nullptr, nullptr, nullptr, nullptr,
@@ -1502,7 +1516,7 @@ extern "C" int li_delta_scan(const float* xkq, long x_stride, const float* ba, l
         pmat = carry + (size_t)max_chunks * heads * N * vdim;
     }
 #define DR_ARGS xkq, x_stride, ba, ba_stride, dt_bias, A_log, state, slots, q_start, q_len, chunk_tab, carry, pmat, y, y_stride, heads, \
-                vdim, N, G, Q, q_scale, segs, max_chunks, chunked, stream
+                vdim, N, G, Q, q_scale, segs, max_chunks, chunked, max_q_len == 1, stream
     const bool aligned = ((uintptr_t)state | (uintptr_t)y | (uintptr_t)carry) % 16 == 0 && y_stride % 4 == 0;
     int qs = 0, qr = 0;
     if (aligned && ssm_quad_layout(N, vdim, &qs, &qr)) {
