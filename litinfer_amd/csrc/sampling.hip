@@ -19,8 +19,8 @@ __device__ __forceinline__ void argmax_combine(float& v, int& i, float ov, int o
 __device__ __forceinline__ void block_argmax(float& v, int& i, float* sv, int* si) {
 #pragma unroll
     for (int o = LI_WAVE / 2; o > 0; o >>= 1) {
-        const float ov = lane_xor(v, o);
-        const int oi = lane_xor(i, o);
+        const float ov = __shfl_xor(v, o, LI_WAVE);
+        const int oi = __shfl_xor(i, o, LI_WAVE);
         argmax_combine(v, i, ov, oi);
     }
     const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
@@ -60,8 +60,8 @@ __global__ __launch_bounds__(64) void argmax_final_kernel(const float* __restric
     for (int c = threadIdx.x; c < nchunks; c += 64) argmax_combine(v, i, pv[blockIdx.x * nchunks + c], pi[blockIdx.x * nchunks + c]);
 #pragma unroll
     for (int o = LI_WAVE / 2; o > 0; o >>= 1) {
-        const float ov = lane_xor(v, o);
-        const int oi = lane_xor(i, o);
+        const float ov = __shfl_xor(v, o, LI_WAVE);
+        const int oi = __shfl_xor(i, o, LI_WAVE);
         argmax_combine(v, i, ov, oi);
     }
     if (threadIdx.x == 0) out[blockIdx.x] = i;
@@ -174,7 +174,7 @@ __device__ __forceinline__ bool sample_unfiltered(int k, float p, int V) { retur
 
 __device__ __forceinline__ int block_sum_int(int v, int* smem) {
 #pragma unroll
-    for (int o = LI_WAVE / 2; o > 0; o >>= 1) v += lane_xor(v, o);
+    for (int o = LI_WAVE / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, LI_WAVE);
     const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
     __syncthreads();
     if (lane == 0) smem[w] = v;
@@ -199,7 +199,7 @@ __device__ __forceinline__ float block_max_f(float v, float* smem) {
 
 __device__ __forceinline__ int block_min_int(int v, int* smem) {
 #pragma unroll
-    for (int o = LI_WAVE / 2; o > 0; o >>= 1) v = min(v, lane_xor(v, o));
+    for (int o = LI_WAVE / 2; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, LI_WAVE));
     const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
     __syncthreads();
     if (lane == 0) smem[w] = v;
@@ -224,7 +224,7 @@ __device__ __forceinline__ void block_sum16(T (&c)[16], T* work, T* tot) {
         _Pragma("unroll") for (int i = 0; i < (H); ++i) {                         \
             const T give = upper ? c[i] : c[i + (H)];                             \
             const T keep = upper ? c[i + (H)] : c[i];                             \
-            c[i] = keep + lane_xor(give, (MASK));                                    \
+            c[i] = keep + __shfl_xor(give, (MASK), LI_WAVE);                      \
         }                                                                         \
     }
     LI_HALVE(8, 1)
@@ -232,8 +232,8 @@ __device__ __forceinline__ void block_sum16(T (&c)[16], T* work, T* tot) {
     LI_HALVE(2, 4)
     LI_HALVE(1, 8)
 #undef LI_HALVE
-    c[0] += lane_xor(c[0], 16);
-    c[0] += lane_xor(c[0], 32);
+    c[0] += __shfl_xor(c[0], 16, LI_WAVE);
+    c[0] += __shfl_xor(c[0], 32, LI_WAVE);
     // lane l < 16 now holds the wave's sum number 8 (l & 1) + 4 (l >> 1 & 1) + 2 (l >> 2 & 1) + (l >> 3 & 1)
     __syncthreads();                                 // (the last pass's totals have been read)
     if (lane < 16) work[w * 16 + 8 * (lane & 1) + 4 * ((lane >> 1) & 1) + 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1)] = c[0];
