@@ -1965,6 +1965,7 @@ extern "C" long li_linear_work_bytes(int M, int N, int K, int in_dtype);
 // the bias, rotates query and key heads (half-split pairs over the whole head, float32 tables
 // [M, dh / 2]) and writes keys and values into their page slots, so that the rotation needs no
 // kernel of its own.  Thread (row, head, pair): consecutive threads read consecutive sums.
+template <int HELD>
 __global__ __launch_bounds__(256) void splitk_reduce_rope_store_kernel(
     const float* __restrict__ part, int nsplit, size_t mn, int N, const float* __restrict__ bias, bf16_t* __restrict__ out,
     const float* __restrict__ cosv, const float* __restrict__ sinv, const int* __restrict__ slot_map,
@@ -1974,8 +1975,18 @@ __global__ __launch_bounds__(256) void splitk_reduce_rope_store_kernel(
     const int half = dh / 2, heads = nh + 2 * nkv;
     const int j = (int)(i % half), head = (int)((i / half) % heads), m = (int)(i / ((long)half * heads));
     const size_t i0 = (size_t)m * N + (size_t)head * dh + j, i1 = i0 + half;
-    float a = part[i0], b = part[i1];
-    for (int sp = 1; sp < nsplit; ++sp) { a += part[(size_t)sp * mn + i0]; b += part[(size_t)sp * mn + i1]; }
+    float a, b;
+    if constexpr (HELD > 0) {
+        Parts<(HELD > PARTS_HELD)> pa, pb;
+        pa.ask(part, nsplit, mn, i0);
+        pb.ask(part, nsplit, mn, i1);
+        a = pa.sum(nsplit);
+        b = pb.sum(nsplit);
+    } else {
+        a = part[i0];
+        b = part[i1];
+        for (int sp = 1; sp < nsplit; ++sp) { a += part[(size_t)sp * mn + i0]; b += part[(size_t)sp * mn + i1]; }
+    }
     if (bias) { a += bias[head * dh + j]; b += bias[head * dh + j + half]; }
     if (head < nh + nkv) {
         const float c = cosv[(size_t)m * half + j], sn = sinv[(size_t)m * half + j];
@@ -2021,9 +2032,14 @@ extern "C" int li_linear_rope_store_parts(const void* x, const void* w, const fl
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit);
     if (rc != LI_OK) return rc;
     const long total = (long)M * (nh + 2 * nkv) * (dh / 2);
-    splitk_reduce_rope_store_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(
-        (const float*)work, nsplit, mn, N, bias, (bf16_t*)out, cos, sin, slot_map, (bf16_t*)kc, (bf16_t*)vc,
-        nh, nkv, dh, page_size, num_pages, total);
+#define LI_RR(HELD) splitk_reduce_rope_store_kernel<HELD><<<(unsigned)((total + 255) / 256), 256, 0, stream>>>( \
+        (const float*)work, nsplit, mn, N, bias, (bf16_t*)out, cos, sin, slot_map, (bf16_t*)kc, (bf16_t*)vc, nh, nkv, dh, page_size, num_pages, total)
+    // (few rows: all parts at once, as in the other kernels that add them up; read part after part, sixteen were slower than eight had been: 33 rows of
+    // 2,048 x 8,960 15.3 -> 16.5 us)
+    if (nsplit > PARTS_HELD) LI_RR(MID_PARTS);
+    else if (M <= 64) LI_RR(PARTS_HELD);
+    else LI_RR(0);
+#undef LI_RR
     return li_launch_status();
 }
 
