@@ -54,6 +54,8 @@ __device__ __forceinline__ float route_dot16(const uint4 r, const float* xs, con
 // What a plan is made of (see moe_plan_kernel below); plan null: none.
 struct MoePlanOut { int* plan; int* row_token; int* pair_row; float* row_wt; int* count; int max_tiles, tile_rows, experts; };
 #define MOE_PLAN_HELD 4
+#define MOE_PLACES_CHOICE 16      // router outputs a choice, up to 64 in all, up to which all places are found at once,
+#define MOE_PLACES_ONE 8          // ... and for one choice
 #define MOE_PLAN_EXPERTS 64       // experts up to which the router makes the plan: one a lane
 
 // A wave's fence: what its lanes wrote to LDS is there for its other lanes
@@ -280,7 +282,10 @@ __device__ __forceinline__ void moe_route_token(const MoeRoute<TX, TW>& a, const
     float chosen = 0.f, mx = 0.f, sum = 0.f;
     int mine = -1;
     unsigned long long taken = 0;                      // (up to 64 router outputs: those that were chosen)
-    if (E <= 64) {
+    // All places at once is a turn an output, a round of a maximum twelve exchanges between lanes: where the choices are few for the outputs,
+    // rounds (places / rounds, 3 tokens, 1 of 64 outputs of 256 columns 9.3 / 7.1 us, 2 of 64 of 2,240 12.0 / 10.3; 128 tokens, 1 of 48 7.0 / 5.4; 16
+    // tokens, 1 of 32 10.0 / 9.1).
+    if (E <= 64 && E <= (top == 1 ? MOE_PLACES_ONE : MOE_PLACES_CHOICE * top)) {
         // An output a lane: its place is the number of those that go before it (a larger value, or an equal one and a lower number), all
         // places at once, where rounds of a maximum took twelve exchanges between lanes a choice.  The values are compared as whole
         // numbers of the same order (both zeros the same; what is no number before all others), so every place is some output's.
@@ -322,6 +327,7 @@ __device__ __forceinline__ void moe_route_token(const MoeRoute<TX, TW>& a, const
         const float ex = mode != 0 ? sc[bi] : expf(best - mx);
         sum += ex;
         if (lane == r) { mine = bi; chosen = ex; }
+        if (E <= 64) taken |= 1ull << (bi & 63);
         if (lane == 0) lg[bi] = -INFINITY;
         // (a wave's LDS instructions are carried out in the order of their issue: the next round reads what lane 0 wrote)
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");

@@ -511,6 +511,21 @@ def test_the_routers_launch_makes_the_plan_too(dt, T, K, n_router, experts, top,
         assert torch.equal(p2.row_wt.cpu()[at[have]], w2.cpu().view(-1)[have])
 
 
+@pytest.mark.parametrize("dt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("T,n_router,experts,top", [(1, 64, 60, 1), (3, 64, 64, 3), (3, 64, 64, 4), (1, 64, 64, 4), (1, 9, 7, 1), (5, 8, 8, 1), (1, 33, 33, 2), (2, 32, 30, 2)])
+def test_few_choices_of_many_outputs(dt, T, n_router, experts, top):
+    """Both ways to pick, at the lines between them: the choices in 64 bits, and the plan made of them."""
+    from litinfer_amd.kernels import ops
+    g = torch.Generator().manual_seed(n_router + top)
+    x, router = torch.randn(T, 256, generator=g).to(DT[dt]), torch.randn(n_router, 256, generator=g).to(DT[dt])
+    idx, wt = torch.empty(T, top, dtype=torch.int32, device=DEV), torch.empty(T, top, device=DEV)
+    ops.moe_route(x.to(DEV), router.to(DEV), None, None, idx, wt, None)
+    best = (x.double() @ router.double().t()).sort(descending=True, stable=True)
+    assert torch.equal(idx.cpu().long(), best.indices[:, :top])
+    assert np.abs(wt.cpu().numpy() - torch.softmax(best.values[:, :top], 1).numpy()).max() < 1e-4
+    test_the_routers_launch_makes_the_plan_too(dt, T, 256, n_router, experts, top, 32)
+
+
 def test_difference_of_two_maps_and_its_norm():
     from litinfer_amd.kernels import ops
     rng = np.random.default_rng(2)
