@@ -57,6 +57,17 @@ def test_rmsnorm(ops, dtype, shape, eps):
     assert rel(out, ref) < tol(dtype, 2e-6, 8e-3)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("shape", [(2, 70), (255, 1024), (255, 1025), (3, 9001), (256, 1025), (1100, 300)])      # few rows of one column a thread and more, many rows
+def test_rmsnorm_of_bfloat16_rows(ops, dtype, shape):
+    g = torch.Generator().manual_seed(84)
+    x = (torch.randn(*shape, generator=g) * 3).to(torch.bfloat16)
+    w = 1 + 0.1 * torch.randn(shape[1], generator=g)
+    out = torch.full(shape, float("nan"), dtype=dtype, device=DEV)
+    ops.rmsnorm(x.to(DEV), w.to(DEV), 1e-6, out)
+    assert rel(out, plain_impl.rms_norm(x.double().numpy(), w.double().numpy(), 1e-6)) < tol(dtype, 2e-6, 8e-3)
+
+
 def test_rmsnorm_zero_row_is_zero_not_nan(ops):
     x = torch.zeros(2, 64, device=DEV)
     out = torch.empty(2, 64, device=DEV)
@@ -1587,6 +1598,12 @@ def test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, weigh, g
     assert rel(out, y.numpy()) < (8 * math.sqrt(k) * 2.0 ** -24 if out_dtype is torch.float32 else 8e-3)
 
 
+@pytest.mark.parametrize("counts,n_out,k,act,out_dtype", [([1, 0, 2], 20, 2560, 0, torch.float32), ([1, 0, 3], 22, 2568, 2, torch.bfloat16),
+                                                           ([1], 37, 4096, 0, torch.float32)])      # pieces held by a wave, and one piece more
+def test_routed_product_of_few_long_rows(ops, counts, n_out, k, act, out_dtype):
+    test_routed_product_of_a_decoding_batch(ops, counts, n_out, k, act, False, True, out_dtype)
+
+
 @pytest.mark.parametrize("counts,tile,n_out,k,act,weigh,gather,out_dtype", [
     ([1, 64, 0, 65, 63], 64, 32, 64, 0, False, True, torch.float32),           # one step of k; a quarter of a block's outputs
     ([130, 5, 200], 64, 160, 192, 2, False, True, torch.bfloat16),             # three steps, pairs of gate and up
@@ -1736,6 +1753,13 @@ def test_recurrences_of_a_decoding_step(ops, kind, n, heads, vdim, n_state, grou
     assert rel(y, want.reshape(n, -1).numpy()) < tol_
     assert rel(dev_state[torch.arange(n - 1, -1, -1)], new.numpy()) < tol_
     assert torch.equal(dev_state[n].cpu(), state[n])                       # a slot that is not in the batch
+
+
+@pytest.mark.parametrize("n,heads,vdim,n_state,groups", [(40, 5, 32, 16, 5), (3, 3, 20, 12, 3), (70, 6, 128, 64, 2)])
+@pytest.mark.parametrize("kind", ["ssm", "fixed", "delta"])
+def test_recurrences_of_a_decoding_step_with_idle_waves(ops, kind, n, heads, vdim, n_state, groups):
+    """Heads that fill no whole block: waves without columns, lanes without columns and values."""
+    test_recurrences_of_a_decoding_step(ops, kind, n, heads, vdim, n_state, groups)
 
 
 @pytest.mark.parametrize("lens,heads,vdim,n_state,groups,skip_d", [
