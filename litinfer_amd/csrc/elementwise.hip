@@ -43,7 +43,7 @@ extern "C" int li_embedding(const int* ids, const int* id_src, const int* feedba
 // read once and kept in registers (up to RN_PER elements a thread); longer rows are read again.
 // Few rows (a decoding step): 1024 threads a row, so that the one row is read with the least
 // latency; many rows (a prompt): 256 threads a row, less of a block's time goes into meeting.
-template <typename TI, typename TO, int NT, int PER>
+template <typename TI, typename TO, int NT, int PER, bool AHEAD>
 __global__ __launch_bounds__(NT) void rmsnorm_kernel(const TI* __restrict__ x, const float* __restrict__ w,
                                                       float eps, TO* __restrict__ out, int H) {
     __shared__ float red[NT / LI_WAVE];
@@ -51,20 +51,31 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(const TI* __restrict__ x, c
     TO* o = out + (size_t)blockIdx.x * H;
     // The weights come with the row: behind the sum they were a trip of their own, and, read once a step, one to memory.  (Few rows, here and in
     // the norms below, never a load under a thread's own condition: a column past the row is the last one again, and counts for nothing.)
+    // AHEAD: few rows of more than one column a thread.  Others do not gain by it and pay for the loads past the row's end (2,048 bfloat16 rows of 768
+    // 5.8 / 5.2 us, 600 of 896 4.0 / 3.9, 16 rows of 64 3.0 / 2.8).
     float v[PER], g[PER];
     float ss = 0.f;
+    if constexpr (AHEAD) {
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        if (i * NT >= H) continue;
-        const int j = threadIdx.x + i * NT, jj = j < H ? j : H - 1;
-        v[i] = load_as_float(row + jj);
-        g[i] = w[jj];
-    }
+        for (int i = 0; i < PER; ++i) {
+            if (i * NT >= H) continue;
+            const int j = threadIdx.x + i * NT, jj = j < H ? j : H - 1;
+            v[i] = load_as_float(row + jj);
+            g[i] = w[jj];
+        }
 #pragma unroll
-    for (int i = 0; i < PER; ++i) {
-        if (i * NT >= H) continue;
-        v[i] = (int)threadIdx.x + i * NT < H ? v[i] : 0.f;
-        ss = fmaf(v[i], v[i], ss);
+        for (int i = 0; i < PER; ++i) {
+            if (i * NT >= H) continue;
+            v[i] = (int)threadIdx.x + i * NT < H ? v[i] : 0.f;
+            ss = fmaf(v[i], v[i], ss);
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < PER; ++i) {
+            const int j = threadIdx.x + i * NT;
+            v[i] = (j < H) ? load_as_float(row + j) : 0.f;
+            ss += v[i] * v[i];
+        }
     }
     for (int j = threadIdx.x + PER * NT; j < H; j += NT) { const float t = load_as_float(row + j); ss += t * t; }
     ss = block_sum<NT>(ss, red);
@@ -72,7 +83,7 @@ __global__ __launch_bounds__(NT) void rmsnorm_kernel(const TI* __restrict__ x, c
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int j = threadIdx.x + i * NT;
-        if (j < H) store_from_float(o + j, g[i] * v[i] * inv);
+        if (j < H) store_from_float(o + j, (AHEAD ? g[i] : w[j]) * v[i] * inv);
     }
     for (int j = threadIdx.x + PER * NT; j < H; j += NT)
         store_from_float(o + j, w[j] * load_as_float(row + j) * inv);
@@ -117,8 +128,9 @@ extern "C" int li_rmsnorm(const void* x, int x_dtype, const float* w, float eps,
     if (T <= 0 || H <= 0) return LI_ERR_SIZE;
 #define LI_NORM(TI, TO)                                                                                        \
     {                                                                                                          \
-        if (T >= 256) rmsnorm_kernel<TI, TO, 256, 16><<<T, 256, 0, stream>>>((const TI*)x, w, eps, (TO*)out, H); \
-        else rmsnorm_kernel<TI, TO, 1024, 8><<<T, 1024, 0, stream>>>((const TI*)x, w, eps, (TO*)out, H);        \
+        if (T >= 256) rmsnorm_kernel<TI, TO, 256, 16, false><<<T, 256, 0, stream>>>((const TI*)x, w, eps, (TO*)out, H);          \
+        else if (H > 1024) rmsnorm_kernel<TI, TO, 1024, 8, true><<<T, 1024, 0, stream>>>((const TI*)x, w, eps, (TO*)out, H);     \
+        else rmsnorm_kernel<TI, TO, 1024, 8, false><<<T, 1024, 0, stream>>>((const TI*)x, w, eps, (TO*)out, H);                   \
     }
     if (x_dtype == LI_F32 && T >= 256 && H % 4 == 0 && H <= 4 * 256 * 8 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0) {
         if (out_dtype == LI_F32) rmsnorm_vec_kernel<float, 256, 8><<<T, 256, 0, stream>>>((const float*)x, w, eps, (float*)out, H);
@@ -1421,7 +1433,10 @@ __global__ __launch_bounds__(NT) void hyper_step_kernel(
     const int np = H / V;
     hyper_piece<V> u[PER], gw[PER];
     float ss = 0.f;
-    if (win) {                                             // the norm's weights come with the streams, not behind the sum (4 streams, 2 tokens 4.5 -> 3.8 us)
+    // the norm's weights come with the streams, not behind the sum (4 streams, 2 tokens 4.5 -> 3.8 us); many rows of more than four streams have no
+    // registers left for it (2,048 tokens of 5 x 896 16.3 / 15.6)
+    constexpr bool AHEAD = S <= 4 || NT == 1024;
+    if (AHEAD && win) {
 #pragma unroll
         for (int i = 0; i < PER; ++i)
             if (i * NT < np) {
