@@ -1521,7 +1521,7 @@ __global__ __launch_bounds__(NT) void hyper_step_kernel(
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const int p = threadIdx.x + i * NT;
-        if (p < np) finish(p * V, u[i], gw[i]);
+        if (p < np) finish(p * V, u[i], AHEAD ? gw[i] : hyper_load<V>(w + p * V));
     }
     for (int p = threadIdx.x + PER * NT; p < np; p += NT) {          // long rows: the sum once more, from what this thread left
         const int j = p * V;

@@ -487,6 +487,12 @@ def test_streams_step(dt, n, T, H):
     assert np.abs(out.cpu().numpy() - sum(xs)[pick]).max() < 1e-5 * np.abs(sum(xs)).max()
 
 
+@pytest.mark.parametrize("n,T,H", [(5, 300, 1028), (8, 255, 1028), (4, 300, 1024)])
+def test_streams_step_of_many_tokens(n, T, H):
+    """The norm's weights come with the streams, or, where many tokens have more than four, behind them."""
+    test_streams_step("bfloat16", n, T, H)
+
+
 @pytest.mark.parametrize("dt", ["float32", "bfloat16"])
 def test_small_kernels_of_the_design(dt):
     from litinfer_amd.kernels import ops
