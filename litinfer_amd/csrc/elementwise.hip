@@ -479,7 +479,7 @@ extern "C" int li_embedding_add(const int* ids, const int* id_src, const int* fe
 // reads the stream next, xn[t, :] = the RMS norm of the NEW x with weights w2 and eps2 (next 1) or the new x itself in
 // xn's type (next 2): one block a row.
 #define RA_HELD 4         // columns of a row that a thread holds
-template <typename TO, int NT>
+template <typename TO, int NT, bool HELD>
 __global__ __launch_bounds__(NT) void rmsnorm_add_kernel(const float* __restrict__ y, const float* __restrict__ y2, float a1, float a2,
                                                           const float* __restrict__ w, float eps,
                                                           float* __restrict__ x, const float* __restrict__ w2, float eps2,
@@ -489,9 +489,8 @@ __global__ __launch_bounds__(NT) void rmsnorm_add_kernel(const float* __restrict
     const float* yr2 = y2 ? y2 + (size_t)blockIdx.x * H : nullptr;
     float* xr = x + (size_t)blockIdx.x * H;
     float ss = 0.f;
-    // Short rows: a thread's columns wait in registers, all asked for at once (8 x 1,536 3.8 -> 3.2 us).  Not where there are thousands and most
-    // threads have no column of their own, whose loads are then what the chip is busy with (2,048 x 64 3.6 -> 3.9).
-    if (H <= RA_HELD * NT && (2 * H > NT || gridDim.x <= 1024)) {
+    // Short rows: a thread's columns wait in registers, all asked for at once (8 x 1,536 3.8 -> 3.2 us).
+    if constexpr (HELD) {
         float b[RA_HELD], u[RA_HELD], r[RA_HELD], g[RA_HELD], g2[RA_HELD];
 #pragma unroll
         for (int i = 0; i < RA_HELD; ++i) {
@@ -556,15 +555,21 @@ extern "C" int li_rmsnorm_add(const float* y, const float* y2, float a1, float a
     if (T <= 0 || H <= 0 || next < 0 || next > 2) return LI_ERR_SIZE;
     if ((next && !xn) || (next == 1 && !w2)) return LI_ERR_SIZE;
     const bool wide = T < 256 && H > 1024;
+    // Held rows: not where there are thousands and most threads have no column of their own, whose loads are then what the chip is busy with (2,048 x
+    // 64 3.6 / 3.9 us); an instance of its own, as long rows pay for its registers (300 x 8,192 17.6 / 18.2).
+    const int nt = wide ? 1024 : 256;
+    const bool held = H <= RA_HELD * nt && (2 * H > nt || T <= 1024);
+#define LI_RAH(TO, NT, HELD) rmsnorm_add_kernel<TO, NT, HELD><<<T, NT, 0, stream>>>(y, y2, a1, a2, w, eps, x, w2, eps2, (TO*)xn, next, H)
 #define LI_RA(TO)                                                                                             \
     {                                                                                                         \
-        if (wide) rmsnorm_add_kernel<TO, 1024><<<T, 1024, 0, stream>>>(y, y2, a1, a2, w, eps, x, w2, eps2, (TO*)xn, next, H);   \
-        else rmsnorm_add_kernel<TO, 256><<<T, 256, 0, stream>>>(y, y2, a1, a2, w, eps, x, w2, eps2, (TO*)xn, next, H);          \
+        if (wide) { if (held) LI_RAH(TO, 1024, true); else LI_RAH(TO, 1024, false); }                         \
+        else { if (held) LI_RAH(TO, 256, true); else LI_RAH(TO, 256, false); }                                \
     }
     if (!next || xn_dtype == LI_F32) LI_RA(float)
     else if (xn_dtype == LI_BF16) LI_RA(bf16_t)
     else return LI_ERR_DTYPE;
 #undef LI_RA
+#undef LI_RAH
     return li_launch_status();
 }
 
@@ -957,7 +962,7 @@ extern "C" int li_qk_head_norm_store(float* qkv, long row_stride, int nh, int nk
 // Where the queries go through a latent of their own, `ql` holds its q_rank columns before the norm and `cq` takes
 // the RMS norm with weights wq (in the dtype of the product that follows).
 #define LN_HELD 4         // columns of a latent that a thread holds
-template <typename T, typename TQ, int NT>
+template <typename T, typename TQ, int NT, bool HELD>
 __global__ __launch_bounds__(NT) void latent_norm_pairs_store_kernel(
     const float* __restrict__ q, long q_stride, int nh, int dn, int dr, const float* __restrict__ down, long down_stride,
     int rank, const float* __restrict__ wc, float eps, const float* __restrict__ cosv, const float* __restrict__ sinv,
@@ -968,11 +973,11 @@ __global__ __launch_bounds__(NT) void latent_norm_pairs_store_kernel(
     const int second = split ? half : 1, step = split ? 1 : 2;       // a pair is (step * i, step * i + second)
     const float* c = cosv + (size_t)t * half;
     const float* sn = sinv + (size_t)t * half;
-    // both latents and their weights are asked for before the heads are rotated (32 tokens, latents of 768 and 256: 6.2 -> 4.5 us)
-    const bool held = (q_rank <= LN_HELD * NT) && rank <= LN_HELD * NT;
+    // both latents and their weights are asked for before the heads are rotated (32 tokens, latents of 768 and 256: 6.2 -> 4.5 us).  One latent
+    // alone has nothing to wait behind (64 tokens, 28 heads on 256 columns 3.9 us held, 3.8 not).
     float lv[LN_HELD], lw[LN_HELD], dv[LN_HELD], dww[LN_HELD];
     int slot = 0;
-    if (held) {
+    if constexpr (HELD) {
         if (q_rank > 0)
 #pragma unroll
             for (int i = 0; i < LN_HELD; ++i) {
@@ -1004,7 +1009,7 @@ __global__ __launch_bounds__(NT) void latent_norm_pairs_store_kernel(
             dst[0] = ra; dst[second] = rb;
         }
     }
-    if (held) {
+    if constexpr (HELD) {
         float s = 0.f;
         if (q_rank > 0) {
 #pragma unroll
@@ -1039,9 +1044,9 @@ __global__ __launch_bounds__(NT) void latent_norm_pairs_store_kernel(
     }
     if (!store) return;
     const float* dw = down + (size_t)t * down_stride;
-    if (!held) slot = slot_map[t];
+    if (!HELD) slot = slot_map[t];
     T* row = cache + (size_t)slot * (rank + dr);
-    if (!held) {
+    if (!HELD) {
         float s = 0.f;
         for (int j = threadIdx.x; j < rank; j += NT) s += dw[j] * dw[j];
         s = block_sum<NT>(s, red);
@@ -1065,16 +1070,19 @@ extern "C" int li_latent_norm_pairs_store(const float* q, long q_stride, int nh,
     if ((nh > 0 && (!q || !qfull || q_stride < (long)nh * (dn + dr))) || (store && (!down || !cache || !slot_map || down_stride < rank + dr)) ||
         (q_rank > 0 && (!ql || !wq || !cq || ql_stride < q_rank)))
         return LI_ERR_SIZE;
-#define LI_LN(T_, TQ_)                                                                                                          \
-    latent_norm_pairs_store_kernel<T_, TQ_, 256><<<T, 256, 0, stream>>>(q, q_stride, nh, dn, dr, down, down_stride, rank, wc, eps, \
+    const bool held = q_rank > 0 && q_rank <= LN_HELD * 256 && rank <= LN_HELD * 256;
+#define LI_LNH(T_, TQ_, HELD)                                                                                                   \
+    latent_norm_pairs_store_kernel<T_, TQ_, 256, HELD><<<T, 256, 0, stream>>>(q, q_stride, nh, dn, dr, down, down_stride, rank, wc, eps, \
                                                                         cosv, sinv, slot_map, (T_*)cache, qfull, store, split, ql, \
                                                                         ql_stride, q_rank, wq, (TQ_*)cq)
-    if (cache_dtype == LI_F32 && cq_dtype == LI_F32) LI_LN(float, float);
-    else if (cache_dtype == LI_BF16 && cq_dtype == LI_BF16) LI_LN(bf16_t, bf16_t);
-    else if (cache_dtype == LI_F32 && cq_dtype == LI_BF16) LI_LN(float, bf16_t);
-    else if (cache_dtype == LI_BF16 && cq_dtype == LI_F32) LI_LN(bf16_t, float);
+#define LI_LN(T_, TQ_) { if (held) LI_LNH(T_, TQ_, true); else LI_LNH(T_, TQ_, false); }
+    if (cache_dtype == LI_F32 && cq_dtype == LI_F32) LI_LN(float, float)
+    else if (cache_dtype == LI_BF16 && cq_dtype == LI_BF16) LI_LN(bf16_t, bf16_t)
+    else if (cache_dtype == LI_F32 && cq_dtype == LI_BF16) LI_LN(float, bf16_t)
+    else if (cache_dtype == LI_BF16 && cq_dtype == LI_F32) LI_LN(bf16_t, float)
     else return LI_ERR_DTYPE;
 #undef LI_LN
+#undef LI_LNH
     return li_launch_status();
 }
 
