@@ -1505,29 +1505,36 @@ def _seg_of_token(meta, takes: bool = True) -> int:
     return 0 if in_order else meta.seg_of_token.data_ptr()
 
 
-def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int):
+def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, aligned: bool = True):
     """Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of
     four runs a (token, kv head), which joins them itself and needs no list of runs; a pair of least lengths, runs of their own and the
-    kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan.
+    kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan; `aligned`: no window and
+    pages of a multiple of 8 keys (the kernel's quicker form).
     A run of 32 keys is a step, whose instructions (bfloat16, 0.9 us) or matrix products (float32, 1.8 us: six heads in tiles of 16) are
     what it takes, and the second kernel with its trips to memory is 3 us.  Us a call, before / now:
     bfloat16, beside portions, whose tables are as wide as they must be: 12 heads on 2 of 128, a table of 208 keys, 1 / 64 / 128 requests
     8.3 / 10.0 / 13.2 -> 6.4 / 7.3 / 8.9; contexts of 30 to 300, 64 / 128 requests 11.0 / 15.2 -> 8.4 / 9.5, 3 requests 7.7 / 7.5; of 50 to 500, 3
-    requests 8.3 / 9.6 (so not there), 64 12.7 / 10.7; of 100 to 1,000, 16 / 64 / 128 requests 10.1 / 14.0, 16.7 / 16.0, 25.4 / 20.0.  Few requests of
+    requests 8.3 / 9.6 (so not there), 64 12.7 / 10.7; of 44 to 352, 50 to 400 and 56 to 448, 3 requests 8.2 / 7.8, 8.4 / 8.5, 8.4 / 8.8, 28 heads on 4, 8 requests 9.1 / 8.4,
+    8.8 / 9.3, 9.1 / 9.5 (heads of 128 therefore up to 384, of 64, 14 on 2, 8 requests of 100 to 440 8.1 / 6.6); of 100 to 1,000, 16 / 64 / 128 requests 10.1 / 14.0, 16.7 / 16.0, 25.4 / 20.0.  Few requests of
     heads of 128, tables of 592 / 704 / 832 keys: the four runs of a block 9.3 / 9.9 / 11.1 (1 request), 9.8 / 10.3 / 11.3 (16), runs of 64 keys and more
     8.1 / 8.1 / 8.3, 9.1 / 9.4 / 9.7 (496 keys, 8 kv heads: 7.7 / 7.9, so not there).  Recorded steps, whose tables are 256, 512 or 1,024 keys wide, contexts of
     three quarters of that / spread from a tenth of it on: 14 heads on 2 of 64, 1 request 8.1 -> 5.2 at 256, 64 requests 9.7 / 10.0 -> 6.0 / 6.2, 6.8 /
     10.9 -> 7.0 / 7.6, 11.7 / 13.1 -> 9.7 / 10.4; 12 on 2 of 128, 1 request 8.3 -> 6.6 at 256, 64 requests 10.0 / 10.9 -> 7.7 / 8.1, 9.3 / 12.6 -> 9.4 / 10.1,
-    15.7 / 16.1 -> 15.7 / 14.6.
+    15.7 / 16.1 -> 15.7 / 14.6.  Pages of 12 keys: 16 heads on 16 of 64, 8 requests of 105 to 840 11.4 / 11.0, of 153 to 1,224 12.1 / 14.6, 12 on 2 of 128, 64 of 1,224
+    21.1 / 22.0 (so up to 896).
     float32, tables and contexts likewise: 12 heads on 2 of 128, 1 request 13.5, 15.4, 13.9 -> 8.7, 11.1, 11.9, 16 requests 14.3 / 12.6, 16.5 / 12.9, 15.5 / 14.6 -> 9.5 /
     10.3, 12.4 / 11.4, 14.1 / 13.8; 14 on 2 of 64, 1 request 10.7, 8.6 (its whole table 10.4), 11.0 -> 7.8, 9.1 (9.2), 9.6, 16 requests 10.6 / 10.2, 9.2 / 10.8,
     11.7 / 11.8 -> 7.7 / 9.0, 9.8 / 9.9, 11.1 / 12.2.  Not beyond 1,024 keys (2,048, 8 requests: 15.9 / 15.1 against 16.3 / 15.4, heads of 64 12.2 / 12.6 against
-    12.6 / 14.3; 1 request 14.6 / 15.0).  32 requests: 128 columns at 832 keys 25.2 / 16.1 -> 17.4 / 15.5, at 1,024 20.4 / 18.3 against 19.2 / 20.6; 64 columns at 304 keys
+    12.6 / 14.3; 1 request 14.6 / 15.0).  A table of 256 keys is also that of every shorter context: 58 keys in one run / in runs of 32 / in a block of four 7.5 / 8.1 /
+    5.5 (heads of 64), 8.6 / 9.0 / 7.1, 100 keys 9.0 / 8.2 / 6.0, 11.1 / 9.0 / 8.4, 192 10.7 / 7.8 / 7.2, 13.5 / 8.7 / 10.9; behind a window of 128 58 keys 6.1 / 7.7, 8.5 / 8.7, at 112 keys
+    7.2 / 7.5 / 5.3, 10.4 / 8.5 / 7.6: the block for heads of 64 up to 256 keys and for heads of 128 up to 128.  32 requests: 128 columns at 832 keys 25.2 / 16.1 -> 17.4 / 15.5, at 1,024 20.4 / 18.3 against 19.2 / 20.6; 64 columns at 304 keys
     12.0 / 11.8 -> 9.9 / 10.3, at 400 9.2 / 11.8 against 10.4 / 10.6, at 512 9.5 / 11.9 against 11.3 / 11.4.  Up to 96 keys one run is the faster (7.8 / 8.5)."""
     if dtype is torch.bfloat16:
-        if 128 < keys <= min(max(448, 10 * pairs), 1280):
+        if 128 < keys <= min(max(384 if dh == 128 else 448, 10 * pairs), 1280 if aligned else 896):
             return DECODE_QUAD
         return (64,) if dh == 128 and quads == DECODE_QUAD and 512 < keys <= 1024 and pairs <= 32 else None
+    if 96 < keys <= (128 if dh == 128 else 256) and pairs <= 64:
+        return DECODE_QUAD
     most = 1024 if pairs <= 32 else 0 if pairs > 64 else 1023 if dh == 128 else 320
     return (32, 64) if 96 < keys <= most else None
 
@@ -1665,7 +1672,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
                 quad = 1
                 planned = decode_splits(n_single * nkv, keys, simds, quad)
                 nsplit = _ragged_splits(planned, meta, window, quad)
-            runs = None if _decode_single_waves else _short_runs(n_single * nkv, keys, dh, qkv.dtype, nsplit if quad > 1 else 0)
+            runs = None if _decode_single_waves else _short_runs(
+                n_single * nkv, keys, dh, qkv.dtype, nsplit if quad > 1 else 0, window <= 0 and page_size % 8 == 0)
             if runs == DECODE_QUAD:
                 quad = nsplit = planned = DECODE_QUAD
             elif runs is not None:

@@ -177,8 +177,17 @@ def test_products_are_cut_into_no_more_parts_than_are_added_up():
     assert most[True] == ops.SPLITK_MAX_PARTS == 16 and most[False] == 8
 
 
-@pytest.mark.parametrize("pairs,dh,ends", [(2, 64, 1024), (32, 64, 1024), (32, 128, 1024), (33, 64, 320), (64, 128, 1008), (64, 64, 320), (65, 128, 0)])
-def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh, ends):
-    """Beyond these widths runs of 32 keys and the kernel that joins them took longer than the ordinary cut."""
+@pytest.mark.parametrize("pairs,dh,block,ends", [(2, 64, 256, 1024), (32, 64, 256, 1024), (32, 128, 128, 1024), (33, 64, 256, 320), (64, 128, 128, 1008),
+                                                 (65, 128, 0, 0), (65, 64, 0, 0)])
+def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh, block, ends):
+    """One block of four runs, then runs of 32 keys and the kernel that joins them; beyond, the ordinary cut was the faster."""
     for keys in range(16, 8192, 16):
-        assert (ops._short_runs(pairs, keys, dh, ops.torch.float32, 4) is not None) == (96 < keys <= ends), keys
+        want = None if keys <= 96 or keys > ends else ops.DECODE_QUAD if keys <= block else (32, 64)
+        assert ops._short_runs(pairs, keys, dh, ops.torch.float32, 4) == want, keys
+
+
+@pytest.mark.parametrize("pairs,dh,aligned,ends", [(2, 128, True, 384), (32, 128, False, 384), (2, 64, True, 448), (64, 128, True, 640), (512, 64, True, 1280),
+                                                   (512, 128, False, 896)])
+def test_bfloat16_decoding_takes_one_block_only_where_that_was_measured(pairs, dh, aligned, ends):
+    for keys in range(16, 8192, 16):
+        assert (ops._short_runs(pairs, keys, dh, ops.torch.bfloat16, 0, aligned) == ops.DECODE_QUAD) == (128 < keys <= ends), keys
