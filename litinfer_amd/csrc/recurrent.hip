@@ -1157,6 +1157,19 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
     float* st = state + ((size_t)slot * heads + head) * N * vdim;
     const float* src = chunk_seg ? carry + ((size_t)bx * heads + head) * N * vdim : st;
     float S[NR][CW];
+    if constexpr (ONE && CW == 4) {
+        if (active) {                                   // (one head a group leaves waves idle: they read nothing)
+#pragma unroll
+            for (int r = 0; r < NR; ++r) {
+                const int n = s * NR + r;
+                const float4 v4 = *reinterpret_cast<const float4*>(src + (size_t)(n < N ? n : N - 1) * vdim + (p < vdim ? p : 0));
+                S[r][0] = v4.x; S[r][1] = v4.y; S[r][2] = v4.z; S[r][3] = v4.w;
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < NR; ++r) S[r][0] = S[r][1] = S[r][2] = S[r][3] = 0.f;
+        }
+    } else
 #pragma unroll
     for (int r = 0; r < NR; ++r) {
         const int n = s * NR + r;
@@ -1164,9 +1177,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
 #pragma unroll
             for (int cc = 0; cc < CW; ++cc) S[r][cc] = (is_p && n == p + cc) ? 1.f : 0.f;
         } else if constexpr (CW == 4) {
-            float4 v4;
-            if constexpr (ONE) v4 = *reinterpret_cast<const float4*>(src + (size_t)(n < N ? n : N - 1) * vdim + (p < vdim ? p : 0));
-            else v4 = (active && n < N && p < vdim) ? *reinterpret_cast<const float4*>(src + (size_t)n * vdim + p) : float4{0.f, 0.f, 0.f, 0.f};
+            const float4 v4 = (active && n < N && p < vdim) ? *reinterpret_cast<const float4*>(src + (size_t)n * vdim + p) : float4{0.f, 0.f, 0.f, 0.f};
             S[r][0] = v4.x; S[r][1] = v4.y; S[r][2] = v4.z; S[r][3] = v4.w;
         } else {
 #pragma unroll
@@ -1197,7 +1208,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
     if constexpr (ONE && CW == 4) {
 #pragma unroll
         for (int r = 0; r < NR; ++r)
-            if (!(active && s * NR + r < N && p < vdim)) S[r][0] = S[r][1] = S[r][2] = S[r][3] = 0.f;
+            if (!(s * NR + r < N && p < vdim)) S[r][0] = S[r][1] = S[r][2] = S[r][3] = 0.f;
     }
     for (int b0 = 0; b0 < ntok; b0 += DR_TB) {
         __syncthreads();
