@@ -1505,11 +1505,11 @@ def _seg_of_token(meta, takes: bool = True) -> int:
     return 0 if in_order else meta.seg_of_token.data_ptr()
 
 
-def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, aligned: bool = True):
+def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, aligned: bool = True, differ: bool = True):
     """Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of
     four runs a (token, kv head), which joins them itself and needs no list of runs; a pair of least lengths, runs of their own and the
     kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan; `aligned`: no window and
-    pages of a multiple of 8 keys (the kernel's quicker form).
+    pages of a multiple of 8 keys (the kernel's quicker form); `differ`: the contexts do, by `_ragged_splits`.
     A run of 32 keys is a step, whose instructions (bfloat16, 0.9 us) or matrix products (float32, 1.8 us: six heads in tiles of 16) are
     what it takes, and the second kernel with its trips to memory is 3 us.  Us a call, before / now:
     bfloat16, beside portions, whose tables are as wide as they must be: 12 heads on 2 of 128, a table of 208 keys, 1 / 64 / 128 requests
@@ -1521,7 +1521,9 @@ def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, 
     three quarters of that / spread from a tenth of it on: 14 heads on 2 of 64, 1 request 8.1 -> 5.2 at 256, 64 requests 9.7 / 10.0 -> 6.0 / 6.2, 6.8 /
     10.9 -> 7.0 / 7.6, 11.7 / 13.1 -> 9.7 / 10.4; 12 on 2 of 128, 1 request 8.3 -> 6.6 at 256, 64 requests 10.0 / 10.9 -> 7.7 / 8.1, 9.3 / 12.6 -> 9.4 / 10.1,
     15.7 / 16.1 -> 15.7 / 14.6.  Pages of 12 keys: 16 heads on 16 of 64, 8 requests of 105 to 840 11.4 / 11.0, of 153 to 1,224 12.1 / 14.6, 12 on 2 of 128, 64 of 1,224
-    21.1 / 22.0 (so up to 896).
+    21.1 / 22.0 (so up to 896).  More than 512 pairs are two waves a SIMD as they are: equal contexts of 144 / 256 keys, 16 heads on 16 of 64, 36 requests 0.88 / 0.94 times as
+    fast in blocks, 64 requests 9.2 / 11.7, 13.6 / 14.7 us, 28 on 4 of 128, 144 requests 0.68 / 0.82; contexts that differ 1.2 to 2.4 times (heads of 128, 2,048 and 4,096 pairs
+    under 256 keys 0.94 to 1.06).  576 and 640 pairs of equal contexts of 352 keys 1.06 to 1.6, 704 0.89 to 1.02.
     float32, tables and contexts likewise: 12 heads on 2 of 128, 1 request 13.5, 15.4, 13.9 -> 8.7, 11.1, 11.9, 16 requests 14.3 / 12.6, 16.5 / 12.9, 15.5 / 14.6 -> 9.5 /
     10.3, 12.4 / 11.4, 14.1 / 13.8; 14 on 2 of 64, 1 request 10.7, 8.6 (its whole table 10.4), 11.0 -> 7.8, 9.1 (9.2), 9.6, 16 requests 10.6 / 10.2, 9.2 / 10.8,
     11.7 / 11.8 -> 7.7 / 9.0, 9.8 / 9.9, 11.1 / 12.2.  Not beyond 1,024 keys (2,048, 8 requests: 15.9 / 15.1 against 16.3 / 15.4, heads of 64 12.2 / 12.6 against
@@ -1530,7 +1532,13 @@ def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, 
     7.2 / 7.5 / 5.3, 10.4 / 8.5 / 7.6: the block for heads of 64 up to 256 keys and for heads of 128 up to 128.  32 requests: 128 columns at 832 keys 25.2 / 16.1 -> 17.4 / 15.5, at 1,024 20.4 / 18.3 against 19.2 / 20.6; 64 columns at 304 keys
     12.0 / 11.8 -> 9.9 / 10.3, at 400 9.2 / 11.8 against 10.4 / 10.6, at 512 9.5 / 11.9 against 11.3 / 11.4.  Up to 96 keys one run is the faster (7.8 / 8.5)."""
     if dtype is torch.bfloat16:
-        if 128 < keys <= min(max(384 if dh == 128 else 448, 10 * pairs), 1280 if aligned else 896):
+        if pairs <= 512:
+            blocks = True
+        elif differ:
+            blocks = dh != 128 or pairs < 2048 or keys >= 256
+        else:
+            blocks = pairs <= 640 and keys > 320
+        if blocks and 128 < keys <= min(max(384 if dh == 128 else 448, 10 * pairs), 1280 if aligned else 896):
             return DECODE_QUAD
         return (64,) if dh == 128 and quads == DECODE_QUAD and 512 < keys <= 1024 and pairs <= 32 else None
     if 96 < keys <= (128 if dh == 128 else 256) and pairs <= 64:
@@ -1673,7 +1681,8 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
                 planned = decode_splits(n_single * nkv, keys, simds, quad)
                 nsplit = _ragged_splits(planned, meta, window, quad)
             runs = None if _decode_single_waves else _short_runs(
-                n_single * nkv, keys, dh, qkv.dtype, nsplit if quad > 1 else 0, window <= 0 and page_size % 8 == 0)
+                n_single * nkv, keys, dh, qkv.dtype, nsplit if quad > 1 else 0, window <= 0 and page_size % 8 == 0,
+                nsplit > planned)
             if runs == DECODE_QUAD:
                 quad = nsplit = planned = DECODE_QUAD
             elif runs is not None:

@@ -191,3 +191,10 @@ def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh,
 def test_bfloat16_decoding_takes_one_block_only_where_that_was_measured(pairs, dh, aligned, ends):
     for keys in range(16, 8192, 16):
         assert (ops._short_runs(pairs, keys, dh, ops.torch.bfloat16, 0, aligned) == ops.DECODE_QUAD) == (128 < keys <= ends), keys
+
+
+@pytest.mark.parametrize("pairs,dh,differ,begins,ends", [(512, 64, False, 128, 1280), (513, 64, True, 128, 1280), (513, 64, False, 320, 1280), (640, 128, False, 320, 1280),
+                                                         (641, 64, False, 0, 0), (2047, 128, True, 128, 1280), (2048, 128, True, 255, 1280), (2048, 64, True, 128, 1280)])
+def test_many_equal_contexts_are_not_decoded_in_blocks(pairs, dh, differ, begins, ends):
+    for keys in range(1, 4096):
+        assert (ops._short_runs(pairs, keys, dh, ops.torch.bfloat16, 0, True, differ) == ops.DECODE_QUAD) == (begins < keys <= ends), keys
