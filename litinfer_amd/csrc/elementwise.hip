@@ -680,14 +680,15 @@ extern "C" int li_rope_pairs_apply(void* x, int dtype, int row_stride, int n_hea
 // norms the WHOLE query projection and the WHOLE key projection (all heads at once, before they are split) and
 // rotates pairs of columns (neighbours, or with half_split column i and column i + rotary_dim / 2): q is normed and rotated in place (it stays float32), k is normed, rotated and
 // written to its page slot, v is copied to its page slot.  wq / wk null: no norm.  One block a token.
-template <typename T, int NT, bool NORMED>
+enum QkForm { QK_PLAIN, QK_NORMED, QK_HELD };             // no norm; a norm; a norm over a row that the threads hold
+template <typename T, int NT, QkForm FORM>
 __global__ __launch_bounds__(NT) void qk_norm_pairs_store_kernel(
     float* __restrict__ qkv, int row_stride, int nh, int nkv, int dk, int dv, int rotary_dim,
     const float* __restrict__ wq, const float* __restrict__ wk, float eps,
     const float* __restrict__ cosv, const float* __restrict__ sinv, const int* __restrict__ slot_map,
     T* __restrict__ kc, T* __restrict__ vc, int page_size, int store, int half_split) {
     __shared__ float red[NT / LI_WAVE];
-    if constexpr (!NORMED) wq = wk = nullptr;
+    if constexpr (FORM == QK_PLAIN) wq = wk = nullptr;
     const int t = blockIdx.x, half = rotary_dim / 2;
     float* q = qkv + (size_t)t * row_stride;
     float* k = q + (size_t)nh * dk;
@@ -695,10 +696,11 @@ __global__ __launch_bounds__(NT) void qk_norm_pairs_store_kernel(
     const int nq = nh * dk, nk = nkv * dk;
     float inv_q = 1.f, inv_k = 1.f;
     const int units = half + (dk - rotary_dim);            // per head: the pairs, then the columns that are not rotated
-    if (NORMED && nh * units <= 2 * NT && nkv * units <= NT && nkv * dv <= NT) {
+    if constexpr (FORM == QK_HELD) {
         // A short row (a decoding step) with a norm: a thread holds two units of q, one of k and one of v with all that belongs to them, asked for
         // at once (sum after sum and part after part, each with its own trip to weights and angles: 8 tokens of 12 heads of 128 8.3 -> 3.8 us).
         // Without one the loops below are independent as they stand, and there is nothing to wait for (2.9 us, here 3.8; 28 heads 3.3, 4.0).
+        // An instance of its own: longer rows would pay for its registers (1,027 tokens of 28 heads on 4 of 192 20.3 / 22.6 us).
         __shared__ float red2[NT / LI_WAVE];
         struct Unit { int j, j2, i; bool on, pair; float a, b, wa, wb, c, s; } un[3];
         const int slot = store ? slot_map[t] : 0;
@@ -832,14 +834,17 @@ extern "C" int li_qk_norm_pairs_store(float* qkv, int row_stride, int nh, int nk
         return LI_ERR_SIZE;
     // few rows (a decoding step): 1024 threads a row, so that the one row is gone through with the least latency
     const bool wide = T < 256 && nh * dk > 1024;
-#define LI_QKN(TC, NT, NORMED)                                                                                                              \
-    qk_norm_pairs_store_kernel<TC, NT, NORMED><<<T, NT, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, cosv, sinv, \
+    const int units = dk - rotary_dim / 2, nt = wide ? 1024 : 256;
+    const bool held = (long)nh * units <= 2 * nt && (long)nkv * units <= nt && (long)nkv * dv <= nt;
+#define LI_QKN(TC, NT, FORM)                                                                                                                \
+    qk_norm_pairs_store_kernel<TC, NT, FORM><<<T, NT, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, cosv, sinv, \
                                                                      slot_map, (TC*)kc, (TC*)vc, page_size, store, half_split)
 #define LI_QK(TC)                                                                            \
     {                                                                                        \
-        if (wq || wk) { if (wide) LI_QKN(TC, 1024, true); else LI_QKN(TC, 256, true); }      \
-        else if (wide) LI_QKN(TC, 1024, false);                                              \
-        else LI_QKN(TC, 256, false);                                                         \
+        if (!wq && !wk) { if (wide) LI_QKN(TC, 1024, QK_PLAIN); else LI_QKN(TC, 256, QK_PLAIN); }   \
+        else if (held) { if (wide) LI_QKN(TC, 1024, QK_HELD); else LI_QKN(TC, 256, QK_HELD); }      \
+        else if (wide) LI_QKN(TC, 1024, QK_NORMED);                                                 \
+        else LI_QKN(TC, 256, QK_NORMED);                                                            \
     }
     if (cache_dtype == LI_F32) LI_QK(float)
     else if (cache_dtype == LI_BF16) LI_QK(bf16_t)
@@ -852,7 +857,7 @@ extern "C" int li_qk_norm_pairs_store(float* qkv, int row_stride, int nh, int nk
 // The same step for a mixer that norms every query head and every key head BY ITSELF, with one weight vector of dk
 // values for all query heads (wq) and one for all key heads (wk): rows [q | k | v], or, with keys_are_values, rows
 // [q | k], where the value of a token is its key as projected, before the norm.  A wave a (token, head).
-template <typename T>
+template <typename T, bool HELD>
 __global__ __launch_bounds__(256) void qk_head_norm_store_kernel(
     float* __restrict__ qkv, long row_stride, int nh, int nkv, int dk, int dv, int rotary_dim,
     const float* __restrict__ wq, const float* __restrict__ wk, float eps,
@@ -874,7 +879,7 @@ __global__ __launch_bounds__(256) void qk_head_norm_store_kernel(
     float* x = row + (size_t)unit * dk;                    // (the key heads lie behind the query heads)
     const float* w = is_q ? wq : wk;
     float ss = 0.f;
-    if (dk <= 2 * LI_WAVE && rotary_dim <= 2 * LI_WAVE && rotary_dim % 2 == 0) {
+    if constexpr (HELD) {
         // A lane holds its pair of rotated columns and its two other columns with their weights and angles, asked for at once (4.1 -> 3.1 us).
         const int hf = rotary_dim / 2, i0 = lane < hf ? lane : 0;
         const int d1 = half_split ? i0 : 2 * i0, d2 = half_split ? i0 + hf : 2 * i0 + 1, rest = dk - rotary_dim;
@@ -942,13 +947,13 @@ extern "C" int li_qk_head_norm_store(float* qkv, long row_stride, int nh, int nk
     const int units = nh + (store ? (keys_are_values ? nkv : 2 * nkv) : 0);
     if ((units + 3) / 4 > 65535) return LI_ERR_SIZE;
     const dim3 grid(T, (units + 3) / 4);
-    if (cache_dtype == LI_F32)
-        qk_head_norm_store_kernel<float><<<grid, 256, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, cosv, sinv,
-                                                                   slot_map, (float*)kc, (float*)vc, page_size, store, half_split, keys_are_values);
-    else if (cache_dtype == LI_BF16)
-        qk_head_norm_store_kernel<bf16_t><<<grid, 256, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, cosv, sinv,
-                                                                    slot_map, (bf16_t*)kc, (bf16_t*)vc, page_size, store, half_split, keys_are_values);
+#define LI_QKH(TC, HELD)                                                                                                              \
+    qk_head_norm_store_kernel<TC, HELD><<<grid, 256, 0, stream>>>(qkv, row_stride, nh, nkv, dk, dv, rotary_dim, wq, wk, eps, cosv, sinv, \
+                                                                  slot_map, (TC*)kc, (TC*)vc, page_size, store, half_split, keys_are_values)
+    if (cache_dtype == LI_F32) { if (dk <= 2 * LI_WAVE) LI_QKH(float, true); else LI_QKH(float, false); }
+    else if (cache_dtype == LI_BF16) { if (dk <= 2 * LI_WAVE) LI_QKH(bf16_t, true); else LI_QKH(bf16_t, false); }
     else return LI_ERR_DTYPE;
+#undef LI_QKH
     return li_launch_status();
 }
 
