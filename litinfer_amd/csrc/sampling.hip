@@ -214,8 +214,8 @@ __device__ __forceinline__ int block_min_int(int v, int* smem) {
 // wave the lanes halve what they hold step by step (a lane keeps one half of its sums and gets the
 // other lane's part of that half: 8 + 4 + 2 + 1 exchanges), until each lane holds one sum of its 16
 // lanes, then the four groups of 16 lanes are added: 17 exchanges instead of 96; then the waves in
-// their order.  The order of the additions is fixed.  work: SMP_WAVES * 16 values.
-template <typename T>
+// their order.  The order of the additions is fixed.  work: WAVES * 16 values.
+template <int WAVES, typename T>
 __device__ __forceinline__ void block_sum16(T (&c)[16], T* work, T* tot) {
     const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
 #define LI_HALVE(H, MASK)                                                         \
@@ -240,14 +240,14 @@ __device__ __forceinline__ void block_sum16(T (&c)[16], T* work, T* tot) {
     __syncthreads();
     if (threadIdx.x < 16) {
         T t = 0;
-        for (int i = 0; i < SMP_WAVES; ++i) t += work[i * 16 + threadIdx.x];
+        for (int i = 0; i < WAVES; ++i) t += work[i * 16 + threadIdx.x];
         tot[threadIdx.x] = t;
     }
     __syncthreads();
 }
 
-// Sum of v over the threads before this one, in thread order.  work: SMP_WAVES values.
-template <typename T>
+// Sum of v over the threads before this one, in thread order.  work: WAVES values.
+template <int WAVES = SMP_WAVES, typename T>
 __device__ __forceinline__ T block_sum_before(T v, T* work) {
     const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
     T inc = v;
@@ -263,20 +263,25 @@ __device__ __forceinline__ T block_sum_before(T v, T* work) {
     __syncthreads();
     T base = 0;
 #pragma unroll
-    for (int i = 0; i < SMP_WAVES; ++i) base += i < w ? work[i] : T(0);      // (all reads at once; adding a zero changes nothing)
+    for (int i = 0; i < WAVES; ++i) base += i < w ? work[i] : T(0);      // (all reads at once; adding a zero changes nothing)
     return base + before;
 }
 
-// A thread's 8 ids of a tile as z = logit / T (whole 16-byte loads where the row allows them)
-__device__ __forceinline__ void load_ids8(const float* __restrict__ row, int j0, int V, float T, bool vec, float (&z)[8]) {
+// A thread's 8 ids of a tile (whole 16-byte loads where the row allows them): the logits; and z = logit / T
+__device__ __forceinline__ void load_ids8(const float* __restrict__ row, int j0, int V, bool vec, float (&x)[8]) {
     if (vec && j0 + 8 <= V) {
         const float4 a = *reinterpret_cast<const float4*>(row + j0), b = *reinterpret_cast<const float4*>(row + j0 + 4);
-        z[0] = a.x / T; z[1] = a.y / T; z[2] = a.z / T; z[3] = a.w / T;
-        z[4] = b.x / T; z[5] = b.y / T; z[6] = b.z / T; z[7] = b.w / T;
+        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+        x[4] = b.x; x[5] = b.y; x[6] = b.z; x[7] = b.w;
     } else {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) z[e] = (j0 + e < V) ? row[j0 + e] / T : -INFINITY;
+        for (int e = 0; e < 8; ++e) x[e] = (j0 + e < V) ? row[j0 + e] : -INFINITY;
     }
+}
+__device__ __forceinline__ void load_ids8(const float* __restrict__ row, int j0, int V, float T, bool vec, float (&z)[8]) {
+    load_ids8(row, j0, V, vec, z);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) z[e] /= T;
 }
 
 // f(z, id) for this thread's ids of all tiles, ascending
@@ -296,7 +301,7 @@ __device__ __forceinline__ void each_id(const float* __restrict__ row, int V, fl
 // tau = the kk-th largest key among the z that `each` hands out (to all threads of the block together),
 // need (>= 1) = how many of the keys equal to tau are among the kk largest.  Four bits a pass: counts of
 // the 16 values of the next digit among the keys that agree with the digits found so far.
-template <typename Each>
+template <int WAVES = SMP_WAVES, typename Each>
 __device__ __forceinline__ void radix_kth(Each&& each, int kk, uint32_t& tau, int& need, int* work_i, int* tot_i) {
     tau = 0u;
     for (int shift = 28; shift >= 0; shift -= 4) {
@@ -311,7 +316,7 @@ __device__ __forceinline__ void radix_kth(Each&& each, int kk, uint32_t& tau, in
                 for (int b = 0; b < 16; ++b) cnt[b] += (d == b);
             }
         });
-        block_sum16(cnt, work_i, tot_i);
+        block_sum16<WAVES>(cnt, work_i, tot_i);
         int above = 0, d = 15;
         for (; d > 0; --d) {
             if (above + tot_i[d] >= kk) break;
@@ -333,7 +338,8 @@ __device__ __forceinline__ void radix_kth(Each&& each, int kk, uint32_t& tau, in
 // bound leaves fewer than kk keys (a wave without enough of them sets none) or more than SMP_LIST (many equal logits):
 // radix_kth then.
 // 64 rows of 151,936 ids, top-k 50: tiles kernel 58 -> 45 us (one row 26 -> 13), rows kernel 22 -> 14.  Both are shorter since a tile hands
-// over all that it listed (below): top-k with top-p 44 + 25 -> 24 + 19.
+// over all that it listed (below; top-k with top-p 44 + 25 -> 24 + 19), and by tile_bound and rows_by_list (11 + 10).  What is left for this function is rows
+// whose tiles hand over exactly kc ids, and those that rows_by_list leaves.
 constexpr int SMP_LIST = 1024;
 // the bound, as above (0: none): at least kk of the block's keys are no smaller
 __device__ __forceinline__ uint32_t bound_of_kth(const uint32_t (&key)[8], int kk, int waves, int* work_i) {
@@ -372,12 +378,13 @@ __device__ __forceinline__ void put_from(const uint32_t (&key)[8], uint32_t boun
         if (key[e] >= bound) put(pos++, e);
 }
 // n keys in the list (n at least kk): tau and need
+template <int NT = SMP_NT>
 __device__ __forceinline__ void kth_of_list(uint32_t* list, int n, int kk, uint32_t& tau, int& need, int* res) {
     const int tid = threadIdx.x;
     if (tid < 4 && n + tid < SMP_LIST) list[n + tid] = 0u;      // (whole pieces of four below)
     __syncthreads();
-    if (tid < n) {
-        const uint32_t own = list[tid];
+    for (int i = tid; i < n; i += NT) {
+        const uint32_t own = list[i];
         int above = 0, from = 0;
 #pragma unroll 8
         for (int j = 0; j < n; j += 4) {
@@ -485,7 +492,7 @@ __device__ __forceinline__ void radix_mass(Each&& each, bool cut, uint32_t tau, 
                 for (int b = 0; b < 16; ++b) mass[b] += (d == b) ? e : 0.f;
             }
         });
-        block_sum16(mass, work_f, tot_f);
+        block_sum16<SMP_WAVES>(mass, work_f, tot_f);
         const bool ties_here = cut && ties > 0 && (shift == 28 || (tau >> (shift + 4)) == (tp >> (shift + 4)));
         const int d_ties = (tau >> shift) & 15;
         float above = 0.f;
@@ -551,105 +558,547 @@ __device__ __forceinline__ bool sample_wide(int k, int V, int rows, int ntiles) 
     return ntiles * SMP_KC <= SMP_NT * SMP_CAND_PER_THREAD && ((k > 0 && k < V) || rows * ntiles > SMP_WIDE_TILES);
 }
 
-// (eight waves a SIMD, two blocks a compute unit: with the 71 registers that the compiler would take, one block, 64 greedy rows took
-// 18 us instead of 13)
-__global__ __launch_bounds__(SMP_NT, 8) void sample_tiles_kernel(
+// ---- the first kernel.  A wave takes STEPS stretches of 512 ids that follow each other, a lane 8 neighbouring ids of each (two 16-byte
+// loads): a block of 1,024 threads with one stretch a wave for few tiles, where the time is one block's, and of 256 threads with four where
+// the tiles are many (TILE_MANY): 64 rows of 151,936 ids are 9.7 million values, 6.3 us at 6 TB/s, and four instructions a value are a
+// microsecond of the vector ALU's, so what is done once a thread (reductions over the block, barriers, scans) is spread over 32
+// values there.  What is done a value is little: quotients are only worked out where the tile's mass is asked for, by five
+// instructions; the largest ids are found among the logits themselves, whose order division by T keeps.
+// 64 rows of 151,936 ids, us, with blocks of 1,024 threads and every value divided first, and now: greedy 11.6 / 7.2, at a temperature 12.9 / 11.0,
+// top-k 50 with top-p 0.9 22.2 / 10.9, a third each 18.4 / 10.4.  One stretch a wave below 768 tiles: at a temperature alone a thread's 32
+// exponentials one behind the other are the longer time there (32 rows, 608 tiles, both kernels: 15.7 against 17.8, before 17.5; 48 rows 18.1 / 18.8, before
+// 19.9), while the other rows gain at any number (16 rows with top-k 19.0 / 17.1, before 25.4).
+constexpr int TILE_STRETCH = 8 * LI_WAVE;
+constexpr size_t TILE_MANY = 768;           // (rows x tiles)
+template <int STEPS> constexpr int TILE_NT = SMP_NT / STEPS;
+template <int STEPS> constexpr int TILE_WAVES = SMP_WAVES / STEPS;
+
+// x / T, correctly rounded (the same bits as the division) for T and x between 2^-40 and 2^40 in size, y = 1 / T rounded: the first
+// quotient is off by less than two units of its last place, the second by hardly more than half of one, so that its remainder is
+// exact, and by Markstein's theorem the third is the rounded quotient.  Five instructions; the division, which also serves
+// the ends of the range, is twelve.
+__device__ __forceinline__ float quotient(float x, float T, float y) {
+    const float q0 = x * y, q1 = fmaf(fmaf(-q0, T, x), y, q0);
+    return fmaf(fmaf(-q1, T, x), y, q1);
+}
+
+// The sums over the wave of a value each stretch, to smem[stretch] (numbered over the block), in the lanes' order of wave_sum.  Four at once:
+// with two values in a swap's operands one half of its result is the one's sums over the lanes l and l ^ 32, the other half the
+// other's, and so on, so that each row of 16 lanes is left with one value (the same sums, the same bits).
+__device__ __forceinline__ void tile_sums(const float (&v)[1], float* smem) {
+    const float s = wave_sum(v[0]);
+    if ((threadIdx.x & (LI_WAVE - 1)) == 0) smem[threadIdx.x / LI_WAVE] = s;
+}
+__device__ __forceinline__ void tile_sums(const float (&v)[4], float* smem) {
+    auto two = [](float a, float b, auto swap) {
+        const auto r = swap(__float_as_uint(a), __float_as_uint(b));
+        return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    };
+    auto halves = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane32_swap(a, b, false, false); };
+    auto rows = [](uint32_t a, uint32_t b) { return __builtin_amdgcn_permlane16_swap(a, b, false, false); };
+    // lanes 0..31 of the first hold v[0], 32..63 v[1]; of the second v[2] and v[3]; then rows 0, 1, 2, 3 of lanes: v[0], v[2], v[1], v[3]
+    float s = two(two(v[0], v[1], halves), two(v[2], v[3], halves), rows);
+    s += __int_as_float(dpp_mov<0x128>(__float_as_int(s)));
+    s += __int_as_float(dpp_mov<0x124>(__float_as_int(s)));
+    s += __int_as_float(dpp_mov<0x122>(__float_as_int(s)));
+    s += __int_as_float(dpp_mov<0x121>(__float_as_int(s)));
+    const int lane = threadIdx.x & (LI_WAVE - 1), row = lane >> 4;
+    if ((lane & 15) == 0) smem[4 * (threadIdx.x / LI_WAVE) + 2 * (row & 1) + (row >> 1)] = s;
+}
+
+// In the order of ids (wave, stretch, lane): how many of the block's n[c] lie before each of this thread's stretches; the block's number.
+// work: a value a wave.
+template <int STEPS>
+__device__ __forceinline__ int tile_places(const int (&n)[STEPS], int (&place)[STEPS], int* work) {
+    static_assert(STEPS == 1 || STEPS == 4, "one count, or two in each of two words (512 at most a stretch and wave)");
+    const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
+    uint32_t a = (uint32_t)n[0], b = 0u;
+    if constexpr (STEPS == 4) { a |= (uint32_t)n[1] << 16; b = (uint32_t)n[2] | (uint32_t)n[3] << 16; }
+    const uint32_t a0 = a, b0 = b;
+#pragma unroll
+    for (int o = 1; o < LI_WAVE; o <<= 1) {
+        const uint32_t ta = __shfl_up(a, o, LI_WAVE), tb = STEPS == 4 ? __shfl_up(b, o, LI_WAVE) : 0u;
+        if (lane >= o) { a += ta; b += tb; }
+    }
+    const uint32_t wa = __shfl(a, LI_WAVE - 1, LI_WAVE), wb = STEPS == 4 ? __shfl(b, LI_WAVE - 1, LI_WAVE) : 0u;
+    __syncthreads();
+    if (lane == 0) work[w] = (int)((wa & 0xffff) + (wa >> 16) + (wb & 0xffff) + (wb >> 16));
+    __syncthreads();
+    int base = 0, total = 0;
+#pragma unroll
+    for (int i = 0; i < TILE_WAVES<STEPS>; ++i) { const int t = work[i]; base += i < w ? t : 0; total += t; }
+    a -= a0;
+    b -= b0;
+    place[0] = base + (int)(a & 0xffff);
+    if constexpr (STEPS == 4) {
+        base += wa & 0xffff;
+        place[1] = base + (int)(a >> 16);
+        base += wa >> 16;
+        place[2] = base + (int)(b & 0xffff);
+        base += wb & 0xffff;
+        place[3] = base + (int)(b >> 16);
+    }
+    return total;
+}
+
+// the rounds-th largest of the wave's keys, bit by bit from the highest down to bit LAST (a bound; 0: the wave has fewer)
+template <int LAST>
+__device__ __forceinline__ uint32_t wave_bound(uint32_t key, int rounds) {
+    uint32_t largest = 0u;
+#pragma unroll
+    for (int b = 31; b >= LAST; --b) {
+        const uint32_t trial = largest | (1u << b);
+        if (__popcll((unsigned long long)__ballot(key >= trial)) >= rounds) largest = trial;
+    }
+    return largest;
+}
+// A key (sort_key) that at least kk of the tile's values are no smaller than (0: none found): as bound_of_kth, from the largest values of
+// the lanes' stretches; where a wave has four and few are asked of it, from the lanes' largest of all four (8,192 normal logits, kk = 50: some 75 values
+// from that bound on; from those of the stretches 150).  Only whole stretches (waves) count.  top[c]: the lane's largest value of stretch c.
+template <int STEPS>
+__device__ __forceinline__ uint32_t tile_bound(const float (&top)[STEPS], int kk, int in_tile, int* work) {
+    const int lane = threadIdx.x & (LI_WAVE - 1), w = threadIdx.x / LI_WAVE;
+    __syncthreads();                                 // (work has been read)
+    const int waves = in_tile / (STEPS * TILE_STRETCH);
+    const bool by_wave = STEPS > 1 && waves > 0 && (kk + waves - 1) / waves <= 24;
+    int parts = max(in_tile / TILE_STRETCH, 1);
+    if (by_wave) {
+        float all = top[0];
+#pragma unroll
+        for (int c = 1; c < STEPS; ++c) all = fmaxf(all, top[c]);
+        const uint32_t largest = wave_bound<14>(sort_key(all), (kk + waves - 1) / waves);
+        if (lane == 0) work[w] = (int)largest;
+        parts = waves;
+    } else {
+        const int rounds = (kk + parts - 1) / parts;
+        if (rounds > LI_WAVE) return 0u;
+#pragma unroll
+        for (int c = 0; c < STEPS; ++c) {
+            const uint32_t largest = wave_bound<16>(sort_key(top[c]), rounds);
+            if (lane == 0) work[STEPS * w + c] = (int)largest;
+        }
+    }
+    __syncthreads();
+    uint32_t bound = 0xffffffffu;
+#pragma unroll
+    for (int i = 0; i < SMP_WAVES; ++i) bound = i < parts ? min(bound, (uint32_t)work[i] - 1u) : bound;      // (0, no bound, becomes the largest)
+    return bound + 1u;
+}
+
+template <int STEPS>
+__global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_tiles_kernel(
     const float* __restrict__ logits, const float* __restrict__ temperature, const int* __restrict__ top_k,
     const float* __restrict__ top_p, float* __restrict__ tile_m, float* __restrict__ tile_s,
     int* __restrict__ tile_i, float* __restrict__ cand_z, int* __restrict__ cand_id, int V) {
+    constexpr int NT = TILE_NT<STEPS>, WAVES = TILE_WAVES<STEPS>, ITEMS = SMP_LIST / NT;
     __shared__ float sf[SMP_WAVES];
     __shared__ int si[SMP_WAVES];
-    __shared__ int work_i[SMP_WAVES * 16], tot_i[16];
+    __shared__ int work_i[WAVES * 16], tot_i[16];
     __shared__ __align__(16) uint32_t list[SMP_LIST];
+    __shared__ int list_id[SMP_LIST];
     const int tile = blockIdx.x, ntiles = gridDim.x, r = blockIdx.y, tid = threadIdx.x;
+    const int lane = tid & (LI_WAVE - 1), w = tid / LI_WAVE;
     const float* row = logits + (size_t)r * V;
-    const float T = temperature[r];
-    const int j0 = tile * SMP_TILE + tid * 8;
+    const int j0 = tile * SMP_TILE + w * STEPS * TILE_STRETCH + lane * 8;
     const size_t slot = (size_t)r * ntiles + tile;
-    if (!(T > 0.f)) {                                          // greedy: the tile's (maximum, lowest index)
-        float v = -INFINITY, x[8];
-        int i = 0x7fffffff;
-        load_ids8(row, j0, V, 1.0f, (reinterpret_cast<uintptr_t>(row) & 15) == 0, x);
+    const float T = temperature[r];
+    const int k = top_k[r];
+    const float p = top_p[r];
+    float x[STEPS][8];                                         // the logits; past the end -inf
+    const bool vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
 #pragma unroll
-        for (int e = 0; e < 8; ++e)
-            if (j0 + e < V && (x[e] > v || i == 0x7fffffff)) { v = x[e]; i = j0 + e; }
-        block_argmax(v, i, sf, si);
-        if (tid == 0) { tile_m[slot] = v; tile_i[slot] = i; }
+    for (int c = 0; c < STEPS; ++c) load_ids8(row, j0 + c * TILE_STRETCH, V, vec, x[c]);
+    if (!(T > 0.f)) {                                          // greedy: the tile's (maximum, lowest index)
+        float v = -INFINITY;
+        int i = 0x7fffffff;
+#pragma unroll
+        for (int c = 0; c < STEPS; ++c) {
+            const int j = j0 + c * TILE_STRETCH;
+            float vc = -INFINITY;
+            int ic = 0x7fffffff;
+#pragma unroll
+            for (int e = 0; e < 8; ++e)
+                if (j + e < V && (x[c][e] > vc || ic == 0x7fffffff)) { vc = x[c][e]; ic = j + e; }
+            argmax_combine(v, i, vc, ic);
+        }
+#pragma unroll
+        for (int o = LI_WAVE / 2; o > 0; o >>= 1) argmax_combine(v, i, lane_xor(v, o), lane_xor(i, o));
+        if (lane == 0) { sf[w] = v; si[w] = i; }
+        __syncthreads();
+        if (tid == 0) {
+#pragma unroll
+            for (int q = 1; q < WAVES; ++q) argmax_combine(v, i, sf[q], si[q]);
+            tile_m[slot] = v;
+            tile_i[slot] = i;
+        }
         return;
     }
-    float z[8], m = -INFINITY;
-    load_ids8(row, j0, V, T, (reinterpret_cast<uintptr_t>(row) & 15) == 0, z);
+    float top[STEPS], m;                                       // (the largest quotient is the largest logit's)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) m = fmaxf(m, z[e]);
-    m = block_max_f(m, sf);
-    const int k = top_k[r], kc = sample_candidates(k, top_p[r], V, ntiles);
-    if (kc == 0 || !(k > 0 && k < V)) {                        // (behind top-k nothing is taken of the whole row's mass)
-        float sum = 0.f;
+    for (int c = 0; c < STEPS; ++c) {
+        top[c] = x[c][0];
 #pragma unroll
-        for (int e = 0; e < 8; ++e) sum += (j0 + e < V && m > -INFINITY) ? expf(z[e] - m) : 0.f;       // (a tile of -inf alone has no mass)
-        sum = block_sum<SMP_NT>(sum, sf);
-        if (tid == 0) tile_s[slot] = sum;
+        for (int e = 1; e < 8; ++e) top[c] = fmaxf(top[c], x[c][e]);
     }
+    m = top[0];
+#pragma unroll
+    for (int c = 1; c < STEPS; ++c) m = fmaxf(m, top[c]);
+    m = wave_max(m);
+    if (lane == 0) sf[w] = m;
+    __syncthreads();
+    m = sf[0];
+#pragma unroll
+    for (int i = 1; i < WAVES; ++i) m = fmaxf(m, sf[i]);
+    m /= T;
     if (tid == 0) tile_m[slot] = m;
+    const int kc = sample_candidates(k, p, V, ntiles);
+    if (kc == 0 || !(k > 0 && k < V)) {                        // (behind top-k nothing is taken of the whole row's mass)
+        // between 2^-40 and 2^40 in size, all of them: the bits without the sign, doubled, minus the bound's
+        constexpr uint32_t LO = 2u * 0x2b800000u, HI = 2u * 0x53800000u;
+        uint32_t off = (2u * __float_as_uint(T)) - LO;
+#pragma unroll
+        for (int c = 0; c < STEPS; ++c)
+            if (j0 + c * TILE_STRETCH < V)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) off = max(off, 2u * __float_as_uint(x[c][e]) - LO);
+        const bool plain = __all(off <= HI - LO);
+        const float y = 1.0f / T;
+        float sum[STEPS];
+        if (plain) {                                           // (where ids end within a thread's eight, one of these is -inf: not plain)
+#pragma unroll
+            for (int c = 0; c < STEPS; ++c) {
+                float e_of[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) e_of[e] = expf(quotient(x[c][e], T, y) - m);
+                sum[c] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sum[c] += e_of[e];
+                if (j0 + c * TILE_STRETCH >= V) sum[c] = 0.f;
+            }
+        } else {
+#pragma unroll
+            for (int c = 0; c < STEPS; ++c) {
+                const int j = j0 + c * TILE_STRETCH;
+                sum[c] = 0.f;
+#pragma unroll 1
+                for (int e = 0; e < 8; ++e) {
+                    float xe = x[c][0];
+#pragma unroll
+                    for (int q = 1; q < 8; ++q) xe = e == q ? x[c][q] : xe;
+                    sum[c] += (j + e < V && m > -INFINITY) ? expf(xe / T - m) : 0.f;       // (a tile of -inf alone has no mass)
+                }
+            }
+        }
+        __syncthreads();                                       // (sf has been read)
+        tile_sums(sum, sf);
+        __syncthreads();
+        if (tid == 0) {
+            float t = 0.f;
+#pragma unroll
+            for (int i = 0; i < SMP_WAVES; ++i) t += sf[i];
+            tile_s[slot] = t;
+        }
+    }
     if (kc == 0) return;
-    // the tile's kc largest ids, written in id order; or, where the second kernel has room for them, all from the bound on: these
-    // hold the kc largest too, and finding exactly those takes as long again
+    // The tile's kc largest ids, written in id order; or, where the second kernel has room for them, all from the bound on: these
+    // hold the kc largest too, and finding exactly those takes as long again.  The bound is found among the logits.  Neighbouring
+    // logits may have one quotient, three at most where it is no smaller than 2^-126, and ids of one quotient count by their number: so
+    // all ids from a bound four places lower are taken.
     const int in_tile = min(SMP_TILE, V - tile * SMP_TILE);
     const size_t base = slot * SMP_KC;
     const bool all = in_tile <= kc;
     uint32_t tau = 0u;
-    int need = 0x7fffffff;
+    int need = 0x7fffffff, n[STEPS], place[STEPS];
     if (!all) {
-        uint32_t key[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) key[e] = j0 + e < V ? sort_key(z[e]) : 0u;
         const bool wide = sample_wide(k, V, gridDim.y, ntiles);
-        const uint32_t bound = bound_of_kth(key, kc, max(in_tile / (8 * LI_WAVE), 1), work_i);
-        bool found = false;
-        if (bound != 0u) {
-            put_from(key, bound, work_i, tot_i, [&](int at, int e) {
-                if (at < SMP_LIST) list[at] = key[e];
-                if (wide && at < SMP_KC) { cand_z[base + at] = z[e]; cand_id[base + at] = j0 + e; }
-            });
-            __syncthreads();
-            const int n = tot_i[0];
-            if (wide && n >= kc && n <= SMP_KC) {
-                if (tid == 0) tile_i[slot] = n;
+        const uint32_t bound = tile_bound(top, kc, in_tile, si);
+        const float from = bound > 4u ? key_value(bound - 4u) : -INFINITY;
+        if (from > -INFINITY && fabsf(from / T) > 0x1p-120f) {
+            // (by value, not by key: a zero more of the other sign does no harm.  A NaN counts as large)
+            uint32_t mask = 0u;                                // bit 8 c + e
+#pragma unroll
+            for (int c = STEPS - 1; c >= 0; --c)
+#pragma unroll
+                for (int e = 7; e >= 0; --e) mask = (mask << 1) | (!(x[c][e] < from) ? 1u : 0u);
+#pragma unroll
+            for (int c = 0; c < STEPS; ++c) n[c] = __popc((mask >> (8 * c)) & 255u);
+            const int total = tile_places(n, place, work_i);
+            const bool direct = wide && total >= kc && total <= SMP_KC;
+            if (direct || (total >= kc && total <= SMP_LIST)) {
+                for (uint32_t left = mask; left; left &= left - 1u) {
+                    const int i = __ffs((int)left) - 1, c = i >> 3, id = j0 + c * TILE_STRETCH + (i & 7);
+                    const float z = row[id] / T;               // (once more from memory: a register cannot be chosen by number)
+                    int at = place[0];
+#pragma unroll
+                    for (int q = 1; q < STEPS; ++q) at = c == q ? place[q] : at;
+                    at += __popc(mask & ((1u << i) - 1u) & (255u << (8 * c)));
+                    if (direct) { cand_z[base + at] = z; cand_id[base + at] = id; }
+                    else { list[at] = sort_key(z); list_id[at] = id; }
+                }
+                if (direct) {
+                    if (tid == 0) tile_i[slot] = total;
+                    return;
+                }
+                kth_of_list<NT>(list, total, kc, tau, need, tot_i);
+                // of the list, in its order: the keys above tau and the first `need` equal to it; a thread has the next ITEMS
+                uint32_t key[ITEMS];
+                int eq = 0, mine = 0;
+#pragma unroll
+                for (int e = 0; e < ITEMS; ++e) {
+                    key[e] = tid * ITEMS + e < total ? list[tid * ITEMS + e] : 0u;      // (no key of a number)
+                    eq += key[e] == tau;
+                }
+                const int rank0 = block_sum_before<WAVES>(eq, work_i);
+                int rank = rank0;
+#pragma unroll
+                for (int e = 0; e < ITEMS; ++e) mine += key[e] > tau || (key[e] == tau && rank++ < need);
+                int pos = block_sum_before<WAVES>(mine, work_i);
+                if (tid == NT - 1) tile_i[slot] = pos + mine;
+                rank = rank0;
+#pragma unroll
+                for (int e = 0; e < ITEMS; ++e)
+                    if (key[e] > tau || (key[e] == tau && rank++ < need)) {
+                        cand_z[base + pos] = key_value(key[e]);
+                        cand_id[base + pos] = list_id[tid * ITEMS + e];
+                        ++pos;
+                    }
                 return;
             }
-            found = n >= kc && n <= SMP_LIST;
-            if (found) kth_of_list(list, n, kc, tau, need, tot_i);
         }
-        if (!found) {
-            __syncthreads();                            // (tot_i has been read)
-            radix_kth([&](auto f) {
+        __syncthreads();                                       // (work_i has been read)
+    }
+    // in general: among the quotients
+#pragma unroll
+    for (int c = 0; c < STEPS; ++c)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[c][e] /= T;
+    if (!all)
+        radix_kth<WAVES>([&](auto f) {
+#pragma unroll
+            for (int c = 0; c < STEPS; ++c)
 #pragma unroll
                 for (int e = 0; e < 8; ++e)
-                    if (j0 + e < V) f(z[e]);
-            }, kc, tau, need, work_i, tot_i);
-        }
+                    if (j0 + c * TILE_STRETCH + e < V) f(x[c][e]);
+        }, kc, tau, need, work_i, tot_i);
+    int rank[STEPS];
+#pragma unroll
+    for (int c = 0; c < STEPS; ++c) {
+        n[c] = 0;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n[c] += (j0 + c * TILE_STRETCH + e < V) && sort_key(x[c][e]) == tau;
+        rank[c] = 0;
     }
+    if (!all) tile_places(n, rank, si);
+    auto in = [&](int c, int e, int& place_at_tau) {
+        const uint32_t key = sort_key(x[c][e]);
+        return (j0 + c * TILE_STRETCH + e < V) && (all || key > tau || (key == tau && place_at_tau++ < need));
+    };
+#pragma unroll
+    for (int c = 0; c < STEPS; ++c) {
+        n[c] = 0;
+        int at = rank[c];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) n[c] += in(c, e, at);
+    }
+    const int total = tile_places(n, place, si);
+    if (tid == 0) tile_i[slot] = total;
+#pragma unroll
+    for (int c = 0; c < STEPS; ++c) {
+        int at = rank[c];
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            if (in(c, e, at)) {
+                cand_z[base + place[c]] = x[c][e];
+                cand_id[base + place[c]] = j0 + c * TILE_STRETCH + e;
+                ++place[c];
+            }
+    }
+}
+
+// Inverse CDF over the survivors in a list (keys above tau and the first `need` equal to it), in id order: the first wave alone, a lane the
+// `per` next ones.
+__device__ __forceinline__ void pick_of_list(const uint32_t* list, const int* list_id, int n, uint32_t tau, int need, float m, float u, int* out) {
+    if (threadIdx.x >= LI_WAVE) return;
+    const int lane = threadIdx.x;
+    const int per = (n + LI_WAVE - 1) / LI_WAVE, from = lane * per, to = min(from + per, n);
     int eq = 0;
+    for (int j = from; j < to; ++j) eq += list[j] == tau;
+    int rank0 = eq;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) eq += (j0 + e < V) && sort_key(z[e]) == tau;
-    int rank = all ? 0 : block_sum_before(eq, si);
-    bool in[8];
-    int mine = 0;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        const uint32_t key = sort_key(z[e]);
-        in[e] = (j0 + e < V) && (all || key > tau || (key == tau && rank++ < need));
-        mine += in[e];
+    for (int o = 1; o < LI_WAVE; o <<= 1) {
+        const int t = __shfl_up(rank0, o, LI_WAVE);
+        if (lane >= o) rank0 += t;
     }
-    int pos = block_sum_before(mine, si);
-    if (tid == SMP_NT - 1) tile_i[slot] = pos + mine;
+    rank0 -= eq;                            // keys at tau before this lane's
+    auto in = [&](int j, int& rank) { return list[j] > tau || (list[j] == tau && rank++ < need); };
+    float mine = 0.f;
+    bool any = false;
+    for (int j = from, rank = rank0; j < to; ++j)
+        if (in(j, rank)) { mine += expf(key_value(list[j]) - m); any = true; }
+    float upto = mine;
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-        if (in[e]) {
-            cand_z[base + pos] = z[e];
-            cand_id[base + pos] = j0 + e;
-            ++pos;
+    for (int o = 1; o < LI_WAVE; o <<= 1) {
+        const float t = __shfl_up(upto, o, LI_WAVE);
+        if (lane >= o) upto += t;
+    }
+    float run = __shfl_up(upto, 1, LI_WAVE);
+    if (lane == 0) run = 0.f;
+    const float target = u * __shfl(upto, LI_WAVE - 1, LI_WAVE);
+    const unsigned long long reach = __ballot(any && run + mine >= target), some = __ballot(any);
+    const int chosen = reach ? __ffsll((long long)reach) - 1 : 63 - __clzll((long long)some);      // (else the last one with a survivor)
+    if (lane == chosen) {
+        int pick = -1;
+        for (int j = from, rank = rank0; j < to; ++j) {
+            if (!in(j, rank)) continue;
+            pick = list_id[j];
+            run += expf(key_value(list[j]) - m);
+            if (run >= target) break;
         }
+        *out = pick;
+    }
+}
+
+// A row with top-k (and top-p) whose tiles handed over up to SMP_KC ids each (sample_wide), from the candidates to the token; false, with nothing
+// done, where the general way has to be taken.  The same as select_kth, mass_of_list and pick_of_list one after the other, in fewer and
+// shorter steps: a wave takes the candidates of one tile or two (asked for with the tiles' counts, before these are known), so that places in the
+// list come from ballots; and the list is held against itself once, by four threads a key (each the entries whose number is its
+// own modulo four), for the number and the mass above it and from it on together: the masses above tau need no tau.
+// Top-k 50 with top-p 0.9, the rows kernel: 64 rows of 151,936 ids 18.2 -> 10.4 us, one row 13.9 -> 9.2.
+__device__ __forceinline__ bool rows_by_list(const float* cand_z, const int* cand_id, const int* tile_i, int ntiles, int k, float p, int V, float m, float u, int* out,
+                                             uint32_t* list, float* list_e, int* list_id, int* work_i, int* counts, float* res_f, int* res) {
+    constexpr int HOLD = SMP_KC / LI_WAVE, TILES = 2;            // (up to 32 tiles: sample_wide)
+    const int tid = threadIdx.x, lane = tid & (LI_WAVE - 1), w = __builtin_amdgcn_readfirstlane(tid / LI_WAVE);
+    const int full = V - (ntiles - 1) * SMP_TILE >= k ? ntiles : ntiles - 1;       // tiles with at least k candidates
+    const int parts = min(full, SMP_WAVES), rounds = parts > 0 ? (k + parts - 1) / parts : 0;
+    if (parts == 0 || rounds > LI_WAVE) return false;
+    float z[TILES][HOLD];
+    int id[TILES][HOLD], held[TILES];
+    uint32_t key[TILES][HOLD];
+#pragma unroll
+    for (int h = 0; h < TILES; ++h) {
+        const int t = w + h * SMP_WAVES;
+        held[h] = 0;
+        if (t < ntiles) {
+            held[h] = tile_i[t];
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                z[h][c] = cand_z[t * SMP_KC + c * LI_WAVE + lane];
+                id[h][c] = cand_id[t * SMP_KC + c * LI_WAVE + lane];
+            }
+        }
+    }
+    uint32_t most = 0u;
+#pragma unroll
+    for (int h = 0; h < TILES; ++h) {
+        const int t = w + h * SMP_WAVES;
+        if (held[h] > 2 * LI_WAVE)
+#pragma unroll
+            for (int c = 2; c < HOLD; ++c) {
+                z[h][c] = cand_z[t * SMP_KC + c * LI_WAVE + lane];
+                id[h][c] = cand_id[t * SMP_KC + c * LI_WAVE + lane];
+            }
+#pragma unroll
+        for (int c = 0; c < HOLD; ++c) {
+            key[h][c] = c * LI_WAVE + lane < held[h] ? sort_key(z[h][c]) : 0u;
+            most = max(most, key[h][c]);
+        }
+    }
+    const uint32_t largest = wave_bound<16>(most, rounds);
+    if (lane == 0) work_i[w] = (int)largest;
+    if (tid == 0) res[0] = 0;
+    __syncthreads();
+    uint32_t bound = 0xffffffffu;
+#pragma unroll
+    for (int i = 0; i < SMP_WAVES; ++i) bound = i < parts ? min(bound, (uint32_t)work_i[i] - 1u) : bound;
+    bound += 1u;                                                // (0, no bound, became the largest)
+    if (bound == 0u) return false;
+    unsigned long long in[TILES][HOLD];
+#pragma unroll
+    for (int h = 0; h < TILES; ++h) {
+        int n = 0;
+#pragma unroll
+        for (int c = 0; c < HOLD; ++c) { in[h][c] = __ballot(key[h][c] >= bound); n += __popcll(in[h][c]); }
+        if (lane == 0) counts[w + h * SMP_WAVES] = n;
+    }
+    __syncthreads();
+    const int own = lane < TILES * SMP_WAVES ? counts[lane] : 0;
+    auto sum = [](int v) {
+#pragma unroll
+        for (int o = 1; o < LI_WAVE; o <<= 1) v += lane_xor(v, o);
+        return __builtin_amdgcn_readfirstlane(v);
+    };
+    const int n = sum(own);
+    if (n > SMP_LIST) return false;
+#pragma unroll
+    for (int h = 0; h < TILES; ++h) {
+        if (w + h * SMP_WAVES >= ntiles) continue;
+        int at = sum(lane < w + h * SMP_WAVES ? own : 0);
+#pragma unroll
+        for (int c = 0; c < HOLD; ++c) {
+            if (!in[h][c]) continue;
+            if (key[h][c] >= bound) {
+                const int place = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(in[h][c] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in[h][c], 0));
+                list[place] = key[h][c];
+                list_id[place] = id[h][c];
+                list_e[place] = expf(z[h][c] - m);
+            }
+            at += __popcll(in[h][c]);
+        }
+    }
+    __syncthreads();
+    constexpr int TURNS = 4 * SMP_LIST / SMP_NT;
+    uint32_t mykey[TURNS];
+    float above_e[TURNS], from_e[TURNS];
+#pragma unroll
+    for (int q = 0; q < TURNS; ++q) {
+        const int i = (tid >> 2) + q * (SMP_NT / 4);
+        mykey[q] = 0u;
+        if (q * (SMP_NT / 4) >= n) continue;                    // (the same for all threads)
+        mykey[q] = i < n ? list[i] : 0u;
+        int above = 0, from = 0;
+        float ga = 0.f, gf = 0.f;
+#pragma unroll 8
+        for (int j = tid & 3; j < n; j += 4) {
+            const uint32_t v = list[j];
+            const float e = list_e[j];
+            above += v > mykey[q];
+            from += v >= mykey[q];
+            ga += v > mykey[q] ? e : 0.f;
+            gf += v >= mykey[q] ? e : 0.f;
+        }
+        above += lane_xor(above, 1); above += lane_xor(above, 2);
+        from += lane_xor(from, 1); from += lane_xor(from, 2);
+        above_e[q] = lane_xor_add(lane_xor_add(ga, 1), 2);
+        from_e[q] = lane_xor_add(lane_xor_add(gf, 1), 2);
+        if (i < n && above < k && from >= k) {                  // (all threads with this key write the same)
+            res[1] = (int)mykey[q];
+            res[2] = k - above;
+            res_f[0] = above_e[q];
+        }
+    }
+    __syncthreads();
+    uint32_t tau = (uint32_t)res[1];
+    int need = res[2];
+    if (p > 0.f && p < 1.f) {
+        const float mass = res_f[0], e_ties = (float)need * expf(key_value(tau) - m), want = p * (mass + e_ties);
+#pragma unroll
+        for (int q = 0; q < TURNS; ++q) {
+            if (mykey[q] < tau || mykey[q] == 0u) continue;
+            if (mykey[q] > tau ? above_e[q] < want && from_e[q] >= want : mass < want && mass + e_ties >= want) {
+                res[0] = 1;
+                res[3] = (int)mykey[q];
+                res_f[1] = want - (mykey[q] > tau ? above_e[q] : mass);
+            }
+        }
+        __syncthreads();
+        if (!res[0]) return false;                              // (rounding, or masses of zero)
+        const uint32_t tp = (uint32_t)res[3];
+        const int need_p = ties_needed(res_f[1], tp, m);
+        need = tp == tau ? min(need, need_p) : need_p;
+        tau = tp;
+    }
+    pick_of_list(list, list_id, n, tau, need, m, u, out);
+    return true;
 }
 
 // tile_m, tile_s, tile_i, cand_z, cand_id: what sample_tiles_kernel left for the row's ntiles tiles (ntiles <= SMP_NT)
@@ -672,21 +1121,22 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     __shared__ int pick_i[1];
     const int r = blockIdx.x, tid = threadIdx.x;
     const float* row = logits + (size_t)r * V;
-    const float T = temperature[r];
+    const float T = temperature[r], p = top_p[r], u = uniform[r];      // (together: one trip to memory)
+    const int k = top_k[r];
     tile_m += (size_t)r * ntiles;
     tile_s += (size_t)r * ntiles;
     tile_i += (size_t)r * ntiles;
     if (!(T > 0.f)) {                                          // greedy: the tiles' maxima, ties to the lower id
+        if (tid >= LI_WAVE) return;
         float v = -INFINITY;
         int i = 0x7fffffff;
-        for (int t = tid; t < ntiles; t += SMP_NT) argmax_combine(v, i, tile_m[t], tile_i[t]);
-        block_argmax(v, i, sf, si);
+        for (int t = tid; t < ntiles; t += LI_WAVE) argmax_combine(v, i, tile_m[t], tile_i[t]);
+#pragma unroll
+        for (int o = LI_WAVE / 2; o > 0; o >>= 1) argmax_combine(v, i, lane_xor(v, o), lane_xor(i, o));
         if (tid == 0) out[r] = i;
         return;
     }
     const bool vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
-    const int k = top_k[r];
-    const float p = top_p[r];
     const bool filtered = !sample_unfiltered(k, p, V);
     const bool by_k = k > 0 && k < V, by_p = p > 0.f && p < 1.f;
 
@@ -701,6 +1151,11 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     }
 
     const int kc = sample_candidates(k, p, V, ntiles);
+    if (kc > 0 && by_k && sample_wide(k, V, gridDim.x, ntiles)) {
+        const size_t at = (size_t)r * ntiles * SMP_KC;
+        if (rows_by_list(cand_z + at, cand_id + at, tile_i, ntiles, k, p, V, m, u, out + r, list, list_e, list_id, work_i, ties_before, pick_f, tot_i)) return;
+        __syncthreads();
+    }
     if (kc > 0) {
         // ---- among the candidates, in ascending ids: thread t has the C of them from t * C on
         float cz[SMP_CAND_PER_THREAD];
@@ -776,44 +1231,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
             }
         }
         if (by_k && listed && (done || !by_p)) {
-            // inverse CDF over the survivors in the list, in id order: the first wave alone, a lane the `per` next ones
-            if (tid >= LI_WAVE) return;
-            const int per = (n + LI_WAVE - 1) / LI_WAVE, from = lane * per, to = min(from + per, n);
-            int eq = 0;
-            for (int j = from; j < to; ++j) eq += list[j] == tau;
-            int rank0 = eq;
-#pragma unroll
-            for (int o = 1; o < LI_WAVE; o <<= 1) {
-                const int t = __shfl_up(rank0, o, LI_WAVE);
-                if (lane >= o) rank0 += t;
-            }
-            rank0 -= eq;                            // keys at tau before this lane's
-            auto in = [&](int j, int& rank) { return list[j] > tau || (list[j] == tau && rank++ < need); };
-            float mine = 0.f;
-            bool any = false;
-            for (int j = from, rank = rank0; j < to; ++j)
-                if (in(j, rank)) { mine += expf(key_value(list[j]) - m); any = true; }
-            float upto = mine;
-#pragma unroll
-            for (int o = 1; o < LI_WAVE; o <<= 1) {
-                const float t = __shfl_up(upto, o, LI_WAVE);
-                if (lane >= o) upto += t;
-            }
-            float run = __shfl_up(upto, 1, LI_WAVE);
-            if (lane == 0) run = 0.f;
-            const float target = uniform[r] * __shfl(upto, LI_WAVE - 1, LI_WAVE);
-            const unsigned long long reach = __ballot(any && run + mine >= target), some = __ballot(any);
-            const int chosen = reach ? __ffsll((long long)reach) - 1 : 63 - __clzll((long long)some);      // (else the last one with a survivor)
-            if (lane == chosen) {
-                int pick = -1;
-                for (int j = from, rank = rank0; j < to; ++j) {
-                    if (!in(j, rank)) continue;
-                    pick = list_id[j];
-                    run += expf(key_value(list[j]) - m);
-                    if (run >= target) break;
-                }
-                out[r] = pick;
-            }
+            pick_of_list(list, list_id, n, tau, need, m, u, out + r);
             return;
         }
         if (by_p && !done) {
@@ -858,7 +1276,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
                 }
             }
             const float run0 = block_sum_before(mine, work_f);
-            if (tid == SMP_NT - 1) pick_f[0] = uniform[r] * (run0 + mine);
+            if (tid == SMP_NT - 1) pick_f[0] = u * (run0 + mine);
             __syncthreads();
             const float target = pick_f[0];
             int chosen = block_min_int((any && run0 + mine >= target) ? tid : 0x7fffffff, si);
@@ -941,9 +1359,8 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     }
     // this thread's ids of a tile: their mass (sum in id order), whether any survives, and the place
     // among the ids at tau of its first one
-    auto mine_of = [&](int t, bool& any, int& rank0) {
+    auto mine_of = [&](int t, bool& any, int& rank0, float (&z)[8]) {
         const int j0 = t * SMP_TILE + tid * 8;
-        float z[8];
         any = false;
         rank0 = 0;
         if (j0 < V) load_ids8(row, j0, V, T, vec, z);
@@ -971,50 +1388,49 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     if (!filtered) {
         // The tiles' sums are there, each against its tile's own maximum: brought to the row's maximum
         // they give the tile that holds the target; within it the search goes on in the tile's own scale.
-        float top = -INFINITY;
-        if (ntiles == 1) {                           // (a vocabulary of one tile: nothing to do side by side, 12.1 -> 11.4 us)
-            top = tile_m[0];
-            if (tid == 0) tile_sum[0] = tile_s[0] * expf(tile_m[0] - top);
-        } else {
-            for (int t = tid & (LI_WAVE - 1); t < ntiles; t += LI_WAVE) top = fmaxf(top, tile_m[t]);
-            top = wave_max(top);
-            for (int t = tid; t < ntiles; t += SMP_NT) tile_sum[t] = tile_s[t] * expf(tile_m[t] - top);
-            __syncthreads();
-        }
-        if (tid == 0) {
+        auto look = [&](auto sum_of, float top) {
             float total = 0.f;
-#pragma unroll 8
-            for (int t = 0; t < ntiles; ++t) total += tile_sum[t];
-            const float want = uniform[r] * total;
+            for (int t = 0; t < ntiles; ++t) total += sum_of(t);
+            const float want = u * total;
             float run = 0.f;
             int pick = -1, last = 0;                 // (a tile far below the maximum has no mass at all in float32)
             for (int t = 0; t < ntiles; ++t) {
-                const float w = tile_sum[t];
+                const float w = sum_of(t);
                 if (w > 0.f) last = t;
                 if (w > 0.f && run + w >= want) { pick = t; break; }
                 run += w;
             }
             const bool past = pick < 0;              // rounding left the target just above the total:
-            if (past) pick = last;                   // the last id with mass (no sum reaches infinity below)
-            pick_i[0] = pick;
-            pick_f[0] = 0.f;
-            pick_f[1] = past ? INFINITY : (want - run) / expf(tile_m[pick] - top);
-            pick_f[2] = tile_m[pick];
+            tile = past ? last : pick;               // the last id with mass (no sum reaches infinity below)
+            m = tile_m[tile];
+            target = past ? INFINITY : (want - run) / expf(m - top);
+        };
+        if (ntiles <= LI_WAVE) {                     // every wave by itself, a lane a tile: no barrier
+            const int lane = tid & (LI_WAVE - 1), t = lane < ntiles ? lane : 0;
+            const float own = tile_m[t], own_s = tile_s[t], top = wave_max(own);
+            const int sum = __float_as_int(lane < ntiles ? own_s * expf(own - top) : 0.f);
+            look([&](int i) { return __int_as_float(__builtin_amdgcn_readlane(sum, i)); }, top);
+        } else {
+            float top = -INFINITY;
+            for (int t = tid & (LI_WAVE - 1); t < ntiles; t += LI_WAVE) top = fmaxf(top, tile_m[t]);
+            top = wave_max(top);
+            for (int t = tid; t < ntiles; t += SMP_NT) tile_sum[t] = tile_s[t] * expf(tile_m[t] - top);
+            __syncthreads();
+            look([&](int i) { return tile_sum[i]; }, top);
         }
-        __syncthreads();
-        m = pick_f[2];
     } else {
         for (int t = 0; t < ntiles; ++t) {
             bool any;
             int rank0;
-            const float ts = block_sum<SMP_NT>(mine_of(t, any, rank0), sf);
+            float z[8];
+            const float ts = block_sum<SMP_NT>(mine_of(t, any, rank0, z), sf);
             if (tid == 0) tile_sum[t] = ts;
         }
         __syncthreads();
         if (tid == 0) {
             float total = 0.f;
             for (int t = 0; t < ntiles; ++t) total += tile_sum[t];
-            const float want = uniform[r] * total;
+            const float want = u * total;
             float run = 0.f;
             int pick = -1, last = 0;
             for (int t = 0; t < ntiles; ++t) {
@@ -1029,30 +1445,31 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
             pick_f[1] = past ? INFINITY : want;
         }
         __syncthreads();
+        tile = pick_i[0];
+        before = pick_f[0];
+        target = pick_f[1];
     }
-    tile = pick_i[0];
-    before = pick_f[0];
-    target = pick_f[1];
     // within the tile: the first thread whose ids bring the running sum to the target, else the last one with a survivor
     bool any;
     int rank0;
-    const float mine = mine_of(tile, any, rank0);
+    float z[8];
+    const float mine = mine_of(tile, any, rank0, z);
     const float run0 = before + block_sum_before(mine, work_f);
     int chosen = block_min_int((any && run0 + mine >= target) ? tid : 0x7fffffff, si);
     if (chosen == 0x7fffffff) chosen = -block_min_int(any ? -tid : 1, si);     // (the tile has a survivor: its sum is above zero)
     if (tid == chosen) {
         const int j0 = tile * SMP_TILE + tid * 8;
-        float z[8];
-        load_ids8(row, j0, V, T, vec, z);
         float run = run0;
         int rank = rank0, pick = j0;
-        for (int e = 0; e < 8 && j0 + e < V; ++e) {
+        bool done = false;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
             const uint32_t key = sort_key(z[e]);
-            const bool in = !cut || key > tau || (key == tau && (!ranked || rank++ < need));
+            const bool in = !done && j0 + e < V && (!cut || key > tau || (key == tau && (!ranked || rank++ < need)));
             if (!in) continue;
             pick = j0 + e;
             run += expf(z[e] - m);
-            if (run >= target) break;
+            done = run >= target;
         }
         out[r] = pick;
     }
@@ -1130,7 +1547,9 @@ extern "C" int li_sample_rows(const float* logits, const float* temperature, con
     int* ti = reinterpret_cast<int*>(tiles + 2 * per);
     float* cz = tiles + 3 * per;
     int* ci = reinterpret_cast<int*>(tiles + (3 + (size_t)SMP_KC) * per);
-    sample_tiles_kernel<<<dim3(ntiles, n), SMP_NT, 0, stream>>>(logits, temperature, top_k, top_p, tm, ts, ti, cz, ci, V);
+    const dim3 grid(ntiles, n);
+    if (per >= TILE_MANY) sample_tiles_kernel<4><<<grid, TILE_NT<4>, 0, stream>>>(logits, temperature, top_k, top_p, tm, ts, ti, cz, ci, V);
+    else sample_tiles_kernel<1><<<grid, TILE_NT<1>, 0, stream>>>(logits, temperature, top_k, top_p, tm, ts, ti, cz, ci, V);
     sample_rows_kernel<<<n, SMP_NT, 0, stream>>>(logits, temperature, top_k, top_p, uniform, out, V, tm, ts, ti, cz, ci, ntiles);
     return li_launch_status();
 }

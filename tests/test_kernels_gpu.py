@@ -1491,6 +1491,43 @@ def test_sample_rows_with_tiles_that_hand_over_different_numbers_of_candidates(o
             assert _pick_is_right(rows[r], 0.8, top_k[r], top_p, u[r], picks[r]), (r, top_k[r], top_p)
 
 
+@pytest.mark.parametrize("vocab", [6 * 8192 + 1, 6 * 8192 + 2049, 7 * 8192 - 1, 7 * 8192])
+def test_sample_rows_takes_the_same_ids_where_the_tiles_are_many(ops, vocab):
+    # 768 tiles and more are taken by other blocks (four stretches of ids a wave): the same sums in the same order, so the same ids, as
+    # when a few rows are sampled alone; the largest are found among the logits (neighbours of one quotient included), quotients come from
+    # a reciprocal where all sizes allow it
+    g = torch.Generator().manual_seed(18)
+    n = 110
+    logits = torch.randn(n, vocab, generator=g) * 3
+    logits[10:20] = torch.round(logits[10:20] * 2) / 2                  # ids of one value, zeros of both signs among them
+    logits[20:25] = logits[20:25].to(torch.bfloat16).float()
+    logits[25:30, ::3] = float("-inf")
+    logits[30:33] = -logits[30:33].abs() - 100.0
+    logits[33:36] *= 1e-13                                              # (too small for the reciprocal)
+    logits[36:39] *= 1e12
+    logits[39, : vocab - 40] = float("-inf")
+    big = torch.full((vocab,), 8388608.0) + torch.randint(0, 40, (vocab,), generator=g)
+    logits[40:44] = big                                                 # neighbouring float32 numbers, two of which share a quotient now and then
+    temperature = [(0.0, 0.7, 3.0, 0.8, 1.3)[i % 5] for i in range(n)]
+    for r in range(33, 36):
+        temperature[r] = 1e-13
+    for r in (*range(36, 39), *range(40, 44)):
+        temperature[r] = (3e12, 3.0, 5.0, 3.0, 7.0, 1e12, 1.7)[r % 7]
+    top_k = [(0, 50, 3, 256, 0, 200, 1)[i % 7] for i in range(n)]
+    top_p = [(1.0, 0.9, 0.5)[i % 3] if top_k[i] else 1.0 for i in range(n)]
+    u = torch.rand(n, generator=g).tolist()
+    picks = _sample(ops, logits, temperature, top_k, top_p, u)
+    for r in range(n):
+        one = _sample(ops, logits[r:r + 1], temperature[r:r + 1], top_k[r:r + 1], top_p[r:r + 1], u[r:r + 1])[0]
+        assert picks[r] == one, r
+        if r < 45:
+            row = logits[r].double().numpy()
+            if temperature[r] == 0.0:
+                assert picks[r] == plain_impl.argmax_first(row), r
+            elif r < 40:                                                # (beyond: the float64 quotients differ where the float32 ones are one)
+                assert _pick_is_right(row, temperature[r], top_k[r], top_p[r], u[r], picks[r], 1e-4), r
+
+
 def test_sample_rows_frequencies_and_ties(ops):
     lg = torch.tensor([[2.0, 1.0, 3.0, 3.0, -1.0, 0.5, 2.5, 0.0]])
     n = 4000
