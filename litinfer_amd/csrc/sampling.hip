@@ -685,10 +685,21 @@ __device__ __forceinline__ uint32_t tile_bound(const float (&top)[STEPS], int kk
     return bound + 1u;
 }
 
-template <int STEPS>
+// A step's options, a row each: arrays on the device, or, up to N rows, in the launch's own arguments (which takes a copy to the device, its
+// kernel and its event out of a step: SampleCall below).
+struct SampleArrays {
+    const float *temperature, *top_p, *uniform;
+    const int* top_k;
+};
+template <int N>
+struct SampleValues {
+    float temperature[N], top_p[N], uniform[N];
+    int top_k[N];
+};
+
+template <int STEPS, typename Options>
 __global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_tiles_kernel(
-    const float* __restrict__ logits, const float* __restrict__ temperature, const int* __restrict__ top_k,
-    const float* __restrict__ top_p, float* __restrict__ tile_m, float* __restrict__ tile_s,
+    const float* __restrict__ logits, const Options o, float* __restrict__ tile_m, float* __restrict__ tile_s,
     int* __restrict__ tile_i, float* __restrict__ cand_z, int* __restrict__ cand_id, int V) {
     constexpr int NT = TILE_NT<STEPS>, WAVES = TILE_WAVES<STEPS>, ITEMS = SMP_LIST / NT;
     __shared__ float sf[SMP_WAVES];
@@ -701,9 +712,8 @@ __global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_til
     const float* row = logits + (size_t)r * V;
     const int j0 = tile * SMP_TILE + w * STEPS * TILE_STRETCH + lane * 8;
     const size_t slot = (size_t)r * ntiles + tile;
-    const float T = temperature[r];
-    const int k = top_k[r];
-    const float p = top_p[r];
+    const float T = o.temperature[r], p = o.top_p[r];
+    const int k = o.top_k[r];
     float x[STEPS][8];                                         // the logits; past the end -inf
     const bool vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
 #pragma unroll
@@ -917,7 +927,8 @@ __global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_til
 
 // Inverse CDF over the survivors in a list (keys above tau and the first `need` equal to it), in id order: the first wave alone, a lane the
 // `per` next ones.
-__device__ __forceinline__ void pick_of_list(const uint32_t* list, const int* list_id, int n, uint32_t tau, int need, float m, float u, int* out) {
+template <typename Choose>
+__device__ __forceinline__ void pick_of_list(const uint32_t* list, const int* list_id, int n, uint32_t tau, int need, float m, float u, Choose&& choose) {
     if (threadIdx.x >= LI_WAVE) return;
     const int lane = threadIdx.x;
     const int per = (n + LI_WAVE - 1) / LI_WAVE, from = lane * per, to = min(from + per, n);
@@ -954,7 +965,7 @@ __device__ __forceinline__ void pick_of_list(const uint32_t* list, const int* li
             run += expf(key_value(list[j]) - m);
             if (run >= target) break;
         }
-        *out = pick;
+        choose(pick);
     }
 }
 
@@ -964,7 +975,8 @@ __device__ __forceinline__ void pick_of_list(const uint32_t* list, const int* li
 // list come from ballots; and the list is held against itself once, by four threads a key (each the entries whose number is its
 // own modulo four), for the number and the mass above it and from it on together: the masses above tau need no tau.
 // Top-k 50 with top-p 0.9, the rows kernel: 64 rows of 151,936 ids 18.2 -> 10.4 us, one row 13.9 -> 9.2.
-__device__ __forceinline__ bool rows_by_list(const float* cand_z, const int* cand_id, const int* tile_i, int ntiles, int k, float p, int V, float m, float u, int* out,
+template <typename Choose>
+__device__ __forceinline__ bool rows_by_list(const float* cand_z, const int* cand_id, const int* tile_i, int ntiles, int k, float p, int V, float m, float u, Choose&& choose,
                                              uint32_t* list, float* list_e, int* list_id, int* work_i, int* counts, float* res_f, int* res) {
     constexpr int HOLD = SMP_KC / LI_WAVE, TILES = 2;            // (up to 32 tiles: sample_wide)
     const int tid = threadIdx.x, lane = tid & (LI_WAVE - 1), w = __builtin_amdgcn_readfirstlane(tid / LI_WAVE);
@@ -1097,15 +1109,15 @@ __device__ __forceinline__ bool rows_by_list(const float* cand_z, const int* can
         need = tp == tau ? min(need, need_p) : need_p;
         tau = tp;
     }
-    pick_of_list(list, list_id, n, tau, need, m, u, out);
+    pick_of_list(list, list_id, n, tau, need, m, u, choose);
     return true;
 }
 
 // tile_m, tile_s, tile_i, cand_z, cand_id: what sample_tiles_kernel left for the row's ntiles tiles (ntiles <= SMP_NT)
+// out: [rows] on the device; host (may be null): the same ids once more, in memory of the host that the device can write
+template <typename Options>
 __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
-    const float* __restrict__ logits, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ top_p,
-    const float* __restrict__ uniform, int* __restrict__ out, int V,
+    const float* __restrict__ logits, const Options o, int* __restrict__ out, int* __restrict__ host, int V,
     const float* __restrict__ tile_m, const float* __restrict__ tile_s, const int* __restrict__ tile_i,
     const float* __restrict__ cand_z, const int* __restrict__ cand_id, int ntiles) {
     __shared__ float sf[SMP_WAVES];
@@ -1121,8 +1133,12 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     __shared__ int pick_i[1];
     const int r = blockIdx.x, tid = threadIdx.x;
     const float* row = logits + (size_t)r * V;
-    const float T = temperature[r], p = top_p[r], u = uniform[r];      // (together: one trip to memory)
-    const int k = top_k[r];
+    const float T = o.temperature[r], p = o.top_p[r], u = o.uniform[r];      // (together: one trip to memory)
+    const int k = o.top_k[r];
+    auto choose = [&](int id) {
+        out[r] = id;
+        if (host) host[r] = id;
+    };
     tile_m += (size_t)r * ntiles;
     tile_s += (size_t)r * ntiles;
     tile_i += (size_t)r * ntiles;
@@ -1133,7 +1149,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
         for (int t = tid; t < ntiles; t += LI_WAVE) argmax_combine(v, i, tile_m[t], tile_i[t]);
 #pragma unroll
         for (int o = LI_WAVE / 2; o > 0; o >>= 1) argmax_combine(v, i, lane_xor(v, o), lane_xor(i, o));
-        if (tid == 0) out[r] = i;
+        if (tid == 0) choose(i);
         return;
     }
     const bool vec = (reinterpret_cast<uintptr_t>(row) & 15) == 0;
@@ -1153,7 +1169,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
     const int kc = sample_candidates(k, p, V, ntiles);
     if (kc > 0 && by_k && sample_wide(k, V, gridDim.x, ntiles)) {
         const size_t at = (size_t)r * ntiles * SMP_KC;
-        if (rows_by_list(cand_z + at, cand_id + at, tile_i, ntiles, k, p, V, m, u, out + r, list, list_e, list_id, work_i, ties_before, pick_f, tot_i)) return;
+        if (rows_by_list(cand_z + at, cand_id + at, tile_i, ntiles, k, p, V, m, u, choose, list, list_e, list_id, work_i, ties_before, pick_f, tot_i)) return;
         __syncthreads();
     }
     if (kc > 0) {
@@ -1231,7 +1247,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
             }
         }
         if (by_k && listed && (done || !by_p)) {
-            pick_of_list(list, list_id, n, tau, need, m, u, out + r);
+            pick_of_list(list, list_id, n, tau, need, m, u, choose);
             return;
         }
         if (by_p && !done) {
@@ -1293,7 +1309,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
                     run += expf(cz[c] - m);
                     if (run >= target) break;
                 }
-                out[r] = pick;
+                choose(pick);
             }
             return;
         }
@@ -1471,7 +1487,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
             run += expf(z[e] - m);
             done = run >= target;
         }
-        out[r] = pick;
+        choose(pick);
     }
 }
 
@@ -1487,7 +1503,7 @@ __global__ __launch_bounds__(SMP_NT) void sample_rows_kernel(
 // stream `seed`: a splitmix64 hash of both, its upper 24 bits as a value in [0, 1).  A row that samples
 // (temperature > 0) advances its slot's count.  A slot outside the table gives a greedy row.
 #define SAMPLE_SLOT_WORDS 8
-__device__ __forceinline__ float stream_uniform(unsigned long long seed, unsigned long long counter) {
+__host__ __device__ __forceinline__ float stream_uniform(unsigned long long seed, unsigned long long counter) {
     unsigned long long z = seed * 0x9E3779B97F4A7C15ull + (counter + 1ull) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
@@ -1535,9 +1551,8 @@ extern "C" long li_sample_rows_scratch_floats(int n, int V) {
 }
 
 // tiles: scratch of li_sample_rows_scratch_floats(n, V) floats, in which the first kernel leaves every tile's part.
-extern "C" int li_sample_rows(const float* logits, const float* temperature, const int* top_k,
-                              const float* top_p, const float* uniform, int* out, int n, int V,
-                              float* tiles, long tiles_floats, hipStream_t stream) {
+template <typename Options>
+static int launch_sample(const float* logits, const Options& o, int* out, int* host, int n, int V, float* tiles, long tiles_floats, hipStream_t stream) {
     if (n <= 0 || n > 65535 || V <= 0) return LI_ERR_SIZE;
     const int ntiles = (V + SMP_TILE - 1) / SMP_TILE;
     if (ntiles > SMP_NT || !tiles || tiles_floats < li_sample_rows_scratch_floats(n, V)) return LI_ERR_SIZE;
@@ -1548,8 +1563,47 @@ extern "C" int li_sample_rows(const float* logits, const float* temperature, con
     float* cz = tiles + 3 * per;
     int* ci = reinterpret_cast<int*>(tiles + (3 + (size_t)SMP_KC) * per);
     const dim3 grid(ntiles, n);
-    if (per >= TILE_MANY) sample_tiles_kernel<4><<<grid, TILE_NT<4>, 0, stream>>>(logits, temperature, top_k, top_p, tm, ts, ti, cz, ci, V);
-    else sample_tiles_kernel<1><<<grid, TILE_NT<1>, 0, stream>>>(logits, temperature, top_k, top_p, tm, ts, ti, cz, ci, V);
-    sample_rows_kernel<<<n, SMP_NT, 0, stream>>>(logits, temperature, top_k, top_p, uniform, out, V, tm, ts, ti, cz, ci, ntiles);
+    if (per >= TILE_MANY) sample_tiles_kernel<4, Options><<<grid, TILE_NT<4>, 0, stream>>>(logits, o, tm, ts, ti, cz, ci, V);
+    else sample_tiles_kernel<1, Options><<<grid, TILE_NT<1>, 0, stream>>>(logits, o, tm, ts, ti, cz, ci, V);
+    sample_rows_kernel<Options><<<n, SMP_NT, 0, stream>>>(logits, o, out, host, V, tm, ts, ti, cz, ci, ntiles);
     return li_launch_status();
+}
+
+extern "C" int li_sample_rows(const float* logits, const float* temperature, const int* top_k,
+                              const float* top_p, const float* uniform, int* out, int n, int V,
+                              float* tiles, long tiles_floats, hipStream_t stream) {
+    return launch_sample(logits, SampleArrays{temperature, top_p, uniform, top_k}, out, nullptr, n, V, tiles, tiles_floats, stream);
+}
+
+// The same from the host's own records of the rows' options (SamplingParams keeps one, so that a step only strings them together) and their
+// streams' counters: nothing is sent to the device but the launches, and the ids go to the host's pinned memory by the kernel that chooses them.
+// Up to SAMPLE_CALL_ROWS rows (2 KB of the 4 KB that a launch's arguments may take).  A step of 64 rows of 151,936 ids from call to call: the host's
+// 52 us (packing 18, sending the arrays 14, launches 11, copying the ids back and its event 9) are 23, the step 60 -> 28 us, alone 105 -> 48.
+struct SampleRecord {
+    float temperature, top_p;
+    unsigned long long seed;
+    int top_k, unused;
+};
+static_assert(sizeof(SampleRecord) == 24, "as the host packs it");
+#define SAMPLE_CALL_ROWS 128
+template <int N>
+static int sample_call(const float* logits, const SampleRecord* rec, const unsigned long long* counters, int* out, int* host, int n, int V, float* tiles,
+                       long tiles_floats, hipStream_t stream) {
+    SampleValues<N> v;
+    for (int i = 0; i < n; ++i) {
+        v.temperature[i] = rec[i].temperature > 0.f ? rec[i].temperature : 0.f;
+        v.top_p[i] = rec[i].top_p;
+        v.uniform[i] = stream_uniform(rec[i].seed, counters[i]);
+        v.top_k[i] = rec[i].top_k;
+    }
+    return launch_sample(logits, v, out, host, n, V, tiles, tiles_floats, stream);
+}
+extern "C" int li_sample_call_rows(void) { return SAMPLE_CALL_ROWS; }
+extern "C" int li_sample_call(const float* logits, const void* records, const unsigned long long* counters, int* out, int* host, int n, int V,
+                              float* tiles, long tiles_floats, hipStream_t stream) {
+    if (n <= 0 || n > SAMPLE_CALL_ROWS || !records || !counters || !out) return LI_ERR_SIZE;
+    const SampleRecord* rec = reinterpret_cast<const SampleRecord*>(records);
+    if (n <= 16) return sample_call<16>(logits, rec, counters, out, host, n, V, tiles, tiles_floats, stream);
+    if (n <= 64) return sample_call<64>(logits, rec, counters, out, host, n, V, tiles, tiles_floats, stream);
+    return sample_call<SAMPLE_CALL_ROWS>(logits, rec, counters, out, host, n, V, tiles, tiles_floats, stream);
 }

@@ -9,8 +9,9 @@ from __future__ import annotations
 
 import ctypes
 import math
+from array import array
 from dataclasses import dataclass
-from ctypes import c_float, c_int, c_long, c_void_p
+from ctypes import c_char_p, c_float, c_int, c_long, c_void_p
 from typing import Dict, Optional, Union
 
 import numpy as np
@@ -108,6 +109,7 @@ _SIGNATURES = {
     "sampling": {
         "li_argmax_rows": [P, P, P, P, I, I],
         "li_sample_rows": [P, P, P, P, P, P, I, I, P, L],
+        "li_sample_call": [P, c_char_p, P, P, P, I, I, P, L],
         "li_sample_prepare": [P, I, P, I, P, P, P, P],
     },
 }
@@ -1826,14 +1828,37 @@ def sample_rows_packed(logits: torch.Tensor, rows: torch.Tensor, out: torch.Tens
     _sample_rows(logits, n, at, at + 12 * n, at + 4 * n, at + 8 * n, out)
 
 
+SAMPLE_CALL_ROWS = 128         # rows up to which `sample_call` takes a step's options
+
+
+def sample_call(logits: torch.Tensor, records: bytes, counters: array, out: torch.Tensor, host: torch.Tensor) -> None:
+    """`sample_rows` with the rows' options and streams in the launch's own arguments: `records`, 24 bytes a row (temperature and top_p as
+    float32, the seed as uint64, top_k as int32, four more), `counters`, array("Q"), the number of each row's draw; row i's token goes
+    to out[i] on the device and to host[i], pinned memory of the host (complete when the stream has come past the call).  At most SAMPLE_CALL_ROWS rows."""
+    _gpu(logits, out)
+    _chk(logits.dim() == 2 and logits.dtype is torch.float32 and logits.is_contiguous(), "sample: logits")
+    n, v = logits.shape
+    _chk(0 < n <= SAMPLE_CALL_ROWS and len(records) == 24 * n and len(counters) == n and counters.itemsize == 8, "sample: per-row options")
+    _chk(out.dtype is torch.int32 and out.numel() == n and out.is_contiguous(), "sample: out")
+    _chk(host.dtype is torch.int32 and host.numel() >= n and host.is_contiguous() and host.is_pinned(), "sample: host")
+    tiles = _sample_tiles(logits, n, v)
+    _run("sampling", "li_sample_call", logits.data_ptr(), records, counters.buffer_info()[0], out.data_ptr(), host.data_ptr(), n, v, tiles.data_ptr(),
+         tiles.numel())
+
+
+def _sample_tiles(logits: torch.Tensor, n: int, v: int) -> torch.Tensor:
+    """What the first of the two kernels leaves for the second."""
+    key = (logits.device, n, v)
+    if key not in _sample_scratch:
+        _sample_scratch[key] = torch.empty(_sample_scratch_floats(n, v), dtype=torch.float32, device=logits.device)
+    return _sample_scratch[key]
+
+
 def _sample_rows(logits: torch.Tensor, n: int, temperature: int, top_k: int, top_p: int, uniform: int, out: torch.Tensor) -> None:
     if not n:
         return
     v = logits.shape[1]
-    key = (logits.device, n, v)
-    if key not in _sample_scratch:                   # what the first of the two kernels leaves for the second
-        _sample_scratch[key] = torch.empty(_sample_scratch_floats(n, v), dtype=torch.float32, device=logits.device)
-    tiles = _sample_scratch[key]
+    tiles = _sample_tiles(logits, n, v)
     _run("sampling", "li_sample_rows", logits.data_ptr(), temperature, top_k, top_p, uniform, out.data_ptr(), n, v,
          tiles.data_ptr(), tiles.numel())
 

@@ -18,6 +18,7 @@ device.
 """
 from __future__ import annotations
 
+import struct
 from array import array
 from dataclasses import dataclass
 from operator import attrgetter
@@ -30,6 +31,7 @@ from ..kernels import ops
 from ..utils.pinned import BatchUploader, record_event
 
 _MASK = (1 << 64) - 1
+_RECORD = struct.Struct("<ffQii")       # a row's options as the device's library takes them (csrc/sampling.hip: SampleRecord)
 
 
 @dataclass(frozen=True)
@@ -38,6 +40,14 @@ class SamplingParams:
     top_k: int = 0                  # active when 0 < top_k < vocabulary (:903)
     top_p: float = 1.0              # active when 0 < top_p < 1 (:904)
     seed: int = 0
+
+    def __post_init__(self):
+        # what a step sends of these options, packed once (None: numbers that only the arrays' own conversions judge)
+        try:
+            packed = _RECORD.pack(self.temperature, self.top_p, self.seed & _MASK, self.top_k, 0)
+        except (struct.error, OverflowError, TypeError):
+            packed = None
+        object.__setattr__(self, "_packed", packed)
 
     @property
     def greedy(self) -> bool:
@@ -55,6 +65,7 @@ def uniform(seed: int, counter: int) -> float:
 
 
 _OPTIONS = attrgetter("temperature", "top_p", "seed", "top_k")
+_PACKED = attrgetter("_packed")
 _WEYL, _MIX1, _MIX2 = np.uint64(0x9E3779B97F4A7C15), np.uint64(0xBF58476D1CE4E5B9), np.uint64(0x94D049BB133111EB)
 
 
@@ -70,12 +81,21 @@ def _uniforms(seeds: Sequence[int], counters: Sequence[int]) -> np.ndarray:
     return (z >> np.uint64(40)).astype(np.float32) * np.float32(2.0 ** -24)
 
 
+_unread: List[tuple] = []               # (event, host memory) of results that were let go before they were there
+
+
 class PendingTokens:
     """Tokens that were chosen on the device and are on their way to the host."""
 
     def __init__(self, sampler, host: torch.Tensor, n: int, event):
         self._sampler, self._host, self._n, self._event = sampler, host, n, event
         self._tokens: Optional[List[int]] = None
+
+    def __del__(self):
+        # Nobody has asked for the tokens, and the device may not have written them yet: until it has, the memory is not free.  (A copy
+        # into pinned memory says so to torch's allocator; a kernel that writes there does not.)
+        if self._tokens is None and self._event is not None and not self._event.query():
+            _unread.append((self._event, self._host))
 
     def result(self) -> List[int]:
         """The tokens; waits for the device if they are not there yet."""
@@ -162,6 +182,27 @@ class Sampler:
         if len(self._free_host) < 8:
             self._free_host.append(buf)
 
+    def _call(self, logits: torch.Tensor, params: Sequence[SamplingParams], counters: Sequence[int], ids: torch.Tensor) -> Optional["PendingTokens"]:
+        """The rows' options in the launch's arguments and the ids written to the host by the kernel that chooses them: no array, copy or
+        event to the device (of a step of 64 rows, 30 of the host's 52 us).  None where the options are not packed or the rows too many."""
+        n = logits.shape[0]
+        if n > ops.SAMPLE_CALL_ROWS or not logits.is_cuda:
+            return None
+        try:
+            records, draws = b"".join(map(_PACKED, params)), array("Q", counters)
+        except (AttributeError, TypeError, OverflowError):
+            return None
+        if len(records) != _RECORD.size * n:
+            return None
+        while _unread and _unread[0][0].query():
+            try:
+                _unread.pop(0)
+            except IndexError:                       # (another thread's sampler was here first)
+                break
+        hb = self._host_buffer(n)
+        ops.sample_call(logits, records, draws, ids, hb)
+        return PendingTokens(self, hb, n, record_event())
+
     def sample_async(self, logits: torch.Tensor, params: Sequence[SamplingParams], counters: Sequence[int],
                      out: Optional[torch.Tensor] = None) -> PendingTokens:
         """One token for each row of logits [n, vocab] (float32, on the device),
@@ -177,6 +218,9 @@ class Sampler:
         if all(p.greedy for p in params):
             ops.argmax_rows(logits, ids)
         else:
+            pending = self._call(logits, params, counters, ids)
+            if pending is not None:
+                return pending
             host = np.empty((4, n), dtype=np.float32)
             host[0], host[1], seeds, top_k = zip(*map(_OPTIONS, params))
             host[0][~(host[0] > 0)] = 0.0

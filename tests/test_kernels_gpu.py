@@ -1528,6 +1528,30 @@ def test_sample_rows_takes_the_same_ids_where_the_tiles_are_many(ops, vocab):
                 assert _pick_is_right(row, temperature[r], top_k[r], top_p[r], u[r], picks[r], 1e-4), r
 
 
+@pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 128, 129])
+def test_options_in_the_arguments_choose_what_options_in_arrays_choose(ops, n):
+    # sample_async hands options that are packed to the launch itself, up to 128 rows; objects that hold the same numbers unpacked go
+    # the arrays' way.  Several results at a time, one of them never asked for
+    from types import SimpleNamespace
+
+    from litinfer_amd.sampling import Sampler, SamplingParams, sampler
+    sm, g = Sampler(DEV), torch.Generator().manual_seed(19)
+    logits = (torch.randn(n, 5000, generator=g) * 3).to(DEV)
+    params = [SamplingParams(temperature=(0.7, 0.0, 1.2, float("nan"), -1.0)[i % 5], top_k=(0, 5, 50, -3, 6000)[i % 5], top_p=(1.0, 0.9, 2.0)[i % 3],
+                             seed=(i, -i, 2 ** 64 - 1 - i, 2 ** 70 + i)[i % 4]) for i in range(n)]
+    plain = [SimpleNamespace(temperature=p.temperature, top_k=p.top_k, top_p=p.top_p, seed=p.seed, greedy=p.greedy) for p in params]
+    counters = [3 * i for i in range(n)]
+    ids, other = torch.empty(n, dtype=torch.int32, device=DEV), torch.empty(n, dtype=torch.int32, device=DEV)
+    first = sm.sample_async(logits, params, counters, out=ids)
+    sm.sample_async(logits, params, counters)                            # (let go at once)
+    second = sm.sample_async(logits, plain, counters, out=other)
+    third = sm.sample_async(logits * 0.5, params, counters)
+    want = second.result()
+    assert first.result() == want == ids.tolist() == other.tolist()
+    assert third.result() == sm.sample_async(logits * 0.5, plain, counters).result()
+    assert all(e.query() for e, _ in sampler._unread) or len(sampler._unread) <= 1
+
+
 def test_sample_rows_frequencies_and_ties(ops):
     lg = torch.tensor([[2.0, 1.0, 3.0, 3.0, -1.0, 0.5, 2.5, 0.0]])
     n = 4000
