@@ -297,66 +297,67 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
     }
 }
 
-// Merging the splits of a (token, head), in split order.  The weights exp(m_s - m) are
-// computed once per split by the first lanes, then every thread adds up one output
-// dimension with all its loads independent of each other.
+// Merging the splits of a (token, head): MERGE_SHARE splits a group of 128 threads, added in split order, then the groups' sums in
+// theirs.  Every thread asks for all it adds before the weights are known, so that the partial results' way from memory runs beside
+// the weights' way and arithmetic, whatever the number of splits: with one group, that asked for 32 and then for eight at a time, and one lane that added up
+// the weights, 54 splits of 8 x 28 heads took 6.7 us, 20 of 64 x 12 5.0; now 3.6 and 3.8.
 #define MERGE_MAX_SPLITS 64
+#define MERGE_SHARE 16
 
-template <typename T>
-__global__ __launch_bounds__(128) void attention_merge_kernel(
+template <typename T, int GROUPS>
+__global__ __launch_bounds__(128 * GROUPS) void attention_merge_kernel(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml,
     const int* __restrict__ token_list, T* __restrict__ out, int nh, int dh, int nsplit_all,
     const int* __restrict__ nruns = nullptr) {
-    __shared__ float wgt[MERGE_MAX_SPLITS];
-    __shared__ float inv_l;
+    __shared__ float sums[GROUPS > 1 ? GROUPS - 1 : 1][128];
     const int ti = blockIdx.x, head = blockIdx.y;
+    const int lane = threadIdx.x & 63, col = threadIdx.x & 127, group = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);
     const int t = token_list ? token_list[ti] : ti;
     const size_t base = ((size_t)ti * nh + head) * nsplit_all;
-    // nruns: the token's runs that were written (the others of its nsplit_all places hold anything)
-    int nsplit = nsplit_all;
-    if (nruns) {
-        nsplit = nruns[ti];
-        nsplit = nsplit < 1 ? 1 : (nsplit > nsplit_all ? nsplit_all : nsplit);
-    }
-    // The partial results of this thread's first dimension are asked for before the weights
-    // are known (up to 32 splits, all loads at once and never conditional): their way from
-    // memory then runs beside the weights' way and arithmetic, not behind them.
-    constexpr int AHEAD = 32;
-    float pa[AHEAD];
-    const int d0 = threadIdx.x < dh ? threadIdx.x : 0;
-    if (nruns) {                                     // (the number of runs is not known yet: the first place is always written)
+    const int first = group * MERGE_SHARE;
+    for (int d0 = 0; d0 < dh; d0 += 128) {
+        // (never conditional: a split past the last repeats the first, which is always written; its weight is 0)
+        const int d = d0 + col < dh ? d0 + col : dh - 1;
+        float pa[MERGE_SHARE];
 #pragma unroll
-        for (int sp = 0; sp < AHEAD; ++sp) pa[sp] = part_acc[(base + (sp < nsplit_all ? sp : 0)) * dh + d0];
-    } else {
-#pragma unroll
-        for (int sp = 0; sp < AHEAD; ++sp) pa[sp] = part_acc[(base + (sp < nsplit ? sp : nsplit - 1)) * dh + d0];
-    }
-    if (threadIdx.x < 64) {
-        const int sp = threadIdx.x;
-        const float ms = sp < nsplit ? part_ml[(base + sp) * 2] : -INFINITY;
-        const float ls = sp < nsplit ? part_ml[(base + sp) * 2 + 1] : 0.f;
-        const float mx = wave_max(ms);
-        const float f = (mx == -INFINITY) ? 0.f : expf(ms - mx);
-        if (sp < nsplit) wgt[sp] = f;
-        // the sum over splits in split order (one lane adds them up: at most 64 terms)
-        float lt = 0.f;
-        for (int i = 0; i < nsplit; ++i) lt += __shfl(ls * f, i, LI_WAVE);
-        if (sp == 0) inv_l = lt != 0.f ? 1.0f / lt : 0.f;
-    }
-    __syncthreads();
-    for (int d = threadIdx.x; d < dh; d += 128) {
-        float at = 0.f;
-        if (d == d0) {                               // (the same order of additions as below)
-#pragma unroll
-            for (int sp = 0; sp < AHEAD; ++sp) at += sp < nsplit ? pa[sp] * wgt[sp] : 0.f;
-#pragma unroll 8
-            for (int sp = AHEAD; sp < nsplit; ++sp) at += part_acc[(base + sp) * dh + d] * wgt[sp];
-        } else {
-#pragma unroll 8
-            for (int sp = 0; sp < nsplit; ++sp) at += part_acc[(base + sp) * dh + d] * wgt[sp];
+        for (int i = 0; i < MERGE_SHARE; ++i) pa[i] = part_acc[(base + (first + i < nsplit_all ? first + i : 0)) * dh + d];
+        // every wave works out the weights exp(m_s - m) for itself, lane s split s
+        const int own = lane < nsplit_all ? lane : 0;
+        float ms = part_ml[(base + own) * 2], ls = part_ml[(base + own) * 2 + 1];
+        // nruns: the token's runs that were written (the others of its nsplit_all places hold anything)
+        int nsplit = nsplit_all;
+        if (nruns) {
+            nsplit = nruns[ti];
+            nsplit = nsplit < 1 ? 1 : (nsplit > nsplit_all ? nsplit_all : nsplit);
         }
-        store_from_float(out + (size_t)t * nh * dh + (size_t)head * dh + d, at * inv_l);
+        ms = lane < nsplit ? ms : -INFINITY;
+        const float mx = wave_max(ms);
+        const float w = (mx == -INFINITY || lane >= nsplit) ? 0.f : expf(ms - mx);
+        const float lt = wave_sum(lane < nsplit ? ls * w : 0.f);
+        float at = 0.f;
+#pragma unroll
+        for (int i = 0; i < MERGE_SHARE; ++i) {
+            const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), first + i));
+            at += first + i < nsplit ? pa[i] * wi : 0.f;
+        }
+        if constexpr (GROUPS > 1) {
+            if (d0) __syncthreads();
+            if (group) sums[group - 1][col] = at;
+            __syncthreads();
+            if (group) continue;
+#pragma unroll
+            for (int g = 1; g < GROUPS; ++g) at += sums[g - 1][col];
+        }
+        if (d0 + col < dh) store_from_float(out + (size_t)t * nh * dh + (size_t)head * dh + d, lt != 0.f ? at * (1.0f / lt) : 0.f);
     }
+}
+template <typename T>
+static void launch_merge(const float* part_acc, const float* part_ml, const int* token_list, T* out, int n_tokens, int nh, int dh, int nsplit, const int* nruns,
+                         hipStream_t stream) {
+    const dim3 grid(n_tokens, nh);
+    if (nsplit <= MERGE_SHARE) attention_merge_kernel<T, 1><<<grid, 128, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
+    else if (nsplit <= 2 * MERGE_SHARE) attention_merge_kernel<T, 2><<<grid, 256, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
+    else attention_merge_kernel<T, 4><<<grid, 512, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
 }
 
 // The same for the runs of a prompt portion's keys, whose tokens are many: a block takes four heads of a
@@ -453,26 +454,6 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-
-// Stores and loads that other compute units' blocks of the SAME kernel can rely on: they go through to
-// memory (each of the chip's eight L2 caches serves its own compute units only, and ordinary stores may
-// stay in the writer's).  A device-wide fence would do the same for ordinary accesses, but it writes back
-// and invalidates a whole L2 every time: with hundreds of blocks doing so a decode attention took 27 us more.
-__device__ __forceinline__ void store_through(float* p, float v) {
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ float load_through(const float* p) {
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// two floats that lie side by side (8-byte aligned), in one load
-__device__ __forceinline__ void load_through2(const float* p, float& a, float& b) {
-    const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-    a = __uint_as_float((unsigned)(v & 0xffffffffull));
-    b = __uint_as_float((unsigned)(v >> 32));
-}
-// all of this wave's loads and stores have been carried out (stores: have arrived where they go)
-#define LI_WAIT_ALL_VMEM() __builtin_amdgcn_s_waitcnt(0x0F70)
 
 #define DEC_TABLE_CAP 1024      // pages of one split that fit the kernel's copy of the block table
 
@@ -595,21 +576,16 @@ extern "C" int li_decode_run_keys(const int* token_list, int n_tokens, const int
     return li_launch_status();
 }
 
-// WAVES is 1 or 4.  With four, a block takes four runs of the keys of its (token, kv head) that follow each
-// other, one a wave (a wave works alone through its run: no barrier in the loop, the runs' lengths may differ),
-// and joins their results in LDS, in the order of the runs; `nsplit` then counts such blocks ("quads") and is
-// the number of partial results a (token, head) has in part_acc / part_ml.  With one quad the block writes
-// the output itself.  With more, the block that finishes last for a (token, kv head) joins the quads'
-// results in quad order and writes the output, so that no second kernel is needed: every block adds 1 to
-// `done[token * nkv + kv head]` after its results have been made visible to the device, and the block that
-// finds the count complete sets it back to 0 (the array is zero before the first call and after every
-// call).  Nobody waits for anybody.
+// WAVES is 1 or 4.  With four, a block takes the four runs that a token's keys are cut into, one a wave (a wave works alone through its run: no
+// barrier in the loop, the runs' lengths may differ), and joins their results in LDS, in the order of the runs: no partial results, no second
+// kernel (nsplit is 1 then).  With one, a block is one wave with one of nsplit runs, and attention_merge_kernel joins them.  (Blocks of four that
+// joined several of them by the last one to finish were three trips to memory at the kernel's end: 5 to 11 % slower than single waves and
+// that kernel: 8 requests of 4,096 keys, 28 heads on 4, 20.9 us against 19.7, 32 of 1,000 21.7 / 19.5.)
 template <int WAVES, int DH> struct DecodeJoin {
     float ml[WAVES][16][2];                       // per wave and head of the pass: maximum, sum
     float acc[WAVES][16][DH];                     // per wave and head: the unscaled output
-    int last;
 };
-template <int DH> struct DecodeJoin<1, DH> { int last; };
+template <int DH> struct DecodeJoin<1, DH> { int unused; };
 
 #define DEC_WHOLE_TABLE 64       // pages up to which a wave asks for a request's whole table before it knows the request's length
 
@@ -624,8 +600,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     int max_blocks, const int* __restrict__ token_list, const int* __restrict__ seg_of_token,
     const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len,
     float* __restrict__ part_acc, float* __restrict__ part_ml, int nh, int nkv, int page_size,
-    int num_pages, int window, float scale, int nsplit, const int* __restrict__ run_keys, int n_list,
-    int* __restrict__ done) {
+    int num_pages, int window, float scale, int nsplit, const int* __restrict__ run_keys, int n_list) {
     static_assert(DH <= ATT_MAX_DH / 2, "the join buffer holds head sizes up to 128");
     constexpr bool F32 = sizeof(T) == 4;        // float32: v_mfma_f32_16x16x4f32 on float32 operands
     constexpr int KS = DH / 32;                 // bfloat16: MFMA steps of Q K^T
@@ -644,23 +619,18 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     T* p_lds = p_lds_all[wave];
     int* pages = pages_all[wave];
     const int nruns_all = nsplit * WAVES;       // runs that the keys are cut into at most
-    // run_keys given: block x takes the x-th item of the list behind it, a (token, first run) pair, and ends
+    // run_keys given (single waves): block x takes the x-th item of the list behind it, a (token, run) pair, and ends
     // at once if the list is shorter (blocks go to the XCDs in turn, in the order of their numbers, so every
-    // XCD gets its share of the runs that have keys).  Else block (token, kv head, quad) of the grid.
-    int ti = blockIdx.x, quad = blockIdx.z;
+    // XCD gets its share of the runs that have keys).  Else block (token, kv head, run) of the grid.
+    int ti = blockIdx.x, split = WAVES > 1 ? wave : blockIdx.z;
     const int kvh = blockIdx.y;
-    int quads_of_token = nsplit;
-    if (run_keys) {
+    if (WAVES == 1 && run_keys) {
         const int count = run_keys[1];
         const int item = run_keys[2 + n_list + blockIdx.x];
         if ((int)blockIdx.x >= count) return;
         ti = item & 0xffff;
-        quad = (item >> 16) / WAVES;
-        const int nr = run_keys[2 + ti];
-        quads_of_token = (nr + WAVES - 1) / WAVES;
-        quads_of_token = quads_of_token < 1 ? 1 : (quads_of_token > nsplit ? nsplit : quads_of_token);
+        split = item >> 16;
     }
-    const int split = quad * WAVES + wave;
     const int t = token_list ? token_list[ti] : ti;
     const int G = nh / nkv;
     const int lane = threadIdx.x & 63, g = lane >> 4, c = lane & 15;
@@ -676,7 +646,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     const int nkeys = p - lo + 1;
     // (the quotient as below in row_of: exact, the keys and the 64 runs at most being fewer than 2^22)
     int per = ((int)(((float)(nkeys + nruns_all - 1) + 0.5f) * (1.0f / (float)nruns_all)) + 31) & ~31;
-    if (run_keys) {
+    if (WAVES == 1 && run_keys) {
         // one run length for the whole batch (decode_run_keys_kernel): never shorter than this token's keys
         // need to fit the runs, never longer than the runs the host sized the page table in LDS for
         long widest = (long)max_blocks * page_size;
@@ -981,70 +951,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
                     at += join.acc[w][hr][d] * f;
                 }
                 const int head = kvh * G + h0 + hr;
-                if (nsplit == 1) {
-                    store_from_float(out + (size_t)t * nh * DH + (size_t)head * DH + d, lt != 0.f ? at / lt : 0.f);
-                } else {
-                    const size_t pi = ((size_t)ti * nh + head) * nsplit + quad;
-                    store_through(&part_acc[pi * DH + d], at);
-                    if (d == 0) { store_through(&part_ml[pi * 2], mx); store_through(&part_ml[pi * 2 + 1], lt); }
-                }
-            }
-        }
-    }
-    if constexpr (WAVES > 1) {
-        if (nsplit > 1 && done) {
-            // ---- the quads of this (token, kv head): the block that finishes last joins them, in quad order.
-            // The partial results were stored through to memory; once every thread's stores have arrived,
-            // the block counts itself (an atomic carried out in memory), and the block that completes the
-            // count reads the others' results from memory, past its own L2.
-            LI_WAIT_ALL_VMEM();
-            __syncthreads();
-            if (threadIdx.x == 0) {
-                const int before = atomicAdd(&done[ti * nkv + kvh], 1);
-                join.last = before == quads_of_token - 1;
-                if (join.last) atomicExch(&done[ti * nkv + kvh], 0);   // as the next call expects it
-            }
-            __syncthreads();
-            if (!join.last) return;
-            // A thread takes four neighbouring dimensions of one head and asks for everything it needs of all
-            // quads at once, never conditionally (a quad or head past the last repeats the last): one trip to
-            // memory for the whole join.
-            constexpr int TPH = DH / 4, HPC = 64 * WAVES / TPH;        // threads a head, heads a chunk of the block
-            for (int hb = 0; hb < G; hb += HPC) {
-                const int hg_own = hb + (int)threadIdx.x / TPH, hg = hg_own < G ? hg_own : G - 1;
-                const int d = 4 * ((int)threadIdx.x % TPH);
-                const int head = kvh * G + hg;
-                const size_t base = ((size_t)ti * nh + head) * nsplit;
-                float mq[16], lq[16], aq[16][4];                   // (quads <= MERGE_MAX_SPLITS / WAVES = 16)
-#pragma unroll
-                for (int qd = 0; qd < 16; ++qd) {
-                    const int q_ = qd < quads_of_token ? qd : quads_of_token - 1;
-                    load_through2(&part_ml[(base + q_) * 2], mq[qd], lq[qd]);
-                    load_through2(&part_acc[(base + q_) * DH + d], aq[qd][0], aq[qd][1]);
-                    load_through2(&part_acc[(base + q_) * DH + d + 2], aq[qd][2], aq[qd][3]);
-                }
-                float mx = -INFINITY;
-#pragma unroll
-                for (int qd = 0; qd < 16; ++qd) mx = fmaxf(mx, mq[qd]);
-                float lt = 0.f, at[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                for (int qd = 0; qd < 16; ++qd) {
-                    const float f = (qd < quads_of_token && mx != -INFINITY) ? expf(mq[qd] - mx) : 0.f;
-                    lt += lq[qd] * f;
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) at[i] += aq[qd][i] * f;
-                }
-                if (hg_own < G) {
-                    const float inv = lt != 0.f ? 1.0f / lt : 0.f;
-                    T* dst = out + (size_t)t * nh * DH + (size_t)head * DH + d;
-                    if constexpr (F32) {
-                        *reinterpret_cast<f32x4_t*>(dst) = f32x4_t{at[0] * inv, at[1] * inv, at[2] * inv, at[3] * inv};
-                    } else {
-                        uint32_t* dw = reinterpret_cast<uint32_t*>(dst);
-                        dw[0] = pack2_bf16(at[0] * inv, at[1] * inv);
-                        dw[1] = pack2_bf16(at[2] * inv, at[3] * inv);
-                    }
-                }
+                store_from_float(out + (size_t)t * nh * DH + (size_t)head * DH + d, lt != 0.f ? at / lt : 0.f);
             }
         }
     }
@@ -2457,23 +2364,21 @@ static int launch_decode(const T* q, int q_row_stride, T* out, const T* kc, cons
     }
 #undef LI_DEC
     if (nsplit > 1) {
-        dim3 g2(n_tokens, nh);
-        attention_merge_kernel<T><<<g2, 128, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit);
+        launch_merge(part_acc, part_ml, token_list, out, n_tokens, nh, dh, nsplit, nullptr, stream);
     }
     return li_launch_status();
 }
 
 // The matrix-core decode kernel (bfloat16 or float32, head sizes 64 and 128), in its three forms: one run a
-// (token, kv head); single-wave blocks with the merge kernel behind them (use_mfma 2); blocks of LI_DECODE_QUAD
-// waves that join their runs themselves.
+// (token, kv head); single-wave blocks with the merge kernel behind them (use_mfma 2); one block of LI_DECODE_QUAD
+// waves, which joins its runs itself.
 #define LI_DECODE_QUAD 4
 template <typename T>
 static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc, const T* vc, const int* block_table,
                               int max_blocks, const int* token_list, int n_tokens, const int* seg_of_token,
                               const int* q_start, const int* q_len, const int* ctx_len, float* part_acc,
                               float* part_ml, int nh, int nkv, int dh, int page_size, int num_pages, int window,
-                              float scale, int nsplit, int use_mfma, const int* run_keys, int* done,
-                              hipStream_t stream) {
+                              float scale, int nsplit, int use_mfma, const int* run_keys, hipStream_t stream) {
     if (nkv > 65535) return LI_ERR_SIZE;
     // a split's pages must fit the kernel's copy of the block table: `per` keys that begin
     // anywhere in a page touch at most (per + page_size - 2) / page_size + 1 pages
@@ -2481,11 +2386,11 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
     if (dh != 128 && dh != 64) return LI_ERR_SIZE;
     if ((long)max_blocks * page_size > (1L << 21) || page_size > (1 << 16)) return LI_ERR_SIZE;   // (the kernel's key / page_size)
     const bool aligned = window <= 0 && page_size % 8 == 0;
-    const bool listed = run_keys != nullptr && nsplit > 1;
+    const bool listed = run_keys != nullptr && nsplit > 1 && use_mfma == 2;
     if (listed && (n_tokens > RUN_KEYS_MAX_TOKENS || nsplit > 0x7fff)) return LI_ERR_SIZE;
 #define LI_DM4(DHV, W, AL, BLOCKS) paged_attention_decode_mfma_kernel<T, DHV, W, AL><<<grid, 64 * W, 0, stream>>>( \
         q, q_row_stride, out, kc, vc, block_table, max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, \
-        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, BLOCKS, listed ? run_keys : nullptr, n_tokens, done)
+        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, BLOCKS, listed ? run_keys : nullptr, n_tokens)
 #define LI_DM(W, BLOCKS)                                                                                     \
     {                                                                                                        \
         if (dh == 128) { if (aligned) LI_DM4(128, W, true, BLOCKS); else LI_DM4(128, W, false, BLOCKS); }    \
@@ -2500,17 +2405,12 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
         if (!part_acc || !part_ml) return LI_ERR_SIZE;
         const dim3 grid(listed ? n_tokens * nsplit : n_tokens, nkv, listed ? 1 : nsplit);
         LI_DM(1, nsplit)
-        dim3 g2(n_tokens, nh);
-        attention_merge_kernel<T><<<g2, 128, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit,
-                                                          listed ? run_keys + 2 : nullptr);
+        launch_merge(part_acc, part_ml, token_list, out, n_tokens, nh, dh, nsplit, listed ? run_keys + 2 : nullptr, stream);
         return li_launch_status();
     }
-    if (nsplit % LI_DECODE_QUAD) return LI_ERR_SIZE;
-    const int quads = nsplit / LI_DECODE_QUAD;
-    if (quads > 1 && (!done || !part_acc || !part_ml)) return LI_ERR_SIZE;
-    if ((long)n_tokens * quads > 0x7fffffffL) return LI_ERR_SIZE;
-    const dim3 grid(listed ? n_tokens * quads : n_tokens, nkv, listed ? 1 : quads);
-    LI_DM(LI_DECODE_QUAD, quads)
+    if (nsplit != LI_DECODE_QUAD) return LI_ERR_SIZE;
+    const dim3 grid(n_tokens, nkv, 1);
+    LI_DM(LI_DECODE_QUAD, 1)
 #undef LI_DM
 #undef LI_DM4
     return li_launch_status();
@@ -2518,11 +2418,10 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
 
 // Single-query tokens of the batch (token_list, or all tokens when it is null).
 // part_acc: float [n_tokens, nh, nsplit, dh]; part_ml: float [n_tokens, nh, nsplit, 2] (unused when nsplit is 1).
-// run_keys (may be null; the matrix-core kernel with nsplit > 1 only): what li_decode_run_keys (with group
-// LI_DECODE_QUAD) left on the device for this batch: the run length and the list of the runs that have keys.
-// The matrix-core kernel with nsplit > 1 takes nsplit as a multiple of LI_DECODE_QUAD (a block works through
-// that many runs and joins them) and needs `done`: int [n_tokens * nkv], zero before the first call; every
-// call leaves it zero.  Its blocks join their results themselves; the other kernels run a merge kernel.
+// run_keys (may be null; the matrix-core kernel's single waves only): what li_decode_run_keys left on the device for this batch: the run
+// length and the list of the runs that have keys.
+// use_mfma: 0 the vector kernel; 1 the matrix-core kernel with nsplit 1 or LI_DECODE_QUAD, whose blocks write the output; 2 its single waves,
+// whose nsplit runs the merge kernel joins, as it does the vector kernel's.
 extern "C" int li_decode_quad(void) { return LI_DECODE_QUAD; }
 extern "C" int li_paged_attention_decode(const void* q, int q_row_stride, void* out, const void* kc,
                                          const void* vc, int dtype, const int* block_table, int max_blocks,
@@ -2530,7 +2429,7 @@ extern "C" int li_paged_attention_decode(const void* q, int q_row_stride, void* 
                                          const int* q_start, const int* q_len, const int* ctx_len,
                                          float* part_acc, float* part_ml, int nh, int nkv, int dh,
                                          int page_size, int num_pages, int window, float scale, int nsplit,
-                                         int use_mfma, const int* run_keys, int* done, hipStream_t stream) {
+                                         int use_mfma, const int* run_keys, hipStream_t stream) {
     if (n_tokens <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || dh <= 0 || dh > ATT_MAX_DH || page_size <= 0 ||
         max_blocks <= 0)
         return LI_ERR_SIZE;
@@ -2544,12 +2443,12 @@ extern "C" int li_paged_attention_decode(const void* q, int q_row_stride, void* 
         return launch_decode_mfma<float>((const float*)q, q_row_stride, (float*)out, (const float*)kc, (const float*)vc,
                                          block_table, max_blocks, token_list, n_tokens, seg_of_token, q_start, q_len,
                                          ctx_len, part_acc, part_ml, nh, nkv, dh, page_size, num_pages, window, scale,
-                                         nsplit, use_mfma, run_keys, done, stream);
+                                         nsplit, use_mfma, run_keys, stream);
     if (dtype == LI_BF16 && use_mfma)
         return launch_decode_mfma<bf16_t>((const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc,
                                           (const bf16_t*)vc, block_table, max_blocks, token_list, n_tokens, seg_of_token,
                                           q_start, q_len, ctx_len, part_acc, part_ml, nh, nkv, dh, page_size, num_pages,
-                                          window, scale, nsplit, use_mfma, run_keys, done, stream);
+                                          window, scale, nsplit, use_mfma, run_keys, stream);
     if (dtype == LI_BF16)
         return launch_decode<bf16_t>((const bf16_t*)q, q_row_stride, (bf16_t*)out, (const bf16_t*)kc,
                                      (const bf16_t*)vc, block_table, max_blocks, token_list, n_tokens,

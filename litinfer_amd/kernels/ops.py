@@ -103,7 +103,7 @@ _SIGNATURES = {
         "li_paged_attention": [P, I, P, P, P, I, P, I, P, P, P, P, P, I, I, I, I, I, I, I, I, I, I, F],
         "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I, I, I],
         "li_paged_attention_prefill_f32": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I],
-        "li_paged_attention_decode": [P, I, P, P, P, I, P, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, P],
+        "li_paged_attention_decode": [P, I, P, P, P, I, P, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P],
         "li_decode_run_keys": [P, I, P, P, P, P, I, I, I, I, I, I, I, P],
     },
     "sampling": {
@@ -1461,8 +1461,7 @@ def linear_rope_store_parts(x: torch.Tensor, w: torch.Tensor, bias: Optional[tor
 
 
 # ----------------------------------------------------------------- attention
-# waves that the split-key decode kernel on the matrix cores is cut into at least (where the keys allow):
-# four a compute unit; more splits cost more in the merge than they gain (measured at 8 and 64 requests)
+# waves that the split-key decode kernel on the matrix cores is cut into at least (where the keys allow): four a compute unit
 _DEC_WAVES = 1024
 PREFILL_TILE_ROWS = 32       # queries of one segment that a block of the matrix-core kernel for portions takes
 DECODE_MAX_SPLITS = 64       # the merge kernel keeps a weight per split
@@ -1481,17 +1480,7 @@ def _simd_count(device: torch.device) -> int:
     return _simds[i]
 
 
-DECODE_QUAD = 4              # runs of a token's keys that one block of the matrix-core decode kernel takes, one a wave
-# measurements only: single-wave blocks and a merge kernel behind them, as before the blocks joined their runs
-_decode_single_waves = False
-# Share of the SIMDs that a step's waves must fill for the blocks of four waves (below).  Most batch sizes give a
-# number of runs whose waves fill the SIMDs nearly, not wholly (17 requests x 2 kv heads x 28 runs = 952 of
-# 1,024); asked for all of them, those took single-wave blocks and the merge kernel: 17 / 24 / 28 requests of
-# 4,096 keys at the 1.5B head layout 23.5 / 29.4 / 31.5 us a layer against 21.8 / 26.9 / 29.9 with the blocks of
-# four (7B layout, 28 requests: 53.6 against 50.0); from a half on the short contexts lose (17.0 against 16.0 us).
-_DECODE_FILLS = 0.7
-
-
+DECODE_QUAD = 4              # runs of a token's keys that one block of the matrix-core decode kernel takes, one a wave, and joins itself
 
 
 def _seg_of_token(meta, takes: bool = True) -> int:
@@ -1507,8 +1496,55 @@ def _seg_of_token(meta, takes: bool = True) -> int:
     return 0 if in_order else meta.seg_of_token.data_ptr()
 
 
+def _one_block(pairs: int, keys: int, dh: int, simds: int) -> bool:
+    """Whether a block of DECODE_QUAD waves takes all of a (token, kv head)'s keys and joins its runs itself, rather than runs of single waves and the
+    kernel that joins them (bfloat16, up to 512 pairs, the kernel's quicker form).  Four waves sit on one compute unit, so it pays where the
+    pairs fill the chip with a block each, or nearly, and where the keys are too few for the second kernel.  Us a call, one block against
+    single runs, contexts all as long as the table, three quarters of it, spread from an eighth of it on.  12 heads on 2 of 128, 64 pairs: tables of 256 keys 8.8 / 8.1, 7.8 / 7.8,
+    8.1 / 8.1, 512 11.7 / 9.8, 9.8 / 9.3, 11.2 / 9.8; 128 pairs: 384 10.4 / 11.5, 9.2 / 10.4, 9.8 / 10.5, 512 13.9 / 12.7, 10.4 / 11.0, 11.6 / 11.8, 768 18.1 / 15.7, 13.2 / 13.4,
+    14.7 / 13.5; 160: 1,024 21.9 / 24.2, 17.2 / 18.5, 18.2 / 18.2, 2,048 37.6 / 38.7, 29.9 / 30.9, 32.2 / 29.0; 200: 2,048 42.7 / 46.1, 33.5 / 37.2, 34.3 / 35.0; 256: 52.8 /
+    56.5, 41.5 / 45.3, 37.9 / 41.0; 320: 512 24.0 / 23.5, 18.8 / 19.2, 18.4 / 19.4, 1,024 41.6 / 39.7, 33.1 / 31.6, 31.1 / 30.2; 512: 1,024 54.3 / 58.1, 41.9 / 46.3, 39.5 / 46.1.  Heads
+    of 64, 14 on 2, 2 pairs: 256 5.4 / 5.3, 4.8 / 5.3, 384 6.1 / 5.4, 5.8 / 5.4; 8: 384 6.3 / 6.1, 5.9 / 5.9, 6.1 / 6.1, 512 7.3 / 6.7; 64: 512 8.6 / 8.5, 7.2 / 8.1, 7.9 / 8.3, 768
+    10.4 / 9.2, 9.2 / 8.9, 10.1 / 9.2; 96: 768 10.7 / 11.1, 9.3 / 9.9, 10.2 / 9.8, 1,024 12.6 / 11.8; 160: 1,024 13.7 / 15.7, 11.4 / 13.2, 12.4 / 12.7, 1,536 20.2 / 19.3, 14.9 /
+    16.2, 16.7 / 15.5; 200 and more 5 to 30 % faster in one block up to 2,048 keys; 320: 1,024 23.9 / 24.4, 18.4 / 19.9, 17.9 / 19.3, 2,048 41.5 / 40.3."""
+    if keys <= 128:
+        return False
+    room = simds // DECODE_QUAD                     # blocks that the chip takes at one time
+    if 4 * pairs >= 3 * room * -(-pairs // room):
+        return True
+    if pairs > room:
+        return keys <= (640 if dh == 128 else 1024)
+    if dh == 128:
+        return keys <= max(4 * pairs, 16 * (pairs - 96))
+    return keys <= (min(512, 256 + 16 * pairs) if pairs <= 64 else 256 + 5 * pairs)
+
+
+def _decode_cut(pairs: int, keys: int, dh: int, dtype: torch.dtype, simds: int, aligned: bool, meta, window: int):
+    """(runs that each token's keys are cut into, waves a block, runs if all contexts were as long as the longest) for the matrix-core decode kernel.
+    One block a (token, kv head) by `_one_block`, or by `_short_runs` where that was measured instead; else single waves, their runs of 128 keys at
+    least, or of 32 (64 where contexts differ) and to a finer cut where the pairs are few: the kernel that joins runs asks for all of
+    them at once, so that a run costs it little.  Us a call, runs of 128 and the coarser cut / so: 2 pairs, 12 heads on 2 of 128, tables of 512, 1,024 and 4,096 keys
+    8.2 / 6.7, 8.5 / 6.8, 9.5 / 8.4; 8 pairs 8.5 / 7.0, 8.8 / 7.0, 10.7 / 10.5; 32 pairs 9.7 / 8.3, 10.1 / 9.5, at 2,048 12.5 / 13.2 (so not there); heads of 64, 32
+    pairs, 2,048 10.3 / 9.9; float32, 2 pairs 15.6 / 10.5, 15.5 / 8.4, 18.0 / 12.6; 32 pairs 17.4 / 12.4, 18.6 / 13.6, heads of 64 at 2,048 14.3 / 13.8."""
+    bf16 = dtype is torch.bfloat16
+    differ = _ragged_splits(1, meta, window, 1) > 1
+    planned = decode_splits(pairs, keys, simds)
+    measured = bf16 and aligned and pairs <= 512
+    few = pairs * keys <= (65536 if dh == 64 else 32768) and keys > (128 if bf16 else 96)
+    if measured:
+        runs = DECODE_QUAD if _one_block(pairs, keys, dh, simds) else (32, 64) if few else (128,)
+    else:
+        runs = _short_runs(pairs, keys, dh, dtype, DECODE_QUAD if planned == DECODE_QUAD and not differ else 0, aligned, differ)
+        if runs is None:
+            runs = DECODE_QUAD if planned == DECODE_QUAD and not differ else (32, 64) if few and pairs <= 32 and not bf16 else (128,)
+    if runs == DECODE_QUAD:
+        return DECODE_QUAD, DECODE_QUAD, DECODE_QUAD
+    planned = decode_splits(pairs, keys, simds, 1, runs[-1] if differ else runs[0], 1 if few and pairs <= 32 else 4)
+    return _ragged_splits(planned, meta, window, 1), 1, planned
+
+
 def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, aligned: bool = True, differ: bool = True):
-    """Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of
+    """Asked for float32, for more than 512 pairs, and for a window or pages of no multiple of 8 keys (else: `_one_block`).  Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of
     four runs a (token, kv head), which joins them itself and needs no list of runs; a pair of least lengths, runs of their own and the
     kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan; `aligned`: no window and
     pages of a multiple of 8 keys (the kernel's quicker form); `differ`: the contexts do, by `_ragged_splits`.
@@ -1549,19 +1585,18 @@ def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, 
     return (32, 64) if 96 < keys <= most else None
 
 
-def decode_splits(pairs: int, keys: int, simds: int = _DEC_WAVES, quad: int = DECODE_QUAD, least: int = 128) -> int:
+def decode_splits(pairs: int, keys: int, simds: int = _DEC_WAVES, quad: int = DECODE_QUAD, least: int = 128, join: int = 4) -> int:
     """Into how many runs the keys of a decoding token are cut.  Every (token, kv head) pair and
     run is one wave, and a SIMD holds one wave of this kernel: the waves go over the SIMDs in
     rounds, each as long as a run (plus a wave's start and end, about 24 keys' time), so the
     number of runs with the least rounds x run length is taken, a run being a multiple of 32
-    keys and at least 128 where the keys allow; every run costs the join a little (4 keys' time).
-    The runs come in blocks of `quad` waves (a block joins its runs itself), so their number is 1
-    or a multiple of `quad`.  Few pairs: as many runs as fill the SIMDs once."""
+    keys and at least `least` where the keys allow; every run costs the join a little (`join` keys' time).
+    The runs' number is 1 or a multiple of `quad`.  Few pairs: as many runs as fill the SIMDs once."""
     most = max(1, min(-(-keys // least), DECODE_MAX_SPLITS))
     best, best_cost = 1, None
     for ns in [1] + list(range(quad, most + 1, quad)):
         run = (-(-keys // ns) + 31) & ~31
-        cost = -(-pairs * ns // simds) * (run + 24) + 4 * ns
+        cost = -(-pairs * ns // simds) * (run + 24) + join * ns
         if best_cost is None or cost < best_cost:
             best, best_cost = ns, cost
     return best
@@ -1663,48 +1698,17 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
             _chk(meta.max_blocks * page_size <= 1 << 21 and page_size <= 1 << 16,
                  f"attention: block tables of {meta.max_blocks} pages of {page_size} keys are beyond the decode "
                  f"kernel's {1 << 21} keys")
-            # Blocks of four waves that join their runs themselves, or single-wave blocks and a merge kernel
-            # behind them.  Four waves sit on ONE compute unit and the join is three trips to memory at the
-            # kernel's end: it pays where one block holds all runs of a (token, kv head) (no join, no second
-            # kernel: 64 requests at the 7B head layout 105 -> 96 us a layer), and where the waves fill the
-            # chip anyway and the runs are not many or long (8 requests, 4,096 keys: 22.3 -> 21.6 us; 8
-            # requests of the 1.5B layout with 64 short runs each: 17.3 -> 18.9 us, so not there).  Not for
-            # contexts that differ (one run length for the batch and a list of the runs that have keys): a
-            # token's runs then fill its last block of four only partly, and a block's waves end at different
-            # times (64 requests with 16 to 4,600 keys, 7B head layout: 73.8 us against 82.7; 1.5B: 41.3 / 52.5).
-            simds = _simd_count(qkv.device)
-            quad = DECODE_QUAD
-            planned = decode_splits(n_single * nkv, keys, simds, quad)
-            nsplit = _ragged_splits(planned, meta, window)
-            fills = n_single * nkv * nsplit >= _DECODE_FILLS * simds
-            if (_decode_single_waves or nsplit > planned
-                    or not (nsplit == DECODE_QUAD or (fills and (nsplit <= 32 or keys >= 8192)))):
-                quad = 1
-                planned = decode_splits(n_single * nkv, keys, simds, quad)
-                nsplit = _ragged_splits(planned, meta, window, quad)
-            runs = None if _decode_single_waves else _short_runs(
-                n_single * nkv, keys, dh, qkv.dtype, nsplit if quad > 1 else 0, window <= 0 and page_size % 8 == 0,
-                nsplit > planned)
-            if runs == DECODE_QUAD:
-                quad = nsplit = planned = DECODE_QUAD
-            elif runs is not None:
-                quad = 1
-                for least in runs:                     # (contexts that differ: the longer runs, the second number)
-                    planned = decode_splits(n_single * nkv, keys, simds, quad, least)
-                    nsplit = _ragged_splits(planned, meta, window, quad)
-                    if nsplit == planned:
-                        break
+            nsplit, quad, planned = _decode_cut(n_single * nkv, keys, dh, qkv.dtype, _simd_count(qkv.device), window <= 0 and page_size % 8 == 0,
+                                                meta, window)
             # a split's pages must fit the kernel's copy of the block table
             while nsplit <= DECODE_MAX_SPLITS and decode_split_blocks(meta.max_blocks, page_size, window, nsplit) > DECODE_TABLE_CAP:
-                nsplit += 1 if nsplit < quad else quad
-            if 1 < nsplit < quad:
-                nsplit = quad
+                nsplit, quad = nsplit + 1, 1
             _chk(nsplit <= DECODE_MAX_SPLITS, f"attention: block tables of {meta.max_blocks} pages of {page_size} "
                                               f"are too long for the decode kernel")
         else:
             nsplit = max(1, min(-(-512 // (n_single * nkv)), -(-keys // 256), DECODE_MAX_SPLITS))
         acc = ml = None
-        if nsplit > 1:
+        if nsplit > 1 and (not mfma or quad == 1):
             shape_a, shape_m = (n_single, nh, nsplit, dh), (n_single, nh, nsplit, 2)
             if ws is not None:
                 acc = ws.buffer("attn.part_acc", shape_a, torch.float32)
@@ -1713,12 +1717,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
                 acc = torch.empty(shape_a, dtype=torch.float32, device=qkv.device)
                 ml = torch.empty(shape_m, dtype=torch.float32, device=qkv.device)
         lst = meta.single_tokens if n_single < t else None
-        run_keys = done = None
-        if mfma and nsplit > DECODE_QUAD and quad > 1:
-            # the blocks of a (token, kv head) count themselves here, and the last one joins their results
-            # (zero before the first call; every call leaves it zero)
-            done = (ws.buffer("attn.done", (n_single * nkv,), torch.int32, zero=True) if ws is not None
-                    else torch.zeros(n_single * nkv, dtype=torch.int32, device=qkv.device))
+        run_keys = None
         if mfma and nsplit > planned and n_single <= DECODE_LIST_MAX_TOKENS:
             # contexts that differ: one run length for the batch and the list of the runs that have keys, made
             # on the device from the context lengths, once a step for all layers with these numbers (a
@@ -1732,8 +1731,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
                 size = 2 + n_single + n_single * DECODE_MAX_SPLITS
                 run_keys = (ws.buffer(name, (size,), torch.int32) if ws is not None
                             else torch.empty(size, dtype=torch.int32, device=qkv.device))
-                decode_run_keys(meta, lst, n_single, page_size, window, nkv, nsplit, _simd_count(qkv.device), run_keys,
-                                group=quad)
+                decode_run_keys(meta, lst, n_single, page_size, window, nkv, nsplit, _simd_count(qkv.device), run_keys)
                 meta.extra[key] = run_keys
         _run("attention", "li_paged_attention_decode", qkv.data_ptr(), qkv.stride(0), out.data_ptr(),
              k.data_ptr(), v.data_ptr(), _DT[qkv.dtype], bt.data_ptr(), meta.max_blocks,
@@ -1742,7 +1740,7 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
              0 if acc is None else acc.data_ptr(), 0 if ml is None else ml.data_ptr(),
              nh, nkv, dh, page_size, k.shape[0], int(window), float(scale), nsplit,
              (2 if quad == 1 and nsplit > 1 else 1) if mfma else 0,
-             0 if run_keys is None else run_keys.data_ptr(), 0 if done is None else done.data_ptr())
+             0 if run_keys is None else run_keys.data_ptr())
     # the matrix-core kernel for portions keeps a tile's pages in LDS (8192 entries) and divides
     # positions by the page size in float, exact below 2^21 keys; longer tables take the general kernel
     if (n_multi and qkv.dtype is torch.bfloat16 and dh in (64, 128) and meta.num_tiles

@@ -186,6 +186,29 @@ def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh,
         assert ops._short_runs(pairs, keys, dh, ops.torch.float32, 4) == want, keys
 
 
+@pytest.mark.parametrize("pairs,dh,ends", [(1, 64, 272), (8, 64, 384), (64, 64, 512), (65, 64, 581), (160, 64, 1056), (191, 64, 1211), (192, 64, None), (256, 64, None),
+                                           (257, 64, 1024), (383, 64, 1024), (384, 64, None), (512, 64, None), (32, 128, 0), (64, 128, 256), (128, 128, 512),
+                                           (160, 128, 1024), (192, 128, None), (320, 128, 640)])
+def test_a_block_takes_all_runs_only_where_that_was_measured(pairs, dh, ends):
+    for keys in range(1, 20000, 7):
+        assert ops._one_block(pairs, keys, dh, 1024) == (keys > 128 and (ends is None or keys <= ends)), keys
+
+
+def test_every_decoding_step_is_cut_into_runs_that_the_kernels_take():
+    """One run, one block of four, or up to DECODE_MAX_SPLITS single waves, whatever the step (the first number) and its contexts."""
+    from types import SimpleNamespace
+    for dtype in (ops.torch.bfloat16, ops.torch.float32):
+        for pairs in (1, 2, 8, 31, 64, 65, 150, 192, 256, 320, 512, 513, 1000, 3000):
+            for keys in (1, 32, 96, 97, 128, 129, 256, 500, 1024, 4096, 30000):
+                for dh in (64, 128):
+                    for aligned in (True, False):
+                        for low in (keys, max(1, keys // 8)):
+                            ctx = np.linspace(low, keys, max(2, pairs)).astype(np.int32)
+                            meta = SimpleNamespace(host_q_len=np.ones(len(ctx), np.int32), host_ctx_len=ctx)
+                            ns, waves, planned = ops._decode_cut(pairs, keys, dh, dtype, 1024, aligned, meta, 0)
+                            assert 1 <= planned <= ns <= ops.DECODE_MAX_SPLITS and (waves == 1 or ns == planned == waves == ops.DECODE_QUAD)
+
+
 @pytest.mark.parametrize("pairs,dh,aligned,ends", [(2, 128, True, 384), (32, 128, False, 384), (2, 64, True, 448), (64, 128, True, 640), (512, 64, True, 1280),
                                                    (512, 128, False, 896)])
 def test_bfloat16_decoding_takes_one_block_only_where_that_was_measured(pairs, dh, aligned, ends):

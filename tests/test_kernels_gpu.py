@@ -935,6 +935,26 @@ def test_a_far_key_stands_out_in_a_decode_batch_of_unequal_contexts(ops, far, dt
     assert rel(got, ref) < tol(dtype, 1e-5, 8e-3)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("runs", [2, 16, 17, 32, 33, 64])
+def test_any_number_of_runs_is_joined(ops, monkeypatch, runs, dtype):
+    # sixteen runs a group of the joining kernel's threads, one group, two or four; contexts that are equal, and that leave some of
+    # the runs without keys
+    monkeypatch.setattr(ops, "_decode_cut", lambda *a: (runs, 1, runs))
+    out, ref = _paged_case(ops, dtype, [(64 * 32, 1), (64 * 32, 1)], 6, 2, 64, 16, 0, seed=61, scale_one=777, ws=_Lender())
+    assert rel(out, ref) < tol(dtype, 1e-5, 8e-3)
+    monkeypatch.setattr(ops, "_decode_cut", lambda *a: (runs, 1, 1))
+    out, ref = _paged_case(ops, dtype, [(64 * 32, 1), (70, 1), (1, 1), (1033, 1)], 6, 2, 128, 16, 0, seed=62, ws=_Lender())
+    assert rel(out, ref) < tol(dtype, 1e-5, 8e-3)
+
+
+@pytest.mark.parametrize("dh,ctx", [(256, 16 * 256), (256, 17 * 256), (128 + 64, 33 * 256), (16, 20 * 256)])
+def test_runs_of_the_vector_kernel_are_joined(ops, dh, ctx):
+    for dtype in DTYPES:
+        out, ref = _paged_case(ops, dtype, [(ctx, 1)], 2, 1, dh, 16, 0, seed=63, ws=_Lender())
+        assert rel(out, ref) < tol(dtype, 1e-5, 8e-3)
+
+
 @pytest.mark.parametrize("window", [0, 900])
 def test_decode_run_length_of_a_batch_with_unequal_contexts(ops, window):
     # the run length chosen on the device against the same search written out, for contexts from 3 to 5,000
