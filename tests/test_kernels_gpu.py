@@ -485,6 +485,13 @@ def test_linear_into_the_residual_sum_with_its_norm(ops, m, n, k, bias, taken):
     assert (own.float() - xn.float()).abs().max().item() <= 2.0 ** -7 * own.float().abs().max().item()
 
 
+@pytest.mark.parametrize("m,n,k,bias", [(255, 1536, 1536, True), (256, 1536, 1536, True), (1027, 1536, 1024, False), (300, 512, 8192, True), (700, 896, 1088, False),
+                                        (257, 2052, 2048, True), (256, 4096, 1024, False), (300, 5124, 1024, True), (256, 8192, 1024, False), (300, 1538, 4096, True)])
+def test_parts_of_many_rows_with_their_norm(ops, m, n, k, bias):
+    """From 256 rows on four columns a load: two, three, four and eight parts; one to eight pieces a thread; rows of no multiple of four."""
+    test_linear_into_the_residual_sum_with_its_norm(ops, m, n, k, bias, ops._work_bytes(m, n, k, ops._DT[torch.bfloat16]) > 0)
+
+
 @pytest.mark.parametrize("m,n,k", [
     (8, 200, 96),                # few rows: the decode kernel
     (13, 9500, 128),             # 13 to 64 rows: tiles of 64 rows
