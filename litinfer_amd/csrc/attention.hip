@@ -1250,9 +1250,13 @@ typedef short tr4 __attribute__((ext_vector_type(4)));
 #define LI_ATT_LOAD_TO_LDS(gptr, lptr)                                                                    \
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"                        \
                  :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(gptr) : "memory", "m0")
-// P32: the page size divides 32, so a row keeps its place in its page from block to block
+// (the same with an address that the wave has in common and 32 bits a lane)
+#define LI_ATT_LOAD_AT_TO_LDS(base, place, lptr)                                                          \
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"                        \
+                 :: "s"((uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)(lptr)), "v"(place), "s"(base) : "memory", "m0")
+// P32: the page size divides 32, so a row keeps its place in its page from block to block, and has whole loads of 1 KB
 template <int DH, bool P32, int HEADS>
-__global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_kernel(
+__global__ __launch_bounds__(PRE_WAVES * 64, DH == 64 ? 4 : 2) void paged_attention_prefill_dma_kernel(
     const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __restrict__ out,
     const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc, const int* __restrict__ block_table,
     int max_blocks, const int* __restrict__ tiles, const int* __restrict__ q_start,
@@ -1272,6 +1276,7 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     constexpr int CPR = DH / 8;                 // 16-byte chunks in a row of K
     constexpr int NT = PRE_WAVES * 64;
     constexpr int NST = 3;                      // stages of LDS: one worked on, two on their way
+    constexpr bool AHEAD = DH == 128;           // a block's scores are made a turn ahead of its probabilities (below)
     __shared__ __attribute__((aligned(16))) uint16_t Ks[NST][32 * DH];    // [key][dimension], chunks swizzled by key
     __shared__ __attribute__((aligned(16))) uint16_t Vs[NST][32 * DH];    // the same for V, another swizzle
     __shared__ uint32_t pageoff[PRE2_TABLE_CAP];                          // byte offset / 128 of each page of the tile's part of the table
@@ -1308,10 +1313,9 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     const int nrows = left - (t0 - t00) < 32 ? left - (t0 - t00) : 32;
     const int head = kvh * G + (hw < G ? hw : 0);
     const int ql = lane & 31, h = lane >> 5;
-    const int p00 = ctx_len[s] - seg_rows + (t00 - seg0);               // position of the block's first token,
-    const int p0 = p00 + (t0 - t00), p_last = p0 + nrows - 1;           // of the wave's tile's first and last
-    const int lo0 = (window > 0 && p00 - window + 1 > 0) ? p00 - window + 1 : 0;      // the first key that any of the block's tokens sees,
-    const int lo_tile = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;    // ... the wave's
+    const int p00 = ctx_len[s] - seg_rows + (t00 - seg0);               // position of the block's first token
+    const int p0 = p00 + (t0 - t00), p_last = p0 + nrows - 1;           // of the tile's first and last
+    const int lo0 = (window > 0 && p00 - window + 1 > 0) ? p00 - window + 1 : 0;      // the first key that any of the block's tokens sees
     int k_begin = lo0 & ~31, k_end = p00 + (left < 32 * abreast ? left : 32 * abreast);
     int first_key = lo0;
     if (cuts > 1) {                                     // this run's blocks of 32 keys
@@ -1359,46 +1363,58 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
     constexpr int NL = (32 * CPR) / NT;                 // loads of K (and of V) a thread makes per block
     static_assert(NL * NT == 32 * CPR, "whole load instructions a block of keys");
     int row_blk[NL], row_in[NL], kcol[NL], vcol[NL];
+    uint32_t kplace[NL], vplace[NL];                    // P32: the row's place in its page and its chunk, once and for all
     const char* kbase = reinterpret_cast<const char*>(kc) + (size_t)kvh * page_size * DH * 2;
     const char* vbase = reinterpret_cast<const char*>(vc) + (size_t)kvh * page_size * DH * 2;
-    const char* krow[NL];                               // P32: the row's place in its page and its chunk, once and for all
-    const char* vrow[NL];
 #pragma unroll
     for (int i = 0; i < NL; ++i) {
         const int ci = 64 * (NL * wave + i) + lane, key = ci / CPR, place = ci % CPR;
         kcol[i] = 8 * (place ^ (key & (CPR - 1)));
         vcol[i] = 8 * (place ^ ((2 * (key & 7)) & (CPR - 1)));
         const int kk = k_begin + key;
-        row_blk[i] = kk / page_size - first_block;
+        // (P32: a load's 512 / DH rows lie in one page, so its number and what follows from it are the wave's and kept in scalar registers)
+        row_blk[i] = (P32 ? k_begin + 64 * (NL * wave + i) / CPR : kk) / page_size - first_block;
         row_in[i] = kk % page_size;
-        krow[i] = kbase + (size_t)(row_in[i] * DH + kcol[i]) * 2;
-        vrow[i] = vbase + (size_t)(row_in[i] * DH + vcol[i]) * 2;
+        kplace[i] = (uint32_t)(row_in[i] * DH + kcol[i]) * 2;
+        vplace[i] = (uint32_t)(row_in[i] * DH + vcol[i]) * 2;
     }
     const int step_blk = 32 / page_size, step_in = 32 % page_size;      // a turn moves every row 32 keys on
     const int uwave = __builtin_amdgcn_readfirstlane(wave);
-    // (fetches are made for consecutive blocks: k_begin, k_begin + 32, ...)
-#define LI_PRE_FETCH(stage)                                                                          \
-    {                                                                                                \
-        unsigned long long off_[NL];                                                                 \
-        _Pragma("unroll") for (int i = 0; i < NL; ++i) {                                             \
-            const int ix_ = row_blk[i] < 0 ? 0 : (row_blk[i] > last_entry ? last_entry : row_blk[i]); \
-            off_[i] = (unsigned long long)pageoff[ix_] << 7;                                         \
-        }                                                                                            \
-        _Pragma("unroll") for (int i = 0; i < NL; ++i) {                                             \
-            if constexpr (P32) {                                                                     \
-                row_blk[i] += step_blk;                                                              \
-                LI_ATT_LOAD_TO_LDS(krow[i] + off_[i], &Ks[stage][512 * (NL * uwave + i)]);           \
-                LI_ATT_LOAD_TO_LDS(vrow[i] + off_[i], &Vs[stage][512 * (NL * uwave + i)]);           \
-            } else {                                                                                 \
-                const size_t o_ = off_[i] + (unsigned)(row_in[i] * DH * 2);                          \
-                row_in[i] += step_in;                                                                \
-                row_blk[i] += step_blk;                                                              \
-                if (row_in[i] >= page_size) { row_in[i] -= page_size; row_blk[i] += 1; }             \
-                LI_ATT_LOAD_TO_LDS(kbase + o_ + 2 * kcol[i], &Ks[stage][512 * (NL * uwave + i)]);    \
-                LI_ATT_LOAD_TO_LDS(vbase + o_ + 2 * vcol[i], &Vs[stage][512 * (NL * uwave + i)]);    \
-            }                                                                                        \
-        }                                                                                            \
-    }
+    // Fetches are made for consecutive blocks: k_begin, k_begin + 32, ...  A block's values are asked for a turn behind its keys (below), at
+    // the same places of their cache layer: `held` keeps these.
+    // (a row's page is looked up a turn before it is asked for: `ahead`.  A load's address in scalar registers and 32 bits a lane: as 64-bit
+    // sums in every lane the addresses took a twelfth of the kernel's time)
+    unsigned long long held[NL];
+    uint32_t ahead[NL];
+    auto look_up = [&]() {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) ahead[i] = pageoff[row_blk[i] < 0 ? 0 : (row_blk[i] > last_entry ? last_entry : row_blk[i])];
+    };
+    look_up();
+    auto fetch_k = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            row_blk[i] += step_blk;
+            if constexpr (P32) {
+                held[i] = (unsigned long long)__builtin_amdgcn_readfirstlane(ahead[i]) << 7;
+                LI_ATT_LOAD_AT_TO_LDS(kbase + held[i], kplace[i], &Ks[stage][512 * (NL * uwave + i)]);
+            } else {
+                held[i] = (unsigned long long)ahead[i] << 7;
+                held[i] += (unsigned)(row_in[i] * DH * 2);
+                row_in[i] += step_in;
+                if (row_in[i] >= page_size) { row_in[i] -= page_size; row_blk[i] += 1; }
+                LI_ATT_LOAD_TO_LDS(kbase + held[i] + 2 * kcol[i], &Ks[stage][512 * (NL * uwave + i)]);
+            }
+        }
+        look_up();
+    };
+    auto fetch_v = [&](int stage) {
+#pragma unroll
+        for (int i = 0; i < NL; ++i) {
+            if constexpr (P32) LI_ATT_LOAD_AT_TO_LDS(vbase + held[i], vplace[i], &Vs[stage][512 * (NL * uwave + i)]);
+            else LI_ATT_LOAD_TO_LDS(vbase + held[i] + 2 * vcol[i], &Vs[stage][512 * (NL * uwave + i)]);
+        }
+    };
     // ---- this wave's queries
     frag8 qf[KS];
     {
@@ -1417,13 +1433,27 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
         for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
     float m = -INFINITY, l = 0.f;
 
-    // Order of a turn: the block two on is asked for, into the stage that the turn before read
-    // (its readers are past the barrier); then the block in this stage is worked on; then the wave
-    // waits for its own loads of the NEXT block (the loads of the block after it may stay in
-    // flight: a wave's loads retire in order) and meets the others at the barrier.
+    // Order of a turn.  Heads of 128: while block j's scores become probabilities, on the vector ALU, the matrix cores make block j + 1's
+    // scores, whose keys are in LDS a turn ahead of their values; then O^T takes block j.  First the values of block j + 2
+    // and the keys of block j + 3 are asked for, into the stages that the turn before read (their readers are past the barrier);
+    // last the wave waits for its own loads of the turn before (those of this turn may stay in flight: a wave's loads retire in
+    // order) and meets the others at the barrier.  Done one behind the other, the vector ALU and the matrix cores were each busy 44 % of
+    // the time; so the kernel needs a tenth fewer cycles, of which the clock, held by the power that the chip draws, takes back a part: 28
+    // heads of 4, 2,048 tokens 58.5 -> 55.5 us, 8,192 560 -> 547; 32 heads of 32, 2,048 behind 4,000 203 -> 195; 5 segments of 256 to
+    // 1,000 tokens 142 -> 136.5; 40 of 8, 1,999 behind 16,000 is as long as it was (769 -> 767 and 811 -> 813 on two cards, at 1,875 MHz where
+    // it was 2,050).  Eight waves a block that share the keys, with one tile each or four with two each (half the loads, or
+    // half the reads of LDS too), are no faster: 743 and 764 where that takes 750, 66 and 74 where 2,048 tokens take 52.
+    // Heads of 64 make a block's scores in its own turn: four waves a SIMD cover for each other, and the sums of both blocks
+    // leave room for three (32 heads of 8, 4,096 tokens: 95.7 and, on the same card, 88.6 so).
     const int nblk = (k_end - k_begin + 31) / 32;
-    LI_PRE_FETCH(0);
-    if (nblk > 1) { LI_PRE_FETCH(1); LI_ATT_VMCNT(2 * NL); } else { LI_ATT_VMCNT(0); }
+    fetch_k(0);
+    fetch_v(0);
+    if (nblk > 1) { fetch_k(1); fetch_v(1); }
+    if constexpr (!AHEAD) {
+        if (nblk > 1) { LI_ATT_VMCNT(2 * NL); } else { LI_ATT_VMCNT(0); }
+    } else {
+        if (nblk > 2) { fetch_k(2); LI_ATT_VMCNT(2 * NL); } else if (nblk > 1) { LI_ATT_VMCNT(NL); } else { LI_ATT_VMCNT(0); }
+    }
     // The queries have arrived by now: they were asked for before the blocks of keys, and a wave's loads retire
     // in order.  The compiler counts only the loads it made itself and would wait for "its" eight at their first
     // use, inside the loop, where the same count stands for the blocks of keys that are on their way: every turn
@@ -1456,82 +1486,185 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
             vaddr[dt] = vkey * DH + 8 * (chunk ^ swz) + 4 * (gi & 1);
         }
     }
-    // three turns a trip, so that the stage is a constant of the code and the LDS addresses are
-    // a register plus an immediate
-    for (int j3 = 0; j3 < nblk; j3 += NST) {
+    // S^T = K Q^T of a block whose keys lie in a stage
+    frag8 kf[KS];
+    auto read_k = [&](int stage) {
 #pragma unroll
-      for (int stage = 0; stage < NST; ++stage) {
-        const int jb = j3 + stage;
-        if (jb >= nblk) break;
-        const int kb = k_begin + 32 * jb;
-        if (jb + 2 < nblk) LI_PRE_FETCH((stage + 2) % NST);
-        if (active && (abreast == 1 || (kb <= p_last && kb + 31 >= lo_tile))) {
-            // ---- S^T = K Q^T
-            f32x16_t sv;
+        for (int st = 0; st < KS; ++st) kf[st].raw = *reinterpret_cast<const u32x4*>(&Ks[stage][kaddr[st]]);
+    };
+    f32x16_t sv;
+    float top = -INFINITY;                              // this lane's largest score of the block (the other half of the query's keys: 32 lanes on)
+    auto scores = [&](int stage) {
+        read_k(stage);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sv[r] = 0.f;
-            frag8 kf[KS];
+        for (int r = 0; r < 16; ++r) sv[r] = 0.f;
 #pragma unroll
-            for (int st = 0; st < KS; ++st) kf[st].raw = *reinterpret_cast<const u32x4*>(&Ks[stage][kaddr[st]]);
-            // (raising the wave's priority while it issues its MFMAs, so that the SIMD's other wave does its
-            // softmax meanwhile, was measured in turn with this form on one machine: 2 to 5 % SLOWER at 2,048 to
-            // 30,000 keys, so the waves keep the default priority)
-#pragma unroll
-            for (int st = 0; st < KS; ++st) sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[st].v, qf[st].v, sv, 0, 0, 0);
-            // ---- softmax over the keys of this lane's query.  The running maximum m is only moved
-            // (and the sums so far rescaled, for the whole wave) when some query's scores pass it by
-            // more than 2^8: until then the exponentials are taken against the older maximum, which
-            // changes no result (numerator and denominator carry the same factor) and stays far
-            // inside the range of float and bfloat16.
-            // A block that every query of the tile sees whole (most are) needs no masks.
-            if (!(kb + 31 <= p0 && kb >= l_last)) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int key = kb + 8 * (r >> 2) + 4 * h + (r & 3);
-                    sv[r] = (key <= pq && key >= lq) ? sv[r] : -INFINITY;
-                }
-            }
-            const float mx = both_halves_max(largest_of(sv)) * scale2;                          // (scale2 > 0)
-            if (__any(mx > m + 8.0f)) {
-                const float mn = fmaxf(m, mx);
-                const float alpha = (mn == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - mn);   // (m = -inf: nothing summed yet)
-                l *= alpha;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[dt][r] *= alpha;
-                m = mn;
-            }
-            const float ms = (m == -INFINITY) ? 0.f : m;         // a query may see no key yet
-            float ps = 0.f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) { sv[r] = __builtin_amdgcn_exp2f(fmaf(sv[r], scale2, -ms)); ps += sv[r]; }
-            l += ps;
-            frag8 pf[2];
-#pragma unroll
-            for (int st = 0; st < 2; ++st)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) pf[st].raw.w[i] = pack2_bf16(sv[8 * st + 2 * i], sv[8 * st + 2 * i + 1]);
-            // ---- O^T += V^T P^T
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-#pragma unroll
-                for (int st = 0; st < 2; ++st) {
-                    frag8 vf;
-                    const tr4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr4 __attribute__((address_space(3)))*)&Vs[stage][vaddr[dt] + (16 * st) * DH]);
-                    const tr4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr4 __attribute__((address_space(3)))*)&Vs[stage][vaddr[dt] + (16 * st + 8) * DH]);
-                    vf.raw.w[0] = (uint32_t)(uint16_t)v0[0] | ((uint32_t)(uint16_t)v0[1] << 16);
-                    vf.raw.w[1] = (uint32_t)(uint16_t)v0[2] | ((uint32_t)(uint16_t)v0[3] << 16);
-                    vf.raw.w[2] = (uint32_t)(uint16_t)v1[0] | ((uint32_t)(uint16_t)v1[1] << 16);
-                    vf.raw.w[3] = (uint32_t)(uint16_t)v1[2] | ((uint32_t)(uint16_t)v1[3] << 16);
-                    acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[st].v, acc[dt], 0, 0, 0);
-                }
-            }
+        for (int st = 0; st < KS; ++st) sv = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[st].v, qf[st].v, sv, 0, 0, 0);
+        top = largest_of(sv);
+    };
+    // A tile of several abreast sees the blocks first .. mine - 1 of the block's nblk; its wave helps to fetch the others
+    int first = 0, mine = active ? nblk : 0;
+    if constexpr (abreast > 1) {
+        const int lo_tile = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
+        if (lo_tile > k_begin) first = (lo_tile - k_begin) >> 5;
+        const int seen = p_last < k_begin ? 0 : ((p_last - k_begin) >> 5) + 1;
+        if (seen < mine) mine = seen;
+    }
+    const bool works = first < mine;
+    if constexpr (AHEAD) {
+        if (works && first == 0) scores(0);
+        __builtin_amdgcn_s_barrier();                   // (the first stage of keys is asked for anew by the first turn)
+        asm volatile("" ::: "memory");
+    }
+    // What a turn does beside its block: asks for a block's values and another's keys, and waits for what the next turn reads.
+    auto ask = [&](int jb, int v_stage, int k_stage) {
+        if constexpr (!AHEAD) {
+            if (jb + 2 < nblk) { fetch_k(v_stage); fetch_v(v_stage); }
+        } else {
+            if (jb + 2 < nblk) fetch_v(v_stage);
+            if (jb + 3 < nblk) fetch_k(k_stage);
         }
-        if (jb + 2 < nblk) { LI_ATT_VMCNT(2 * NL); } else { LI_ATT_VMCNT(0); }
+    };
+    auto meet = [&](int jb) {
+        if (AHEAD ? jb + 3 < nblk : jb + 2 < nblk) { LI_ATT_VMCNT(2 * NL); } else if (AHEAD && jb + 2 < nblk) { LI_ATT_VMCNT(NL); } else { LI_ATT_VMCNT(0); }
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-      }
+    };
+    // Block jb, whose values lie at vs and whose scores are in sv; NEXT: beside it the scores of the block behind it, whose keys lie in k_stage.
+    auto work = [&](auto next_tag, int jb, const uint16_t* vs, int k_stage) {
+        constexpr bool NEXT = AHEAD && decltype(next_tag)::value;
+        if constexpr (NEXT) read_k(k_stage);
+        if constexpr (!AHEAD) scores(k_stage);
+        const int kb = k_begin + 32 * jb;
+        // ---- softmax over the keys of this lane's query.  The running maximum m is only moved
+        // (and the sums so far rescaled, for the whole wave) when some query's scores pass it by
+        // more than 2^8: until then the exponentials are taken against the older maximum, which
+        // changes no result (numerator and denominator carry the same factor) and stays far
+        // inside the range of float and bfloat16.
+        // A block that every query of the tile sees whole (most are) needs no masks.
+        if (!(kb + 31 <= p0 && kb >= l_last)) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int key = kb + 8 * (r >> 2) + 4 * h + (r & 3);
+                sv[r] = (key <= pq && key >= lq) ? sv[r] : -INFINITY;
+            }
+            top = largest_of(sv);
+        }
+        const float mx = both_halves_max(top) * scale2;                          // (scale2 > 0)
+        if (__any(mx > m + 8.0f)) {
+            const float mn = fmaxf(m, mx);
+            const float alpha = (mn == -INFINITY) ? 1.0f : __builtin_amdgcn_exp2f(m - mn);   // (m = -inf: nothing summed yet)
+            l *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[dt][r] *= alpha;
+            m = mn;
+        }
+        const float ms = (m == -INFINITY) ? 0.f : -m;        // a query may see no key yet
+        f32x16_t sn;
+        tr4 vr[2][DT][2];
+        frag8 pf[2];
+        float ps = 0.f;
+        auto read_v = [&](int i) {
+            const int st = i / (2 * DT), dt = (i / 2) % DT, e = i % 2;
+            vr[st][dt][e] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((tr4 __attribute__((address_space(3)))*)&vs[vaddr[dt] + (16 * st + 8 * e) * DH]);
+        };
+        // probability r; its sum and packing run one behind it
+        auto sum_prob = [&](int r) {
+            ps += sv[r];
+            if (r & 1) pf[r / 8].raw.w[(r % 8) / 2] = pack2_bf16(sv[r - 1], sv[r]);
+        };
+        auto prob = [&](int r) {
+            sv[r] = __builtin_amdgcn_exp2f(fmaf(sv[r], scale2, ms));
+            if (r) sum_prob(r - 1);
+        };
+        // ---- O^T += V^T P^T
+        auto value = [&](int i) {
+            const int st = i / DT, dt = i % DT;
+            frag8 vf;
+            const tr4 v0 = vr[st][dt][0], v1 = vr[st][dt][1];
+            vf.raw.w[0] = (uint32_t)(uint16_t)v0[0] | ((uint32_t)(uint16_t)v0[1] << 16);
+            vf.raw.w[1] = (uint32_t)(uint16_t)v0[2] | ((uint32_t)(uint16_t)v0[3] << 16);
+            vf.raw.w[2] = (uint32_t)(uint16_t)v1[0] | ((uint32_t)(uint16_t)v1[1] << 16);
+            vf.raw.w[3] = (uint32_t)(uint16_t)v1[2] | ((uint32_t)(uint16_t)v1[3] << 16);
+            acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf.v, pf[st].v, acc[dt], 0, 0, 0);
+        };
+        if constexpr (NEXT) {
+            // One MFMA of the next scores, two reads of the values and 16 / KS probabilities, KS times; then one MFMA of the output
+            // and a part of the next scores' largest, 2 DT times.  (Left to itself the compiler puts all MFMAs ahead of the rest.)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) sn[r] = 0.f;
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int st = 0; st < KS; ++st) {
+                sn = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[st].v, qf[st].v, sn, 0, 0, 0);
+                read_v(2 * st);
+                read_v(2 * st + 1);
+#pragma unroll
+                for (int r = st * 16 / KS; r < (st + 1) * 16 / KS; ++r) prob(r);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            sum_prob(15);
+            constexpr int EACH = 16 / (2 * DT);
+#pragma unroll
+            for (int i = 0; i < 2 * DT; ++i) {
+                value(i);
+                if (i == 0) { l += ps; top = fmaxf(sn[0], sn[1]); }
+#pragma unroll
+                for (int r = EACH * i; r < EACH * (i + 1); r += 2)
+                    if (r) top = max3f(top, sn[r], sn[r + 1]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            sv = sn;
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4 * DT; ++i) read_v(i);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) prob(r);
+            sum_prob(15);
+            l += ps;
+#pragma unroll
+            for (int i = 0; i < 2 * DT; ++i) value(i);
+        }
+    };
+    // three turns a trip, so that the stage is a constant of the code and the LDS addresses are
+    // a register plus an immediate
+    auto one_block = [&](int jb, int stage) {
+        ask(jb, (stage + 2) % NST, stage);
+        work(std::true_type{}, jb, Vs[stage], AHEAD ? (stage + 1) % NST : stage);
+        meet(jb);
+    };
+    auto help = [&](int from, int to) {                 // (a wave without a head, tile or key helps to fetch and keeps the barriers)
+        for (int jb = from; jb < to; ++jb) {
+            ask(jb, (jb + 2) % NST, jb % NST);
+            if (AHEAD && works && jb + 1 == first) scores((jb + 1) % NST);
+            meet(jb);
+        }
+    };
+    if (works) {
+        int j3 = first;
+        if constexpr (abreast > 1) {
+            help(0, first);
+            if (j3 % NST == 1 && j3 + 1 < mine) { one_block(j3, 1); ++j3; }
+            if (j3 % NST == 2 && j3 + 1 < mine) { one_block(j3, 2); ++j3; }
+        }
+        for (; j3 + 1 < mine; j3 += NST) {
+#pragma unroll
+            for (int stage = 0; stage < NST; ++stage) {
+                if (j3 + stage + 1 >= mine) break;
+                one_block(j3 + stage, stage);
+            }
+        }
+        const int last = (mine - 1) % NST;
+        if (abreast > 1 && mine < nblk) ask(mine - 1, (last + 2) % NST, last);
+        work(std::false_type{}, mine - 1, Vs[last], last);
+        if (abreast > 1 && mine < nblk) {
+            meet(mine - 1);
+            help(mine, nblk - 1);
+        }
+    } else {
+        help(0, nblk - 1);
     }
     if (!active || ql >= nrows) return;
     l += __shfl_xor(l, 32, LI_WAVE);               // (both halves of a query are past the return together)
@@ -1564,7 +1697,6 @@ __global__ __launch_bounds__(PRE_WAVES * 64) void paged_attention_prefill_dma_ke
         }
 }
 
-#undef LI_PRE_FETCH
 // The same for prompts of so few tiles that a compute unit holds one or two blocks and the time is that of
 // the longest tile, one block of keys after the other: eight waves a block, two groups of four, each group
 // with its own stages of LDS takes half of the tile's blocks of keys (the first half, the second half), and
@@ -2318,7 +2450,7 @@ extern "C" int li_paged_attention_prefill(const void* q, int q_row_stride, void*
         else return LI_ERR_SIZE;
     } else
     if (max_blocks <= PRE2_TABLE_CAP) {                       // (longer block tables: the form that keeps 8,192 entries in LDS)
-        const bool p32 = 32 % page_size == 0;
+        const bool p32 = 32 % page_size == 0 && page_size * dh >= 512;
         if (dh == 128) { if (p32) LI_PRE2(128, true) else LI_PRE2(128, false) }
         else if (dh == 64) { if (p32) LI_PRE2(64, true) else LI_PRE2(64, false) }
         else return LI_ERR_SIZE;

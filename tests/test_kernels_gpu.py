@@ -1046,6 +1046,16 @@ def test_prompt_attention_with_several_tiles_a_block(ops, monkeypatch, segs, nh,
     assert rel(out, ref) < 1.5e-2
 
 
+@pytest.mark.parametrize("dh,page,window", [(128, 16, 0), (128, 4, 0), (128, 2, 40), (64, 8, 0), (64, 4, 33), (128, 32, 70)])
+@pytest.mark.parametrize("heads", [1, 2])
+def test_prompt_attention_over_few_blocks_of_keys(ops, monkeypatch, dh, page, window, heads):
+    # one to seven blocks of 32 keys: the turns before the stages of LDS are all in use and the last ones; pages down to less than a load
+    monkeypatch.setattr(ops, "_prefill_heads", lambda *a: heads)
+    segs = [(2, 2), (32, 32), (33, 33), (64, 2), (65, 64), (97, 33), (128, 128), (130, 5), (161, 161), (224, 31)]
+    out, ref = _paged_case(ops, torch.bfloat16, segs, 6, 2, dh, page, window, seed=37)
+    assert rel(out, ref) < 1.5e-2
+
+
 @pytest.mark.parametrize("heads,tiles,runs", [(4, 1, 2), (4, 7, 5), (2, 2, 3), (2, 10, 16), (1, 4, 4), (1, 12, 2)])
 def test_prompt_attention_with_the_keys_of_its_first_tiles_in_runs(ops, monkeypatch, heads, tiles, runs):
     segs = [(700, 300), (1, 1), (90, 70), (400, 40), (257, 129)]                # 10 + 3 + 2 + 5 tiles, a decoding token among them
