@@ -35,11 +35,14 @@ __device__ __forceinline__ int lower_edge(int p, int window, int chunk) {
 
 // What a (token, head)'s sums of values are multiplied by at the end: one over the sum of the weights (with the sink's
 // term, counted once), and the head's gate where heads have one.
-__device__ __forceinline__ float finish_factor(float l, float m, const MaExtras& ex, int t, int head) {
-    if (ex.sink && l != 0.f) l += expf(ex.sink[head] - m);
+__device__ __forceinline__ float finish_factor_of(float l, float m, const MaExtras& ex, float sink, float gate) {
+    if (ex.sink && l != 0.f) l += expf(sink - m);
     float f = l != 0.f ? 1.0f / l : 0.f;
-    if (ex.gate && !ex.per_column) f *= 1.0f / (1.0f + expf(-ex.gate[(size_t)t * ex.gate_stride + head]));
+    if (ex.gate && !ex.per_column) f *= 1.0f / (1.0f + expf(-gate));
     return f;
+}
+__device__ __forceinline__ float finish_factor(float l, float m, const MaExtras& ex, int t, int head) {
+    return finish_factor_of(l, m, ex, ex.sink ? ex.sink[head] : 0.f, ex.gate && !ex.per_column ? ex.gate[(size_t)t * ex.gate_stride + head] : 0.f);
 }
 
 // The gate of one value column (1 where the columns have none of their own), and of four neighbouring ones at once.
@@ -495,8 +498,7 @@ __global__ __launch_bounds__(NW * 64) void masked_attention_tile_kernel(
         }
 }
 
-__global__ void masked_attention_join_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out,
-                                             const int* __restrict__ token_list, int nh, int dv, int nsplit, MaExtras ex, int by_token = 0);
+static void launch_join(const float* parts, void* out, const int* token_list, int n_tokens, int nh, int dv, int nsplit, const MaExtras& ex, int by_token, hipStream_t stream);
 
 // ------------------------------------------------------------------------------------------- single tokens, MFMA
 // Decoding where a kv head serves many query heads (a compressed cache serves ALL of them): the same transposed
@@ -757,7 +759,7 @@ extern "C" int li_masked_attention_tiles(const float* q, int q_token_stride, int
                 max_blocks, tiles, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, keep_first, softcap, scale, ex, \
                 nsplit, parts);                                                                                            \
         if (nsplit > 1)                                                                                                    \
-            masked_attention_join_kernel<<<dim3(num_multi, nh), dv >= 256 ? 256 : 128, 0, stream>>>(parts, (bf16_t*)out, multi_tokens, nh, dv, nsplit, ex, 1); \
+            launch_join(parts, out, multi_tokens, num_multi, nh, dv, nsplit, ex, 1, stream);                               \
         return li_launch_status();                                                                                         \
     }
     MT_GO(64, 64) MT_GO(128, 128) MT_GO(128, 64) MT_GO(64, 128) MT_GO(96, 64) MT_GO(160, 128) MT_GO(192, 128)
@@ -790,7 +792,7 @@ extern "C" int li_masked_attention_heads(const float* q, int q_token_stride, int
             max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, nh, nkv, page_size, num_pages, window, keep_first, \
             softcap, scale, ex, nsplit, parts);                                                                                \
         if (nsplit > 1)                                                                                                    \
-            masked_attention_join_kernel<<<dim3(n_tokens, nh), dv >= 256 ? 256 : 128, 0, stream>>>(parts, (bf16_t*)out, token_list, nh, dv, nsplit, ex); \
+            launch_join(parts, out, token_list, n_tokens, nh, dv, nsplit, ex, 0, stream);                                  \
         return li_launch_status();                                                                                         \
     }
     MH_GO(64, 64) MH_GO(128, 128) MH_GO(128, 64) MH_GO(64, 128) MH_GO(96, 64) MH_GO(160, 128) MH_GO(192, 128)
@@ -1083,98 +1085,150 @@ __global__ __launch_bounds__(256) void masked_attention_single_kernel(
     }
 }
 
-// joins the splits of every (token, head) in split order: a block a (token, head)
+// joins the splits of every (token, head): a block a (token, head, 128 value columns)
 // (the parts of a token lie at its place in the list, or, with by_token, at its own number)
-// The first wave takes the splits' maxima and sums side by side and leaves every split's factor in LDS; a column's parts are
-// then asked for eight at a time.  (Maxima, factors and parts split after split were a chain of three loads and an
-// exponential for each: 24 to 48 splits 6.6 to 10 us, now 4.6 to 5.3.)
-#define JOIN_MAX_SPLITS 64
-__global__ void masked_attention_join_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out,
-                                             const int* __restrict__ token_list, int nh, int dv, int nsplit, MaExtras ex, int by_token) {
-    __shared__ float fac[JOIN_MAX_SPLITS], sums[JOIN_MAX_SPLITS], top[1];
+// Bound by its trips to memory.  A wave takes JOIN_SHARE splits of the 128 columns, two columns a lane, and asks for all of them, the
+// splits' maxima and sums (lane x split x) and the extras at once; the waves' sums are added in wave order.  With the factors
+// through LDS first and then eight splits a trip, a thread a column, two tokens of 12 heads of 64 and 128 columns took 4.4 us (24 and 32 splits), now
+// 3.7, and 32 tokens of 12 heads, two splits, 4.6, now 4.2.
+#define JOIN_SHARE 8
+template <int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void masked_attention_join_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out,
+                                                                           const int* __restrict__ token_list, int nh, int dv, int nsplit, MaExtras ex, int by_token) {
+    __shared__ float2 sums[WAVES > 1 ? WAVES - 1 : 1][64];
     const int t = token_list ? token_list[blockIdx.x] : blockIdx.x, head = blockIdx.y;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), first = w * JOIN_SHARE;
     const float* base = parts + ((size_t)(by_token ? t : (int)blockIdx.x) * nh + head) * nsplit * (dv + 2);
-    if (threadIdx.x < LI_WAVE) {                       // (at most as many splits as a wave has lanes)
-        const int x = threadIdx.x < nsplit ? threadIdx.x : nsplit - 1;
-        const float m = base[(size_t)x * (dv + 2) + dv], l = base[(size_t)x * (dv + 2) + dv + 1];
-        const float mm = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - mm);
-        fac[threadIdx.x] = f;
-        sums[threadIdx.x] = l * f;
-        if (threadIdx.x == 0) top[0] = mm;
+    const int d = 128 * blockIdx.z + 2 * lane, at = d < dv ? d : dv - 2;      // (dv is a multiple of 8)
+    float2 r[JOIN_SHARE];
+#pragma unroll
+    for (int i = 0; i < JOIN_SHARE; ++i) r[i] = *reinterpret_cast<const float2*>(base + (size_t)(first + i < nsplit ? first + i : 0) * (dv + 2) + at);
+    const float2 ml = *reinterpret_cast<const float2*>(base + (size_t)(lane < nsplit ? lane : 0) * (dv + 2) + dv);
+    const float sink = ex.sink ? ex.sink[head] : 0.f;
+    float head_gate = 0.f;
+    float2 gate{0.f, 0.f};
+    if (ex.gate) {
+        const float* g = ex.gate + (size_t)t * ex.gate_stride;
+        if (ex.per_column) { gate.x = g[(size_t)head * dv + at]; gate.y = g[(size_t)head * dv + at + 1]; }
+        else head_gate = g[head];
     }
-    __syncthreads();
-    const float mm = top[0];
-    float ll = 0.f;
-#pragma unroll 8
-    for (int x = 0; x < nsplit; ++x) ll += sums[x];
-    for (int d = threadIdx.x; d < dv; d += blockDim.x) {
-        float a = 0.f;
-        for (int x0 = 0; x0 < nsplit; x0 += 8) {
-            float r[8];
+    const float m = lane < nsplit ? ml.x : -INFINITY, mm = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - mm);
+    const float ll = wave_sum(lane < nsplit ? ml.y * f : 0.f);
+    float2 a{0.f, 0.f};
 #pragma unroll
-            for (int i = 0; i < 8; ++i) r[i] = base[(size_t)(x0 + i < nsplit ? x0 + i : nsplit - 1) * (dv + 2) + d];
+    for (int i = 0; i < JOIN_SHARE; ++i) {
+        const float fi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), first + i));
+        a.x = first + i < nsplit ? fmaf(r[i].x, fi, a.x) : a.x;
+        a.y = first + i < nsplit ? fmaf(r[i].y, fi, a.y) : a.y;
+    }
+    if constexpr (WAVES > 1) {
+        if (w) sums[w - 1][lane] = a;
+        __syncthreads();
+        if (w) return;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) a = x0 + i < nsplit ? fmaf(r[i], fac[x0 + i], a) : a;
-        }
-        out[((size_t)t * nh + head) * dv + d].bits = float_to_bf16(a * finish_factor(ll, mm, ex, t, head) * column_gate(ex, t, head, dv, d));
+        for (int x = 1; x < WAVES; ++x) { a.x += sums[x - 1][lane].x; a.y += sums[x - 1][lane].y; }
+    }
+    const float fin = finish_factor_of(ll, mm, ex, sink, head_gate);
+    a.x *= fin; a.y *= fin;
+    if (ex.gate && ex.per_column) { a.x *= 1.0f / (1.0f + expf(-gate.x)); a.y *= 1.0f / (1.0f + expf(-gate.y)); }
+    if (d < dv) {
+        bf16_t* o = out + ((size_t)t * nh + head) * dv + d;
+        o[0].bits = float_to_bf16(a.x);
+        o[1].bits = float_to_bf16(a.y);
     }
 }
 
+static void launch_join(const float* parts, void* out, const int* token_list, int n_tokens, int nh, int dv, int nsplit, const MaExtras& ex, int by_token, hipStream_t stream) {
+    const dim3 grid(n_tokens, nh, (dv + 127) / 128);
+#define MS_JOIN_BY(W) masked_attention_join_kernel<W><<<grid, 64 * W, 0, stream>>>(parts, (bf16_t*)out, token_list, nh, dv, nsplit, ex, by_token)
+    if (nsplit <= JOIN_SHARE) MS_JOIN_BY(1);
+    else if (nsplit <= 2 * JOIN_SHARE) MS_JOIN_BY(2);
+    else if (nsplit <= 4 * JOIN_SHARE) MS_JOIN_BY(4);
+    else MS_JOIN_BY(8);                             // (at most 64 splits, a lane each)
+#undef MS_JOIN_BY
+}
+
 // The same for two maps: both joined, their difference a1 - lambda a2 and its norm over the head's columns, times `mult` (what
-// diff_combine_kernel does, here without the maps' rounding between).  A block of two waves a (token, head), a wave the factors of one
-// map's splits.  Bound by the launches: a step's five kernels of 4 to 8 us, each waiting for the one before it, are two (an answer of
-// a model with such layers 12.35 -> 11.83 ms).
-#define JOIN_DIFF_COLUMNS 2         // columns a thread holds: dv up to 256, the most that the kernel before it has
-__global__ __launch_bounds__(128) void masked_attention_join_diff_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out, int n, int nh, int dv, int nsplit,
-                                                                         float lambda, float eps, float mult) {
-    __shared__ float fac[2][JOIN_MAX_SPLITS], sums[2][JOIN_MAX_SPLITS], squares[2];
-    const int t = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const size_t map = (size_t)n * nh * nsplit * (dv + 2);
-    const float* base = parts + ((size_t)t * nh + head) * nsplit * (dv + 2);
-    {
-        const float* mine = base + w * map + (size_t)(lane < nsplit ? lane : nsplit - 1) * (dv + 2) + dv;
-        const float m = mine[0], l = mine[1];
-        const float mm = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - mm);
-        fac[w][lane] = f;
-        sums[w][lane] = l * f;
+// diff_combine_kernel does, here without the maps' rounding between).  A block a (token, head), WAVES waves a map, each with JOIN_SHARE splits
+// of all columns.  Bound by the launches: a step's five kernels of 4 to 8 us, each waiting for the one before it, are two (an answer of
+// a model with such layers 12.35 -> 11.83 ms); 12 heads of 128 columns, 12 splits, a thread a column and eight splits a trip 4.3 us, so 3.5.
+#define JOIN_DIFF_CHUNKS 2          // times 128 columns: dv up to 256, the most that the kernel before it has
+template <int WAVES>
+__global__ __launch_bounds__(128 * WAVES) void masked_attention_join_diff_kernel(const float* __restrict__ parts, bf16_t* __restrict__ out, int n, int nh, int dv, int nsplit,
+                                                                                 float lambda, float eps, float mult) {
+    __shared__ float2 sums[2][WAVES][JOIN_DIFF_CHUNKS][64];
+    __shared__ float total[2];
+    const int t = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q = wave / WAVES, w = wave % WAVES, first = w * JOIN_SHARE;
+    const float* base = parts + (size_t)q * n * nh * nsplit * (dv + 2) + ((size_t)t * nh + head) * nsplit * (dv + 2);
+    float2 r[JOIN_DIFF_CHUNKS][JOIN_SHARE];
+#pragma unroll
+    for (int c = 0; c < JOIN_DIFF_CHUNKS; ++c) {
+        if (c && 128 * c >= dv) break;
+        const int d = 128 * c + 2 * lane, at = d < dv ? d : dv - 2;
+#pragma unroll
+        for (int i = 0; i < JOIN_SHARE; ++i) r[c][i] = *reinterpret_cast<const float2*>(base + (size_t)(first + i < nsplit ? first + i : 0) * (dv + 2) + at);
+    }
+    const float2 ml = *reinterpret_cast<const float2*>(base + (size_t)(lane < nsplit ? lane : 0) * (dv + 2) + dv);
+    const float m = lane < nsplit ? ml.x : -INFINITY, mm = wave_max(m), f = m == -INFINITY ? 0.f : expf(m - mm);
+    const float ll = wave_sum(lane < nsplit ? ml.y * f : 0.f);
+    if (w == 0 && lane == 0) total[q] = ll;
+#pragma unroll
+    for (int c = 0; c < JOIN_DIFF_CHUNKS; ++c) {
+        if (c && 128 * c >= dv) break;
+        float2 a{0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < JOIN_SHARE; ++i) {
+            const float fi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), first + i));
+            a.x = first + i < nsplit ? fmaf(r[c][i].x, fi, a.x) : a.x;
+            a.y = first + i < nsplit ? fmaf(r[c][i].y, fi, a.y) : a.y;
+        }
+        sums[q][w][c][lane] = a;
     }
     __syncthreads();
+    if (wave) return;
     float inv[2];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
-        float ll = 0.f;
-#pragma unroll 8
-        for (int x = 0; x < nsplit; ++x) ll += sums[q][x];
-        inv[q] = ll != 0.f ? 1.0f / ll : 0.f;
-    }
-    float o[JOIN_DIFF_COLUMNS], ss = 0.f;
+    for (int x = 0; x < 2; ++x) inv[x] = total[x] != 0.f ? 1.0f / total[x] : 0.f;
+    float2 o[JOIN_DIFF_CHUNKS];
+    float ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < JOIN_DIFF_COLUMNS; ++c) {
-        const int d = threadIdx.x + 128 * c;
-        o[c] = 0.f;
-        if (d >= dv) continue;
-        float a[2] = {0.f, 0.f};
+    for (int c = 0; c < JOIN_DIFF_CHUNKS; ++c) {
+        o[c] = float2{0.f, 0.f};
+        if (128 * c + 2 * lane >= dv) continue;
+        float2 a[2];
 #pragma unroll
-        for (int q = 0; q < 2; ++q)
-            for (int x0 = 0; x0 < nsplit; x0 += 8) {
-                float r[8];
+        for (int x = 0; x < 2; ++x) {
+            a[x] = sums[x][0][c][lane];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) r[i] = base[q * map + (size_t)(x0 + i < nsplit ? x0 + i : nsplit - 1) * (dv + 2) + d];
-#pragma unroll
-                for (int i = 0; i < 8; ++i) a[q] = x0 + i < nsplit ? fmaf(r[i], fac[q][x0 + i], a[q]) : a[q];
-            }
-        o[c] = fmaf(-lambda, a[1] * inv[1], a[0] * inv[0]);
-        ss = fmaf(o[c], o[c], ss);
+            for (int y = 1; y < WAVES; ++y) { a[x].x += sums[x][y][c][lane].x; a[x].y += sums[x][y][c][lane].y; }
+        }
+        o[c].x = fmaf(-lambda, a[1].x * inv[1], a[0].x * inv[0]);
+        o[c].y = fmaf(-lambda, a[1].y * inv[1], a[0].y * inv[0]);
+        ss = fmaf(o[c].x, o[c].x, ss);
+        ss = fmaf(o[c].y, o[c].y, ss);
     }
     ss = wave_sum(ss);
-    if (lane == 0) squares[w] = ss;
-    __syncthreads();
-    const float f = mult / sqrtf((squares[0] + squares[1]) / (float)dv + eps);
+    const float scale = mult / sqrtf(ss / (float)dv + eps);
 #pragma unroll
-    for (int c = 0; c < JOIN_DIFF_COLUMNS; ++c) {
-        const int d = threadIdx.x + 128 * c;
-        if (d < dv) out[((size_t)t * nh + head) * dv + d].bits = float_to_bf16(o[c] * f);
+    for (int c = 0; c < JOIN_DIFF_CHUNKS; ++c) {
+        const int d = 128 * c + 2 * lane;
+        if (d < dv) {
+            bf16_t* dst = out + ((size_t)t * nh + head) * dv + d;
+            dst[0].bits = float_to_bf16(o[c].x * scale);
+            dst[1].bits = float_to_bf16(o[c].y * scale);
+        }
     }
+}
+
+static void launch_join_diff(const float* parts, void* out, int n_tokens, int nh, int dv, int nsplit, float lambda, float eps, float mult, hipStream_t stream) {
+    const dim3 grid(n_tokens, nh);
+#define MS_JOIN_BY(W) masked_attention_join_diff_kernel<W><<<grid, 128 * W, 0, stream>>>(parts, (bf16_t*)out, n_tokens, nh, dv, nsplit, lambda, eps, mult)
+    if (nsplit <= JOIN_SHARE) MS_JOIN_BY(1);
+    else if (nsplit <= 2 * JOIN_SHARE) MS_JOIN_BY(2);
+    else if (nsplit <= 4 * JOIN_SHARE) MS_JOIN_BY(4);
+    else MS_JOIN_BY(8);
+#undef MS_JOIN_BY
 }
 
 // 1 if the kernel for single tokens takes these sizes (bfloat16 cache and output)
@@ -1229,9 +1283,9 @@ static int single_launch(const float* q, int q_token_stride, int q_head_stride, 
         keep_first, softcap, scale, ex, tab_cap, pshift, nsplit, parts, second)
 #define MS_JOIN                                                                                                             \
     if (maps > 1)                                                                                                           \
-        masked_attention_join_diff_kernel<<<dim3(n_tokens, nh), 128, 0, stream>>>(parts, (bf16_t*)out, n_tokens, nh, dv, nsplit, lambda, eps, mult); \
+        launch_join_diff(parts, out, n_tokens, nh, dv, nsplit, lambda, eps, mult, stream);                                  \
     else if (nsplit > 1)                                                                                                         \
-        masked_attention_join_kernel<<<dim3(n_tokens, nh), dv >= 256 ? 256 : 128, 0, stream>>>(parts, (bf16_t*)out, token_list, nh, dv, nsplit, ex);
+        launch_join(parts, out, token_list, n_tokens, nh, dv, nsplit, ex, 0, stream);
 #define MS_SMALL(K, V)                                                                                                      \
     if (npk == K && npv == V) {                                                                                             \
         if (rh == 4) MS_GO(K, V, 4, 4); else if (rh == 2) MS_GO(K, V, 2, 4); else MS_GO(K, V, 1, 4);                        \
@@ -1271,7 +1325,7 @@ extern "C" int li_masked_attention_single_pair(const float* q, int q_token_strid
                                                const int* q_len, const int* ctx_len, int nh, int nkv, int dk, int dv, int page_size,
                                                int num_pages, int window, int keep_first, float softcap, float scale, int nsplit, float* parts,
                                                long parts_floats, float lambda, float eps, float mult, hipStream_t stream) {
-    if (!k2 || (uintptr_t)k2 % 16 || q_off % 4 || n_tokens <= 0 || dv > 128 * JOIN_DIFF_COLUMNS) return LI_ERR_SIZE;
+    if (!k2 || (uintptr_t)k2 % 16 || q_off % 4 || n_tokens <= 0 || dv > 128 * JOIN_DIFF_CHUNKS) return LI_ERR_SIZE;
     return single_launch(q, q_token_stride, q_head_stride, out, kc, vc, k_row, v_row, block_table, max_blocks, nullptr, n_tokens, seg_of_token,
                          q_start, q_len, ctx_len, nh, nkv, dk, dv, page_size, num_pages, window, keep_first, softcap, scale, nullptr, nullptr, 0, 0,
                          nullptr, 0, nsplit, parts, parts_floats, MaSecond{(const bf16_t*)k2, q_off, n_tokens}, lambda, eps, mult, stream);

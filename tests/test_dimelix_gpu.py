@@ -631,6 +631,17 @@ def test_slopes_gates_and_sinks_in_every_attention_kernel(dtype, segs, nh, nkv, 
     assert err < (2e-5 if dtype is torch.float32 else 1.2e-2), err
 
 
+@pytest.mark.parametrize("splits", [2, 8, 9, 17, 32])
+@pytest.mark.parametrize("dk,dv", [(64, 40), (256, 256)])
+def test_any_number_of_splits_is_joined(monkeypatch, splits, dk, dv):
+    from litinfer_amd.kernels import ops
+    rounds = 1 if dk > 128 else 2                      # (blocks a compute unit)
+    monkeypatch.setattr(ops, "_single_blocks", lambda *a: rounds * ops._compute_units(torch.device(DEV)) // splits)
+    got, ref = _attention_case(torch.bfloat16, [(4200, 1), (3, 1), (900, 1)], 6, 2, dk, dv, 16, 0, seed=splits, heads_kernel=False, sinks=True)
+    err = float(np.abs(got - ref).max() / np.abs(ref).max())
+    assert err < 1.2e-2, err
+
+
 @pytest.mark.parametrize("dt", ["float32", "bfloat16"])
 @pytest.mark.parametrize("T,nh,n_out,n_in", [(1, 3, 12, 28), (40, 2, 64, 96), (33, 5, 20, 16), (70, 4, 128, 64), (17, 1, 7, 5)])
 def test_per_head_products_with_a_gate_an_element(dt, T, nh, n_out, n_in):

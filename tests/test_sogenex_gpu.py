@@ -594,6 +594,15 @@ def test_difference_of_two_maps_in_a_decoding_step(ctxs, nh, nkv, dk, dv, page, 
     assert not ops.masked_attention_difference(qd.view(-1), q.shape[1], dk, nh * dk, out, k1, k2, v, meta, *args, 0.37, 1e-5, 0.8, ws)
 
 
+@pytest.mark.parametrize("splits", [2, 8, 9, 32])
+@pytest.mark.parametrize("dk,dv", [(64, 64), (320, 256)])
+def test_any_number_of_splits_of_two_maps_is_joined(monkeypatch, splits, dk, dv):
+    from litinfer_amd.kernels import ops
+    units = ops._compute_units(torch.device(DEV)) * (2 if dk < 256 else 1)
+    monkeypatch.setattr(ops, "_single_blocks", lambda *a: units // 2 // splits)
+    test_difference_of_two_maps_in_a_decoding_step([4200, 3, 900], 6, 2, dk, dv, 16, 0, 0, 0.0)
+
+
 @pytest.mark.parametrize("fill", [float("inf"), float("nan")])
 @pytest.mark.parametrize("nh,nkv,dk,dv,window,keep", [(12, 2, 128, 128, 0, 0), (12, 12, 64, 64, 0, 0), (4, 1, 320, 256, 0, 0), (8, 2, 64, 128, 40, 3)])
 def test_rows_that_are_not_the_request_s_own_do_not_reach_it(nh, nkv, dk, dv, window, keep, fill):
