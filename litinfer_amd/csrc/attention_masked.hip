@@ -1343,42 +1343,101 @@ extern "C" int li_masked_attention_single_pair(const float* q, int q_token_strid
 // long).  Us, 8 tokens piece by piece whatever there are / as it is now: 12 heads of 128 x 256, float32, 2 / 8 / 16 tokens
 // 9.8 / 11.2 / 11.2 -> 6.9 / 8.5 / 8.5; 4 of 512 x 520, bfloat16, 8 tokens 20.0 -> 12.1; 28 of 512 x 128, float32, 16 tokens 8.3 -> 7.8;
 // four a block would take 15.5 there instead of 13.2 at 33 tokens, and 58.9 instead of 46.9 at 500 of 4 x 512 x 520.  Sums
-// are float32, in the order of k.
+// are float32, in the order of k.  One or two tokens' blocks ask for their first pieces before the inputs have come: 1 token, 12 heads of
+// 128 x 256, bfloat16, 5.1 -> 3.9; 2 tokens, float32 inputs, 5.8 -> 4.75 (four tokens' sums leave no registers for it: 5 % longer).
 #define HL_TOK 8
 #define HL_FEW 16
 #define HL_AHEAD 8
+// bfloat16 inputs from two tokens on, float32 ones (which are rounded there) from 16 on take the matrix cores, below, where the sizes allow: their
+// products are exact and their sums float32 as here.  12 heads of 128 x 256, bfloat16, 2 / 8 / 15 tokens 6.4 / 9.2 / 9.0 -> 3.8 / 3.95 / 4.05 (one token
+// would be 3.9 in either).  Up to HL_SPREAD tiles (three quarters of it for float32 inputs, whose loads are twice as long) a wave is a block.
+#define HL_SPREAD 1024
+#define HL_MFMA_FROM 2
 
 // Behind a head's n_in inputs may lie `n` more columns that are not multiplied but ROTATED by the token's angles
 // (cos, sin [T, n / 2]) and written behind the head's n_out outputs: pairs of neighbouring columns, or (split)
 // column i with column i + n / 2.
 struct HeadTail { int n; int split; const float* cosv; const float* sinv; };
 
+// The pairs of a head's `nt` tokens from t0 on, dealt to the threads of the z blocks behind the products' (first, n: this thread's number
+// among theirs and their number): blocks of their own, so that no product waits for the angles.  A thread asks for four pairs at once.
+#define TAIL_AT_ONCE 4
 template <typename TX, typename TO>
-__device__ __forceinline__ void head_tail_rotate(const TX* __restrict__ src, TO* __restrict__ dst, int t, int i, const HeadTail& tail) {
-    const int half = tail.n / 2, a = tail.split ? i : 2 * i, b = tail.split ? i + half : 2 * i + 1;
-    const float c = tail.cosv[(size_t)t * half + i], sn = tail.sinv[(size_t)t * half + i];
-    const float u = load_as_float(src + a), v = load_as_float(src + b);
-    store_from_float(dst + a, fmaf(u, c, -__fmul_rn(v, sn)));
-    store_from_float(dst + b, fmaf(v, c, __fmul_rn(u, sn)));
+__device__ __forceinline__ void head_tail_rotate(const TX* __restrict__ x, long x_token_stride, TO* __restrict__ out, long o_token_stride, int t0, int nt,
+                                                 int first, int n, const HeadTail& tail) {
+    const int half = tail.n / 2;
+    for (int u0 = first; u0 < nt * half; u0 += TAIL_AT_ONCE * n) {
+        float c[TAIL_AT_ONCE], sn[TAIL_AT_ONCE], u[TAIL_AT_ONCE], v[TAIL_AT_ONCE];
+#pragma unroll
+        for (int e = 0; e < TAIL_AT_ONCE; ++e) {
+            const int w = u0 + e * n < nt * half ? u0 + e * n : u0, tt = w / half, i = w % half;
+            const TX* src = x + (size_t)(t0 + tt) * x_token_stride;
+            c[e] = tail.cosv[(size_t)(t0 + tt) * half + i];
+            sn[e] = tail.sinv[(size_t)(t0 + tt) * half + i];
+            u[e] = load_as_float(src + (tail.split ? i : 2 * i));
+            v[e] = load_as_float(src + (tail.split ? i + half : 2 * i + 1));
+        }
+#pragma unroll
+        for (int e = 0; e < TAIL_AT_ONCE; ++e) {
+            const int w = u0 + e * n, tt = w / half, i = w % half;
+            if (w >= nt * half) break;
+            TO* dst = out + (size_t)(t0 + tt) * o_token_stride;
+            store_from_float(dst + (tail.split ? i : 2 * i), fmaf(u[e], c[e], -__fmul_rn(v[e], sn[e])));
+            store_from_float(dst + (tail.split ? i + half : 2 * i + 1), fmaf(v[e], c[e], __fmul_rn(u[e], sn[e])));
+        }
+    }
+}
+// z blocks of `threads` threads that the pairs of up to `tokens` tokens take
+static int tail_blocks(const HeadTail& tail, int tokens, int threads) {
+    const long each = (long)TAIL_AT_ONCE * threads, n = ((long)tokens * (tail.n / 2) + each - 1) / each;
+    return (int)(n < 16 ? n : 16);
 }
 
 template <typename TX, typename TM, typename TO, bool VEC, int TOK>
 __global__ __launch_bounds__(256) void headwise_linear_kernel(
     const TX* __restrict__ x, long x_token_stride, int x_head_stride, const TM* __restrict__ m, TO* __restrict__ out,
     long o_token_stride, int o_head_stride, int T_, int n_out, int n_in, const float* __restrict__ gate, long gate_stride,
-    int gate_per_column, HeadTail tail) {
+    int gate_per_column, HeadTail tail, int zs) {
     extern __shared__ float xs[];                    // [TOK][n_in]
     const int h = blockIdx.y, t0 = blockIdx.x * TOK;
     const int nt = (T_ - t0 < TOK) ? T_ - t0 : TOK;
-    if (tail.n > 0 && blockIdx.z == 0)
-        for (int u = threadIdx.x; u < nt * (tail.n / 2); u += 256) {
-            const int tt = u / (tail.n / 2), i = u % (tail.n / 2);
-            head_tail_rotate(x + (size_t)(t0 + tt) * x_token_stride + (size_t)h * x_head_stride + n_in,
-                             out + (size_t)(t0 + tt) * o_token_stride + (size_t)h * o_head_stride + n_out, t0 + tt, i, tail);
+    if ((int)blockIdx.z >= zs) {
+        head_tail_rotate(x + (size_t)h * x_head_stride + n_in, x_token_stride, out + (size_t)h * o_head_stride + n_out, o_token_stride, t0, nt,
+                         ((int)blockIdx.z - zs) * 256 + (int)threadIdx.x, ((int)gridDim.z - zs) * 256, tail);
+        return;
+    }
+    constexpr int E = VEC ? 16 / (int)sizeof(TM) : 1;
+    constexpr bool AHEAD = VEC && TOK < HL_TOK, EARLY = TOK <= 2;
+    const int part = threadIdx.x & 3, pieces = n_in / E;       // (VEC: a whole number; a thread takes the pieces part, part + 4, ...)
+    [[maybe_unused]] uint4 raw[HL_AHEAD];
+    auto ask = [&](int j, int c0) {
+        const TM* row = m + ((size_t)h * n_out + (j < n_out ? j : 0)) * n_in;
+#pragma unroll
+        for (int u = 0; u < HL_AHEAD; ++u) raw[u] = *reinterpret_cast<const uint4*>(row + (size_t)(c0 + 4 * u < pieces ? c0 + 4 * u : pieces - 1) * E);
+    };
+    const int j_first = blockIdx.z * 64 + (threadIdx.x >> 2);
+    if constexpr (AHEAD && EARLY) ask(j_first, part);         // (on its way beside the tokens' inputs)
+    if constexpr (EARLY) {
+        for (int i0 = threadIdx.x; i0 < TOK * n_in; i0 += 256 * 4) {
+            float v[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                int tt = 0, k = i0 + 256 * e < TOK * n_in ? i0 + 256 * e : 0;
+#pragma unroll
+                for (int x_ = 1; x_ < TOK; ++x_)
+                    if (k >= n_in) { k -= n_in; ++tt; }
+                v[e] = load_as_float(x + (size_t)(t0 + (tt < nt ? tt : 0)) * x_token_stride + (size_t)h * x_head_stride + k);
+                if (tt >= nt) v[e] = 0.f;
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (i0 + 256 * e < TOK * n_in) xs[i0 + 256 * e] = v[e];
         }
-    for (int i = threadIdx.x; i < TOK * n_in; i += 256) {
-        const int tt = i / n_in, k = i % n_in;
-        xs[i] = tt < nt ? load_as_float(x + (size_t)(t0 + tt) * x_token_stride + (size_t)h * x_head_stride + k) : 0.f;
+    } else {
+        for (int i = threadIdx.x; i < TOK * n_in; i += 256) {
+            const int tt = i / n_in, k = i % n_in;
+            xs[i] = tt < nt ? load_as_float(x + (size_t)(t0 + tt) * x_token_stride + (size_t)h * x_head_stride + k) : 0.f;
+        }
     }
     // the heads' gates are asked for before the products, so that they have arrived when the outputs are ready
     float gf[TOK];
@@ -1386,9 +1445,7 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
     for (int tt = 0; tt < TOK; ++tt) gf[tt] = gate && !gate_per_column ? gate[(size_t)(t0 + (tt < nt ? tt : 0)) * gate_stride + h] : 0.f;
     __syncthreads();
     // four neighbouring threads share an output: each takes every fourth piece of the matrix row
-    constexpr int E = VEC ? 16 / (int)sizeof(TM) : 1;
-    const int part = threadIdx.x & 3;
-    for (int j = blockIdx.z * 64 + (threadIdx.x >> 2); j < n_out + 63; j += gridDim.z * 64) {       // (whole groups of four go round together)
+    for (int j = j_first; j < n_out + 63; j += zs * 64) {       // (whole groups of four go round together)
         const bool on = j < n_out;
         const TM* row = m + ((size_t)h * n_out + (on ? j : 0)) * n_in;
         float acc[TOK];
@@ -1413,12 +1470,9 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
 #pragma unroll
                 for (int tt = 0; tt < TOK; ++tt) acc[tt] = fmaf(wv[e], xs[tt * n_in + k + e], acc[tt]);
         };
-        if constexpr (VEC && TOK < HL_TOK) {
-            const int pieces = n_in / E;             // (a whole number; a thread takes the pieces part, part + 4, ...)
+        if constexpr (AHEAD) {
             for (int c0 = part; c0 < pieces; c0 += 4 * HL_AHEAD) {
-                uint4 raw[HL_AHEAD];
-#pragma unroll
-                for (int u = 0; u < HL_AHEAD; ++u) raw[u] = *reinterpret_cast<const uint4*>(row + (size_t)(c0 + 4 * u < pieces ? c0 + 4 * u : pieces - 1) * E);
+                if (!EARLY || j != j_first || c0 != part) ask(j, c0);
 #pragma unroll
                 for (int u = 0; u < HL_AHEAD; ++u) {
                     if ((c0 + 4 * u) * E >= n_in) break;
@@ -1461,55 +1515,85 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
 // 32: a wave takes 32 tokens and 32 outputs of one head and works on the transposed tile (outputs x tokens), so
 // that both operands are 16-byte pieces of rows as they lie in memory (a matrix row's k-values; a token's
 // inputs, rounded to bfloat16 if they are float32) and a lane ends with four consecutive outputs of its token.
-template <typename TX, typename TO>
-__global__ __launch_bounds__(256) void headwise_linear_mfma_kernel(
+// A wave asks for HL_STEPS k-steps of both operands, and for the gates, at once, and is a block by itself where there are few; as a chain of a
+// trip a step, four waves a block and the rotated columns in the first block, us before and now: 32 tokens, 12 heads of 128 x 256 bfloat16 6.4 ->
+// 4.1, of 256 x 128 with float32 inputs 5.2 -> 4.2; 200 tokens 6.8 -> 5.2 and 5.7 -> 5.15; the same from 1,000 on, where float32 inputs
+// go a step at a time as before (eight at once: 14.6 -> 15.2, 39.0 -> 46.0 at 3,000).
+template <typename TX, typename TO, int HL_STEPS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void headwise_linear_mfma_kernel(
     const TX* __restrict__ x, long x_token_stride, int x_head_stride, const bf16_t* __restrict__ m, TO* __restrict__ out,
     long o_token_stride, int o_head_stride, int T_, int n_out, int n_in, const float* __restrict__ gate, long gate_stride,
-    int gate_per_column, HeadTail tail) {
+    int gate_per_column, HeadTail tail, int zs) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ql = lane & 31, h2 = lane >> 5;
     const int head = blockIdx.y, t0 = blockIdx.x * 32;
-    if (tail.n > 0 && blockIdx.z == 0) {
-        const int nt = (T_ - t0 < 32) ? T_ - t0 : 32;
-        for (int u = threadIdx.x; u < nt * (tail.n / 2); u += 256) {
-            const int tt = u / (tail.n / 2), i = u % (tail.n / 2);
-            head_tail_rotate(x + (size_t)(t0 + tt) * x_token_stride + (size_t)head * x_head_stride + n_in,
-                             out + (size_t)(t0 + tt) * o_token_stride + (size_t)head * o_head_stride + n_out, t0 + tt, i, tail);
-        }
+    if ((int)blockIdx.z >= zs) {
+        head_tail_rotate(x + (size_t)head * x_head_stride + n_in, x_token_stride, out + (size_t)head * o_head_stride + n_out, o_token_stride, t0,
+                         T_ - t0 < 32 ? T_ - t0 : 32, ((int)blockIdx.z - zs) * 64 * WAVES + (int)threadIdx.x, ((int)gridDim.z - zs) * 64 * WAVES, tail);
+        return;
     }
-    const int j0 = (blockIdx.z * 4 + w) * 32;
+    const int j0 = (blockIdx.z * WAVES + w) * 32;
     if (j0 >= n_out) return;
     const int tok = t0 + ql < T_ ? t0 + ql : T_ - 1;
     const TX* xrow = x + (size_t)tok * x_token_stride + (size_t)head * x_head_stride + 8 * h2;
     const bf16_t* mrow = m + ((size_t)head * n_out + j0 + ql) * n_in + 8 * h2;
+    float head_gate = 0.f;
+    float4 gates[4];
+    auto ask_gates = [&]() {
+        if (gate && gate_per_column) {             // (a lane's outputs come in fours: 16-byte pieces of the gates' row)
+            const float* grow = gate + (size_t)tok * gate_stride + (size_t)head * n_out + j0 + 4 * h2;
+#pragma unroll
+            for (int rg = 0; rg < 4; ++rg) gates[rg] = *reinterpret_cast<const float4*>(grow + 8 * rg);
+        } else if (gate) {
+            head_gate = gate[(size_t)tok * gate_stride + head];
+        }
+    };
+    if constexpr (HL_STEPS > 1) ask_gates();
     ma_f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
-    for (int k = 0; k < n_in; k += 16) {
-        ma_frag8 a, b;
-        a.raw = *reinterpret_cast<const uint4*>(mrow + k);
-        if constexpr (sizeof(TX) == 2) {
-            b.raw = *reinterpret_cast<const uint4*>(xrow + k);
-        } else {
-            const float4 u = *reinterpret_cast<const float4*>(xrow + k);
-            const float4 v = *reinterpret_cast<const float4*>(xrow + k + 4);
-            b.w[0] = pack2_bf16(u.x, u.y); b.w[1] = pack2_bf16(u.z, u.w);
-            b.w[2] = pack2_bf16(v.x, v.y); b.w[3] = pack2_bf16(v.z, v.w);
+    // (whole: no step is past the end.  Else both operands of those that are are zeros: a question a step would have its loads wait for it)
+    auto steps = [&](int k0, auto whole_tag) {
+        constexpr bool WHOLE = decltype(whole_tag)::value;
+        ma_frag8 a[HL_STEPS], b[HL_STEPS];
+        [[maybe_unused]] float4 u[HL_STEPS][2];
+#pragma unroll
+        for (int i = 0; i < HL_STEPS; ++i) {
+            const int k = WHOLE || k0 + 16 * i < n_in ? k0 + 16 * i : n_in - 16;
+            a[i].raw = *reinterpret_cast<const uint4*>(mrow + k);
+            if constexpr (sizeof(TX) == 2) {
+                b[i].raw = *reinterpret_cast<const uint4*>(xrow + k);
+            } else {
+                u[i][0] = *reinterpret_cast<const float4*>(xrow + k);
+                u[i][1] = *reinterpret_cast<const float4*>(xrow + k + 4);
+            }
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, acc, 0, 0, 0);
-    }
+#pragma unroll
+        for (int i = 0; i < HL_STEPS; ++i) {
+            if constexpr (sizeof(TX) != 2) {
+                b[i].w[0] = pack2_bf16(u[i][0].x, u[i][0].y); b[i].w[1] = pack2_bf16(u[i][0].z, u[i][0].w);
+                b[i].w[2] = pack2_bf16(u[i][1].x, u[i][1].y); b[i].w[3] = pack2_bf16(u[i][1].z, u[i][1].w);
+            }
+            if (!WHOLE && k0 + 16 * i >= n_in) a[i].raw = b[i].raw = uint4{0u, 0u, 0u, 0u};
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i].v, b[i].v, acc, 0, 0, 0);
+        }
+    };
+    int k0 = 0;
+    for (; k0 + 16 * HL_STEPS <= n_in; k0 += 16 * HL_STEPS) steps(k0, std::true_type{});
+    if constexpr (HL_STEPS > 1)
+        if (k0 < n_in) steps(k0, std::false_type{});
     if (t0 + ql >= T_) return;
-    if (gate && gate_per_column) {                 // (a lane's outputs come in fours: 16-byte pieces of the gates' row)
-        const float* grow = gate + (size_t)(t0 + ql) * gate_stride + (size_t)head * n_out + j0 + 4 * h2;
+    if constexpr (HL_STEPS == 1) ask_gates();
+    if (gate && gate_per_column) {
 #pragma unroll
         for (int rg = 0; rg < 4; ++rg) {
-            const float4 g = *reinterpret_cast<const float4*>(grow + 8 * rg);
+            const float4 g = gates[rg];
             acc[4 * rg] *= 1.0f / (1.0f + expf(-g.x));
             acc[4 * rg + 1] *= 1.0f / (1.0f + expf(-g.y));
             acc[4 * rg + 2] *= 1.0f / (1.0f + expf(-g.z));
             acc[4 * rg + 3] *= 1.0f / (1.0f + expf(-g.w));
         }
     } else if (gate) {
-        const float f = 1.0f / (1.0f + expf(-gate[(size_t)(t0 + ql) * gate_stride + head]));
+        const float f = 1.0f / (1.0f + expf(-head_gate));
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[r] *= f;
     }
@@ -1531,13 +1615,18 @@ template <typename TX, typename TO>
 static bool headwise_mfma(const void* x, long xts, int xhs, const void* m, void* out, long ots, int ohs, int T_, int nh,
                           int n_out, int n_in, const float* gate, long gate_stride, int gate_per_column, HeadTail tail, hipStream_t stream) {
     const int ex = 16 / (int)sizeof(TX) / 2 * 2, eo = 4;       // elements that the 16-byte (32-byte) loads and the stores must start on
-    if (T_ < 16 || n_in % 16 || n_out % 32 || xts % ex || xhs % ex || ots % eo || ohs % eo ||
+    if (T_ < (sizeof(TX) == 2 ? HL_MFMA_FROM : 16) || n_in % 16 || n_out % 32 || xts % ex || xhs % ex || ots % eo || ohs % eo ||
         (uintptr_t)x % 16 || (uintptr_t)m % 16 || (uintptr_t)out % 16 ||
         (gate && gate_per_column && (gate_stride % 4 || (uintptr_t)gate % 16)))
         return false;
-    const dim3 grid((T_ + 31) / 32, nh, (n_out + 127) / 128);
-    headwise_linear_mfma_kernel<TX, TO><<<grid, 256, 0, stream>>>((const TX*)x, xts, xhs, (const bf16_t*)m, (TO*)out, ots, ohs,
-                                                                  T_, n_out, n_in, gate, gate_stride, gate_per_column, tail);
+    // (so few tiles that each takes a compute unit of its own: a wave a block)
+    const long rows = (T_ + 31) / 32, tiles = rows * nh * (n_out / 32);
+    const int waves = tiles <= (sizeof(TX) == 2 ? HL_SPREAD : HL_SPREAD / 4 * 3) ? 1 : 4, zs = (n_out + 32 * waves - 1) / (32 * waves);
+    const dim3 grid((unsigned)rows, nh, zs + tail_blocks(tail, T_ < 32 ? T_ : 32, 64 * waves));
+#define HL_MFMA(STEPS, WAVES) headwise_linear_mfma_kernel<TX, TO, STEPS, WAVES><<<grid, 64 * WAVES, 0, stream>>>(         \
+        (const TX*)x, xts, xhs, (const bf16_t*)m, (TO*)out, ots, ohs, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail, zs)
+    if (waves == 1) HL_MFMA(8, 1); else HL_MFMA((sizeof(TX) == 2 ? 8 : 1), 4);
+#undef HL_MFMA
     return true;
 }
 
@@ -1558,12 +1647,12 @@ extern "C" int li_headwise_linear(const void* x, int x_dtype, long x_token_strid
         else if (x_dtype == LI_BF16 && out_dtype == LI_F32) took = headwise_mfma<bf16_t, float>(x, x_token_stride, x_head_stride, m, out, o_token_stride, o_head_stride, T_, nh, n_out, n_in, gate, gate_stride, gate_per_column, tail, stream);
         if (took) return li_launch_status();
     }
-    const int zs = (n_out + 63) / 64, tok = T_ <= 1 ? 1 : T_ <= 2 ? 2 : T_ <= HL_FEW ? 4 : HL_TOK;
-    const dim3 grid((T_ + tok - 1) / tok, nh, zs < 64 ? zs : 64);
+    const int all = (n_out + 63) / 64, zs = all < 64 ? all : 64, tok = T_ <= 1 ? 1 : T_ <= 2 ? 2 : T_ <= HL_FEW ? 4 : HL_TOK;
+    const dim3 grid((T_ + tok - 1) / tok, nh, zs + tail_blocks(tail, T_ < tok ? T_ : tok, 256));
     const size_t lds = (size_t)tok * n_in * 4;
 #define HL_AS(TX, TM, TO, VEC, TOK)                                                                                        \
     headwise_linear_kernel<TX, TM, TO, VEC, TOK><<<grid, 256, lds, stream>>>(                                              \
-        (const TX*)x, x_token_stride, x_head_stride, (const TM*)m, (TO*)out, o_token_stride, o_head_stride, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail)
+        (const TX*)x, x_token_stride, x_head_stride, (const TM*)m, (TO*)out, o_token_stride, o_head_stride, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail, zs)
 #define HL_GO(TX, TM, TO)                                                                                                  \
     {                                                                                                                      \
         constexpr int E = 16 / sizeof(TM);                                                                                 \

@@ -375,6 +375,37 @@ def test_layer_norm_gelu_rows_side_by_side_and_gated_products():
         assert np.abs(out.float().cpu().numpy().reshape(T, nh, n_out) - ref).max() < (1e-5 if dt is torch.float32 else 2e-2) * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("T,nh,n_out,n_in,tail", [(1, 3, 96, 272, 10), (2, 3, 96, 272, 0), (2, 1, 32, 16, 2), (4, 2, 64, 144, 6), (15, 5, 32, 128, 64), (16, 2, 64, 48, 2),
+                                                  (31, 4, 128, 512, 0), (33, 2, 96, 80, 34), (70, 16, 512, 16, 8)])
+@pytest.mark.parametrize("gate", [None, "head", "column"])
+@pytest.mark.parametrize("xdt,odt", [("bfloat16", "bfloat16"), ("bfloat16", "float32"), ("float32", "float32")])
+def test_per_head_products_from_one_token_on(T, nh, n_out, n_in, tail, gate, xdt, odt):
+    from litinfer_amd.kernels import ops
+    rng = np.random.default_rng(n_in + T)
+    f32 = lambda a: torch.tensor(a, dtype=torch.float32, device=DEV)
+    pad = -tail % 8                                                               # (rows that start on 16 bytes)
+    m = torch.tensor(rng.normal(size=(nh, n_out, n_in)) / n_in ** 0.5, dtype=torch.float32).to(torch.bfloat16)
+    x = torch.tensor(rng.normal(size=(T, nh, n_in + tail + pad)), dtype=torch.float32).to(getattr(torch, xdt))
+    ang = rng.normal(size=(T, tail // 2))
+    out = torch.full((T, nh, n_out + tail + pad), 7.0, dtype=getattr(torch, odt), device=DEV)
+    g = None if gate is None else f32(rng.normal(size=(T, nh * (n_out if gate == "column" else 1))))
+    ops.headwise_linear(x.to(DEV).view(T, -1), nh * (n_in + tail + pad), n_in + tail + pad, m.to(DEV), out.view(T, -1), nh * (n_out + tail + pad), n_out + tail + pad, T,
+                        gate=g, gate_columns=gate == "column", rotate_tail=(tail, f32(np.cos(ang)), f32(np.sin(ang)), False) if tail else None)
+    got, xs = out.double().cpu().numpy(), x.double().numpy()
+    ref = np.einsum("hjk,thk->thj", m.double().numpy(), xs[:, :, :n_in])
+    if g is not None:
+        ref = ref * plain.sigmoid(g.double().cpu().numpy()).reshape(T, nh, -1)
+    # float32 sums of products that are exact; a bfloat16 has eight bits, so rounding to it costs up to 2^-8: a result's, and each input's that is
+    # float32 from 16 tokens on, whose errors add up like the square root of their number, as the products do
+    each = (2 ** -8 if odt == "bfloat16" else 0.0) + (2 ** -8 if xdt == "float32" and T >= 16 else 0.0) + 3e-6
+    assert np.abs(got[:, :, :n_out] - ref).max() < each * max(np.abs(ref).max(), 2.0)
+    if tail:
+        r, c, s = xs[:, :, n_in:n_in + tail], np.cos(ang)[:, None], np.sin(ang)[:, None]
+        want = np.stack([r[..., 0::2] * c - r[..., 1::2] * s, r[..., 1::2] * c + r[..., 0::2] * s], -1).reshape(T, nh, tail)
+        assert np.abs(got[:, :, n_out:n_out + tail] - want).max() < (2 ** -8 if odt == "bfloat16" else 2e-6) * max(1.0, np.abs(want).max())
+    assert (got[:, :, n_out + tail:] == 7.0).all()
+
+
 @pytest.mark.parametrize("split", [False, True])
 @pytest.mark.parametrize("T,nh,n_out,n_in,tail,mdt", [(5, 3, 40, 24, 8, torch.float32), (70, 4, 64, 32, 64, torch.bfloat16),
                                                       (33, 2, 20, 48, 2, torch.bfloat16), (200, 8, 192, 64, 32, torch.bfloat16)])
