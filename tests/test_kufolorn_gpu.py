@@ -442,6 +442,11 @@ def test_delta_rule_across_steps_and_slots(heads, groups, N, vdim, chunked):
     assert torch.all(state[1] == 7.0)
 
 
+@pytest.mark.parametrize("heads,groups,N,vdim", [(2, 1, 256, 64), (3, 3, 100, 40), (4, 4, 64, 64), (3, 3, 48, 36)])
+def test_delta_rule_in_chunks_with_half_the_state_values_a_lane(heads, groups, N, vdim):
+    test_delta_rule_across_steps_and_slots(heads, groups, N, vdim, True)
+
+
 @pytest.mark.parametrize("heads,N,vdim", [(3, 12, 20), (2, 64, 32), (4, 128, 64), (1, 20, 8), (2, 16, 16)])
 def test_retention_is_the_recurrence_with_a_fixed_decay(heads, N, vdim):
     """Portions up to 100 tokens (chunks that run side by side) and single tokens, on two slots."""
