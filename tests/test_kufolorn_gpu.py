@@ -447,6 +447,25 @@ def test_delta_rule_in_chunks_with_half_the_state_values_a_lane(heads, groups, N
     test_delta_rule_across_steps_and_slots(heads, groups, N, vdim, True)
 
 
+@pytest.mark.parametrize("N,vdim", [(64, 48), (64, 20), (40, 32), (128, 16), (128, 40), (100, 64), (256, 16), (192, 24)])
+def test_delta_rule_carried_over_many_chunks(N, vdim):
+    """Requests of one to eight chunks, side by side, give what the recurrence in one piece gives."""
+    from litinfer_amd.engine.workspace import Workspace
+    from litinfer_amd.kernels import ops
+    rng = np.random.default_rng(N + vdim)
+    heads, lens = 3, [1, 64, 65, 128, 200, 321, 450, 512]
+    x, ba = _f32(rng.normal(size=(sum(lens), heads * (vdim + 2 * N)))), _f32(rng.normal(size=(sum(lens), 2 * heads)))
+    bias, a_log, begun = _f32(rng.normal(0, 0.5, heads)), _f32(rng.uniform(-5, 0, heads)), rng.normal(size=(len(lens), heads, N, vdim))
+    out, states = [], []
+    for ws in (None, Workspace(DEV)):
+        state, y = _f32(begun), torch.empty(sum(lens), heads * vdim, device=DEV)
+        ops.delta_scan(x, ba, bias, a_log, state, _ctx(lens, list(range(len(lens)))), y, heads, vdim, N, heads, N ** -0.5, ws=ws)
+        out.append(y.cpu().numpy())
+        states.append(state.cpu().numpy())
+    for a, b in (out, states):
+        assert np.abs(a - b).max() < 2e-5 * max(1.0, np.abs(a).max())
+
+
 @pytest.mark.parametrize("heads,N,vdim", [(3, 12, 20), (2, 64, 32), (4, 128, 64), (1, 20, 8), (2, 16, 16)])
 def test_retention_is_the_recurrence_with_a_fixed_decay(heads, N, vdim):
     """Portions up to 100 tokens (chunks that run side by side) and single tokens, on two slots."""
