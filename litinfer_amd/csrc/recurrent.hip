@@ -1362,7 +1362,7 @@ __global__ __launch_bounds__(64 * SSM_WAVES) void delta_scan_kernel(
 // LDS, chunk after chunk: S_in(c + 1) = P_c S_in(c) + S_own(c), on the float32 matrix cores (v_mfma_f32_16x16x4_f32: row
 // operand P, one value a lane (row lane % 16, k lane / 16), which lie side by side in a row of the stored transpose; column
 // operand the state from LDS; the accumulator starts as S_own and holds rows 4 (lane / 16) + r of column lane % 16).  A
-// wave owns RT tiles of 16 rows; P comes in groups of 64 k's, as many as RT.  Up to 128 rows a chunk's P and S_own are asked for while
+// wave owns RT tiles of 16 rows; P comes in groups of 64 k's, as many as RT (up to 128 rows, 128 k's).  A chunk's P and S_own are asked for while
 // the chunk before it is worked on (they do not depend on the state), without a question about it, and where the sizes are whole (WHOLE) nothing else is
 // asked either: the loads on their way can then be counted, and less than 64 of them (a lane's rows lie side by side) fit the counter.
 // Bound by those trips: asked for under questions, every group waited for the next one as well.  Blocks are numbered head by head: numbered
@@ -1375,7 +1375,7 @@ template <int RT, bool WHOLE>
 __global__ __launch_bounds__(256) void delta_carry_kernel(
     float* __restrict__ carry, const float* __restrict__ pmat, const float* __restrict__ state, const int* __restrict__ slots,
     const int* __restrict__ q_len, const int* __restrict__ chunk_first, int heads, int vdim, int N, int Q) {
-    constexpr int GROUPS = RT, AHEAD = RT == 4 ? 1 : RT;      // groups of a chunk; groups that are on their way
+    constexpr int GROUPS = RT;                          // of a chunk, all of them on their way
     __shared__ float run[64 * GROUPS * 16];             // [N rounded up][16]
     const int cols = (vdim + 15) / 16, head = blockIdx.x % heads, c0 = blockIdx.x / heads % cols * 16, seg = blockIdx.x / heads / cols;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, cl = lane & 15, kq = lane >> 4, col = c0 + cl;
@@ -1391,7 +1391,7 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
     const int row0 = 16 * RT * w;
     auto arow = [&](int rt) { const int r = row0 + RT * cl + rt; return WHOLE || r < N ? r : N - 1; };      // a lane's row of P,
     auto crow = [&](int rt, int r) { return row0 + RT * (4 * kq + r) + rt; };                               // and of the result
-    float p[2][AHEAD][RT][DC_GROUP], own[2][RT][4];
+    float p[2][GROUPS][RT][DC_GROUP], own[RT][4];
     dc_f32x4 acc[RT];
     const int last = nch - 2;                           // (a request's last chunk only takes the state it begins with; chunks past it are asked for as that one)
     auto fetch = [&](int k, int g, float (&to)[RT][DC_GROUP]) {
@@ -1404,21 +1404,16 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
                 to[0][x] = v.x; to[1][x] = v.y;
                 continue;
             }
-            if constexpr (WHOLE && RT == 4) {
-                const float4 v = *reinterpret_cast<const float4*>(pt + (size_t)n * N + arow(0));
-                to[0][x] = v.x; to[1][x] = v.y; to[2][x] = v.z; to[3][x] = v.w;
-                continue;
-            }
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) to[rt][x] = pt[(size_t)n * N + arow(rt)];
         }
     };
-    auto own_of = [&](int k, float (&to)[RT][4]) {
+    auto own_of = [&](int k) {
         const float* at = carry + ((size_t)(base + (k < last ? k : last)) * heads + head) * N * vdim + (on ? col : 0);
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) to[rt][r] = at[(size_t)(WHOLE || crow(rt, r) < N ? crow(rt, r) : N - 1) * vdim];
+            for (int r = 0; r < 4; ++r) own[rt][r] = at[(size_t)(WHOLE || crow(rt, r) < N ? crow(rt, r) : N - 1) * vdim];
     };
     auto leave = [&](int k) {                           // the state with which chunk k begins
         float* at = carry + ((size_t)(base + k) * heads + head) * N * vdim + col;
@@ -1436,25 +1431,17 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
             for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[rt][x], b, acc[rt], 0, 0, 0);
         }
     };
-    // chunk k from cur, whose own state is in own[cur]; a chunk whose own state was read may be written: its place is the state it begins with
+    // chunk k from cur; a chunk whose own state was read may be written: its place is the state it begins with
     auto chunk = [&](int k, int cur) {
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[rt][r] = own[cur][rt][r];
-        own_of(k + 1, own[cur ^ 1]);
-        if constexpr (AHEAD == GROUPS) {
+            for (int r = 0; r < 4; ++r) acc[rt][r] = own[rt][r];
+        own_of(k + 1);
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g) fetch(k + 1, g, p[cur ^ 1][g]);
+        for (int g = 0; g < GROUPS; ++g) fetch(k + 1, g, p[cur ^ 1][g]);
 #pragma unroll
-            for (int g = 0; g < GROUPS; ++g) work(g, p[cur][g]);
-        } else {
-#pragma unroll
-            for (int g = 0; g < GROUPS; ++g) {
-                fetch(g + 1 < GROUPS ? k : k + 1, (g + 1) % GROUPS, p[(g + 1) & 1][0]);
-                work(g, p[g & 1][0]);
-            }
-        }
+        for (int g = 0; g < GROUPS; ++g) work(g, p[cur][g]);
         leave(k);
         __syncthreads();
 #pragma unroll
@@ -1465,9 +1452,9 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
         __syncthreads();
     };
     if (nch > 1) {
-        own_of(0, own[0]);
+        own_of(0);
 #pragma unroll
-        for (int g = 0; g < AHEAD; ++g) fetch(0, g, p[0][g]);
+        for (int g = 0; g < GROUPS; ++g) fetch(0, g, p[0][g]);
     }
     __syncthreads();
     for (int k = 0; k + 1 < nch; k += 2) {
@@ -1477,12 +1464,109 @@ __global__ __launch_bounds__(256) void delta_carry_kernel(
     leave(nch - 1);
 }
 
+// The same for more rows, whose chunks are too much for the registers: four tiles a wave, a group on its way while the one before it is used, across the
+// chunks' borders too.  (As above with a group ahead: 64 -> 80 us, 16 heads of 256 x 64, and 296 -> 398, 4 of 256 x 256 over 2,048 tokens.)
+__global__ __launch_bounds__(256) void delta_carry_wide_kernel(
+    float* __restrict__ carry, const float* __restrict__ pmat, const float* __restrict__ state, const int* __restrict__ slots,
+    const int* __restrict__ q_len, const int* __restrict__ chunk_first, int heads, int vdim, int N, int Q) {
+    constexpr int RT = 4;
+    extern __shared__ float run[];                      // [N rounded up to 64][16]
+    const int seg = blockIdx.x, head = blockIdx.y, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int cl = lane & 15, kq = lane >> 4, col = blockIdx.z * 16 + cl;
+    const int nch = (q_len[seg] + Q - 1) / Q, base = chunk_first[seg];
+    const bool on = col < vdim;
+    const int groups = (N + 4 * DC_GROUP - 1) / (4 * DC_GROUP);
+    const float* stp = state + ((size_t)slots[seg] * heads + head) * N * vdim;
+    for (int i = threadIdx.x; i < groups * 4 * DC_GROUP * 16; i += 256) {
+        const int n = i / 16, cc = blockIdx.z * 16 + i % 16;
+        run[i] = (n < N && cc < vdim) ? stp[(size_t)n * vdim + cc] : 0.f;
+    }
+    int arow[RT], crow[RT];                             // this lane's row of P (operand) and its first row of the result
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        const int r = 16 * (w * RT + rt);
+        arow[rt] = r + cl < N ? r + cl : N - 1;
+        crow[rt] = r + 4 * kq;
+    }
+    float pa[RT][DC_GROUP], pb[RT][DC_GROUP], own[RT][4];
+    dc_f32x4 acc[RT];
+    const int steps = (nch - 1) * groups;               // a request's last chunk only takes the state it begins with
+    auto fetch = [&](int st, float (&p)[RT][DC_GROUP]) {
+        if (st >= steps) return;
+        const float* pt = pmat + ((size_t)(base + st / groups) * heads + head) * N * N;
+        const int k0 = (st % groups) * 4 * DC_GROUP + kq;
+#pragma unroll
+        for (int x = 0; x < DC_GROUP; ++x) {
+            const int k = k0 + 4 * x < N ? k0 + 4 * x : N - 1;
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) p[rt][x] = pt[(size_t)k * N + arow[rt]];
+        }
+    };
+    auto own_of = [&](int k) {
+        if (k + 1 >= nch) return;
+        const float* at = carry + ((size_t)(base + k) * heads + head) * N * vdim + (on ? col : 0);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) own[rt][r] = at[(size_t)(crow[rt] + r < N ? crow[rt] + r : N - 1) * vdim];
+    };
+    auto leave = [&](int k) {                           // the state with which chunk k begins
+        float* at = carry + ((size_t)(base + k) * heads + head) * N * vdim + col;
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                if (on && crow[rt] + r < N) at[(size_t)(crow[rt] + r) * vdim] = run[(crow[rt] + r) * 16 + cl];
+    };
+    auto step = [&](int st, const float (&p)[RT][DC_GROUP]) {
+        const int k = st / groups, g = st % groups;
+        if (g == 0) {
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) acc[rt][r] = own[rt][r];
+            own_of(k + 1);
+            leave(k);
+        }
+#pragma unroll
+        for (int x = 0; x < DC_GROUP; ++x) {
+            const float b = run[(g * 4 * DC_GROUP + 4 * x + kq) * 16 + cl];
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) acc[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(p[rt][x], b, acc[rt], 0, 0, 0);
+        }
+        if (g == groups - 1) {
+            __syncthreads();
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (crow[rt] + r < N) run[(crow[rt] + r) * 16 + cl] = acc[rt][r];
+            __syncthreads();
+        }
+    };
+    fetch(0, pa);
+    own_of(0);
+    __syncthreads();
+    for (int st = 0; st < steps; st += 2) {
+        fetch(st + 1, pb);
+        step(st, pa);
+        fetch(st + 2, pa);
+        if (st + 1 < steps) step(st + 1, pb);
+    }
+    leave(nch - 1);
+}
+
 static void delta_carry_launch(float* carry, const float* pmat, const float* state, const int* slots, const int* q_len,
                                const int* chunk_first, int heads, int vdim, int N, int Q, int segs, hipStream_t stream) {
     const dim3 grid((unsigned)heads * ((vdim + 15) / 16) * segs);
 #define DC_AS(R_, W_) delta_carry_kernel<R_, W_><<<grid, 256, 0, stream>>>(carry, pmat, state, slots, q_len, chunk_first, heads, vdim, N, Q)
 #define DC_GO(R_) { if (N == 64 * R_ && vdim % 16 == 0) DC_AS(R_, true); else DC_AS(R_, false); }
-    if (N <= 64) DC_GO(1) else if (N <= 128) DC_GO(2) else DC_GO(4)
+    if (N <= 64) DC_GO(1)
+    else if (N <= 128) DC_GO(2)
+    else {
+        const size_t lds = (size_t)((N + 4 * DC_GROUP - 1) / (4 * DC_GROUP) * 4 * DC_GROUP) * 16 * sizeof(float);
+        delta_carry_wide_kernel<<<dim3(segs, heads, (vdim + 15) / 16), 256, lds, stream>>>(carry, pmat, state, slots, q_len, chunk_first, heads, vdim, N, Q);
+    }
 #undef DC_GO
 #undef DC_AS
 }
