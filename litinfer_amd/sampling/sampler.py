@@ -19,7 +19,9 @@ device.
 from __future__ import annotations
 
 import struct
+import threading
 from array import array
+from collections import deque
 from dataclasses import dataclass
 from operator import attrgetter
 from typing import List, Optional, Sequence
@@ -81,21 +83,42 @@ def _uniforms(seeds: Sequence[int], counters: Sequence[int]) -> np.ndarray:
     return (z >> np.uint64(40)).astype(np.float32) * np.float32(2.0 ** -24)
 
 
-_unread: List[tuple] = []               # (event, host memory) of results that were let go before they were there
+# (event, host memory) of results that a kernel writes to the host and that were let go before anybody had asked for them.  Until the event
+# has come the device may still write there, so the memory must not go back to torch's allocator (which knows of copies, not of kernels).
+_unread: "deque[tuple]" = deque()
+_unread_lock = threading.Lock()
+_DRAIN_AT_ONCE = 8                      # entries that a look takes; a call adds one at most, so what has been written does not pile up
+
+
+def _drain() -> None:
+    """Let go of memory of `_unread` that has been written by now.  An entry is taken out, asked, and put back if its event has not come: only the
+    holder of the lock takes entries out, so no entry goes that was not asked; a thread that finds the lock held leaves it to the holder."""
+    if not _unread or torch.cuda.is_current_stream_capturing() or not _unread_lock.acquire(blocking=False):
+        return
+    try:
+        for _ in range(min(len(_unread), _DRAIN_AT_ONCE)):
+            entry, done = _unread.popleft(), False
+            try:
+                done = entry[0].query()
+            finally:
+                if not done:
+                    _unread.append(entry)
+    finally:
+        _unread_lock.release()
 
 
 class PendingTokens:
     """Tokens that were chosen on the device and are on their way to the host."""
 
-    def __init__(self, sampler, host: torch.Tensor, n: int, event):
-        self._sampler, self._host, self._n, self._event = sampler, host, n, event
+    def __init__(self, sampler, host: torch.Tensor, n: int, event, by_kernel: bool = False):
+        """by_kernel: the host memory is written by the kernel that chooses the tokens, not by a copy."""
+        self._sampler, self._host, self._n, self._event, self._by_kernel = sampler, host, n, event, by_kernel
         self._tokens: Optional[List[int]] = None
 
-    def __del__(self):
-        # Nobody has asked for the tokens, and the device may not have written them yet: until it has, the memory is not free.  (A copy
-        # into pinned memory says so to torch's allocator; a kernel that writes there does not.)
-        if self._tokens is None and self._event is not None and not self._event.query():
-            _unread.append((self._event, self._host))
+    def __del__(self, keep=_unread.append):
+        # (the collector may run this anywhere, in a recording or in `_drain` itself: it takes no lock and asks the device nothing)
+        if self._by_kernel and self._tokens is None:
+            keep((self._event, self._host))
 
     def result(self) -> List[int]:
         """The tokens; waits for the device if they are not there yet."""
@@ -173,6 +196,7 @@ class Sampler:
         return PendingTokens(self, hb, n, ev)
 
     def _host_buffer(self, n: int) -> torch.Tensor:
+        _drain()
         for i, b in enumerate(self._free_host):
             if b.numel() >= n:
                 return self._free_host.pop(i)
@@ -184,9 +208,10 @@ class Sampler:
 
     def _call(self, logits: torch.Tensor, params: Sequence[SamplingParams], counters: Sequence[int], ids: torch.Tensor) -> Optional["PendingTokens"]:
         """The rows' options in the launch's arguments and the ids written to the host by the kernel that chooses them: no array, copy or
-        event to the device (of a step of 64 rows, 30 of the host's 52 us).  None where the options are not packed or the rows too many."""
+        event to the device (of a step of 64 rows, 30 of the host's 52 us).  None where the options are not packed or the rows too many, and
+        in a recording, whose replays would write to the host's memory of this call."""
         n = logits.shape[0]
-        if n > ops.SAMPLE_CALL_ROWS or not logits.is_cuda:
+        if n > ops.SAMPLE_CALL_ROWS or not logits.is_cuda or torch.cuda.is_current_stream_capturing():
             return None
         try:
             records, draws = b"".join(map(_PACKED, params)), array("Q", counters)
@@ -194,14 +219,9 @@ class Sampler:
             return None
         if len(records) != _RECORD.size * n:
             return None
-        while _unread and _unread[0][0].query():
-            try:
-                _unread.pop(0)
-            except IndexError:                       # (another thread's sampler was here first)
-                break
         hb = self._host_buffer(n)
         ops.sample_call(logits, records, draws, ids, hb)
-        return PendingTokens(self, hb, n, record_event())
+        return PendingTokens(self, hb, n, record_event(), by_kernel=True)
 
     def sample_async(self, logits: torch.Tensor, params: Sequence[SamplingParams], counters: Sequence[int],
                      out: Optional[torch.Tensor] = None) -> PendingTokens:

@@ -1,0 +1,103 @@
+"""What the sampler keeps on the host between a step and its result, with stand-ins for the device's events."""
+import threading
+import weakref
+
+import pytest
+import torch
+
+from litinfer_amd.sampling import Sampler, sampler
+
+
+class Event:
+    def __init__(self, done=False, wait=None):
+        self.done, self.wait = done, wait
+
+    def query(self):
+        if self.wait is not None:
+            self.wait()
+        return self.done
+
+
+@pytest.fixture(autouse=True)
+def nothing_unread(monkeypatch):
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)      # (there is no device to ask here)
+    sampler._unread.clear()
+    yield
+    sampler._unread.clear()
+
+
+def _let_go(event, by_kernel=True):
+    host = torch.empty(4, dtype=torch.int32)
+    seen = weakref.ref(host)
+    sampler.PendingTokens(Sampler("cpu"), host, 4, event, by_kernel=by_kernel)
+    del host
+    return seen
+
+
+def test_memory_of_an_unread_result_stays_until_the_device_has_written_it():
+    first, second = Event(), Event()
+    a, b = _let_go(first), _let_go(second)
+    smp = Sampler("cpu")
+    smp._host_buffer(4)
+    assert a() is not None and b() is not None
+    second.done = True
+    smp._host_buffer(4)                                    # (the entry at the head has not come: the one behind it goes all the same)
+    assert a() is not None and b() is None
+    first.done = True
+    smp._host_buffer(4)
+    assert a() is None and not sampler._unread
+
+
+def test_two_threads_never_drop_an_entry_that_was_not_asked():
+    both = threading.Barrier(2)
+
+    def meet():                                            # (until the other thread is here too, or is known not to come)
+        try:
+            both.wait(timeout=0.5)
+        except threading.BrokenBarrierError:
+            pass
+    kept = []
+    for _ in range(3):
+        both.reset()
+        _let_go(Event(done=True, wait=meet))
+        kept.append(_let_go(Event(done=False)))
+        threads = [threading.Thread(target=sampler._drain) for _ in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert all(k() is not None for k in kept)
+
+
+def test_an_event_that_cannot_be_asked_keeps_its_entry():
+    def broken():
+        raise RuntimeError("no answer")
+    a = _let_go(Event(wait=broken))
+    with pytest.raises(RuntimeError):
+        sampler._drain()
+    assert a() is not None and not sampler._unread_lock.locked()
+
+
+def test_a_recording_asks_no_event(monkeypatch):
+    a = _let_go(Event(done=True))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    Sampler("cpu")._host_buffer(4)
+    assert a() is not None
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    Sampler("cpu")._host_buffer(4)
+    assert a() is None
+
+
+def test_results_that_are_let_go_do_not_pile_up():
+    smp = Sampler("cpu")
+    for i in range(1000):
+        smp._host_buffer(4)
+        assert _let_go(Event(done=True), by_kernel=i % 2 == 0)() is None or i % 2 == 0
+        assert len(sampler._unread) <= 1
+    for _ in range(200):                                   # a device that stands still for a while
+        _let_go(Event(done=False))
+    for entry in sampler._unread:
+        entry[0].done = True
+    for _ in range(26):
+        smp._host_buffer(4)
+    assert not sampler._unread
