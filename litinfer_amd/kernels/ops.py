@@ -8,7 +8,9 @@ GPU, or without the built library, a call raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
+import threading
 from array import array
 from dataclasses import dataclass
 from ctypes import c_char_p, c_float, c_int, c_long, c_void_p
@@ -137,6 +139,7 @@ def _work_bytes(m: int, n: int, k: int, dtype: int) -> int:
     return int(f(m, n, k, dtype))
 
 
+@functools.lru_cache(maxsize=1024)
 def _sample_scratch_floats(n: int, v: int) -> int:
     f = _fn_cache.get(("sampling", "li_sample_rows_scratch_floats"))
     if f is None:
@@ -1774,8 +1777,27 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
 
 
 # ------------------------------------------------------------------ sampling
-_argmax_scratch = {}
-_sample_scratch = {}
+class _Scratch(threading.local):
+    """What the first of two kernels leaves for the second.  A thread's launches on a stream follow each other, so a buffer a thread and stream is
+    enough, however many samplers share it; it grows to the most that was asked for and goes with its thread."""
+    STREAMS = 8                        # streams of a thread whose buffers are kept
+
+    def __init__(self):
+        self.buffers: Dict[tuple, torch.Tensor] = {}
+
+    def floats(self, n: int, device: torch.device) -> torch.Tensor:
+        if torch.cuda.is_current_stream_capturing():
+            return torch.empty(n, dtype=torch.float32, device=device)       # (the recording's own: its replays use it whatever is asked for later)
+        key = (device, _stream())
+        buf = self.buffers.get(key)
+        if buf is None or buf.numel() < n:
+            if buf is None and len(self.buffers) >= self.STREAMS:
+                self.buffers.clear()
+            buf = self.buffers[key] = torch.empty(n if buf is None else max(n, buf.numel() * 3 // 2), dtype=torch.float32, device=device)
+        return buf
+
+
+_scratch = _Scratch()
 
 
 def argmax_rows(logits: torch.Tensor, out: torch.Tensor) -> None:
@@ -1785,13 +1807,9 @@ def argmax_rows(logits: torch.Tensor, out: torch.Tensor) -> None:
     _chk(out.dtype is torch.int32 and out.numel() == logits.shape[0] and out.is_contiguous(), "argmax: out")
     n = logits.shape[0]
     if n:
-        key = (logits.device, n)
-        if key not in _argmax_scratch:
-            _argmax_scratch[key] = (torch.empty(n * 32, dtype=torch.float32, device=logits.device),
-                                    torch.empty(n * 32, dtype=torch.int32, device=logits.device))
-        sv, si = _argmax_scratch[key]
-        _run("sampling", "li_argmax_rows", logits.data_ptr(), out.data_ptr(), sv.data_ptr(), si.data_ptr(),
-             n, logits.shape[1])
+        values = _scratch.floats(64 * n, logits.device)              # (32 values a row, then their 32 ids)
+        at = values.data_ptr()
+        _run("sampling", "li_argmax_rows", logits.data_ptr(), out.data_ptr(), at, at + 4 * 32 * n, n, logits.shape[1])
 
 
 def sample_rows(logits: torch.Tensor, temperature: torch.Tensor, top_k: torch.Tensor,
@@ -1839,24 +1857,16 @@ def sample_call(logits: torch.Tensor, records: bytes, counters: array, out: torc
     _chk(0 < n <= SAMPLE_CALL_ROWS and len(records) == 24 * n and len(counters) == n and counters.itemsize == 8, "sample: per-row options")
     _chk(out.dtype is torch.int32 and out.numel() == n and out.is_contiguous(), "sample: out")
     _chk(host.dtype is torch.int32 and host.numel() >= n and host.is_contiguous() and host.is_pinned(), "sample: host")
-    tiles = _sample_tiles(logits, n, v)
+    tiles = _scratch.floats(_sample_scratch_floats(n, v), logits.device)
     _run("sampling", "li_sample_call", logits.data_ptr(), records, counters.buffer_info()[0], out.data_ptr(), host.data_ptr(), n, v, tiles.data_ptr(),
          tiles.numel())
-
-
-def _sample_tiles(logits: torch.Tensor, n: int, v: int) -> torch.Tensor:
-    """What the first of the two kernels leaves for the second."""
-    key = (logits.device, n, v)
-    if key not in _sample_scratch:
-        _sample_scratch[key] = torch.empty(_sample_scratch_floats(n, v), dtype=torch.float32, device=logits.device)
-    return _sample_scratch[key]
 
 
 def _sample_rows(logits: torch.Tensor, n: int, temperature: int, top_k: int, top_p: int, uniform: int, out: torch.Tensor) -> None:
     if not n:
         return
     v = logits.shape[1]
-    tiles = _sample_tiles(logits, n, v)
+    tiles = _scratch.floats(_sample_scratch_floats(n, v), logits.device)
     _run("sampling", "li_sample_rows", logits.data_ptr(), temperature, top_k, top_p, uniform, out.data_ptr(), n, v,
          tiles.data_ptr(), tiles.numel())
 

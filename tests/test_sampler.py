@@ -101,3 +101,52 @@ def test_results_that_are_let_go_do_not_pile_up():
     for _ in range(26):
         smp._host_buffer(4)
     assert not sampler._unread
+
+
+def test_what_one_kernel_leaves_for_the_next_is_a_thread_s_and_a_stream_s_own(monkeypatch):
+    from litinfer_amd.kernels import ops
+    cpu, stream = torch.device("cpu"), [1]
+    monkeypatch.setattr(ops, "_stream", lambda: stream[0])
+    room = ops._Scratch()
+    a = room.floats(100, cpu)
+    assert room.floats(40, cpu) is a and room.floats(100, cpu) is a
+    stream[0] = 2
+    b = room.floats(100, cpu)
+    assert b.data_ptr() != a.data_ptr()
+    other = []
+    t = threading.Thread(target=lambda: other.append(room.floats(100, cpu)))
+    t.start()
+    t.join()
+    assert other[0].data_ptr() not in (a.data_ptr(), b.data_ptr())
+    stream[0] = 1
+    grown = room.floats(101, cpu)
+    assert grown.numel() >= 101 and room.floats(100, cpu) is grown and len(room.buffers) == 2
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: True)
+    own = room.floats(10, cpu)
+    assert own is not grown and room.floats(10, cpu) is not own                     # (a recording's replays outlive what is kept here)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    for stream[0] in range(3, 40):
+        room.floats(8, cpu)
+        assert len(room.buffers) <= room.STREAMS
+
+
+@pytest.mark.parametrize("name", ["argmax_rows", "sample_rows"])
+def test_the_kernels_are_given_room_for_their_rows(monkeypatch, name):
+    """The first kernel's part for the second, by the library's own count, whatever sizes came before."""
+    from litinfer_amd.kernels import ops
+    calls = []
+    monkeypatch.setattr(ops, "_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(ops, "_run", lambda module, fn, *args: calls.append(args))
+    for n, v in ((3, 9000), (64, 151936), (1, 17), (128, 33)):
+        x, out = torch.zeros(n, v), torch.zeros(n, dtype=torch.int32)
+        if name == "argmax_rows":
+            ops.argmax_rows(x, out)
+            at = calls[-1][2:4]
+            assert at[1] - at[0] == 4 * 32 * n and list(ops._scratch.buffers.values())[0].numel() >= 64 * n
+        else:
+            f = torch.zeros(n)
+            ops.sample_rows(x, f, f.int(), f, f, out)
+            assert calls[-1][-1] >= ops._sample_scratch_floats(n, v)
+            assert list(ops._scratch.buffers.values())[0].data_ptr() == calls[-1][-2]
+    ops._scratch.buffers.clear()
