@@ -774,7 +774,10 @@ __global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_til
         const bool plain = __all(off <= HI - LO);
         const float y = 1.0f / T;
         float sum[STEPS];
-        if (plain) {                                           // (where ids end within a thread's eight, one of these is -inf: not plain)
+        if (!(m > -INFINITY)) {                                // (a tile of -inf alone has no mass)
+#pragma unroll
+            for (int c = 0; c < STEPS; ++c) sum[c] = 0.f;
+        } else if (plain) {                                    // (where ids end within a thread's eight, one of these is -inf: not plain)
 #pragma unroll
             for (int c = 0; c < STEPS; ++c) {
                 float e_of[8];
@@ -786,17 +789,17 @@ __global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_til
                 if (j0 + c * TILE_STRETCH >= V) sum[c] = 0.f;
             }
         } else {
+            // (Masked logits come here.  64 rows of 151,936 ids, half of them -inf, at a temperature, both kernels: 22.6; as a loop that picks its value
+            // from the registers 25.9, every stretch read once more 24.7; one row 11.7 / 12.6.)
 #pragma unroll
             for (int c = 0; c < STEPS; ++c) {
                 const int j = j0 + c * TILE_STRETCH;
-                sum[c] = 0.f;
-#pragma unroll 1
-                for (int e = 0; e < 8; ++e) {
-                    float xe = x[c][0];
+                float z[8];
 #pragma unroll
-                    for (int q = 1; q < 8; ++q) xe = e == q ? x[c][q] : xe;
-                    sum[c] += (j + e < V && m > -INFINITY) ? expf(xe / T - m) : 0.f;       // (a tile of -inf alone has no mass)
-                }
+                for (int e = 0; e < 8; ++e) z[e] = expf(x[c][e] / T - m);
+                sum[c] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) sum[c] += j + e < V ? z[e] : 0.f;
             }
         }
         __syncthreads();                                       // (sf has been read)
@@ -882,14 +885,87 @@ __global__ __launch_bounds__(TILE_NT<STEPS>, STEPS == 1 ? 8 : 5) void sample_til
     for (int c = 0; c < STEPS; ++c)
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[c][e] /= T;
-    if (!all)
-        radix_kth<WAVES>([&](auto f) {
+    if (!all) {
+        // Of masked logits a tile may have fewer than kc above its lowest, which then is the kc-th; and where masked ids follow each other, the bound of
+        // tile_bound comes from those stretches in which every lane has a value above the lowest.  (Four bits a pass over 32 values a thread are
+        // the longest way: 64 rows of top-k with top-p, the first kernel, all but one id in a thousand masked 142 -> 63, the upper half masked 103 -> 67.)
+        uint32_t lowest = 0xffffffffu;
 #pragma unroll
-            for (int c = 0; c < STEPS; ++c)
+        for (int c = 0; c < STEPS; ++c)
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (j0 + c * TILE_STRETCH + e < V) f(x[c][e]);
-        }, kc, tau, need, work_i, tot_i);
+            for (int e = 0; e < 8; ++e)
+                if (j0 + c * TILE_STRETCH + e < V) lowest = min(lowest, sort_key(x[c][e]));
+#pragma unroll
+        for (int o = LI_WAVE / 2; o > 0; o >>= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, o, LI_WAVE));
+        if (lane == 0) work_i[w] = (int)lowest;
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < WAVES; ++i) lowest = min(lowest, (uint32_t)work_i[i]);
+#pragma unroll
+        for (int c = 0; c < STEPS; ++c) {
+            n[c] = 0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) n[c] += (j0 + c * TILE_STRETCH + e < V) && sort_key(x[c][e]) > lowest;
+        }
+        const int above = tile_places(n, place, si);
+        bool found = above < kc;
+        if (found) {
+            tau = lowest;
+            need = kc - above;
+        } else {
+            uint32_t key[STEPS];
+            int whole = 0;
+#pragma unroll
+            for (int c = 0; c < STEPS; ++c) {
+                key[c] = 0u;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) key[c] = max(key[c], sort_key(x[c][e]));
+                const bool takes = __all(j0 + c * TILE_STRETCH + 8 <= V && key[c] > lowest);
+                key[c] = takes ? key[c] : 0xffffffffu;
+                whole += takes;
+            }
+            if (lane == 0) work_i[w] = whole;
+            __syncthreads();
+            whole = 0;
+#pragma unroll
+            for (int i = 0; i < WAVES; ++i) whole += work_i[i];
+            const int rounds = whole ? (kc + whole - 1) / whole : LI_WAVE + 1;
+            if (rounds <= LI_WAVE) {
+                uint32_t bound = 0xffffffffu;
+#pragma unroll
+                for (int c = 0; c < STEPS; ++c) bound = min(bound, wave_bound<16>(key[c], rounds));
+                __syncthreads();                               // (work_i has been read)
+                if (lane == 0) work_i[w] = (int)bound;
+                __syncthreads();
+#pragma unroll
+                for (int i = 0; i < WAVES; ++i) bound = min(bound, (uint32_t)work_i[i]);
+#pragma unroll
+                for (int c = 0; c < STEPS; ++c) {
+                    n[c] = 0;
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) n[c] += (j0 + c * TILE_STRETCH + e < V) && sort_key(x[c][e]) >= bound;
+                }
+                const int total = tile_places(n, place, si);
+                found = total <= SMP_LIST;
+                if (found) {
+#pragma unroll
+                    for (int c = 0; c < STEPS; ++c)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e)
+                            if ((j0 + c * TILE_STRETCH + e < V) && sort_key(x[c][e]) >= bound) list[place[c]++] = sort_key(x[c][e]);
+                    kth_of_list<NT>(list, total, kc, tau, need, tot_i);
+                }
+            }
+        }
+        if (!found)
+            radix_kth<WAVES>([&](auto f) {
+#pragma unroll
+                for (int c = 0; c < STEPS; ++c)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (j0 + c * TILE_STRETCH + e < V) f(x[c][e]);
+            }, kc, tau, need, work_i, tot_i);
+    }
     int rank[STEPS];
 #pragma unroll
     for (int c = 0; c < STEPS; ++c) {

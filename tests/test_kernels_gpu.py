@@ -1565,6 +1565,37 @@ def test_sample_rows_takes_the_same_ids_where_the_tiles_are_many(ops, vocab):
                 assert _pick_is_right(row, temperature[r], top_k[r], top_p[r], u[r], picks[r], 1e-4), r
 
 
+@pytest.mark.parametrize("mask", ["half", "lowest", "behind", "few", "zeros", "tiny"])
+def test_masked_logits_where_the_tiles_are_many_and_few(ops, mask):
+    # ids that may not come (-inf, the lowest number), scattered, behind a place within a tile (its stretches without a mask give the
+    # bound), or all but a few (fewer than are wanted above a tile's lowest); zeros and values too small for the reciprocal; top-p alone too
+    g = torch.Generator().manual_seed(72)
+    vocab, n = 6 * 8192 + 2049, 112                                     # 784 tiles of seven a row; six rows are 42
+    logits = torch.randn(n, vocab, generator=g) * 3
+    hit = torch.rand(n, vocab, generator=g)
+    if mask == "behind":
+        logits[:, 3 * 8192 + 2100:] = float("-inf")
+        logits[1::2, :8192 + 4090] = float("-inf")
+    elif mask in ("zeros", "tiny"):
+        logits[hit < 0.02] = 0.0 if mask == "zeros" else 1e-20
+    else:
+        logits[hit < (0.9995 if mask == "few" else 0.5)] = torch.finfo(torch.float32).min if mask == "lowest" else float("-inf")
+    temperature = [(0.7, 1.3, 0.0, 0.9, 2.0)[i % 5] for i in range(n)]
+    top_k = [(0, 50, 200, 0, 3, 0, 256)[i % 7] for i in range(n)]
+    top_p = [(1.0, 0.9, 0.5, 0.7, 1.0, 1.0, 0.95)[i % 7] for i in range(n)]
+    u = torch.rand(n, generator=g).tolist()
+    many = _sample(ops, logits, temperature, top_k, top_p, u)
+    few = sum((_sample(ops, logits[r:r + 6], temperature[r:r + 6], top_k[r:r + 6], top_p[r:r + 6], u[r:r + 6]) for r in range(0, 42, 6)), [])
+    assert many[:42] == few
+    for r in range(42):
+        row = logits[r].double().numpy()
+        assert row[many[r]] > -1e30, r
+        if temperature[r] == 0.0:
+            assert many[r] == plain_impl.argmax_first(row), r
+        else:
+            assert _pick_is_right(row, temperature[r], top_k[r], top_p[r], u[r], many[r], 1e-4), r
+
+
 @pytest.mark.parametrize("n", [1, 16, 17, 64, 65, 128, 129])
 def test_options_in_the_arguments_choose_what_options_in_arrays_choose(ops, n):
     # sample_async hands options that are packed to the launch itself, up to 128 rows; objects that hold the same numbers unpacked go
