@@ -303,8 +303,13 @@ __global__ __launch_bounds__(256) void paged_attention_decode_kernel(
 // the weights, 54 splits of 8 x 28 heads took 6.7 us, 20 of 64 x 12 5.0; now 3.6 and 3.8.
 #define MERGE_MAX_SPLITS 64
 #define MERGE_SHARE 16
+#define MERGE_BLOCKS 1024       // (token, head)s of a listed batch up to which four groups a block are the faster
 
-template <typename T, int GROUPS>
+// LISTED: one group, and what a token has beyond its first sixteen runs sixteen at a time behind them, for batches of many tokens whose contexts
+// differ.  Most have few of the 64 runs that the grid is cut into, and of blocks of eight waves the chip takes 1,024 at a time: us a layer with
+// four groups, which ask for 64 runs whatever there are, and so: 12 heads on 2, one of 4,608 keys beside 299 of 200 43.7 / 31.6, 64 of 2,001 and
+// less 14.1 / 14.9; 28 on 4, one of 1,500 beside 39 of 187 16.9 / 13.4.
+template <typename T, int GROUPS, bool LISTED = false>
 __global__ __launch_bounds__(128 * GROUPS) void attention_merge_kernel(
     const float* __restrict__ part_acc, const float* __restrict__ part_ml,
     const int* __restrict__ token_list, T* __restrict__ out, int nh, int dh, int nsplit_all,
@@ -340,6 +345,17 @@ __global__ __launch_bounds__(128 * GROUPS) void attention_merge_kernel(
             const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), first + i));
             at += first + i < nsplit ? pa[i] * wi : 0.f;
         }
+        if constexpr (LISTED) {
+            for (int from = MERGE_SHARE; from < nsplit; from += MERGE_SHARE) {
+#pragma unroll
+                for (int i = 0; i < MERGE_SHARE; ++i) pa[i] = part_acc[(base + (from + i < nsplit ? from + i : 0)) * dh + d];
+#pragma unroll
+                for (int i = 0; i < MERGE_SHARE; ++i) {
+                    const float wi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(w), from + i));
+                    at += from + i < nsplit ? pa[i] * wi : 0.f;
+                }
+            }
+        }
         if constexpr (GROUPS > 1) {
             if (d0) __syncthreads();
             if (group) sums[group - 1][col] = at;
@@ -356,6 +372,7 @@ static void launch_merge(const float* part_acc, const float* part_ml, const int*
                          hipStream_t stream) {
     const dim3 grid(n_tokens, nh);
     if (nsplit <= MERGE_SHARE) attention_merge_kernel<T, 1><<<grid, 128, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
+    else if (nruns && (long)n_tokens * nh > MERGE_BLOCKS) attention_merge_kernel<T, 1, true><<<grid, 128, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
     else if (nsplit <= 2 * MERGE_SHARE) attention_merge_kernel<T, 2><<<grid, 256, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
     else attention_merge_kernel<T, 4><<<grid, 512, 0, stream>>>(part_acc, part_ml, token_list, out, nh, dh, nsplit, nruns);
 }

@@ -955,6 +955,18 @@ def test_any_number_of_runs_is_joined(ops, monkeypatch, runs, dtype):
     assert rel(out, ref) < tol(dtype, 1e-5, 8e-3)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("requests,runs", [(171, 64), (172, 17), (172, 33), (560, 64)])
+def test_runs_of_many_tokens_with_a_long_one_among_them_are_joined(ops, monkeypatch, requests, runs, dtype):
+    # 171 x 6 (token, head)s and more: one group of the joining kernel's threads takes a token's runs sixteen at a time; 560 x 64
+    # items of the list are more than one slice of the decode kernel's grid
+    monkeypatch.setattr(ops, "_decode_cut", lambda *a: (runs, 1, 1))
+    segs = [(1 + (7 * i) % 45, 1) for i in range(requests)]
+    segs[requests // 2], segs[3] = (32 * runs - 5, 1), (16 * 32, 1)
+    out, ref = _paged_case(ops, dtype, segs, 6, 2, 64, 16, 0, seed=64, ws=_Lender())
+    assert rel(out, ref) < tol(dtype, 1e-5, 8e-3)
+
+
 @pytest.mark.parametrize("dh,ctx", [(256, 16 * 256), (256, 17 * 256), (128 + 64, 33 * 256), (16, 20 * 256)])
 def test_runs_of_the_vector_kernel_are_joined(ops, dh, ctx):
     for dtype in DTYPES:
