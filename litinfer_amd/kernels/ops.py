@@ -1643,6 +1643,17 @@ def decode_run_keys(meta, token_list: Optional[torch.Tensor], n_tokens: int, pag
          meta.max_blocks, page_size, int(window), nkv, nsplit, simds, int(group), out.data_ptr())
 
 
+def _decode_plan(meta, pairs: int, keys: int, dh: int, dtype: torch.dtype, page_size: int, window: int, simds: int):
+    """`_decode_cut`, or a finer one where a run's pages would not fit the kernel's copy of the block table.  The same for all layers of a step (in
+    its first pass, which is not replayed, 10 us of the host's time a layer)."""
+    nsplit, quad, planned = _decode_cut(pairs, keys, dh, dtype, simds, window <= 0 and page_size % 8 == 0, meta, window)
+    while nsplit <= DECODE_MAX_SPLITS and decode_split_blocks(meta.max_blocks, page_size, window, nsplit) > DECODE_TABLE_CAP:
+        nsplit, quad = nsplit + 1, 1
+    _chk(nsplit <= DECODE_MAX_SPLITS, f"attention: block tables of {meta.max_blocks} pages of {page_size} "
+                                      f"are too long for the decode kernel")
+    return nsplit, quad, planned
+
+
 def decode_split_blocks(max_blocks: int, page_size: int, window: int, nsplit: int) -> int:
     """The most pages one of `nsplit` splits of the keys can touch, for block tables of
     `max_blocks` pages: the keys (at most the table's, or the window's) are cut into runs
@@ -1701,13 +1712,11 @@ def paged_attention(qkv: torch.Tensor, out: torch.Tensor, k: torch.Tensor, v: to
             _chk(meta.max_blocks * page_size <= 1 << 21 and page_size <= 1 << 16,
                  f"attention: block tables of {meta.max_blocks} pages of {page_size} keys are beyond the decode "
                  f"kernel's {1 << 21} keys")
-            nsplit, quad, planned = _decode_cut(n_single * nkv, keys, dh, qkv.dtype, _simd_count(qkv.device), window <= 0 and page_size % 8 == 0,
-                                                meta, window)
-            # a split's pages must fit the kernel's copy of the block table
-            while nsplit <= DECODE_MAX_SPLITS and decode_split_blocks(meta.max_blocks, page_size, window, nsplit) > DECODE_TABLE_CAP:
-                nsplit, quad = nsplit + 1, 1
-            _chk(nsplit <= DECODE_MAX_SPLITS, f"attention: block tables of {meta.max_blocks} pages of {page_size} "
-                                              f"are too long for the decode kernel")
+            key = ("decode_cut", n_single, nkv, dh, qkv.dtype, page_size, int(window))
+            plan = meta.extra.get(key)
+            if plan is None:
+                plan = meta.extra[key] = _decode_plan(meta, n_single * nkv, keys, dh, qkv.dtype, page_size, int(window), _simd_count(qkv.device))
+            nsplit, quad, planned = plan
         else:
             nsplit = max(1, min(-(-512 // (n_single * nkv)), -(-keys // 256), DECODE_MAX_SPLITS))
         acc = ml = None

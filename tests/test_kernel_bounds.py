@@ -89,6 +89,39 @@ def test_prompt_attention_is_planned_once_a_step(monkeypatch):
     assert len(asked) == 9
 
 
+def test_decoding_is_planned_once_a_step(monkeypatch):
+    """A step's layers share the cut of their keys; another window, layout or step asks again."""
+    import torch
+    from litinfer_amd.engine.batch import AttentionMeta
+    asked, sent = [], []
+    cut = ops._decode_cut
+    monkeypatch.setattr(ops, "_decode_cut", lambda *a: (asked.append(a), cut(*a))[1])
+    monkeypatch.setattr(ops, "_gpu", lambda *a: None)
+    monkeypatch.setattr(ops, "_simd_count", lambda device: 1024)
+    monkeypatch.setattr(ops, "_run", lambda *a: sent.append(a))
+    n, page, width = 3, 16, 64
+    ints = lambda *v: torch.tensor(v, dtype=torch.int32)
+
+    def step(longest):
+        ctx = np.array([200, longest, 5], np.int32)
+        return AttentionMeta(block_table=torch.zeros(n, width, dtype=torch.int32), max_blocks=width, seg_of_token=ints(0, 1, 2), q_start=ints(0, 1, 2),
+                             q_len=ints(1, 1, 1), ctx_len=torch.from_numpy(ctx), num_segments=n, num_tokens=n, max_q_len=1, max_ctx_len=longest,
+                             host_q_start=np.arange(n, dtype=np.int32), host_q_len=np.ones(n, np.int32), host_ctx_len=ctx, num_single=n, max_single_ctx=width * page)
+
+    def call(meta, nh, nkv, window):
+        cache = torch.zeros(8, nkv, page, 64, dtype=torch.bfloat16)
+        q = torch.zeros(n, nh * 64, dtype=torch.bfloat16)
+        ops.paged_attention(q, torch.empty_like(q), cache, cache.clone(), meta, nh, nkv, 64, page, window, 0.1)
+    first = step(1000)
+    for _ in range(28):
+        call(first, 14, 2, 0)
+    assert len(asked) == 1 and len({s[-2] for s in sent if s[1] == "li_paged_attention_decode"}) == 1
+    call(first, 14, 2, 100)
+    call(first, 8, 4, 0)
+    call(step(900), 14, 2, 0)
+    assert len(asked) == 4
+
+
 def _segments(segs):
     return np.array([q for _, q in segs], dtype=np.int32), np.array([c for c, _ in segs], dtype=np.int32)      # (context, new tokens)
 
