@@ -1499,50 +1499,83 @@ def _seg_of_token(meta, takes: bool = True) -> int:
     return 0 if in_order else meta.seg_of_token.data_ptr()
 
 
-def _one_block(pairs: int, keys: int, dh: int, simds: int) -> bool:
+def _single_keys(meta, window: int):
+    """(mean, longest) keys that the step's single tokens see, as far as the host knows them; None where it does not, or there is one."""
+    ql, cl = getattr(meta, "host_q_len", None), getattr(meta, "host_ctx_len", None)
+    if ql is None or cl is None:
+        return None
+    keys = cl[ql == 1]
+    if keys.size < 2:
+        return None
+    if window > 0:
+        keys = np.minimum(keys, window)
+    return max(float(keys.mean()), 1.0), float(keys.max())
+
+
+def _one_block(pairs: int, keys: int, dh: int, simds: int, spread=None, padded: bool = False) -> bool:
     """Whether a block of DECODE_QUAD waves takes all of a (token, kv head)'s keys and joins its runs itself, rather than runs of single waves and the
-    kernel that joins them (bfloat16, up to 512 pairs, the kernel's quicker form).  Four waves sit on one compute unit, so it pays where the
-    pairs fill the chip with a block each, or nearly, and where the keys are too few for the second kernel.  Us a call, one block against
-    single runs, contexts all as long as the table, three quarters of it, spread from an eighth of it on.  12 heads on 2 of 128, 64 pairs: tables of 256 keys 8.8 / 8.1, 7.8 / 7.8,
-    8.1 / 8.1, 512 11.7 / 9.8, 9.8 / 9.3, 11.2 / 9.8; 128 pairs: 384 10.4 / 11.5, 9.2 / 10.4, 9.8 / 10.5, 512 13.9 / 12.7, 10.4 / 11.0, 11.6 / 11.8, 768 18.1 / 15.7, 13.2 / 13.4,
-    14.7 / 13.5; 160: 1,024 21.9 / 24.2, 17.2 / 18.5, 18.2 / 18.2, 2,048 37.6 / 38.7, 29.9 / 30.9, 32.2 / 29.0; 200: 2,048 42.7 / 46.1, 33.5 / 37.2, 34.3 / 35.0; 256: 52.8 /
-    56.5, 41.5 / 45.3, 37.9 / 41.0; 320: 512 24.0 / 23.5, 18.8 / 19.2, 18.4 / 19.4, 1,024 41.6 / 39.7, 33.1 / 31.6, 31.1 / 30.2; 512: 1,024 54.3 / 58.1, 41.9 / 46.3, 39.5 / 46.1.  Heads
-    of 64, 14 on 2, 2 pairs: 256 5.4 / 5.3, 4.8 / 5.3, 384 6.1 / 5.4, 5.8 / 5.4; 8: 384 6.3 / 6.1, 5.9 / 5.9, 6.1 / 6.1, 512 7.3 / 6.7; 64: 512 8.6 / 8.5, 7.2 / 8.1, 7.9 / 8.3, 768
-    10.4 / 9.2, 9.2 / 8.9, 10.1 / 9.2; 96: 768 10.7 / 11.1, 9.3 / 9.9, 10.2 / 9.8, 1,024 12.6 / 11.8; 160: 1,024 13.7 / 15.7, 11.4 / 13.2, 12.4 / 12.7, 1,536 20.2 / 19.3, 14.9 /
-    16.2, 16.7 / 15.5; 200 and more 5 to 30 % faster in one block up to 2,048 keys; 320: 1,024 23.9 / 24.4, 18.4 / 19.9, 17.9 / 19.3, 2,048 41.5 / 40.3."""
+    kernel that joins them (bfloat16, up to 512 pairs, the kernel's quicker form).  `spread`: `_single_keys`; padded: the step may be recorded,
+    and replayed for other contexts of the same tables.
+    Few keys: it saves the second kernel.  A whole step of 28 layers, 12 heads on 2 of 128, runs / one block, contexts of 0.58 and of 0.5 to 1 of the table: 48
+    pairs, 512 keys 1,677 and 1,686 / 1,681 and 1,746, 80 pairs 1,735 and 1,746 / 1,712 and 1,760, 128 pairs, 1,024 keys 2,161 and 2,126 / 2,133 and 2,133; 24 layers, 14 on 2 of 64: 16
+    pairs, 512 keys 797 and 798 / 801 and 833, 48 pairs 997 and 1,004 / 977 and 1,002, 80 pairs, 1,024 keys 1,227 and 1,230 / 1,263 and 1,258, 128 pairs 1,402 and 1,393 / 1,378 and 1,377.
+    Many keys: it pays where the pairs fill the chip with a block each, or nearly, and where no context is much longer than the others: its four waves take
+    the longest alone, while runs are shared out among all SIMDs.  By the keys that the busiest SIMD works on: a quarter of the longest context (of the mean one
+    in the rounds of blocks before the last) against 1.2 times its share of all keys and 200 for the second kernel, fitted to 115 batches, of which it chooses
+    0.4 % above the faster form on average and 8 % at most.  Us a call, runs / one block, 28 heads on 4, 64 requests: 1,024 to 2,048 keys evenly 51 / 44, 256 to
+    2,048 41 / 38, 16 to 4,600 69 / 74, eight of 1,000 to 2,048 beside 56 of 128 19 / 28, eight of 15,000 to 30,000 beside 56 of 1,875 124 / 331; 48 requests, 16 to 4,600
+    56 / 64; 12 on 2, 120 requests of 16 to 4,600 65 / 71, 200 102 / 124, 256 of 16 to 2,048 66 / 65; 14 on 2 of 64, 100 requests of 16 to 4,600 32 / 41, 256 77 / 74.
+    Contexts that differ in tables of more than 2,048 keys that a recording brings take runs whatever they are now: the replays' may be those of
+    one long document."""
     if keys <= 128:
         return False
     room = simds // DECODE_QUAD                     # blocks that the chip takes at one time
-    if 4 * pairs >= 3 * room * -(-pairs // room):
+    rounds = -(-pairs // room)
+    fills = 4 * pairs >= 3 * room * rounds
+    if keys <= 1280:
+        if pairs > room and not fills:
+            return keys <= (640 if dh == 128 else 1024)
+        if dh == 64:
+            return keys <= max(256 + 7 * pairs, 10 * pairs)
+        return pairs > 48 and keys <= 10 * pairs
+    if not fills:
+        return False
+    if spread is None:
         return True
-    if pairs > room:
-        return keys <= (640 if dh == 128 else 1024)
-    if dh == 128:
-        return keys <= max(4 * pairs, 16 * (pairs - 96))
-    return keys <= (min(512, 256 + 16 * pairs) if pairs <= 64 else 256 + 5 * pairs)
+    mean, longest = spread
+    if longest < 1.15 * mean:
+        return True
+    if padded and keys > 2048:
+        return False
+    return ((rounds - 1) * mean + longest) / DECODE_QUAD <= 1.2 * pairs * mean / simds + 200
 
 
 def _decode_cut(pairs: int, keys: int, dh: int, dtype: torch.dtype, simds: int, aligned: bool, meta, window: int):
     """(runs that each token's keys are cut into, waves a block, runs if all contexts were as long as the longest) for the matrix-core decode kernel.
     One block a (token, kv head) by `_one_block`, or by `_short_runs` where that was measured instead; else single waves, their runs of 128 keys at
-    least, or of 32 (64 where contexts differ) and to a finer cut where the pairs are few: the kernel that joins runs asks for all of
-    them at once, so that a run costs it little.  Us a call, runs of 128 and the coarser cut / so: 2 pairs, 12 heads on 2 of 128, tables of 512, 1,024 and 4,096 keys
-    8.2 / 6.7, 8.5 / 6.8, 9.5 / 8.4; 8 pairs 8.5 / 7.0, 8.8 / 7.0, 10.7 / 10.5; 32 pairs 9.7 / 8.3, 10.1 / 9.5, at 2,048 12.5 / 13.2 (so not there); heads of 64, 32
-    pairs, 2,048 10.3 / 9.9; float32, 2 pairs 15.6 / 10.5, 15.5 / 8.4, 18.0 / 12.6; 32 pairs 17.4 / 12.4, 18.6 / 13.6, heads of 64 at 2,048 14.3 / 13.8."""
+    least, or of 32 and to a finer cut where the pairs are few: the kernel that joins runs asks for all of them at once, so that a run costs it
+    little.  Where all runs are at work at one time anyway, no run is longer than 128 keys and no context much longer than the others, every token's keys are cut
+    into the same number of runs: one run length for the batch, and the list of the runs that have keys, would cost a kernel of its own and a trip in every
+    layer.  A step of 28 layers, 12 heads on 2 of 128, the list / none: 4 requests of 260 to 500 keys 1,208 / 1,178, 16 of 90 to 181 1,397 / 1,373, 64 of 600 to 1,000
+    2,159 / 2,126; a call of 28 heads on 4, 8 requests of 512 to 4,096 keys 18.5 / 16.4, one of 4,096 beside 7 of 200 11.1 / 14.9 (so not there)."""
     bf16 = dtype is torch.bfloat16
-    differ = _ragged_splits(1, meta, window, 1) > 1
+    spread = _single_keys(meta, window)
+    differ = spread is not None and spread[1] >= 1.15 * spread[0]
     planned = decode_splits(pairs, keys, simds)
     measured = bf16 and aligned and pairs <= 512
     few = pairs * keys <= (65536 if dh == 64 else 32768) and keys > (128 if bf16 else 96)
     if measured:
-        runs = DECODE_QUAD if _one_block(pairs, keys, dh, simds) else (32, 64) if few else (128,)
+        runs = DECODE_QUAD if _one_block(pairs, keys, dh, simds, spread, getattr(meta, "padded", False)) else (32, 32) if few else (128,)
     else:
         runs = _short_runs(pairs, keys, dh, dtype, DECODE_QUAD if planned == DECODE_QUAD and not differ else 0, aligned, differ)
         if runs is None:
             runs = DECODE_QUAD if planned == DECODE_QUAD and not differ else (32, 64) if few and pairs <= 32 and not bf16 else (128,)
     if runs == DECODE_QUAD:
         return DECODE_QUAD, DECODE_QUAD, DECODE_QUAD
-    planned = decode_splits(pairs, keys, simds, 1, runs[-1] if differ else runs[0], 1 if few and pairs <= 32 else 4)
+    join = 4 if not few or pairs > 32 else 1 if pairs <= 8 or not bf16 else 3
+    planned = decode_splits(pairs, keys, simds, 1, runs[-1] if differ else runs[0], join)
+    if measured and differ and spread[1] <= 2.5 * spread[0] and pairs * planned <= simds and -(-keys // planned) <= 128:
+        return planned, 1, planned
     return _ragged_splits(planned, meta, window, 1), 1, planned
 
 

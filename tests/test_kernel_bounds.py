@@ -219,12 +219,66 @@ def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh,
         assert ops._short_runs(pairs, keys, dh, ops.torch.float32, 4) == want, keys
 
 
-@pytest.mark.parametrize("pairs,dh,ends", [(1, 64, 272), (8, 64, 384), (64, 64, 512), (65, 64, 581), (160, 64, 1056), (191, 64, 1211), (192, 64, None), (256, 64, None),
-                                           (257, 64, 1024), (383, 64, 1024), (384, 64, None), (512, 64, None), (32, 128, 0), (64, 128, 256), (128, 128, 512),
-                                           (160, 128, 1024), (192, 128, None), (320, 128, 640)])
+def _decode_batch(ctx, padded=False):
+    from types import SimpleNamespace
+    ctx = np.asarray(ctx, np.int32)
+    return SimpleNamespace(host_q_len=np.ones(len(ctx), np.int32), host_ctx_len=ctx, padded=padded)
+
+
+def _decode_plan_of(ctx, nkv, dh=128, table=0, padded=False):
+    """What `_decode_cut` says, and the keys of the longest wave: with a list, at the run length that the device chooses."""
+    keys = max(table, max(ctx))
+    ns, waves, planned = ops._decode_cut(len(ctx) * nkv, keys, dh, ops.torch.bfloat16, 1024, True, _decode_batch(ctx, padded), 0)
+    up = lambda a, b: (-(-a // b) + 31) & ~31
+    longest = max(ctx)
+    if ns <= planned:
+        return (ns, waves), up(longest, ns)
+    keys_of, lower, cap = np.asarray(ctx), up(longest, ns), up(keys, ns)
+    cost = {c: -(-int(nkv * np.sum(-(-keys_of // c))) // 1024) * (c + 24) for c in range(lower, max(cap, lower) + 1, 32)}
+    return (ns, waves), min(cost, key=lambda c: (cost[c], c))
+
+
+@pytest.mark.parametrize("pairs,dh,ends", [(1, 64, 263), (8, 64, 312), (36, 64, 508), (37, 64, 515), (65, 64, 711), (85, 64, 851), (86, 64, 860), (128, 64, 1280), (191, 64, 1280),
+                                           (192, 64, None), (256, 64, None), (257, 64, 1024), (383, 64, 1024), (384, 64, None), (512, 64, None), (32, 128, 0), (48, 128, 0),
+                                           (49, 128, 490), (64, 128, 640), (128, 128, 1280), (160, 128, 1280), (192, 128, None), (320, 128, 640)])
 def test_a_block_takes_all_runs_only_where_that_was_measured(pairs, dh, ends):
+    """Of contexts that are alike, or that the host does not know."""
     for keys in range(1, 20000, 7):
-        assert ops._one_block(pairs, keys, dh, 1024) == (keys > 128 and (ends is None or keys <= ends)), keys
+        for spread in (None, (float(keys), float(keys)), (keys / 1.14, float(keys))):
+            assert ops._one_block(pairs, keys, dh, 1024, spread) == (keys > 128 and (ends is None or keys <= ends)), keys
+
+
+@pytest.mark.parametrize("ctx,nkv,dh,most", [
+    ([30000] + [200] * 63, 4, 128, 480), ([8000] + [300] * 63, 4, 128, 128), ([16000] + [500] * 47, 4, 128, 256), ([30000] + [200] * 119, 2, 128, 480),
+    (np.linspace(16, 4600, 64).astype(int), 4, 128, 672), (np.linspace(16, 4600, 128).astype(int), 2, 64, 672), ([30000] + [200] * 99, 2, 128, 480),
+    ([20000] * 4 + [100] * 252, 2, 128, 480)])
+@pytest.mark.parametrize("padded", [False, True])
+def test_a_long_context_beside_short_ones_is_shared_out_among_the_waves(ctx, nkv, dh, most, padded):
+    """One long document beside many short requests: no block of four waves takes it alone, whether the step is recorded or not."""
+    ctx = [int(c) for c in ctx]
+    table = 1 << (max(ctx) - 1).bit_length() if padded else 0
+    (ns, waves), longest = _decode_plan_of(ctx, nkv, dh, table, padded)
+    assert waves == 1 and longest <= most, (ns, waves, longest)
+
+
+@pytest.mark.parametrize("n,nkv,table", [(64, 4, 4096), (48, 4, 16384), (120, 2, 8192), (256, 2, 4096), (128, 2, 32768)])
+def test_a_recording_of_contexts_that_differ_does_not_take_blocks_of_four(n, nkv, table):
+    """Its replays' contexts may be others of the same tables, as spread as they like; of contexts that are alike it does."""
+    for low in (1.5, 2, 8, 100):
+        assert _decode_plan_of([int(c) for c in np.linspace(table * 0.9 / low, table * 0.9, n)], nkv, 128, table, True)[0][1] == 1, low
+    assert _decode_plan_of([int(table * 0.9)] * n, nkv, 128, table, True)[0] == (4, 4)
+
+
+@pytest.mark.parametrize("ctx,nkv,table,listed", [(np.linspace(260, 500, 4), 2, 512, False), (np.linspace(600, 1000, 48), 2, 1024, False), ([512] + [100] * 3, 2, 512, True),
+                                                  (np.linspace(2047, 4090, 8), 4, 4096, False), (np.linspace(100, 2001, 64), 2, 2048, True),
+                                                  (np.linspace(500, 1900, 80), 2, 2048, True)])
+def test_runs_are_listed_only_where_they_can_be_shared_out(ctx, nkv, table, listed):
+    """Not where all of them are at work at one time, short and of contexts that are not far apart."""
+    ctx = [int(c) for c in ctx]
+    ns, waves, planned = ops._decode_cut(len(ctx) * nkv, table, 128, ops.torch.bfloat16, 1024, True, _decode_batch(ctx, True), 0)
+    assert waves == 1 and (ns > planned) == listed
+    if not listed:
+        assert len(ctx) * nkv * ns <= 1024 and -(-table // ns) <= 128
 
 
 def test_every_decoding_step_is_cut_into_runs_that_the_kernels_take():
@@ -242,11 +296,11 @@ def test_every_decoding_step_is_cut_into_runs_that_the_kernels_take():
                             assert 1 <= planned <= ns <= ops.DECODE_MAX_SPLITS and (waves == 1 or ns == planned == waves == ops.DECODE_QUAD)
 
 
-@pytest.mark.parametrize("pairs,dh,aligned,ends", [(2, 128, True, 384), (32, 128, False, 384), (2, 64, True, 448), (64, 128, True, 640), (512, 64, True, 1280),
-                                                   (512, 128, False, 896)])
-def test_bfloat16_decoding_takes_one_block_only_where_that_was_measured(pairs, dh, aligned, ends):
+@pytest.mark.parametrize("pairs,dh,ends", [(2, 128, 384), (32, 128, 384), (2, 64, 448), (64, 128, 640), (512, 64, 896), (512, 128, 896)])
+def test_bfloat16_decoding_over_other_pages_takes_one_block_only_where_that_was_measured(pairs, dh, ends):
+    """A window, or pages of no multiple of 8 keys (else `_one_block` is asked)."""
     for keys in range(16, 8192, 16):
-        assert (ops._short_runs(pairs, keys, dh, ops.torch.bfloat16, 0, aligned) == ops.DECODE_QUAD) == (128 < keys <= ends), keys
+        assert (ops._short_runs(pairs, keys, dh, ops.torch.bfloat16, 0, False) == ops.DECODE_QUAD) == (128 < keys <= ends), keys
 
 
 @pytest.mark.parametrize("pairs,dh,differ,begins,ends", [(512, 64, False, 128, 1280), (513, 64, True, 128, 1280), (513, 64, False, 320, 1280), (640, 128, False, 320, 1280),
