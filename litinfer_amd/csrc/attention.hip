@@ -495,14 +495,11 @@ extern "C" long li_decode_split_blocks(int max_blocks, int page_size, int window
 // then the items, token | run << 16, a token's runs in a row: the decode kernel starts a block for every
 // item the grid could hold (tokens x nsplit) and those beyond [1] end at once, without a look at their
 // token.  At most RUN_KEYS_MAX_TOKENS tokens (the host checks).
-// `group` > 1: the decode kernel's blocks take `group` runs of a token that follow each other, one a wave
-// (a block with fewer runs still holds `group` SIMDs): the items are then the FIRST runs of such groups
-// (run 0, group, 2 group, ...), [1] counts them, and a candidate length costs its groups x `group` waves.
 #define RUN_KEYS_MAX_TOKENS 4096
 __global__ __launch_bounds__(256) void decode_run_keys_kernel(
     const int* __restrict__ token_list, int n_tokens, const int* __restrict__ seg_of_token,
     const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len,
-    int cap_keys, int window, int nkv, int nsplit, int simds, int group, int* __restrict__ out) {
+    int cap_keys, int window, int nkv, int nsplit, int simds, int* __restrict__ out) {
     __shared__ int nkeys[RUN_KEYS_MAX_TOKENS];
     __shared__ int red_i[4];
     __shared__ unsigned long long red_c[4];
@@ -535,7 +532,7 @@ __global__ __launch_bounds__(256) void decode_run_keys_kernel(
     const int c = lower + 32 * stride * tid;
     if (c <= cap) {
         long waves = 0;
-        for (int i = 0; i < n_tokens; ++i) waves += ((nkeys[i] + c - 1) / c + group - 1) / group * group;
+        for (int i = 0; i < n_tokens; ++i) waves += (nkeys[i] + c - 1) / c;
         waves *= nkv;
         const long rounds = (waves + simds - 1) / simds;
         best = ((unsigned long long)(rounds * (c + 24)) << 32) | (unsigned)c;
@@ -557,7 +554,7 @@ __global__ __launch_bounds__(256) void decode_run_keys_kernel(
     const int each = (n_tokens + 255) / 256;
     const int i0 = tid * each, i1 = i0 + each < n_tokens ? i0 + each : n_tokens;
     int mine = 0;
-    for (int i = i0; i < i1; ++i) mine += ((nkeys[i] + per - 1) / per + group - 1) / group;
+    for (int i = i0; i < i1; ++i) mine += (nkeys[i] + per - 1) / per;
     first[tid] = mine;
     __syncthreads();
     if (tid == 0) {
@@ -573,23 +570,22 @@ __global__ __launch_bounds__(256) void decode_run_keys_kernel(
     for (int i = i0; i < i1; ++i) {
         const int n = (nkeys[i] + per - 1) / per;
         nruns[i] = n;
-        const int ng = (n + group - 1) / group;
-        for (int r = 0; r < ng; ++r) items[at + r] = i | ((r * group) << 16);
-        at += ng;
+        for (int r = 0; r < n; ++r) items[at + r] = i | (r << 16);
+        at += n;
     }
 }
 
 extern "C" int li_decode_run_keys(const int* token_list, int n_tokens, const int* seg_of_token, const int* q_start,
                                   const int* q_len, const int* ctx_len, int max_blocks, int page_size, int window,
-                                  int nkv, int nsplit, int simds, int group, int* out, hipStream_t stream) {
+                                  int nkv, int nsplit, int simds, int* out, hipStream_t stream) {
     if (n_tokens <= 0 || n_tokens > RUN_KEYS_MAX_TOKENS || max_blocks <= 0 || page_size <= 0 || nkv <= 0 ||
-        nsplit <= 0 || nsplit > 0x7fff || simds <= 0 || group <= 0 || !out)
+        nsplit <= 0 || nsplit > 0x7fff || simds <= 0 || !out)
         return LI_ERR_SIZE;
     long keys = (long)max_blocks * page_size;
     if (window > 0 && window < keys) keys = window;
     if (keys > 0x7fffffffL - 64) return LI_ERR_SIZE;
     decode_run_keys_kernel<<<1, 256, 0, stream>>>(token_list, n_tokens, seg_of_token, q_start, q_len, ctx_len,
-                                                  (int)keys, window, nkv, nsplit, simds, group, out);
+                                                  (int)keys, window, nkv, nsplit, simds, out);
     return li_launch_status();
 }
 
@@ -2574,7 +2570,6 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
 // length and the list of the runs that have keys.
 // use_mfma: 0 the vector kernel; 1 the matrix-core kernel with nsplit 1 or LI_DECODE_QUAD, whose blocks write the output; 2 its single waves,
 // whose nsplit runs the merge kernel joins, as it does the vector kernel's.
-extern "C" int li_decode_quad(void) { return LI_DECODE_QUAD; }
 extern "C" int li_paged_attention_decode(const void* q, int q_row_stride, void* out, const void* kc,
                                          const void* vc, int dtype, const int* block_table, int max_blocks,
                                          const int* token_list, int n_tokens, const int* seg_of_token,
@@ -2585,7 +2580,7 @@ extern "C" int li_paged_attention_decode(const void* q, int q_row_stride, void* 
     if (n_tokens <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || dh <= 0 || dh > ATT_MAX_DH || page_size <= 0 ||
         max_blocks <= 0)
         return LI_ERR_SIZE;
-    if (nsplit < 1 || nsplit > MERGE_MAX_SPLITS) return LI_ERR_SIZE;      // the merge kernel keeps a weight per split in LDS
+    if (nsplit < 1 || nsplit > MERGE_MAX_SPLITS) return LI_ERR_SIZE;      // a wave of the merge kernel has a lane for each split, its groups sixteen each
     if (dtype == LI_F32 && !use_mfma)
         return launch_decode<float>((const float*)q, q_row_stride, (float*)out, (const float*)kc, (const float*)vc,
                                     block_table, max_blocks, token_list, n_tokens, seg_of_token, q_start, q_len,

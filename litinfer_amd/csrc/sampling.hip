@@ -1674,7 +1674,6 @@ static int sample_call(const float* logits, const SampleRecord* rec, const unsig
     }
     return launch_sample(logits, v, out, host, n, V, tiles, tiles_floats, stream);
 }
-extern "C" int li_sample_call_rows(void) { return SAMPLE_CALL_ROWS; }
 extern "C" int li_sample_call(const float* logits, const void* records, const unsigned long long* counters, int* out, int* host, int n, int V,
                               float* tiles, long tiles_floats, hipStream_t stream) {
     if (n <= 0 || n > SAMPLE_CALL_ROWS || !records || !counters || !out) return LI_ERR_SIZE;

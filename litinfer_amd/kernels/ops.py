@@ -106,7 +106,7 @@ _SIGNATURES = {
         "li_paged_attention_prefill": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I, P, P, P, I, I, I],
         "li_paged_attention_prefill_f32": [P, I, P, P, P, P, I, P, I, P, P, P, I, I, I, I, I, I, F, I],
         "li_paged_attention_decode": [P, I, P, P, P, I, P, I, P, I, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P],
-        "li_decode_run_keys": [P, I, P, P, P, P, I, I, I, I, I, I, I, P],
+        "li_decode_run_keys": [P, I, P, P, P, P, I, I, I, I, I, I, P],
     },
     "sampling": {
         "li_argmax_rows": [P, P, P, P, I, I],
@@ -1467,7 +1467,7 @@ def linear_rope_store_parts(x: torch.Tensor, w: torch.Tensor, bias: Optional[tor
 # waves that the split-key decode kernel on the matrix cores is cut into at least (where the keys allow): four a compute unit
 _DEC_WAVES = 1024
 PREFILL_TILE_ROWS = 32       # queries of one segment that a block of the matrix-core kernel for portions takes
-DECODE_MAX_SPLITS = 64       # the merge kernel keeps a weight per split
+DECODE_MAX_SPLITS = 64       # the merge kernel: a lane a split, four groups of sixteen
 DECODE_TABLE_CAP = 1024      # pages of one split that the matrix-core decode kernel copies into LDS
 DECODE_LIST_MAX_TOKENS = 4096    # single tokens whose runs the device lists (`decode_run_keys`)
 
@@ -1580,31 +1580,22 @@ def _decode_cut(pairs: int, keys: int, dh: int, dtype: torch.dtype, simds: int, 
 
 
 def _short_runs(pairs: int, keys: int, dh: int, dtype: torch.dtype, quads: int, aligned: bool = True, differ: bool = True):
-    """Asked for float32, for more than 512 pairs, and for a window or pages of no multiple of 8 keys (else: `_one_block`).  Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of
-    four runs a (token, kv head), which joins them itself and needs no list of runs; a pair of least lengths, runs of their own and the
-    kernel that joins them, from so short a run on; None, nothing else.  `quads`: the runs where blocks of four were the plan; `aligned`: no window and
-    pages of a multiple of 8 keys (the kernel's quicker form); `differ`: the contexts do, by `_ragged_splits`.
-    A run of 32 keys is a step, whose instructions (bfloat16, 0.9 us) or matrix products (float32, 1.8 us: six heads in tiles of 16) are
-    what it takes, and the second kernel with its trips to memory is 3 us.  Us a call, before / now:
-    bfloat16, beside portions, whose tables are as wide as they must be: 12 heads on 2 of 128, a table of 208 keys, 1 / 64 / 128 requests
-    8.3 / 10.0 / 13.2 -> 6.4 / 7.3 / 8.9; contexts of 30 to 300, 64 / 128 requests 11.0 / 15.2 -> 8.4 / 9.5, 3 requests 7.7 / 7.5; of 50 to 500, 3
-    requests 8.3 / 9.6 (so not there), 64 12.7 / 10.7; of 44 to 352, 50 to 400 and 56 to 448, 3 requests 8.2 / 7.8, 8.4 / 8.5, 8.4 / 8.8, 28 heads on 4, 8 requests 9.1 / 8.4,
-    8.8 / 9.3, 9.1 / 9.5 (heads of 128 therefore up to 384, of 64, 14 on 2, 8 requests of 100 to 440 8.1 / 6.6); of 100 to 1,000, 16 / 64 / 128 requests 10.1 / 14.0, 16.7 / 16.0, 25.4 / 20.0.  Few requests of
-    heads of 128, tables of 592 / 704 / 832 keys: the four runs of a block 9.3 / 9.9 / 11.1 (1 request), 9.8 / 10.3 / 11.3 (16), runs of 64 keys and more
-    8.1 / 8.1 / 8.3, 9.1 / 9.4 / 9.7 (496 keys, 8 kv heads: 7.7 / 7.9, so not there).  Recorded steps, whose tables are 256, 512 or 1,024 keys wide, contexts of
-    three quarters of that / spread from a tenth of it on: 14 heads on 2 of 64, 1 request 8.1 -> 5.2 at 256, 64 requests 9.7 / 10.0 -> 6.0 / 6.2, 6.8 /
-    10.9 -> 7.0 / 7.6, 11.7 / 13.1 -> 9.7 / 10.4; 12 on 2 of 128, 1 request 8.3 -> 6.6 at 256, 64 requests 10.0 / 10.9 -> 7.7 / 8.1, 9.3 / 12.6 -> 9.4 / 10.1,
-    15.7 / 16.1 -> 15.7 / 14.6.  Pages of 12 keys: 16 heads on 16 of 64, 8 requests of 105 to 840 11.4 / 11.0, of 153 to 1,224 12.1 / 14.6, 12 on 2 of 128, 64 of 1,224
-    21.1 / 22.0 (so up to 896).  More than 512 pairs are two waves a SIMD as they are: equal contexts of 144 / 256 keys, 16 heads on 16 of 64, 36 requests 0.88 / 0.94 times as
-    fast in blocks, 64 requests 9.2 / 11.7, 13.6 / 14.7 us, 28 on 4 of 128, 144 requests 0.68 / 0.82; contexts that differ 1.2 to 2.4 times (heads of 128, 2,048 and 4,096 pairs
-    under 256 keys 0.94 to 1.06).  576 and 640 pairs of equal contexts of 352 keys 1.06 to 1.6, 704 0.89 to 1.02.
-    float32, tables and contexts likewise: 12 heads on 2 of 128, 1 request 13.5, 15.4, 13.9 -> 8.7, 11.1, 11.9, 16 requests 14.3 / 12.6, 16.5 / 12.9, 15.5 / 14.6 -> 9.5 /
-    10.3, 12.4 / 11.4, 14.1 / 13.8; 14 on 2 of 64, 1 request 10.7, 8.6 (its whole table 10.4), 11.0 -> 7.8, 9.1 (9.2), 9.6, 16 requests 10.6 / 10.2, 9.2 / 10.8,
-    11.7 / 11.8 -> 7.7 / 9.0, 9.8 / 9.9, 11.1 / 12.2.  Not beyond 1,024 keys (2,048, 8 requests: 15.9 / 15.1 against 16.3 / 15.4, heads of 64 12.2 / 12.6 against
-    12.6 / 14.3; 1 request 14.6 / 15.0).  A table of 256 keys is also that of every shorter context: 58 keys in one run / in runs of 32 / in a block of four 7.5 / 8.1 /
-    5.5 (heads of 64), 8.6 / 9.0 / 7.1, 100 keys 9.0 / 8.2 / 6.0, 11.1 / 9.0 / 8.4, 192 10.7 / 7.8 / 7.2, 13.5 / 8.7 / 10.9; behind a window of 128 58 keys 6.1 / 7.7, 8.5 / 8.7, at 112 keys
-    7.2 / 7.5 / 5.3, 10.4 / 8.5 / 7.6: the block for heads of 64 up to 256 keys and for heads of 128 up to 128.  32 requests: 128 columns at 832 keys 25.2 / 16.1 -> 17.4 / 15.5, at 1,024 20.4 / 18.3 against 19.2 / 20.6; 64 columns at 304 keys
-    12.0 / 11.8 -> 9.9 / 10.3, at 400 9.2 / 11.8 against 10.4 / 10.6, at 512 9.5 / 11.9 against 11.3 / 11.4.  Up to 96 keys one run is the faster (7.8 / 8.5)."""
+    """Where the keys are few (as far as the host knows: a table's width), another cut than by `decode_splits` alone: DECODE_QUAD, one block of four runs a
+    (token, kv head), which joins them itself and needs no list of runs; a pair of least lengths, runs of their own and the kernel that joins them,
+    from so short a run on; None, nothing else.  `quads`: the runs where a block of four was the plan; `aligned`: no window and pages of a multiple of
+    8 keys (the kernel's quicker form); `differ`: the contexts do.  Asked for float32, for more than 512 pairs, and for other windows and pages (else
+    `_one_block`).  A run of 32 keys is a step, whose instructions (bfloat16, 0.9 us) or matrix products (float32, 1.8 us: six heads in tiles of 16) are what it
+    takes, and the second kernel with its trips to memory is 3 us.  Us a call, before / now:
+    bfloat16.  Up to 384 keys of 128 columns and 448 of 64, and more where the pairs are many; pages of 12 keys, 16 heads on 16 of 64, 8 requests of 105 to 840 11.4 / 11.0, of
+    153 to 1,224 12.1 / 14.6, 12 on 2 of 128, 64 of 1,224 21.1 / 22.0 (so up to 896).  More than 512 pairs are two waves a SIMD as they are: equal contexts of 144 / 256
+    keys, 16 heads on 16 of 64, 36 requests 0.88 / 0.94 times as fast in blocks, 64 requests 9.2 / 11.7, 13.6 / 14.7 us, 28 on 4 of 128, 144 requests 0.68 / 0.82; contexts that
+    differ 1.2 to 2.4 times (heads of 128, 2,048 and 4,096 pairs under 256 keys 0.94 to 1.06).  576 and 640 pairs of equal contexts of 352 keys 1.06 to 1.6, 704 0.89 to 1.02.
+    float32, contexts of the table / three quarters of it: 12 heads on 2 of 128, 1 request, tables of 256, 512 and 1,024 keys 13.5, 15.4, 13.9 -> 8.7, 11.1, 11.9, 16 requests 14.3 / 12.6,
+    16.5 / 12.9, 15.5 / 14.6 -> 9.5 / 10.3, 12.4 / 11.4, 14.1 / 13.8; 14 on 2 of 64, 1 request 10.7, 8.6 (its whole table 10.4), 11.0 -> 7.8, 9.1 (9.2), 9.6.  Not beyond
+    1,024 keys (2,048, 8 requests: 15.9 / 15.1 against 16.3 / 15.4, heads of 64 12.2 / 12.6 against 12.6 / 14.3).  A table of 256 keys is also that of every
+    shorter context: 58 keys in one run / in runs of 32 / in a block of four 7.5 / 8.1 / 5.5 (heads of 64), 8.6 / 9.0 / 7.1, 192 10.7 / 7.8 / 7.2, 13.5 / 8.7 / 10.9: the block for heads of
+    64 up to 256 keys and for heads of 128 up to 128.  32 requests: 128 columns at 832 keys 25.2 / 16.1 -> 17.4 / 15.5, at 1,024 20.4 / 18.3 against 19.2 / 20.6; 64 columns at
+    304 keys 12.0 / 11.8 -> 9.9 / 10.3, at 400 9.2 / 11.8 against 10.4 / 10.6.  Up to 96 keys one run is the faster (7.8 / 8.5)."""
     if dtype is torch.bfloat16:
         if pairs <= 512:
             blocks = True
@@ -1658,22 +1649,20 @@ def _ragged_splits(nsplit: int, meta, window: int, quad: int = DECODE_QUAD) -> i
 
 
 def decode_run_keys(meta, token_list: Optional[torch.Tensor], n_tokens: int, page_size: int, window: int,
-                    nkv: int, nsplit: int, simds: int, out: torch.Tensor, group: int = 1) -> None:
+                    nkv: int, nsplit: int, simds: int, out: torch.Tensor) -> None:
     """out[0] = the run length, in keys, for the split-key decode kernel over these single tokens
     (`token_list`, or the batch's first n_tokens tokens): the multiple of 32 with the least rounds of
     working waves over `simds` x (length + 24), between what the longest context needs to fit
     `nsplit` runs and what the block table's width would need.  out[1] = the number of runs with
     keys at that length, out[2 : 2 + n_tokens] = the runs of each token, then the runs themselves as
-    token | run << 16.  With `group` > 1 the runs are taken `group` at a time (one block of the decode
-    kernel): the list then holds the first run of every group, out[1] counts the groups, and a length's
-    cost counts `group` waves a group.  At most 4,096 tokens."""
+    token | run << 16.  At most 4,096 tokens."""
     _gpu(out, meta.ctx_len, token_list)
     _chk(0 < n_tokens <= DECODE_LIST_MAX_TOKENS, "decode_run_keys: too many tokens")
     _chk(out.dtype is torch.int32 and out.is_contiguous() and out.numel() >= 2 + n_tokens + n_tokens * nsplit,
          "decode_run_keys: out must be int32 [2 + tokens + tokens * nsplit]")
     _run("attention", "li_decode_run_keys", 0 if token_list is None else token_list.data_ptr(), n_tokens,
          meta.seg_of_token.data_ptr(), meta.q_start.data_ptr(), meta.q_len.data_ptr(), meta.ctx_len.data_ptr(),
-         meta.max_blocks, page_size, int(window), nkv, nsplit, simds, int(group), out.data_ptr())
+         meta.max_blocks, page_size, int(window), nkv, nsplit, simds, out.data_ptr())
 
 
 def _decode_plan(meta, pairs: int, keys: int, dh: int, dtype: torch.dtype, page_size: int, window: int, simds: int):
@@ -1886,7 +1875,7 @@ def sample_rows_packed(logits: torch.Tensor, rows: torch.Tensor, out: torch.Tens
     _sample_rows(logits, n, at, at + 12 * n, at + 4 * n, at + 8 * n, out)
 
 
-SAMPLE_CALL_ROWS = 128         # rows up to which `sample_call` takes a step's options
+SAMPLE_CALL_ROWS = 128         # rows up to which `sample_call` takes a step's options (as csrc/sampling.hip has it, which refuses more)
 
 
 def sample_call(logits: torch.Tensor, records: bytes, counters: array, out: torch.Tensor, host: torch.Tensor) -> None:
