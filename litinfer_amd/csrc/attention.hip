@@ -600,6 +600,7 @@ template <int WAVES, int DH> struct DecodeJoin {
 };
 template <int DH> struct DecodeJoin<1, DH> { int unused; };
 
+#define HEADS_FIRST_BLOCKS 20480
 #define DEC_WHOLE_TABLE 64       // pages up to which a wave asks for a request's whole table before it knows the request's length
 
 // ALIGNED: no window and pages of a multiple of 8 keys, so that 8 (4) keys from a multiple of 8 (4) lie in one page and their rows behind each
@@ -613,7 +614,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     int max_blocks, const int* __restrict__ token_list, const int* __restrict__ seg_of_token,
     const int* __restrict__ q_start, const int* __restrict__ q_len, const int* __restrict__ ctx_len,
     float* __restrict__ part_acc, float* __restrict__ part_ml, int nh, int nkv, int page_size,
-    int num_pages, int window, float scale, int nsplit, const int* __restrict__ run_keys, int n_list) {
+    int num_pages, int window, float scale, int nsplit, const int* __restrict__ run_keys, int n_list, int heads_first) {
     static_assert(DH <= ATT_MAX_DH / 2, "the join buffer holds head sizes up to 128");
     constexpr bool F32 = sizeof(T) == 4;        // float32: v_mfma_f32_16x16x4f32 on float32 operands
     constexpr int KS = DH / 32;                 // bfloat16: MFMA steps of Q K^T
@@ -632,17 +633,19 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     T* p_lds = p_lds_all[wave];
     int* pages = pages_all[wave];
     const int nruns_all = nsplit * WAVES;       // runs that the keys are cut into at most
-    // run_keys given (single waves): the kv heads of an item of the list behind it, a (token, run) pair, are blocks that follow each other, and blocks past
-    // the list's end leave at once.  Blocks go to the XCDs and their compute units in turn, in the order of their numbers, so those that have keys
-    // come first, all heads', and are dealt out evenly (head by head, each with its empty blocks behind it, some units had more of the next head's
-    // than others: 64 requests of 16 to 4,600 keys, 28 heads on 4, 76.6 -> 68.0 us a layer).  Else block (token, kv head, run) of the grid.
+    // run_keys given (single waves): a block takes a kv head of an item of the list behind it, a (token, run) pair, and leaves at once if the list is
+    // shorter.  Blocks go to the XCDs and their compute units in turn, in the order of their numbers.  heads_first: an item's heads follow each
+    // other, so that the blocks that have keys come first and are dealt out evenly (head by head, each with its empty blocks behind it, some
+    // units had more of the next head's than others: 64 requests of 16 to 4,600 keys, 28 heads on 4, 76.6 -> 68.0 us a layer).  Of a very large
+    // grid head by head all the same: there the empty blocks' time is what counts, and it passes beside the work of the heads before (37,600 blocks, one
+    // of 1,500 keys beside 99 of 187, 32 heads on 8 of 64: 24.0 so, 30.4 heads first).  Else block (token, kv head, run) of the grid.
     int ti = blockIdx.x, split = WAVES > 1 ? wave : blockIdx.z, kvh = blockIdx.y;
     if (WAVES == 1 && run_keys) {
-        const int place = blockIdx.z * gridDim.y + blockIdx.y, last = n_list * nsplit - 1;
+        const int place = heads_first ? blockIdx.y : blockIdx.x;
         const int count = run_keys[1];
-        const int item = run_keys[2 + n_list + (place < last ? place : last)];
+        const int item = run_keys[2 + n_list + place];
         if (place >= count) return;
-        kvh = blockIdx.x;
+        kvh = heads_first ? blockIdx.x : blockIdx.y;
         ti = item & 0xffff;
         split = item >> 16;
     }
@@ -2535,9 +2538,10 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
     const bool aligned = window <= 0 && page_size % 8 == 0;
     const bool listed = run_keys != nullptr && nsplit > 1 && use_mfma == 2;
     if (listed && (n_tokens > RUN_KEYS_MAX_TOKENS || nsplit > 0x7fff)) return LI_ERR_SIZE;
+    const int heads_first = listed && (long)n_tokens * nsplit * nkv <= HEADS_FIRST_BLOCKS;
 #define LI_DM4(DHV, W, AL, BLOCKS) paged_attention_decode_mfma_kernel<T, DHV, W, AL><<<grid, 64 * W, 0, stream>>>( \
         q, q_row_stride, out, kc, vc, block_table, max_blocks, token_list, seg_of_token, q_start, q_len, ctx_len, \
-        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, BLOCKS, listed ? run_keys : nullptr, n_tokens)
+        part_acc, part_ml, nh, nkv, page_size, num_pages, window, scale, BLOCKS, listed ? run_keys : nullptr, n_tokens, heads_first)
 #define LI_DM(W, BLOCKS)                                                                                     \
     {                                                                                                        \
         if (dh == 128) { if (aligned) LI_DM4(128, W, true, BLOCKS); else LI_DM4(128, W, false, BLOCKS); }    \
@@ -2550,8 +2554,7 @@ static int launch_decode_mfma(const T* q, int q_row_stride, T* out, const T* kc,
     }
     if (use_mfma == 2) {
         if (!part_acc || !part_ml) return LI_ERR_SIZE;
-        const int items = n_tokens * nsplit, slice = items < 32768 ? items : 32768;      // (of a listed batch: at most 4,096 tokens)
-        const dim3 grid = listed ? dim3(nkv, slice, (items + slice - 1) / slice) : dim3(n_tokens, nkv, nsplit);
+        const dim3 grid = heads_first ? dim3(nkv, n_tokens * nsplit) : listed ? dim3(n_tokens * nsplit, nkv) : dim3(n_tokens, nkv, nsplit);
         LI_DM(1, nsplit)
         launch_merge(part_acc, part_ml, token_list, out, n_tokens, nh, dh, nsplit, listed ? run_keys + 2 : nullptr, stream);
         return li_launch_status();

@@ -956,10 +956,10 @@ def test_any_number_of_runs_is_joined(ops, monkeypatch, runs, dtype):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("requests,runs", [(171, 64), (172, 17), (172, 33), (560, 64)])
+@pytest.mark.parametrize("requests,runs", [(160, 64), (161, 64), (171, 17), (172, 33), (560, 64)])
 def test_runs_of_many_tokens_with_a_long_one_among_them_are_joined(ops, monkeypatch, requests, runs, dtype):
-    # 171 x 6 (token, head)s and more: one group of the joining kernel's threads takes a token's runs sixteen at a time; 560 x 64
-    # items of the list are more than one slice of the decode kernel's grid
+    # from 171 x 6 (token, head)s on one group of the joining kernel's threads takes a token's runs sixteen at a time; from 161 x 64 x 2
+    # blocks on the listed runs go head by head
     monkeypatch.setattr(ops, "_decode_cut", lambda *a: (runs, 1, 1))
     segs = [(1 + (7 * i) % 45, 1) for i in range(requests)]
     segs[requests // 2], segs[3] = (32 * runs - 5, 1), (16 * 32, 1)
