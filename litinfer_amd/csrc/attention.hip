@@ -638,7 +638,7 @@ __global__ __launch_bounds__(64 * WAVES) void paged_attention_decode_mfma_kernel
     // other, so that the blocks that have keys come first and are dealt out evenly (head by head, each with its empty blocks behind it, some
     // units had more of the next head's than others: 64 requests of 16 to 4,600 keys, 28 heads on 4, 76.6 -> 68.0 us a layer).  Of a very large
     // grid head by head all the same: there the empty blocks' time is what counts, and it passes beside the work of the heads before (37,600 blocks, one
-    // of 1,500 keys beside 99 of 187, 32 heads on 8 of 64: 24.0 so, 30.4 heads first).  Else block (token, kv head, run) of the grid.
+    // of 1,500 keys beside 99 of 187, 32 heads on 8 of 64, a window of 4,096: 20.9 so, 30.4 heads first).  Else block (token, kv head, run) of the grid.
     int ti = blockIdx.x, split = WAVES > 1 ? wave : blockIdx.z, kvh = blockIdx.y;
     if (WAVES == 1 && run_keys) {
         const int place = heads_first ? blockIdx.y : blockIdx.x;

@@ -1516,8 +1516,8 @@ def _one_block(pairs: int, keys: int, dh: int, simds: int, spread=None, padded: 
     """Whether a block of DECODE_QUAD waves takes all of a (token, kv head)'s keys and joins its runs itself, rather than runs of single waves and the
     kernel that joins them (bfloat16, up to 512 pairs, the kernel's quicker form).  `spread`: `_single_keys`; padded: the step may be recorded,
     and replayed for other contexts of the same tables.
-    Few keys: it saves the second kernel.  A whole step of 28 layers, 12 heads on 2 of 128, runs / one block, contexts of 0.58 and of 0.5 to 1 of the table: 48
-    pairs, 512 keys 1,677 and 1,686 / 1,681 and 1,746, 80 pairs 1,735 and 1,746 / 1,712 and 1,760, 128 pairs, 1,024 keys 2,161 and 2,126 / 2,133 and 2,133; 24 layers, 14 on 2 of 64: 16
+    Few keys: it saves the second kernel.  A whole step of 28 layers, 12 heads on 2 of 128, runs / one block: 6 pairs, 256 keys, contexts of 7 to 59 1,169 / 1,147, 14 pairs,
+    47 to 94 1,278 / 1,260 (16 pairs, 200 to 250 1,283 / 1,322); contexts of 0.58 and of 0.5 to 1 of the table, 48 pairs, 512 keys 1,677 and 1,686 / 1,681 and 1,746, 80 pairs 1,735 and 1,746 / 1,712 and 1,760, 128 pairs, 1,024 keys 2,161 and 2,126 / 2,133 and 2,133; 24 layers, 14 on 2 of 64: 16
     pairs, 512 keys 797 and 798 / 801 and 833, 48 pairs 997 and 1,004 / 977 and 1,002, 80 pairs, 1,024 keys 1,227 and 1,230 / 1,263 and 1,258, 128 pairs 1,402 and 1,393 / 1,378 and 1,377.
     Many keys: it pays where the pairs fill the chip with a block each, or nearly, and where no context is much longer than the others: its four waves take
     the longest alone, while runs are shared out among all SIMDs.  By the keys that the busiest SIMD works on: a quarter of the longest context (of the mean one
@@ -1537,7 +1537,7 @@ def _one_block(pairs: int, keys: int, dh: int, simds: int, spread=None, padded: 
             return keys <= (640 if dh == 128 else 1024)
         if dh == 64:
             return keys <= max(256 + 7 * pairs, 10 * pairs)
-        return pairs > 48 and keys <= 10 * pairs
+        return keys <= (10 * pairs if pairs > 48 else 256)
     if not fills:
         return False
     if spread is None:
@@ -1556,7 +1556,7 @@ def _decode_cut(pairs: int, keys: int, dh: int, dtype: torch.dtype, simds: int, 
     least, or of 32 and to a finer cut where the pairs are few: the kernel that joins runs asks for all of them at once, so that a run costs it
     little.  Where all runs are at work at one time anyway, no run is longer than 128 keys and no context much longer than the others, every token's keys are cut
     into the same number of runs: one run length for the batch, and the list of the runs that have keys, would cost a kernel of its own and a trip in every
-    layer.  A step of 28 layers, 12 heads on 2 of 128, the list / none: 4 requests of 260 to 500 keys 1,208 / 1,178, 16 of 90 to 181 1,397 / 1,373, 64 of 600 to 1,000
+    layer.  A step of 28 layers, 12 heads on 2 of 128, the list / none: 4 requests of 260 to 500 keys 1,208 / 1,178, 16 of 260 to 500 1,428 / 1,381, 64 of 600 to 1,000
     2,159 / 2,126; a call of 28 heads on 4, 8 requests of 512 to 4,096 keys 18.5 / 16.4, one of 4,096 beside 7 of 200 11.1 / 14.9 (so not there)."""
     bf16 = dtype is torch.bfloat16
     spread = _single_keys(meta, window)

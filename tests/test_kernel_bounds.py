@@ -210,6 +210,14 @@ def test_products_are_cut_into_no_more_parts_than_are_added_up():
     assert most[True] == ops.SPLITK_MAX_PARTS == 16 and most[False] == 8
 
 
+@pytest.mark.parametrize("aligned,dtype", [(False, ops.torch.bfloat16), (True, ops.torch.float32)])
+def test_many_equal_contexts_that_fill_the_simds_keep_one_run(aligned, dtype):
+    for n, keys, runs in ((100, 1500, 1), (100, 1024, 1), (64, 1500, None)):
+        ns, waves, planned = ops._decode_cut(8 * n, keys, 64, dtype, 1024, aligned, _decode_batch([keys] * n), 0)
+        assert ns == planned and (ns == 1) == (runs == 1), (n, keys, ns)
+    assert ops._decode_cut(800, 1500, 64, dtype, 1024, aligned, _decode_batch([1500] + [200] * 99), 0)[0] > 1
+
+
 @pytest.mark.parametrize("pairs,dh,block,ends", [(2, 64, 256, 1024), (32, 64, 256, 1024), (32, 128, 128, 1024), (33, 64, 256, 320), (64, 128, 128, 1008),
                                                  (65, 128, 0, 0), (65, 64, 0, 0)])
 def test_float32_decoding_is_cut_shorter_only_where_that_was_measured(pairs, dh, block, ends):
@@ -239,7 +247,7 @@ def _decode_plan_of(ctx, nkv, dh=128, table=0, padded=False):
 
 
 @pytest.mark.parametrize("pairs,dh,ends", [(1, 64, 263), (8, 64, 312), (36, 64, 508), (37, 64, 515), (65, 64, 711), (85, 64, 851), (86, 64, 860), (128, 64, 1280), (191, 64, 1280),
-                                           (192, 64, None), (256, 64, None), (257, 64, 1024), (383, 64, 1024), (384, 64, None), (512, 64, None), (32, 128, 0), (48, 128, 0),
+                                           (192, 64, None), (256, 64, None), (257, 64, 1024), (383, 64, 1024), (384, 64, None), (512, 64, None), (1, 128, 256), (32, 128, 256), (48, 128, 256),
                                            (49, 128, 490), (64, 128, 640), (128, 128, 1280), (160, 128, 1280), (192, 128, None), (320, 128, 640)])
 def test_a_block_takes_all_runs_only_where_that_was_measured(pairs, dh, ends):
     """Of contexts that are alike, or that the host does not know."""
