@@ -1393,7 +1393,7 @@ static int tail_blocks(const HeadTail& tail, int tokens, int threads) {
     return (int)(n < 16 ? n : 16);
 }
 
-template <typename TX, typename TM, typename TO, bool VEC, int TOK>
+template <typename TX, typename TM, typename TO, bool VEC, int TOK, int ASK = HL_AHEAD>
 __global__ __launch_bounds__(256) void headwise_linear_kernel(
     const TX* __restrict__ x, long x_token_stride, int x_head_stride, const TM* __restrict__ m, TO* __restrict__ out,
     long o_token_stride, int o_head_stride, int T_, int n_out, int n_in, const float* __restrict__ gate, long gate_stride,
@@ -1409,11 +1409,11 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
     constexpr int E = VEC ? 16 / (int)sizeof(TM) : 1;
     constexpr bool AHEAD = VEC && TOK < HL_TOK, EARLY = TOK <= 2;
     const int part = threadIdx.x & 3, pieces = n_in / E;       // (VEC: a whole number; a thread takes the pieces part, part + 4, ...)
-    [[maybe_unused]] uint4 raw[HL_AHEAD];
+    [[maybe_unused]] uint4 raw[ASK];
     auto ask = [&](int j, int c0) {
         const TM* row = m + ((size_t)h * n_out + (j < n_out ? j : 0)) * n_in;
 #pragma unroll
-        for (int u = 0; u < HL_AHEAD; ++u) raw[u] = *reinterpret_cast<const uint4*>(row + (size_t)(c0 + 4 * u < pieces ? c0 + 4 * u : pieces - 1) * E);
+        for (int u = 0; u < ASK; ++u) raw[u] = *reinterpret_cast<const uint4*>(row + (size_t)(c0 + 4 * u < pieces ? c0 + 4 * u : pieces - 1) * E);
     };
     const int j_first = blockIdx.z * 64 + (threadIdx.x >> 2);
     if constexpr (AHEAD && EARLY) ask(j_first, part);         // (on its way beside the tokens' inputs)
@@ -1471,10 +1471,10 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
                 for (int tt = 0; tt < TOK; ++tt) acc[tt] = fmaf(wv[e], xs[tt * n_in + k + e], acc[tt]);
         };
         if constexpr (AHEAD) {
-            for (int c0 = part; c0 < pieces; c0 += 4 * HL_AHEAD) {
+            for (int c0 = part; c0 < pieces; c0 += 4 * ASK) {
                 if (!EARLY || j != j_first || c0 != part) ask(j, c0);
 #pragma unroll
-                for (int u = 0; u < HL_AHEAD; ++u) {
+                for (int u = 0; u < ASK; ++u) {
                     if ((c0 + 4 * u) * E >= n_in) break;
                     take(raw[u], (c0 + 4 * u) * E);
                 }
@@ -1520,7 +1520,7 @@ __global__ __launch_bounds__(256) void headwise_linear_kernel(
 // 4.1, of 256 x 128 with float32 inputs 5.2 -> 4.2; 200 tokens 6.8 -> 5.2 and 5.7 -> 5.15; the same from 1,000 on, where float32 inputs
 // go a step at a time as before (eight at once: 14.6 -> 15.2, 39.0 -> 46.0 at 3,000).
 template <typename TX, typename TO, int HL_STEPS, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void headwise_linear_mfma_kernel(
+__global__ __launch_bounds__(64 * WAVES, HL_STEPS == 1 ? 8 : 1) void headwise_linear_mfma_kernel(
     const TX* __restrict__ x, long x_token_stride, int x_head_stride, const bf16_t* __restrict__ m, TO* __restrict__ out,
     long o_token_stride, int o_head_stride, int T_, int n_out, int n_in, const float* __restrict__ gate, long gate_stride,
     int gate_per_column, HeadTail tail, int zs) {
@@ -1551,6 +1551,21 @@ __global__ __launch_bounds__(64 * WAVES) void headwise_linear_mfma_kernel(
     ma_f32x16 acc;
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    if constexpr (HL_STEPS == 1) {
+        for (int k = 0; k < n_in; k += 16) {
+            ma_frag8 a, b;
+            a.raw = *reinterpret_cast<const uint4*>(mrow + k);
+            if constexpr (sizeof(TX) == 2) {
+                b.raw = *reinterpret_cast<const uint4*>(xrow + k);
+            } else {
+                const float4 u = *reinterpret_cast<const float4*>(xrow + k);
+                const float4 v = *reinterpret_cast<const float4*>(xrow + k + 4);
+                b.w[0] = pack2_bf16(u.x, u.y); b.w[1] = pack2_bf16(u.z, u.w);
+                b.w[2] = pack2_bf16(v.x, v.y); b.w[3] = pack2_bf16(v.z, v.w);
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a.v, b.v, acc, 0, 0, 0);
+        }
+    }
     // (whole: no step is past the end.  Else both operands of those that are are zeros: a question a step would have its loads wait for it)
     auto steps = [&](int k0, auto whole_tag) {
         constexpr bool WHOLE = decltype(whole_tag)::value;
@@ -1577,10 +1592,11 @@ __global__ __launch_bounds__(64 * WAVES) void headwise_linear_mfma_kernel(
             acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[i].v, b[i].v, acc, 0, 0, 0);
         }
     };
-    int k0 = 0;
-    for (; k0 + 16 * HL_STEPS <= n_in; k0 += 16 * HL_STEPS) steps(k0, std::true_type{});
-    if constexpr (HL_STEPS > 1)
+    if constexpr (HL_STEPS > 1) {
+        int k0 = 0;
+        for (; k0 + 16 * HL_STEPS <= n_in; k0 += 16 * HL_STEPS) steps(k0, std::true_type{});
         if (k0 < n_in) steps(k0, std::false_type{});
+    }
     if (t0 + ql >= T_) return;
     if constexpr (HL_STEPS == 1) ask_gates();
     if (gate && gate_per_column) {
@@ -1625,7 +1641,13 @@ static bool headwise_mfma(const void* x, long xts, int xhs, const void* m, void*
     const dim3 grid((unsigned)rows, nh, zs + tail_blocks(tail, T_ < 32 ? T_ : 32, 64 * waves));
 #define HL_MFMA(STEPS, WAVES) headwise_linear_mfma_kernel<TX, TO, STEPS, WAVES><<<grid, 64 * WAVES, 0, stream>>>(         \
         (const TX*)x, xts, xhs, (const bf16_t*)m, (TO*)out, ots, ohs, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail, zs)
-    if (waves == 1) HL_MFMA(8, 1); else HL_MFMA((sizeof(TX) == 2 ? 8 : 1), 4);
+    // (as many steps as a row has, or that divide it: asked for past its end they cost what the others do.  64 heads of 64 x 64, 100 / 300 / 1,000 tokens, a step at a
+    // time 3.6 / 5.1 / 11.2, eight at once 3.9 / 6.3 / 14.1, four 3.5 / 5.0 / 10.6; float32 inputs a step at a time in eight waves a SIMD, which
+    // the registers of seven made 4 to 6 % longer: 28 heads of 512 x 128, 1,000 tokens 49.8 / 52.3)
+    const int at_once = n_in <= 32 || (waves == 4 && sizeof(TX) == 4) ? 1 : n_in <= 64 || (n_in % 128 && n_in % 64 == 0) ? 4 : 8;
+    if (waves == 1) { if (at_once == 1) HL_MFMA(1, 1); else if (at_once == 4) HL_MFMA(4, 1); else HL_MFMA(8, 1); }
+    else if (at_once == 1) HL_MFMA(1, 4);
+    else if constexpr (sizeof(TX) == 2) { if (at_once == 4) HL_MFMA(4, 4); else HL_MFMA(8, 4); }
 #undef HL_MFMA
     return true;
 }
@@ -1650,15 +1672,17 @@ extern "C" int li_headwise_linear(const void* x, int x_dtype, long x_token_strid
     const int all = (n_out + 63) / 64, zs = all < 64 ? all : 64, tok = T_ <= 1 ? 1 : T_ <= 2 ? 2 : T_ <= HL_FEW ? 4 : HL_TOK;
     const dim3 grid((T_ + tok - 1) / tok, nh, zs + tail_blocks(tail, T_ < tok ? T_ : tok, 256));
     const size_t lds = (size_t)tok * n_in * 4;
-#define HL_AS(TX, TM, TO, VEC, TOK)                                                                                        \
-    headwise_linear_kernel<TX, TM, TO, VEC, TOK><<<grid, 256, lds, stream>>>(                                              \
+#define HL_AS(TX, TM, TO, VEC, ...)                                                                                        \
+    headwise_linear_kernel<TX, TM, TO, VEC, __VA_ARGS__><<<grid, 256, lds, stream>>>(                                              \
         (const TX*)x, x_token_stride, x_head_stride, (const TM*)m, (TO*)out, o_token_stride, o_head_stride, T_, n_out, n_in, gate, gate_stride, gate_per_column, tail, zs)
 #define HL_GO(TX, TM, TO)                                                                                                  \
     {                                                                                                                      \
         constexpr int E = 16 / sizeof(TM);                                                                                 \
         if (n_in % E == 0 && ((uintptr_t)m % 16) == 0) {                                                                   \
-            if (tok == 1) HL_AS(TX, TM, TO, true, 1); else if (tok == 2) HL_AS(TX, TM, TO, true, 2);                       \
-            else if (tok == 4) HL_AS(TX, TM, TO, true, 4); else HL_AS(TX, TM, TO, true, HL_TOK);                           \
+            if (tok == HL_TOK) HL_AS(TX, TM, TO, true, HL_TOK);                                                            \
+            else if (tok == 4) HL_AS(TX, TM, TO, true, 4);                                                                 \
+            else if (n_in <= 8 * E) { if (tok == 1) HL_AS(TX, TM, TO, true, 1, 2); else HL_AS(TX, TM, TO, true, 2, 2); }   \
+            else if (tok == 1) HL_AS(TX, TM, TO, true, 1); else HL_AS(TX, TM, TO, true, 2);                                \
         } else {                                                                                                           \
             if (tok == 1) HL_AS(TX, TM, TO, false, 1); else if (tok == 2) HL_AS(TX, TM, TO, false, 2);                     \
             else if (tok == 4) HL_AS(TX, TM, TO, false, 4); else HL_AS(TX, TM, TO, false, HL_TOK);                         \
