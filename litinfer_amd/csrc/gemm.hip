@@ -1690,6 +1690,13 @@ __global__ __launch_bounds__(NT) void splitk_reduce_norm_kernel(const float* __r
 // multiple of 4, up to 1,024 PER.
 #define REDUCE_ROWS_NT 256
 #define REDUCE_ROWS_FROM 256
+// Not where a unit has one row (256 rows) and this is long, nor, below 600 rows, where a quarter of the threads has one piece of many parts less than
+// the others: us, the product with those blocks / with these, 256 x 2,048 x 4,864 (8 parts) 20.3 / 20.7, 256 x 3,584 x 4,864 (4) 25.1 / 25.5, 280 x 1,536 x
+// 8,960 (7) 23.1 / 23.9, 450 (5) 28.1 / 28.7, 700 (3) 35.1 / 34.2, 280 x 2,048 x 4,864 (5) 23.7 / 23.4.
+static bool reduce_by_rows(int M, int N, int nsplit) {
+    if (nsplit > 4 && N > 1024 && N < 2048) return M >= 600;
+    return M > REDUCE_ROWS_FROM || (M == REDUCE_ROWS_FROM && N * nsplit <= 6144);
+}
 template <int HELD, int PER>
 __global__ __launch_bounds__(REDUCE_ROWS_NT) void splitk_reduce_norm_rows_kernel(const float* __restrict__ part, int nsplit, size_t mn, int N,
                                                                                   const float* __restrict__ bias, float* __restrict__ out,
@@ -2273,7 +2280,7 @@ extern "C" int li_linear_then_norm(const void* x, const void* w, const float* bi
         : launch_dma<128, 128, 64, 4, false, float>((const bf16_t*)x, (const bf16_t*)w, nullptr, (float*)work, M, N, K, 0, stream, nsplit);
     if (rc != LI_OK) return rc;
     const uintptr_t places = (uintptr_t)work | (uintptr_t)bias | (uintptr_t)out | (uintptr_t)gamma | (uintptr_t)xn;
-    if (M >= REDUCE_ROWS_FROM && xn_dtype == LI_BF16 && N % 4 == 0 && places % 16 == 0) {
+    if (reduce_by_rows(M, N, nsplit) && xn_dtype == LI_BF16 && N % 4 == 0 && places % 16 == 0) {
         (nsplit <= 2 ? launch_reduce_norm_rows<2> : nsplit <= 4 ? launch_reduce_norm_rows<4> : launch_reduce_norm_rows<PARTS_HELD>)(
             (const float*)work, nsplit, M, N, bias, out, factor, gamma, eps, (bf16_t*)xn, stream);
         return li_launch_status();

@@ -486,7 +486,8 @@ def test_linear_into_the_residual_sum_with_its_norm(ops, m, n, k, bias, taken):
 
 
 @pytest.mark.parametrize("m,n,k,bias", [(255, 1536, 1536, True), (256, 1536, 1536, True), (1027, 1536, 1024, False), (300, 512, 8192, True), (700, 896, 1088, False),
-                                        (257, 2052, 2048, True), (256, 4096, 1024, False), (300, 5124, 1024, True), (256, 8192, 1024, False), (300, 1538, 4096, True)])
+                                        (257, 2052, 2048, True), (256, 4096, 1024, False), (300, 5124, 1024, True), (256, 8192, 1024, False), (300, 1538, 4096, True),
+                                        (257, 4096, 1024, True), (258, 8192, 1024, False), (280, 2048, 4864, True), (599, 1536, 8960, True), (600, 1536, 8960, True)])
 def test_parts_of_many_rows_with_their_norm(ops, m, n, k, bias):
     """From 256 rows on four columns a load: two, three, four and eight parts; one to eight pieces a thread; rows of no multiple of four."""
     test_linear_into_the_residual_sum_with_its_norm(ops, m, n, k, bias, ops._work_bytes(m, n, k, ops._DT[torch.bfloat16]) > 0)
