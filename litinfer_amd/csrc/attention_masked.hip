@@ -35,14 +35,18 @@ __device__ __forceinline__ int lower_edge(int p, int window, int chunk) {
 
 // What a (token, head)'s sums of values are multiplied by at the end: one over the sum of the weights (with the sink's
 // term, counted once), and the head's gate where heads have one.
+__device__ __forceinline__ float finish_factor(float l, float m, const MaExtras& ex, int t, int head) {
+    if (ex.sink && l != 0.f) l += expf(ex.sink[head] - m);
+    float f = l != 0.f ? 1.0f / l : 0.f;
+    if (ex.gate && !ex.per_column) f *= 1.0f / (1.0f + expf(-ex.gate[(size_t)t * ex.gate_stride + head]));
+    return f;
+}
+// the same of a sink and a gate that were asked for before (the kernels that asked so for nothing took 0.1 to 0.2 us more)
 __device__ __forceinline__ float finish_factor_of(float l, float m, const MaExtras& ex, float sink, float gate) {
     if (ex.sink && l != 0.f) l += expf(sink - m);
     float f = l != 0.f ? 1.0f / l : 0.f;
     if (ex.gate && !ex.per_column) f *= 1.0f / (1.0f + expf(-gate));
     return f;
-}
-__device__ __forceinline__ float finish_factor(float l, float m, const MaExtras& ex, int t, int head) {
-    return finish_factor_of(l, m, ex, ex.sink ? ex.sink[head] : 0.f, ex.gate && !ex.per_column ? ex.gate[(size_t)t * ex.gate_stride + head] : 0.f);
 }
 
 // The gate of one value column (1 where the columns have none of their own), and of four neighbouring ones at once.
