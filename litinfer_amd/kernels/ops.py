@@ -1818,10 +1818,11 @@ class _Scratch(threading.local):
     def __init__(self):
         self.buffers: Dict[tuple, torch.Tensor] = {}
 
-    def floats(self, n: int, device: torch.device) -> torch.Tensor:
-        if torch.cuda.is_current_stream_capturing():
+    def floats(self, n: int, device: torch.device, recording: Optional[bool] = None) -> torch.Tensor:
+        """recording: whether the current stream is, where the caller knows it (to ask takes 0.3 us)."""
+        if torch.cuda.is_current_stream_capturing() if recording is None else recording:
             return torch.empty(n, dtype=torch.float32, device=device)       # (the recording's own: its replays use it whatever is asked for later)
-        key = (device, _stream())
+        key = (device.index, _stream())
         buf = self.buffers.get(key)
         if buf is None or buf.numel() < n:
             if buf is None and len(self.buffers) >= self.STREAMS:
@@ -1880,7 +1881,8 @@ def sample_rows_packed(logits: torch.Tensor, rows: torch.Tensor, out: torch.Tens
 SAMPLE_CALL_ROWS = 128         # rows up to which `sample_call` takes a step's options (as csrc/sampling.hip has it, which refuses more)
 
 
-def sample_call(logits: torch.Tensor, records: bytes, counters: array, out: torch.Tensor, host: torch.Tensor) -> None:
+def sample_call(logits: torch.Tensor, records: bytes, counters: array, out: torch.Tensor, host: torch.Tensor,
+                recording: Optional[bool] = None) -> None:
     """`sample_rows` with the rows' options and streams in the launch's own arguments: `records`, 24 bytes a row (temperature and top_p as
     float32, the seed as uint64, top_k as int32, four more), `counters`, array("Q"), the number of each row's draw; row i's token goes
     to out[i] on the device and to host[i], pinned memory of the host (complete when the stream has come past the call).  At most SAMPLE_CALL_ROWS rows."""
@@ -1890,7 +1892,7 @@ def sample_call(logits: torch.Tensor, records: bytes, counters: array, out: torc
     _chk(0 < n <= SAMPLE_CALL_ROWS and len(records) == 24 * n and len(counters) == n and counters.itemsize == 8, "sample: per-row options")
     _chk(out.dtype is torch.int32 and out.numel() == n and out.is_contiguous(), "sample: out")
     _chk(host.dtype is torch.int32 and host.numel() >= n and host.is_contiguous() and host.is_pinned(), "sample: host")
-    tiles = _scratch.floats(_sample_scratch_floats(n, v), logits.device)
+    tiles = _scratch.floats(_sample_scratch_floats(n, v), logits.device, recording)
     _run("sampling", "li_sample_call", logits.data_ptr(), records, counters.buffer_info()[0], out.data_ptr(), host.data_ptr(), n, v, tiles.data_ptr(),
          tiles.numel())
 

@@ -90,11 +90,15 @@ _unread_lock = threading.Lock()
 _DRAIN_AT_ONCE = 8                      # entries that a look takes; a call adds one at most, so what has been written does not pile up
 
 
-def _drain() -> None:
-    """Let go of memory of `_unread` that has been written by now.  An entry is taken out, asked, and put back if its event has not come: only the
-    holder of the lock takes entries out, so no entry goes that was not asked; a thread that finds the lock held leaves it to the holder."""
-    if not _unread or torch.cuda.is_current_stream_capturing() or not _unread_lock.acquire(blocking=False):
-        return
+def _drain(n: int = 0, recording: Optional[bool] = None) -> Optional[torch.Tensor]:
+    """Let go of memory of `_unread` that has been written by now; what holds n ids of it is the caller's, if he wants it (a new allocation takes
+    longer).  An entry is taken out, asked, and put back if its event has not come: only the holder of the lock takes entries out, so no entry
+    goes that was not asked; a thread that finds the lock held leaves it to the holder.  recording: whether the stream is, where that is known."""
+    if recording is None:
+        recording = torch.cuda.is_current_stream_capturing()
+    if recording or not _unread_lock.acquire(blocking=False):
+        return None
+    room = None
     try:
         for _ in range(min(len(_unread), _DRAIN_AT_ONCE)):
             entry, done = _unread.popleft(), False
@@ -103,8 +107,11 @@ def _drain() -> None:
             finally:
                 if not done:
                     _unread.append(entry)
+            if done and entry[1].numel() >= n:
+                room = entry[1]
     finally:
         _unread_lock.release()
+    return room
 
 
 class PendingTokens:
@@ -126,8 +133,8 @@ class PendingTokens:
             if self._event is not None:
                 self._event.synchronize()
             self._tokens = self._host[:self._n].tolist()
-            self._sampler._give_back(self._host)
-            self._host = None
+            self._sampler._give_back(self._host, self._event)
+            self._host = self._event = None
         return self._tokens
 
 
@@ -137,6 +144,7 @@ class Sampler:
         every call brings its rows' options and counters from the host."""
         self.device = torch.device(device)
         self._free_host: List[torch.Tensor] = []
+        self._free_events: list = []
         self._params_up = None
         self.slots = int(slots)
         self.table = (torch.zeros((self.slots, ops.SAMPLE_SLOT_WORDS), dtype=torch.int32, device=self.device)
@@ -189,22 +197,33 @@ class Sampler:
         hb = self._host_buffer(n)
         if self.device.type == "cuda":
             hb[:n].copy_(ids, non_blocking=True)
-            ev = record_event()
+            ev = self._record()
         else:
             hb[:n].copy_(ids)
             ev = None
         return PendingTokens(self, hb, n, ev)
 
-    def _host_buffer(self, n: int) -> torch.Tensor:
-        _drain()
+    def _host_buffer(self, n: int, recording: Optional[bool] = None) -> torch.Tensor:
+        room = _drain(n, recording) if _unread else None
         for i, b in enumerate(self._free_host):
             if b.numel() >= n:
                 return self._free_host.pop(i)
+        if room is not None:
+            return room
         return torch.empty(max(n, 256), dtype=torch.int32, pin_memory=self.device.type == "cuda")
 
-    def _give_back(self, buf: torch.Tensor) -> None:
+    def _give_back(self, buf: torch.Tensor, event=None) -> None:
         if len(self._free_host) < 8:
             self._free_host.append(buf)
+        if event is not None and len(self._free_events) < 8:
+            self._free_events.append(event)
+
+    def _record(self):
+        """An event on the current stream, one that has been waited for where there is one (a new one takes 0.8 us more)."""
+        try:
+            return record_event(self._free_events.pop())
+        except (IndexError, RuntimeError):             # (none is there, or it belongs to another device)
+            return record_event()
 
     def _call(self, logits: torch.Tensor, params: Sequence[SamplingParams], counters: Sequence[int], ids: torch.Tensor) -> Optional["PendingTokens"]:
         """The rows' options in the launch's arguments and the ids written to the host by the kernel that chooses them: no array, copy or
@@ -219,9 +238,9 @@ class Sampler:
             return None
         if len(records) != _RECORD.size * n:
             return None
-        hb = self._host_buffer(n)
-        ops.sample_call(logits, records, draws, ids, hb)
-        return PendingTokens(self, hb, n, record_event(), by_kernel=True)
+        hb = self._host_buffer(n, recording=False)
+        ops.sample_call(logits, records, draws, ids, hb, recording=False)
+        return PendingTokens(self, hb, n, self._record(), by_kernel=True)
 
     def sample_async(self, logits: torch.Tensor, params: Sequence[SamplingParams], counters: Sequence[int],
                      out: Optional[torch.Tensor] = None) -> PendingTokens:

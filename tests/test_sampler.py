@@ -103,6 +103,43 @@ def test_results_that_are_let_go_do_not_pile_up():
     assert not sampler._unread
 
 
+def test_written_memory_of_an_unread_result_serves_the_next_call():
+    smp, event = Sampler("cpu"), Event()
+    seen = _let_go(event)
+    assert smp._host_buffer(4) is not seen()               # (still to be written)
+    event.done = True
+    assert smp._host_buffer(5) is not seen() and not sampler._unread       # (too short: it goes)
+    seen = _let_go(Event(done=True))
+    got = smp._host_buffer(4)
+    assert got is seen() and smp._host_buffer(4) is not got
+
+
+def test_an_event_is_recorded_again_only_after_it_was_waited_for(monkeypatch):
+    recorded, smp = [], Sampler("cpu")
+
+    def record(ev=None):
+        if ev is not None and ev.wait is not None:
+            ev.wait()
+        recorded.append(ev)
+        return ev or Event()
+    monkeypatch.setattr(sampler, "record_event", record)
+    monkeypatch.setattr(Event, "synchronize", lambda self: setattr(self, "done", True), raising=False)
+    first = sampler.PendingTokens(smp, torch.zeros(4, dtype=torch.int32), 4, smp._record())
+    own = first._event
+    assert smp._record() is not own                        # (nobody has waited for it)
+    assert first.result() == first.result() == [0] * 4
+    assert smp._record() is own and smp._record() is not own
+    assert recorded == [None, None, own, None]
+
+    def other_device():
+        raise RuntimeError("an event of another device")
+    smp._free_events.append(Event(done=True, wait=other_device))
+    assert smp._record().wait is None
+    for _ in range(20):
+        smp._give_back(torch.zeros(4, dtype=torch.int32), Event(done=True))
+    assert len(smp._free_events) <= 8
+
+
 def test_what_one_kernel_leaves_for_the_next_is_a_thread_s_and_a_stream_s_own(monkeypatch):
     from litinfer_amd.kernels import ops
     cpu, stream = torch.device("cpu"), [1]
