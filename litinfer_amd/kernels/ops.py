@@ -1518,7 +1518,8 @@ def _one_block(pairs: int, keys: int, dh: int, simds: int, spread=None, padded: 
     and replayed for other contexts of the same tables.
     Few keys: it saves the second kernel.  A whole step of 28 layers, 12 heads on 2 of 128, runs / one block: 6 pairs, 256 keys, contexts of 7 to 59 1,169 / 1,147, 14 pairs,
     47 to 94 1,278 / 1,260 (16 pairs, 200 to 250 1,283 / 1,322); contexts of 0.58 and of 0.5 to 1 of the table, 48 pairs, 512 keys 1,677 and 1,686 / 1,681 and 1,746, 80 pairs 1,735 and 1,746 / 1,712 and 1,760, 128 pairs, 1,024 keys 2,161 and 2,126 / 2,133 and 2,133; 24 layers, 14 on 2 of 64: 16
-    pairs, 512 keys 797 and 798 / 801 and 833, 48 pairs 997 and 1,004 / 977 and 1,002, 80 pairs, 1,024 keys 1,227 and 1,230 / 1,263 and 1,258, 128 pairs 1,402 and 1,393 / 1,378 and 1,377.
+    pairs, 512 keys 797 and 798 / 801 and 833, 48 pairs 997 and 1,004 / 977 and 1,002, 80 pairs, 1,024 keys 1,227 and 1,230 / 1,263 and 1,258, 128 pairs 1,402 and 1,393 / 1,378 and 1,377;
+    2 pairs, one context of 260, 300, 400 and 500 keys 738, 737, 737 and 737 / 731, 737, 765 and 767, 8 pairs of 300 and 480 755 and 757 / 760 and 790.
     Many keys: it pays where the pairs fill the chip with a block each, or nearly, and where no context is much longer than the others: its four waves take
     the longest alone, while runs are shared out among all SIMDs.  By the keys that the busiest SIMD works on: a quarter of the longest context (of the mean one
     in the rounds of blocks before the last) against 1.2 times its share of all keys and 200 for the second kernel, fitted to 115 batches, of which it chooses
